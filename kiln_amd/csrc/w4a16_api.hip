@@ -1,6 +1,7 @@
 // extern "C" entry points of libkiln_marlin_gemm (device side) and the
 // dispatcher that replaces `marlin_cuda` (crates/kiln-marlin-gemm/csrc/marlin_kernel.cu:731-819).
 #include <initializer_list>
+#include <memory>
 #include <mutex>
 #include <unordered_map>
 
@@ -764,6 +765,40 @@ WorkspaceLayout workspace_layout(const GemmPlan &gp, int m, int n, int k) {
     return w;
 }
 
+// The plan and the workspace layout of a call.  Forming them costs 0.3 us (matrix-core path) to 25 us (calls
+// with adapters of up to 16 rows, which price two kernels) of host time, as much as the launches they
+// describe, and a program asks for the same few shapes again and again, so they are kept by what they are a
+// function of.  Not in the tuning build, whose overrides change the answer.
+struct PlannedCall {
+    GemmPlan gp;
+    WorkspaceLayout wl;
+};
+std::shared_ptr<const PlannedCall> plan_call(int m, int n, int k, int cus, int thread_k, int thread_n, int lora) {
+    auto form = [&]() {
+        auto pc = std::make_shared<PlannedCall>();
+        plan_gemm(m, n, k, cus, thread_k, thread_n, lora, &pc->gp);
+        pc->wl = workspace_layout(pc->gp, m, n, k);
+        return pc;
+    };
+#ifdef KILN_W4A16_TUNING_HOOKS
+    return form();
+#else
+    static std::mutex mutex;
+    static std::unordered_map<SlabKey, std::shared_ptr<const PlannedCall>, SlabKeyHash> kept;
+    const SlabKey key{m, n, k, cus, thread_k, thread_n, lora};
+    {
+        std::lock_guard<std::mutex> lock(mutex);
+        auto it = kept.find(key);
+        if (it != kept.end()) return it->second;
+    }
+    std::shared_ptr<const PlannedCall> pc = form();
+    std::lock_guard<std::mutex> lock(mutex);
+    if (kept.size() > 4096) kept.clear();  // a caller cycling through many shapes; calls under way hold their own
+    kept.emplace(key, pc);
+    return pc;
+#endif
+}
+
 __global__ void dequant_f32_kernel(const u32x4 *__restrict__ B, const uint16_t *__restrict__ S,
                                    float *__restrict__ out, int K, int N, int Gs) {
     const int G = K / kGroupK;
@@ -879,10 +914,11 @@ kiln_marlin_status_t gemm_any(const void *A, const void *B, void *C, const void 
 
     const int cus = sms > 0 ? sms : compute_units(dev);
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    GemmPlan gp;
     const int lora_kind = !lora ? 0 : (lora->r_total % 8 == 0 ? 1 : 2);
-    plan_gemm(prob_m, prob_n, prob_k, cus, thread_k, thread_n, lora_kind, &gp);
-    const WorkspaceLayout wl = workspace_layout(gp, prob_m, prob_n, prob_k);
+    const std::shared_ptr<const PlannedCall> planned =
+        plan_call(prob_m, prob_n, prob_k, cus, thread_k > 0 ? thread_k : -1, thread_n > 0 ? thread_n : -1, lora_kind);
+    const GemmPlan &gp = planned->gp;
+    const WorkspaceLayout &wl = planned->wl;
     char *ws = reinterpret_cast<char *>(workspace);
     char *lora_t = ws + wl.lora_t;
     if (gp.prefill) {
@@ -1146,9 +1182,7 @@ kiln_marlin_status_t kiln_marlin_w4a16_gemm_static_scratch(const void *A, const 
     int current = -1;
     if (hipGetDevice(&current) != hipSuccess || current != dev || dev < 0 || dev >= kMaxDevices)
         return KILN_W4A16_ERR_ARGUMENT;
-    GemmPlan gp;
-    plan_gemm(prob_m, prob_n, prob_k, compute_units(dev), -1, -1, false, &gp);
-    if (workspace_layout(gp, prob_m, prob_n, prob_k).plain > kStaticScratchBytes) return KILN_W4A16_ERR_SCRATCH;
+    if (plan_call(prob_m, prob_n, prob_k, compute_units(dev), -1, -1, 0)->wl.plain > kStaticScratchBytes) return KILN_W4A16_ERR_SCRATCH;
     void *ws = static_scratch_ptr(current);
     if (!ws) return KILN_W4A16_ERR_LAUNCH;
     return gemm_any(A, B, C, s, prob_m, prob_n, prob_k, ws, groupsize, dev, stream, -1, -1, -1, nullptr);
