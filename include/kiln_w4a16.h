@@ -236,6 +236,20 @@ kiln_marlin_status_t kiln_w4a16_mlp(
 size_t kiln_w4a16_mlp_workspace_bytes(int prob_m, int hidden, int n_out, int n_down);
 
 /*
+ * The adapters of `count` <= 8 projections that run as one GEMM of prob_n columns, as one stacked set in the
+ * form the two entry points with adapters read: a_cat bf16 [r_total, k] = the A matrices (bf16 [ranks[i], k])
+ * one below the other, b_cat bf16 [prob_n, r_total] zero but for every projection's B (bf16 [rows[i],
+ * ranks[i]]) in its own rows, from first_rows[i] on, and its own rank columns.  With `interleaved` the columns
+ * are a fused gate/up pack: rows[i] = prob_n / 2, first_rows[i] 0 for gate and 8 for up.  r_total: the sum of
+ * the ranks rounded up to a multiple of 8, <= 64 (the columns past the sum are zero).  One launch on
+ * `stream`.  For adapters that arrive per call; a caller whose adapters stay does it once.
+ */
+kiln_marlin_status_t kiln_w4a16_stack_adapters(
+    const void *const *lora_a, const void *const *lora_b, const int *ranks, const int *first_rows,
+    const int *rows, int count, int prob_k, int prob_n, int r_total, int interleaved,
+    void *a_cat, void *b_cat, void *stream);
+
+/*
  * out[k, n] (f32, row-major) = (code - 8) * f32(scale), read from the tile
  * layout on the device.  The device-side statement of lib.rs:425; used to
  * prove the repack bit-exact.  No counterpart entry point in the reference.

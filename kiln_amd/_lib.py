@@ -26,6 +26,7 @@ EXPORTS = (
     "kiln_w4a16_gemm_swiglu_lora",
     "kiln_w4a16_mlp",
     "kiln_w4a16_mlp_workspace_bytes",
+    "kiln_w4a16_stack_adapters",
     "kiln_w4a16_quantize_and_pack_device",
     "kiln_w4a16_interleave_gate_up_device",
     "kiln_w4a16_repack_gptq_device",
@@ -88,6 +89,19 @@ TUNING_EXPORTS = (
 
 _libs: dict[bool, ctypes.CDLL] = {}
 _active_tuning = False
+_listeners: list = []   # told which library the wrappers call
+
+
+def on_active_library(fn) -> None:
+    """`fn(library)` whenever the library the wrappers call is loaded or changes (now, if there is one)."""
+    _listeners.append(fn)
+    if _active_tuning in _libs:
+        fn(_libs[_active_tuning])
+
+
+def _tell_active() -> None:
+    for fn in _listeners:
+        fn(_libs[_active_tuning])
 
 
 class LibraryMissing(RuntimeError):
@@ -104,6 +118,7 @@ def load_tuning() -> ctypes.CDLL:
     global _active_tuning
     L = _load(True)
     _active_tuning = True
+    _tell_active()
     return L
 
 
@@ -127,7 +142,9 @@ def use_shipped() -> None:
         L.kiln_w4a16_debug_lora_fold(-1)
         L.kiln_w4a16_debug_rowsum_fold(-1)
         L.kiln_w4a16_debug_mid_waves(0)
-    _active_tuning = False
+        _active_tuning = False
+        _load(False)
+        _tell_active()
 
 
 def _load(tuning: bool) -> ctypes.CDLL:
@@ -180,6 +197,9 @@ def _load(tuning: bool) -> ctypes.CDLL:
     L.kiln_w4a16_mlp.argtypes = [vp, vp, vp, vp, vp, vp, i, i, i, i, vp, i, i, vp]
     L.kiln_w4a16_mlp_workspace_bytes.restype = c.c_size_t
     L.kiln_w4a16_mlp_workspace_bytes.argtypes = [i, i, i, i]
+    L.kiln_w4a16_stack_adapters.restype = i
+    L.kiln_w4a16_stack_adapters.argtypes = [c.POINTER(vp), c.POINTER(vp), c.POINTER(i), c.POINTER(i), c.POINTER(i), i, i, i, i, i,
+                                            vp, vp, vp]
     L.kiln_w4a16_quantize_and_pack_device.restype = i
     L.kiln_w4a16_quantize_and_pack_device.argtypes = [vp, i, i, i, vp, vp, i, vp]
     L.kiln_w4a16_repack_gptq_device.restype = i
@@ -240,6 +260,8 @@ def _load(tuning: bool) -> ctypes.CDLL:
     L.kiln_marlin_proj_load.restype = i
     L.kiln_marlin_proj_load.argtypes = [c.c_char_p, i, pp]
     _libs[tuning] = L
+    if tuning == _active_tuning:
+        _tell_active()
     return L
 
 

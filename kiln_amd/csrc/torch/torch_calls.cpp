@@ -1,0 +1,450 @@
+// The entry points of libkiln_marlin_gemm called from Python without Python: operand checks, output allocation,
+// workspace lookup and the C call in one extension function each (CPython fast calls).
+//
+// What bounds a decode step driven from Python is the host: through ctypes one call cost 9.6 us (argument
+// checks, a device context, the stream handle, an allocation and fifteen converted arguments), more than the 4
+// to 8 us its kernel runs, so the GPU waited.
+//
+// Every function handles the plain case -- contiguous tensors of the right types on one device, a workspace that
+// is already there -- and answers None to anything else, which tells the caller to take its checked route
+// (whose error texts are the reference's).  The library's functions come as addresses (bind), so that the
+// callers' choice between the shipped library and the tuning build holds here too.
+#include <Python.h>
+
+#include <array>
+#include <cstdint>
+#include <mutex>
+#include <unordered_map>
+#include <vector>
+
+#include <ATen/ATen.h>
+#include <ATen/hip/EmptyTensor.h>
+#include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
+#include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include "kiln_w4a16.h"
+
+namespace {
+
+struct Library {
+    decltype(&kiln_marlin_w4a16_gemm) gemm = nullptr;
+    decltype(&kiln_w4a16_gemm_lora) gemm_lora = nullptr;
+    decltype(&kiln_w4a16_gemm_swiglu) swiglu = nullptr;
+    decltype(&kiln_w4a16_gemm_swiglu_lora) swiglu_lora = nullptr;
+    decltype(&kiln_w4a16_mlp) mlp = nullptr;
+    decltype(&kiln_w4a16_workspace_bytes) workspace_bytes = nullptr;
+    decltype(&kiln_w4a16_mlp_workspace_bytes) mlp_workspace_bytes = nullptr;
+    decltype(&kiln_w4a16_stack_adapters) stack_adapters = nullptr;
+};
+Library g_lib;  // written by bind() under the interpreter lock, like everything below
+
+PyTypeObject *g_stacked_type = nullptr, *g_single_type = nullptr;  // lora.StackedLora, lora.LoraProjectionWeights
+PyObject *g_names[6] = {};                                         // interned: a_cat b_cat ranks scales a b
+enum { kACat, kBCat, kRanks, kScales, kA, kB };
+
+// The workspaces marlin_gemm keeps, one per (device, stream): the same tensors, found without Python.
+struct StreamKey {
+    int device;
+    uintptr_t stream;
+    bool operator==(const StreamKey &o) const { return device == o.device && stream == o.stream; }
+};
+struct StreamKeyHash {
+    size_t operator()(const StreamKey &k) const { return (k.stream >> 4) * 31 + (size_t)k.device; }
+};
+std::unordered_map<StreamKey, at::Tensor, StreamKeyHash> &workspaces() {
+    static auto *map = new std::unordered_map<StreamKey, at::Tensor, StreamKeyHash>();  // outlives the interpreter's end
+    return *map;
+}
+
+const at::Tensor *tensor_of(PyObject *o) { return THPVariable_CheckExact(o) ? &THPVariable_Unpack(o) : nullptr; }
+
+bool plain(const at::Tensor &t, at::ScalarType type, int64_t dims, c10::Device device) {
+    return t.dim() == dims && t.scalar_type() == type && t.device() == device && t.layout() == at::kStrided && t.is_contiguous();
+}
+
+// One GEMM's operands, checked: everything marlin_gemm._check_gemm_args asks for, and contiguity.
+struct Problem {
+    const at::Tensor *x = nullptr, *b = nullptr, *s = nullptr;
+    int m = 0, n = 0, k = 0, groupsize = 0;
+    c10::Device device{c10::DeviceType::CPU};
+};
+
+bool packed_ok(const at::Tensor &b, const at::Tensor &s, int64_t k, int groupsize, c10::Device device, int64_t *n) {
+    if (!plain(b, at::kInt, 2, device) || !plain(s, at::kHalf, 2, device)) return false;
+    *n = s.size(1);
+    if (groupsize != 128 && groupsize != -1) return false;
+    return k > 0 && k % 128 == 0 && *n > 0 && *n % 256 == 0 && b.size(0) == k / 16 && b.size(1) == 2 * *n &&
+           s.size(0) == (groupsize == -1 ? 1 : k / 128) && k <= INT32_MAX && *n <= INT32_MAX / 2;
+}
+
+// max_rank: 2 for the GEMM entry points, 3 where a [batch, seq, k] activation is taken as well
+bool problem_of(PyObject *const *args, int max_rank, Problem *p) {
+    p->x = tensor_of(args[0]);
+    p->b = tensor_of(args[1]);
+    p->s = tensor_of(args[2]);
+    if (!p->x || !p->b || !p->s || !g_lib.gemm) return false;
+    const long g = PyLong_AsLong(args[3]);
+    if (g == -1 && PyErr_Occurred()) {
+        PyErr_Clear();
+        return false;
+    }
+    p->groupsize = (int)g;
+    const at::Tensor &x = *p->x;
+    const int64_t rank = x.dim();
+    if (rank < 2 || rank > max_rank || !x.is_cuda()) return false;
+    p->device = x.device();
+    if (!plain(x, at::kBFloat16, rank, p->device)) return false;
+    const int64_t k = x.size(rank - 1);
+    int64_t n = 0;
+    if (!packed_ok(*p->b, *p->s, k, p->groupsize, p->device, &n)) return false;
+    const int64_t m = x.numel() / k;
+    if (m < 1 || m > INT32_MAX) return false;
+    p->m = (int)m;
+    p->n = (int)n;
+    p->k = (int)k;
+    return true;
+}
+
+at::Tensor empty_bf16(at::IntArrayRef sizes, c10::Device device) {
+    return at::Tensor(at::detail::empty_cuda(sizes, at::kBFloat16, device, std::nullopt));
+}
+
+// the result: `given` if the caller passed one of the right form (false: it is of another), else a new tensor
+bool output_of(PyObject *given, const at::Tensor &x, int64_t columns, c10::Device device, at::Tensor *out) {
+    if (given && given != Py_None) {
+        const at::Tensor *t = tensor_of(given);
+        if (!t || !plain(*t, at::kBFloat16, 2, device) || t->size(1) != columns || t->size(0) != x.numel() / x.size(x.dim() - 1)) return false;
+        *out = *t;
+        return true;
+    }
+    const int64_t rank = x.dim();
+    std::array<int64_t, 3> sizes{x.size(0), rank == 3 ? x.size(1) : columns, columns};
+    *out = empty_bf16(at::IntArrayRef(sizes.data(), (size_t)rank), device);
+    return true;
+}
+
+// The device made current for the call, its stream, and that stream's workspace if it holds `bytes`.
+struct Launch {
+    c10::hip::HIPGuardMasqueradingAsCUDA guard;
+    void *stream;
+    at::Tensor workspace;
+    explicit Launch(c10::Device device)
+        : guard(device), stream((void *)c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(device.index()).stream()) {}
+    bool find_workspace(c10::Device device, size_t bytes) {
+        auto it = workspaces().find(StreamKey{device.index(), (uintptr_t)stream});
+        if (it == workspaces().end() || (size_t)it->second.numel() < bytes) return false;
+        workspace = it->second;
+        return true;
+    }
+};
+
+bool ints_of(PyObject *o, std::vector<int> *v) {
+    if (!PyTuple_CheckExact(o) && !PyList_CheckExact(o)) return false;
+    const Py_ssize_t count = PySequence_Fast_GET_SIZE(o);
+    for (Py_ssize_t i = 0; i < count; ++i) {
+        PyObject *e = PySequence_Fast_GET_ITEM(o, i);
+        if (!PyLong_CheckExact(e)) return false;
+        const long value = PyLong_AsLong(e);
+        if (value < 1 || value > INT32_MAX) {
+            PyErr_Clear();
+            return false;
+        }
+        v->push_back((int)value);
+    }
+    return true;
+}
+bool floats_of(PyObject *o, std::vector<float> *v) {
+    if (!PyTuple_CheckExact(o) && !PyList_CheckExact(o)) return false;
+    const Py_ssize_t count = PySequence_Fast_GET_SIZE(o);
+    for (Py_ssize_t i = 0; i < count; ++i) {
+        PyObject *e = PySequence_Fast_GET_ITEM(o, i);
+        if (!PyFloat_CheckExact(e)) return false;
+        v->push_back((float)PyFloat_AS_DOUBLE(e));
+    }
+    return true;
+}
+
+// Adapters as the library takes them.
+struct Adapters {
+    at::Tensor a, b;
+    std::vector<int> ranks;
+    std::vector<float> scales;
+    int r_total = 0;
+};
+
+bool adapters_ok(const Adapters &l, const Problem &p) {
+    return l.r_total >= 1 && l.r_total <= 64 && !l.ranks.empty() && l.ranks.size() <= 8 && l.ranks.size() == l.scales.size() &&
+           plain(l.a, at::kBFloat16, 2, p.device) && plain(l.b, at::kBFloat16, 2, p.device) && l.a.size(0) == l.r_total &&
+           l.a.size(1) == p.k && l.b.size(0) == p.n && l.b.size(1) == l.r_total;
+}
+
+// The launch itself, without the interpreter lock: a full queue makes it wait for the GPU.
+int call(const Problem &p, const at::Tensor &out, bool swiglu, const Adapters *l, const Launch &at_) {
+    const void *x = p.x->data_ptr(), *b = p.b->data_ptr();
+    void *s = p.s->data_ptr(), *c = out.data_ptr(), *ws = at_.workspace.data_ptr();
+    const int dev = p.device.index();
+    int st;
+    Py_BEGIN_ALLOW_THREADS
+    if (l) {
+        const void *a = l->a.data_ptr(), *lb = l->b.data_ptr();
+        const int count = (int)l->ranks.size();
+        st = swiglu ? g_lib.swiglu_lora(x, b, c, s, p.m, p.n / 2, p.k, ws, p.groupsize, dev, at_.stream, a, lb, l->r_total, count,
+                                        l->ranks.data(), l->scales.data())
+                    : g_lib.gemm_lora(x, b, c, s, p.m, p.n, p.k, ws, p.groupsize, dev, at_.stream, a, lb, l->r_total, count,
+                                      l->ranks.data(), l->scales.data());
+    } else {
+        st = swiglu ? g_lib.swiglu(x, b, c, s, p.m, p.n / 2, p.k, ws, p.groupsize, dev, at_.stream)
+                    : g_lib.gemm(x, b, c, s, p.m, p.n, p.k, ws, p.groupsize, dev, at_.stream, -1, -1, -1, 16);
+    }
+    Py_END_ALLOW_THREADS
+    return st;
+}
+
+// linear(x, b_packed, scales, groupsize, out, swiglu, max_rank)
+PyObject *py_linear(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
+    HANDLE_TH_ERRORS
+    Problem p;
+    if (nargs != 7 || !problem_of(args, (int)PyLong_AsLong(args[6]), &p)) Py_RETURN_NONE;
+    const bool swiglu = args[5] == Py_True;
+    Launch at_(p.device);
+    if (!at_.find_workspace(p.device, g_lib.workspace_bytes(p.m, p.n, p.k))) Py_RETURN_NONE;
+    at::Tensor out;
+    if (!output_of(args[4], *p.x, swiglu ? p.n / 2 : p.n, p.device, &out)) Py_RETURN_NONE;
+    if (call(p, out, swiglu, nullptr, at_) != KILN_W4A16_OK) Py_RETURN_NONE;
+    return THPVariable_Wrap(std::move(out));
+    END_HANDLE_TH_ERRORS
+}
+
+// linear_lora(x, b_packed, scales, groupsize, out, swiglu, lora_a, lora_b, ranks, lora_scales)
+PyObject *py_linear_lora(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
+    HANDLE_TH_ERRORS
+    Problem p;
+    if (nargs != 10 || !problem_of(args, 2, &p)) Py_RETURN_NONE;
+    const bool swiglu = args[5] == Py_True;
+    const at::Tensor *a = tensor_of(args[6]), *b = tensor_of(args[7]);
+    Adapters l;
+    if (!a || !b || !ints_of(args[8], &l.ranks) || !floats_of(args[9], &l.scales)) Py_RETURN_NONE;
+    l.a = *a;
+    l.b = *b;
+    for (int r : l.ranks) l.r_total += r <= 64 ? r : 65;
+    if (!adapters_ok(l, p)) Py_RETURN_NONE;
+    Launch at_(p.device);
+    if (!at_.find_workspace(p.device, g_lib.workspace_bytes(p.m, p.n, p.k))) Py_RETURN_NONE;
+    at::Tensor out;
+    if (!output_of(args[4], *p.x, swiglu ? p.n / 2 : p.n, p.device, &out)) Py_RETURN_NONE;
+    if (call(p, out, swiglu, &l, at_) != KILN_W4A16_OK) Py_RETURN_NONE;
+    return THPVariable_Wrap(std::move(out));
+    END_HANDLE_TH_ERRORS
+}
+
+// One projection's adapters among those of a fused call.
+struct Side {
+    at::Tensor a, b;
+    int rank = 0, first = 0, rows = 0;
+};
+
+// The adapters of one side (a StackedLora, or a LoraProjectionWeights scaled by `scale`), appended to `l`.
+bool add_side(PyObject *o, double scale, const Problem &p, int first, int rows, std::vector<Side> *sides, Adapters *l) {
+    const bool stacked = Py_TYPE(o) == g_stacked_type;
+    if (!stacked && Py_TYPE(o) != g_single_type) return false;
+    PyObject *pa = PyObject_GetAttr(o, g_names[stacked ? kACat : kA]), *pb = PyObject_GetAttr(o, g_names[stacked ? kBCat : kB]);
+    PyObject *pr = stacked ? PyObject_GetAttr(o, g_names[kRanks]) : nullptr, *ps = stacked ? PyObject_GetAttr(o, g_names[kScales]) : nullptr;
+    Side side;
+    bool ok = pa && pb && (!stacked || (pr && ps));
+    if (!ok) PyErr_Clear();
+    if (ok) {
+        const at::Tensor *a = tensor_of(pa), *b = tensor_of(pb);
+        ok = a && b && plain(*a, at::kBFloat16, 2, p.device) && plain(*b, at::kBFloat16, 2, p.device) && a->size(1) == p.k &&
+             b->size(0) == rows && a->size(0) == b->size(1) && a->size(0) >= 1 && a->size(0) <= 64;
+        if (ok) {
+            side.a = *a;
+            side.b = *b;
+            side.rank = (int)a->size(0);
+            side.first = first;
+            side.rows = rows;
+        }
+    }
+    if (ok && stacked) {
+        const size_t before = l->ranks.size();
+        ok = ints_of(pr, &l->ranks) && floats_of(ps, &l->scales) && l->ranks.size() == l->scales.size();
+        int sum = 0;
+        for (size_t i = before; i < l->ranks.size(); ++i) sum += l->ranks[i] <= 64 ? l->ranks[i] : 65;
+        ok = ok && sum == side.rank;
+    } else if (ok) {
+        l->ranks.push_back(side.rank);
+        l->scales.push_back((float)scale);
+    }
+    Py_XDECREF(pa);
+    Py_XDECREF(pb);
+    Py_XDECREF(pr);
+    Py_XDECREF(ps);
+    if (!ok) return false;
+    l->r_total += side.rank;
+    sides->push_back(std::move(side));
+    return l->r_total <= 64 && l->ranks.size() <= 8 && sides->size() <= 8;
+}
+
+// linear_sides(x, b_packed, scales, groupsize, swiglu, sides, widths, lora_scale, split): a GEMM whose columns belong
+// to several projections -- side by side, `widths` columns each, or with `swiglu` gate and up interleaved
+// (widths = n_out twice) -- each with its adapters or None.  Several sides, and stacked ranks that are not
+// multiples of 8, become one stacked set in a launch of their own in front.  `split`: the result comes as
+// one view per projection.
+PyObject *py_linear_sides(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
+    HANDLE_TH_ERRORS
+    Problem p;
+    if (nargs != 9 || !problem_of(args, 3, &p)) Py_RETURN_NONE;
+    const bool swiglu = args[4] == Py_True, split = args[8] == Py_True;
+    std::vector<int> widths;
+    if (!PyTuple_CheckExact(args[5]) || !ints_of(args[6], &widths) || PyTuple_GET_SIZE(args[5]) != (Py_ssize_t)widths.size()) Py_RETURN_NONE;
+    const double scale = PyFloat_AsDouble(args[7]);
+    if (scale == -1.0 && PyErr_Occurred()) {
+        PyErr_Clear();
+        Py_RETURN_NONE;
+    }
+    Adapters l;
+    std::vector<Side> sides;
+    int64_t first = 0;
+    for (size_t i = 0; i < widths.size(); ++i) {
+        PyObject *o = PyTuple_GET_ITEM(args[5], (Py_ssize_t)i);
+        if (o != Py_None && !add_side(o, scale, p, swiglu ? (int)(8 * i) : (int)first, widths[i], &sides, &l)) Py_RETURN_NONE;
+        first += widths[i];
+    }
+    if (first != p.n || (swiglu && (widths.size() != 2 || widths[0] != widths[1]))) Py_RETURN_NONE;
+    Launch at_(p.device);
+    if (!at_.find_workspace(p.device, g_lib.workspace_bytes(p.m, p.n, p.k))) Py_RETURN_NONE;
+    if (!sides.empty()) {
+        const int padded = (l.r_total + 7) / 8 * 8;
+        if (sides.size() == 1 && padded == l.r_total && sides[0].rows == p.n) {
+            l.a = sides[0].a;
+            l.b = sides[0].b;
+        } else {
+            const int64_t a_elems = (int64_t)padded * p.k;  // a multiple of 1024 elements: both parts keep their alignment
+            at::Tensor both = empty_bf16({a_elems + (int64_t)p.n * padded}, p.device);
+            l.a = both.narrow(0, 0, a_elems).view({padded, p.k});
+            l.b = both.narrow(0, a_elems, (int64_t)p.n * padded).view({p.n, padded});
+            const void *pa[8], *pb[8];
+            int ranks[8], firsts[8], rows[8];
+            for (size_t i = 0; i < sides.size(); ++i) {
+                pa[i] = sides[i].a.data_ptr();
+                pb[i] = sides[i].b.data_ptr();
+                ranks[i] = sides[i].rank;
+                firsts[i] = sides[i].first;
+                rows[i] = sides[i].rows;
+            }
+            l.ranks.back() += padded - l.r_total;  // the last adapter gets the zero columns
+            l.r_total = padded;
+            const int st = g_lib.stack_adapters(pa, pb, ranks, firsts, rows, (int)sides.size(), p.k, p.n, padded, swiglu ? 1 : 0,
+                                                l.a.data_ptr(), l.b.data_ptr(), at_.stream);
+            if (st != KILN_W4A16_OK) Py_RETURN_NONE;
+        }
+        if (!adapters_ok(l, p)) Py_RETURN_NONE;
+    }
+    at::Tensor out;
+    if (!output_of(nullptr, *p.x, swiglu ? p.n / 2 : p.n, p.device, &out)) Py_RETURN_NONE;
+    if (call(p, out, swiglu, sides.empty() ? nullptr : &l, at_) != KILN_W4A16_OK) Py_RETURN_NONE;
+    if (!split) return THPVariable_Wrap(std::move(out));
+    std::vector<int64_t> w(widths.begin(), widths.end());
+    std::vector<at::Tensor> parts = out.split_with_sizes(w, -1);
+    PyObject *tuple = PyTuple_New((Py_ssize_t)parts.size());
+    if (!tuple) return nullptr;
+    for (size_t i = 0; i < parts.size(); ++i) {
+        PyObject *t = THPVariable_Wrap(std::move(parts[i]));
+        if (!t) {
+            Py_DECREF(tuple);
+            return nullptr;
+        }
+        PyTuple_SET_ITEM(tuple, (Py_ssize_t)i, t);
+    }
+    return tuple;
+    END_HANDLE_TH_ERRORS
+}
+
+// mlp(x, b_gate_up, s_gate_up, groupsize, b_down, s_down, out)
+PyObject *py_mlp(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
+    HANDLE_TH_ERRORS
+    Problem p;
+    if (nargs != 7 || !problem_of(args, 2, &p)) Py_RETURN_NONE;
+    const at::Tensor *bd = tensor_of(args[4]), *sd = tensor_of(args[5]);
+    int64_t n_down = 0;
+    const int n_out = p.n / 2;
+    if (!bd || !sd || !packed_ok(*bd, *sd, n_out, p.groupsize, p.device, &n_down)) Py_RETURN_NONE;
+    Launch at_(p.device);
+    if (!at_.find_workspace(p.device, g_lib.mlp_workspace_bytes(p.m, p.k, n_out, (int)n_down))) Py_RETURN_NONE;
+    at::Tensor out;
+    if (!output_of(args[6], *p.x, n_down, p.device, &out)) Py_RETURN_NONE;
+    const void *x = p.x->data_ptr(), *bgu = p.b->data_ptr(), *sgu = p.s->data_ptr(), *b2 = bd->data_ptr(), *s2 = sd->data_ptr();
+    void *y = out.data_ptr(), *ws = at_.workspace.data_ptr();
+    int st;
+    Py_BEGIN_ALLOW_THREADS
+    st = g_lib.mlp(x, bgu, sgu, b2, s2, y, p.m, p.k, n_out, (int)n_down, ws, p.groupsize, p.device.index(), at_.stream);
+    Py_END_ALLOW_THREADS
+    if (st != KILN_W4A16_OK) Py_RETURN_NONE;
+    return THPVariable_Wrap(std::move(out));
+    END_HANDLE_TH_ERRORS
+}
+
+// set_workspace(device index, stream handle, tensor)
+PyObject *py_set_workspace(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
+    HANDLE_TH_ERRORS
+    const at::Tensor *t = nargs == 3 ? tensor_of(args[2]) : nullptr;
+    if (!t || !t->is_cuda() || t->scalar_type() != at::kByte || !t->is_contiguous()) {
+        PyErr_SetString(PyExc_TypeError, "set_workspace takes (device index, stream handle, uint8 CUDA tensor)");
+        return nullptr;
+    }
+    const long device = PyLong_AsLong(args[0]);
+    const unsigned long long stream = PyLong_AsUnsignedLongLong(args[1]);
+    if (PyErr_Occurred()) return nullptr;
+    workspaces()[StreamKey{(int)device, (uintptr_t)stream}] = *t;
+    Py_RETURN_NONE;
+    END_HANDLE_TH_ERRORS
+}
+
+// bind(addresses of the library's functions, in the order of Library)
+PyObject *py_bind(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
+    if (nargs != 8) {
+        PyErr_SetString(PyExc_TypeError, "bind takes eight function addresses");
+        return nullptr;
+    }
+    void *p[8];
+    for (int i = 0; i < 8; ++i) p[i] = PyLong_AsVoidPtr(args[i]);
+    if (PyErr_Occurred()) return nullptr;
+    g_lib.gemm = reinterpret_cast<decltype(g_lib.gemm)>(p[0]);
+    g_lib.gemm_lora = reinterpret_cast<decltype(g_lib.gemm_lora)>(p[1]);
+    g_lib.swiglu = reinterpret_cast<decltype(g_lib.swiglu)>(p[2]);
+    g_lib.swiglu_lora = reinterpret_cast<decltype(g_lib.swiglu_lora)>(p[3]);
+    g_lib.mlp = reinterpret_cast<decltype(g_lib.mlp)>(p[4]);
+    g_lib.workspace_bytes = reinterpret_cast<decltype(g_lib.workspace_bytes)>(p[5]);
+    g_lib.mlp_workspace_bytes = reinterpret_cast<decltype(g_lib.mlp_workspace_bytes)>(p[6]);
+    g_lib.stack_adapters = reinterpret_cast<decltype(g_lib.stack_adapters)>(p[7]);
+    Py_RETURN_NONE;
+}
+
+// set_adapter_types(StackedLora, LoraProjectionWeights)
+PyObject *py_set_adapter_types(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
+    if (nargs != 2 || !PyType_Check(args[0]) || !PyType_Check(args[1])) {
+        PyErr_SetString(PyExc_TypeError, "set_adapter_types takes two classes");
+        return nullptr;
+    }
+    Py_INCREF(args[0]);
+    Py_INCREF(args[1]);
+    g_stacked_type = reinterpret_cast<PyTypeObject *>(args[0]);
+    g_single_type = reinterpret_cast<PyTypeObject *>(args[1]);
+    Py_RETURN_NONE;
+}
+
+#define FAST(name, fn) {name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(fn)), METH_FASTCALL, nullptr}
+PyMethodDef g_methods[] = {FAST("linear", py_linear), FAST("linear_lora", py_linear_lora), FAST("linear_sides", py_linear_sides),
+                           FAST("mlp", py_mlp), FAST("set_workspace", py_set_workspace), FAST("bind", py_bind),
+                           FAST("set_adapter_types", py_set_adapter_types), {nullptr, nullptr, 0, nullptr}};
+PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_torch_calls", nullptr, -1, g_methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__torch_calls(void) {
+    static const char *const names[6] = {"a_cat", "b_cat", "ranks", "scales", "a", "b"};
+    for (int i = 0; i < 6; ++i)
+        if (!(g_names[i] = PyUnicode_InternFromString(names[i]))) return nullptr;
+    return PyModule_Create(&g_module);
+}

@@ -28,7 +28,7 @@ from typing import Dict, List, Optional, Sequence, Tuple
 
 import torch
 
-from . import marlin_gemm, marlin_proj
+from . import _calls, marlin_gemm, marlin_proj
 from .lora import fuse_column_blocks, proj_forward, swiglu_forward, swiglu_lora_fits
 from .marlin_proj import MarlinPackedProj, MarlinProjError
 
@@ -47,6 +47,9 @@ class PackKind(Enum):
     GateProj = "gate_proj"
     UpProj = "up_proj"
     DownProj = "down_proj"
+
+    # members are singletons, so identity serves; Enum's own hash is a Python function, 0.2 us on every lookup
+    __hash__ = object.__hash__
 
 
 FULL_ATTENTION_KINDS = (PackKind.QProj, PackKind.KProj, PackKind.VProj, PackKind.OProj)
@@ -104,6 +107,11 @@ class LayerProjections:
         kinds = tuple(kinds)
         loras = loras or {}
         fused = self.same_input_fused.get(kinds)
+        if fused is not None:
+            ys = _calls.linear_sides(x, fused.b_packed, fused.scales, fused.groupsize, False, tuple(map(loras.get, kinds)),
+                                     tuple(self.packed[k].n for k in kinds), lora_scale, True)
+            if ys is not None:
+                return ys
         stacked = None
         if fused is not None and any(loras.get(k) is not None for k in kinds):
             widths = [self.packed[k].n for k in kinds]

@@ -14,7 +14,7 @@ from typing import Optional, Sequence
 
 import torch
 
-from . import marlin_gemm
+from . import _calls, marlin_gemm
 from .marlin_proj import MarlinPackedProj, MarlinProjError, matmul_bf16
 
 
@@ -31,6 +31,9 @@ class StackedLora:
     b_cat: torch.Tensor        # [out_features, r_total] bf16
     ranks: tuple
     scales: tuple              # per-adapter scale (alpha / rank times the adapter weight)
+
+
+_calls.set_adapter_types(StackedLora, LoraProjectionWeights)
 
 
 def stack_adapters(adapters: Sequence[LoraProjectionWeights], scales: Sequence[float]) -> StackedLora:
@@ -75,6 +78,9 @@ def proj_forward(x: torch.Tensor, packed: MarlinPackedProj, lora, lora_scale: fl
     or a StackedLora."""
     if lora is None:
         return matmul_bf16(x, packed)
+    y = _calls.linear_sides(x, packed.b_packed, packed.scales, packed.groupsize, False, (lora,), (packed.n,), lora_scale, False)
+    if y is not None:
+        return y
     if isinstance(lora, LoraProjectionWeights):
         lora = stack_adapters([lora], [lora_scale])
     if x.dim() not in (2, 3) or x.shape[-1] != packed.k:
@@ -98,6 +104,10 @@ def swiglu_forward(x: torch.Tensor, gate_up: MarlinPackedProj, gate_lora=None, u
     the two `mlp_proj_forward` calls with `lora_layer.gate_proj` / `up_proj`, `silu` and the multiply of
     forward.rs:2771-2819.  `gate_lora` / `up_lora` are None, a LoraProjectionWeights (scaled by
     `lora_scale`) or a StackedLora; together at most 64 rank columns and 8 adapters."""
+    y = _calls.linear_sides(x, gate_up.b_packed, gate_up.scales, gate_up.groupsize, True, (gate_lora, up_lora),
+                            (gate_up.n // 2, gate_up.n // 2), lora_scale, False)
+    if y is not None:
+        return y
     if x.dim() not in (2, 3) or x.shape[-1] != gate_up.k:
         raise MarlinProjError(f"marlin_proj: x last-dim {x.shape[-1]} != packed weight k {gate_up.k}")
     n_out = gate_up.n // 2

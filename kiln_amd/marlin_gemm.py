@@ -15,7 +15,7 @@ from types import SimpleNamespace
 import numpy as np
 import torch
 
-from . import _lib
+from . import _calls, _lib
 
 
 class MarlinGemmError(ValueError):
@@ -39,6 +39,7 @@ def _workspace(device: torch.device, stream_ptr: int, nbytes: int) -> torch.Tens
         ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
         ws[:_lib.load().kiln_w4a16_workspace_zeroed_bytes()].zero_()
         _workspaces[key] = ws
+        _calls.set_workspace(key[0], stream_ptr, ws)
     return ws
 
 
@@ -120,6 +121,10 @@ def marlin_w4a16_gemm(a: torch.Tensor, b_packed: torch.Tensor, scales: torch.Ten
     `thread_k` / `thread_n` are the tile overrides of the C entry point
     (the reference wrapper always passes -1, lib.rs:252-253).
     """
+    if thread_k <= 0 and thread_n <= 0:
+        y = _calls.linear(a, b_packed, scales, groupsize, out, False, 2)
+        if y is not None:
+            return y
     m, k, n = _check_gemm_args(a, b_packed, scales, groupsize)
     lib = _lib.load()
     a = a.contiguous()
@@ -338,6 +343,9 @@ def marlin_w4a16_gemm_swiglu(a: torch.Tensor, b_packed: torch.Tensor, scales: to
     Fused form of the gate GEMM, up GEMM, silu and multiply the reference issues separately
     (crates/kiln-model/src/forward.rs:2771-2819).
     """
+    y = _calls.linear(a, b_packed, scales, groupsize, out, True, 2)
+    if y is not None:
+        return y
     m, k, n = _check_gemm_args(a, b_packed, scales, groupsize)
     if n % 256 != 0:
         _bail(f"fused gate+up width {n} must be a multiple of 256")
@@ -365,6 +373,9 @@ def marlin_w4a16_mlp(x: torch.Tensor, b_gate_up: torch.Tensor, s_gate_up: torch.
     (crates/kiln-model/src/forward.rs:2723-2848) as one call: the fused gate+up SwiGLU GEMM, then the down
     GEMM, `silu(gate) * up` kept in the workspace between them.
     `b_gate_up` / `s_gate_up` from `pack.interleave_gate_up`, `b_down` / `s_down` the packed down projection."""
+    y = _calls.mlp(x, b_gate_up, s_gate_up, groupsize, b_down, s_down, out)
+    if y is not None:
+        return y
     m, k, n = _check_gemm_args(x, b_gate_up, s_gate_up, groupsize)
     if n % 256 != 0:
         _bail(f"fused gate+up width {n} must be a multiple of 256")
@@ -407,6 +418,9 @@ def marlin_w4a16_gemm_lora(a: torch.Tensor, b_packed: torch.Tensor, scales: torc
     `[n, r_total]` (B matrices stacked along columns), both bf16; `ranks` / `lora_scales`
     give each adapter's rank and scale.
     """
+    y = _calls.linear_lora(a, b_packed, scales, groupsize, out, False, lora_a, lora_b, ranks, lora_scales)
+    if y is not None:
+        return y
     m, k, n = _check_gemm_args(a, b_packed, scales, groupsize)
     ranks = [int(r) for r in ranks]
     lora_scales = [float(v) for v in lora_scales]
@@ -477,6 +491,9 @@ def marlin_w4a16_gemm_swiglu_lora(a: torch.Tensor, b_packed: torch.Tensor, scale
     then up's, stacked along rows), `lora_b` `[2 n_out, r_total]` from `interleave_gate_up_lora_b`;
     `ranks` / `lora_scales` one entry per stacked adapter.
     """
+    y = _calls.linear_lora(a, b_packed, scales, groupsize, out, True, lora_a, lora_b, ranks, lora_scales)
+    if y is not None:
+        return y
     m, k, n = _check_gemm_args(a, b_packed, scales, groupsize)
     if n % 256 != 0:
         _bail(f"fused gate+up width {n} must be a multiple of 256")

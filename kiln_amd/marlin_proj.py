@@ -26,7 +26,7 @@ import torch
 
 import ctypes
 
-from . import _lib, marlin_gemm
+from . import _calls, _lib, marlin_gemm
 
 
 class MarlinProjError(ValueError):
@@ -203,6 +203,9 @@ def pack_from_gptq(qweight: torch.Tensor, scales: torch.Tensor, qzeros: Optional
 
 def matmul_bf16(x: torch.Tensor, w: MarlinPackedProj) -> torch.Tensor:
     """marlin_proj.rs:285-319: `[m, k]` or `[batch, seq, k]` bf16 -> same rank, last dim n."""
+    y = _calls.linear(x, w.b_packed, w.scales, w.groupsize, None, False, 3)
+    if y is not None:
+        return y
     rank = x.dim()
     if w.native is None or rank not in (2, 3):
         return _matmul_bf16_py(x, w)
