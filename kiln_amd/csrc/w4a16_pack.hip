@@ -6,9 +6,8 @@
 // column s = f16(2 * max|w| / 15) (max == 0 -> 1.0), code = clamp(round(w / f32(s)) + 8, 0, 15) with
 // ties away from zero and Rust's saturating float-to-int cast.  The reference has no device-side
 // counterpart: marlin_proj.rs:86-181 downloads every weight, quantises on the host (17-58 s per
-// model load for its 104 projections, ARCHITECTURE.md:570) and uploads the result.  Both kernels
-// are bound by memory traffic that is small next to a single GEMM's (read the weight twice, write
-// an eighth of it), so they are written for exactness and simple indexing, not tuned.
+// model load for its 104 projections, ARCHITECTURE.md:570) and uploads the result.  Bound by memory
+// traffic: 2 bytes read and half a byte written per weight.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -67,65 +66,196 @@ __device__ float pack_f16_to_f32(uint16_t h) {
 
 __device__ __forceinline__ float bf16_bits_to_f32(uint16_t b) { return __builtin_bit_cast(float, (uint32_t)b << 16); }
 
-// max of |w| as the host forms it: std::max(acc, fabs(w)) starting from 0 keeps acc when w is NaN
-__device__ __forceinline__ float max_abs_step(float acc, float w) {
-    const float a = __builtin_fabsf(w);
-    return acc < a ? a : acc;
+__device__ __forceinline__ uint16_t scale_of_max(float mx) {  // lib.rs:408-411
+    return pack_f32_to_f16(__fdiv_rn(2.0f * (mx == 0.f ? 1.f : mx), 15.0f));
 }
 
-// Scales: block = 256 threads = 64 columns x 4 row lanes; grid (n / 64, scale groups).
-// lib.rs:394-412.
-__global__ __launch_bounds__(256) void w4a16_pack_scales_kernel(const uint16_t *__restrict__ w, int n, int g_rows,
-                                                                int Gs, uint16_t *__restrict__ scales) {
-    __shared__ float part[4][64];
-    const int c = threadIdx.x & 63, rl = threadIdx.x >> 6;
-    const int col = blockIdx.x * 64 + c, gs = blockIdx.y;
-    const uint16_t *src = w + (size_t)gs * g_rows * n + col;
-    float mx = 0.f;
-    for (int r = rl; r < g_rows; r += 4) mx = max_abs_step(mx, bf16_bits_to_f32(src[(size_t)r * n]));
-    part[rl][c] = mx;
-    __syncthreads();
-    if (rl != 0) return;
-    // rows in ascending order of their row lane: max is exact, so the order only matters for NaN,
-    // which max_abs_step never keeps
-    for (int i = 1; i < 4; ++i) mx = max_abs_step(mx, part[i][c]);
-    if (mx == 0.f) mx = 1.f;
-    scales[scale_index(gs, col, Gs)] = pack_f32_to_f16(__fdiv_rn(2.0f * mx, 15.0f));
+// The quantiser word for word (lib.rs:416-427).
+__device__ __forceinline__ uint32_t code_exactly(float w, float s) {
+    const float q = roundf(__fdiv_rn(w, s));
+    long long raw;  // Rust `as i32`: saturating, NaN -> 0
+    if (q != q) raw = 0;
+    else if (q >= 2147483647.0f) raw = 2147483647LL;
+    else if (q <= -2147483648.0f) raw = -2147483648LL;
+    else raw = (long long)q;
+    long long code = raw + 8;  // an i32 sum in the reference (lib.rs:423): wraps from a saturated raw
+    if (code > 2147483647LL) code -= 4294967296LL;
+    return (uint32_t)(code < 0 ? 0 : (code > 15 ? 15 : code));
 }
 
-// Codes: one wavefront per chunk (column tile nt, group g); lane = c + 16 kq writes its four words
-// (t = 0...3: rows 128 g + 32 t + 8 kq + j, j = 0...7, row j in nibble nibble_pos(j)) as one 16-byte store.
-// Block = 4 wavefronts = 4 neighbouring column tiles of one group.  lib.rs:416-427.
-__global__ __launch_bounds__(256) void w4a16_pack_codes_kernel(const uint16_t *__restrict__ w, int n, int G, int Gs,
-                                                               const uint16_t *__restrict__ scales,
-                                                               u32x4 *__restrict__ b_packed) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int nt = blockIdx.x * 4 + wave, g = blockIdx.y;
-    const int c = lane & 15, kq = lane >> 4;
-    const int col = nt * kTileN + c;
-    const int gs = Gs == 1 ? 0 : g;
-    const float s = pack_f16_to_f32(scales[scale_index(gs, col, Gs)]);
-    uint32_t words[4];
+// A block of the quantiser covers 128 columns x 128 rows (one group): wavefront t its rows 32 t ... 32 t + 31, lane
+// cg + 16 kq the eight columns 8 cg ... of the eight rows 8 kq ..., i.e. eight 16-byte loads a thread, all in flight at
+// once, and exactly the rows of one word of each of its columns (layout.h).
+constexpr int kQuantCols = 128;
+struct QuantTile {
+    u32x4 row[8];
+    __device__ __forceinline__ void load(const uint16_t *__restrict__ w, int n, int g, int col0, int lane, int t) {
+        const uint16_t *src = w + (size_t)(g * kGroupK + 32 * t + 8 * (lane >> 4)) * n + col0 + 8 * (lane & 15);
+        if (__builtin_expect((reinterpret_cast<uintptr_t>(w) & 15) == 0, 1)) {
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
+            for (int j = 0; j < 8; ++j) row[j] = *reinterpret_cast<const u32x4 *>(src + (size_t)j * n);
+        } else {  // a weight that starts off the 16-byte grid
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    row[j][i] = src[(size_t)j * n + 2 * i] | ((uint32_t)src[(size_t)j * n + 2 * i + 1] << 16);
+        }
+    }
+    __device__ __forceinline__ bool all_finite() const {  // no half at or above 0x7F80
+        const u32x4 m = fold([](uint32_t v) { return v & 0x7FFF7FFFu; });
+        uint32_t over = 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) over |= (m[i] + 0x00800080u) & 0x80008000u;
+        return over == 0;
+    }
+    // bits of max |w| of the lane's column pairs over its eight rows; a NaN counts as 0, as in the host's
+    // std::max(acc, fabs(w)), which keeps acc where w is NaN
+    __device__ __forceinline__ u32x4 max_bits() const {
+        u32x4 m = fold([](uint32_t v) { return v & 0x7FFF7FFFu; });
+        uint32_t nan = 0;  // a half above 0x7F80 (infinity) carries into its sign bit
+#pragma unroll
+        for (int i = 0; i < 4; ++i) nan |= (m[i] + 0x007F007Fu) & 0x80008000u;
+        if (nan) m = fold([](uint32_t v) {
+            v &= 0x7FFF7FFFu;
+            return ((v & 0xFFFFu) > 0x7F80u ? 0u : v & 0xFFFFu) | ((v >> 16) > 0x7F80u ? 0u : v & 0xFFFF0000u);
+        });
+        return m;
+    }
+    template <class F>
+    __device__ __forceinline__ u32x4 fold(F f) const {
+        u32x4 m;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            m[i] = f(row[0][i]);
+#pragma unroll
+            for (int j = 1; j < 8; ++j) m[i] = max_pair(m[i], f(row[j][i]));
+        }
+        return m;
+    }
+    static __device__ __forceinline__ uint32_t max_pair(uint32_t a, uint32_t b) {  // v_pk_max_u16
+        typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+        return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, a), __builtin_bit_cast(u16x2, b)));
+    }
+};
+
+// Column maxima of one group's 128 columns, in LDS as bf16 pairs [wavefront][cg]; a barrier makes them readable.
+__device__ __forceinline__ void meet_maxima(u32x4 m, int lane, int t, u32x4 (*part)[16]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        m[i] = QuantTile::max_pair(m[i], (uint32_t)__shfl_xor((int)m[i], 16));
+        m[i] = QuantTile::max_pair(m[i], (uint32_t)__shfl_xor((int)m[i], 32));
+    }
+    if (lane < 16) part[t][lane] = m;
+}
+__device__ __forceinline__ uint32_t column_max_bits(const u32x4 (*part)[16], int col) {
+    const uint16_t *p = reinterpret_cast<const uint16_t *>(part);
+    uint32_t m = 0;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) m = max(m, (uint32_t)p[t * kQuantCols + col]);
+    return m;
+}
+
+// One scale for all of K: first the maxima of every group, [G][n] bf16 bits (they lie where the words will) ...
+__global__ __launch_bounds__(256) void w4a16_pack_group_max_kernel(const uint16_t *__restrict__ w, int n,
+                                                                   uint16_t *__restrict__ group_max) {
+    __shared__ u32x4 part[4][16];
+    const int lane = threadIdx.x & 63, t = threadIdx.x >> 6, col0 = blockIdx.x * kQuantCols, g = blockIdx.y;
+    QuantTile tile;
+    tile.load(w, n, g, col0, lane, t);
+    meet_maxima(tile.max_bits(), lane, t, part);
+    __syncthreads();
+    if (threadIdx.x < kQuantCols) group_max[(size_t)g * n + col0 + threadIdx.x] = (uint16_t)column_max_bits(part, threadIdx.x);
+}
+// ... then theirs: block = 64 columns x 4 lanes over the groups.
+__global__ __launch_bounds__(256) void w4a16_pack_column_scale_kernel(const uint16_t *__restrict__ group_max, int n, int G,
+                                                                      uint16_t *__restrict__ scales) {
+    __shared__ uint32_t part[4][64];
+    const int c = threadIdx.x & 63, gl = threadIdx.x >> 6, col = blockIdx.x * 64 + c;
+    uint32_t m = 0;
+#pragma unroll 4
+    for (int g = gl; g < G; g += 4) m = max(m, (uint32_t)group_max[(size_t)g * n + col]);
+    part[gl][c] = m;
+    __syncthreads();
+    if (gl != 0) return;
+#pragma unroll
+    for (int i = 1; i < 4; ++i) m = max(m, part[i][c]);
+    scales[scale_index(0, col, 1)] = scale_of_max(bf16_bits_to_f32((uint16_t)m));
+}
+
+// Quantise and pack, the weight read once (it is held in registers between the maxima and the codes; as a kernel
+// for the scales and one for the codes with 2-byte loads the same work ran at 1.4 TB/s: 2560 x 9216 34 + 39 us).
+// GROUP_SCALES: form the group's scales and write them; else they are there.
+//
+// Codes by multiplication, the same integers as roundf(fl(w / s)): w has 8 significant bits and s 11, so for a half
+// h <= 8.5 (beyond, the code is 0 or 15 whatever the digits) h * s has 16 and w / s is either h itself or at least
+// 2^-15 of h away from it.  y = w * rcp(s) * (1 + 2^-19) is within 2^-18 of w / s, relatively: it lies past every half that
+// w / s reaches, ties among them, and short of every other, so its nearest integer is w / s rounded with ties
+// away from zero.  (Ties are common -- 2 max / 15 is often exact in fp16, then max / s = 7.5 -- so they cannot be left
+// to a slow path.)  Only where a weight is not finite or the scale is zero are codes formed step by step.  An IEEE
+// division per weight would be 110 us of vector work for the 107 M weights of a layer that take 43 us to read.
+template <bool GROUP_SCALES>
+__global__ __launch_bounds__(256) void w4a16_pack_quantise_kernel(const uint16_t *__restrict__ w, int n, int G,
+                                                                  uint16_t *__restrict__ scales, u32x4 *__restrict__ b_packed) {
+    __shared__ u32x4 part[4][16];
+    __shared__ __attribute__((aligned(16))) float s_col[kQuantCols], r_col[kQuantCols];
+    constexpr int kLanePad = 68, kTilePad = 4 * kLanePad;  // words per 16 lanes / per column tile: 64 and 256, padded against bank conflicts
+    __shared__ __attribute__((aligned(16))) uint32_t words[8 * kTilePad];
+    const int lane = threadIdx.x & 63, t = threadIdx.x >> 6, col0 = blockIdx.x * kQuantCols, g = blockIdx.y;
+    const int cg = lane & 15, kq = lane >> 4;
+    QuantTile tile;
+    tile.load(w, n, g, col0, lane, t);
+    const bool finite = tile.all_finite();
+    if constexpr (GROUP_SCALES) {
+        meet_maxima(tile.max_bits(), lane, t, part);
+        __syncthreads();
+    }
+    if (threadIdx.x < kQuantCols) {
+        const size_t si = scale_index(GROUP_SCALES ? g : 0, col0 + threadIdx.x, GROUP_SCALES ? G : 1);
+        uint16_t bits;
+        if constexpr (GROUP_SCALES) {
+            bits = scale_of_max(bf16_bits_to_f32((uint16_t)column_max_bits(part, threadIdx.x)));
+            scales[si] = bits;
+        } else {
+            bits = scales[si];
+        }
+        const float s = pack_f16_to_f32(bits);
+        s_col[threadIdx.x] = s;
+        r_col[threadIdx.x] = __builtin_amdgcn_rcpf(s) * (1.f + 0x1p-19f);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+        const float r = r_col[8 * cg + c];
         uint32_t word = 0;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int row = g * kGroupK + 32 * t + 8 * kq + j;
-            const float q = roundf(__fdiv_rn(bf16_bits_to_f32(w[(size_t)row * n + col]), s));
-            long long raw;  // Rust `as i32`: saturating, NaN -> 0
-            if (q != q) raw = 0;
-            else if (q >= 2147483647.0f) raw = 2147483647LL;
-            else if (q <= -2147483648.0f) raw = -2147483648LL;
-            else raw = (long long)q;
-            long long code = raw + 8;  // an i32 sum in the reference (lib.rs:423): wraps from a saturated raw
-            if (code > 2147483647LL) code -= 4294967296LL;
-            code = code < 0 ? 0 : (code > 15 ? 15 : code);
-            word |= (uint32_t)code << (4 * nibble_pos(j));
+        for (int b = 0; b < 4; ++b) {
+            // byte b of the word: rows j, j + 2 (nibble_pos), the first in its low nibble
+            float v[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const uint32_t pair = tile.row[4 * (b & 1) + (b >> 1) + 2 * i][c >> 1];
+                const float x = __builtin_bit_cast(float, (c & 1) ? pair & 0xFFFF0000u : pair << 16);
+                v[i] = __builtin_amdgcn_fmed3f(__builtin_rintf(x * r), -8.f, 7.f);
+            }
+            word = (uint32_t)__builtin_amdgcn_cvt_pk_u8_f32(__builtin_fmaf(v[1], 16.f, v[0]) + 136.f, b, word);
         }
-        words[t] = word;
+        if (__builtin_expect(!finite || r == __builtin_inff(), 0)) {
+            const uint16_t *src = w + (size_t)(g * kGroupK + 32 * t + 8 * kq) * n + col0 + 8 * cg + c;
+            const float s = s_col[8 * cg + c];
+            word = 0;
+#pragma unroll 1
+            for (int j = 0; j < 8; ++j) word |= code_exactly(bf16_bits_to_f32(src[(size_t)j * n]), s) << (4 * nibble_pos(j));
+        }
+        words[(cg >> 1) * kTilePad + kq * kLanePad + ((cg & 1) * 8 + c) * 4 + t] = word;
     }
-    b_packed[((size_t)nt * G + g) * (kChunkWords / 4) + lane] = u32x4{words[0], words[1], words[2], words[3]};
+    __syncthreads();
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+        const int u = p * 256 + threadIdx.x, nt = u >> 6, l = u & 63;  // chunk lane l of column tile nt
+        b_packed[((size_t)(col0 / kTileN + nt) * G + g) * (kChunkWords / 4) + l] =
+            *reinterpret_cast<const u32x4 *>(words + nt * kTilePad + (l >> 4) * kLanePad + (l & 15) * 4);
+    }
 }
 
 // Gate and up of equal shape into the pack the fused SwiGLU entry point reads (output tile j = gate
@@ -240,13 +370,19 @@ extern "C" kiln_marlin_status_t kiln_w4a16_quantize_and_pack_device(const void *
     if (k <= 0 || n <= 0 || k % 128 != 0 || n % 256 != 0 || !(groupsize == -1 || groupsize == 128))
         return KILN_W4A16_ERR_PROB_SHAPE;
     if (!weight_bf16 || !b_packed || !scales_f16) return KILN_W4A16_ERR_ARGUMENT;
-    const int G = k / kGroupK, Gs = groupsize == -1 ? 1 : G, g_rows = groupsize == -1 ? k : kGroupK;
-    if (Gs > 65535 || G > 65535) return KILN_W4A16_ERR_PROB_SHAPE;  // grid y
+    const int G = k / kGroupK;
+    if (G > 65535) return KILN_W4A16_ERR_PROB_SHAPE;  // grid y
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    w4a16_pack_scales_kernel<<<dim3(n / 64, Gs), 256, 0, st>>>((const uint16_t *)weight_bf16, n, g_rows, Gs,
-                                                                (uint16_t *)scales_f16);
-    if (hipGetLastError() != hipSuccess) return KILN_W4A16_ERR_LAUNCH;
-    w4a16_pack_codes_kernel<<<dim3(n / 64, G), 256, 0, st>>>((const uint16_t *)weight_bf16, n, G, Gs,
-                                                              (const uint16_t *)scales_f16, (u32x4 *)b_packed);
+    const uint16_t *w = (const uint16_t *)weight_bf16;
+    uint16_t *scales = (uint16_t *)scales_f16;
+    const dim3 grid(n / kQuantCols, G);
+    if (groupsize == 128) {
+        w4a16_pack_quantise_kernel<true><<<grid, 256, 0, st>>>(w, n, G, scales, (u32x4 *)b_packed);
+    } else {
+        uint16_t *group_max = (uint16_t *)b_packed;  // 2 n G bytes of the 64 n G that the words take afterwards
+        w4a16_pack_group_max_kernel<<<grid, 256, 0, st>>>(w, n, group_max);
+        w4a16_pack_column_scale_kernel<<<n / 64, 256, 0, st>>>(group_max, n, G, scales);
+        w4a16_pack_quantise_kernel<false><<<grid, 256, 0, st>>>(w, n, G, scales, (u32x4 *)b_packed);
+    }
     return hipGetLastError() == hipSuccess ? KILN_W4A16_OK : KILN_W4A16_ERR_LAUNCH;
 }
