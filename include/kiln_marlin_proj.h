@@ -78,6 +78,14 @@ int kiln_marlin_proj_pack_from_gptq(const int32_t *qweight, const uint16_t *scal
                                     kiln_marlin_packed_proj_t **out);
 
 /*
+ * A packed projection over device memory that the caller owns and keeps (words int32 [k/16, 2n] and scales fp16
+ * [k/g, n] as kiln_w4a16_quantize_and_pack_device and the repack entry points write them): for hosts whose
+ * tensors come from an allocator of their own.  kiln_marlin_proj_free frees the handle only.
+ */
+int kiln_marlin_proj_wrap(const void *b_packed, const void *scales, int64_t k, int64_t n, int groupsize, int dev,
+                          kiln_marlin_packed_proj_t **out);
+
+/*
  * matmul_bf16 (marlin_proj.rs:285-319): x is bf16, rank 2 [m, k] or rank 3
  * [batch, seq, k], contiguous; y receives [.., n] bf16.  `workspace` holds at
  * least kiln_w4a16_workspace_bytes(m, n, k) zero-initialised bytes (m = the

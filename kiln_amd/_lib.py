@@ -51,6 +51,7 @@ PROJ_EXPORTS = (
     "kiln_marlin_proj_pack_from_bf16",
     "kiln_marlin_proj_pack_from_bf16_batch",
     "kiln_marlin_proj_pack_from_gptq",
+    "kiln_marlin_proj_wrap",
     "kiln_marlin_proj_matmul_bf16",
     "kiln_marlin_proj_k",
     "kiln_marlin_proj_n",
@@ -239,6 +240,8 @@ def _load(tuning: bool) -> ctypes.CDLL:
                                                         c.POINTER(i), i, i, pp]
     L.kiln_marlin_proj_pack_from_gptq.restype = i
     L.kiln_marlin_proj_pack_from_gptq.argtypes = [vp, vp, vp, i64, i64, i, i, pp]
+    L.kiln_marlin_proj_wrap.restype = i
+    L.kiln_marlin_proj_wrap.argtypes = [vp, vp, i64, i64, i, i, pp]
     L.kiln_marlin_proj_matmul_bf16.restype = i
     L.kiln_marlin_proj_matmul_bf16.argtypes = [vp, vp, c.POINTER(i64), i, vp, vp, c.c_size_t, vp]
     for name, res in (("k", i64), ("n", i64), ("groupsize", i), ("b_packed", vp), ("scales", vp)):

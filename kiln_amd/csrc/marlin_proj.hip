@@ -26,6 +26,8 @@ struct kiln_marlin_packed_proj {
     int groupsize = 128;
     int64_t k = 0, n = 0;
     int dev = 0;
+    bool owned = true;         // b_packed and scales are freed with it (scales may lie behind b_packed: same_block)
+    bool same_block = false;
 };
 
 namespace kiln {
@@ -152,9 +154,10 @@ int upload_packed(const PackedHost &packed, int dev, kiln_marlin_packed_proj_t *
     return KILN_PROJ_OK;
 }
 
-// The three phases in one: the weight is quantised and packed where it lies, by two kernels on the
-// device's default stream (same bits as the host quantiser; KILN_W4A16_HOST_PACK=1 keeps the host
-// route of marlin_proj.rs:86-181).  Same validation, same results and messages as prepare_pack_job.
+// The three phases in one: the weight is quantised and packed where it lies, on the device's default stream
+// (same bits as the host quantiser; KILN_W4A16_HOST_PACK=1 keeps the host route of marlin_proj.rs:86-181).
+// Same validation, same results and messages as prepare_pack_job.  Words and scales share one allocation, and
+// only the caller waits for the stream: an allocation costs 5 to 70 us and a round trip to the device 10 to 20.
 int pack_on_device(const void *weight_t, int64_t k, int64_t n, int groupsize, int dev,
                    kiln_marlin_packed_proj_t **out) {
     *out = nullptr;
@@ -171,29 +174,40 @@ int pack_on_device(const void *weight_t, int64_t k, int64_t n, int groupsize, in
     w->n = n;
     w->groupsize = groupsize;
     w->dev = dev;
-    const size_t b_bytes = (size_t)k * n / 8 * sizeof(int32_t);
+    w->same_block = true;
+    const size_t b_bytes = (size_t)k * n / 8 * sizeof(int32_t);  // a multiple of 16 KiB
     const size_t s_bytes = num_groups(k, groupsize) * (size_t)n * sizeof(uint16_t);
-    if (hipMalloc(&w->b_packed, b_bytes) != hipSuccess) return fail("marlin_proj: allocate b_packed on device");
-    if (hipMalloc(&w->scales, s_bytes) != hipSuccess) {
-        (void)hipFree(w->b_packed);
-        return fail("marlin_proj: allocate scales on device");
-    }
+    if (hipMalloc(&w->b_packed, b_bytes + s_bytes) != hipSuccess) return fail("marlin_proj: allocate b_packed on device");
+    w->scales = static_cast<char *>(w->b_packed) + b_bytes;
     const int st = kiln_w4a16_quantize_and_pack_device(weight_t, (int)k, (int)n, groupsize, w->b_packed, w->scales, dev,
                                                        nullptr);
-    if (st != KILN_W4A16_OK || hipStreamSynchronize(nullptr) != hipSuccess) {
+    if (st != KILN_W4A16_OK) {
         (void)hipFree(w->b_packed);
-        (void)hipFree(w->scales);
         return fail(std::string("marlin_proj: pack on device: ") + kiln_w4a16_status_string((kiln_marlin_status_t)st));
     }
     *out = w.release();
     return KILN_PROJ_OK;
 }
 
+// waits for what pack_on_device enqueued; frees and clears `outs` if that failed
+int wait_for_packs(int dev, int count, kiln_marlin_packed_proj_t **outs) {
+    DeviceScope scope(dev);
+    if (scope.ok && hipStreamSynchronize(nullptr) == hipSuccess) return KILN_PROJ_OK;
+    for (int i = 0; i < count; ++i) {
+        kiln_marlin_proj_free(outs[i]);
+        outs[i] = nullptr;
+    }
+    return fail(std::string("marlin_proj: pack on device: ") + kiln_w4a16_status_string(KILN_W4A16_ERR_LAUNCH));
+}
+
 // marlin_proj.rs:198-207
 int pack_from_bf16(const void *weight_t, int64_t k, int64_t n, int groupsize, int dev,
                    kiln_marlin_packed_proj_t **out) {
     *out = nullptr;
-    if (!env_truthy("KILN_W4A16_HOST_PACK")) return pack_on_device(weight_t, k, n, groupsize, dev, out);
+    if (!env_truthy("KILN_W4A16_HOST_PACK")) {
+        const int st = pack_on_device(weight_t, k, n, groupsize, dev, out);
+        return st == KILN_PROJ_OK ? wait_for_packs(dev, 1, out) : st;
+    }
     std::optional<PackJobHost> job;
     const int st = prepare_pack_job(weight_t, k, n, groupsize, dev, job);
     if (st != KILN_PROJ_OK) return st;
@@ -216,7 +230,7 @@ int pack_from_bf16_batch(const void *const *weights_t, const int64_t *ks, const 
                 return st;
             }
         }
-        return KILN_PROJ_OK;
+        return dev < 0 ? KILN_PROJ_OK : wait_for_packs(dev, count, outs);
     }
     std::vector<std::optional<PackJobHost>> jobs((size_t)count);
     for (int i = 0; i < count; ++i) {
@@ -498,6 +512,25 @@ int kiln_marlin_proj_pack_from_gptq(const int32_t *qweight, const uint16_t *scal
     return pack_from_gptq(qweight, scales_f16, qzeros, k, n, groupsize, dev, out);
 }
 
+int kiln_marlin_proj_wrap(const void *b_packed, const void *scales, int64_t k, int64_t n, int groupsize, int dev,
+                          kiln_marlin_packed_proj_t **out) {
+    if (!out || !b_packed || !scales || dev < 0) return fail("marlin_proj: null argument");
+    *out = nullptr;
+    if (!shape_is_supported(k, n)) return KILN_PROJ_SKIPPED;
+    if (!(groupsize == -1 || groupsize == 128))
+        return fail("marlin_proj: groupsize must be -1 or 128 (got " + std::to_string(groupsize) + ")");
+    auto *w = new kiln_marlin_packed_proj;
+    w->b_packed = const_cast<void *>(b_packed);
+    w->scales = const_cast<void *>(scales);
+    w->k = k;
+    w->n = n;
+    w->groupsize = groupsize;
+    w->dev = dev;
+    w->owned = false;
+    *out = w;
+    return KILN_PROJ_OK;
+}
+
 int kiln_marlin_proj_matmul_bf16(const kiln_marlin_packed_proj_t *w, const void *x, const int64_t *dims, int rank,
                                  void *y, void *workspace, size_t workspace_bytes, void *stream) {
     return matmul_bf16(w, x, dims, rank, y, workspace, workspace_bytes, stream);
@@ -513,9 +546,9 @@ void kiln_marlin_proj_free(kiln_marlin_packed_proj_t *w) {
     if (!w) return;
     int prev = 0;
     const bool have_prev = hipGetDevice(&prev) == hipSuccess;
-    if (hipSetDevice(w->dev) == hipSuccess) {
+    if (w->owned && hipSetDevice(w->dev) == hipSuccess) {
         (void)hipFree(w->b_packed);
-        (void)hipFree(w->scales);
+        if (!w->same_block) (void)hipFree(w->scales);
     }
     if (have_prev) (void)hipSetDevice(prev);
     delete w;

@@ -37,6 +37,7 @@ struct Library {
     decltype(&kiln_w4a16_workspace_bytes) workspace_bytes = nullptr;
     decltype(&kiln_w4a16_mlp_workspace_bytes) mlp_workspace_bytes = nullptr;
     decltype(&kiln_w4a16_stack_adapters) stack_adapters = nullptr;
+    decltype(&kiln_w4a16_quantize_and_pack_device) quantize = nullptr;
 };
 Library g_lib;  // written by bind() under the interpreter lock, like everything below
 
@@ -385,6 +386,97 @@ PyObject *py_mlp(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     END_HANDLE_TH_ERRORS
 }
 
+// quantize(inputs, side_by_side): every (contiguous bf16 [k, n] weight, groupsize) of the tuple `inputs`, all on one
+// device, quantised and packed on the current stream -> a list of (words, scales), None where the shape is not
+// supported.  The inputs each tuple of `side_by_side` names by position (one k, one groupsize) get packed tensors that
+// lie one after the other in memory.
+PyObject *py_quantize(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
+    HANDLE_TH_ERRORS
+    if (nargs != 2 || !g_lib.quantize || !PyTuple_CheckExact(args[0]) || !PyTuple_CheckExact(args[1]) || PyTuple_GET_SIZE(args[0]) == 0)
+        Py_RETURN_NONE;
+    struct Item {
+        at::Tensor w, b, s;
+        int64_t k = 0, n = 0, groups = 0;
+        int g = 0;
+        bool supported = false;
+    };
+    std::vector<Item> items((size_t)PyTuple_GET_SIZE(args[0]));
+    for (size_t i = 0; i < items.size(); ++i) {
+        Item &it = items[i];
+        PyObject *pair = PyTuple_GET_ITEM(args[0], (Py_ssize_t)i);
+        if (!PyTuple_CheckExact(pair) || PyTuple_GET_SIZE(pair) != 2 || !PyLong_CheckExact(PyTuple_GET_ITEM(pair, 1))) Py_RETURN_NONE;
+        const at::Tensor *w = tensor_of(PyTuple_GET_ITEM(pair, 0));
+        it.g = (int)PyLong_AsLong(PyTuple_GET_ITEM(pair, 1));
+        if (!w || !w->is_cuda() || !plain(*w, at::kBFloat16, 2, i ? items[0].w.device() : w->device()) || (it.g != 128 && it.g != -1))
+            Py_RETURN_NONE;
+        it.w = *w;
+        it.k = w->size(0);
+        it.n = w->size(1);
+        if (it.k > INT32_MAX || it.n > INT32_MAX) Py_RETURN_NONE;
+        it.supported = it.k > 0 && it.n > 0 && it.k % 128 == 0 && it.n % 256 == 0;
+        it.groups = it.g == -1 ? 1 : it.k / 128;
+    }
+    const c10::Device device = items[0].w.device();
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(device);
+    void *stream = (void *)c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(device.index()).stream();
+    auto empty = [&](int64_t elems, at::ScalarType type) { return at::Tensor(at::detail::empty_cuda({elems}, type, device, std::nullopt)); };
+    // piece [first, first + n) of the columns of a packed pair of `total` columns
+    auto place = [](Item &it, const at::Tensor &b, const at::Tensor &s, int64_t first) {
+        it.b = b.as_strided({it.k / 16, 2 * it.n}, {2 * it.n, 1}, first * (it.k / 8));
+        it.s = s.as_strided({it.groups, it.n}, {it.n, 1}, first * it.groups);
+    };
+    for (Py_ssize_t r = 0; r < PyTuple_GET_SIZE(args[1]); ++r) {
+        std::vector<int> run;
+        PyObject *o = PyTuple_GET_ITEM(args[1], r);
+        if (!PyTuple_CheckExact(o) || PyTuple_GET_SIZE(o) == 0) Py_RETURN_NONE;
+        int64_t columns = 0;
+        for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(o); ++i) {
+            const long at_ = PyLong_AsLong(PyTuple_GET_ITEM(o, i));
+            if (at_ < 0 || at_ >= (long)items.size() || !items[(size_t)at_].supported || items[(size_t)at_].b.defined()) {
+                PyErr_Clear();
+                Py_RETURN_NONE;
+            }
+            run.push_back((int)at_);
+            const Item &it = items[(size_t)at_], &head = items[(size_t)run[0]];
+            if (it.k != head.k || it.g != head.g) Py_RETURN_NONE;
+            columns += it.n;
+        }
+        const Item &head = items[(size_t)run[0]];
+        at::Tensor b = empty(head.k / 8 * columns, at::kInt), s = empty(head.groups * columns, at::kHalf);
+        int64_t first = 0;
+        for (int i : run) {
+            place(items[(size_t)i], b, s, first);
+            first += items[(size_t)i].n;
+        }
+    }
+    for (Item &it : items) {
+        if (!it.supported) continue;
+        if (!it.b.defined()) place(it, empty(it.k / 8 * it.n, at::kInt), empty(it.groups * it.n, at::kHalf), 0);
+        if (g_lib.quantize(it.w.data_ptr(), (int)it.k, (int)it.n, it.g, it.b.data_ptr(), it.s.data_ptr(), device.index(), stream) != KILN_W4A16_OK)
+            Py_RETURN_NONE;
+    }
+    PyObject *list = PyList_New((Py_ssize_t)items.size());
+    if (!list) return nullptr;
+    for (size_t i = 0; i < items.size(); ++i) {
+        PyObject *entry = Py_None;
+        if (items[i].supported) {
+            PyObject *b = THPVariable_Wrap(std::move(items[i].b)), *s = THPVariable_Wrap(std::move(items[i].s));
+            entry = b && s ? PyTuple_Pack(2, b, s) : nullptr;
+            Py_XDECREF(b);
+            Py_XDECREF(s);
+            if (!entry) {
+                Py_DECREF(list);
+                return nullptr;
+            }
+        } else {
+            Py_INCREF(entry);
+        }
+        PyList_SET_ITEM(list, (Py_ssize_t)i, entry);
+    }
+    return list;
+    END_HANDLE_TH_ERRORS
+}
+
 // set_workspace(device index, stream handle, tensor)
 PyObject *py_set_workspace(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     HANDLE_TH_ERRORS
@@ -403,12 +495,12 @@ PyObject *py_set_workspace(PyObject *, PyObject *const *args, Py_ssize_t nargs) 
 
 // bind(addresses of the library's functions, in the order of Library)
 PyObject *py_bind(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
-    if (nargs != 8) {
-        PyErr_SetString(PyExc_TypeError, "bind takes eight function addresses");
+    if (nargs != 9) {
+        PyErr_SetString(PyExc_TypeError, "bind takes nine function addresses");
         return nullptr;
     }
-    void *p[8];
-    for (int i = 0; i < 8; ++i) p[i] = PyLong_AsVoidPtr(args[i]);
+    void *p[9];
+    for (int i = 0; i < 9; ++i) p[i] = PyLong_AsVoidPtr(args[i]);
     if (PyErr_Occurred()) return nullptr;
     g_lib.gemm = reinterpret_cast<decltype(g_lib.gemm)>(p[0]);
     g_lib.gemm_lora = reinterpret_cast<decltype(g_lib.gemm_lora)>(p[1]);
@@ -418,6 +510,7 @@ PyObject *py_bind(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     g_lib.workspace_bytes = reinterpret_cast<decltype(g_lib.workspace_bytes)>(p[5]);
     g_lib.mlp_workspace_bytes = reinterpret_cast<decltype(g_lib.mlp_workspace_bytes)>(p[6]);
     g_lib.stack_adapters = reinterpret_cast<decltype(g_lib.stack_adapters)>(p[7]);
+    g_lib.quantize = reinterpret_cast<decltype(g_lib.quantize)>(p[8]);
     Py_RETURN_NONE;
 }
 
@@ -436,7 +529,7 @@ PyObject *py_set_adapter_types(PyObject *, PyObject *const *args, Py_ssize_t nar
 
 #define FAST(name, fn) {name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(fn)), METH_FASTCALL, nullptr}
 PyMethodDef g_methods[] = {FAST("linear", py_linear), FAST("linear_lora", py_linear_lora), FAST("linear_sides", py_linear_sides),
-                           FAST("mlp", py_mlp), FAST("set_workspace", py_set_workspace), FAST("bind", py_bind),
+                           FAST("mlp", py_mlp), FAST("quantize", py_quantize), FAST("set_workspace", py_set_workspace), FAST("bind", py_bind),
                            FAST("set_adapter_types", py_set_adapter_types), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_torch_calls", nullptr, -1, g_methods, nullptr, nullptr, nullptr, nullptr};
 

@@ -165,10 +165,38 @@ def install_packed(layer: LayerProjections, kind: PackKind, packed: MarlinPacked
         layer.weights_t[kind] = None
 
 
+def _one_after_the_other(tensors: Sequence[torch.Tensor]) -> torch.Tensor:
+    """The contiguous tensors' elements in one tensor: a view if they lie so in one storage, else a copy."""
+    first = tensors[0]
+    end, storage = first.storage_offset(), first.untyped_storage().data_ptr()
+    for t in tensors:
+        if t.untyped_storage().data_ptr() != storage or t.storage_offset() != end or not t.is_contiguous():
+            return torch.cat([t.reshape(-1) for t in tensors])
+        end += t.numel()
+    return first.as_strided((end - first.storage_offset(),), (1,))
+
+
+def _same_input_runs(inputs: Sequence[Tuple[torch.Tensor, int]], meta: Sequence[PackEntry]) -> List[List[int]]:
+    """Which of the queued inputs `fuse_same_input` will pack side by side: lists of positions in the queue."""
+    at = {(e.layer_idx, e.kind): i for i, e in enumerate(meta)}
+    runs = []
+    for layer_idx in sorted({e.layer_idx for e in meta}):
+        for kinds in SAME_INPUT_GROUPS:
+            run = [at.get((layer_idx, k)) for k in kinds]
+            if any(i is None for i in run):
+                continue
+            weights = [inputs[i] for i in run]
+            if all(w.dim() == 2 and w.shape[0] == weights[0][0].shape[0] and g == weights[0][1] and
+                   marlin_proj.shape_is_supported(*w.shape) for w, g in weights):
+                runs.append(run)
+    return runs
+
+
 def fuse_same_input(layer: LayerProjections) -> int:
     """Pack the members of every group of SAME_INPUT_GROUPS that the layer has packed (same k, same
     groupsize) side by side as one projection.  In the tile layout a packed weight is a sequence of column
-    tiles, each with all of its K, and so are its scales: side by side is one after the other."""
+    tiles, each with all of its K, and so are its scales: side by side is one after the other -- where the members
+    lie so in memory already (`pack_layers` has them packed that way) nothing is copied."""
     built = 0
     for kinds in SAME_INPUT_GROUPS:
         members = [layer.packed.get(k) for k in kinds]
@@ -178,8 +206,8 @@ def fuse_same_input(layer: LayerProjections) -> int:
         if any(p.k != k or p.groupsize != g for p in members):
             continue
         n = sum(p.n for p in members)
-        b = torch.cat([p.b_packed.reshape(-1) for p in members]).reshape(k // 16, 2 * n)
-        s = torch.cat([p.scales.reshape(-1) for p in members]).reshape(-1, n)
+        b = _one_after_the_other([p.b_packed for p in members]).reshape(k // 16, 2 * n)
+        s = _one_after_the_other([p.scales for p in members]).reshape(-1, n)
         layer.same_input_fused[tuple(kinds)] = MarlinPackedProj(b, s, g, k, n)
         built += 1
     return built
@@ -201,7 +229,9 @@ def pack_layers(layers: Sequence[LayerProjections], kinds: Optional[Sequence[Pac
         li, lm = queue_layer(i, layer, kinds, groupsize)
         inputs += li
         meta += lm
-    packed = marlin_proj.pack_from_bf16_batch(inputs)
+    packed = marlin_proj.pack_on_device(inputs, _same_input_runs(inputs, meta)) if fuse_same_input_groups else None
+    if packed is None:
+        packed = marlin_proj.pack_from_bf16_batch(inputs)
     n_packed = 0
     for entry, p in zip(meta, packed):
         if p is not None:

@@ -213,6 +213,9 @@ def quantize_and_pack_device(weight_t: torch.Tensor, groupsize: int):
     if k % 128 != 0 or n % 256 != 0 or not (groupsize == -1 or groupsize == 128):
         _bail(f"unsupported shape k={k} n={n} groupsize={groupsize} (k % 128, n % 256, groupsize -1 or 128)")
     weight_t = weight_t.contiguous()
+    made = _calls.quantize(((weight_t, groupsize),), ())
+    if made is not None:
+        return made[0]
     g = k if groupsize == -1 else groupsize
     b_packed = torch.empty((k // 16, 2 * n), dtype=torch.int32, device=weight_t.device)
     scales = torch.empty((k // g, n), dtype=torch.float16, device=weight_t.device)

@@ -21,10 +21,11 @@ from __future__ import annotations
 from dataclasses import dataclass
 from typing import Optional, Sequence
 
+import ctypes
+import os
+
 import numpy as np
 import torch
-
-import ctypes
 
 from . import _calls, _lib, marlin_gemm
 
@@ -45,6 +46,24 @@ class _NativeOwner:
             self.handle = 0
 
 
+class _WrappingOwner:
+    """A handle over packed tensors of this process's allocator, made when the library first needs one."""
+
+    def __init__(self, b: torch.Tensor, s: torch.Tensor, k: int, n: int, groupsize: int):
+        self._args = (b, s, k, n, groupsize)
+        self._owner: Optional[_NativeOwner] = None
+
+    @property
+    def handle(self) -> int:
+        if self._owner is None:
+            b, s, k, n, groupsize = self._args
+            out = ctypes.c_void_p()
+            if _lib.load().kiln_marlin_proj_wrap(b.data_ptr(), s.data_ptr(), k, n, groupsize, _device_index(b), ctypes.byref(out)) != _lib.PROJ_OK:
+                _raise_last()
+            self._owner = _NativeOwner(out.value)
+        return self._owner.handle
+
+
 class _DeviceView:
     """Device memory of a native projection, exposed through the array interface torch reads."""
 
@@ -62,7 +81,7 @@ class MarlinPackedProj:
     groupsize: int           # -1 (per column) or 128
     k: int
     n: int
-    native: Optional[_NativeOwner] = None   # set when the C++ layer owns the memory
+    native: Optional[_NativeOwner | _WrappingOwner] = None   # the C++ layer's handle: it owns the memory, or wraps the tensors
 
 
 def _raise_last():
@@ -139,10 +158,49 @@ def upload_packed(packed: PackedHost, device: torch.device) -> MarlinPackedProj:
     return MarlinPackedProj(b, s, packed.groupsize, packed.k, packed.n)
 
 
+def _host_pack() -> bool:
+    """`KILN_W4A16_HOST_PACK`: the reference's download / host pack / upload instead of the device's quantiser."""
+    return os.environ.get("KILN_W4A16_HOST_PACK", "").strip().lower() in ("1", "true", "yes")
+
+
+def _empty_packed(k: int, n: int, groupsize: int, device: torch.device) -> tuple[torch.Tensor, torch.Tensor]:
+    return (torch.empty((k // 16, 2 * n), dtype=torch.int32, device=device),
+            torch.empty((1 if groupsize == -1 else k // groupsize, n), dtype=torch.float16, device=device))
+
+
+def _wrap(b: torch.Tensor, s: torch.Tensor, k: int, n: int, groupsize: int) -> MarlinPackedProj:
+    """A projection over packed tensors of this process's allocator."""
+    return MarlinPackedProj(b, s, groupsize, k, n, _WrappingOwner(b, s, k, n, groupsize))
+
+
+def pack_on_device(inputs: Sequence[tuple[torch.Tensor, int]],
+                   side_by_side: Sequence[Sequence[int]] = ()) -> Optional[list[Optional[MarlinPackedProj]]]:
+    """Every `(weight [k, n] bf16 on one GPU, groupsize)` quantised and packed where it lies, into memory of torch's
+    allocator, on the current stream; returns when it is done.  (Through the library's own allocations a layer of
+    seven projections spent 300 us on allocating and freeing 54 MB.)  Each list of `side_by_side` names inputs of
+    one k and groupsize whose packed forms are to lie one after the other in memory, which is what their
+    side-by-side pack is (`layer_pack.fuse_same_input`).  An unsupported shape yields None; anything the library's own
+    route refuses or treats otherwise makes the result None as a whole."""
+    if _host_pack() or not inputs or not inputs[0][0].is_cuda:
+        return None
+    device = inputs[0][0].device
+    torch.cuda.synchronize(device)    # the weights may come from any stream
+    inputs = tuple((t.to(torch.bfloat16).contiguous() if t.is_cuda else t, g) for t, g in inputs)
+    made = _calls.quantize(inputs, tuple(map(tuple, side_by_side)))
+    if made is None:
+        return None
+    outs = [None if bs is None else _wrap(*bs, *t.shape, g) for bs, (t, g) in zip(made, inputs)]
+    torch.cuda.current_stream(device).synchronize()
+    return outs
+
+
 def pack_from_bf16(weight_t: torch.Tensor, groupsize: int) -> Optional[MarlinPackedProj]:
     """marlin_proj.rs:198-207: `[k, n] = [in, out]` bf16 weight -> packed projection."""
     if weight_t.dim() != 2:
         raise MarlinProjError("marlin_proj: weight_t must be a 2D [k, n] tensor")
+    here = pack_on_device([(weight_t, groupsize)])
+    if here is not None:
+        return here[0]
     if weight_t.is_cuda and weight_t.dtype != torch.bfloat16:
         weight_t = weight_t.to(torch.bfloat16)
     w = weight_t.contiguous()
@@ -158,15 +216,18 @@ def pack_from_bf16(weight_t: torch.Tensor, groupsize: int) -> Optional[MarlinPac
 
 
 def pack_from_bf16_batch(inputs: Sequence[tuple[torch.Tensor, int]]) -> list[Optional[MarlinPackedProj]]:
-    """marlin_proj.rs:229-262: serial download, parallel CPU pack, serial upload; order kept."""
+    """marlin_proj.rs:229-262: every weight packed on the device in turn; on the host route serial download,
+    parallel CPU pack, serial upload.  Order kept."""
     if not inputs:
         return []
     device = inputs[0][0].device
-    ws = []
     for t, _ in inputs:
         if t.dim() != 2:
             raise MarlinProjError("marlin_proj: weight_t must be a 2D [k, n] tensor")
-        ws.append((t.to(torch.bfloat16) if t.is_cuda else t).contiguous())
+    here = pack_on_device(inputs)
+    if here is not None:
+        return here
+    ws = [(t.to(torch.bfloat16) if t.is_cuda else t).contiguous() for t, _ in inputs]
     if device.type == "cuda":
         torch.cuda.synchronize()
     count = len(ws)
@@ -187,6 +248,9 @@ def pack_from_gptq(qweight: torch.Tensor, scales: torch.Tensor, qzeros: Optional
     The reference has no such path (it dequantises GPTQ to bf16 and re-quantises)."""
     k, n = qweight.shape[0] * 8, qweight.shape[1]
     device = torch.device(device)
+    here = _repack_on_device(qweight, scales, qzeros, k, n, groupsize, device)
+    if here is not None:
+        return here
     q = np.ascontiguousarray(qweight.cpu().numpy().view(np.int32))
     s = np.ascontiguousarray(scales.cpu().numpy().view(np.uint16))
     z = None if qzeros is None else np.ascontiguousarray(qzeros.cpu().numpy().view(np.int32))
@@ -199,6 +263,64 @@ def pack_from_gptq(qweight: torch.Tensor, scales: torch.Tensor, qzeros: Optional
     if st != _lib.PROJ_OK:
         _raise_last()
     return _wrap_native(out.value, device)
+
+
+# Host tensors go to the device through pinned memory of torch's pool, at most this much at a time ...
+_STAGE_BYTES = 32 << 20
+# ... the first copy a short one, so that the link is busy while the rest is still being moved into the pinned
+# memory (12 MiB: 229 us from pinned memory alone, 248 in pieces of 2 and 10 MiB, 253 in one, 260 to 340 in
+# three or more, 354 as the runtime's own pageable copy)
+_FIRST_PIECE_BYTES = 2 << 20
+
+
+def _upload(sources: Sequence[torch.Tensor], dst: torch.Tensor, device: torch.device) -> None:
+    """Copy contiguous host tensors one after the other, each from a multiple of 256 bytes on, into the uint8 tensor
+    `dst` on the current stream; the host tensors may change once this returns, the copies may still be running."""
+    stage = torch.empty(min(_STAGE_BYTES, dst.numel()), dtype=torch.uint8, pin_memory=True)
+    base = sent = at = 0       # stage holds dst[base:]; dst[:sent] is on its way; dst[:at] is staged
+
+    def send():
+        nonlocal sent
+        dst[sent:at].copy_(stage[sent - base:at - base], non_blocking=True)
+        sent = at
+
+    for src in sources:
+        flat, done, at = src.view(-1).view(torch.uint8), 0, -(-at // 256) * 256
+        while done < flat.numel():
+            if at - base >= stage.numel():
+                send()
+                torch.cuda.current_stream(device).synchronize()   # the copies still read the stage
+                base = at
+            piece = min(_FIRST_PIECE_BYTES if sent == 0 else stage.numel(), flat.numel() - done, base + stage.numel() - at)
+            stage[at - base:at - base + piece].copy_(flat[done:done + piece])
+            done, at = done + piece, at + piece
+            if sent == 0:
+                send()
+    send()
+
+
+def _repack_on_device(qweight: torch.Tensor, scales: torch.Tensor, qzeros: Optional[torch.Tensor], k: int, n: int,
+                      groupsize: int, device: torch.device) -> Optional[MarlinPackedProj]:
+    """`pack_from_gptq` for contiguous host tensors of the checkpoint's types: uploaded through pinned memory and
+    rearranged on the device.  None where the library's route has the checks (or the error) to make."""
+    if _host_pack() or device.type != "cuda" or groupsize not in (-1, 128) or k == 0 or n == 0 or k % 128 != 0 or n % 256 != 0:
+        return None
+    groups = 1 if groupsize == -1 else k // groupsize
+    for t, dtype, size in ((qweight, torch.int32, k // 8 * n), (scales, torch.float16, groups * n), (qzeros, torch.int32, groups * n // 8)):
+        if t is not None and (t.is_cuda or t.dtype != dtype or t.numel() != size or not t.is_contiguous()):
+            return None
+    with torch.cuda.device(device):
+        device = torch.device("cuda", torch.cuda.current_device())
+        q_bytes, s_bytes = k // 2 * n, groups * n * 2     # (q_bytes is a multiple of 16 KiB)
+        raw = torch.empty(q_bytes + s_bytes, dtype=torch.uint8, device=device)
+        b_packed, s_tiled = _empty_packed(k, n, groupsize, device)
+        _upload((qweight, scales), raw, device)
+        if qzeros is not None and not (qzeros.numpy() == -0x77777778).all():   # 0x88888888, looked at while the copies run
+            return None
+        st = _lib.load().kiln_w4a16_repack_gptq_device(raw.data_ptr(), raw.data_ptr() + q_bytes, None, k, n, groupsize, b_packed.data_ptr(),
+                                                       s_tiled.data_ptr(), device.index, torch.cuda.current_stream(device).cuda_stream)
+        torch.cuda.current_stream(device).synchronize()
+    return _wrap(b_packed, s_tiled, k, n, groupsize) if st == 0 else None
 
 
 def matmul_bf16(x: torch.Tensor, w: MarlinPackedProj) -> torch.Tensor:
