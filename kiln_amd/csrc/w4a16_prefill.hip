@@ -103,6 +103,16 @@ __device__ __forceinline__ void direct_load_b128(const void *gptr, unsigned lds_
                  : "memory", "m0");
 }
 
+// A pointer that is the same in all lanes, in scalar registers whatever the compiler can prove.  A vector memory
+// instruction may read a scalar register only five wait states after a vector instruction (v_readfirstlane) wrote
+// it; the compiler keeps that distance for its own loads and cannot for those inside inline asm, so it is kept here.
+__device__ __forceinline__ const char *uniform(const char *p) {
+    const uint64_t v = reinterpret_cast<uint64_t>(p);
+    uint32_t lo = __builtin_amdgcn_readfirstlane((int)(uint32_t)v), hi = __builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
+    asm volatile("s_nop 4" : "+s"(lo), "+s"(hi));
+    return reinterpret_cast<const char *>(((uint64_t)hi << 32) | lo);
+}
+
 // Probe builds only (-DKILN_PREFILL_TIMELINE): wall-clock stamps per block.
 #ifdef KILN_PREFILL_TIMELINE
 __device__ long long *g_timeline;
@@ -343,10 +353,7 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
     const int g_begin = sliced ? ks * GSb : 0, g_end = sliced ? min(G, g_begin + GSb) : G;
 
     // --- A: global -> LDS without passing through registers --------------------
-    // A stage is BM rows x 32 columns of bf16 = 64 B per row, 4 units of 16 B;
-    // four stages form a ring and loads run three stages ahead of the products
-    // (a stage lasts about as long as one L2 round trip, so a shallower
-    // pipeline leaves the matrix cores waiting at every barrier).
+    // A stage is BM rows x 32 columns of bf16 = 64 B per row, 4 units of 16 B; four stages form a ring.
     // Unit c of row r is stored at unit position c ^ ((r >> 2) & 3): with four units
     // per row, any 16 consecutive rows read at one unit index then touch the 16
     // different 16-byte positions of a 256-byte bank line, so the 128-bit fragment
@@ -356,39 +363,40 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
     // unit (i % 4) ^ ((i / 16) & 3).
     // Wavefront w moves the 16-row blocks w, w + NW, ...
     // Rows past M re-read row M - 1: their products are never stored.
-    const uint16_t *a_src[APW];
+    // Addresses are a uniform base in scalar registers, advanced there, plus a lane's constant byte offset.
+    uint32_t a_off_g[APW];
 #pragma unroll
     for (int p = 0; p < APW; ++p) {
-        const int blk = wave + NW * p;
-        int row = m0 + blk * 16 + (lane >> 2);
-        row = row < M ? row : M - 1;
-        a_src[p] = A + (size_t)row * K + (size_t)g_begin * kGroupK + (((lane & 3) ^ ((lane >> 4) & 3)) * 8);
+        const int row = min(m0 + (wave + NW * p) * 16 + (lane >> 2), M - 1) - m0;
+        a_off_g[p] = (uint32_t)row * (uint32_t)K * 2u + (((lane & 3) ^ ((lane >> 4) & 3)) * 16);
     }
-    const int n_stages = 4 * (g_end - g_begin);
+    const char *a_ptr = uniform(reinterpret_cast<const char *>(A) + ((size_t)m0 * K + (size_t)g_begin * kGroupK) * 2);  // this group's stages
     const unsigned lds_base = (unsigned)(size_t)(lds_ptr_t)lds;
-    auto load_a = [&](int st) {  // stage st (32 columns of K) -> ring slot st & 3
-        const unsigned slot = lds_base + (st & 3) * kAStageBytes;
+    auto load_a = [&](const char *base, int slot) {
 #pragma unroll
-        for (int p = 0; p < APW; ++p) direct_load_b128(a_src[p] + (size_t)st * 32, slot + (wave + NW * p) * 1024);
+        for (int p = 0; p < APW; ++p) load_to_lds_b128(base, a_off_g[p], lds_base + slot * kAStageBytes + (wave + NW * p) * 1024);
     };
 
     // --- B: column sub-tile ni (32 columns = chunks 2ni, 2ni+1 of this wavefront);
     // load v (0/1) fetches lane (l32 % 16) + 16 * (2v + h) of chunk (l32 / 16).
     const int nt_base = (n0 + wn * 64) / kTileN;  // first 16-column tile of this wavefront
-    const u32x4 *b_src[2][2];
+    uint32_t b_off[2], s_off[2];
     const uint16_t *s_src[2];
 #pragma unroll
     for (int ni = 0; ni < 2; ++ni) {
         // SWIGLU: every 16-column tile holds 8 gate columns, then the 8 matching up columns; sub-tile 0
         // gathers the gate columns of the wavefront's four tiles, sub-tile 1 their up columns, so a lane
         // holds a gate value and its up value in the same register of the two accumulators
-        const int nt = SWIGLU ? nt_base + (l32 >> 3) : nt_base + 2 * ni + (l32 >> 4);
+        const int nt = SWIGLU ? (l32 >> 3) : 2 * ni + (l32 >> 4);
         const int c = SWIGLU ? (l32 & 7) + 8 * ni : (l32 & 15);
-#pragma unroll
-        for (int v = 0; v < 2; ++v) b_src[ni][v] = B + (size_t)nt * G * 64 + c + 16 * (2 * v + h);
-        s_src[ni] = S + (size_t)nt * Gs * kTileN + c;
+        b_off[ni] = ((uint32_t)nt * (uint32_t)G * 64u + c + 16 * h) * 16u;  // + 512 for v = 1
+        s_off[ni] = ((uint32_t)nt * (uint32_t)Gs * kTileN + c) * 2u;
+        s_src[ni] = S + (size_t)nt_base * Gs * kTileN + s_off[ni] / 2;
     }
     const int gs_mask = (Gs == 1) ? 0 : -1;
+    const int s_step = (Gs == 1) ? 0 : kTileN * 2;  // bytes from a group's scales to the next one's
+    const char *b_ptr = uniform(reinterpret_cast<const char *>(B) + ((size_t)nt_base * G + g_begin) * 1024);
+    const char *s_ptr = uniform(reinterpret_cast<const char *>(S) + (size_t)nt_base * Gs * kTileN * 2 + (size_t)(g_begin & gs_mask) * kTileN * 2);
     // a zero scale would break the running rescale below; it is replaced by a
     // value too small to matter (the same value in the extension contraction)
     auto scale_value = [&](uint32_t raw) {
@@ -412,21 +420,39 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[mi][ni][r] = 0.f;
 
-    // prologue: three stages of A, the first group's weights
-    load_a(0);
-    load_a(1);
-    load_a(2);
-    u32x4 bw[2][2], bw_next[2][2];
-    uint32_t sc_raw[2], sc_raw_next[2];
+    // --- the main loop's schedule ---------------------------------------------
+    // The matrix cores bound this loop, so everything else is placed under their products, by hand: a stage
+    // (32 of K) is MI phases of four products each, phase mi = row tile mi, both column sub-tiles, both k16 steps.
+    //   * Fragments of A are read a stage ahead: the two of row tile mi right behind phase mi's products, for the
+    //     next stage.  They are used MI phases later, so no product waits for LDS.
+    //   * Behind phase 0 comes the stage's one barrier: the next stage has landed (counted waits), and every
+    //     wavefront holds all of this stage's fragments, so its slot is free at once -- the loads asked for then
+    //     fill it, four stages ahead of their use with a ring of four.
+    //   * The next stage's four operands of B are expanded from their words half an operand at a time (3 or 4
+    //     vector instructions) behind a product each.
+    //   * The group's change of scale (below) goes tile by tile behind products of other tiles: from phase 1 of
+    //     the group's last stage on, and over the first phases of the next group's first stage.
+    // sched_barrier pins the order; left to itself the compiler gathers the fragment reads, the expansions and the
+    // 128 multiplies of a group in front of the products that need them, and the matrix cores idle there (measured
+    // with such a loop, 2560 -> 2 x 9216 at 8192 rows: 56 % of the cycles busy).
+    u32x4 bw[2][2], bw_next[2][2];  // the group's words of B, and the next group's
+    uint32_t sc_raw[2];
+    auto request_b = [&](u32x4(&w)[2][2], const char *base, const char *sbase) {
 #pragma unroll
-    for (int ni = 0; ni < 2; ++ni) {
-        bw[ni][0] = async_load_b128(b_src[ni][0] + (size_t)g_begin * 64);
-        bw[ni][1] = async_load_b128(b_src[ni][1] + (size_t)g_begin * 64);
-        sc_raw[ni] = async_load_u16(s_src[ni] + (size_t)(g_begin & gs_mask) * kTileN);
-    }
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-    __syncthreads();
-    float sc[2];
+        for (int ni = 0; ni < 2; ++ni) {
+            asm volatile("global_load_dwordx4 %0, %1, %2" : "=&v"(w[ni][0]) : "v"(b_off[ni]), "s"(base) : "memory");
+            asm volatile("global_load_dwordx4 %0, %1, %2 offset:512" : "=&v"(w[ni][1]) : "v"(b_off[ni]), "s"(base) : "memory");
+            load_u16(sc_raw[ni], sbase, s_off[ni]);
+        }
+    };
+    // prologue: the first group's words, four stages of A
+    request_b(bw, b_ptr, s_ptr);
+#pragma unroll
+    for (int st = 0; st < 4; ++st) load_a(a_ptr + st * 64, st);
+    wait_vector_loads<3 * APW>();  // the words and stage 0
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" : : : "memory");
+    float sc[2], f[2] = {1.f, 1.f};
 #pragma unroll
     for (int ni = 0; ni < 2; ++ni) {
         pin(bw[ni][0]);
@@ -434,141 +460,158 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
         pin(sc_raw[ni]);
         sc[ni] = scale_value(sc_raw[ni]);
     }
-
-    // RS: c[group][row] = -136 * (row sum of the group), f32, behind the ring
+    bf16x8 af[MI][2], bf[2][2];
+    auto read_a = [&](auto slotc, int mi) {
+#pragma unroll
+        for (int sp = 0; sp < 2; ++sp)
+            af[mi][sp] = *reinterpret_cast<const bf16x8 *>(lds + decltype(slotc)::value * kAStageBytes + a_off[sp] + mi * 32 * 64);
+    };
+    // RS: c[group][row] = -136 * (row sum of the group), f32, behind the ring.  Wavefront w sums rows w * RPW ...: lane ->
+    // row lane / 4, unit lane % 4 of a stage; the four lanes of a row meet when the group ends.
+    int g_now = g_begin;
     [[maybe_unused]] float gsum[RS ? RPW / 16 : 1] = {};
     [[maybe_unused]] float *csum = reinterpret_cast<float *>(lds + kAStages * kAStageBytes);
-    [[maybe_unused]] const int g_peek = max(g_begin, g_end - 3);
-    for (int g = g_begin; g < g_end; ++g) {
-        const bool more = g + 1 < g_end;
+    [[maybe_unused]] auto sum_rows = [&](auto slotc) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int st = 4 * (g - g_begin) + q;
-            if (st + 3 < n_stages) load_a(st + 3);  // into the slot read one stage ago
-            if (q == 0 && more) {
+        for (int rr = 0; rr < RPW / 16; ++rr) {
+            const int row = wave * RPW + rr * 16 + (lane >> 2);
+            const u32x4 v = *reinterpret_cast<const u32x4 *>(lds + decltype(slotc)::value * kAStageBytes + row * 64 + (((lane & 3) ^ ((row >> 2) & 3)) * 16));
+            gsum[rr] += sum_bf16x8(v);
+        }
+    };
+    [[maybe_unused]] auto flush_rows = [&](int gl) {
 #pragma unroll
-                for (int ni = 0; ni < 2; ++ni) {
-                    bw_next[ni][0] = async_load_b128(b_src[ni][0] + (size_t)(g + 1) * 64);
-                    bw_next[ni][1] = async_load_b128(b_src[ni][1] + (size_t)(g + 1) * 64);
-                    sc_raw_next[ni] = async_load_u16(s_src[ni] + (size_t)((g + 1) & gs_mask) * kTileN);
-                }
-            }
-            if constexpr (FOLD) {
-                // (one more load in flight only makes the counted waits below stricter)
-                if (q == 0 && g == g_peek)
-                    prefill_fold_peek(pf, m0, min(BM, M - m0), lane, lds_base + kFoldPeekOffset + wave * 256);
-            }
-            const unsigned char *slot = lds + (st & 3) * kAStageBytes;
-            // Two k16 steps per stage (step u = 2q + sp uses word q of load sp).
-            // Fragments of the second step are read while the first step's
-            // products run, and each expansion of codes is placed between
-            // products: a product occupies the matrix pipe for 32 cycles, enough
-            // to issue the 7 VALU instructions of one expansion behind it.
-            if constexpr (RS) {
-                // this wavefront's rows of the stage: lane -> row lane / 4, unit lane % 4 (8 columns)
+        for (int rr = 0; rr < RPW / 16; ++rr) {
+            float s8 = gsum[rr];
+            s8 += dpp_move<0xB1>(s8);  // quad_perm [1,0,3,2]
+            s8 += dpp_move<0x4E>(s8);  // quad_perm [2,3,0,1]
+            csum[gl * BM + wave * RPW + rr * 16 + (lane >> 2)] = -kCodeBias * s8;  // the same value from all four lanes
+            gsum[rr] = 0.f;
+        }
+    };
+    auto word_of = [](const u32x4(&w)[2][2], auto qc, int ni, int sp) {
+        constexpr int q = decltype(qc)::value;
+        return (q == 0) ? w[ni][sp].x : (q == 1) ? w[ni][sp].y : (q == 2) ? w[ni][sp].z : w[ni][sp].w;
+    };
+    if constexpr (RS) sum_rows(std::integral_constant<int, 0>{});
 #pragma unroll
-                for (int rr = 0; rr < RPW / 16; ++rr) {
-                    const int row = wave * RPW + rr * 16 + (lane >> 2);
-                    const u32x4 v = *reinterpret_cast<const u32x4 *>(slot + row * 64 + (((lane & 3) ^ ((row >> 2) & 3)) * 16));
-                    const uint32_t wd[4] = {v.x, v.y, v.z, v.w};
-                    float s8 = 0.f;
+    for (int mi = 0; mi < MI; ++mi) read_a(std::integral_constant<int, 0>{}, mi);
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        s8 += __builtin_bit_cast(float, wd[i] << 16);
-                        s8 += __builtin_bit_cast(float, wd[i] & 0xFFFF0000u);
+    for (int ni = 0; ni < 2; ++ni)
+#pragma unroll
+        for (int sp = 0; sp < 2; ++sp) bf[ni][sp] = codes_to_bf16x8(word_of(bw, std::integral_constant<int, 0>{}, ni, sp), dq);
+
+    auto rescale_tile = [&](int t) {  // tile t = 2 mi + ni
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[t >> 1][t & 1][r] *= f[t & 1];
+    };
+    // one group; LAST: no further group, so nothing is asked for or read ahead past its end
+    auto group = [&](auto lastc) {
+        constexpr bool LAST = decltype(lastc)::value;
+        unrolled<0, 4>([&](auto qc) {
+            constexpr int q = decltype(qc)::value;
+            constexpr bool ahead = !(LAST && q == 3);  // there is a next stage
+            u32x4 bn[2][2];
+            unrolled<0, MI>([&](auto mc) {
+                constexpr int mi = decltype(mc)::value;
+                unrolled<0, 4>([&](auto jc) {
+                    constexpr int j = decltype(jc)::value, ni = j & 1, sp = j >> 1, slot = 4 * mi + j;
+                    acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[mi][sp], bf[ni][sp], acc[mi][ni], 0, 0, 0);
+                    // behind this product: halves of the next stage's operands of B ...
+                    constexpr int first = q == 3 ? 4 : 0, room = 4 * MI - first;  // (the next group's words are there behind the barrier)
+                    if constexpr (ahead && slot >= first) {
+                        constexpr int h0 = (slot - first) * 8 / room, h1 = (slot - first + 1) * 8 / room;
+                        unrolled<h0, h1>([&](auto hc) {
+                            constexpr int hh = decltype(hc)::value, en = (hh >> 1) & 1, es = hh >> 2;
+                            const uint32_t w = q == 3 ? word_of(bw_next, std::integral_constant<int, 0>{}, en, es)
+                                                      : word_of(bw, std::integral_constant<int, (q + 1) & 3>{}, en, es);
+                            if constexpr ((hh & 1) == 0) {
+                                bn[en][es].x = (w & dq.mask) | dq.magic;
+                                bn[en][es].y = ((w >> 4) & dq.mask) | dq.magic;
+                            } else {
+                                bn[en][es].z = ((w >> 8) & dq.mask) | dq.magic;
+                                bn[en][es].w = ((w >> 12) & dq.mask) | dq.magic;
+                            }
+                        });
                     }
-                    s8 += dpp_move<0xB1>(s8);  // quad_perm [1,0,3,2]
-                    s8 += dpp_move<0x4E>(s8);  // quad_perm [2,3,0,1]: the row's 32 columns
-                    gsum[rr] += s8;
+                    // ... and a part of the change of scale
+                    // tile t is complete behind phase t / 2 of the last stage and needed by that phase of the next
+                    // stage; MI = 4: tiles 0 | 1 2 | 3 4 in phases 1, 2, 3, tiles 5 | 6 | 7 in phases 0, 1, 2 of the next group
+                    constexpr int t0 = q == 3 ? (MI == 4 ? (mi < 2 ? 0 : 2 * mi - 3) : 0) : (MI == 4 ? 5 + mi : 2);
+                    constexpr int t1 = q == 3 ? (MI == 4 ? (mi == 0 ? 0 : 2 * mi - 1) : (mi == 0 ? 0 : 2)) : (MI == 4 ? 6 + mi : (mi == 0 ? 4 : 2));
+                    if constexpr ((q == 3 && !LAST) || (q == 0 && mi < MI - 1)) {
+                        unrolled<t0, t1>([&](auto tc) {
+                            constexpr int t = decltype(tc)::value;
+#pragma unroll
+                            for (int r = 4 * j; r < 4 * j + 4; ++r) acc[t >> 1][t & 1][r] *= f[t & 1];
+                        });
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                });
+                if constexpr (mi == 0 && ahead) {
+                    // Loads complete in issue order; behind the next stage's there are at most those of the two stages
+                    // after it and, unless they are needed now, the next group's six.
+                    constexpr int stages_behind = LAST ? 2 - q : 2;
+                    constexpr int others = (!LAST && (q == 1 || q == 2)) ? 6 : (LAST && FOLD && q > 0) ? 1 : 0;
+                    wait_vector_loads<stages_behind * APW + others>();
+                    wait_lds_reads();
+                    __builtin_amdgcn_s_barrier();
+                    asm volatile("" : : : "memory");
+                    if constexpr (!LAST) {
+                        load_a(a_ptr + (q + 4) * 64, q);
+                        if constexpr (q == 0) request_b(bw_next, b_ptr + 1024, s_ptr + s_step);
+                        if constexpr (q == 3) {
+#pragma unroll
+                            for (int i = 0; i < 2; ++i) {
+                                pin(bw_next[i][0]);
+                                pin(bw_next[i][1]);
+                                pin(sc_raw[i]);
+                                // Running rescale: the accumulator holds (sum so far) / scale(g).  Switching to
+                                // the next group's scale multiplies it by scale(g) / scale(g+1); after the last
+                                // group, by scale(g).  Nothing is ever rounded to bf16.
+                                const float sn = scale_value(sc_raw[i]);
+                                f[i] = sc[i] * __builtin_amdgcn_rcpf(sn);
+                                sc[i] = sn;
+                            }
+                        }
+                    }
+                    // the early look at the words of a folded launch: a group of products ahead of its use
+                    if constexpr (FOLD && LAST && q == 0) prefill_fold_peek(pf, m0, min(BM, M - m0), lane, lds_base + kFoldPeekOffset + wave * 256);
                 }
-            }
-            bf16x8 a0[MI], a1[MI];
-#pragma unroll
-            for (int mi = 0; mi < MI; ++mi)
-                a0[mi] = *reinterpret_cast<const bf16x8 *>(slot + a_off[0] + mi * 32 * 64);
-            auto word_of = [&](int ni, int sp) {
-                return (q == 0) ? bw[ni][sp].x : (q == 1) ? bw[ni][sp].y : (q == 2) ? bw[ni][sp].z : bw[ni][sp].w;
-            };
-            bf16x8 b00 = codes_to_bf16x8(word_of(0, 0), dq);
-#pragma unroll
-            for (int mi = 0; mi < MI; ++mi)
-                a1[mi] = *reinterpret_cast<const bf16x8 *>(slot + a_off[1] + mi * 32 * 64);
-            const bf16x8 b10 = codes_to_bf16x8(word_of(1, 0), dq);
-#pragma unroll
-            for (int mi = 0; mi < MI; ++mi)
-                acc[mi][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0[mi], b00, acc[mi][0], 0, 0, 0);
-            const bf16x8 b01 = codes_to_bf16x8(word_of(0, 1), dq);
-#pragma unroll
-            for (int mi = 0; mi < MI; ++mi)
-                acc[mi][1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0[mi], b10, acc[mi][1], 0, 0, 0);
-            const bf16x8 b11 = codes_to_bf16x8(word_of(1, 1), dq);
-#pragma unroll
-            for (int mi = 0; mi < MI; ++mi)
-                acc[mi][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1[mi], b01, acc[mi][0], 0, 0, 0);
-#pragma unroll
-            for (int mi = 0; mi < MI; ++mi)
-                acc[mi][1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1[mi], b11, acc[mi][1], 0, 0, 0);
-            if constexpr (MI == 4) {
-                // scheduling hint: 4 x (product, 2 VALU, 1 LDS read), then 12 x (product, 2 VALU)
-    #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                if constexpr (ahead) {
+                    if constexpr (RS && mi == 0) {
+                        if constexpr (q == 3) flush_rows(g_now - g_begin);
+                        sum_rows(std::integral_constant<int, (q + 1) & 3>{});
+                    }
+                    read_a(std::integral_constant<int, (q + 1) & 3>{}, mi);
+                    __builtin_amdgcn_sched_barrier(0);
                 }
-    #pragma unroll
-                for (int i = 0; i < 12; ++i) {
-                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
-                }
-            }
-            // Stage st + 1 must have landed.  Loads complete in issue order; still
-            // allowed in flight are the loads of stages st + 2 and st + 3 (APW each)
-            // and, in three of four steps, the 6 weight/scale loads issued after
-            // stage st + 1's.  After step 3 that leaves the next group's weights
-            // complete as well.  The last group drains everything.
-            if (!more) __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-            else if (q == 3) __builtin_amdgcn_s_waitcnt(0x0F70 | (2 * APW));  // vmcnt(2 APW)
-            else __builtin_amdgcn_s_waitcnt(0x0F70 | (2 * APW + 6));          // vmcnt(2 APW + 6)
-            __syncthreads();
-        }
-        if constexpr (RS) {
-            if ((lane & 3) == 0) {
+            });
+            if constexpr (ahead) {
 #pragma unroll
-                for (int rr = 0; rr < RPW / 16; ++rr)
-                    csum[(g - g_begin) * BM + wave * RPW + rr * 16 + (lane >> 2)] = -kCodeBias * gsum[rr];
-            }
+                for (int ni = 0; ni < 2; ++ni)
 #pragma unroll
-            for (int rr = 0; rr < RPW / 16; ++rr) gsum[rr] = 0.f;
-        }
-        // Running rescale: the accumulator holds (sum so far) / scale(g).
-        // Switching to the next group's scale multiplies it by
-        // scale(g) / scale(g+1); after the last group, by scale(g).  One multiply
-        // per accumulator register and group; nothing is ever rounded to bf16.
-        float f[2];
-        if (more) {
-#pragma unroll
-            for (int ni = 0; ni < 2; ++ni) {
-                pin(bw_next[ni][0]);
-                pin(bw_next[ni][1]);
-                pin(sc_raw_next[ni]);
-                const float sn = scale_value(sc_raw_next[ni]);
-                f[ni] = sc[ni] * __builtin_amdgcn_rcpf(sn);
-                bw[ni][0] = bw_next[ni][0];
-                bw[ni][1] = bw_next[ni][1];
-                sc[ni] = sn;
+                    for (int sp = 0; sp < 2; ++sp) bf[ni][sp] = __builtin_bit_cast(bf16x8, bn[ni][sp]);
             }
-        } else {
-            f[0] = sc[0];
-            f[1] = sc[1];
-        }
+        });
+    };
+    for (; g_now + 1 < g_end; ++g_now) {
+        group(std::false_type{});
 #pragma unroll
         for (int ni = 0; ni < 2; ++ni)
 #pragma unroll
-            for (int mi = 0; mi < MI; ++mi)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) acc[mi][ni][r] *= f[ni];
+            for (int v = 0; v < 2; ++v) bw[ni][v] = bw_next[ni][v];
+        a_ptr += 256;
+        b_ptr += 1024;
+        s_ptr += s_step;
     }
+    group(std::true_type{});
+    if constexpr (RS) flush_rows(g_now - g_begin);
+    f[0] = sc[0];
+    f[1] = sc[1];
+#pragma unroll
+    for (int t = 0; t < 2 * MI; ++t) rescale_tile(t);
+    wait_vector_loads<0>();  // the early look
 
     KILN_TL(1);
     if constexpr (RS) __syncthreads();  // every wavefront's row sums are in LDS
