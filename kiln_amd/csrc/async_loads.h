@@ -39,6 +39,14 @@ __device__ __forceinline__ void load_to_lds_b128(const void *base, uint32_t lane
                  : "memory", "m0");
 }
 
+// ... and 4 bytes per lane, at lds_addr + 4 * lane.
+__device__ __forceinline__ void load_to_lds_b32(const void *base, uint32_t lane_off, unsigned lds_addr) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
+                 :
+                 : "v"(lane_off), "s"(base), "s"(lds_addr)
+                 : "memory", "m0");
+}
+
 // A zero the compiler cannot see through, defined where it is called: arithmetic that depends on
 // it stays behind the preceding asm statements instead of being hoisted to the top of a long
 // straight-line kernel (where it would hold registers for its whole length).

@@ -135,6 +135,15 @@ __device__ __forceinline__ float dpp_move(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
 }
 
+// Two values of a lane's column in neighbouring rows -> two bf16 values of neighbouring columns in one row: even lanes
+// get the first row's, odd lanes the second's (each pair of lanes swaps one value).
+__device__ __forceinline__ uint32_t neighbours_of_a_row(float first, float second, int lane) {
+    const uint32_t own = f32_to_bf16_bits(first) | ((uint32_t)f32_to_bf16_bits(second) << 16);
+    const uint32_t other = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)own, 0xB1, 0xF, 0xF, true);  // quad_perm [1,0,3,2]
+    // v_perm_b32: bytes 0-3 of `other`'s register are 0-3, of own 4-7
+    return __builtin_amdgcn_perm(own, other, (lane & 1) ? 0x07060302u : 0x01000504u);
+}
+
 // Block shape: WM x NWN wavefronts, each owning MI x 2 tiles of 32 x 32 (MI * 32 rows x 64
 // columns).  WM = 2, MI = 4: 256-row blocks (256 x 128 with 4 wavefronts, 256 x 256 with 8);
 // WM = 1: 128-row (MI = 4) and 64-row (MI = 2) blocks for small M.
@@ -381,7 +390,6 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
     // load v (0/1) fetches lane (l32 % 16) + 16 * (2v + h) of chunk (l32 / 16).
     const int nt_base = (n0 + wn * 64) / kTileN;  // first 16-column tile of this wavefront
     uint32_t b_off[2], s_off[2];
-    const uint16_t *s_src[2];
 #pragma unroll
     for (int ni = 0; ni < 2; ++ni) {
         // SWIGLU: every 16-column tile holds 8 gate columns, then the 8 matching up columns; sub-tile 0
@@ -391,7 +399,6 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
         const int c = SWIGLU ? (l32 & 7) + 8 * ni : (l32 & 15);
         b_off[ni] = ((uint32_t)nt * (uint32_t)G * 64u + c + 16 * h) * 16u;  // + 512 for v = 1
         s_off[ni] = ((uint32_t)nt * (uint32_t)Gs * kTileN + c) * 2u;
-        s_src[ni] = S + (size_t)nt_base * Gs * kTileN + s_off[ni] / 2;
     }
     const int gs_mask = (Gs == 1) ? 0 : -1;
     const int s_step = (Gs == 1) ? 0 : kTileN * 2;  // bytes from a group's scales to the next one's
@@ -501,13 +508,34 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
 #pragma unroll
         for (int sp = 0; sp < 2; ++sp) bf[ni][sp] = codes_to_bf16x8(word_of(bw, std::integral_constant<int, 0>{}, ni, sp), dq);
 
-    auto rescale_tile = [&](int t) {  // tile t = 2 mi + ni
+    // The operands of the extension contraction (behind the main loop) ride in the ring like further stages: an
+    // extension stage is four groups, [group][row] 16 bytes of the rows' sums (not with RS, whose sums are in LDS),
+    // and beside it the four groups' scales of every wavefront's 64 columns, [group][column] fp16.  The last group
+    // of the main loop asks for the first four in place of further stages of A.
+    const int ng = g_end - g_begin;
+    const char *const s_base = s_ptr;
+    constexpr int kExtLoads = (RS ? 0 : APW) + 2;  // per wavefront and extension stage
+    const uint32_t ext_off = (uint32_t)min(m0 + (RS ? 0 : (wave % (BM / 64)) * 64) + lane, M - 1) * 16u;
+    auto ext_scales = [&](int slot) { return RS ? slot * kAStageBytes + wave * 512 : kAStages * kAStageBytes + (slot * NW + wave) * 512; };
+    auto request_ext = [&](int e, int slot) {  // groups past the last re-read it
+        if constexpr (!RS) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[t >> 1][t & 1][r] *= f[t & 1];
+            for (int p = 0; p < APW; ++p) {
+                const int i = wave + NW * p, g = g_begin + min(4 * e + i / (BM / 64), ng - 1);
+                load_to_lds_b128(uniform(reinterpret_cast<const char *>(aext + (size_t)g * M)), ext_off,
+                                 lds_base + slot * kAStageBytes + i * 1024);
+            }
+        }
+#pragma unroll
+        for (int v = 0; v < 2; ++v) {
+            const int g = min(4 * e + 2 * v + h, ng - 1) & gs_mask;
+            const uint32_t off = ((uint32_t)((lane >> 3) & 3) * (uint32_t)Gs + (uint32_t)g) * (kTileN * 2) + (lane & 7) * 4;
+            load_to_lds_b32(s_base, off, lds_base + ext_scales(slot) + v * 256);
+        }
     };
-    // one group; LAST: no further group, so nothing is asked for or read ahead past its end
-    auto group = [&](auto lastc) {
-        constexpr bool LAST = decltype(lastc)::value;
+    // one group; LAST: no further group; PEEK: ask for the words of a folded launch
+    auto group = [&](auto lastc, auto peekc) {
+        constexpr bool LAST = decltype(lastc)::value, PEEK = decltype(peekc)::value;
         unrolled<0, 4>([&](auto qc) {
             constexpr int q = decltype(qc)::value;
             constexpr bool ahead = !(LAST && q == 3);  // there is a next stage
@@ -548,12 +576,13 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
                     }
                     __builtin_amdgcn_sched_barrier(0);
                 });
-                if constexpr (mi == 0 && ahead) {
-                    // Loads complete in issue order; behind the next stage's there are at most those of the two stages
-                    // after it and, unless they are needed now, the next group's six.
-                    constexpr int stages_behind = LAST ? 2 - q : 2;
-                    constexpr int others = (!LAST && (q == 1 || q == 2)) ? 6 : (LAST && FOLD && q > 0) ? 1 : 0;
-                    wait_vector_loads<stages_behind * APW + others>();
+                if constexpr (mi == 0) {
+                    // Loads complete in issue order; behind the next stage's there are those of the two stages after
+                    // it (in the last group extension stages take the place of stages) and, unless they are needed now,
+                    // the next group's six.
+                    constexpr int a_behind = LAST && q > 0 ? (q == 1 ? 1 : 0) : 2;
+                    constexpr int others = (!LAST && (q == 1 || q == 2)) ? 6 + (PEEK ? 1 : 0) : 0;
+                    wait_vector_loads<a_behind * APW + (2 - a_behind) * kExtLoads + others>();
                     wait_lds_reads();
                     __builtin_amdgcn_s_barrier();
                     asm volatile("" : : : "memory");
@@ -575,8 +604,8 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
                             }
                         }
                     }
-                    // the early look at the words of a folded launch: a group of products ahead of its use
-                    if constexpr (FOLD && LAST && q == 0) prefill_fold_peek(pf, m0, min(BM, M - m0), lane, lds_base + kFoldPeekOffset + wave * 256);
+                    if constexpr (LAST) request_ext(q, q);
+                    if constexpr (PEEK && q == 0) prefill_fold_peek(pf, m0, min(BM, M - m0), lane, lds_base + kFoldPeekOffset + wave * 256);
                 }
                 if constexpr (ahead) {
                     if constexpr (RS && mi == 0) {
@@ -595,8 +624,7 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
             }
         });
     };
-    for (; g_now + 1 < g_end; ++g_now) {
-        group(std::false_type{});
+    auto next_group = [&]() {
 #pragma unroll
         for (int ni = 0; ni < 2; ++ni)
 #pragma unroll
@@ -604,120 +632,93 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
         a_ptr += 256;
         b_ptr += 1024;
         s_ptr += s_step;
+        ++g_now;
+    };
+    while (g_now + 1 + (FOLD ? 1 : 0) < g_end) {
+        group(std::false_type{}, std::false_type{});
+        next_group();
     }
-    group(std::true_type{});
-    if constexpr (RS) flush_rows(g_now - g_begin);
+    if constexpr (FOLD) {
+        // The rows of this block in the extension operand and in T are written during this launch.  The look at
+        // their words is asked for two groups before the main loop ends and answered one group later; the
+        // operands may be asked for from then on.
+        bool seen = false;
+        if (ng > 1) {
+            group(std::false_type{}, std::true_type{});
+            next_group();
+            seen = prefill_fold_seen(lds + kFoldPeekOffset + wave * 256, lane);
+        }
+        if (!seen) prefill_fold_wait(pf, m0, min(BM, M - m0), lane);
+    }
+    group(std::true_type{}, std::false_type{});
+    if constexpr (RS) {
+        flush_rows(g_now - g_begin);
+        __syncthreads();  // every wavefront's row sums are in LDS
+    }
     f[0] = sc[0];
     f[1] = sc[1];
 #pragma unroll
-    for (int t = 0; t < 2 * MI; ++t) rescale_tile(t);
-    wait_vector_loads<0>();  // the early look
+    for (int t = 0; t < 2 * MI; ++t) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[t >> 1][t & 1][r] *= f[t & 1];
+    }
 
     KILN_TL(1);
-    if constexpr (RS) __syncthreads();  // every wavefront's row sums are in LDS
-    if constexpr (FOLD) {
-        // the rows of this block in the extension operand and in T: written during this launch
-        // (the last group's waits have drained every load, the early look included)
-        if (!prefill_fold_seen(lds + kFoldPeekOffset + wave * 256, lane)) prefill_fold_wait(pf, m0, min(BM, M - m0), lane);
-        if (wave == 0) prefill_fold_done(pf, consumer, lane);
-    }
     // --- remove the 136 * sum(a) * scale surplus: extension contraction ------
-    // Step e covers groups g_begin + 2e (lanes 0-31) and g_begin + 2e + 1 (lanes
-    // 32-63), 8 slots each.  Operands come straight from global memory, loaded
-    // several steps ahead: every step issues its loads unconditionally (the group
-    // index is clamped, dead slots are zeroed), so the loads of later steps are
-    // in flight while the products of this one run.
-    {
-        int ext_row[MI];
+    // A product step covers two groups (lanes 0-31 and 32-63), 8 slots each; an extension stage is two steps.
+    // Stage e has landed and is visible when its turn comes (the last group's last barrier for stage 0).
+    for (int e = 0; 4 * e < ng; ++e) {
+        const int slot = e & 3;
+        bf16x8 ax[2][MI], bx[2][2];
 #pragma unroll
-        for (int mi = 0; mi < MI; ++mi) {
-            const int row = m0 + wm * MI * 32 + mi * 32 + l32;
-            ext_row[mi] = row < M ? row : M - 1;
-        }
-        struct ExtOps {
-            u32x4 a[MI];
-            uint32_t s[2];
-        };
-        auto ext_load = [&](int e, ExtOps &o) {  // writes the registers of o in place: no copies of pending loads
-            int g = g_begin + 2 * e + h;
-            g = g < g_end ? g : g_end - 1;
+        for (int u = 0; u < 2; ++u) {
+            const bool live = 4 * e + 2 * u + h < ng;
 #pragma unroll
-            for (int mi = 0; mi < MI; ++mi)
-                if constexpr (!RS) o.a[mi] = async_load_b128(aext + (size_t)g * M + ext_row[mi]);
-#pragma unroll
-            for (int ni = 0; ni < 2; ++ni) o.s[ni] = async_load_u16(s_src[ni] + (size_t)(g & gs_mask) * kTileN);
-        };
-        constexpr int kExtDepth = MI == 4 ? 5 : 6;
-        constexpr int kExtLoads = RS ? 2 : MI + 2;  // loads per step
-        auto ext_step = [&](int e, ExtOps &o) {
-            // this step's operands have landed when at most the later steps' loads are pending
-            __builtin_amdgcn_s_waitcnt(vmcnt_imm((kExtDepth - 1) * kExtLoads));
-#pragma unroll
-            for (int mi = 0; mi < MI; ++mi)
-                if constexpr (!RS) pin(o.a[mi]);
-            pin(o.s[0]);
-            pin(o.s[1]);
-            const bool live = g_begin + 2 * e + h < g_end;
-            if constexpr (RS) {
-                // c from LDS, split exactly into three bf16 terms: [hi, hi, mid, mid, lo, lo, 0, 0]
-                const int gl = live ? 2 * e + h : 0;  // group inside this block's K range
-#pragma unroll
-                for (int mi = 0; mi < MI; ++mi) {
-                    const float c = csum[gl * BM + wm * MI * 32 + mi * 32 + l32];
+            for (int mi = 0; mi < MI; ++mi) {
+                const int row = wm * MI * 32 + mi * 32 + l32;
+                if constexpr (RS) {
+                    // c from LDS, split exactly into three bf16 terms: [hi, hi, mid, mid, lo, lo, 0, 0]
+                    const float c = csum[(live ? 4 * e + 2 * u + h : 0) * BM + row];
                     const uint32_t hi = __builtin_bit_cast(uint32_t, c) & 0xFFFF0000u;
                     const float r1 = c - __builtin_bit_cast(float, hi);                     // exact
                     const uint32_t mid = __builtin_bit_cast(uint32_t, r1) & 0xFFFF0000u;
                     const float r2 = r1 - __builtin_bit_cast(float, mid);                   // exact, <= 8 significant bits
                     const uint32_t lo = __builtin_bit_cast(uint32_t, r2) & 0xFFFF0000u;
-                    o.a[mi] = live ? u32x4{(hi >> 16) | hi, (mid >> 16) | mid, (lo >> 16) | lo, 0u} : u32x4{0u, 0u, 0u, 0u};
+                    ax[u][mi] = __builtin_bit_cast(bf16x8, live ? u32x4{(hi >> 16) | hi, (mid >> 16) | mid, (lo >> 16) | lo, 0u} : u32x4{0u, 0u, 0u, 0u});
+                } else {
+                    ax[u][mi] = *reinterpret_cast<const bf16x8 *>(lds + slot * kAStageBytes + ((2 * u + h) * BM + row) * 16);
                 }
             }
-            bf16x8 bx[2];
 #pragma unroll
             for (int ni = 0; ni < 2; ++ni) {
-                const float sv = scale_value(o.s[ni]);
+                const int col = SWIGLU ? (l32 >> 3) * 16 + (l32 & 7) + 8 * ni : 32 * ni + l32;
+                const float sv = scale_value(*reinterpret_cast<const uint16_t *>(lds + ext_scales(slot) + (2 * u + h) * 128 + col * 2));
                 const uint32_t hi = __builtin_bit_cast(uint32_t, sv) & 0xFFFF0000u;
                 const float lo_f = sv - __builtin_bit_cast(float, hi);  // exact: f16 has 11 significant bits
                 const uint32_t pair = live ? ((hi >> 16) | (__builtin_bit_cast(uint32_t, lo_f) & 0xFFFF0000u)) : 0u;
-                const u32x4 r = {pair, pair, pair, 0u};
-                bx[ni] = __builtin_bit_cast(bf16x8, r);
-            }
-#pragma unroll
-            for (int mi = 0; mi < MI; ++mi) {
-                const bf16x8 ax = __builtin_bit_cast(bf16x8, o.a[mi]);
-#pragma unroll
-                for (int ni = 0; ni < 2; ++ni)
-                    acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ax, bx[ni], acc[mi][ni], 0, 0, 0);
-            }
-        };
-        // kExtDepth register sets rotate by position, never by copying (a copy of
-        // a register whose load is still in flight would wait for it); the step
-        // count is rounded up to a multiple of the depth, the extra steps multiply
-        // by zero.  The main loop's weight and fragment registers are dead here,
-        // which is what pays for the depth.
-        const int n_ext = (g_end - g_begin + 1) / 2;
-        ExtOps o[kExtDepth];
-#pragma unroll
-        for (int d = 0; d < kExtDepth; ++d) ext_load(d, o[d]);
-        for (int e = 0; e < n_ext; e += kExtDepth) {
-#pragma unroll
-            for (int d = 0; d < kExtDepth; ++d) {
-                ext_step(e + d, o[d]);
-                ext_load(e + d + kExtDepth, o[d]);
-                __builtin_amdgcn_sched_barrier(0);
+                bx[u][ni] = __builtin_bit_cast(bf16x8, u32x4{pair, pair, pair, 0u});
             }
         }
-        // the look-ahead loads of steps past the end are still in flight; nothing may reuse
-        // their registers before they land
-        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-#pragma unroll
-        for (int d = 0; d < kExtDepth; ++d) {
-#pragma unroll
-            for (int mi = 0; mi < MI; ++mi)
-                if constexpr (!RS) pin(o[d].a[mi]);
-            pin(o[d].s[0]);
-            pin(o[d].s[1]);
+        if (4 * (e + 1) < ng) {
+            // the next stage: behind it there are those of the two stages after it, where they were asked for
+            if (e == 0 || 4 * (e + 3) < ng) wait_vector_loads<2 * kExtLoads>();
+            else wait_vector_loads<0>();
+            wait_lds_reads();
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" : : : "memory");
+            if (4 * (e + 4) < ng) request_ext(e + 4, slot);
         }
+#pragma unroll
+        for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+            for (int ni = 0; ni < 2; ++ni)
+#pragma unroll
+                for (int u = 0; u < 2; ++u)
+                    acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ax[u][mi], bx[u][ni], acc[mi][ni], 0, 0, 0);
+    }
+    wait_vector_loads<0>();  // stages asked for past the end still write to LDS, which the store reuses behind its barrier
+    if constexpr (FOLD) {
+        if (wave == 0) prefill_fold_done(pf, consumer, lane);
     }
 
     // --- fused LoRA epilogue: y += T * B_cat^T with T = scaled x * A_cat^T from the
@@ -762,51 +763,52 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
     KILN_TL(2);
     if (sliced && KS > 1) {
         // Combine the K slices of this tile.  Every block writes its f32 partial
-        // tile with device-scope accesses (element (mi, ni, r) of thread t at
-        // ((mi*2+ni)*16 + r) * NT + t: coalesced both ways); the last block to
+        // tile with device-scope accesses, 16 bytes each (registers 4 i ... 4 i + 3 of tile (mi, ni) of thread t at
+        // 16-byte unit ((mi*2+ni)*4 + i) * NT + t: coalesced both ways); the last block to
         // arrive reads all KS partial tiles back and adds them in slice order,
         // so the result does not depend on arrival order.
         __shared__ int s_last;
         const int tile = (nb - nb_full) * m_blocks + mb;
-        float *mine = partial + ((size_t)tile * KS + ks) * (BM * BN);
+        float *mine = partial + ((size_t)tile * KS + ks) * (BM * BN) + tid * 4;
 #pragma unroll
         for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
             for (int ni = 0; ni < 2; ++ni)
 #pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    __hip_atomic_store(mine + ((mi * 2 + ni) * 16 + r) * NT + tid, acc[mi][ni][r],
-                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                for (int i = 0; i < 4; ++i) {
+                    const f32x4 v = {acc[mi][ni][4 * i], acc[mi][ni][4 * i + 1], acc[mi][ni][4 * i + 2], acc[mi][ni][4 * i + 3]};
+                    store_b128_device_scope(mine + ((mi * 2 + ni) * 4 + i) * NT * 4, __builtin_bit_cast(u32x4, v));
+                }
         // each wavefront waits until its own stores have been acknowledged (a barrier alone
         // orders nothing outside the workgroup); after the barrier the arrival is counted
-        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+        wait_vector_loads<0>();
         __syncthreads();
         KILN_TL(3);
         if (tid == 0)
             s_last = (__hip_atomic_fetch_add(counters + tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == KS - 1);
         __syncthreads();
         if (!s_last) return;
-        // slice 0 lands straight in the accumulators; the others go through a
-        // 64-register staging array, MI / 2 batches per slice
-        const float *all = partial + (size_t)tile * KS * (BM * BN) + tid;
-#pragma unroll
-        for (int mi = 0; mi < MI; ++mi)
-#pragma unroll
-            for (int ni = 0; ni < 2; ++ni)
-#pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    acc[mi][ni][r] = __hip_atomic_load(all + ((mi * 2 + ni) * 16 + r) * NT, __ATOMIC_RELAXED,
-                                                       __HIP_MEMORY_SCOPE_AGENT);
-        for (int s2 = 1; s2 < KS; ++s2) {
+        // 16 loads (64 registers) a batch, MI / 2 batches per slice
+        const float *all = partial + (size_t)tile * KS * (BM * BN) + tid * 4;
+        for (int s2 = 0; s2 < KS; ++s2) {
             const float *src = all + (size_t)s2 * (BM * BN);
 #pragma unroll
             for (int half = 0; half < MI / 2; ++half) {
-                float t[64];
+                u32x4 t[16];
 #pragma unroll
-                for (int i = 0; i < 64; ++i)
-                    t[i] = __hip_atomic_load(src + (half * 64 + i) * NT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                for (int i = 0; i < 16; ++i) load_b128_device_scope(t[i], src + (half * 16 + i) * NT * 4);
+                wait_vector_loads<0>();
 #pragma unroll
-                for (int i = 0; i < 64; ++i) acc[half * 2 + i / 32][(i / 16) & 1][i & 15] += t[i];
+                for (int i = 0; i < 16; ++i) {
+                    pin_loaded(t[i]);
+                    const f32x4 v = __builtin_bit_cast(f32x4, t[i]);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int at = 4 * (i & 3) + r;
+                        f32x16 &a = acc[half * 2 + i / 8][(i / 4) & 1];
+                        a[at] = s2 == 0 ? v[r] : a[at] + v[r];
+                    }
+                }
             }
         }
         if (tid == 0) __hip_atomic_store(counters + tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -817,14 +819,23 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
         // acc[mi][0] holds gate, acc[mi][1] the matching up columns: h = gate / (1 + exp(-gate)) * up.
         // The wavefront's tile becomes (MI * 32) x 32: rows of 64 bytes, 4 lanes per row.
         uint16_t *tile = reinterpret_cast<uint16_t *>(lds + wave * (MI * 32 * 32 * 2));  // [MI * 32][32] bf16
+        uint32_t *dst[2];  // of row pairs 0 and 2 of every four
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int row = 4 * h + 2 * i + (lane & 1);
+            dst[i] = reinterpret_cast<uint32_t *>(tile + row * 32 + ((((l32 >> 3) ^ (row & 3)) << 3) | (l32 & 6)));
+        }
 #pragma unroll
         for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const float gate = acc[mi][0][r], up = acc[mi][1][r];
-                const float hval = gate * __builtin_amdgcn_rcpf(1.f + __expf(-gate)) * up;
-                const int row = mi * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
-                tile[row * 32 + ((((l32 >> 3) ^ (row & 3)) << 3) | (l32 & 7))] = f32_to_bf16_bits(hval);
+            for (int r = 0; r < 16; r += 2) {
+                float hval[2];
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    const float gate = acc[mi][0][r + i], up = acc[mi][1][r + i];
+                    hval[i] = gate * __builtin_amdgcn_rcpf(1.f + __expf(-gate)) * up;
+                }
+                dst[(r >> 1) & 1][(mi * 32 + 8 * (r >> 2)) * 16] = neighbours_of_a_row(hval[0], hval[1], lane);
             }
         __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
 #pragma unroll
@@ -837,17 +848,22 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
         }
     } else {
         uint16_t *tile = reinterpret_cast<uint16_t *>(lds + wave * (MI * 32 * 64 * 2));  // [MI * 32][64] bf16
+        uint32_t *dst[2][2];  // of sub-tile ni, row pairs 0 and 2 of every four
+#pragma unroll
+        for (int ni = 0; ni < 2; ++ni)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                // 16-byte unit index XOR (row & 7): keeps the row reads below conflict free
+                const int row = 4 * h + 2 * i + (lane & 1), col = ni * 32 + l32;
+                dst[ni][i] = reinterpret_cast<uint32_t *>(tile + row * 64 + ((((col >> 3) ^ (row & 7)) << 3) | (col & 6)));
+            }
 #pragma unroll
         for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
             for (int ni = 0; ni < 2; ++ni)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int row = mi * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
-                    // 16-byte unit index XOR (row & 7): keeps the row reads below conflict free
-                    const int col = ni * 32 + l32;
-                    tile[row * 64 + ((((col >> 3) ^ (row & 7)) << 3) | (col & 7))] = f32_to_bf16_bits(acc[mi][ni][r]);
-                }
+                for (int r = 0; r < 16; r += 2)
+                    dst[ni][(r >> 1) & 1][(mi * 32 + 8 * (r >> 2)) * 32] = neighbours_of_a_row(acc[mi][ni][r], acc[mi][ni][r + 1], lane);
         // same wavefront wrote and reads: only the LDS counter needs to drain
         __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
 #pragma unroll
@@ -1067,7 +1083,7 @@ template <int NWN, int WM, int MI, bool SWIGLU, bool RS, bool FOLD = false>
 hipError_t launch_shape_as(const PrefillArgs &a, int grid, int m_blocks, int RP, int KS, int GSb, int max_groups,
                            hipStream_t stream, const PrefillFold &pf = PrefillFold{}) {
     constexpr int BM = WM * MI * 32, NW = WM * NWN;
-    constexpr int kRing = kAStages * BM * 64;       // the A ring
+    constexpr int kRing = kAStages * BM * 64 + (RS ? 0 : kAStages * NW * 512);  // the A ring, the extension's scales behind it
     constexpr int kStore = NW * MI * 32 * 64 * 2;   // the store's per-wavefront transposes (reuses the ring)
     // RS: the row sums sit behind the ring and are dead by the time the store reuses the space
     constexpr int kLdsMax = RS ? (kRing + kMaxRowSumBytes > kStore ? kRing + kMaxRowSumBytes : kStore)
