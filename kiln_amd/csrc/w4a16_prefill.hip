@@ -666,55 +666,79 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
     KILN_TL(1);
     // --- remove the 136 * sum(a) * scale surplus: extension contraction ------
     // A product step covers two groups (lanes 0-31 and 32-63), 8 slots each; an extension stage is two steps.
-    // Stage e has landed and is visible when its turn comes (the last group's last barrier for stage 0).
-    for (int e = 0; 4 * e < ng; ++e) {
+    // While one step is multiplied the other's operands are read from LDS: a stage's second step behind its first
+    // one's products, the next stage's first step behind the barrier between the two steps -- there the next
+    // stage has landed, and every wavefront holds what it needs of this one, whose slot takes the fourth ahead.
+    struct ExtStep {
+        bf16x8 a[RS ? 1 : MI];
+        float c[RS ? MI : 1];
+        uint32_t s[2];
+    };
+    auto ext_read = [&](int e, int u, ExtStep &x) {
         const int slot = e & 3;
-        bf16x8 ax[2][MI], bx[2][2];
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const bool live = 4 * e + 2 * u + h < ng;
-#pragma unroll
-            for (int mi = 0; mi < MI; ++mi) {
-                const int row = wm * MI * 32 + mi * 32 + l32;
-                if constexpr (RS) {
-                    // c from LDS, split exactly into three bf16 terms: [hi, hi, mid, mid, lo, lo, 0, 0]
-                    const float c = csum[(live ? 4 * e + 2 * u + h : 0) * BM + row];
-                    const uint32_t hi = __builtin_bit_cast(uint32_t, c) & 0xFFFF0000u;
-                    const float r1 = c - __builtin_bit_cast(float, hi);                     // exact
-                    const uint32_t mid = __builtin_bit_cast(uint32_t, r1) & 0xFFFF0000u;
-                    const float r2 = r1 - __builtin_bit_cast(float, mid);                   // exact, <= 8 significant bits
-                    const uint32_t lo = __builtin_bit_cast(uint32_t, r2) & 0xFFFF0000u;
-                    ax[u][mi] = __builtin_bit_cast(bf16x8, live ? u32x4{(hi >> 16) | hi, (mid >> 16) | mid, (lo >> 16) | lo, 0u} : u32x4{0u, 0u, 0u, 0u});
-                } else {
-                    ax[u][mi] = *reinterpret_cast<const bf16x8 *>(lds + slot * kAStageBytes + ((2 * u + h) * BM + row) * 16);
-                }
-            }
-#pragma unroll
-            for (int ni = 0; ni < 2; ++ni) {
-                const int col = SWIGLU ? (l32 >> 3) * 16 + (l32 & 7) + 8 * ni : 32 * ni + l32;
-                const float sv = scale_value(*reinterpret_cast<const uint16_t *>(lds + ext_scales(slot) + (2 * u + h) * 128 + col * 2));
-                const uint32_t hi = __builtin_bit_cast(uint32_t, sv) & 0xFFFF0000u;
-                const float lo_f = sv - __builtin_bit_cast(float, hi);  // exact: f16 has 11 significant bits
-                const uint32_t pair = live ? ((hi >> 16) | (__builtin_bit_cast(uint32_t, lo_f) & 0xFFFF0000u)) : 0u;
-                bx[u][ni] = __builtin_bit_cast(bf16x8, u32x4{pair, pair, pair, 0u});
-            }
-        }
-        if (4 * (e + 1) < ng) {
-            // the next stage: behind it there are those of the two stages after it, where they were asked for
-            if (e == 0 || 4 * (e + 3) < ng) wait_vector_loads<2 * kExtLoads>();
-            else wait_vector_loads<0>();
-            wait_lds_reads();
-            __builtin_amdgcn_s_barrier();
-            asm volatile("" : : : "memory");
-            if (4 * (e + 4) < ng) request_ext(e + 4, slot);
+        for (int mi = 0; mi < MI; ++mi) {
+            const int row = wm * MI * 32 + mi * 32 + l32;
+            if constexpr (RS) x.c[mi] = csum[min(4 * e + 2 * u + h, ng - 1) * BM + row];
+            else x.a[mi] = *reinterpret_cast<const bf16x8 *>(lds + slot * kAStageBytes + ((2 * u + h) * BM + row) * 16);
         }
 #pragma unroll
-        for (int mi = 0; mi < MI; ++mi)
+        for (int ni = 0; ni < 2; ++ni) {
+            const int col = SWIGLU ? (l32 >> 3) * 16 + (l32 & 7) + 8 * ni : 32 * ni + l32;
+            x.s[ni] = *reinterpret_cast<const uint16_t *>(lds + ext_scales(slot) + (2 * u + h) * 128 + col * 2);
+        }
+    };
+    auto ext_multiply = [&](int e, int u, const ExtStep &x) {
+        const bool live = 4 * e + 2 * u + h < ng;
+        bf16x8 bx[2];
 #pragma unroll
-            for (int ni = 0; ni < 2; ++ni)
+        for (int ni = 0; ni < 2; ++ni) {
+            const float sv = scale_value(x.s[ni]);
+            const uint32_t hi = __builtin_bit_cast(uint32_t, sv) & 0xFFFF0000u;
+            const float lo_f = sv - __builtin_bit_cast(float, hi);  // exact: f16 has 11 significant bits
+            const uint32_t pair = live ? ((hi >> 16) | (__builtin_bit_cast(uint32_t, lo_f) & 0xFFFF0000u)) : 0u;
+            bx[ni] = __builtin_bit_cast(bf16x8, u32x4{pair, pair, pair, 0u});
+        }
 #pragma unroll
-                for (int u = 0; u < 2; ++u)
-                    acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ax[u][mi], bx[u][ni], acc[mi][ni], 0, 0, 0);
+        for (int mi = 0; mi < MI; ++mi) {
+            bf16x8 ax;
+            if constexpr (RS) {
+                // c split exactly into three bf16 terms: [hi, hi, mid, mid, lo, lo, 0, 0]
+                const float c = x.c[mi];
+                const uint32_t hi = __builtin_bit_cast(uint32_t, c) & 0xFFFF0000u;
+                const float r1 = c - __builtin_bit_cast(float, hi);                     // exact
+                const uint32_t mid = __builtin_bit_cast(uint32_t, r1) & 0xFFFF0000u;
+                const float r2 = r1 - __builtin_bit_cast(float, mid);                   // exact, <= 8 significant bits
+                const uint32_t lo = __builtin_bit_cast(uint32_t, r2) & 0xFFFF0000u;
+                ax = __builtin_bit_cast(bf16x8, live ? u32x4{(hi >> 16) | hi, (mid >> 16) | mid, (lo >> 16) | lo, 0u} : u32x4{0u, 0u, 0u, 0u});
+            } else {
+                ax = x.a[mi];
+            }
+#pragma unroll
+            for (int ni = 0; ni < 2; ++ni) acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ax, bx[ni], acc[mi][ni], 0, 0, 0);
+        }
+    };
+    {
+        ExtStep x0, x1;
+        ext_read(0, 0, x0);  // visible since the last group's last barrier
+        for (int e = 0; 4 * e < ng; ++e) {
+            ext_read(e, 1, x1);
+            __builtin_amdgcn_sched_barrier(0);
+            ext_multiply(e, 0, x0);
+            __builtin_amdgcn_sched_barrier(0);
+            if (4 * (e + 1) < ng) {
+                // behind the next stage there are those of the two stages after it, where they were asked for
+                if (e == 0 || 4 * (e + 3) < ng) wait_vector_loads<2 * kExtLoads>();
+                else wait_vector_loads<0>();
+                wait_lds_reads();
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" : : : "memory");
+                if (4 * (e + 4) < ng) request_ext(e + 4, e & 3);
+                ext_read(e + 1, 0, x0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            ext_multiply(e, 1, x1);
+        }
     }
     wait_vector_loads<0>();  // stages asked for past the end still write to LDS, which the store reuses behind its barrier
     if constexpr (FOLD) {
@@ -788,9 +812,14 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
             s_last = (__hip_atomic_fetch_add(counters + tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == KS - 1);
         __syncthreads();
         if (!s_last) return;
-        // 16 loads (64 registers) a batch, MI / 2 batches per slice
+        // 16 loads (64 registers) a batch, MI / 2 batches per slice, each batch a round trip.  The block's own part is
+        // still in its registers: as slice 0 or 1 the others are added to it as they come (a + b is b + a, so the
+        // sum is the one in slice order); further on the sum before it would need registers of its own, and
+        // it is read back like the others.
         const float *all = partial + (size_t)tile * KS * (BM * BN) + tid * 4;
         for (int s2 = 0; s2 < KS; ++s2) {
+            if (ks < 2 && s2 == ks) continue;
+            const bool first = ks >= 2 && s2 == 0;
             const float *src = all + (size_t)s2 * (BM * BN);
 #pragma unroll
             for (int half = 0; half < MI / 2; ++half) {
@@ -806,7 +835,7 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
                     for (int r = 0; r < 4; ++r) {
                         const int at = 4 * (i & 3) + r;
                         f32x16 &a = acc[half * 2 + i / 8][(i / 4) & 1];
-                        a[at] = s2 == 0 ? v[r] : a[at] + v[r];
+                        a[at] = first ? v[r] : a[at] + v[r];
                     }
                 }
             }
