@@ -897,11 +897,24 @@ size_t workspace_bytes_upto(int m, int n, int k, int cus, int thread_k, int thre
     return most;
 }
 
+// The row sums of an MLP's intermediate H, written by the launch that writes H and read by the one that reads it
+// (matrix-core kernel on both sides, mlp_passes_row_sums)
+struct MlpSums {
+    void *write = nullptr;
+    void *read = nullptr;
+};
+bool mlp_passes_row_sums(int m, int hidden, int n_out, int n_down, int cus) {
+    const auto gate_up = plan_call(m, 2 * n_out, hidden, cus, -1, -1, 0), down = plan_call(m, n_down, n_out, cus, -1, -1, 0);
+    return gate_up->gp.prefill && prefill_forms_next_sums(gate_up->gp.pf) && down->gp.prefill &&
+           prefill_reads_row_sums(m, n_down, n_out, down->gp.pf);
+}
+
 // The GEMM behind every entry point: small-M or matrix-core path by row count, with the
 // optional low-rank term.
 kiln_marlin_status_t gemm_any(const void *A, const void *B, void *C, const void *s, int prob_m, int prob_n,
                               int prob_k, void *workspace, int groupsize, int dev, void *stream, int thread_k,
-                              int thread_n, int sms, const LoraSpec *lora, bool swiglu = false) {
+                              int thread_n, int sms, const LoraSpec *lora, bool swiglu = false,
+                              const MlpSums &sums = MlpSums{}) {
     if (prob_m < 0 || prob_n < 0 || prob_k < 0) return KILN_W4A16_ERR_PROB_SHAPE;
     if (!shape_ok(prob_n, prob_k, groupsize)) return KILN_W4A16_ERR_PROB_SHAPE;
     if (thread_k > 0 && thread_k % 128 != 0) return KILN_W4A16_ERR_PROB_SHAPE;
@@ -945,6 +958,11 @@ kiln_marlin_status_t gemm_any(const void *A, const void *B, void *C, const void 
             pa.lora_words = reinterpret_cast<unsigned *>(ws + kFoldFlagOffset);
         }
         pa.swiglu = swiglu;
+        pa.next_aext = sums.write;
+        if (sums.read) {
+            pa.aext = sums.read;
+            pa.aext_ready = true;
+        }
         pa.cus = cus;
         pa.KS = gp.pf.ks;
         pa.bn = gp.pf.bn;
@@ -1374,7 +1392,7 @@ kiln_marlin_status_t kiln_w4a16_gemm_swiglu_lora(const void *A, const void *B, v
 }
 
 // ---- the MLP of a layer as one call -------------------------------------------------------------------
-// workspace: [what the two GEMMs need, the larger of the two] | H = bf16 [m, n_out]
+// workspace: [what the two GEMMs need, the larger of the two] | H = bf16 [m, n_out] | H's row sums for the down GEMM
 static size_t mlp_h_offset(int m, int k1, int n_out, int n2) {
     const size_t a = kiln_w4a16_swiglu_workspace_bytes(m, n_out, k1), b = kiln_w4a16_workspace_bytes(m, n2, n_out);
     return ((a > b ? a : b) + 255) & ~(size_t)255;
@@ -1383,7 +1401,7 @@ static size_t mlp_h_offset(int m, int k1, int n_out, int n2) {
 size_t kiln_w4a16_mlp_workspace_bytes(int prob_m, int hidden, int n_out, int n_down) {
     if (prob_m < 1) prob_m = 1;
     if (hidden <= 0 || n_out <= 0 || n_down <= 0 || n_out > INT32_MAX / 2) return kZeroedBytes;
-    return mlp_h_offset(prob_m, hidden, n_out, n_down) + (size_t)prob_m * n_out * 2;
+    return mlp_h_offset(prob_m, hidden, n_out, n_down) + (size_t)prob_m * n_out * 2 + prefill_aext_bytes(prob_m, n_out);
 }
 
 kiln_marlin_status_t kiln_w4a16_mlp(const void *x, const void *b_gate_up, const void *s_gate_up, const void *b_down,
@@ -1398,10 +1416,16 @@ kiln_marlin_status_t kiln_w4a16_mlp(const void *x, const void *b_gate_up, const 
     // Two launches with H in between.  (One launch for both -- down blocks resident from the start, their weights
     // in registers, waiting for their columns of H -- measured level with the two, 15.2 us at 16 rows: every hop
     // of the hand-over inside a launch crosses the dies' memory system, about a microsecond each.)
+    // Where both are the matrix-core kernel's, the first one's blocks form the row sums of H that the second one needs
+    // as they store H, whose columns they hold in whole groups: the second launch neither reads H for them beforehand
+    // (8192 rows 973 -> 953 us) nor gives block slots to blocks that do (2048 rows 282 -> 276).
+    MlpSums write, read;
+    if (mlp_passes_row_sums(prob_m, hidden, n_out, n_down, compute_units(dev)))
+        write.write = read.read = reinterpret_cast<char *>(h) + (size_t)prob_m * n_out * 2;
     const kiln_marlin_status_t st = gemm_any(x, b_gate_up, h, s_gate_up, prob_m, 2 * n_out, hidden, workspace, groupsize, dev,
-                                             stream, -1, -1, -1, nullptr, true);
+                                             stream, -1, -1, -1, nullptr, true, write);
     if (st != KILN_W4A16_OK) return st;
-    return gemm_any(h, b_down, y, s_down, prob_m, n_down, n_out, workspace, groupsize, dev, stream, -1, -1, -1, nullptr);
+    return gemm_any(h, b_down, y, s_down, prob_m, n_down, n_out, workspace, groupsize, dev, stream, -1, -1, -1, nullptr, false, read);
 }
 
 size_t kiln_w4a16_swiglu_workspace_bytes(int prob_m, int n_out, int prob_k) {

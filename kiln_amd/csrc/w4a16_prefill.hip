@@ -285,7 +285,7 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
     const uint16_t *__restrict__ A, const u32x4 *__restrict__ B, const uint16_t *__restrict__ S,
     uint16_t *__restrict__ C, const u32x4 *__restrict__ aext, int M, int N, int K, int Gs, int m_blocks,
     const uint16_t *__restrict__ lora_t, const uint16_t *__restrict__ lora_b, int r_total, int RP, int nb_full,
-    int KS, int GSb, float *partial, int *counters, int die_rows, PrefillFold pf) {
+    int KS, int GSb, float *partial, int *counters, int die_rows, u32x4 *next_aext, PrefillFold pf) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];  // the A ring; reused by the store
     static_assert(!FOLD || WM * NWN == 4, "the projection's blocks have four wavefronts");
     if constexpr (FOLD) {
@@ -848,6 +848,7 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
         // acc[mi][0] holds gate, acc[mi][1] the matching up columns: h = gate / (1 + exp(-gate)) * up.
         // The wavefront's tile becomes (MI * 32) x 32: rows of 64 bytes, 4 lanes per row.
         uint16_t *tile = reinterpret_cast<uint16_t *>(lds + wave * (MI * 32 * 32 * 2));  // [MI * 32][32] bf16
+        [[maybe_unused]] float *unit_sums = reinterpret_cast<float *>(lds + NW * (MI * 32 * 32 * 2));  // [BM][16 units of 8 columns]
         uint32_t *dst[2];  // of row pairs 0 and 2 of every four
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
@@ -874,6 +875,29 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
             const int grow = m0 + wm * MI * 32 + row;
             if (grow < M)
                 *reinterpret_cast<u32x4 *>(C + (size_t)grow * (N / 2) + (n0 + wn * 64) / 2 + unit * 8) = v;
+            if constexpr (WM == 1 && NWN == 4) {
+                if (next_aext) unit_sums[row * 16 + wn * 4 + unit] = sum_bf16x8(v);
+            }
+        }
+        if constexpr (WM == 1 && NWN == 4) {
+            // The rows' sums for a GEMM over this output (an MLP's down projection): the block's 128 output columns are
+            // one group of that GEMM's K, so its rows' sums are formed here, from the stored bf16 values and in the pre-pass
+            // kernel's order of additions (bit-equal), and no pass over H is needed for them: 16 bytes per 256 of H
+            // written here, from values already in registers (2560 -> 2 x 9216 -> 2560: 8192 rows 973 -> 953 us, the pass read
+            // 151 MB in a launch of its own; 2048 rows 282 -> 276, blocks of the down projection's own launch read them).
+            if (next_aext) {
+                __syncthreads();
+                if (tid < BM && m0 + tid < M) {
+                    float u[16];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) *reinterpret_cast<f32x4 *>(u + 4 * i) = *reinterpret_cast<const f32x4 *>(unit_sums + tid * 16 + 4 * i);
+#pragma unroll
+                    for (int off = 8; off >= 1; off >>= 1)
+#pragma unroll
+                        for (int i = 0; i < off; ++i) u[i] += u[i + off];
+                    next_aext[(size_t)nb * M + m0 + tid] = extension_operand(u[0]);
+                }
+            }
         }
     } else {
         uint16_t *tile = reinterpret_cast<uint16_t *>(lds + wave * (MI * 32 * 64 * 2));  // [MI * 32][64] bf16
@@ -1132,7 +1156,7 @@ hipError_t launch_shape_as(const PrefillArgs &a, int grid, int m_blocks, int RP,
         (const uint16_t *)a.A, (const u32x4 *)a.B, (const uint16_t *)a.S, (uint16_t *)a.C, (const u32x4 *)a.aext,
         a.M, a.N, a.K, a.Gs, m_blocks, (const uint16_t *)a.lora_t, (const uint16_t *)a.lora_b, a.r_total, RP,
         a.nb_full, KS, GSb, a.partial, a.counters,
-        prefill_die_rows(m_blocks, a.nb_full, (a.N / (NWN * 64) - a.nb_full) * KS, KS), pf);
+        prefill_die_rows(m_blocks, a.nb_full, (a.N / (NWN * 64) - a.nb_full) * KS, KS), (u32x4 *)a.next_aext, pf);
     return hipGetLastError();
 }
 
@@ -1260,6 +1284,9 @@ int prefill_rowsum_producers(int M, int N, int K, const PrefillPlan &p, int cus)
     return producers < 128 ? producers : 128;
 }
 
+bool prefill_forms_next_sums(const PrefillPlan &p) { return p.bn == 256 && (p.bm == 64 || p.bm == 128); }
+bool prefill_reads_row_sums(int M, int N, int K, const PrefillPlan &p) { return !blocks_sum_their_rows(M, N, K, p); }
+
 hipError_t launch_prefill(const PrefillArgs &a, hipStream_t stream) {
     const int G = a.K / kGroupK;
     if (a.bm != 64 && a.bm != 128 && a.bm != 256) return hipErrorInvalidValue;
@@ -1274,9 +1301,10 @@ hipError_t launch_prefill(const PrefillArgs &a, hipStream_t stream) {
     hipError_t err = hipSuccess;
     // with adapters the projection's launch forms the row sums on its way over x
     const bool sums_with_projection = !rs && a.r_total > 0;
-    const int inside = a.r_total == 0 && a.lora_words ? prefill_rowsum_producers(a.M, a.N, a.K, shape, a.cus) : 0;
+    if (a.next_aext && !prefill_forms_next_sums(shape)) return hipErrorInvalidValue;
+    const int inside = a.r_total == 0 && a.lora_words && !a.aext_ready ? prefill_rowsum_producers(a.M, a.N, a.K, shape, a.cus) : 0;
     const int sum_producers = inside > 0 ? inside : 0;
-    if (!rs && !sums_with_projection && sum_producers == 0) {
+    if (!rs && !sums_with_projection && sum_producers == 0 && !a.aext_ready) {
         const int items = a.M * G;
         w4a16_prefill_rowsum_kernel<<<(items + 15) / 16, 256, 0, stream>>>((const uint16_t *)a.A, (u32x4 *)a.aext,
                                                                           a.M, a.K);

@@ -108,3 +108,42 @@ def test_mlp_workspace_bytes_and_argument_checks():
     assert L.kiln_w4a16_mlp(p, p, p, p, p, p, 4, HIDDEN, INTER, HIDDEN, p, 64, 0, stream) == _lib.ERR_PROB_SHAPE
     assert L.kiln_w4a16_mlp(p, p, p, p, p, None, 4, HIDDEN, INTER, HIDDEN, p, 128, 0, stream) == _lib.ERR_ARGUMENT
     assert L.kiln_w4a16_mlp(p, p, p, p, p, p, 0, HIDDEN, INTER, HIDDEN, p, 128, 0, stream) == _lib.OK
+
+
+@pytest.mark.parametrize("m,hidden,inter,n_down,g,passed", [
+    (777, HIDDEN, INTER, HIDDEN, 128, True),     # ragged rows, K slices on both sides
+    (2049, HIDDEN, INTER, HIDDEN, 128, True),    # a last row block of one row, behind whole rounds
+    (1500, 1024, 6144, 4352, -1, True),
+    (600, 2560, 4864, 6144, 128, None),          # either block height
+    (130, HIDDEN, INTER, HIDDEN, 128, False),    # another kernel, or blocks that sum their rows themselves
+])
+def test_mlp_row_sums_formed_with_h_equal_those_read_from_h(m, hidden, inter, n_down, g, passed):
+    """Where the launch that writes H also writes the row sums the down projection needs, they are added in the order of
+    the pass over H that they replace: the call equals the two entry points in every bit.  The activations have a mean, so that the term the
+    sums remove is far larger than the result; the workspace holds garbage behind its zeroed prefix, and the prefix is zero again."""
+    L = _lib.load()
+    gen = torch.Generator(device="cuda").manual_seed(m + inter)
+
+    def weight(k, n):
+        words = torch.randint(-2**31, 2**31, (k // 16, 2 * n), dtype=torch.int64, device="cuda", generator=gen).to(torch.int32)
+        scales = (torch.rand(1 if g == -1 else k // g, n, device="cuda", generator=gen) * 0.01 + 0.002).half()
+        return words, scales
+
+    (b_gu, s_gu), (bd, sd) = weight(hidden, 2 * inter), weight(inter, n_down)
+    x = (torch.randn(m, hidden, device="cuda", generator=gen) * 0.5 + 0.5).to(torch.bfloat16)
+    z, size = L.kiln_w4a16_workspace_zeroed_bytes(), L.kiln_w4a16_mlp_workspace_bytes(m, hidden, inter, n_down)
+    sums = m * (inter // 128) * 16
+    ws = torch.full((size + 256,), 0xA5, dtype=torch.uint8, device="cuda")
+    ws[:z].zero_()
+    y = torch.empty(m, n_down, dtype=torch.bfloat16, device="cuda")
+    for _ in range(3):
+        rc = L.kiln_w4a16_mlp(x.data_ptr(), b_gu.data_ptr(), s_gu.data_ptr(), bd.data_ptr(), sd.data_ptr(), y.data_ptr(), m, hidden, inter,
+                              n_down, ws.data_ptr(), g, torch.cuda.current_device(), torch.cuda.current_stream().cuda_stream)
+        assert rc == _lib.OK, _lib.status_string(rc)
+    torch.cuda.synchronize()
+    if passed is not None:
+        assert bool((ws[size - sums:size] != 0xA5).any()) == passed
+    assert int(ws[:z].count_nonzero()) == 0 and bool((ws[size:] == 0xA5).all())
+    h = marlin_gemm.marlin_w4a16_gemm_swiglu(x, b_gu, s_gu, g)
+    want = marlin_gemm.marlin_w4a16_gemm(h, bd, sd, g)
+    assert bool(torch.isfinite(want).all()) and torch.equal(y.view(torch.int16), want.view(torch.int16))
