@@ -8,7 +8,8 @@ namespace kiln {
 __device__ __forceinline__ u32x4 extension_operand(float sum) {
     const float c = -kCodeBias * sum;
     const uint32_t hi = __builtin_bit_cast(uint32_t, c) & 0xFFFF0000u;
-    const float r1 = c - __builtin_bit_cast(float, hi);                     // exact
+    // the rest of the product, not of its rounded value (and the same everywhere, whatever the compiler contracts)
+    const float r1 = fmaf(-kCodeBias, sum, -__builtin_bit_cast(float, hi));
     const uint32_t mid = __builtin_bit_cast(uint32_t, r1) & 0xFFFF0000u;
     const float r2 = r1 - __builtin_bit_cast(float, mid);                   // exact, <= 8 significant bits
     const uint32_t lo = __builtin_bit_cast(uint32_t, r2) & 0xFFFF0000u;

@@ -901,10 +901,12 @@ size_t workspace_bytes_upto(int m, int n, int k, int cus, int thread_k, int thre
 // (matrix-core kernel on both sides, mlp_passes_row_sums)
 struct MlpSums {
     void *write = nullptr;
+    bool write_plain = false;  // prefill_adds_sums_in_loop() of the reader
     void *read = nullptr;
 };
-bool mlp_passes_row_sums(int m, int hidden, int n_out, int n_down, int cus) {
+bool mlp_passes_row_sums(int m, int hidden, int n_out, int n_down, int cus, bool *plain) {
     const auto gate_up = plan_call(m, 2 * n_out, hidden, cus, -1, -1, 0), down = plan_call(m, n_down, n_out, cus, -1, -1, 0);
+    *plain = down->gp.prefill && prefill_adds_sums_in_loop(m, n_down, n_out, down->gp.pf, cus);
     return gate_up->gp.prefill && prefill_forms_next_sums(gate_up->gp.pf) && down->gp.prefill &&
            prefill_reads_row_sums(m, n_down, n_out, down->gp.pf);
 }
@@ -957,8 +959,10 @@ kiln_marlin_status_t gemm_any(const void *A, const void *B, void *C, const void 
         } else if (g_tune.rowsum_fold != 0) {
             pa.lora_words = reinterpret_cast<unsigned *>(ws + kFoldFlagOffset);
         }
+        pa.plan_forced = thread_k > 0 || thread_n > 0;
         pa.swiglu = swiglu;
         pa.next_aext = sums.write;
+        pa.next_plain = sums.write_plain;
         if (sums.read) {
             pa.aext = sums.read;
             pa.aext_ready = true;
@@ -1420,7 +1424,7 @@ kiln_marlin_status_t kiln_w4a16_mlp(const void *x, const void *b_gate_up, const 
     // as they store H, whose columns they hold in whole groups: the second launch neither reads H for them beforehand
     // (8192 rows 973 -> 953 us) nor gives block slots to blocks that do (2048 rows 282 -> 276).
     MlpSums write, read;
-    if (mlp_passes_row_sums(prob_m, hidden, n_out, n_down, compute_units(dev)))
+    if (mlp_passes_row_sums(prob_m, hidden, n_out, n_down, compute_units(dev), &write.write_plain))
         write.write = read.read = reinterpret_cast<char *>(h) + (size_t)prob_m * n_out * 2;
     const kiln_marlin_status_t st = gemm_any(x, b_gate_up, h, s_gate_up, prob_m, 2 * n_out, hidden, workspace, groupsize, dev,
                                              stream, -1, -1, -1, nullptr, true, write);

@@ -26,6 +26,8 @@
 // split exactly into three bf16 terms by the pre-pass kernel below, times the
 // group scale split exactly into two bf16 terms; six exact products per group
 // accumulate c * scale into the result (about 5 % extra matrix work).
+// Launches of several rounds of 128-row blocks take c as f32 and add it where a
+// group begins, in the rescale's multiplication (INC below): no extra matrix work.
 #include <type_traits>
 
 #include "device_common.h"
@@ -40,9 +42,15 @@ namespace {
 
 constexpr int kAStages = 4;
 
-// c[m][g] = -136 * sum_{k in group g} a[m][k], split into bf16 hi/mid/lo and
-// stored (group-major, [g][m]) as the 8-slot extension operand
-// [hi, hi, mid, mid, lo, lo, 0, 0].
+__device__ __forceinline__ void store_row_sum(u32x4 *__restrict__ aext, size_t at, float sum, bool plain) {
+    if (plain) reinterpret_cast<float *>(aext)[at] = -kCodeBias * sum;
+    else aext[at] = extension_operand(sum);
+}
+
+// c[m][g] = -136 * sum_{k in group g} a[m][k], group-major ([g][m]), for instances of the kernel that add it at every
+// change of group: as f32 (PLAIN); for the others split into bf16 hi/mid/lo and stored as the 8-slot extension
+// operand [hi, hi, mid, mid, lo, lo, 0, 0].
+template <bool PLAIN>
 __global__ __launch_bounds__(256) void w4a16_prefill_rowsum_kernel(const uint16_t *__restrict__ A,
                                                                  u32x4 *__restrict__ aext, int M, int K) {
     const int G = K / kGroupK;
@@ -53,7 +61,7 @@ __global__ __launch_bounds__(256) void w4a16_prefill_rowsum_kernel(const uint16_
     float sum = sum_bf16x8(*reinterpret_cast<const u32x4 *>(A + (size_t)row * K + (size_t)g * kGroupK + sub * 8));
 #pragma unroll
     for (int off = 8; off >= 1; off >>= 1) sum += __shfl_xor(sum, off, 16);
-    if (sub == 0) aext[(size_t)g * M + row] = extension_operand(sum);  // group-major: the 32 rows of a half-wavefront are contiguous
+    if (sub == 0) store_row_sum(aext, (size_t)g * M + row, sum, PLAIN);  // group-major: the 32 rows of a half-wavefront are contiguous
 }
 
 template <int RB>
@@ -280,14 +288,22 @@ __device__ __forceinline__ void prefill_fold_done(const PrefillFold &pf, int con
             __hip_atomic_store(pf.words + r * kLoraFoldReplicaWords + lane, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-template <int NWN, int WM, int MI, bool SWIGLU, bool RS, bool FOLD = false>
+// INC: c = -136 * sum(a) of every (row, group) is there, in f32, when the launch begins (the pre-pass kernel, or the
+// launch that wrote A), and joins the accumulators at the change of group that begins it: the change's multiplication
+// by scale(g) / scale(g+1) becomes a multiply-add, and there is no extension contraction (6 % of the products at any
+// K, and 2 us a tile).  What it costs is LDS reads: a lane's accumulators lie in 16 rows of every row tile, whose
+// values of c it reads (broadcast) in 16-byte pieces, 16 of them a group beside 32 fragments.  For launches of several
+// rounds, whose row sums come from in front anyway; where the launch's own blocks form them (FOLD, RS) they are not there
+// when a block begins.
+template <int NWN, int WM, int MI, bool SWIGLU, bool RS, bool FOLD = false, bool INC = false>
 __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void w4a16_prefill_kernel(
     const uint16_t *__restrict__ A, const u32x4 *__restrict__ B, const uint16_t *__restrict__ S,
     uint16_t *__restrict__ C, const u32x4 *__restrict__ aext, int M, int N, int K, int Gs, int m_blocks,
     const uint16_t *__restrict__ lora_t, const uint16_t *__restrict__ lora_b, int r_total, int RP, int nb_full,
-    int KS, int GSb, float *partial, int *counters, int die_rows, u32x4 *next_aext, PrefillFold pf) {
+    int KS, int GSb, float *partial, int *counters, int die_rows, u32x4 *next_aext, bool next_plain, PrefillFold pf) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];  // the A ring; reused by the store
     static_assert(!FOLD || WM * NWN == 4, "the projection's blocks have four wavefronts");
+    static_assert(!INC || (!FOLD && !RS && WM == 1 && NWN == 4 && MI == 4), "the row sums come from in front");
     if constexpr (FOLD) {
         if ((int)blockIdx.x < pf.producers) {
             const int unit = blockIdx.x;
@@ -453,7 +469,17 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
         }
     };
     // prologue: the first group's words, four stages of A
+    // INC: c of a group's rows, [row] f32, in two slots that take turns; every wavefront asks for 64 rows of it
+    // (wavefronts beyond the block's rows for a copy nobody reads, so that all count the same loads)
+    constexpr int kSumSlot = NW * 256;
+    static_assert((kAStages * kAStageBytes) % (2 * kSumSlot) == 0, "slots alternate by one bit of their offset");
+    [[maybe_unused]] int c_at = kAStages * kAStageBytes + h * 16;  // this group's slot; the next one's is c_at ^ kSumSlot
+    [[maybe_unused]] const char *c_ptr = nullptr;                  // this group's c in memory
+    [[maybe_unused]] const uint32_t c_off = (uint32_t)min(m0 + (wave % (BM / 64)) * 64 + lane, M - 1) * 4u;
+    [[maybe_unused]] int c_to = kAStages * kAStageBytes + wave * 256;  // offsets: the slots' bit is theirs, not the base's
+    if constexpr (INC) c_ptr = uniform(reinterpret_cast<const char *>(aext) + (size_t)g_begin * M * 4);
     request_b(bw, b_ptr, s_ptr);
+    if constexpr (INC) load_to_lds_b32(c_ptr, c_off, lds_base + c_to);
 #pragma unroll
     for (int st = 0; st < 4; ++st) load_a(a_ptr + st * 64, st);
     wait_vector_loads<3 * APW>();  // the words and stage 0
@@ -514,7 +540,7 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
     // of the main loop asks for the first four in place of further stages of A.
     const int ng = g_end - g_begin;
     const char *const s_base = s_ptr;
-    constexpr int kExtLoads = (RS ? 0 : APW) + 2;  // per wavefront and extension stage
+    constexpr int kExtLoads = INC ? 0 : (RS ? 0 : APW) + 2;  // per wavefront and extension stage
     const uint32_t ext_off = (uint32_t)min(m0 + (RS ? 0 : (wave % (BM / 64)) * 64) + lane, M - 1) * 16u;
     auto ext_scales = [&](int slot) { return RS ? slot * kAStageBytes + wave * 512 : kAStages * kAStageBytes + (slot * NW + wave) * 512; };
     auto request_ext = [&](int e, int slot) {  // groups past the last re-read it
@@ -533,6 +559,21 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
             load_to_lds_b32(s_base, off, lds_base + ext_scales(slot) + v * 256);
         }
     };
+    // INC: the change of group in work items of four registers -- (row tile, quarter, column sub-tile) -- behind the
+    // products kChangeAt ... of the old group's last stage (row tiles of the first half) and of the new group's first
+    // (the others, counted without the four products in front of the barrier), kChangeRoom of them, a quarter's c read
+    // kChangeLead products before its first use.
+    constexpr int kChangeAt = 2, kChangeRoom = 10, kChangeLead = 2;
+    if constexpr (INC) {
+#pragma unroll
+        for (int mi = 0; mi < MI / 2; ++mi)  // the others begin at 0 and take c in the first stage
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const f32x4 c = *reinterpret_cast<const f32x4 *>(lds + c_at + mi * 128 + i * 32);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[mi][0][4 * i + r] = acc[mi][1][4 * i + r] = c[r];
+            }
+    }
     // one group; LAST: no further group; PEEK: ask for the words of a folded launch
     auto group = [&](auto lastc, auto peekc) {
         constexpr bool LAST = decltype(lastc)::value, PEEK = decltype(peekc)::value;
@@ -540,6 +581,7 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
             constexpr int q = decltype(qc)::value;
             constexpr bool ahead = !(LAST && q == 3);  // there is a next stage
             u32x4 bn[2][2];
+            [[maybe_unused]] f32x4 cq[INC ? MI * 2 : 1];
             unrolled<0, MI>([&](auto mc) {
                 constexpr int mi = decltype(mc)::value;
                 unrolled<0, 4>([&](auto jc) {
@@ -567,7 +609,27 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
                     // stage; MI = 4: tiles 0 | 1 2 | 3 4 in phases 1, 2, 3, tiles 5 | 6 | 7 in phases 0, 1, 2 of the next group
                     constexpr int t0 = q == 3 ? (MI == 4 ? (mi < 2 ? 0 : 2 * mi - 3) : 0) : (MI == 4 ? 5 + mi : 2);
                     constexpr int t1 = q == 3 ? (MI == 4 ? (mi == 0 ? 0 : 2 * mi - 1) : (mi == 0 ? 0 : 2)) : (MI == 4 ? 6 + mi : (mi == 0 ? 4 : 2));
-                    if constexpr ((q == 3 && !LAST) || (q == 0 && mi < MI - 1)) {
+                    if constexpr (INC && ((q == 3 && !LAST) || q == 0)) {
+                        constexpr int at = slot - (q == 3 ? 4 : 0) - kChangeAt, items = MI * 4;
+                        constexpr int rt0 = q == 3 ? 0 : MI / 2;
+                        constexpr auto begin_of = [](int p) { return p < 0 ? 0 : p > kChangeRoom ? items : p * items / kChangeRoom; };
+                        unrolled<begin_of(at + kChangeLead), begin_of(at + kChangeLead + 1)>([&](auto ec) {
+                            constexpr int e = decltype(ec)::value, quarter = e >> 1;
+                            if constexpr ((e & 1) == 0)
+                                cq[quarter] = *reinterpret_cast<const f32x4 *>(lds + (q == 3 ? c_at ^ kSumSlot : c_at) +
+                                                                               (rt0 + (quarter >> 2)) * 128 + (quarter & 3) * 32);
+                        });
+                        unrolled<begin_of(at), begin_of(at + 1)>([&](auto ec) {
+                            constexpr int e = decltype(ec)::value, quarter = e >> 1, en = e & 1;
+                            f32x16 &a = acc[rt0 + (quarter >> 2)][en];
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) a[4 * (quarter & 3) + r] = fmaf(a[4 * (quarter & 3) + r], f[en], cq[quarter][r]);
+                            // c outlives its last use: left to itself the compiler lets that one write over c's registers
+                            // and copies the accumulator tile together again, or spills
+                            if constexpr (en == 1) asm volatile("" : : "v"(cq[quarter]));
+                        });
+                    }
+                    if constexpr (!INC && ((q == 3 && !LAST) || (q == 0 && mi < MI - 1))) {
                         unrolled<t0, t1>([&](auto tc) {
                             constexpr int t = decltype(tc)::value;
 #pragma unroll
@@ -581,14 +643,14 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
                     // it (in the last group extension stages take the place of stages) and, unless they are needed now,
                     // the next group's six.
                     constexpr int a_behind = LAST && q > 0 ? (q == 1 ? 1 : 0) : 2;
-                    constexpr int others = (!LAST && (q == 1 || q == 2)) ? 6 + (PEEK ? 1 : 0) : 0;
+                    constexpr int others = (!LAST && (q == 1 || q == 2)) ? 6 + (PEEK || INC ? 1 : 0) : 0;
                     wait_vector_loads<a_behind * APW + (2 - a_behind) * kExtLoads + others>();
                     wait_lds_reads();
                     __builtin_amdgcn_s_barrier();
                     asm volatile("" : : : "memory");
                     if constexpr (!LAST) {
                         load_a(a_ptr + (q + 4) * 64, q);
-                        if constexpr (q == 0) request_b(bw_next, b_ptr + 1024, s_ptr + s_step);
+                        if constexpr (q == 0 && !INC) request_b(bw_next, b_ptr + 1024, s_ptr + s_step);
                         if constexpr (q == 3) {
 #pragma unroll
                             for (int i = 0; i < 2; ++i) {
@@ -604,8 +666,13 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
                             }
                         }
                     }
-                    if constexpr (LAST) request_ext(q, q);
+                    if constexpr (LAST && !INC) request_ext(q, q);
                     if constexpr (PEEK && q == 0) prefill_fold_peek(pf, m0, min(BM, M - m0), lane, lds_base + kFoldPeekOffset + wave * 256);
+                }
+                if constexpr (INC && q == 0 && mi == MI - 1 && !LAST) {
+                    // three phases later than without INC: the registers are c's until then
+                    request_b(bw_next, b_ptr + 1024, s_ptr + s_step);
+                    load_to_lds_b32(c_ptr + (size_t)M * 4, c_off, lds_base + (c_to ^ kSumSlot));
                 }
                 if constexpr (ahead) {
                     if constexpr (RS && mi == 0) {
@@ -632,6 +699,11 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
         a_ptr += 256;
         b_ptr += 1024;
         s_ptr += s_step;
+        if constexpr (INC) {
+            c_ptr += (size_t)M * 4;
+            c_at ^= kSumSlot;
+            c_to ^= kSumSlot;
+        }
         ++g_now;
     };
     while (g_now + 1 + (FOLD ? 1 : 0) < g_end) {
@@ -718,7 +790,7 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
             for (int ni = 0; ni < 2; ++ni) acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ax, bx[ni], acc[mi][ni], 0, 0, 0);
         }
     };
-    {
+    if constexpr (!INC) {
         ExtStep x0, x1;
         ext_read(0, 0, x0);  // visible since the last group's last barrier
         for (int e = 0; 4 * e < ng; ++e) {
@@ -895,7 +967,7 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
                     for (int off = 8; off >= 1; off >>= 1)
 #pragma unroll
                         for (int i = 0; i < off; ++i) u[i] += u[i + off];
-                    next_aext[(size_t)nb * M + m0 + tid] = extension_operand(u[0]);
+                    store_row_sum(next_aext, (size_t)nb * M + m0 + tid, u[0], next_plain);
                 }
             }
         }
@@ -1132,11 +1204,11 @@ constexpr int kMaxRowSumBytes = 24 * 1024;
 static int row_sum_bytes(int groups) { return groups * 64 * (int)sizeof(float); }
 
 
-template <int NWN, int WM, int MI, bool SWIGLU, bool RS, bool FOLD = false>
+template <int NWN, int WM, int MI, bool SWIGLU, bool RS, bool FOLD = false, bool INC = false>
 hipError_t launch_shape_as(const PrefillArgs &a, int grid, int m_blocks, int RP, int KS, int GSb, int max_groups,
                            hipStream_t stream, const PrefillFold &pf = PrefillFold{}) {
     constexpr int BM = WM * MI * 32, NW = WM * NWN;
-    constexpr int kRing = kAStages * BM * 64 + (RS ? 0 : kAStages * NW * 512);  // the A ring, the extension's scales behind it
+    constexpr int kRing = kAStages * BM * 64 + (INC ? 2 * NW * 256 : RS ? 0 : kAStages * NW * 512);  // the A ring, behind it the groups' c or the extension's scales
     constexpr int kStore = NW * MI * 32 * 64 * 2;   // the store's per-wavefront transposes (reuses the ring)
     // RS: the row sums sit behind the ring and are dead by the time the store reuses the space
     constexpr int kLdsMax = RS ? (kRing + kMaxRowSumBytes > kStore ? kRing + kMaxRowSumBytes : kStore)
@@ -1148,15 +1220,15 @@ hipError_t launch_shape_as(const PrefillArgs &a, int grid, int m_blocks, int RP,
     // on one unit while others idle.
     constexpr int kLdsSolo0 = (WM == 2 && NWN == 2) ? 96 * 1024 : kLdsMax;
     constexpr int kLdsSolo = FOLD && kLdsSolo0 < kProjectLdsBytes16 ? kProjectLdsBytes16 : kLdsSolo0;
-    const hipError_t attr = allow_dynamic_lds<&w4a16_prefill_kernel<NWN, WM, MI, SWIGLU, RS, FOLD>>(kLdsSolo);
+    const hipError_t attr = allow_dynamic_lds<&w4a16_prefill_kernel<NWN, WM, MI, SWIGLU, RS, FOLD, INC>>(kLdsSolo);
     if (attr != hipSuccess) return attr;
     if (WM == 2 && NWN == 2 && grid <= a.cus) lds_bytes = kLdsSolo;
     if (FOLD && lds_bytes < kProjectLdsBytes16) lds_bytes = kProjectLdsBytes16;  // the projection's blocks stage more
-    w4a16_prefill_kernel<NWN, WM, MI, SWIGLU, RS, FOLD><<<grid + (FOLD ? pf.producers : 0), 64 * NW, lds_bytes, stream>>>(
+    w4a16_prefill_kernel<NWN, WM, MI, SWIGLU, RS, FOLD, INC><<<grid + (FOLD ? pf.producers : 0), 64 * NW, lds_bytes, stream>>>(
         (const uint16_t *)a.A, (const u32x4 *)a.B, (const uint16_t *)a.S, (uint16_t *)a.C, (const u32x4 *)a.aext,
         a.M, a.N, a.K, a.Gs, m_blocks, (const uint16_t *)a.lora_t, (const uint16_t *)a.lora_b, a.r_total, RP,
         a.nb_full, KS, GSb, a.partial, a.counters,
-        prefill_die_rows(m_blocks, a.nb_full, (a.N / (NWN * 64) - a.nb_full) * KS, KS), (u32x4 *)a.next_aext, pf);
+        prefill_die_rows(m_blocks, a.nb_full, (a.N / (NWN * 64) - a.nb_full) * KS, KS), (u32x4 *)a.next_aext, a.next_plain, pf);
     return hipGetLastError();
 }
 
@@ -1284,6 +1356,17 @@ int prefill_rowsum_producers(int M, int N, int K, const PrefillPlan &p, int cus)
     return producers < 128 ? producers : 128;
 }
 
+// Where the row sums are added at the groups' changes (INC): plain calls in 128-row blocks whose row sums
+// prefill_rowsum_producers() leaves to a launch in front.  By the shape alone, since the two routes of a shape's row
+// sums must agree in every bit; and not for calls with overrides (PrefillArgs::plan_forced), whose block shapes
+// must.  64-row blocks keep the extension contraction: their plain calls equal those with adapters of zeros, and a
+// launch that runs the projection has no row sums to begin with.
+// (2560 -> 2 x 9216 -> 2560 at 8192 rows 933 -> 912 us, at 2048 rows 269 -> 260, error beyond the bf16 rounding 2.1e-4 -> 0.9e-4
+// of the result's norm, 1.1e-3 -> 2.2e-4 where the activations have a mean of half their deviation: the surplus leaves group by
+// group instead of piling up in the accumulators.)
+bool prefill_adds_sums_in_loop(int M, int N, int K, const PrefillPlan &p, int cus) {
+    return p.bn == 256 && p.bm == 128 && prefill_rowsum_producers(M, N, K, p, cus) == 0;
+}
 bool prefill_forms_next_sums(const PrefillPlan &p) { return p.bn == 256 && (p.bm == 64 || p.bm == 128); }
 bool prefill_reads_row_sums(int M, int N, int K, const PrefillPlan &p) { return !blocks_sum_their_rows(M, N, K, p); }
 
@@ -1302,12 +1385,13 @@ hipError_t launch_prefill(const PrefillArgs &a, hipStream_t stream) {
     // with adapters the projection's launch forms the row sums on its way over x
     const bool sums_with_projection = !rs && a.r_total > 0;
     if (a.next_aext && !prefill_forms_next_sums(shape)) return hipErrorInvalidValue;
+    const bool inc = a.r_total == 0 && !a.plan_forced && prefill_adds_sums_in_loop(a.M, a.N, a.K, shape, a.cus);
     const int inside = a.r_total == 0 && a.lora_words && !a.aext_ready ? prefill_rowsum_producers(a.M, a.N, a.K, shape, a.cus) : 0;
     const int sum_producers = inside > 0 ? inside : 0;
     if (!rs && !sums_with_projection && sum_producers == 0 && !a.aext_ready) {
         const int items = a.M * G;
-        w4a16_prefill_rowsum_kernel<<<(items + 15) / 16, 256, 0, stream>>>((const uint16_t *)a.A, (u32x4 *)a.aext,
-                                                                          a.M, a.K);
+        (inc ? w4a16_prefill_rowsum_kernel<true> : w4a16_prefill_rowsum_kernel<false>)<<<(items + 15) / 16, 256, 0, stream>>>(
+            (const uint16_t *)a.A, (u32x4 *)a.aext, a.M, a.K);
         err = hipGetLastError();
         if (err != hipSuccess) return err;
     }
@@ -1398,6 +1482,10 @@ hipError_t launch_prefill(const PrefillArgs &a, hipStream_t stream) {
         if (a.bm == 128) return launch_shape_as<4, 1, 4, false, false, true>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream, pf);
         return rs ? launch_shape_as<4, 1, 2, false, true, true>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream, pf)
                   : launch_shape_as<4, 1, 2, false, false, true>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream, pf);
+    }
+    if (inc) {
+        return a.swiglu ? launch_shape_as<4, 1, 4, true, false, false, true>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream)
+                        : launch_shape_as<4, 1, 4, false, false, false, true>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream);
     }
     if (a.bm == 256) {
         return a.bn == 256 ? launch_shape<4, 2, 4>(a, grid, m_blocks, RP, KS, GSb, max_groups, rs, stream)
