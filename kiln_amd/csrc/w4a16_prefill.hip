@@ -4,11 +4,11 @@
 // (crates/kiln-marlin-gemm/csrc/marlin_kernel.cu:754-763, :784-816, :189-700).
 // This regime is a dense contraction bound by the bf16 matrix cores.
 //
-// Block = 4 wavefronts (2 x 2), block tile 256 rows x 128 columns, wavefront
-// tile 128 x 64 = 4 x 2 tiles of v_mfma_f32_32x32x16_bf16 (128 accumulator
-// registers, two wavefronts per SIMD).  Per 32 rows of K:
-//   * a 256 x 32 bf16 tile of A goes global -> LDS with direct 128-bit loads
-//     (no registers, no VALU) into a ring of four stages, three stages ahead
+// Block = 4 wavefronts side by side, block tile 128 (or 64) rows x 256 columns,
+// wavefront tile 128 x 64 = 4 x 2 tiles of v_mfma_f32_32x32x16_bf16 (128
+// accumulator registers, two wavefronts per SIMD).  Per 32 rows of K:
+//   * a 128 x 32 bf16 tile of A goes global -> LDS with direct 128-bit loads
+//     (no registers, no VALU) into a ring of four stages, four stages ahead
 //     of the products, one barrier per stage, stored with an XOR swizzle so
 //     that fragment reads are bank-conflict free;
 //   * each wavefront reads its 64 columns of packed weights straight from
@@ -564,6 +564,7 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
     // (the others, counted without the four products in front of the barrier), kChangeRoom of them, a quarter's c read
     // kChangeLead products before its first use.
     constexpr int kChangeAt = 2, kChangeRoom = 10, kChangeLead = 2;
+    static_assert(kChangeLead <= kChangeAt, "the next group's c is read behind the barrier that shows it");
     if constexpr (INC) {
 #pragma unroll
         for (int mi = 0; mi < MI / 2; ++mi)  // the others begin at 0 and take c in the first stage
