@@ -51,17 +51,20 @@ class _WrappingOwner:
 
     def __init__(self, b: torch.Tensor, s: torch.Tensor, k: int, n: int, groupsize: int):
         self._args = (b, s, k, n, groupsize)
-        self._owner: Optional[_NativeOwner] = None
+        self._made: dict[str, _NativeOwner] = {}
 
     @property
     def handle(self) -> int:
-        if self._owner is None:
+        owner = self._made.get("owner")
+        if owner is None:
             b, s, k, n, groupsize = self._args
             out = ctypes.c_void_p()
             if _lib.load().kiln_marlin_proj_wrap(b.data_ptr(), s.data_ptr(), k, n, groupsize, _device_index(b), ctypes.byref(out)) != _lib.PROJ_OK:
                 _raise_last()
-            self._owner = _NativeOwner(out.value)
-        return self._owner.handle
+            # Threads may be here together (the call lets go of the interpreter): the first one's handle stays for good
+            # -- setdefault is one step -- and the others', which nobody has been given, are freed as they go.
+            owner = self._made.setdefault("owner", _NativeOwner(out.value))
+        return owner.handle
 
 
 class _DeviceView:
