@@ -75,9 +75,21 @@ struct Problem {
 bool packed_ok(const at::Tensor &b, const at::Tensor &s, int64_t k, int groupsize, c10::Device device, int64_t *n) {
     if (!plain(b, at::kInt, 2, device) || !plain(s, at::kHalf, 2, device)) return false;
     *n = s.size(1);
-    if (groupsize != 128 && groupsize != -1) return false;
     return k > 0 && k % 128 == 0 && *n > 0 && *n % 256 == 0 && b.size(0) == k / 16 && b.size(1) == 2 * *n &&
            s.size(0) == (groupsize == -1 ? 1 : k / 128) && k <= INT32_MAX && *n <= INT32_MAX / 2;
+}
+
+// 128 or -1 (per column), compared before it is narrowed; anything else, integers beyond 64 bits included, is the
+// checked route's to refuse
+bool groupsize_of(PyObject *o, int *groupsize) {
+    const long g = PyLong_AsLong(o);
+    if (g == -1 && PyErr_Occurred()) {
+        PyErr_Clear();
+        return false;
+    }
+    if (g != 128 && g != -1) return false;
+    *groupsize = (int)g;
+    return true;
 }
 
 // max_rank: 2 for the GEMM entry points, 3 where a [batch, seq, k] activation is taken as well
@@ -85,13 +97,7 @@ bool problem_of(PyObject *const *args, int max_rank, Problem *p) {
     p->x = tensor_of(args[0]);
     p->b = tensor_of(args[1]);
     p->s = tensor_of(args[2]);
-    if (!p->x || !p->b || !p->s || !g_lib.gemm) return false;
-    const long g = PyLong_AsLong(args[3]);
-    if (g == -1 && PyErr_Occurred()) {
-        PyErr_Clear();
-        return false;
-    }
-    p->groupsize = (int)g;
+    if (!p->x || !p->b || !p->s || !g_lib.gemm || !groupsize_of(args[3], &p->groupsize)) return false;
     const at::Tensor &x = *p->x;
     const int64_t rank = x.dim();
     if (rank < 2 || rank > max_rank || !x.is_cuda()) return false;
@@ -406,8 +412,8 @@ PyObject *py_quantize(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
         PyObject *pair = PyTuple_GET_ITEM(args[0], (Py_ssize_t)i);
         if (!PyTuple_CheckExact(pair) || PyTuple_GET_SIZE(pair) != 2 || !PyLong_CheckExact(PyTuple_GET_ITEM(pair, 1))) Py_RETURN_NONE;
         const at::Tensor *w = tensor_of(PyTuple_GET_ITEM(pair, 0));
-        it.g = (int)PyLong_AsLong(PyTuple_GET_ITEM(pair, 1));
-        if (!w || !w->is_cuda() || !plain(*w, at::kBFloat16, 2, i ? items[0].w.device() : w->device()) || (it.g != 128 && it.g != -1))
+        if (!w || !w->is_cuda() || !plain(*w, at::kBFloat16, 2, i ? items[0].w.device() : w->device()) ||
+            !groupsize_of(PyTuple_GET_ITEM(pair, 1), &it.g))
             Py_RETURN_NONE;
         it.w = *w;
         it.k = w->size(0);
