@@ -24,6 +24,7 @@ _FUNCTIONS = ("kiln_marlin_w4a16_gemm", "kiln_w4a16_gemm_lora", "kiln_w4a16_gemm
 
 _ext = None
 _adapter_types: tuple = ()
+_workspaces: dict | None = None
 
 
 def set_adapter_types(stacked: type, single: type) -> None:
@@ -32,6 +33,14 @@ def set_adapter_types(stacked: type, single: type) -> None:
     _adapter_types = (stacked, single)
     if _ext is not None:
         _ext.set_adapter_types(*_adapter_types)
+
+
+def set_workspaces(workspaces: dict) -> None:
+    """The dictionary `{(device index, stream handle): uint8 tensor}` the calls look their workspace up in."""
+    global _workspaces
+    _workspaces = workspaces
+    if _ext is not None:
+        _ext.set_workspaces(_workspaces)
 
 
 def _bind(ext):
@@ -50,6 +59,8 @@ def _import() -> None:
     _ext = ext
     if _adapter_types:
         ext.set_adapter_types(*_adapter_types)
+    if _workspaces is not None:
+        ext.set_workspaces(_workspaces)
     _lib.on_active_library(_bind(ext))
     _lib.load()
     for name in _NAMES:
@@ -64,5 +75,5 @@ def _stand_in(name: str):
     return first_call
 
 
-_NAMES = ("linear", "linear_lora", "linear_sides", "mlp", "quantize", "set_workspace")
-linear, linear_lora, linear_sides, mlp, quantize, set_workspace = map(_stand_in, _NAMES)
+_NAMES = ("linear", "linear_lora", "linear_sides", "mlp", "quantize")
+linear, linear_lora, linear_sides, mlp, quantize = map(_stand_in, _NAMES)

@@ -13,8 +13,6 @@
 
 #include <array>
 #include <cstdint>
-#include <mutex>
-#include <unordered_map>
 #include <vector>
 
 #include <ATen/ATen.h>
@@ -45,19 +43,9 @@ PyTypeObject *g_stacked_type = nullptr, *g_single_type = nullptr;  // lora.Stack
 PyObject *g_names[6] = {};                                         // interned: a_cat b_cat ranks scales a b
 enum { kACat, kBCat, kRanks, kScales, kA, kB };
 
-// The workspaces marlin_gemm keeps, one per (device, stream): the same tensors, found without Python.
-struct StreamKey {
-    int device;
-    uintptr_t stream;
-    bool operator==(const StreamKey &o) const { return device == o.device && stream == o.stream; }
-};
-struct StreamKeyHash {
-    size_t operator()(const StreamKey &k) const { return (k.stream >> 4) * 31 + (size_t)k.device; }
-};
-std::unordered_map<StreamKey, at::Tensor, StreamKeyHash> &workspaces() {
-    static auto *map = new std::unordered_map<StreamKey, at::Tensor, StreamKeyHash>();  // outlives the interpreter's end
-    return *map;
-}
+// marlin_gemm's workspaces, {(device index, stream handle): uint8 tensor}: looked up on every call, so that the
+// dictionary is their only owner and what happens to its entries holds here at once.
+PyObject *g_workspaces = nullptr;
 
 const at::Tensor *tensor_of(PyObject *o) { return THPVariable_CheckExact(o) ? &THPVariable_Unpack(o) : nullptr; }
 
@@ -140,10 +128,20 @@ struct Launch {
     explicit Launch(c10::Device device)
         : guard(device), stream((void *)c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(device.index()).stream()) {}
     bool find_workspace(c10::Device device, size_t bytes) {
-        auto it = workspaces().find(StreamKey{device.index(), (uintptr_t)stream});
-        if (it == workspaces().end() || (size_t)it->second.numel() < bytes) return false;
-        workspace = it->second;
-        return true;
+        PyObject *key = PyTuple_New(2), *index = PyLong_FromLong(device.index()), *handle = PyLong_FromVoidPtr(stream);
+        if (key && index && handle && g_workspaces) {
+            PyTuple_SET_ITEM(key, 0, index);
+            PyTuple_SET_ITEM(key, 1, handle);
+            index = handle = nullptr;  // the tuple's now
+            const PyObject *found = PyDict_GetItemWithError(g_workspaces, key);
+            const at::Tensor *t = found ? tensor_of(const_cast<PyObject *>(found)) : nullptr;
+            if (t && plain(*t, at::kByte, 1, device) && (size_t)t->numel() >= bytes) workspace = *t;
+        }
+        Py_XDECREF(key);
+        Py_XDECREF(index);
+        Py_XDECREF(handle);
+        PyErr_Clear();
+        return workspace.defined();
     }
 };
 
@@ -483,20 +481,16 @@ PyObject *py_quantize(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     END_HANDLE_TH_ERRORS
 }
 
-// set_workspace(device index, stream handle, tensor)
-PyObject *py_set_workspace(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
-    HANDLE_TH_ERRORS
-    const at::Tensor *t = nargs == 3 ? tensor_of(args[2]) : nullptr;
-    if (!t || !t->is_cuda() || t->scalar_type() != at::kByte || !t->is_contiguous()) {
-        PyErr_SetString(PyExc_TypeError, "set_workspace takes (device index, stream handle, uint8 CUDA tensor)");
+// set_workspaces(marlin_gemm's dictionary of them)
+PyObject *py_set_workspaces(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
+    if (nargs != 1 || !PyDict_CheckExact(args[0])) {
+        PyErr_SetString(PyExc_TypeError, "set_workspaces takes a dictionary");
         return nullptr;
     }
-    const long device = PyLong_AsLong(args[0]);
-    const unsigned long long stream = PyLong_AsUnsignedLongLong(args[1]);
-    if (PyErr_Occurred()) return nullptr;
-    workspaces()[StreamKey{(int)device, (uintptr_t)stream}] = *t;
+    Py_INCREF(args[0]);
+    Py_XDECREF(g_workspaces);
+    g_workspaces = args[0];
     Py_RETURN_NONE;
-    END_HANDLE_TH_ERRORS
 }
 
 // bind(addresses of the library's functions, in the order of Library)
@@ -535,7 +529,7 @@ PyObject *py_set_adapter_types(PyObject *, PyObject *const *args, Py_ssize_t nar
 
 #define FAST(name, fn) {name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(fn)), METH_FASTCALL, nullptr}
 PyMethodDef g_methods[] = {FAST("linear", py_linear), FAST("linear_lora", py_linear_lora), FAST("linear_sides", py_linear_sides),
-                           FAST("mlp", py_mlp), FAST("quantize", py_quantize), FAST("set_workspace", py_set_workspace), FAST("bind", py_bind),
+                           FAST("mlp", py_mlp), FAST("quantize", py_quantize), FAST("set_workspaces", py_set_workspaces), FAST("bind", py_bind),
                            FAST("set_adapter_types", py_set_adapter_types), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_torch_calls", nullptr, -1, g_methods, nullptr, nullptr, nullptr, nullptr};
 

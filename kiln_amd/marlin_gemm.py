@@ -28,8 +28,9 @@ def _bail(msg: str):
 
 # One workspace per (device, stream): only its counter prefix must be zero on first use and the
 # kernels leave it zero on exit, so it is allocated once, grown when a larger call comes, and
-# never cleared again.
+# never cleared again.  The only owner: the direct calls look here too.
 _workspaces: dict[tuple[int, int], torch.Tensor] = {}
+_calls.set_workspaces(_workspaces)
 
 
 def _workspace(device: torch.device, stream_ptr: int, nbytes: int) -> torch.Tensor:
@@ -39,7 +40,6 @@ def _workspace(device: torch.device, stream_ptr: int, nbytes: int) -> torch.Tens
         ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
         ws[:_lib.load().kiln_w4a16_workspace_zeroed_bytes()].zero_()
         _workspaces[key] = ws
-        _calls.set_workspace(key[0], stream_ptr, ws)
     return ws
 
 
