@@ -27,7 +27,7 @@ def build(force: bool = True, jobs: int = 8, verbose: bool = False) -> Path:
     hipcc = Path(rocm) / "bin" / "hipcc"
     if not hipcc.exists():
         raise RuntimeError(f"kiln-marlin-gemm: hipcc not found at {hipcc}; set ROCM_PATH")
-    cmd = ["make", "-C", str(CSRC), f"-j{jobs}", f"ROCM_PATH={rocm}", f"PYTHON={sys.executable}"]
+    cmd = ["make", "-C", str(CSRC), f"-j{jobs}", f"ROCM_PATH={rocm}", f"PYTHON={sys.executable}", "python"]
     if force:
         cmd.append("-B")
     res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)

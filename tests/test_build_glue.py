@@ -84,3 +84,15 @@ def test_crate_extern_block_matches_the_header():
         rust_args = [a for a in args.split(",") if a.strip()]
         assert len(c_args) == len(rust_args), name
         assert hasattr(lib, name)
+
+
+def test_a_c_host_builds_without_python_or_torch():
+    """`make all`, the libraries and the C harness, asks nothing of Python: the extension kiln_amd loads is a target of its
+    own, which kiln_amd.build names."""
+    make = ["make", "-C", str(CSRC), "-n", "-B", "PYTHON=/nonexistent/python3"]
+    res = subprocess.run(make + ["all"], capture_output=True, text=True)
+    assert res.returncode == 0 and "nonexistent" not in res.stdout + res.stderr, res.stderr
+    assert "torch_calls" not in res.stdout and all(t in res.stdout for t in ("libkiln_marlin_gemm.so", "_tuning.so", "c_abi_harness"))
+    res = subprocess.run(["make", "-C", str(CSRC), "-n", "-B", "python"], check=True, capture_output=True, text=True)
+    assert "torch_calls.cpp" in res.stdout and "libkiln_marlin_gemm.so" in res.stdout
+    assert '"python"' in (ROOT / "kiln_amd" / "build.py").read_text()
