@@ -202,7 +202,7 @@ PrefillPlan plan_prefill(int m, int n, int k, int cus, int force_bn = 0, int for
 int prefill_grid(int m, int n, const PrefillPlan &p);
 size_t prefill_partial_bytes(int m, int n, const PrefillPlan &p);
 int prefill_rowsum_producers(int m, int n, int k, const PrefillPlan &p, int cus);  // blocks of a plain launch that form the row sums inside it (0: a launch in front does, -2: every block its own)
-bool prefill_adds_sums_in_loop(int m, int n, int k, const PrefillPlan &p, int cus);  // a plain launch's row sums: f32 [K/128][M]
+bool prefill_adds_sums_in_loop(int m, int n, int k, const PrefillPlan &p, int cus);  // the launch's row sums: f32 [K/128][M]
 bool prefill_forms_next_sums(const PrefillPlan &p);                             // can its swiglu launch write next_aext?
 bool prefill_reads_row_sums(int m, int n, int k, const PrefillPlan &p);         // ... a plain launch take it as aext?
 hipError_t launch_prefill(const PrefillArgs &args, hipStream_t stream);
@@ -210,6 +210,7 @@ hipError_t launch_prefill(const PrefillArgs &args, hipStream_t stream);
 // padding columns zero.  few_rows: the small-M kernels will multiply it, in up to
 // prefill_lora_max_slices(M) slices; otherwise one slice.
 hipError_t launch_lora_project(const PrefillArgs &args, bool few_rows, hipStream_t stream, int *slices,
-                               bool with_row_sums = false);  // many rows: also write the extension operand (args.aext)
+                               bool with_row_sums = false,  // many rows: also write the product's row sums (args.aext),
+                               bool plain_sums = false);    // in the form of prefill_adds_sums_in_loop()
 
 }  // namespace kiln

@@ -15,6 +15,12 @@ __device__ __forceinline__ u32x4 extension_operand(float sum) {
     const uint32_t lo = __builtin_bit_cast(uint32_t, r2) & 0xFFFF0000u;
     return u32x4{(hi >> 16) | hi, (mid >> 16) | mid, (lo >> 16) | lo, 0u};
 }
+// c = -136 * sum as the matrix-core kernel takes it: f32 (`plain`) where it is added at the groups' changes, else the
+// extension contraction's operand
+__device__ __forceinline__ void store_row_sum(u32x4 *__restrict__ aext, size_t at, float sum, bool plain) {
+    if (plain) reinterpret_cast<float *>(aext)[at] = -kCodeBias * sum;
+    else aext[at] = extension_operand(sum);
+}
 // the sum of 8 bf16 values in a 128-bit unit, in the order both kernels below use
 __device__ __forceinline__ float sum_bf16x8(u32x4 v) {
     const uint32_t wd[4] = {v.x, v.y, v.z, v.w};
@@ -69,8 +75,8 @@ __device__ __forceinline__ void store_b128_through(void *ptr, u32x4 v) {
 // extension operand) are in memory -- for a caller that computes the projection inside another
 // kernel's launch instead of in front of it.  Both are then written through to memory: an ordinary
 // store is complete when this die's cache has it, which a reader on another die does not see
-// before the launch ends.
-template <int RB>  // rows per block: 16 or 64
+// before the launch ends.  PLAIN: the row sums' form (store_row_sum); never with `done`.
+template <int RB, bool PLAIN = false>  // rows per block: 16 or 64
 __device__ __forceinline__ void lora_project_block(unsigned char *lds, const uint16_t *__restrict__ X,
                                                    const uint16_t *__restrict__ a_cat, uint16_t *__restrict__ T, int M,
                                                    int K, int r_total, int RP, int steps_per_slice, const LoraScales &ls,
@@ -156,9 +162,13 @@ __device__ __forceinline__ void lora_project_block(unsigned char *lds, const uin
 #pragma unroll
                 for (int off = 8; off >= 1; off >>= 1) sum += __shfl_xor(sum, off, 16);
                 if (sub == 0 && m0 + row < M && c0 + 4 * half < s1) {
-                    u32x4 *dst = aext + (size_t)(c0 / 4 + half) * M + m0 + row;
-                    if (done) store_b128_through(dst, extension_operand(sum));
-                    else *dst = extension_operand(sum);
+                    if constexpr (PLAIN) {
+                        store_row_sum(aext, (size_t)(c0 / 4 + half) * M + m0 + row, sum, true);
+                    } else {
+                        u32x4 *dst = aext + (size_t)(c0 / 4 + half) * M + m0 + row;
+                        if (done) store_b128_through(dst, extension_operand(sum));
+                        else *dst = extension_operand(sum);
+                    }
                 }
             }
         }

@@ -26,8 +26,8 @@
 // split exactly into three bf16 terms by the pre-pass kernel below, times the
 // group scale split exactly into two bf16 terms; six exact products per group
 // accumulate c * scale into the result (about 5 % extra matrix work).
-// Launches of several rounds of 128-row blocks take c as f32 and add it where a
-// group begins, in the rescale's multiplication (INC below): no extra matrix work.
+// Launches of several rounds of 128-row blocks, with adapters or without, take c as f32 and add it
+// where a group begins, in the rescale's multiplication (INC below): no extra matrix work.
 #include <type_traits>
 
 #include "device_common.h"
@@ -41,11 +41,6 @@ namespace kiln {
 namespace {
 
 constexpr int kAStages = 4;
-
-__device__ __forceinline__ void store_row_sum(u32x4 *__restrict__ aext, size_t at, float sum, bool plain) {
-    if (plain) reinterpret_cast<float *>(aext)[at] = -kCodeBias * sum;
-    else aext[at] = extension_operand(sum);
-}
 
 // c[m][g] = -136 * sum_{k in group g} a[m][k], group-major ([g][m]), for instances of the kernel that add it at every
 // change of group: as f32 (PLAIN); for the others split into bf16 hi/mid/lo and stored as the 8-slot extension
@@ -64,15 +59,15 @@ __global__ __launch_bounds__(256) void w4a16_prefill_rowsum_kernel(const uint16_
     if (sub == 0) store_row_sum(aext, (size_t)g * M + row, sum, PLAIN);  // group-major: the 32 rows of a half-wavefront are contiguous
 }
 
-template <int RB>
+template <int RB, bool PLAIN>
 __global__ __launch_bounds__(256) void w4a16_lora_project_kernel(const uint16_t *__restrict__ X,
                                                                 const uint16_t *__restrict__ a_cat,
                                                                 uint16_t *__restrict__ T, int M, int K, int r_total,
                                                                 int RP, int steps_per_slice, LoraScales ls,
                                                                 float *partial, int *counters, u32x4 *aext) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-    lora_project_block<RB>(lds, X, a_cat, T, M, K, r_total, RP, steps_per_slice, ls, partial, counters, aext,
-                           blockIdx.x, blockIdx.y, gridDim.y, nullptr);
+    lora_project_block<RB, PLAIN>(lds, X, a_cat, T, M, K, r_total, RP, steps_per_slice, ls, partial, counters, aext,
+                                  blockIdx.x, blockIdx.y, gridDim.y, nullptr);
 }
 
 typedef __attribute__((address_space(3))) void *lds_ptr_t;
@@ -293,8 +288,9 @@ __device__ __forceinline__ void prefill_fold_done(const PrefillFold &pf, int con
 // by scale(g) / scale(g+1) becomes a multiply-add, and there is no extension contraction (6 % of the products at any
 // K, and 2 us a tile).  What it costs is LDS reads: a lane's accumulators lie in 16 rows of every row tile, whose
 // values of c it reads (broadcast) in 16-byte pieces, 16 of them a group beside 32 fragments.  For launches of several
-// rounds, whose row sums come from in front anyway; where the launch's own blocks form them (FOLD, RS) they are not there
-// when a block begins.
+// rounds, whose row sums come from in front anyway; where the launch's own blocks form them (RS, and FOLD's producers
+// without INC) they are not there when a block begins.  FOLD and INC together: the producers run the projection onto the
+// adapters alone.
 template <int NWN, int WM, int MI, bool SWIGLU, bool RS, bool FOLD = false, bool INC = false>
 __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void w4a16_prefill_kernel(
     const uint16_t *__restrict__ A, const u32x4 *__restrict__ B, const uint16_t *__restrict__ S,
@@ -303,7 +299,7 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
     int KS, int GSb, float *partial, int *counters, int die_rows, u32x4 *next_aext, bool next_plain, PrefillFold pf) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];  // the A ring; reused by the store
     static_assert(!FOLD || WM * NWN == 4, "the projection's blocks have four wavefronts");
-    static_assert(!INC || (!FOLD && !RS && WM == 1 && NWN == 4 && MI == 4), "the row sums come from in front");
+    static_assert(!INC || (!RS && WM == 1 && NWN == 4 && MI == 4), "the row sums come from in front");
     if constexpr (FOLD) {
         if ((int)blockIdx.x < pf.producers) {
             const int unit = blockIdx.x;
@@ -642,9 +638,9 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
                 if constexpr (mi == 0) {
                     // Loads complete in issue order; behind the next stage's there are those of the two stages after
                     // it (in the last group extension stages take the place of stages) and, unless they are needed now,
-                    // the next group's six.
+                    // the next group's six, its c and the look at the words.
                     constexpr int a_behind = LAST && q > 0 ? (q == 1 ? 1 : 0) : 2;
-                    constexpr int others = (!LAST && (q == 1 || q == 2)) ? 6 + (PEEK || INC ? 1 : 0) : 0;
+                    constexpr int others = (!LAST && (q == 1 || q == 2)) ? 6 + (PEEK ? 1 : 0) + (INC ? 1 : 0) : 0;
                     wait_vector_loads<a_behind * APW + (2 - a_behind) * kExtLoads + others>();
                     wait_lds_reads();
                     __builtin_amdgcn_s_barrier();
@@ -1276,7 +1272,8 @@ static void project_slicing(int m, int k, bool have_counters, int *rb_out, int *
     *per_slice_out = per_slice;
 }
 
-hipError_t launch_lora_project(const PrefillArgs &a, bool few_rows, hipStream_t stream, int *slices, bool with_row_sums) {
+hipError_t launch_lora_project(const PrefillArgs &a, bool few_rows, hipStream_t stream, int *slices, bool with_row_sums,
+                               bool plain_sums) {
     if (a.r_total < 1 || a.r_total > kProjectMaxRank || a.n_adapters < 1 || a.n_adapters > 8 || !a.lora_a ||
         !a.lora_t || !a.ranks || !a.scales || a.M < 1 || a.K < kGroupK)
         return hipErrorInvalidValue;
@@ -1299,17 +1296,16 @@ hipError_t launch_lora_project(const PrefillArgs &a, bool few_rows, hipStream_t 
         project_slicing(a.M, a.K, a.counters != nullptr, &rb, &row_tiles, &kz, &per_slice);
         float *partial = reinterpret_cast<float *>(reinterpret_cast<char *>(a.lora_t) + (size_t)a.M * 64 * sizeof(uint16_t));
         const int lds_bytes = (rb + kProjectMaxRank) * kProjectRowBytes + kProjectMaxRank * (int)sizeof(float);
-        if (rb == 16) {
-            w4a16_lora_project_kernel<16><<<dim3(row_tiles, kz), 256, lds_bytes, stream>>>(
-                (const uint16_t *)a.A, (const uint16_t *)a.lora_a, (uint16_t *)a.lora_t, a.M, a.K, a.r_total, RP,
-                per_slice, ls, partial, a.counters, aext);
-        } else {
-            const hipError_t attr = allow_dynamic_lds<&w4a16_lora_project_kernel<64>>(lds_bytes);
+        const auto kernel = rb == 16 ? (plain_sums ? &w4a16_lora_project_kernel<16, true> : &w4a16_lora_project_kernel<16, false>)
+                                     : (plain_sums ? &w4a16_lora_project_kernel<64, true> : &w4a16_lora_project_kernel<64, false>);
+        if (rb == 64) {
+            const hipError_t attr = plain_sums ? allow_dynamic_lds<&w4a16_lora_project_kernel<64, true>>(lds_bytes)
+                                               : allow_dynamic_lds<&w4a16_lora_project_kernel<64, false>>(lds_bytes);
             if (attr != hipSuccess) return attr;
-            w4a16_lora_project_kernel<64><<<dim3(row_tiles, kz), 256, lds_bytes, stream>>>(
-                (const uint16_t *)a.A, (const uint16_t *)a.lora_a, (uint16_t *)a.lora_t, a.M, a.K, a.r_total, RP,
-                per_slice, ls, partial, a.counters, aext);
         }
+        kernel<<<dim3(row_tiles, kz), 256, lds_bytes, stream>>>(
+            (const uint16_t *)a.A, (const uint16_t *)a.lora_a, (uint16_t *)a.lora_t, a.M, a.K, a.r_total, RP, per_slice, ls, partial,
+            a.counters, aext);
         return hipGetLastError();
     }
     int kz = lora_project_slices(a.M, a.K);
@@ -1317,7 +1313,7 @@ hipError_t launch_lora_project(const PrefillArgs &a, bool few_rows, hipStream_t 
     kz = (steps + per_slice - 1) / per_slice;
     *slices = kz;
     const int lds_bytes = (16 + kProjectMaxRank) * kProjectRowBytes + kProjectMaxRank * (int)sizeof(float);
-    w4a16_lora_project_kernel<16><<<dim3((a.M + 15) / 16, kz), 256, lds_bytes, stream>>>(
+    w4a16_lora_project_kernel<16, false><<<dim3((a.M + 15) / 16, kz), 256, lds_bytes, stream>>>(
         (const uint16_t *)a.A, (const uint16_t *)a.lora_a, (uint16_t *)a.lora_t, a.M, a.K, a.r_total, RP, per_slice, ls,
         nullptr, nullptr, nullptr);
     return hipGetLastError();
@@ -1357,14 +1353,17 @@ int prefill_rowsum_producers(int M, int N, int K, const PrefillPlan &p, int cus)
     return producers < 128 ? producers : 128;
 }
 
-// Where the row sums are added at the groups' changes (INC): plain calls in 128-row blocks whose row sums
-// prefill_rowsum_producers() leaves to a launch in front.  By the shape alone, since the two routes of a shape's row
-// sums must agree in every bit; and not for calls with overrides (PrefillArgs::plan_forced), whose block shapes
-// must.  64-row blocks keep the extension contraction: their plain calls equal those with adapters of zeros, and a
-// launch that runs the projection has no row sums to begin with.
+// Where the row sums are added at the groups' changes (INC): 128-row blocks whose row sums prefill_rowsum_producers()
+// leaves to a launch in front, with adapters and without.  By the shape alone, since the two routes of a shape's row
+// sums must agree in every bit, and a call with adapters of zeros must equal the plain call; not for calls with overrides
+// (PrefillArgs::plan_forced), which agree among each other in every bit over the block widths, and so not with an
+// automatic call that comes here.  64-row blocks keep the extension contraction.
 // (2560 -> 2 x 9216 -> 2560 at 8192 rows 933 -> 912 us, at 2048 rows 269 -> 260, error beyond the bf16 rounding 2.1e-4 -> 0.9e-4
 // of the result's norm, 1.1e-3 -> 2.2e-4 where the activations have a mean of half their deviation: the surplus leaves group by
-// group instead of piling up in the accumulators.)
+// group instead of piling up in the accumulators.  With two adapters, the projection inside the launch and the sums from the
+// pre-pass kernel: 2560 -> 18432 at 1024 / 2048 / 4096 / 8192 rows 97.7 -> 98.3, 173.8 -> 172.8, 334 -> 327, 661 -> 650 us, error
+// 1.6e-4 -> 0.7e-4; both from a launch in front: 101.6 at 1024 rows, 174.5 at 2048 where inside took 170.4.  Where the
+// projection takes 64 rows a block, or finds no slots, it is in front and writes the sums: 9216 -> 2560 at 4096 rows 207 -> 200.)
 bool prefill_adds_sums_in_loop(int M, int N, int K, const PrefillPlan &p, int cus) {
     return p.bn == 256 && p.bm == 128 && prefill_rowsum_producers(M, N, K, p, cus) == 0;
 }
@@ -1383,19 +1382,10 @@ hipError_t launch_prefill(const PrefillArgs &a, hipStream_t stream) {
     const int max_groups = a.nb_full > 0 ? G : (G + KS_ - 1) / KS_;
     const bool rs = blocks_sum_their_rows(a.M, a.N, a.K, shape);
     hipError_t err = hipSuccess;
-    // with adapters the projection's launch forms the row sums on its way over x
-    const bool sums_with_projection = !rs && a.r_total > 0;
     if (a.next_aext && !prefill_forms_next_sums(shape)) return hipErrorInvalidValue;
-    const bool inc = a.r_total == 0 && !a.plan_forced && prefill_adds_sums_in_loop(a.M, a.N, a.K, shape, a.cus);
+    const bool inc = !a.plan_forced && prefill_adds_sums_in_loop(a.M, a.N, a.K, shape, a.cus);
     const int inside = a.r_total == 0 && a.lora_words && !a.aext_ready ? prefill_rowsum_producers(a.M, a.N, a.K, shape, a.cus) : 0;
     const int sum_producers = inside > 0 ? inside : 0;
-    if (!rs && !sums_with_projection && sum_producers == 0 && !a.aext_ready) {
-        const int items = a.M * G;
-        (inc ? w4a16_prefill_rowsum_kernel<true> : w4a16_prefill_rowsum_kernel<false>)<<<(items + 15) / 16, 256, 0, stream>>>(
-            (const uint16_t *)a.A, (u32x4 *)a.aext, a.M, a.K);
-        err = hipGetLastError();
-        if (err != hipSuccess) return err;
-    }
     int RP = 0;
     // The projection inside the product's launch (PrefillFold): four-wavefront blocks, 16-row tiles of T,
     // the extension operand from the projection (unless the blocks sum their rows themselves), and room
@@ -1436,7 +1426,9 @@ hipError_t launch_prefill(const PrefillArgs &a, hipStream_t stream) {
         if (fold) {
             pf.a_cat = (const uint16_t *)a.lora_a;
             pf.t = (uint16_t *)a.lora_t;
-            pf.aext = rs ? nullptr : (u32x4 *)a.aext;  // blocks that sum their rows themselves need no operand
+            // blocks that sum their rows themselves need no operand, and with INC the sums have to be there
+            // before a block begins
+            pf.aext = rs || inc ? nullptr : (u32x4 *)a.aext;
             pf.partial = reinterpret_cast<float *>(reinterpret_cast<char *>(a.lora_t) + (size_t)a.M * 64 * sizeof(uint16_t));
             pf.counters = a.counters + kProjectFoldCounters;
             pf.words = a.lora_words;
@@ -1453,10 +1445,18 @@ hipError_t launch_prefill(const PrefillArgs &a, hipStream_t stream) {
             }
         } else {
             int slices = 1;  // many rows: T is whole
-            err = launch_lora_project(a, false, stream, &slices, sums_with_projection);
+            err = launch_lora_project(a, false, stream, &slices, !rs, inc);
             if (err != hipSuccess) return err;
             if (slices != 1) return hipErrorInvalidValue;
         }
+    }
+    // with adapters the projection forms the row sums on its way over x, but for INC's where it runs inside the launch
+    if (!rs && sum_producers == 0 && !a.aext_ready && (a.r_total == 0 || (inc && fold))) {
+        const int items = a.M * G;
+        (inc ? w4a16_prefill_rowsum_kernel<true> : w4a16_prefill_rowsum_kernel<false>)<<<(items + 15) / 16, 256, 0, stream>>>(
+            (const uint16_t *)a.A, (u32x4 *)a.aext, a.M, a.K);
+        err = hipGetLastError();
+        if (err != hipSuccess) return err;
     }
     if (sum_producers > 0) {
         fold = true;
@@ -1475,6 +1475,9 @@ hipError_t launch_prefill(const PrefillArgs &a, hipStream_t stream) {
     const int grid = prefill_grid(a.M, a.N, shape);
     if (fold) {
         pf.consumers = grid;
+        if (inc)
+            return a.swiglu ? launch_shape_as<4, 1, 4, true, false, true, true>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream, pf)
+                            : launch_shape_as<4, 1, 4, false, false, true, true>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream, pf);
         if (a.swiglu) {
             if (a.bm == 128) return launch_shape_as<4, 1, 4, true, false, true>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream, pf);
             return rs ? launch_shape_as<4, 1, 2, true, true, true>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream, pf)
