@@ -181,11 +181,11 @@ struct PrefillArgs {
     int *counters = nullptr;        // one per 256 x 128 tile, zero on entry and on exit
     unsigned *lora_words = nullptr; // 64 KiB that are zero between launches (see lora_tail.h): with them the LoRA
                                     // projection may run inside the product's launch; null: always in front of it
-    bool plan_forced = false;       // the caller's thread_k / thread_n chose the plan
+    bool sums_in_loop = false;      // prefill_adds_sums_in_loop() of the automatic plan; 128-row blocks of either width
     bool aext_ready = false;        // no adapters: `aext` was written by the launch that wrote A (its next_aext)
     void *next_aext = nullptr;      // swiglu, prefill_forms_next_sums(): prefill_aext_bytes(M, N / 2) bytes, the row sums
                                     // of C for a GEMM over it
-    bool next_plain = false;        // ... in the form that GEMM takes: prefill_adds_sums_in_loop()
+    bool next_plain = false;        // ... in the form that GEMM takes: its sums_in_loop
 };
 
 size_t prefill_aext_bytes(int m, int k);
@@ -202,7 +202,7 @@ PrefillPlan plan_prefill(int m, int n, int k, int cus, int force_bn = 0, int for
 int prefill_grid(int m, int n, const PrefillPlan &p);
 size_t prefill_partial_bytes(int m, int n, const PrefillPlan &p);
 int prefill_rowsum_producers(int m, int n, int k, const PrefillPlan &p, int cus);  // blocks of a plain launch that form the row sums inside it (0: a launch in front does, -2: every block its own)
-bool prefill_adds_sums_in_loop(int m, int n, int k, const PrefillPlan &p, int cus);  // the launch's row sums: f32 [K/128][M]
+bool prefill_adds_sums_in_loop(int m, int n, int k, const PrefillPlan &p, int cus);  // row sums as f32 [K/128][M], added at the changes of group
 bool prefill_forms_next_sums(const PrefillPlan &p);                             // can its swiglu launch write next_aext?
 bool prefill_reads_row_sums(int m, int n, int k, const PrefillPlan &p);         // ... a plain launch take it as aext?
 hipError_t launch_prefill(const PrefillArgs &args, hipStream_t stream);
@@ -211,6 +211,6 @@ hipError_t launch_prefill(const PrefillArgs &args, hipStream_t stream);
 // prefill_lora_max_slices(M) slices; otherwise one slice.
 hipError_t launch_lora_project(const PrefillArgs &args, bool few_rows, hipStream_t stream, int *slices,
                                bool with_row_sums = false,  // many rows: also write the product's row sums (args.aext),
-                               bool plain_sums = false);    // in the form of prefill_adds_sums_in_loop()
+                               bool plain_sums = false);    // in the form sums_in_loop takes
 
 }  // namespace kiln

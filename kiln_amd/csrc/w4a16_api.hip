@@ -441,6 +441,7 @@ struct MidPlan {
 struct GemmPlan {
     bool prefill = false;
     PrefillPlan pf{};
+    bool sums_in_loop = false;  // PrefillArgs::sums_in_loop
     bool mid = false;
     MidPlan mp{};
     int launches = 0;
@@ -471,6 +472,9 @@ void plan_as_prefill(int m, int n, int k, int cus, int thread_k, int thread_n, G
     gp->launches = 0;
     gp->decode_partial = 0;
     PrefillPlan p = planned_prefill(m, n, k, cus);
+    // (asked of the automatic plan: an override that changes nothing gives the automatic call's bits, and the block
+    // widths agree in every bit)
+    gp->sums_in_loop = prefill_adds_sums_in_loop(m, n, k, p, cus);
     if ((thread_n == 128 || thread_n == 256) && thread_n != p.bn) {  // block columns: whole tiles only
         p.bn = thread_n;
         p.nb_full = n / thread_n;
@@ -906,7 +910,7 @@ struct MlpSums {
 };
 bool mlp_passes_row_sums(int m, int hidden, int n_out, int n_down, int cus, bool *plain) {
     const auto gate_up = plan_call(m, 2 * n_out, hidden, cus, -1, -1, 0), down = plan_call(m, n_down, n_out, cus, -1, -1, 0);
-    *plain = down->gp.prefill && prefill_adds_sums_in_loop(m, n_down, n_out, down->gp.pf, cus);
+    *plain = down->gp.sums_in_loop;
     return gate_up->gp.prefill && prefill_forms_next_sums(gate_up->gp.pf) && down->gp.prefill &&
            prefill_reads_row_sums(m, n_down, n_out, down->gp.pf);
 }
@@ -959,7 +963,7 @@ kiln_marlin_status_t gemm_any(const void *A, const void *B, void *C, const void 
         } else if (g_tune.rowsum_fold != 0) {
             pa.lora_words = reinterpret_cast<unsigned *>(ws + kFoldFlagOffset);
         }
-        pa.plan_forced = thread_k > 0 || thread_n > 0;
+        pa.sums_in_loop = gp.sums_in_loop;
         pa.swiglu = swiglu;
         pa.next_aext = sums.write;
         pa.next_plain = sums.write_plain;

@@ -299,7 +299,7 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
     int KS, int GSb, float *partial, int *counters, int die_rows, u32x4 *next_aext, bool next_plain, PrefillFold pf) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];  // the A ring; reused by the store
     static_assert(!FOLD || WM * NWN == 4, "the projection's blocks have four wavefronts");
-    static_assert(!INC || (!RS && WM == 1 && NWN == 4 && MI == 4), "the row sums come from in front");
+    static_assert(!INC || (!RS && WM == 1 && MI == 4), "the row sums come from in front");
     if constexpr (FOLD) {
         if ((int)blockIdx.x < pf.producers) {
             const int unit = blockIdx.x;
@@ -1355,9 +1355,9 @@ int prefill_rowsum_producers(int M, int N, int K, const PrefillPlan &p, int cus)
 
 // Where the row sums are added at the groups' changes (INC): 128-row blocks whose row sums prefill_rowsum_producers()
 // leaves to a launch in front, with adapters and without.  By the shape alone, since the two routes of a shape's row
-// sums must agree in every bit, and a call with adapters of zeros must equal the plain call; not for calls with overrides
-// (PrefillArgs::plan_forced), which agree among each other in every bit over the block widths, and so not with an
-// automatic call that comes here.  64-row blocks keep the extension contraction.
+// sums must agree in every bit, and a call with adapters of zeros must equal the plain call.  Calls with overrides follow the
+// automatic plan of their shape, also where they name blocks of 128 columns: the widths agree in every bit, and an override
+// that changes nothing gives the automatic call's bits.  64-row blocks keep the extension contraction.
 // (2560 -> 2 x 9216 -> 2560 at 8192 rows 933 -> 912 us, at 2048 rows 269 -> 260, error beyond the bf16 rounding 2.1e-4 -> 0.9e-4
 // of the result's norm, 1.1e-3 -> 2.2e-4 where the activations have a mean of half their deviation: the surplus leaves group by
 // group instead of piling up in the accumulators.  With two adapters, the projection inside the launch and the sums from the
@@ -1383,8 +1383,9 @@ hipError_t launch_prefill(const PrefillArgs &a, hipStream_t stream) {
     const bool rs = blocks_sum_their_rows(a.M, a.N, a.K, shape);
     hipError_t err = hipSuccess;
     if (a.next_aext && !prefill_forms_next_sums(shape)) return hipErrorInvalidValue;
-    const bool inc = !a.plan_forced && prefill_adds_sums_in_loop(a.M, a.N, a.K, shape, a.cus);
-    const int inside = a.r_total == 0 && a.lora_words && !a.aext_ready ? prefill_rowsum_producers(a.M, a.N, a.K, shape, a.cus) : 0;
+    const bool inc = a.sums_in_loop;
+    if (inc && a.bm != 128) return hipErrorInvalidValue;
+    const int inside = a.r_total == 0 && a.lora_words && !a.aext_ready && !inc ? prefill_rowsum_producers(a.M, a.N, a.K, shape, a.cus) : 0;
     const int sum_producers = inside > 0 ? inside : 0;
     int RP = 0;
     // The projection inside the product's launch (PrefillFold): four-wavefront blocks, 16-row tiles of T,
@@ -1486,6 +1487,10 @@ hipError_t launch_prefill(const PrefillArgs &a, hipStream_t stream) {
         if (a.bm == 128) return launch_shape_as<4, 1, 4, false, false, true>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream, pf);
         return rs ? launch_shape_as<4, 1, 2, false, true, true>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream, pf)
                   : launch_shape_as<4, 1, 2, false, false, true>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream, pf);
+    }
+    if (inc && a.bn == 128) {  // through overrides only, which the fused calls do not take
+        if (a.swiglu) return hipErrorInvalidValue;
+        return launch_shape_as<2, 1, 4, false, false, false, true>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream);
     }
     if (inc) {
         return a.swiglu ? launch_shape_as<4, 1, 4, true, false, false, true>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream)
