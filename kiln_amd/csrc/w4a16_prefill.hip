@@ -1105,8 +1105,10 @@ static PrefillPlan plan_for_shape(int m, int n, int k, int cus, int bn, int bm, 
 // slice, and its launch carries 6 units more (the row sums from a launch in front, a longer prologue and
 // store): fitted to 98 cases -- 14 shapes at 400 ... 4096 rows, each with 64- and 128-row blocks forced --
 // and to 72 more -- 12 shapes of other models at 129 ... 512 rows, the three block shapes forced -- on which
-// the cheaper plan by this cost is the faster one or within 0.8 % (the former) and 0.6 % (the latter) of it
-// on average, 18 % and 5 % at worst.
+// the cheaper plan by this cost was the faster one or within 0.8 % (the former) and 0.6 % (the latter) of it
+// on average, 18 % and 5 % at worst.  That was before the main loop was ordered by hand; on the kernel as it is, 88
+// cases -- eight shapes at 200 ... 2048 rows, both heights forced -- are 2.4 % off on average and 32 % at worst
+// (4096 -> 12288 at 420 rows: 62 us in 128-row blocks and two slices, 47 in 64-row ones).
 static float plan_cost(int m, int n, int k, int cus, const PrefillPlan &p) {
     const int G = k / kGroupK, m_blocks = (m + p.bm - 1) / p.bm, n_blocks = n / p.bn;
     const float rows = p.bm == 128 ? 1.5f : 1.0f;

@@ -74,7 +74,12 @@ class PackEntry:
 @dataclass
 class LayerProjections:
     """One layer's projections: `weights_t[kind]` is the pre-transposed `[k, n]` bf16 weight (the
-    reference's `*_proj_t`), `packed[kind]` the installed packed weight (its `*_proj_marlin`)."""
+    reference's `*_proj_t`), `packed[kind]` the installed packed weight (its `*_proj_marlin`).
+
+    After `pack_layers(..., fuse_same_input_groups=True)` a side-by-side pack and its members share one storage: the
+    members' `b_packed` / `scales` are pieces of it.  Writing one in place changes the other, the storage is freed when the
+    last of them is dropped, and `torch.save` of a member writes the whole run (`marlin_proj.save` writes the member
+    alone).  Clone a member's tensors to have it by itself."""
     weights_t: Dict[PackKind, Optional[torch.Tensor]]
     packed: Dict[PackKind, MarlinPackedProj] = field(default_factory=dict)
     gate_up_fused: Optional[MarlinPackedProj] = None   # gate and up interleaved for the SwiGLU entry point

@@ -268,11 +268,13 @@ def pack_from_gptq(qweight: torch.Tensor, scales: torch.Tensor, qzeros: Optional
     return _wrap_native(out.value, device)
 
 
-# Host tensors go to the device through pinned memory of torch's pool, at most this much at a time ...
+# Host tensors go to the device through pinned memory of torch's host cache, at most this much at a time (the cache keeps it for
+# the process; the first load pays for registering it, 15 ms with the first use of the kernels, the next ones 0.7 and 0.4 ms) ...
 _STAGE_BYTES = 32 << 20
 # ... the first copy a short one, so that the link is busy while the rest is still being moved into the pinned
 # memory (12 MiB: 229 us from pinned memory alone, 248 in pieces of 2 and 10 MiB, 253 in one, 260 to 340 in
-# three or more, 354 as the runtime's own pageable copy)
+# three or more, 354 as the runtime's own pageable copy; a whole load of 12 MiB 292 us against 313 as one piece, of 0.5, 3,
+# 28, 56 and 112 MiB level with one piece)
 _FIRST_PIECE_BYTES = 2 << 20
 
 
