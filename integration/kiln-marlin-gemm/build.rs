@@ -40,7 +40,9 @@ fn main() {
             c.arg(format!("--offload-arch={arch}"))
                 .args(["-O3", "-std=c++17", "-fPIC", "-c"])
                 // packed-f32 VALU instructions are switched off for all device code
-                .args(["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]);
+                .args(["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"])
+                // leading kernel arguments in scalar registers before a wavefront starts
+                .arg("-mllvm=-amdgpu-kernarg-preload-count=16");
             c
         };
         cmd.arg(format!("-I{}", include.display()));

@@ -158,12 +158,27 @@ struct GmpKernelArgs {
     const uint16_t *A;
     const u32x4 *B;
     const uint16_t *S;
+    uint32_t shape, layout;
+    int G, NT, GS, col_blocks;
     uint16_t *C;
     float *partial;
     int *counters;
-    int M, N, K, Gs, KS, GS, full_waves, slot_bytes, col_shift, producers, adapter, col_blocks, nw_all, swiglu, flagged;
     GmpLoraArgs la;
 };
+// `shape` and `layout`: small values that share a word each, so that everything up to C is fourteen words -- as many
+// arguments as a wavefront can find in its scalar registers when it starts (-amdgpu-kernarg-preload-count).  What bounds
+// these launches is a chain of latencies, and it used to begin with a fetch of the arguments (0.2 us), a division for the
+// column block and 64-bit products for every chunk's address, ~130 scalar instructions ahead of the first weight request
+// where ~60 are left.  Measured (16 rows, 2560 / 9216 wide, same box): an MLP as one call 14.64 -> 13.98 us, sixteen
+// launches of a replayed decode step 110.7 -> 106.4 us.
+constexpr uint32_t gmp_shape_word(int M, int full_waves, int nw_all, int KS) {
+    return (uint32_t)M | (uint32_t)full_waves << 8 | (uint32_t)nw_all << 16 | (uint32_t)KS << 24;
+}
+constexpr uint32_t kGmpColumnScales = 1u << 24, kGmpColShift = 1u << 25, kGmpAdapter = 1u << 26, kGmpSwiglu = 1u << 27,
+                   kGmpFlagged = 1u << 28;
+constexpr uint32_t gmp_layout_word(int slot_bytes, int producers, uint32_t bits) {
+    return (uint32_t)slot_bytes | (uint32_t)producers << 16 | bits;
+}
 constexpr int kGmpLoraArgsOffset = (int)offsetof(GmpKernelArgs, la);
 static_assert(sizeof(GmpLoraArgs) % 4 == 0, "read word by word");
 
@@ -174,7 +189,7 @@ struct GmpTailArgs {
     uint16_t *C;
     float *partial;
     int *counters;
-    int swiglu, flagged;
+    uint32_t shape, layout;
 };
 struct GmpParkedTail {
     uint32_t w[8];
@@ -203,23 +218,19 @@ static_assert(sizeof(GmpTailArgs) == 32, "eight words");
 // only; the other rows of the product are computed from whatever LDS holds and never stored).
 template <int T, int GPW, int AQ, bool LORA>
 __global__ __launch_bounds__(kGmpMaxWaves * 64) void w4a16_decode_gmp_kernel(
-    const uint16_t *__restrict__ A, const u32x4 *__restrict__ B, const uint16_t *__restrict__ S,
-    uint16_t *__restrict__ C_arg, float *partial_arg, int *counters_arg, int M, int N, int K, int Gs, int KS, int GS,
-    int full_waves, int slot_bytes, int col_shift, int producers_arg, int adapter_arg, int col_blocks, int nw_all,
-    int swiglu_arg, int flagged_arg, GmpLoraArgs la) {
-    const int producers = LORA ? producers_arg : 0, adapter = LORA ? adapter_arg : 0;
+    const uint16_t *__restrict__ A, const u32x4 *__restrict__ B, const uint16_t *__restrict__ S, uint32_t shape,
+    uint32_t layout, int G, int NT, int GS, int col_blocks, uint16_t *__restrict__ C_arg, float *partial_arg,
+    int *counters_arg, GmpLoraArgs la) {
+    const int M = shape & 255, full_waves = (shape >> 8) & 255, nw_all = (shape >> 16) & 255, KS = shape >> 24;
+    const int slot_bytes = layout & 0xFFFF;
+    const int producers = LORA ? (layout >> 16) & 255 : 0, adapter = LORA && (layout & kGmpAdapter) ? 1 : 0;
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
 #ifdef KILN_GMP_TIMELINE
     long long tl_[8] = {};
 #endif
     KILN_GMP_TL(0, KILN_GMP_NOW());
-    // Everything the first requests depend on is fetched from the kernel arguments in one go: left to
-    // itself the compiler fetches what lies behind the branch below only there, one more scalar
-    // round trip (0.2 us) between the launch and the first weight request.
-    asm volatile("" : : "s"(A), "s"(B), "s"(S), "s"(M), "s"(N), "s"(K), "s"(Gs), "s"(KS), "s"(GS), "s"(full_waves),
-                 "s"(slot_bytes), "s"(col_shift), "s"(producers), "s"(adapter), "s"(col_blocks), "s"(nw_all));
     [[maybe_unused]] GmpParkedTail parked_tail;
-    if constexpr (LORA) parked_tail = gmp_park(GmpTailArgs{C_arg, partial_arg, counters_arg, swiglu_arg, flagged_arg});
+    if constexpr (LORA) parked_tail = gmp_park(GmpTailArgs{C_arg, partial_arg, counters_arg, shape, layout});
     constexpr int NS = gmp_slots(GPW);
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -227,9 +238,7 @@ __global__ __launch_bounds__(kGmpMaxWaves * 64) void w4a16_decode_gmp_kernel(
     // With adapters the block has one wavefront more than the main loop uses: it fetches what the
     // low-rank term needs into LDS while the others stream weights.
     const int nw = nw_all - adapter;  // nw_all = wavefronts of the block
-    const bool adapter_wave = wave == nw;  // never true without adapters
-    const int G = K / kGroupK;
-    const int NT = N / kTileN;
+    const bool adapter_wave = LORA && wave == nw;
     // Calls without a folded projection: grid (column blocks, K slices).  With one, a single row
     // of blocks: the `producers` blocks that compute it first, then the slices one after the other
     // (a second grid dimension would launch the producers' indices once per slice, and the idle
@@ -237,7 +246,7 @@ __global__ __launch_bounds__(kGmpMaxWaves * 64) void w4a16_decode_gmp_kernel(
     int ks = blockIdx.y, bx = blockIdx.x;
     if (__builtin_expect(producers > 0, 0)) {
         if (bx < producers) {
-            lora_project_slice(A, la.fold, la.lo, M, K, bx, lds, wave, lane, nw_all);
+            lora_project_slice(A, la.fold, la.lo, M, G * kGroupK, bx, lds, wave, lane, nw_all);
 #ifdef KILN_GMP_TIMELINE
             if (lane == 0 && g_gmp_tl) {
                 long long *o = g_gmp_tl + ((size_t)blockIdx.x * 16 + wave) * 8;
@@ -256,12 +265,12 @@ __global__ __launch_bounds__(kGmpMaxWaves * 64) void w4a16_decode_gmp_kernel(
     // column block is shifted by col_shift per slice, so that the slices of a tile sit on different
     // dies: a device-scope store and the device-scope load that polls it are slow when they meet
     // in one die's L2 (measured: 2...3 us per poll instead of 0.5).
-    const int col_block = (bx + ks * col_shift) % col_blocks;
+    int col_block = bx + ((layout & kGmpColShift) ? ks : 0);
+    if (col_block >= col_blocks) col_block -= col_blocks;  // at most three past the end, of sixteen tiles or more
     const int tf = col_block * T;  // first tile of the block; tiles from NT on do not exist
     const bool full = wave < full_waves;
     const int g_first = full ? wave * GPW : full_waves * GPW + (wave - full_waves) * (GPW - 1);
     const int g0 = ks * GS + g_first;  // all slices have GS groups
-    const int gs_mask = (Gs == 1) ? 0 : -1;
 
     // chunk j of the wavefront = (group j / T, tile j % T); a tile past the end is read as the last
     // tile and never stored.  Four register sets rotate.
@@ -269,14 +278,19 @@ __global__ __launch_bounds__(kGmpMaxWaves * 64) void w4a16_decode_gmp_kernel(
     uint32_t sc[kGmpHead + 1];
     static_assert(2 * kGmpHead + 8 <= 63, "outstanding loads must fit the wait counter");
     const uint32_t b_lane = lane * 16, s_lane = (lane & 15) * 2;
+    // one 64-bit address per operand, 32-bit distances from it
+    const bool column_scales = (layout & kGmpColumnScales) != 0;
+    const uint32_t scale_groups = column_scales ? 1u : (uint32_t)G;
+    const int last_tile = NT - 1 - tf;
+    const char *const b_first = reinterpret_cast<const char *>(B) + (size_t)((uint32_t)tf * (uint32_t)G + (uint32_t)g0) * 1024;
+    const char *const s_first = reinterpret_cast<const char *>(S) +
+                                (size_t)((uint32_t)tf * scale_groups + (column_scales ? 0u : (uint32_t)g0)) * (kTileN * 2);
     auto request_chunk = [&](auto jc) {
         constexpr int j = decltype(jc)::value;
         constexpr int gi = j / T, ti = j % T, set = j % (kGmpHead + 1);
-        const int tt = min(tf + ti, NT - 1);
-        const char *b_ptr = reinterpret_cast<const char *>(B) + ((size_t)tt * G + (g0 + gi)) * 1024;
-        const char *s_ptr = reinterpret_cast<const char *>(S) + ((size_t)tt * Gs + ((g0 + gi) & gs_mask)) * (kTileN * 2);
-        load_b128_streaming(w[set], b_ptr, b_lane);
-        load_u16(sc[set], s_ptr, s_lane);
+        const uint32_t tile = min(ti, last_tile);
+        load_b128_streaming(w[set], b_first + (tile * (uint32_t)G + gi) * 1024u, b_lane);
+        load_u16(sc[set], s_first + (tile * scale_groups + (column_scales ? 0u : gi)) * (kTileN * 2u), s_lane);
     };
 
     // A of one group: AQ loads of 4 rows x 256 bytes; lane i of load p fetches 16-byte unit
@@ -284,7 +298,7 @@ __global__ __launch_bounds__(kGmpMaxWaves * 64) void w4a16_decode_gmp_kernel(
     // and the 16 lanes that read one unit index of 16 rows hit 16 different positions.
     unsigned char *mine = lds + wave * slot_bytes;
     const unsigned mine_addr = (unsigned)(size_t)(lds_ptr_t)mine;
-    const uint32_t row_pitch = (uint32_t)K * 2;
+    const uint32_t row_pitch = (uint32_t)G * (kGroupK * 2);
     auto request_a = [&](int gi, int slot) {
         const char *base = reinterpret_cast<const char *>(A) + (size_t)(g0 + gi) * 256;
         const uint32_t quad_row = (uint32_t)(lane >> 4) + opaque_zero();  // keeps the offsets local to this request
@@ -452,12 +466,12 @@ __global__ __launch_bounds__(kGmpMaxWaves * 64) void w4a16_decode_gmp_kernel(
         return;
     }
 
-    GmpTailArgs tail{C_arg, partial_arg, counters_arg, swiglu_arg, flagged_arg};
+    GmpTailArgs tail{C_arg, partial_arg, counters_arg, shape, layout};
     if constexpr (LORA) tail = gmp_unpark(parked_tail);
     uint16_t *const C = tail.C;
     float *const partial = tail.partial;
     int *const counters = tail.counters;
-    const int swiglu = tail.swiglu, flagged = tail.flagged;
+    const bool swiglu = (tail.layout & kGmpSwiglu) != 0, flagged = (tail.layout & kGmpFlagged) != 0;
     const int q4 = lane >> 4, c = lane & 15;
     const int tiles = min(T, NT - tf);
     if constexpr (LORA) {
@@ -563,7 +577,7 @@ __global__ __launch_bounds__(kGmpMaxWaves * 64) void w4a16_decode_gmp_kernel(
             lds_signal_wait(lora_ready_addr(), kGmpOperandsReady);  // the term's operands are in LDS
             lora_add_from_lds(sum, lo, lora_t_lds, lora_b_lds, ti, M, lane);
         }
-        store_tile_rows(C, N, M, 4 * q4, tt, c, sum, swiglu != 0);
+        store_tile_rows(C, NT * kTileN, M, 4 * q4, tt, c, sum, swiglu);
     }
 #ifdef KILN_GMP_TIMELINE
     tl_[6] = KILN_GMP_NOW();
@@ -614,10 +628,12 @@ hipError_t launch_gmp_tga(const DecodeArgs &a, hipStream_t stream) {
     const dim3 grid = fold.producers > 0 ? dim3(fold.producers + col_blocks * a.KS, 1) : dim3(col_blocks, a.KS);
     const int adapter = a.r_total > 0 ? 1 : 0;  // one wavefront more: it fetches the low-rank term's operands
     const size_t lds_bytes = (size_t)a.waves * slot + gmp_adapter_lds_bytes(a);
+    const uint32_t bits = (a.Gs == 1 ? kGmpColumnScales : 0u) | (adapter ? kGmpAdapter : 0u) | (a.swiglu ? kGmpSwiglu : 0u) |
+                          (a.flagged ? kGmpFlagged | (exchange_column_shift(col_blocks) ? kGmpColShift : 0u) : 0u);
     w4a16_decode_gmp_kernel<T, GPW, AQ, kGmpLora><<<grid, (a.waves + adapter) * 64, lds_bytes, stream>>>(
-        (const uint16_t *)a.A, (const u32x4 *)a.B, (const uint16_t *)a.S, (uint16_t *)a.C, a.partial, a.counters, a.M,
-        a.N, a.K, a.Gs, a.KS, a.GS, full_waves, slot, a.flagged ? exchange_column_shift(col_blocks) : 0, fold.producers,
-        adapter, col_blocks, a.waves + adapter, a.swiglu ? 1 : 0, a.flagged ? 1 : 0, GmpLoraArgs{lora_tail(a), fold});
+        (const uint16_t *)a.A, (const u32x4 *)a.B, (const uint16_t *)a.S,
+        gmp_shape_word(a.M, full_waves, a.waves + adapter, a.KS), gmp_layout_word(slot, fold.producers, bits), a.K / kGroupK,
+        NT, a.GS, col_blocks, (uint16_t *)a.C, a.partial, a.counters, GmpLoraArgs{lora_tail(a), fold});
     return hipGetLastError();
 }
 
@@ -678,7 +694,7 @@ bool decode_gmp_ok(const DecodeArgs &a) {
         if (a.r_total > 64 || a.r_total % 8 != 0 || a.waves + 1 > kGmpMaxWaves) return false;
         if (a.lora_slices < 1 || a.lora_slices > 16 || a.lora_rows != a.M || !a.lora_t || !a.lora_b) return false;
     }
-    if (a.KS < 1 || a.GS < 1 || a.KS * a.GS != G || a.waves < 1 || a.waves > kGmpMaxWaves || a.waves > a.GS) return false;
+    if (a.KS < 1 || a.KS > 255 || a.GS < 1 || a.KS * a.GS != G || a.waves < 1 || a.waves > kGmpMaxWaves || a.waves > a.GS) return false;
     const int gpw = (a.GS + a.waves - 1) / a.waves, T = a.gm_tiles;
     if (gpw > (T <= 2 ? 6 : 3) || T * gpw > kGmpMaxChunks) return false;
     const int full_waves = a.GS - a.waves * (gpw - 1);

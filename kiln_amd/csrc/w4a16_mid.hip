@@ -130,11 +130,29 @@ struct MidLora {
     // rows behind their main loop, count themselves, and the last one zeroes words and counts.
     const uint16_t *a_cat;
     unsigned *words;
-    int producers, row_tiles, steps_per_slice, col_blocks, consumers;
+    int producers, row_tiles, steps_per_slice, consumers;
     LoraScales ls;
 };
 constexpr int kMidFoldTileWord = 32;  // a copy's words start here (the first words are the small-M kernel's)
 constexpr int kMidFoldSpinLimit = 1 << 20;
+
+// The kernel's arguments ahead of C, in fourteen words with it -- as many as a wavefront can find in its scalar
+// registers when it starts (-amdgpu-kernarg-preload-count): everything the first requests depend on.  `slices` and
+// `layout` hold small values that share a word.  With the division for the column block and the 64-bit products for
+// the addresses gone too, the first requests leave 0.3 us earlier (eight launches of 50 rows, two layers' linears on
+// per-column scales: 92.4 -> 89.4 us).
+struct MidShape {
+    int rows, G, NT;
+    uint32_t slices, layout;
+    int col_blocks;
+    __device__ __forceinline__ int GS() const { return slices & 0xFFFF; }
+    __device__ __forceinline__ int KS() const { return slices >> 16; }
+    __device__ __forceinline__ int full_waves() const { return layout & 255; }               // wavefronts of GPW groups
+    __device__ __forceinline__ int last_full_waves() const { return (layout >> 8) & 255; }  // ... in the last slice
+    __device__ __forceinline__ int waves() const { return (layout >> 16) & 255; }
+    __device__ __forceinline__ bool is(uint32_t bit) const { return (layout & bit) != 0; }
+};
+constexpr uint32_t kMidColumnScales = 1u << 24, kMidColShift = 1u << 25, kMidSwiglu = 1u << 26, kMidFlagged = 1u << 27;
 
 // The work of one block.  RBN: row blocks of 32 its pass computes -- 2, or 1 where the block's run of rows
 // has at most 32 (a launch of up to 32 rows, or the last run of a longer one: half the loads of A, fragment
@@ -143,15 +161,15 @@ constexpr int kMidFoldSpinLimit = 1 << 20;
 template <int TP, int GPW, bool LORA, int RBN>
 __device__ __forceinline__ void mid_block(
     const uint16_t *__restrict__ A_all, const u32x4 *__restrict__ B, const uint16_t *__restrict__ S,
-    uint16_t *__restrict__ C_all, float *partial_all, int *counters_all, int rows, int N, int K, int Gs, int KS,
-    int GS, int full_waves, int swiglu, int flagged, int col_shift, const MidLora &lo, int nw) {
+    uint16_t *__restrict__ C_all, float *partial_all, int *counters_all, const MidShape shape, const MidLora &lo) {
+    const int rows = shape.rows, G = shape.G, NT = shape.NT, N = NT * kTileN, K = G * kGroupK, KS = shape.KS(), nw = shape.waves();
+    const bool swiglu = shape.is(kMidSwiglu), flagged = shape.is(kMidFlagged);
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
     int &s_last = *reinterpret_cast<int *>(lds);  // used between two barriers behind the meeting, when nothing else is in LDS
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, h = lane >> 5;
-    const int G = K / kGroupK;
 #ifdef KILN_MID_TIMELINE
     long long tl_[8] = {};
     struct TimelineWriter {  // on every way out of the kernel
@@ -169,7 +187,8 @@ __device__ __forceinline__ void mid_block(
     KILN_MID_TL(0);
     // Grid (column blocks, K slices, runs of 64 rows) -- or, with the projection in this launch, one row
     // of blocks: the producers, then the same order.
-    int bx = blockIdx.x, by = blockIdx.y, bz = blockIdx.z, ncb = gridDim.x;
+    const int ncb = shape.col_blocks;
+    int bx = blockIdx.x, by = blockIdx.y, bz = blockIdx.z;
     if constexpr (LORA) {
         if (lo.producers > 0) {
             int id = blockIdx.x;
@@ -182,7 +201,6 @@ __device__ __forceinline__ void mid_block(
                 return;
             }
             id -= lo.producers;
-            ncb = lo.col_blocks;
             bx = id % ncb;
             id /= ncb;
             by = id % KS;
@@ -200,16 +218,15 @@ __device__ __forceinline__ void mid_block(
     // counter-free exchange shifts the column block by col_shift per slice so that the slices of a
     // tile sit on different dies (a device-scope store and the device-scope load that polls it
     // are slow when they meet in one die's L2).
-    const int cb = (bx + ks * col_shift) % ncb;
+    int cb = bx + (shape.is(kMidColShift) ? ks : 0);
+    if (cb >= ncb) cb -= ncb;  // at most three past the end, of four blocks or more
     const int tf = cb * (2 * TP);  // first 16-column tile of the block
     // the first `fw` wavefronts own GPW groups each, the others GPW - 1; the last slice may have fewer groups
-    // than the others (K in groups not a multiple of the slices) and then fewer wavefronts of GPW: its count
-    // rides in the argument's second byte
-    const int fw = (ks == KS - 1 ? full_waves >> 8 : full_waves) & 255;
+    // than the others (K in groups not a multiple of the slices) and then fewer wavefronts of GPW
+    const int fw = ks == KS - 1 ? shape.last_full_waves() : shape.full_waves();
     const bool full = wave < fw;
-    const int g_first = full ? wave * GPW : fw * GPW + (wave - fw) * (GPW - 1);
-    const int g0 = ks * GS + g_first;  // all slices have GS groups
-    const int gs_mask = (Gs == 1) ? 0 : -1;
+    const int g_first = wave * (GPW - 1) + min(wave, fw);
+    const int g0 = ks * shape.GS() + g_first;  // all slices start at multiples of GS
 
     // --- A: 16 loads of 4 rows x 256 bytes.  Lane i of load p fetches 16-byte unit
     // (i % 16) ^ (row % 16) of row 4 p + i / 16, so unit u of a row sits at position u ^ (row % 16):
@@ -237,19 +254,24 @@ __device__ __forceinline__ void mid_block(
     constexpr int kSets = D + 1;
     u32x4 bw[kSets][TP][2];
     uint32_t sc_raw[kSets][TP];
+    // one 64-bit address per operand, 32-bit distances from it
+    const bool column_scales = shape.is(kMidColumnScales);
+    const uint32_t scale_groups = column_scales ? 1u : (uint32_t)G;
+    const int last_pair_tile = NT - 2 - tf;  // a pair past the last tile reads the last pair; never stored
     const uint32_t b_lane = (uint32_t)(l32 >> 4) * (uint32_t)G * 1024u + (uint32_t)((l32 & 15) + 16 * h) * 16u;
-    const uint32_t s_lane = (uint32_t)(l32 >> 4) * (uint32_t)Gs * (kTileN * 2) + (uint32_t)(l32 & 15) * 2u;
+    const uint32_t s_lane = (uint32_t)(l32 >> 4) * scale_groups * (kTileN * 2) + (uint32_t)(l32 & 15) * 2u;
+    const char *const b_first = reinterpret_cast<const char *>(B) + (size_t)((uint32_t)tf * (uint32_t)G + (uint32_t)g0) * 1024;
+    const char *const s_first = reinterpret_cast<const char *>(S) +
+                                (size_t)((uint32_t)tf * scale_groups + (column_scales ? 0u : (uint32_t)g0)) * (kTileN * 2);
     auto request_b = [&](auto gc) {
         constexpr int gi = decltype(gc)::value, set = gi % kSets;
-        const int g = g0 + gi;
         unrolled<0, TP>([&](auto pc) {
             constexpr int p = decltype(pc)::value;
-            const int tp = min(tf + 2 * p, N / kTileN - 2);  // a pair past the last tile reads the last pair; never stored
-            const char *bb = reinterpret_cast<const char *>(B) + ((size_t)tp * G + g) * 1024;
+            const uint32_t tile = min(2 * p, last_pair_tile);
+            const char *bb = b_first + (tile * (uint32_t)G + gi) * 1024u;
             load_b128_streaming(bw[set][p][0], bb, b_lane);
             load_b128_streaming(bw[set][p][1], bb, b_lane + 512u);
-            const char *sb = reinterpret_cast<const char *>(S) + ((size_t)tp * Gs + (g & gs_mask)) * (kTileN * 2);
-            load_u16(sc_raw[set][p], sb, s_lane);
+            load_u16(sc_raw[set][p], s_first + (tile * scale_groups + (column_scales ? 0u : gi)) * (kTileN * 2u), s_lane);
         });
     };
 
@@ -486,7 +508,6 @@ __device__ __forceinline__ void mid_block(
     constexpr int kPerPair = RBN * 4;          // items of a pair in this pass, = their stride in a slot
     constexpr int kPhasePairs = 16 / kPerPair; // pairs a slot holds
     constexpr int kPhases = (TP + kPhasePairs - 1) / kPhasePairs;
-    const int NT = N / kTileN;
     auto store_item = [&](f32x4 v, int item) {
         const int q = item & 3, rb = (item >> 2) & 1, p = item >> 3;
         const int row0 = 32 * rb + 8 * q + 4 * h;
@@ -663,15 +684,11 @@ constexpr int kMidWavesOf = ROW_BLOCKS == kMidOneRowBlock || (!LORA && TP == 1) 
 template <int TP, int GPW, bool LORA, int ROW_BLOCKS>
 __global__ __launch_bounds__((kMidWavesOf<TP, ROW_BLOCKS, LORA> * 64)) void w4a16_mid_kernel(
     const uint16_t *__restrict__ A_all, const u32x4 *__restrict__ B, const uint16_t *__restrict__ S,
-    uint16_t *__restrict__ C_all, float *partial_all, int *counters_all, int rows, int N, int K, int Gs, int KS,
-    int GS, int full_waves, int swiglu, int flagged, int col_shift, MidLora lo) {
-    // the block's wavefronts, read here: in the kernel itself the compiler knows every block to be whole
-    // and reads the launch's block size, in a device function it first asks whether this block is a partial
-    // one (a dependent load at the very start)
-    const int nw = blockDim.x >> 6;
+    int rows, int G, int NT, uint32_t slices, uint32_t layout, int col_blocks, uint16_t *__restrict__ C_all,
+    float *partial_all, int *counters_all, MidLora lo) {
+    const MidShape shape{rows, G, NT, slices, layout, col_blocks};
     if constexpr (ROW_BLOCKS != kMidRowBlocksByRun) {
-        mid_block<TP, GPW, LORA, ROW_BLOCKS>(A_all, B, S, C_all, partial_all, counters_all, rows, N, K, Gs, KS, GS,
-                                             full_waves, swiglu, flagged, col_shift, lo, nw);
+        mid_block<TP, GPW, LORA, ROW_BLOCKS>(A_all, B, S, C_all, partial_all, counters_all, shape, lo);
     } else {
         // the run of 64 rows this block belongs to, as mid_block maps its index (a producer block of a call
         // with adapters belongs to none: either instance runs the projection and returns)
@@ -679,15 +696,13 @@ __global__ __launch_bounds__((kMidWavesOf<TP, ROW_BLOCKS, LORA> * 64)) void w4a1
         if constexpr (LORA) {
             if (lo.producers > 0) {
                 const int id = (int)blockIdx.x - lo.producers;
-                bz = id < 0 ? 0 : id / lo.col_blocks / KS;
+                bz = id < 0 ? 0 : id / col_blocks / shape.KS();
             }
         }
         if (rows - bz * kMidRows <= 32)
-            mid_block<TP, GPW, LORA, 1>(A_all, B, S, C_all, partial_all, counters_all, rows, N, K, Gs, KS, GS, full_waves,
-                                        swiglu, flagged, col_shift, lo, nw);
+            mid_block<TP, GPW, LORA, 1>(A_all, B, S, C_all, partial_all, counters_all, shape, lo);
         else
-            mid_block<TP, GPW, LORA, 2>(A_all, B, S, C_all, partial_all, counters_all, rows, N, K, Gs, KS, GS, full_waves,
-                                        swiglu, flagged, col_shift, lo, nw);
+            mid_block<TP, GPW, LORA, 2>(A_all, B, S, C_all, partial_all, counters_all, shape, lo);
     }
 }
 
@@ -698,7 +713,7 @@ hipError_t launch_mid_tgs(const MidArgs &a, hipStream_t stream) {
     const int NT = a.N / kTileN;
     const int runs = (a.M + kMidRows - 1) / kMidRows;
     const int last_groups = a.K / kGroupK - (a.KS - 1) * a.GS;  // of the last slice: GS, or fewer
-    const int full_waves = (a.GS - a.waves * (GPW - 1)) | ((last_groups - a.waves * (GPW - 1)) << 8);
+    const int full_waves = a.GS - a.waves * (GPW - 1), last_full_waves = last_groups - a.waves * (GPW - 1);
     MidLora lo{};
     lo.t = (const uint16_t *)a.lora_t;
     lo.b = (const uint16_t *)a.lora_b;
@@ -713,7 +728,6 @@ hipError_t launch_mid_tgs(const MidArgs &a, hipStream_t stream) {
         lo.producers = a.lora_producers;
         lo.row_tiles = (a.M + 15) / 16;
         lo.steps_per_slice = a.lora_steps_per_slice;
-        lo.col_blocks = col_blocks;
         lo.consumers = col_blocks * runs;
         lo.ls.count = a.lora_adapters;
         for (int i = 0; i < 8; ++i) {
@@ -722,10 +736,12 @@ hipError_t launch_mid_tgs(const MidArgs &a, hipStream_t stream) {
         }
         grid = dim3(a.lora_producers + col_blocks * a.KS * runs, 1, 1);
     }
+    const uint32_t layout = (uint32_t)full_waves | (uint32_t)last_full_waves << 8 | (uint32_t)a.waves << 16 |
+                            (a.Gs == 1 ? kMidColumnScales : 0u) | (a.swiglu ? kMidSwiglu : 0u) |
+                            (a.flagged ? kMidFlagged | (exchange_column_shift(col_blocks) ? kMidColShift : 0u) : 0u);
     w4a16_mid_kernel<TP, GPW, kMidLora, ROW_BLOCKS><<<grid, a.waves * 64, a.waves * kMidSlotBytes, stream>>>(
-        (const uint16_t *)a.A, (const u32x4 *)a.B, (const uint16_t *)a.S, (uint16_t *)a.C, a.partial, a.counters, a.M,
-        a.N, a.K, a.Gs, a.KS, a.GS, full_waves, a.swiglu ? 1 : 0, a.flagged ? 1 : 0,
-        a.flagged ? exchange_column_shift((NT + 2 * TP - 1) / (2 * TP)) : 0, lo);
+        (const uint16_t *)a.A, (const u32x4 *)a.B, (const uint16_t *)a.S, a.M, a.K / kGroupK, NT,
+        (uint32_t)a.GS | (uint32_t)a.KS << 16, layout, col_blocks, (uint16_t *)a.C, a.partial, a.counters, lo);
     return hipGetLastError();
 }
 
@@ -793,7 +809,7 @@ bool mid_plan_ok(const MidArgs &a) {
     if (a.pairs < 1 || a.pairs > 3) return false;
     const int G = a.K / kGroupK;
     // slices of GS groups; the last one may be shorter (11008 = 86 groups = 29 + 29 + 28)
-    if (a.KS < 1 || a.GS < 1 || a.KS * a.GS < G || (a.KS - 1) * a.GS >= G) return false;
+    if (a.KS < 1 || a.KS > 0x7FFF || a.GS < 1 || a.KS * a.GS < G || (a.KS - 1) * a.GS >= G) return false;
     if (a.waves < 1 || a.waves > mid_max_waves(a.M, a.pairs, a.r_total > 0) || a.waves > a.GS) return false;
     const int gpw = (a.GS + a.waves - 1) / a.waves;
     if (gpw > kMidMaxGroups || (a.pairs == 3 && gpw == 4)) return false;  // (3, 4) would spill registers
