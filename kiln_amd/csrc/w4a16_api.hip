@@ -1275,7 +1275,8 @@ int kiln_w4a16_debug_gemm_plan(int m, int n, int k, int cus, int *out) {
     out[0] = gp.prefill; out[1] = gp.launches; out[2] = gp.pf.bm; out[3] = gp.pf.bn; out[4] = gp.pf.nb_full;
     out[5] = gp.pf.ks;
     out[6] = gp.mid;          // the mid-M kernel: pairs of tiles per block, K slices
-    out[7] = gp.mid ? gp.mp.pairs * 16 + gp.mp.KS : 0;
+    // ... or of the matrix-core kernel: whether its wavefronts share K
+    out[7] = gp.mid ? gp.mp.pairs * 16 + gp.mp.KS : gp.prefill ? prefill_halves_k(m, n, k, gp.pf, cus) : 0;
     return 0;
 }
 

@@ -116,6 +116,40 @@ __device__ __forceinline__ const char *uniform(const char *p) {
     return reinterpret_cast<const char *>(((uint64_t)hi << 32) | lo);
 }
 
+// Where some of a block's wavefronts meet without the others: a count in LDS that each raises by one.  LDS serves a
+// wavefront's requests in order, so who raises it has read what it asked for before.  The look is asked for some products
+// later and answered a product after that; who then finds others missing polls (they are resident, so the bound, one
+// second and more, is never reached).  The loop is inside the asm statement: registers that loads in flight will fill must
+// not meet the end of a basic block.  Every lane is active.
+__device__ __forceinline__ void meeting_signal(unsigned lds_addr) {
+    uint32_t at, one;
+    asm volatile("s_mov_b64 exec, 1\n\tv_mov_b32 %0, %2\n\tv_mov_b32 %1, 1\n\tds_add_u32 %0, %1\n\ts_mov_b64 exec, -1"
+                 : "=&v"(at), "=&v"(one)
+                 : "s"(lds_addr)
+                 : "memory");
+}
+__device__ __forceinline__ void meeting_look(unsigned lds_addr, uint32_t &seen) {
+    asm volatile("v_mov_b32 %0, %1\n\tds_read_b32 %0, %0" : "=&v"(seen) : "s"(lds_addr) : "memory");
+}
+__device__ __forceinline__ void meeting_wait(unsigned lds_addr, uint32_t &seen, int expected) {
+    int value, polls;
+    asm volatile("s_mov_b32 %2, 0x400000\n"
+                 "Lmeeting_%=:\n\t"
+                 "s_waitcnt lgkmcnt(0)\n\t"
+                 "v_readfirstlane_b32 %1, %0\n\t"
+                 "s_sub_u32 %2, %2, 1\n\t"
+                 "s_cbranch_scc1 Lmet_%=\n\t"
+                 "s_cmp_ge_i32 %1, %4\n\t"
+                 "s_cbranch_scc1 Lmet_%=\n\t"
+                 "v_mov_b32 %0, %3\n\t"
+                 "ds_read_b32 %0, %0\n\t"
+                 "s_branch Lmeeting_%=\n"
+                 "Lmet_%=:"
+                 : "+v"(seen), "=&s"(value), "=&s"(polls)
+                 : "s"(lds_addr), "s"(expected)
+                 : "memory", "scc");
+}
+
 // Probe builds only (-DKILN_PREFILL_TIMELINE): wall-clock stamps per block.
 #ifdef KILN_PREFILL_TIMELINE
 __device__ long long *g_timeline;
@@ -197,20 +231,21 @@ constexpr int kFoldPeekOffset = kProjectLdsBytes16 - 1024;
 // operand of 16-row tiles [t0, t1) -- a contiguous piece of A, streamed with 24 loads per thread in
 // flight; 16 lanes per (row, group), the order of additions of w4a16_prefill_rowsum_kernel, whose
 // launch this saves -- written through to memory, then the tiles' words.
+template <int THREADS>
 __device__ __forceinline__ void rowsum_producer_block(const uint16_t *__restrict__ A, u32x4 *__restrict__ aext, int M,
                                                       int K, int t0, int t1, unsigned *done) {
-    constexpr int U = 24;
+    constexpr int U = 24, SLOTS = THREADS / 16;
     const int G = K / kGroupK;
     const int r0 = t0 * 16, r1 = min(t1 * 16, M);
     const int items = (r1 - r0) * G;  // item L: the 256 bytes from byte 256 L of the piece on
     const int tid = threadIdx.x, sub = tid & 15, slot = tid >> 4;
     const u32x4 *src = reinterpret_cast<const u32x4 *>(A + (size_t)r0 * K) + sub;
-    for (int base = 0; base < items; base += 16 * U) {
+    for (int base = 0; base < items; base += SLOTS * U) {
         u32x4 v[U];
         float sum[U];
 #pragma unroll
         for (int u = 0; u < U; ++u)  // items past the end re-read the last one
-            v[u] = async_load_b128(src + (size_t)min(base + u * 16 + slot, items - 1) * 16);
+            v[u] = async_load_b128(src + (size_t)min(base + u * SLOTS + slot, items - 1) * 16);
         unrolled<0, U>([&](auto uc) {
             constexpr int u = decltype(uc)::value;
             // loads complete in issue order: load u has landed when at most the U - 1 - u later ones are pending
@@ -222,7 +257,7 @@ __device__ __forceinline__ void rowsum_producer_block(const uint16_t *__restrict
         });
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int L = base + u * 16 + slot;
+            const int L = base + u * SLOTS + slot;
             if (sub == 0 && L < items) {
                 const int row = L / G, g = L - row * G;
                 store_b128_through(aext + (size_t)g * M + r0 + row, extension_operand(sum[u]));
@@ -232,7 +267,7 @@ __device__ __forceinline__ void rowsum_producer_block(const uint16_t *__restrict
     // every wavefront's stores acknowledged, then the words
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
     __syncthreads();
-    for (int t = t0 + tid; t < t1; t += 256) __hip_atomic_store(done + t, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int t = t0 + tid; t < t1; t += THREADS) __hip_atomic_store(done + t, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // A look at the words of rows [m0, m0 + rows) that nobody waits for: one device-scope load per lane
@@ -291,8 +326,20 @@ __device__ __forceinline__ void prefill_fold_done(const PrefillFold &pf, int con
 // rounds, whose row sums come from in front anyway; where the launch's own blocks form them (RS, and FOLD's producers
 // without INC) they are not there when a block begins.  FOLD and INC together: the producers run the projection onto the
 // adapters alone.
-template <int NWN, int WM, int MI, bool SWIGLU, bool RS, bool FOLD = false, bool INC = false>
-__global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void w4a16_prefill_kernel(
+//
+// WK = 2: a block has twice the wavefronts, and each half of them takes half of the block's groups of K, with a ring of
+// its own and the barriers in common; the halves' tiles meet in LDS, and each half goes on with half of the rows (the
+// exchange of K slices and the store).  For launches of at most one block per compute unit: with one wavefront per SIMD
+// nothing covers what one waits for -- a stage's barrier and LDS reads, and its own instruction stream, five cycles an
+// instruction, which in 64-row blocks is longer than the products.  An odd number of groups: the second half begins with
+// the first's last group and multiplies what it got there by 0.  The halves' stages are met half by half, through a word
+// of LDS: half of the wavefronts wait for one another while the other half computes.  (us, one set of wavefronts -> two:
+// 128-row blocks 9216 -> 2560 at 777 rows 59.3 -> 53.4; 64-row blocks 9216 -> 2560 at 640 / 512 / 300 rows 54.8 -> 43.3 /
+// 41 -> 36.5 / 33.7 -> 28.4, 4096 -> 2560 at 1100 45.5 -> 35.2, 4096 -> 4096 at 777 46 -> 37, 2560 -> 2560 at 777 30 -> 24,
+// 1536 -> 1536 at 1300 25.6 -> 17.0.  The sums of K are two shorter ones: error beyond the bf16 rounding 1.79e-4 -> 1.48e-4 of
+// the result's norm at 777 x 9216 -> 2560, 14 to 25 % less in each of eight shapes.)
+template <int NWN, int WM, int MI, bool SWIGLU, bool RS, bool FOLD = false, bool INC = false, int WK = 1>
+__global__ __launch_bounds__(64 * WM * NWN * WK, (WM == 2 && NWN == 4) ? 1 : 2) void w4a16_prefill_kernel(
     const uint16_t *__restrict__ A, const u32x4 *__restrict__ B, const uint16_t *__restrict__ S,
     uint16_t *__restrict__ C, const u32x4 *__restrict__ aext, int M, int N, int K, int Gs, int m_blocks,
     const uint16_t *__restrict__ lora_t, const uint16_t *__restrict__ lora_b, int r_total, int RP, int nb_full,
@@ -300,13 +347,14 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];  // the A ring; reused by the store
     static_assert(!FOLD || WM * NWN == 4, "the projection's blocks have four wavefronts");
     static_assert(!INC || (!RS && WM == 1 && MI == 4), "the row sums come from in front");
+    static_assert(WK == 1 || (WK == 2 && WM == 1 && !INC), "halves of K: one row of wavefronts, the contraction behind the loop");
     if constexpr (FOLD) {
         if ((int)blockIdx.x < pf.producers) {
             const int unit = blockIdx.x;
             if (pf.a_cat == nullptr) {
                 const int t0 = unit * pf.sum_tiles;
                 if (t0 < pf.row_tiles)
-                    rowsum_producer_block(A, pf.aext, M, K, t0, min(t0 + pf.sum_tiles, pf.row_tiles),
+                    rowsum_producer_block<64 * WM * NWN * WK>(A, pf.aext, M, K, t0, min(t0 + pf.sum_tiles, pf.row_tiles),
                                           pf.words + kPrefillFoldTileWord);
                 return;
             }
@@ -318,7 +366,7 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
         }
     }
     constexpr int BM = WM * MI * 32, BN = 64 * NWN;  // block rows and columns
-    constexpr int NW = WM * NWN, NT = 64 * NW;       // wavefronts, threads
+    constexpr int NW = WM * NWN, NT = 64 * NW * WK;  // wavefronts (of a half of K), threads
     constexpr int kAStageBytes = BM * 32 * 2;        // BM rows x 32 columns of bf16 per stage
     constexpr int APW = (BM / 16) / NW;              // A loads (16 rows each) per wavefront and stage
     static_assert(APW * NW * 16 == BM, "A stage must divide evenly over the wavefronts");
@@ -328,7 +376,8 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
     KILN_TL(0);
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave_all = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int half = WK == 1 ? 0 : wave_all / NW, wave = WK == 1 ? wave_all : wave_all % NW;  // ... among its half's
     const int wm = wave / NWN, wn = wave % NWN;
     const int G = K / kGroupK;
     const int l32 = lane & 31, h = lane >> 5;
@@ -359,7 +408,7 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
     const int mb = (die % die_rows) * rows_per_die + seq % rows_per_die;
     if (seq >= rows_per_die * units_per_die || unit >= units || mb >= m_blocks) {  // grid padding (whole block, before any barrier)
         if constexpr (FOLD) {
-            if (wave == 0) prefill_fold_done(pf, consumer, lane);  // counted like the others: it will never look
+            if (wave_all == 0) prefill_fold_done(pf, consumer, lane);  // counted like the others: it will never look
         }
         return;
     }
@@ -371,7 +420,24 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
     const int m0 = mb * BM, n0 = nb * BN;
     // K slice of this block: groups [g_begin, g_end).  With KS > 1 the slices of
     // a tile are combined through the workspace at the end.
-    const int g_begin = sliced ? ks * GSb : 0, g_end = sliced ? min(G, g_begin + GSb) : G;
+    int g_begin = sliced ? ks * GSb : 0, g_end = sliced ? min(G, g_begin + GSb) : G;
+    [[maybe_unused]] bool phantom = false;  // the first group is the other half's: its products are dropped
+    if constexpr (WK == 2) {
+        const int both = g_end - g_begin, each = (both + 1) >> 1;
+        phantom = half == 1 && 2 * each != both;
+        if (half == 0) g_end = g_begin + each;
+        else g_begin = g_end - each;
+    }
+    // LDS: the halves' rings, then (with the look at a folded launch's words in front) what lies behind a ring
+    const int ring = WK == 1 ? 0 : half * (kAStages * kAStageBytes);
+    constexpr int kBehindRings = WK * kAStages * kAStageBytes + (WK == 2 && FOLD ? 1024 : 0);
+    [[maybe_unused]] constexpr int kPeekAt = WK == 1 ? kFoldPeekOffset : WK * kAStages * kAStageBytes;
+
+    __shared__ uint32_t s_meeting[2];
+    if constexpr (WK == 2) {
+        if (tid < 2) s_meeting[tid] = 0;
+        wait_lds_reads();  // zero before the barrier in front of the main loop
+    }
 
     // --- A: global -> LDS without passing through registers --------------------
     // A stage is BM rows x 32 columns of bf16 = 64 B per row, 4 units of 16 B; four stages form a ring.
@@ -391,11 +457,14 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
         const int row = min(m0 + (wave + NW * p) * 16 + (lane >> 2), M - 1) - m0;
         a_off_g[p] = (uint32_t)row * (uint32_t)K * 2u + (((lane & 3) ^ ((lane >> 4) & 3)) * 16);
     }
+    // WK = 2: where a half's wavefronts meet once a stage (meeting_signal), and how many arrivals there will have been
+    [[maybe_unused]] const unsigned meeting = (unsigned)(size_t)(lds_ptr_t)&s_meeting[half];
+    [[maybe_unused]] int met = 0;
     const char *a_ptr = uniform(reinterpret_cast<const char *>(A) + ((size_t)m0 * K + (size_t)g_begin * kGroupK) * 2);  // this group's stages
-    const unsigned lds_base = (unsigned)(size_t)(lds_ptr_t)lds;
+    const unsigned lds_base = (unsigned)(size_t)(lds_ptr_t)lds, ring_base = lds_base + ring;
     auto load_a = [&](const char *base, int slot) {
 #pragma unroll
-        for (int p = 0; p < APW; ++p) load_to_lds_b128(base, a_off_g[p], lds_base + slot * kAStageBytes + (wave + NW * p) * 1024);
+        for (int p = 0; p < APW; ++p) load_to_lds_b128(base, a_off_g[p], ring_base + slot * kAStageBytes + (wave + NW * p) * 1024);
     };
 
     // --- B: column sub-tile ni (32 columns = chunks 2ni, 2ni+1 of this wavefront);
@@ -429,7 +498,7 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
     int a_off[2];
 #pragma unroll
     for (int sp = 0; sp < 2; ++sp)
-        a_off[sp] = (wm * MI * 32 + l32) * 64 + (((2 * sp + h) ^ ((l32 >> 2) & 3)) * 16);
+        a_off[sp] = ring + (wm * MI * 32 + l32) * 64 + (((2 * sp + h) ^ ((l32 >> 2) & 3)) * 16);
 
     f32x16 acc[MI][2];
 #pragma unroll
@@ -487,7 +556,7 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
         pin(bw[ni][0]);
         pin(bw[ni][1]);
         pin(sc_raw[ni]);
-        sc[ni] = scale_value(sc_raw[ni]);
+        sc[ni] = WK == 2 && phantom ? 0.f : scale_value(sc_raw[ni]);  // (the change to the next group's multiplies by it)
     }
     bf16x8 af[MI][2], bf[2][2];
     auto read_a = [&](auto slotc, int mi) {
@@ -499,12 +568,12 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
     // row lane / 4, unit lane % 4 of a stage; the four lanes of a row meet when the group ends.
     int g_now = g_begin;
     [[maybe_unused]] float gsum[RS ? RPW / 16 : 1] = {};
-    [[maybe_unused]] float *csum = reinterpret_cast<float *>(lds + kAStages * kAStageBytes);
+    [[maybe_unused]] float *csum = reinterpret_cast<float *>(lds + kBehindRings) + half * (g_end - g_begin) * BM;
     [[maybe_unused]] auto sum_rows = [&](auto slotc) {
 #pragma unroll
         for (int rr = 0; rr < RPW / 16; ++rr) {
             const int row = wave * RPW + rr * 16 + (lane >> 2);
-            const u32x4 v = *reinterpret_cast<const u32x4 *>(lds + decltype(slotc)::value * kAStageBytes + row * 64 + (((lane & 3) ^ ((row >> 2) & 3)) * 16));
+            const u32x4 v = *reinterpret_cast<const u32x4 *>(lds + ring + decltype(slotc)::value * kAStageBytes + row * 64 + (((lane & 3) ^ ((row >> 2) & 3)) * 16));
             gsum[rr] += sum_bf16x8(v);
         }
     };
@@ -538,14 +607,16 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
     const char *const s_base = s_ptr;
     constexpr int kExtLoads = INC ? 0 : (RS ? 0 : APW) + 2;  // per wavefront and extension stage
     const uint32_t ext_off = (uint32_t)min(m0 + (RS ? 0 : (wave % (BM / 64)) * 64) + lane, M - 1) * 16u;
-    auto ext_scales = [&](int slot) { return RS ? slot * kAStageBytes + wave * 512 : kAStages * kAStageBytes + (slot * NW + wave) * 512; };
+    auto ext_scales = [&](int slot) {
+        return RS ? ring + slot * kAStageBytes + wave * 512 : kBehindRings + ((half * kAStages + slot) * NW + wave) * 512;
+    };
     auto request_ext = [&](int e, int slot) {  // groups past the last re-read it
         if constexpr (!RS) {
 #pragma unroll
             for (int p = 0; p < APW; ++p) {
                 const int i = wave + NW * p, g = g_begin + min(4 * e + i / (BM / 64), ng - 1);
                 load_to_lds_b128(uniform(reinterpret_cast<const char *>(aext + (size_t)g * M)), ext_off,
-                                 lds_base + slot * kAStageBytes + i * 1024);
+                                 ring_base + slot * kAStageBytes + i * 1024);
             }
         }
 #pragma unroll
@@ -579,10 +650,23 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
             constexpr bool ahead = !(LAST && q == 3);  // there is a next stage
             u32x4 bn[2][2];
             [[maybe_unused]] f32x4 cq[INC ? MI * 2 : 1];
+            // Loads complete in issue order; behind the next stage's there are those of the two stages after
+            // it (in the last group extension stages take the place of stages) and, unless they are needed now,
+            // the next group's six, its c and the look at the words.
+            constexpr int a_behind = LAST && q > 0 ? (q == 1 ? 1 : 0) : 2;
+            constexpr int others = (!LAST && (q == 1 || q == 2)) ? 6 + (PEEK ? 1 : 0) + (INC ? 1 : 0) : 0;
+            constexpr int kStageLanded = a_behind * APW + (2 - a_behind) * kExtLoads + others;
+            if constexpr (WK == 2) {  // the half's wavefronts meet: this one's part of the next stage is there, its reads of this stage asked for
+                wait_vector_loads<kStageLanded>();
+                meeting_signal(meeting);
+                met += NW;
+            }
+            [[maybe_unused]] uint32_t seen_met = 0;
             unrolled<0, MI>([&](auto mc) {
                 constexpr int mi = decltype(mc)::value;
                 unrolled<0, 4>([&](auto jc) {
                     constexpr int j = decltype(jc)::value, ni = j & 1, sp = j >> 1, slot = 4 * mi + j;
+                    if constexpr (WK == 2 && slot == 3) meeting_look(meeting, seen_met);
                     acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[mi][sp], bf[ni][sp], acc[mi][ni], 0, 0, 0);
                     // behind this product: halves of the next stage's operands of B ...
                     constexpr int first = q == 3 ? 4 : 0, room = 4 * MI - first;  // (the next group's words are there behind the barrier)
@@ -636,14 +720,13 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
                     __builtin_amdgcn_sched_barrier(0);
                 });
                 if constexpr (mi == 0) {
-                    // Loads complete in issue order; behind the next stage's there are those of the two stages after
-                    // it (in the last group extension stages take the place of stages) and, unless they are needed now,
-                    // the next group's six, its c and the look at the words.
-                    constexpr int a_behind = LAST && q > 0 ? (q == 1 ? 1 : 0) : 2;
-                    constexpr int others = (!LAST && (q == 1 || q == 2)) ? 6 + (PEEK ? 1 : 0) + (INC ? 1 : 0) : 0;
-                    wait_vector_loads<a_behind * APW + (2 - a_behind) * kExtLoads + others>();
-                    wait_lds_reads();
-                    __builtin_amdgcn_s_barrier();
+                    if constexpr (WK == 2) {
+                        meeting_wait(meeting, seen_met, met);
+                    } else {
+                        wait_vector_loads<kStageLanded>();
+                        wait_lds_reads();
+                        __builtin_amdgcn_s_barrier();
+                    }
                     asm volatile("" : : : "memory");
                     if constexpr (!LAST) {
                         load_a(a_ptr + (q + 4) * 64, q);
@@ -664,7 +747,7 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
                         }
                     }
                     if constexpr (LAST && !INC) request_ext(q, q);
-                    if constexpr (PEEK && q == 0) prefill_fold_peek(pf, m0, min(BM, M - m0), lane, lds_base + kFoldPeekOffset + wave * 256);
+                    if constexpr (PEEK && q == 0) prefill_fold_peek(pf, m0, min(BM, M - m0), lane, lds_base + kPeekAt + wave * 256);
                 }
                 if constexpr (INC && q == 0 && mi == MI - 1 && !LAST) {
                     // three phases later than without INC: the registers are c's until then
@@ -715,7 +798,7 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
         if (ng > 1) {
             group(std::false_type{}, std::true_type{});
             next_group();
-            seen = prefill_fold_seen(lds + kFoldPeekOffset + wave * 256, lane);
+            seen = prefill_fold_seen(lds + kPeekAt + wave * 256, lane);  // (WK = 2: of either half's wavefront; raised is raised)
         }
         if (!seen) prefill_fold_wait(pf, m0, min(BM, M - m0), lane);
     }
@@ -749,7 +832,7 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
         for (int mi = 0; mi < MI; ++mi) {
             const int row = wm * MI * 32 + mi * 32 + l32;
             if constexpr (RS) x.c[mi] = csum[min(4 * e + 2 * u + h, ng - 1) * BM + row];
-            else x.a[mi] = *reinterpret_cast<const bf16x8 *>(lds + slot * kAStageBytes + ((2 * u + h) * BM + row) * 16);
+            else x.a[mi] = *reinterpret_cast<const bf16x8 *>(lds + ring + slot * kAStageBytes + ((2 * u + h) * BM + row) * 16);
         }
 #pragma unroll
         for (int ni = 0; ni < 2; ++ni) {
@@ -758,7 +841,7 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
         }
     };
     auto ext_multiply = [&](int e, int u, const ExtStep &x) {
-        const bool live = 4 * e + 2 * u + h < ng;
+        const bool live = 4 * e + 2 * u + h < ng && (WK == 1 || !phantom || 4 * e + 2 * u + h > 0);
         bf16x8 bx[2];
 #pragma unroll
         for (int ni = 0; ni < 2; ++ni) {
@@ -811,13 +894,13 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
     }
     wait_vector_loads<0>();  // stages asked for past the end still write to LDS, which the store reuses behind its barrier
     if constexpr (FOLD) {
-        if (wave == 0) prefill_fold_done(pf, consumer, lane);
+        if (wave_all == 0) prefill_fold_done(pf, consumer, lane);
     }
 
     // --- fused LoRA epilogue: y += T * B_cat^T with T = scaled x * A_cat^T from the
     // pre-pass (crates/kiln-model/src/lora_loader.rs:213-232, unfused at the call
     // sites forward.rs:2932-2939).  RP / 16 more k16 steps on the same accumulators.
-    for (int u = 0; u < (ks == 0 ? RP / 16 : 0); ++u) {  // the LoRA term belongs to one slice only
+    for (int u = 0; u < (ks == 0 && half == 0 ? RP / 16 : 0); ++u) {  // the LoRA term belongs to one slice (and half) only
         const int j8 = 16 * u + 8 * h;  // this lane's 8 rank columns
         bf16x8 lb[2];
 #pragma unroll
@@ -848,6 +931,37 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
         }
     }
 
+    // --- the halves of K meet in LDS: a wavefront hands the other half's wavefront of its columns that one's rows and
+    // adds what it gets to its own, the earlier groups' sum first (a + b is b + a)
+    constexpr int MIS = MI / WK;  // row tiles a wavefront goes on with
+    const int row_first = wm * MI * 32 + half * (MIS * 32);
+    if constexpr (WK == 2) {
+        __syncthreads();  // every wavefront is done with the rings
+        f32x4 *box = reinterpret_cast<f32x4 *>(lds) + lane;  // [half][wavefront][row tile, sub-tile, four registers][lane]
+        auto four = [](const f32x16 &a, int i) { return f32x4{a[4 * i], a[4 * i + 1], a[4 * i + 2], a[4 * i + 3]}; };
+        auto hand_over = [&](auto firstc) {
+            f32x4 *mine = box + (half * NW + wave) * (MIS * 8) * 64;
+            unrolled<0, MIS * 8>([&](auto ec) {
+                constexpr int e = decltype(ec)::value;
+                mine[e * 64] = four(acc[decltype(firstc)::value + e / 8][(e / 4) & 1], e & 3);
+            });
+        };
+        if (half == 0) hand_over(std::integral_constant<int, MIS>{});
+        else hand_over(std::integral_constant<int, 0>{});
+        __syncthreads();
+        const f32x4 *got = box + ((half ^ 1) * NW + wave) * (MIS * 8) * 64;
+        auto add = [&](auto firstc) {
+            unrolled<0, MIS * 8>([&](auto ec) {
+                constexpr int e = decltype(ec)::value;
+                const f32x4 g = got[e * 64], own = four(acc[decltype(firstc)::value + e / 8][(e / 4) & 1], e & 3);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[e / 8][(e / 4) & 1][4 * (e & 3) + i] = own[i] + g[i];
+            });
+        };
+        if (half == 0) add(std::integral_constant<int, 0>{});
+        else add(std::integral_constant<int, MIS>{});
+    }
+
     // --- store.  Register r of a 32x32 tile holds row 8*(r/4) + 4*h + r%4,
     // column l32: a lane owns one column.  Each wavefront transposes its
     // (MI * 32) x 64 tile through its own piece of LDS (the now idle A ring) as bf16, then
@@ -864,7 +978,7 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
         const int tile = (nb - nb_full) * m_blocks + mb;
         float *mine = partial + ((size_t)tile * KS + ks) * (BM * BN) + tid * 4;
 #pragma unroll
-        for (int mi = 0; mi < MI; ++mi)
+        for (int mi = 0; mi < MIS; ++mi)
 #pragma unroll
             for (int ni = 0; ni < 2; ++ni)
 #pragma unroll
@@ -881,29 +995,30 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
             s_last = (__hip_atomic_fetch_add(counters + tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == KS - 1);
         __syncthreads();
         if (!s_last) return;
-        // 16 loads (64 registers) a batch, MI / 2 batches per slice, each batch a round trip.  The block's own part is
+        // 16 loads (64 registers) a batch at most, a round trip each.  The block's own part is
         // still in its registers: as slice 0 or 1 the others are added to it as they come (a + b is b + a, so the
         // sum is the one in slice order); further on the sum before it would need registers of its own, and
         // it is read back like the others.
+        constexpr int kBatch = MIS * 8 < 16 ? MIS * 8 : 16;
         const float *all = partial + (size_t)tile * KS * (BM * BN) + tid * 4;
         for (int s2 = 0; s2 < KS; ++s2) {
             if (ks < 2 && s2 == ks) continue;
             const bool first = ks >= 2 && s2 == 0;
             const float *src = all + (size_t)s2 * (BM * BN);
 #pragma unroll
-            for (int half = 0; half < MI / 2; ++half) {
-                u32x4 t[16];
+            for (int batch = 0; batch < MIS * 8 / kBatch; ++batch) {
+                u32x4 t[kBatch];
 #pragma unroll
-                for (int i = 0; i < 16; ++i) load_b128_device_scope(t[i], src + (half * 16 + i) * NT * 4);
+                for (int i = 0; i < kBatch; ++i) load_b128_device_scope(t[i], src + (batch * kBatch + i) * NT * 4);
                 wait_vector_loads<0>();
 #pragma unroll
-                for (int i = 0; i < 16; ++i) {
+                for (int i = 0; i < kBatch; ++i) {
                     pin_loaded(t[i]);
                     const f32x4 v = __builtin_bit_cast(f32x4, t[i]);
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
                         const int at = 4 * (i & 3) + r;
-                        f32x16 &a = acc[half * 2 + i / 8][(i / 4) & 1];
+                        f32x16 &a = acc[batch * (kBatch / 8) + i / 8][(i / 4) & 1];
                         a[at] = first ? v[r] : a[at] + v[r];
                     }
                 }
@@ -915,9 +1030,9 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
     __syncthreads();  // every wavefront is done reading the A ring
     if constexpr (SWIGLU) {
         // acc[mi][0] holds gate, acc[mi][1] the matching up columns: h = gate / (1 + exp(-gate)) * up.
-        // The wavefront's tile becomes (MI * 32) x 32: rows of 64 bytes, 4 lanes per row.
-        uint16_t *tile = reinterpret_cast<uint16_t *>(lds + wave * (MI * 32 * 32 * 2));  // [MI * 32][32] bf16
-        [[maybe_unused]] float *unit_sums = reinterpret_cast<float *>(lds + NW * (MI * 32 * 32 * 2));  // [BM][16 units of 8 columns]
+        // The wavefront's tile becomes (MIS * 32) x 32: rows of 64 bytes, 4 lanes per row.
+        uint16_t *tile = reinterpret_cast<uint16_t *>(lds + wave_all * (MIS * 32 * 32 * 2));  // [MIS * 32][32] bf16
+        [[maybe_unused]] float *unit_sums = reinterpret_cast<float *>(lds + WK * NW * (MIS * 32 * 32 * 2));  // [BM][16 units of 8 columns]
         uint32_t *dst[2];  // of row pairs 0 and 2 of every four
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
@@ -925,7 +1040,7 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
             dst[i] = reinterpret_cast<uint32_t *>(tile + row * 32 + ((((l32 >> 3) ^ (row & 3)) << 3) | (l32 & 6)));
         }
 #pragma unroll
-        for (int mi = 0; mi < MI; ++mi)
+        for (int mi = 0; mi < MIS; ++mi)
 #pragma unroll
             for (int r = 0; r < 16; r += 2) {
                 float hval[2];
@@ -938,14 +1053,14 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
             }
         __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
 #pragma unroll
-        for (int p = 0; p < MI * 2; ++p) {
+        for (int p = 0; p < MIS * 2; ++p) {
             const int row = p * 16 + (lane >> 2), unit = lane & 3;
             const u32x4 v = *reinterpret_cast<const u32x4 *>(tile + row * 32 + ((unit ^ (row & 3)) << 3));
-            const int grow = m0 + wm * MI * 32 + row;
+            const int grow = m0 + row_first + row;
             if (grow < M)
                 *reinterpret_cast<u32x4 *>(C + (size_t)grow * (N / 2) + (n0 + wn * 64) / 2 + unit * 8) = v;
             if constexpr (WM == 1 && NWN == 4) {
-                if (next_aext) unit_sums[row * 16 + wn * 4 + unit] = sum_bf16x8(v);
+                if (next_aext) unit_sums[(row_first + row) * 16 + wn * 4 + unit] = sum_bf16x8(v);
             }
         }
         if constexpr (WM == 1 && NWN == 4) {
@@ -969,7 +1084,7 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
             }
         }
     } else {
-        uint16_t *tile = reinterpret_cast<uint16_t *>(lds + wave * (MI * 32 * 64 * 2));  // [MI * 32][64] bf16
+        uint16_t *tile = reinterpret_cast<uint16_t *>(lds + wave_all * (MIS * 32 * 64 * 2));  // [MIS * 32][64] bf16
         uint32_t *dst[2][2];  // of sub-tile ni, row pairs 0 and 2 of every four
 #pragma unroll
         for (int ni = 0; ni < 2; ++ni)
@@ -980,7 +1095,7 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
                 dst[ni][i] = reinterpret_cast<uint32_t *>(tile + row * 64 + ((((col >> 3) ^ (row & 7)) << 3) | (col & 6)));
             }
 #pragma unroll
-        for (int mi = 0; mi < MI; ++mi)
+        for (int mi = 0; mi < MIS; ++mi)
 #pragma unroll
             for (int ni = 0; ni < 2; ++ni)
 #pragma unroll
@@ -989,10 +1104,10 @@ __global__ __launch_bounds__(64 * WM * NWN, (WM == 2 && NWN == 4) ? 1 : 2) void 
         // same wavefront wrote and reads: only the LDS counter needs to drain
         __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
 #pragma unroll
-        for (int p = 0; p < MI * 4; ++p) {
+        for (int p = 0; p < MIS * 4; ++p) {
             const int row = p * 8 + (lane >> 3), unit = lane & 7;
             const u32x4 v = *reinterpret_cast<const u32x4 *>(tile + row * 64 + ((unit ^ (row & 7)) << 3));
-            const int grow = m0 + wm * MI * 32 + row;
+            const int grow = m0 + row_first + row;
             if (grow < M)
                 *reinterpret_cast<u32x4 *>(C + (size_t)grow * N + n0 + wn * 64 + unit * 8) = v;
         }
@@ -1203,27 +1318,30 @@ constexpr int kMaxRowSumBytes = 24 * 1024;
 static int row_sum_bytes(int groups) { return groups * 64 * (int)sizeof(float); }
 
 
-template <int NWN, int WM, int MI, bool SWIGLU, bool RS, bool FOLD = false, bool INC = false>
+template <int NWN, int WM, int MI, bool SWIGLU, bool RS, bool FOLD = false, bool INC = false, int WK = 1>
 hipError_t launch_shape_as(const PrefillArgs &a, int grid, int m_blocks, int RP, int KS, int GSb, int max_groups,
                            hipStream_t stream, const PrefillFold &pf = PrefillFold{}) {
     constexpr int BM = WM * MI * 32, NW = WM * NWN;
-    constexpr int kRing = kAStages * BM * 64 + (INC ? 2 * NW * 256 : RS ? 0 : kAStages * NW * 512);  // the A ring, behind it the groups' c or the extension's scales
-    constexpr int kStore = NW * MI * 32 * 64 * 2;   // the store's per-wavefront transposes (reuses the ring)
+    // the A rings, behind them the groups' c or the extension's scales
+    constexpr int kRing = WK * (kAStages * BM * 64 + (INC ? 2 * NW * 256 : RS ? 0 : kAStages * NW * 512)) + (WK == 2 && FOLD ? 1024 : 0);
+    // the store's per-wavefront transposes, or twice that where the halves of K meet (reuses the rings)
+    constexpr int kStore = NW * MI * 32 * 64 * 2 * WK;
     // RS: the row sums sit behind the ring and are dead by the time the store reuses the space
-    constexpr int kLdsMax = RS ? (kRing + kMaxRowSumBytes > kStore ? kRing + kMaxRowSumBytes : kStore)
+    constexpr int kLdsMax = RS ? (kRing + kMaxRowSumBytes + 256 > kStore ? kRing + kMaxRowSumBytes + 256 : kStore)
                                : (kRing > kStore ? kRing : kStore);
     int lds_bytes = kRing > kStore ? kRing : kStore;
-    if (RS && kRing + row_sum_bytes(max_groups) > lds_bytes) lds_bytes = kRing + row_sum_bytes(max_groups);
+    const int sums = row_sum_bytes((max_groups + WK - 1) / WK * WK);  // (each half of K: its own groups')
+    if (RS && kRing + sums > lds_bytes) lds_bytes = kRing + sums;
     // The 256 x 128 block fits twice on a compute unit.  A grid of at most one block per unit
     // asks for more LDS than two blocks could share, so the dispatcher cannot stack two blocks
     // on one unit while others idle.
     constexpr int kLdsSolo0 = (WM == 2 && NWN == 2) ? 96 * 1024 : kLdsMax;
     constexpr int kLdsSolo = FOLD && kLdsSolo0 < kProjectLdsBytes16 ? kProjectLdsBytes16 : kLdsSolo0;
-    const hipError_t attr = allow_dynamic_lds<&w4a16_prefill_kernel<NWN, WM, MI, SWIGLU, RS, FOLD, INC>>(kLdsSolo);
+    const hipError_t attr = allow_dynamic_lds<&w4a16_prefill_kernel<NWN, WM, MI, SWIGLU, RS, FOLD, INC, WK>>(kLdsSolo);
     if (attr != hipSuccess) return attr;
     if (WM == 2 && NWN == 2 && grid <= a.cus) lds_bytes = kLdsSolo;
     if (FOLD && lds_bytes < kProjectLdsBytes16) lds_bytes = kProjectLdsBytes16;  // the projection's blocks stage more
-    w4a16_prefill_kernel<NWN, WM, MI, SWIGLU, RS, FOLD, INC><<<grid + (FOLD ? pf.producers : 0), 64 * NW, lds_bytes, stream>>>(
+    w4a16_prefill_kernel<NWN, WM, MI, SWIGLU, RS, FOLD, INC, WK><<<grid + (FOLD ? pf.producers : 0), 64 * NW * WK, lds_bytes, stream>>>(
         (const uint16_t *)a.A, (const u32x4 *)a.B, (const uint16_t *)a.S, (uint16_t *)a.C, (const u32x4 *)a.aext,
         a.M, a.N, a.K, a.Gs, m_blocks, (const uint16_t *)a.lora_t, (const uint16_t *)a.lora_b, a.r_total, RP,
         a.nb_full, KS, GSb, a.partial, a.counters,
@@ -1231,16 +1349,29 @@ hipError_t launch_shape_as(const PrefillArgs &a, int grid, int m_blocks, int RP,
     return hipGetLastError();
 }
 
-template <int NWN, int WM, int MI>
+template <int NWN, int WM, int MI, int WK = 1>
 hipError_t launch_shape(const PrefillArgs &a, int grid, int m_blocks, int RP, int KS, int GSb, int max_groups,
                         bool rs, hipStream_t stream) {
     if constexpr (MI == 2) {
         if (rs)
-            return a.swiglu ? launch_shape_as<NWN, WM, MI, true, true>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream)
-                            : launch_shape_as<NWN, WM, MI, false, true>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream);
+            return a.swiglu ? launch_shape_as<NWN, WM, MI, true, true, false, false, WK>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream)
+                            : launch_shape_as<NWN, WM, MI, false, true, false, false, WK>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream);
     }
-    return a.swiglu ? launch_shape_as<NWN, WM, MI, true, false>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream)
-                    : launch_shape_as<NWN, WM, MI, false, false>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream);
+    return a.swiglu ? launch_shape_as<NWN, WM, MI, true, false, false, false, WK>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream)
+                    : launch_shape_as<NWN, WM, MI, false, false, false, false, WK>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream);
+}
+
+// A launch whose first blocks write what the others need (PrefillFold): blocks of 256 columns.
+template <int MI, int WK>
+hipError_t launch_fold(const PrefillArgs &a, int grid, int m_blocks, int RP, int KS, int GSb, int max_groups, bool rs,
+                       const PrefillFold &pf, hipStream_t stream) {
+    if constexpr (MI == 2) {
+        if (rs)
+            return a.swiglu ? launch_shape_as<4, 1, MI, true, true, true, false, WK>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream, pf)
+                            : launch_shape_as<4, 1, MI, false, true, true, false, WK>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream, pf);
+    }
+    return a.swiglu ? launch_shape_as<4, 1, MI, true, false, true, false, WK>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream, pf)
+                    : launch_shape_as<4, 1, MI, false, false, true, false, WK>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream, pf);
 }
 
 }  // namespace
@@ -1333,6 +1464,32 @@ static bool blocks_sum_their_rows(int M, int N, int K, const PrefillPlan &p) {
     return p.bm == 64 && row_sum_bytes(max_groups) <= kMaxRowSumBytes && (flops <= 28e9 || N <= 4096);
 }
 
+// Row-sum producers a launch should have: one per 64 rows, in eights.
+static int rowsum_producers_wanted(int M) { return ((M + 63) / 64 + 7) / 8 * 8; }
+
+// Blocks whose wavefronts share K (the kernel's WK): where the plan gives a compute unit one block at most, of enough groups
+// that half of them pay for the halves' meeting, and the row sums need no launch in front -- the blocks form them, or the
+// units without a block do.  By the plan alone, with adapters or without, and alike for both block widths (counted in blocks
+// of 256 columns), so that calls which must agree in every bit add in one order.  (84 shapes and row counts: 12 % faster
+// on average, 1 % slower at worst.  Shorter shares are level or slower: 11 groups in 128-row blocks, 4096 -> 2560 at 777 rows in
+// three slices, 33.7 us either way; 64-row blocks on every unit, 2816 -> 1024 at 2000 rows, 256 blocks of 11 groups, and
+// 2048 -> 2048 at 900, 2 to 7 % slower: the units' store and start then have nothing left to hide behind.)
+bool prefill_halves_k(int M, int N, int K, const PrefillPlan &p, int cus) {
+    if ((p.bm != 64 && p.bm != 128) || p.nb_full < 0 || p.nb_full > N / p.bn) return false;
+    const int G = K / kGroupK, ks = p.ks < 1 || p.nb_full == N / p.bn ? 1 : p.ks;  // (of whole tiles alone: nothing is sliced)
+    PrefillPlan wide = p;
+    wide.bn = 256;
+    wide.nb_full = p.nb_full * p.bn / 256;
+    const int grid = prefill_grid(M, N, wide), row_tiles = (M + 15) / 16;
+    if (grid > cus || (G + ks - 1) / ks < (p.bm == 64 && grid <= cus - 8 ? 6 : 16)) return false;
+    if (blocks_sum_their_rows(M, N, K, p)) return true;
+    // the producers' share must be done before a block's main loop is: 0.7 ns a row tile and value of K against
+    // 1.4 us a group
+    const int producers = (cus - grid) / 8 * 8;
+    if (row_tiles > kPrefillFoldMaxTiles || producers < rowsum_producers_wanted(M)) return false;
+    return (row_tiles + producers - 1) / producers * ks <= 11;
+}
+
 // Without adapters a few of the product's own first blocks form the row sums (rowsum_producer_block)
 // where the launch is a single round of blocks that leaves block slots free: producers in those
 // slots cost the product nothing and save the launch in front (down projection at 2048 rows
@@ -1344,11 +1501,11 @@ static bool blocks_sum_their_rows(int M, int N, int K, const PrefillPlan &p) {
 // their rows themselves.
 int prefill_rowsum_producers(int M, int N, int K, const PrefillPlan &p, int cus) {
     if (blocks_sum_their_rows(M, N, K, p)) return -2;
-    if ( p.bn != 256 || (p.bm != 64 && p.bm != 128) ||
+    if (p.bn != 256 || (p.bm != 64 && p.bm != 128) ||
         (M + 15) / 16 > kPrefillFoldMaxTiles || p.nb_full < 0 || p.nb_full > N / p.bn)
         return 0;
-    const int grid = prefill_grid(M, N, p), slots = cus * (p.bm == 128 ? 2 : 3);
-    const int want = ((M + 63) / 64 + 7) / 8 * 8, tiles8 = ((M + 15) / 16 + 7) / 8 * 8;
+    const int grid = prefill_grid(M, N, p), slots = cus * (prefill_halves_k(M, N, K, p, cus) ? 1 : p.bm == 128 ? 2 : 3);
+    const int want = rowsum_producers_wanted(M), tiles8 = ((M + 15) / 16 + 7) / 8 * 8;
     const int free_slots = (slots - grid) / 8 * 8;
     if (free_slots < want) return 0;
     const int producers = free_slots < tiles8 ? free_slots : tiles8;
@@ -1387,6 +1544,7 @@ hipError_t launch_prefill(const PrefillArgs &a, hipStream_t stream) {
     if (a.next_aext && !prefill_forms_next_sums(shape)) return hipErrorInvalidValue;
     const bool inc = a.sums_in_loop;
     if (inc && a.bm != 128) return hipErrorInvalidValue;
+    const bool halves = !inc && prefill_halves_k(a.M, a.N, a.K, shape, a.cus);
     const int inside = a.r_total == 0 && a.lora_words && !a.aext_ready && !inc ? prefill_rowsum_producers(a.M, a.N, a.K, shape, a.cus) : 0;
     const int sum_producers = inside > 0 ? inside : 0;
     int RP = 0;
@@ -1410,7 +1568,11 @@ hipError_t launch_prefill(const PrefillArgs &a, hipStream_t stream) {
         // so do 64-row blocks, three to a unit, which were never seen to suffer (gate+up at 512 rows, 768 blocks and
         // 256 producers for 768 slots: 62 us inside, 68 in front).
         bool room = true;
-        if (rb == 16 && a.bm == 128) {
+        // (Blocks whose wavefronts share K have a unit each: the projection is inside if all of its slices' blocks find free
+        // units, so that T's sums are added in one order wherever it runs.)
+        if (halves) {
+            room = prefill_grid(a.M, a.N, shape) + (row_tiles * kz + 7) / 8 * 8 <= a.cus;
+        } else if (rb == 16 && a.bm == 128) {
             const int slots = a.cus * 2, product = prefill_grid(a.M, a.N, shape);
             if (product <= slots && product + (row_tiles * kz + 7) / 8 * 8 > slots) {
                 const int cap = (slots - product) / 8 * 8 / row_tiles;
@@ -1481,14 +1643,11 @@ hipError_t launch_prefill(const PrefillArgs &a, hipStream_t stream) {
         if (inc)
             return a.swiglu ? launch_shape_as<4, 1, 4, true, false, true, true>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream, pf)
                             : launch_shape_as<4, 1, 4, false, false, true, true>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream, pf);
-        if (a.swiglu) {
-            if (a.bm == 128) return launch_shape_as<4, 1, 4, true, false, true>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream, pf);
-            return rs ? launch_shape_as<4, 1, 2, true, true, true>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream, pf)
-                      : launch_shape_as<4, 1, 2, true, false, true>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream, pf);
-        }
-        if (a.bm == 128) return launch_shape_as<4, 1, 4, false, false, true>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream, pf);
-        return rs ? launch_shape_as<4, 1, 2, false, true, true>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream, pf)
-                  : launch_shape_as<4, 1, 2, false, false, true>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream, pf);
+        if (halves)
+            return a.bm == 128 ? launch_fold<4, 2>(a, grid, m_blocks, RP, KS, GSb, max_groups, rs, pf, stream)
+                               : launch_fold<2, 2>(a, grid, m_blocks, RP, KS, GSb, max_groups, rs, pf, stream);
+        return a.bm == 128 ? launch_fold<4, 1>(a, grid, m_blocks, RP, KS, GSb, max_groups, rs, pf, stream)
+                           : launch_fold<2, 1>(a, grid, m_blocks, RP, KS, GSb, max_groups, rs, pf, stream);
     }
     if (inc && a.bn == 128) {  // through overrides only, which the fused calls do not take
         if (a.swiglu) return hipErrorInvalidValue;
@@ -1497,6 +1656,13 @@ hipError_t launch_prefill(const PrefillArgs &a, hipStream_t stream) {
     if (inc) {
         return a.swiglu ? launch_shape_as<4, 1, 4, true, false, false, true>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream)
                         : launch_shape_as<4, 1, 4, false, false, false, true>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream);
+    }
+    if (halves) {
+        if (a.bm == 128)
+            return a.bn == 256 ? launch_shape<4, 1, 4, 2>(a, grid, m_blocks, RP, KS, GSb, max_groups, rs, stream)
+                               : launch_shape<2, 1, 4, 2>(a, grid, m_blocks, RP, KS, GSb, max_groups, rs, stream);
+        return a.bn == 256 ? launch_shape<4, 1, 2, 2>(a, grid, m_blocks, RP, KS, GSb, max_groups, rs, stream)
+                           : launch_shape<2, 1, 2, 2>(a, grid, m_blocks, RP, KS, GSb, max_groups, rs, stream);
     }
     if (a.bm == 256) {
         return a.bn == 256 ? launch_shape<4, 2, 4>(a, grid, m_blocks, RP, KS, GSb, max_groups, rs, stream)

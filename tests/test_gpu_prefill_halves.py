@@ -1,0 +1,96 @@
+"""The matrix-core kernel's blocks whose wavefronts share K, each half of them taking half of the block's groups (launches of
+at most one block per compute unit).  Checked against the product in 64 bits where the split can go wrong: an odd number of
+groups (the second half begins with a group that is not its own), K slices whose last one is shorter, down to a single group,
+ragged rows, both block heights and widths, row sums formed by the blocks and by the units without one, per-column scales,
+groups whose scale is zero; with adapters, in the SwiGLU writer and under capture."""
+import ctypes
+
+import pytest
+import torch
+
+from kiln_amd import _lib, marlin_gemm
+
+pytestmark = pytest.mark.gpu
+RANKS, SCALES = (16, 32), (0.5, 1.0)
+
+SHAPES = [
+    (1500, 768, 1536, 128),     # the shortest: six groups, three to a half
+    (1500, 896, 1536, -1),      # seven
+    (1100, 3968, 512, 128),     # six slices of six groups, the last of one
+    (513, 2048, 2048, 128),     # three slices, the last of four groups; one row in the last row block
+    (600, 11008, 2048, 128),    # slices of 29 and 28 groups
+    (1300, 1536, 1536, 128),    # blocks of 128 columns
+    (1300, 1664, 1536, -1),     # the same, 13 groups
+    (777, 2688, 2560, 128),
+    (777, 9216, 2560, 128),     # 128-row blocks, row sums from the units without a block
+    (330, 11008, 4096, -1),     # the same, slices of 18 groups, the last of 14
+]
+
+
+def _operands(m, k, n, g):
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    plan = (ctypes.c_int * 8)()
+    assert _lib.load().kiln_w4a16_debug_gemm_plan(m, n, k, cus, plan) == 0 and (plan[0], plan[6], plan[7]) == (1, 0, 1)
+    gen = torch.Generator(device="cuda").manual_seed(m + k + n)
+    words = torch.randint(-2**31, 2**31, (k // 16, 2 * n), dtype=torch.int64, device="cuda", generator=gen).to(torch.int32)
+    scales = (torch.rand(1 if g == -1 else k // g, n, device="cuda", generator=gen) * 0.018 + 0.002).half()
+    if scales.shape[0] > 1:
+        scales[scales.shape[0] // 2, ::7] = 0
+    x = torch.randn(m, k, device="cuda", generator=gen)
+    return words, scales, [x.to(torch.bfloat16), (x * 0.5 + 0.5).to(torch.bfloat16)]
+
+
+@pytest.mark.parametrize("m,k,n,g", SHAPES)
+def test_result_against_64_bits(m, k, n, g):
+    words, scales, xs = _operands(m, k, n, g)
+    w = marlin_gemm.dequant_f32(words, scales, g).double()
+    eager = []
+    for x in xs:
+        y = marlin_gemm.marlin_w4a16_gemm(x, words, scales, g)
+        assert torch.equal(marlin_gemm.marlin_w4a16_gemm(x, words, scales, g).view(torch.int16), y.view(torch.int16))
+        widths = [marlin_gemm.marlin_w4a16_gemm(x, words, scales, g, thread_k=k, thread_n=t) for t in (128, 256)]
+        assert torch.equal(widths[0].view(torch.int16), widths[1].view(torch.int16))
+        want = x.double() @ w
+        # one rounding to bf16 (half an ulp: 2^-9 of the value's power of two) and f32 sums of a 136-fold surplus, 2e-4 of
+        # the result's norm, 1e-3 where the activations have a mean: together under 2^-8 of a row's norm
+        err = (y.double() - want).norm(dim=1) / want.norm(dim=1)
+        assert float(err.max()) <= 2.0 ** -8, float(err.max())
+        eager.append(y)
+    x, y = xs[0].clone(), torch.empty_like(eager[0])
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y.copy_(marlin_gemm.marlin_w4a16_gemm(x, words, scales, g))
+    for i in (1, 0, 1):
+        x.copy_(xs[i])
+        y.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y.view(torch.int16), eager[i].view(torch.int16)), i
+
+
+@pytest.mark.parametrize("m,k,n,g", SHAPES)
+def test_adapters_and_the_swiglu_writer(m, k, n, g):
+    words, scales, xs = _operands(m, k, n, g)
+    w = marlin_gemm.dequant_f32(words, scales, g).double()
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    a = (torch.randn(sum(RANKS), k, device="cuda", generator=gen) * k ** -0.5).to(torch.bfloat16)
+    b = (torch.randn(n, sum(RANKS), device="cuda", generator=gen) * 0.1).to(torch.bfloat16)
+    zeros = torch.zeros_like(b)
+    col = torch.tensor([s for r, s in zip(RANKS, SCALES) for _ in range(r)], dtype=torch.float64, device="cuda")
+    for x in xs:
+        plain = marlin_gemm.marlin_w4a16_gemm(x, words, scales, g)
+        assert torch.equal(marlin_gemm.marlin_w4a16_gemm_lora(x, words, scales, g, a, zeros, RANKS, SCALES), plain)
+        y = marlin_gemm.marlin_w4a16_gemm_lora(x, words, scales, g, a, b, RANKS, SCALES)
+        t = ((x.double() @ a.double().t()) * col).to(torch.bfloat16)    # rounded once, as T is kept
+        want = x.double() @ w + t.double() @ b.double().t()
+        # the plain call's bound, which has room for T's ties (under 1e-4 of the norm)
+        err = (y.double() - want).norm(dim=1) / want.norm(dim=1)
+        assert float(err.max()) <= 2.0 ** -8, float(err.max())
+        h = marlin_gemm.marlin_w4a16_gemm_swiglu(x, words, scales, g)
+        assert torch.equal(marlin_gemm.marlin_w4a16_gemm_swiglu_lora(x, words, scales, g, a, zeros, RANKS, SCALES), h)
+        # gate and up in turns of 8 columns; the bound of the two factors, each within 2^-8 less its rounding, and one rounding
+        pairs = (x.double() @ w).view(m, n // 16, 2, 8)
+        gate, up = pairs[:, :, 0].reshape(m, -1), pairs[:, :, 1].reshape(m, -1)
+        want_h = torch.nn.functional.silu(gate) * up
+        err = (h.double() - want_h).norm(dim=1) / want_h.norm(dim=1)
+        assert float(err.max()) <= 2.0 ** -7, float(err.max())
