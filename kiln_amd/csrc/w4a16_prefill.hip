@@ -1304,6 +1304,18 @@ PrefillPlan plan_prefill(int m, int n, int k, int cus, int force_bn, int force_b
         const PrefillPlan tall = plan_for_shape(m, n, k, cus, 256, 128, sliced_units);
         if (plan_cost(m, n, k, cus, tall) < plan_cost(m, n, k, cus, best)) best = tall;
     }
+    // 128-row tiles that would be cut in two slices, which sit two to a unit: whole where a unit's two sets of wavefronts can
+    // share them, which needs no exchange (us, two slices -> whole: 4096 -> 4096 at 1300 / 1536 rows 61 -> 54 / 62 -> 55,
+    // 9216 -> 2560 at 2300 / 2560 rows 119 -> 113 / 124 -> 117, 8192 -> 8192 at 768 rows 108 -> 101, 13824 -> 5120 at 1280
+    // rows 177 -> 168; 14 shapes and row counts, the least 1 %, 18944 -> 3584 at 2048 rows).  Tiles for fewer than two thirds
+    // of the units stay in three slices: 160 tiles of 8192 -> 8192 at 640 rows 88 in three, 97 whole, of 14336 -> 4096 at
+    // 1280 rows 143 against 161.
+    if (best.bm == 128 && best.bn == 256 && best.nb_full == 0 && best.ks == 2) {
+        PrefillPlan whole = best;
+        whole.nb_full = n / 256;
+        whole.ks = 1;
+        if (3 * ((m + 127) / 128) * (n / 256) >= 2 * cus && prefill_halves_k(m, n, k, whole, cus)) return whole;
+    }
     return best;
 }
 size_t prefill_partial_bytes(int m, int n, const PrefillPlan &p) {

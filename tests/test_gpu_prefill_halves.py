@@ -24,6 +24,7 @@ SHAPES = [
     (777, 2688, 2560, 128),
     (777, 9216, 2560, 128),     # 128-row blocks, row sums from the units without a block
     (330, 11008, 4096, -1),     # the same, slices of 18 groups, the last of 14
+    (1300, 4096, 4096, 128),    # 128-row blocks, whole tiles for two thirds of the units
 ]
 
 

@@ -112,3 +112,15 @@ def test_mid_m_plans(m, k, n, want):
 def test_matrix_core_block_rows(m, k, n, rows):
     kind, bm, bn = _route(m, k, n)
     assert kind == "matrix-core" and bm == rows and bn in (128, 256)
+
+
+@pytest.mark.parametrize("m,k,n,ks", [
+    (1300, 4096, 4096, 1), (1536, 4096, 4096, 1), (2560, 9216, 2560, 1), (768, 8192, 8192, 1),   # two slices would sit two to a unit
+    (640, 8192, 8192, 3), (2048, 9216, 2560, 3),                                                # too few tiles: three slices
+    (3072, 9216, 2560, 2), (1536, 13824, 5120, 2),                                              # no unit left for the row sums
+])
+def test_tall_tiles_are_whole_where_two_sets_of_wavefronts_share_them(m, k, n, ks):
+    out = (ctypes.c_int * 8)()
+    assert _lib.load().kiln_w4a16_debug_gemm_plan(m, n, k, CUS, out) == 0
+    whole = out[4] == n // 256
+    assert (out[0], out[2], out[3]) == (1, 128, 256) and (1 if whole else out[5]) == ks and out[7] == (ks == 1)
