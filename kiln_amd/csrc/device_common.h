@@ -13,6 +13,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
 
 // bf16 bit pattern 0x4300 | code is exactly 128 + code (bf16 has ulp 1 in
 // [128, 256)), so a packed pair of codes becomes a packed pair of bf16 values

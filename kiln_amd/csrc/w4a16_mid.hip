@@ -23,8 +23,7 @@
 //   * Scales in f32 by a running rescale of the accumulators (as in the prefill kernel); the
 //     B operand carries 136 + d, and the surplus 136 * sum(a) * scale is removed after the
 //     wavefront's last group by a short extra contraction (as in the prefill kernel) over the
-//     groups' row sums, which the vector unit forms from the fragments (v_dot2c_f32_bf16) while
-//     the matrix unit multiplies.
+//     groups' row sums, which small products (4x4x4) form from the fragments.
 // At the end the wavefronts' f32 tiles are summed through LDS in wavefront (= ascending K)
 // order; K slices of a tile meet in the workspace, last arriver adds in slice order.
 #include "async_loads.h"
@@ -304,8 +303,7 @@ __device__ __forceinline__ void mid_block(
         float s_cur[TP];
         float s_of[NG][TP];   // the scale of every group (this lane's column of each pair)
         float c_of[NG][RBN];  // -136 * (sum of the group's activations) of row 32 rb + l32
-        uint32_t ones;
-        asm("s_mov_b32 %0, 0x3f803f80" : "=s"(ones));  // bf16 (1, 1)
+        const s16x4 ones = {0x3F80, 0x3F80, 0x3F80, 0x3F80};  // bf16 1.0
         unrolled<0, NG>([&](auto gc) {
             constexpr int gi = decltype(gc)::value, set = gi % kSets;
             // this group's rows of A are in LDS; their fragments go to registers: lane (l32, h) holds
@@ -324,30 +322,27 @@ __device__ __forceinline__ void mid_block(
             wait_lds_reads();  // the slot (or this half of it) is free again
             if constexpr (gi + kASlots < NG) request_a(gi + kASlots);
             if constexpr (gi + D < NG) request_b(std::integral_constant<int, gi + D>{});
-            // Row sums of the group for the offset term, on the vector unit while the matrix unit
-            // multiplies: v_dot2c_f32_bf16 adds both halves of a register to an f32 sum (products with
-            // 1.0 are exact), two interleaved sums per row block; the lane's half of K here, the other
-            // half from lane + 32.
+            // Row sums of the group for the offset term, on the matrix unit: a 4x4x4 product of ones and four of the
+            // lane's values (products with 1.0 are exact) adds their sum to all four of the lane's results; the lane's
+            // half of K here, the other half from lane + 32.  (A dot instruction of the vector unit, v_dot2c_f32_bf16,
+            // takes 12 cycles from the matrix unit for two values, such a product 8 for four: 64 of the former a group
+            // were as long as half of its products.  Two layers of 50 rows 89.4 -> 86.4 us; 9216 -> 2560 at 48 rows 10.7 ->
+            // 10.3, 2560 -> 8192 at 24 rows 6.5 -> 6.2; the same error.)
+            f32x4 sums[RBN];
 #pragma unroll
-            for (int rb = 0; rb < RBN; ++rb) {
-                float e0 = 0.f, e1 = 0.f;
+            for (int rb = 0; rb < RBN; ++rb) sums[rb] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int s = 0; s < 7; ++s) {
-                    asm("v_dot2c_f32_bf16 %0, %2, %1" : "+v"(e0) : "v"(af[rb][s].x), "s"(ones));
-                    asm("v_dot2c_f32_bf16 %0, %2, %1" : "+v"(e1) : "v"(af[rb][s].y), "s"(ones));
-                    asm("v_dot2c_f32_bf16 %0, %2, %1" : "+v"(e0) : "v"(af[rb][s].z), "s"(ones));
-                    asm("v_dot2c_f32_bf16 %0, %2, %1" : "+v"(e1) : "v"(af[rb][s].w), "s"(ones));
-                }
-                asm("v_dot2c_f32_bf16 %0, %2, %1" : "+v"(e0) : "v"(af[rb][7].x), "s"(ones));
-                asm("v_dot2c_f32_bf16 %0, %2, %1" : "+v"(e1) : "v"(af[rb][7].y), "s"(ones));
-                // A dot instruction may feed its own kind as the addend back to back, but another
-                // vector instruction must wait three states before it reads the result; the compiler
-                // does not know what the asm holds, so the last link of each chain carries the wait.
-                asm("v_dot2c_f32_bf16 %0, %2, %1\n\ts_nop 3" : "+v"(e0) : "v"(af[rb][7].z), "s"(ones));
-                asm("v_dot2c_f32_bf16 %0, %2, %1\n\ts_nop 3" : "+v"(e1) : "v"(af[rb][7].w), "s"(ones));
-                const float half_sum = e0 + e1;
-                c_of[gi][rb] = -kCodeBias * (half_sum + __shfl_xor(half_sum, 32, 64));
-            }
+            for (int s = 0; s < 8; ++s)
+#pragma unroll
+                for (int half = 0; half < 2; ++half)
+#pragma unroll
+                    for (int rb = 0; rb < RBN; ++rb) {
+                        const u32x2 four = half ? u32x2{af[rb][s].z, af[rb][s].w} : u32x2{af[rb][s].x, af[rb][s].y};
+                        sums[rb] = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(ones, __builtin_bit_cast(s16x4, four), sums[rb], 0, 0, 0);
+                    }
+#pragma unroll
+            for (int rb = 0; rb < RBN; ++rb)
+                c_of[gi][rb] = -kCodeBias * (sums[rb][0] + __shfl_xor(sums[rb][0], 32, 64));
             wait_vector_loads<Sch::value.wait_b[gi]>();
             if constexpr (gi == 0) KILN_MID_TL(2);  // B(0) has arrived
 #pragma unroll

@@ -208,3 +208,26 @@ def test_mid_closed_forms_and_positive_activations(oracle):
     x = oracle.np_f32_to_bf16(np.abs(oracle.np_bf16_to_f32(x)))      # |N(0,1)|: what down_proj sees
     b, s = pack.repack_gptq(q, s_bits, None, g)
     _run_case(oracle, m, k, n, g, x, b, s, q, s_bits)
+
+
+@pytest.mark.parametrize("m", [17, 32, 33, 63, 64, 130])
+@pytest.mark.parametrize("k,n,g", [(128, 2048, 128), (1152, 1024, -1), (2560, 2560, 128), (4096, 2560, 128), (5120, 1024, -1)])
+def test_row_sums_against_64_bits(m, k, n, g):
+    """The groups' row sums, one to four groups a wavefront, ragged rows: with activations whose mean is as large as their
+    deviation the surplus they remove is far larger than the result, and with some of 2^-120 beside some of 2^60 a
+    sum that loses small values, or drops denormal ones, would show."""
+    import ctypes
+    out = (ctypes.c_int * 8)()
+    assert _lib.load().kiln_w4a16_debug_gemm_plan(m, n, k, 256, out) == 0 and (out[6] or m > 128)
+    gen = torch.Generator(device="cuda").manual_seed(m + k + n)
+    words = torch.randint(-2**31, 2**31, (k // 16, 2 * n), dtype=torch.int64, device="cuda", generator=gen).to(torch.int32)
+    scales = (torch.rand(1 if g == -1 else k // g, n, device="cuda", generator=gen) * 0.018 + 0.002).half()
+    w = marlin_gemm.dequant_f32(words, scales, g).double()
+    x = torch.randn(m, k, device="cuda", generator=gen)
+    spread = torch.full((m, 1), 2.0, device="cuda") ** torch.randint(-120, 60, (m, 1), device="cuda", generator=gen)
+    for xt in (x.to(torch.bfloat16), (x + 1).to(torch.bfloat16), (x * spread).to(torch.bfloat16)):
+        y = marlin_gemm.marlin_w4a16_gemm(xt, words, scales, g)
+        want = xt.double() @ w
+        # one rounding to bf16, and f32 sums of a 136-fold surplus: 1e-3 of a row's norm where the activations have a mean
+        err = (y.double() - want).norm(dim=1) / want.norm(dim=1)
+        assert float(err.max()) <= 2.0 ** -8, float(err.max())
