@@ -270,6 +270,22 @@ kiln_marlin_status_t kiln_w4a16_quantize_and_pack_device(
     void *b_packed, void *scales_f16, int dev, void *stream);
 
 /*
+ * kiln_w4a16_quantize_and_pack_device for `count` weights of one device at once: one launch for the weights of a
+ * groupsize, up to sixteen (three and one per weight with groupsize -1).  pair_b, pair_s: null, or the pack of gate and up interleaved
+ * (kiln_w4a16_interleave_gate_up, of n columns each), into which the weight goes as well -- pair_side 0: as gate, 1: as
+ * up.  Nothing is launched if any item is refused.
+ */
+typedef struct {
+    const void *weight_bf16;
+    int k, n, groupsize;
+    int pair_side;
+    void *b_packed, *scales_f16;
+    void *pair_b, *pair_s;
+} kiln_w4a16_quantize_item;
+kiln_marlin_status_t kiln_w4a16_quantize_and_pack_many_device(
+    const kiln_w4a16_quantize_item *items, int count, int dev, void *stream);
+
+/*
  * kiln_w4a16_interleave_gate_up (below) for packed projections that are in device memory: one
  * copy kernel on `stream`, same bits.  out_b: k * 2 n_each / 8 int32, out_s: (k/g) * 2 n_each fp16.
  */

@@ -28,6 +28,7 @@ EXPORTS = (
     "kiln_w4a16_mlp_workspace_bytes",
     "kiln_w4a16_stack_adapters",
     "kiln_w4a16_quantize_and_pack_device",
+    "kiln_w4a16_quantize_and_pack_many_device",
     "kiln_w4a16_interleave_gate_up_device",
     "kiln_w4a16_repack_gptq_device",
     "kiln_w4a16_interleave_gate_up",
@@ -203,6 +204,8 @@ def _load(tuning: bool) -> ctypes.CDLL:
                                             vp, vp, vp]
     L.kiln_w4a16_quantize_and_pack_device.restype = i
     L.kiln_w4a16_quantize_and_pack_device.argtypes = [vp, i, i, i, vp, vp, i, vp]
+    L.kiln_w4a16_quantize_and_pack_many_device.restype = i
+    L.kiln_w4a16_quantize_and_pack_many_device.argtypes = [vp, i, i, vp]
     L.kiln_w4a16_repack_gptq_device.restype = i
     L.kiln_w4a16_repack_gptq_device.argtypes = [vp, vp, vp, i, i, i, vp, vp, i, vp]
     L.kiln_w4a16_interleave_gate_up_device.restype = i

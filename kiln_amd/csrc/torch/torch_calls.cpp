@@ -35,7 +35,7 @@ struct Library {
     decltype(&kiln_w4a16_workspace_bytes) workspace_bytes = nullptr;
     decltype(&kiln_w4a16_mlp_workspace_bytes) mlp_workspace_bytes = nullptr;
     decltype(&kiln_w4a16_stack_adapters) stack_adapters = nullptr;
-    decltype(&kiln_w4a16_quantize_and_pack_device) quantize = nullptr;
+    decltype(&kiln_w4a16_quantize_and_pack_many_device) quantize = nullptr;
 };
 Library g_lib;  // written by bind() under the interpreter lock, like everything below
 
@@ -390,19 +390,22 @@ PyObject *py_mlp(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     END_HANDLE_TH_ERRORS
 }
 
-// quantize(inputs, side_by_side): every (contiguous bf16 [k, n] weight, groupsize) of the tuple `inputs`, all on one
+// quantize(inputs, side_by_side, gate_up): every (contiguous bf16 [k, n] weight, groupsize) of the tuple `inputs`, all on one
 // device, quantised and packed on the current stream -> a list of (words, scales), None where the shape is not
-// supported.  The inputs each tuple of `side_by_side` names by position (one k, one groupsize) get packed tensors that
-// lie one after the other in memory.
+// supported, and behind them the interleaved pack of each pair of `gate_up`.  The inputs each tuple of `side_by_side` names by
+// position (one k, one groupsize) get packed tensors that lie one after the other in memory; a pair of `gate_up` names a
+// gate and an up of one shape and groupsize, each in one pair at most.
 PyObject *py_quantize(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     HANDLE_TH_ERRORS
-    if (nargs != 2 || !g_lib.quantize || !PyTuple_CheckExact(args[0]) || !PyTuple_CheckExact(args[1]) || PyTuple_GET_SIZE(args[0]) == 0)
+    if (nargs != 3 || !g_lib.quantize || !PyTuple_CheckExact(args[0]) || !PyTuple_CheckExact(args[1]) || !PyTuple_CheckExact(args[2]) ||
+        PyTuple_GET_SIZE(args[0]) == 0)
         Py_RETURN_NONE;
     struct Item {
         at::Tensor w, b, s;
         int64_t k = 0, n = 0, groups = 0;
         int g = 0;
         bool supported = false;
+        int pair = -1, side = 0;  // the pair it is gate (0) or up (1) of
     };
     std::vector<Item> items((size_t)PyTuple_GET_SIZE(args[0]));
     for (size_t i = 0; i < items.size(); ++i) {
@@ -453,18 +456,47 @@ PyObject *py_quantize(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
             first += items[(size_t)i].n;
         }
     }
+    struct Pair {
+        at::Tensor b, s;
+    };
+    std::vector<Pair> pairs((size_t)PyTuple_GET_SIZE(args[2]));
+    for (size_t p = 0; p < pairs.size(); ++p) {
+        PyObject *o = PyTuple_GET_ITEM(args[2], (Py_ssize_t)p);
+        if (!PyTuple_CheckExact(o) || PyTuple_GET_SIZE(o) != 2) Py_RETURN_NONE;
+        Item *sides[2];
+        for (int i = 0; i < 2; ++i) {
+            const long at_ = PyLong_AsLong(PyTuple_GET_ITEM(o, i));
+            if (at_ < 0 || at_ >= (long)items.size() || !items[(size_t)at_].supported || items[(size_t)at_].pair >= 0) {
+                PyErr_Clear();
+                Py_RETURN_NONE;
+            }
+            sides[i] = &items[(size_t)at_];
+            sides[i]->pair = (int)p;
+            sides[i]->side = i;
+        }
+        const Item &gate = *sides[0], &up = *sides[1];
+        if (gate.k != up.k || gate.n != up.n || gate.g != up.g || gate.n > INT32_MAX / 2) Py_RETURN_NONE;
+        pairs[p].b = empty(gate.k / 8 * 2 * gate.n, at::kInt).view({gate.k / 16, 4 * gate.n});
+        pairs[p].s = empty(gate.groups * 2 * gate.n, at::kHalf).view({gate.groups, 2 * gate.n});
+    }
+    std::vector<kiln_w4a16_quantize_item> calls;
+    calls.reserve(items.size());
     for (Item &it : items) {
         if (!it.supported) continue;
         if (!it.b.defined()) place(it, empty(it.k / 8 * it.n, at::kInt), empty(it.groups * it.n, at::kHalf), 0);
-        if (g_lib.quantize(it.w.data_ptr(), (int)it.k, (int)it.n, it.g, it.b.data_ptr(), it.s.data_ptr(), device.index(), stream) != KILN_W4A16_OK)
-            Py_RETURN_NONE;
+        calls.push_back({it.w.data_ptr(), (int)it.k, (int)it.n, it.g, it.side, it.b.data_ptr(), it.s.data_ptr(),
+                         it.pair < 0 ? nullptr : pairs[(size_t)it.pair].b.data_ptr(),
+                         it.pair < 0 ? nullptr : pairs[(size_t)it.pair].s.data_ptr()});
     }
-    PyObject *list = PyList_New((Py_ssize_t)items.size());
+    if (g_lib.quantize(calls.data(), (int)calls.size(), device.index(), stream) != KILN_W4A16_OK) Py_RETURN_NONE;
+    PyObject *list = PyList_New((Py_ssize_t)(items.size() + pairs.size()));
     if (!list) return nullptr;
-    for (size_t i = 0; i < items.size(); ++i) {
+    for (size_t i = 0; i < items.size() + pairs.size(); ++i) {
         PyObject *entry = Py_None;
-        if (items[i].supported) {
-            PyObject *b = THPVariable_Wrap(std::move(items[i].b)), *s = THPVariable_Wrap(std::move(items[i].s));
+        if (i >= items.size() || items[i].supported) {
+            at::Tensor &tb = i < items.size() ? items[i].b : pairs[i - items.size()].b;
+            at::Tensor &ts = i < items.size() ? items[i].s : pairs[i - items.size()].s;
+            PyObject *b = THPVariable_Wrap(std::move(tb)), *s = THPVariable_Wrap(std::move(ts));
             entry = b && s ? PyTuple_Pack(2, b, s) : nullptr;
             Py_XDECREF(b);
             Py_XDECREF(s);

@@ -197,6 +197,20 @@ def _same_input_runs(inputs: Sequence[Tuple[torch.Tensor, int]], meta: Sequence[
     return runs
 
 
+def _gate_up_pairs(inputs: Sequence[Tuple[torch.Tensor, int]], meta: Sequence[PackEntry]) -> Dict[int, Tuple[int, int]]:
+    """layer -> positions in the queue of its gate and up, where both are there and the SwiGLU pack can be made of them."""
+    at = {(e.layer_idx, e.kind): i for i, e in enumerate(meta)}
+    pairs = {}
+    for layer_idx in sorted({e.layer_idx for e in meta}):
+        gate, up = at.get((layer_idx, PackKind.GateProj)), at.get((layer_idx, PackKind.UpProj))
+        if gate is None or up is None:
+            continue
+        (wg, gg), (wu, gu) = inputs[gate], inputs[up]
+        if wg.dim() == 2 and wg.shape == wu.shape and gg == gu and marlin_proj.shape_is_supported(*wg.shape):
+            pairs[layer_idx] = (gate, up)
+    return pairs
+
+
 def fuse_same_input(layer: LayerProjections) -> int:
     """Pack the members of every group of SAME_INPUT_GROUPS that the layer has packed (same k, same
     groupsize) side by side as one projection.  In the tile layout a packed weight is a sequence of column
@@ -234,24 +248,35 @@ def pack_layers(layers: Sequence[LayerProjections], kinds: Optional[Sequence[Pac
         li, lm = queue_layer(i, layer, kinds, groupsize)
         inputs += li
         meta += lm
-    packed = marlin_proj.pack_on_device(inputs, _same_input_runs(inputs, meta)) if fuse_same_input_groups else None
-    if packed is None:
-        packed = marlin_proj.pack_from_bf16_batch(inputs)
-    n_packed = 0
-    for entry, p in zip(meta, packed):
-        if p is not None:
-            install_packed(layers[entry.layer_idx], entry.kind, p, drop_bf16)
-            n_packed += 1
-    n_fused = 0
-    if fuse_gate_up:
-        for layer in layers:
-            g, u = layer.packed.get(PackKind.GateProj), layer.packed.get(PackKind.UpProj)
-            if g is None or u is None or g.k != u.k or g.n != u.n or g.n % 128 != 0:
-                continue
-            b_gu, s_gu = marlin_gemm.interleave_gate_up_device(g.b_packed, g.scales, u.b_packed, u.scales, g.groupsize)
-            layer.gate_up_fused = MarlinPackedProj(b_gu, s_gu, g.groupsize, g.k, 2 * g.n)
-            n_fused += 1
-    stats = {"inputs": len(inputs), "packed": n_packed, "kept_bf16": len(inputs) - n_packed, "gate_up_fused": n_fused}
-    if fuse_same_input_groups:
-        stats["same_input_fused"] = sum(fuse_same_input(layer) for layer in layers)
+    runs = _same_input_runs(inputs, meta) if fuse_same_input_groups else []
+    pairs = _gate_up_pairs(inputs, meta) if fuse_gate_up else {}
+    # what follows on the host runs beside the quantiser; the weights are let go when it is done
+    made = marlin_proj.pack_on_device_with_pairs(inputs, runs, tuple(pairs.values()), wait=False) if runs or pairs else None
+    try:
+        packed, gate_up = made if made is not None else (marlin_proj.pack_from_bf16_batch(inputs), [])
+        gate_up = dict(zip(pairs, gate_up))
+        n_packed = 0
+        for entry, p in zip(meta, packed):
+            if p is not None:
+                install_packed(layers[entry.layer_idx], entry.kind, p, drop_bf16)
+                n_packed += 1
+        n_fused = 0
+        if fuse_gate_up:
+            for i, layer in enumerate(layers):
+                if i in gate_up:
+                    layer.gate_up_fused = gate_up[i]
+                    n_fused += 1
+                    continue
+                g, u = layer.packed.get(PackKind.GateProj), layer.packed.get(PackKind.UpProj)
+                if g is None or u is None or g.k != u.k or g.n != u.n or g.n % 128 != 0:
+                    continue
+                b_gu, s_gu = marlin_gemm.interleave_gate_up_device(g.b_packed, g.scales, u.b_packed, u.scales, g.groupsize)
+                layer.gate_up_fused = MarlinPackedProj(b_gu, s_gu, g.groupsize, g.k, 2 * g.n)
+                n_fused += 1
+        stats = {"inputs": len(inputs), "packed": n_packed, "kept_bf16": len(inputs) - n_packed, "gate_up_fused": n_fused}
+        if fuse_same_input_groups:
+            stats["same_input_fused"] = sum(fuse_same_input(layer) for layer in layers)
+    finally:
+        if made is not None:
+            torch.cuda.current_stream(inputs[0][0].device).synchronize()
     return stats

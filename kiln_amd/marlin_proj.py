@@ -184,17 +184,30 @@ def pack_on_device(inputs: Sequence[tuple[torch.Tensor, int]],
     one k and groupsize whose packed forms are to lie one after the other in memory, which is what their
     side-by-side pack is (`layer_pack.fuse_same_input`).  An unsupported shape yields None; anything the library's own
     route refuses or treats otherwise makes the result None as a whole."""
+    made = pack_on_device_with_pairs(inputs, side_by_side, ())
+    return None if made is None else made[0]
+
+
+def pack_on_device_with_pairs(inputs: Sequence[tuple[torch.Tensor, int]], side_by_side: Sequence[Sequence[int]],
+                              gate_up: Sequence[tuple[int, int]], wait: bool = True):
+    """`pack_on_device`, and for each pair of `gate_up` (positions of a gate and an up of one shape and groupsize) the two
+    interleaved for the SwiGLU entry point, written as the weights are quantised: `(packed inputs, packed pairs)`.
+    Without `wait` the caller keeps the weights and waits for the device's current stream."""
     if _host_pack() or not inputs or not inputs[0][0].is_cuda:
         return None
     device = inputs[0][0].device
     torch.cuda.synchronize(device)    # the weights may come from any stream
-    inputs = tuple((t.to(torch.bfloat16).contiguous() if t.is_cuda else t, g) for t, g in inputs)
-    made = _calls.quantize(inputs, tuple(map(tuple, side_by_side)))
+    inputs = tuple((t if not t.is_cuda or (t.dtype is torch.bfloat16 and t.is_contiguous()) else t.to(torch.bfloat16).contiguous(), g)
+                   for t, g in inputs)
+    made = _calls.quantize(inputs, tuple(map(tuple, side_by_side)), tuple(map(tuple, gate_up)))
     if made is None:
         return None
     outs = [None if bs is None else _wrap(*bs, *t.shape, g) for bs, (t, g) in zip(made, inputs)]
-    torch.cuda.current_stream(device).synchronize()
-    return outs
+    pairs = [MarlinPackedProj(b, s, inputs[i][1], inputs[i][0].shape[0], 2 * inputs[i][0].shape[1])
+             for (b, s), (i, _) in zip(made[len(inputs):], gate_up)]
+    if wait:
+        torch.cuda.current_stream(device).synchronize()
+    return outs, pairs
 
 
 def pack_from_bf16(weight_t: torch.Tensor, groupsize: int) -> Optional[MarlinPackedProj]:
