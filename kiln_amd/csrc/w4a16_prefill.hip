@@ -347,7 +347,7 @@ __global__ __launch_bounds__(64 * WM * NWN * WK, (WM == 2 && NWN == 4) ? 1 : 2) 
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];  // the A ring; reused by the store
     static_assert(!FOLD || WM * NWN == 4, "the projection's blocks have four wavefronts");
     static_assert(!INC || (!RS && WM == 1 && MI == 4), "the row sums come from in front");
-    static_assert(WK == 1 || (WK == 2 && WM == 1 && !INC), "halves of K: one row of wavefronts, the contraction behind the loop");
+    static_assert(WK == 1 || (WK == 2 && WM == 1), "halves of K: one row of wavefronts");
     if constexpr (FOLD) {
         if ((int)blockIdx.x < pf.producers) {
             const int unit = blockIdx.x;
@@ -431,7 +431,7 @@ __global__ __launch_bounds__(64 * WM * NWN * WK, (WM == 2 && NWN == 4) ? 1 : 2) 
     // LDS: the halves' rings, then (with the look at a folded launch's words in front) what lies behind a ring
     const int ring = WK == 1 ? 0 : half * (kAStages * kAStageBytes);
     constexpr int kBehindRings = WK * kAStages * kAStageBytes + (WK == 2 && FOLD ? 1024 : 0);
-    [[maybe_unused]] constexpr int kPeekAt = WK == 1 ? kFoldPeekOffset : WK * kAStages * kAStageBytes;
+    [[maybe_unused]] constexpr int kPeekAt = WK == 1 ? kFoldPeekOffset : WK * kAStages * kAStageBytes + (INC ? WK * 2 * NW * 256 : 0);
 
     __shared__ uint32_t s_meeting[2];
     if constexpr (WK == 2) {
@@ -538,10 +538,11 @@ __global__ __launch_bounds__(64 * WM * NWN * WK, (WM == 2 && NWN == 4) ? 1 : 2) 
     // (wavefronts beyond the block's rows for a copy nobody reads, so that all count the same loads)
     constexpr int kSumSlot = NW * 256;
     static_assert((kAStages * kAStageBytes) % (2 * kSumSlot) == 0, "slots alternate by one bit of their offset");
-    [[maybe_unused]] int c_at = kAStages * kAStageBytes + h * 16;  // this group's slot; the next one's is c_at ^ kSumSlot
+    const int c_slots = WK * kAStages * kAStageBytes + (WK == 1 ? 0 : half * (2 * kSumSlot));
+    [[maybe_unused]] int c_at = c_slots + h * 16;                  // this group's slot; the next one's is c_at ^ kSumSlot
     [[maybe_unused]] const char *c_ptr = nullptr;                  // this group's c in memory
     [[maybe_unused]] const uint32_t c_off = (uint32_t)min(m0 + (wave % (BM / 64)) * 64 + lane, M - 1) * 4u;
-    [[maybe_unused]] int c_to = kAStages * kAStageBytes + wave * 256;  // offsets: the slots' bit is theirs, not the base's
+    [[maybe_unused]] int c_to = c_slots + wave * 256;              // offsets: the slots' bit is theirs, not the base's
     if constexpr (INC) c_ptr = uniform(reinterpret_cast<const char *>(aext) + (size_t)g_begin * M * 4);
     request_b(bw, b_ptr, s_ptr);
     if constexpr (INC) load_to_lds_b32(c_ptr, c_off, lds_base + c_to);
@@ -1306,7 +1307,7 @@ PrefillPlan plan_prefill(int m, int n, int k, int cus, int force_bn, int force_b
     }
     // 128-row tiles that would be cut in two slices, which sit two to a unit: whole where a unit's two sets of wavefronts can
     // share them, which needs no exchange (us, two slices -> whole: 4096 -> 4096 at 1300 / 1536 rows 61 -> 54 / 62 -> 55,
-    // 9216 -> 2560 at 2300 / 2560 rows 119 -> 113 / 124 -> 117, 8192 -> 8192 at 768 rows 108 -> 101, 13824 -> 5120 at 1280
+    // 9216 -> 2560 at 2300 / 2560 / 3072 rows 119 -> 113 / 124 -> 117 / 141 -> 137, 8192 -> 8192 at 768 rows 108 -> 101, 13824 -> 5120 at 1280
     // rows 177 -> 168; 14 shapes and row counts, the least 1 %, 18944 -> 3584 at 2048 rows).  Tiles for fewer than two thirds
     // of the units stay in three slices: 160 tiles of 8192 -> 8192 at 640 rows 88 in three, 97 whole, of 14336 -> 4096 at
     // 1280 rows 143 against 161.
@@ -1384,6 +1385,14 @@ hipError_t launch_fold(const PrefillArgs &a, int grid, int m_blocks, int RP, int
     }
     return a.swiglu ? launch_shape_as<4, 1, MI, true, false, true, false, WK>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream, pf)
                     : launch_shape_as<4, 1, MI, false, false, true, false, WK>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream, pf);
+}
+
+// A launch that adds the row sums at the groups' changes (INC): blocks of 128 rows and 256 columns.
+template <bool FOLD, int WK>
+hipError_t launch_sums_in_loop(const PrefillArgs &a, int grid, int m_blocks, int RP, int KS, int GSb, int max_groups,
+                               const PrefillFold &pf, hipStream_t stream) {
+    return a.swiglu ? launch_shape_as<4, 1, 4, true, false, FOLD, true, WK>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream, pf)
+                    : launch_shape_as<4, 1, 4, false, false, FOLD, true, WK>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream, pf);
 }
 
 }  // namespace
@@ -1480,12 +1489,16 @@ static bool blocks_sum_their_rows(int M, int N, int K, const PrefillPlan &p) {
 static int rowsum_producers_wanted(int M) { return ((M + 63) / 64 + 7) / 8 * 8; }
 
 // Blocks whose wavefronts share K (the kernel's WK): where the plan gives a compute unit one block at most, of enough groups
-// that half of them pay for the halves' meeting, and the row sums need no launch in front -- the blocks form them, or the
-// units without a block do.  By the plan alone, with adapters or without, and alike for both block widths (counted in blocks
+// that half of them pay for the halves' meeting.  The row sums: from the blocks, from the units without a block where they
+// can be done in time, else, for whole tiles, from a launch in front, which 128-row blocks then add at the changes of group.  By the plan alone, with adapters or without, and alike for both block widths (counted in blocks
 // of 256 columns), so that calls which must agree in every bit add in one order.  (84 shapes and row counts: 12 % faster
 // on average, 1 % slower at worst.  Shorter shares are level or slower: 11 groups in 128-row blocks, 4096 -> 2560 at 777 rows in
 // three slices, 33.7 us either way; 64-row blocks on every unit, 2816 -> 1024 at 2000 rows, 256 blocks of 11 groups, and
-// 2048 -> 2048 at 900, 2 to 7 % slower: the units' store and start then have nothing left to hide behind.)
+// 2048 -> 2048 at 900, 2 to 7 % slower: the units' store and start then have nothing left to hide behind.  With the sums
+// from a launch in front, tiles for nine tenths of the units or all: 4096 -> 4096 at 1900 / 2048 rows 74 -> 67 us, 4096 -> 2560
+// at 3072 82 -> 75, 8192 -> 8192 at 1024 133 -> 123, 14336 -> 4096 at 2048 228 -> 213, 28672 -> 8192 at 1000 470 -> 415,
+// 2560 -> 8192 at 1024 47.0 -> 46.1, the least.  Launches of several rounds are slower so: 2560 -> 18432 at 777 / 4096 rows 72 ->
+// 80 / 307 -> 343, one block of eight wavefronts a unit in place of two of four.)
 bool prefill_halves_k(int M, int N, int K, const PrefillPlan &p, int cus) {
     if ((p.bm != 64 && p.bm != 128) || p.nb_full < 0 || p.nb_full > N / p.bn) return false;
     const int G = K / kGroupK, ks = p.ks < 1 || p.nb_full == N / p.bn ? 1 : p.ks;  // (of whole tiles alone: nothing is sliced)
@@ -1498,7 +1511,7 @@ bool prefill_halves_k(int M, int N, int K, const PrefillPlan &p, int cus) {
     // the producers' share must be done before a block's main loop is: 0.7 ns a row tile and value of K against
     // 1.4 us a group
     const int producers = (cus - grid) / 8 * 8;
-    if (row_tiles > kPrefillFoldMaxTiles || producers < rowsum_producers_wanted(M)) return false;
+    if (row_tiles > kPrefillFoldMaxTiles || producers < rowsum_producers_wanted(M)) return ks == 1;  // (from a launch in front)
     return (row_tiles + producers - 1) / producers * ks <= 11;
 }
 
@@ -1556,7 +1569,7 @@ hipError_t launch_prefill(const PrefillArgs &a, hipStream_t stream) {
     if (a.next_aext && !prefill_forms_next_sums(shape)) return hipErrorInvalidValue;
     const bool inc = a.sums_in_loop;
     if (inc && a.bm != 128) return hipErrorInvalidValue;
-    const bool halves = !inc && prefill_halves_k(a.M, a.N, a.K, shape, a.cus);
+    const bool halves = prefill_halves_k(a.M, a.N, a.K, shape, a.cus);
     const int inside = a.r_total == 0 && a.lora_words && !a.aext_ready && !inc ? prefill_rowsum_producers(a.M, a.N, a.K, shape, a.cus) : 0;
     const int sum_producers = inside > 0 ? inside : 0;
     int RP = 0;
@@ -1653,8 +1666,8 @@ hipError_t launch_prefill(const PrefillArgs &a, hipStream_t stream) {
     if (fold) {
         pf.consumers = grid;
         if (inc)
-            return a.swiglu ? launch_shape_as<4, 1, 4, true, false, true, true>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream, pf)
-                            : launch_shape_as<4, 1, 4, false, false, true, true>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream, pf);
+            return halves ? launch_sums_in_loop<true, 2>(a, grid, m_blocks, RP, KS, GSb, max_groups, pf, stream)
+                          : launch_sums_in_loop<true, 1>(a, grid, m_blocks, RP, KS, GSb, max_groups, pf, stream);
         if (halves)
             return a.bm == 128 ? launch_fold<4, 2>(a, grid, m_blocks, RP, KS, GSb, max_groups, rs, pf, stream)
                                : launch_fold<2, 2>(a, grid, m_blocks, RP, KS, GSb, max_groups, rs, pf, stream);
@@ -1663,12 +1676,12 @@ hipError_t launch_prefill(const PrefillArgs &a, hipStream_t stream) {
     }
     if (inc && a.bn == 128) {  // through overrides only, which the fused calls do not take
         if (a.swiglu) return hipErrorInvalidValue;
-        return launch_shape_as<2, 1, 4, false, false, false, true>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream);
+        return halves ? launch_shape_as<2, 1, 4, false, false, false, true, 2>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream)
+                      : launch_shape_as<2, 1, 4, false, false, false, true>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream);
     }
-    if (inc) {
-        return a.swiglu ? launch_shape_as<4, 1, 4, true, false, false, true>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream)
-                        : launch_shape_as<4, 1, 4, false, false, false, true>(a, grid, m_blocks, RP, KS, GSb, max_groups, stream);
-    }
+    if (inc)
+        return halves ? launch_sums_in_loop<false, 2>(a, grid, m_blocks, RP, KS, GSb, max_groups, pf, stream)
+                      : launch_sums_in_loop<false, 1>(a, grid, m_blocks, RP, KS, GSb, max_groups, pf, stream);
     if (halves) {
         if (a.bm == 128)
             return a.bn == 256 ? launch_shape<4, 1, 4, 2>(a, grid, m_blocks, RP, KS, GSb, max_groups, rs, stream)

@@ -2,7 +2,7 @@
 at most one block per compute unit).  Checked against the product in 64 bits where the split can go wrong: an odd number of
 groups (the second half begins with a group that is not its own), K slices whose last one is shorter, down to a single group,
 ragged rows, both block heights and widths, row sums formed by the blocks and by the units without one, per-column scales,
-groups whose scale is zero; with adapters, in the SwiGLU writer and under capture."""
+groups whose scale is zero; row sums added at the changes of group; with adapters, in the SwiGLU writer and under capture."""
 import ctypes
 
 import pytest
@@ -25,6 +25,9 @@ SHAPES = [
     (777, 9216, 2560, 128),     # 128-row blocks, row sums from the units without a block
     (330, 11008, 4096, -1),     # the same, slices of 18 groups, the last of 14
     (1300, 4096, 4096, 128),    # 128-row blocks, whole tiles for two thirds of the units
+    (3001, 2176, 2560, 128),    # row sums from a launch in front, added at the changes of group: 17 groups
+    (1900, 4096, 4096, -1),     # the same, 32 groups
+    (1024, 2048, 8192, 128),    # the same, a tile for every unit, 16 groups
 ]
 
 

@@ -116,8 +116,8 @@ def test_matrix_core_block_rows(m, k, n, rows):
 
 @pytest.mark.parametrize("m,k,n,ks", [
     (1300, 4096, 4096, 1), (1536, 4096, 4096, 1), (2560, 9216, 2560, 1), (768, 8192, 8192, 1),   # two slices would sit two to a unit
+    (3072, 9216, 2560, 1), (1536, 13824, 5120, 1),                                              # (row sums from a launch in front)
     (640, 8192, 8192, 3), (2048, 9216, 2560, 3),                                                # too few tiles: three slices
-    (3072, 9216, 2560, 2), (1536, 13824, 5120, 2),                                              # no unit left for the row sums
 ])
 def test_tall_tiles_are_whole_where_two_sets_of_wavefronts_share_them(m, k, n, ks):
     out = (ctypes.c_int * 8)()
