@@ -199,7 +199,7 @@ struct PrefillPlan {
     int ks = 1;       // K slices of the remaining column blocks
 };
 PrefillPlan plan_prefill(int m, int n, int k, int cus, int force_bn = 0, int force_bm = 0);
-int prefill_grid(int m, int n, const PrefillPlan &p);
+int prefill_grid(int m, int n, const PrefillPlan &p, int cus);
 size_t prefill_partial_bytes(int m, int n, const PrefillPlan &p);
 bool prefill_halves_k(int m, int n, int k, const PrefillPlan &p, int cus);         // do a block's wavefronts share K?
 int prefill_rowsum_producers(int m, int n, int k, const PrefillPlan &p, int cus);  // blocks of a plain launch that form the row sums inside it (0: a launch in front does, -2: every block its own)

@@ -392,21 +392,32 @@ __global__ __launch_bounds__(64 * WM * NWN * WK, (WM == 2 && NWN == 4) ? 1 : 2) 
     // row blocks of one unit back to back.  Blocks resident on a die at one time
     // therefore share the few row blocks of A the die owns (they stay in its L2,
     // where the loads that feed the matrix cores three stages ahead must hit) and
-    // read each unit's weights from memory once.
+    // read each unit's weights from memory once.  (die_rows == 0: no rectangles, prefill_die_rows.)
     int id = blockIdx.x;
     if constexpr (FOLD) id -= pf.producers;
     [[maybe_unused]] const int consumer = id;
     const int n_blocks = N / BN;
-    const int die_cols = 8 / die_rows, rows_per_die = (m_blocks + die_rows - 1) / die_rows;
-    const int per_die_full = rows_per_die * ((nb_full + die_cols - 1) / die_cols);
-    const bool sliced = id >= 8 * per_die_full;
-    if (sliced) id -= 8 * per_die_full;
-    const int units = sliced ? (n_blocks - nb_full) * KS : nb_full;  // per row block
-    const int units_per_die = (units + die_cols - 1) / die_cols;
-    const int die = id & 7, seq = id >> 3;
-    const int unit = (die / die_rows) * units_per_die + seq / rows_per_die;
-    const int mb = (die % die_rows) * rows_per_die + seq % rows_per_die;
-    if (seq >= rows_per_die * units_per_die || unit >= units || mb >= m_blocks) {  // grid padding (whole block, before any barrier)
+    bool sliced, padding;
+    int unit, mb;
+    if (die_rows == 0) {  // whole tiles one after the other, the same number to every die but for the last
+        const int per_die = (m_blocks * n_blocks + 7) >> 3, seq = id >> 3, tile = (id & 7) * per_die + seq;
+        unit = tile / m_blocks;
+        mb = tile - unit * m_blocks;
+        sliced = nb_full == 0;
+        padding = seq >= per_die || unit >= n_blocks;
+    } else {
+        const int die_cols = 8 / die_rows, rows_per_die = (m_blocks + die_rows - 1) / die_rows;
+        const int per_die_full = rows_per_die * ((nb_full + die_cols - 1) / die_cols);
+        sliced = id >= 8 * per_die_full;
+        if (sliced) id -= 8 * per_die_full;
+        const int units = sliced ? (n_blocks - nb_full) * KS : nb_full;  // per row block
+        const int units_per_die = (units + die_cols - 1) / die_cols;
+        const int die = id & 7, seq = id >> 3;
+        unit = (die / die_rows) * units_per_die + seq / rows_per_die;
+        mb = (die % die_rows) * rows_per_die + seq % rows_per_die;
+        padding = seq >= rows_per_die * units_per_die || unit >= units || mb >= m_blocks;
+    }
+    if (padding) {  // (whole block, before any barrier)
         if constexpr (FOLD) {
             if (wave_all == 0) prefill_fold_done(pf, consumer, lane);  // counted like the others: it will never look
         }
@@ -1154,7 +1165,13 @@ size_t prefill_lora_t_bytes(int m, bool few_rows) {
 // eight columns for any odd count, which leaves dies idle wherever the units are fewer than eight or do not
 // divide by eight: 1024 -> 1024 at 20000 rows, 313 row blocks of three whole column blocks and one more, ran
 // 165 us on three dies and then one, against 58 us at 19968 rows.)
-static int prefill_die_rows(int m_blocks, int units_full, int units_sliced, int ks) {
+//
+// 0: no grid -- whole tiles that are no more than the compute units, where every grid leaves a die more of them than it has
+// units (13 row blocks x 18 column blocks: 36 on six dies of 32 units): they are dealt one after the other, the row blocks
+// of a column block first, and every die gets the same number.  (A second round of a few blocks each, and no second set of
+// wavefronts: 3584 -> 4608 at 777 rows 58 -> 42 us, 4096 -> 3584 at 1100 64 -> 43, 18944 -> 3584 at 1100 233 -> 163; 128-row
+// blocks, 4096 -> 2560 at 3200 rows 93 -> 67, 9216 -> 2560 at 3200 201 -> 140.)
+static int prefill_die_rows(int m_blocks, int units_full, int units_sliced, int ks, int cus) {
     int best = 1;
     long best_work = -1;
     for (int dr = 8; dr >= 1; dr >>= 1) {
@@ -1165,16 +1182,23 @@ static int prefill_die_rows(int m_blocks, int units_full, int units_sliced, int 
             best_work = work;
         }
     }
+    if (units_sliced == 0 || (units_full == 0 && ks == 1)) {
+        const int dc = 8 / best, units = units_full + units_sliced;
+        const long tiles = (long)m_blocks * units, on_a_die = (long)((m_blocks + best - 1) / best) * ((units + dc - 1) / dc);
+        if (8 * on_a_die > cus && (tiles + 7) / 8 * 8 <= cus) return 0;
+    }
     return best;
 }
-static int prefill_die_rows(int m_blocks, int n, const PrefillPlan &p) {
-    return prefill_die_rows(m_blocks, p.nb_full, (n / p.bn - p.nb_full) * p.ks, p.ks);
+static int prefill_die_rows(int m_blocks, int n, const PrefillPlan &p, int cus) {
+    return prefill_die_rows(m_blocks, p.nb_full, (n / p.bn - p.nb_full) * p.ks, p.ks, cus);
 }
 
 // blocks launched: whole tiles, then (tile, K slice) units, each part padded to the die grid
-int prefill_grid(int m, int n, const PrefillPlan &p) {
+int prefill_grid(int m, int n, const PrefillPlan &p, int cus) {
     const int m_blocks = (m + p.bm - 1) / p.bm;
-    const int dr = prefill_die_rows(m_blocks, n, p), dc = 8 / dr, rows = (m_blocks + dr - 1) / dr;
+    const int dr = prefill_die_rows(m_blocks, n, p, cus);
+    if (dr == 0) return (m_blocks * (n / p.bn) + 7) / 8 * 8;
+    const int dc = 8 / dr, rows = (m_blocks + dr - 1) / dr;
     const int units_full = p.nb_full, units_sliced = (n / p.bn - p.nb_full) * p.ks;
     return 8 * rows * ((units_full + dc - 1) / dc) + 8 * rows * ((units_sliced + dc - 1) / dc);
 }
@@ -1204,11 +1228,11 @@ static PrefillPlan plan_for_shape(int m, int n, int k, int cus, int bn, int bm, 
         for (int ks = 2; ks <= 8 && G / ks >= 3; ++ks) {
             const int gsb = (G + ks - 1) / ks;
             if ((ks - 1) * gsb >= G) continue;  // would leave an empty slice
-            const int dr = prefill_die_rows(m_blocks, p.nb_full, rest * ks, ks), dc = 8 / dr;
+            const int dr = prefill_die_rows(m_blocks, p.nb_full, rest * ks, ks, 0), dc = 8 / dr;
             if (8 * ((m_blocks + dr - 1) / dr) * ((rest * ks + dc - 1) / dc) <= sliced_units) p.ks = ks;
         }
         if (p.nb_full == 0 || p.nb_full == n_blocks) break;
-        const int dr = prefill_die_rows(m_blocks, p.nb_full, rest * p.ks, p.ks), dc = 8 / dr;
+        const int dr = prefill_die_rows(m_blocks, p.nb_full, rest * p.ks, p.ks, 0), dc = 8 / dr;
         if (((m_blocks + dr - 1) / dr) * ((p.nb_full + dc - 1) / dc) <= rounds * (cus / 8)) break;
     }
     return p;
@@ -1358,7 +1382,7 @@ hipError_t launch_shape_as(const PrefillArgs &a, int grid, int m_blocks, int RP,
         (const uint16_t *)a.A, (const u32x4 *)a.B, (const uint16_t *)a.S, (uint16_t *)a.C, (const u32x4 *)a.aext,
         a.M, a.N, a.K, a.Gs, m_blocks, (const uint16_t *)a.lora_t, (const uint16_t *)a.lora_b, a.r_total, RP,
         a.nb_full, KS, GSb, a.partial, a.counters,
-        prefill_die_rows(m_blocks, a.nb_full, (a.N / (NWN * 64) - a.nb_full) * KS, KS), (u32x4 *)a.next_aext, a.next_plain, pf);
+        prefill_die_rows(m_blocks, a.nb_full, (a.N / (NWN * 64) - a.nb_full) * KS, KS, a.cus), (u32x4 *)a.next_aext, a.next_plain, pf);
     return hipGetLastError();
 }
 
@@ -1505,7 +1529,7 @@ bool prefill_halves_k(int M, int N, int K, const PrefillPlan &p, int cus) {
     PrefillPlan wide = p;
     wide.bn = 256;
     wide.nb_full = p.nb_full * p.bn / 256;
-    const int grid = prefill_grid(M, N, wide), row_tiles = (M + 15) / 16;
+    const int grid = prefill_grid(M, N, wide, cus), row_tiles = (M + 15) / 16;
     if (grid > cus || (G + ks - 1) / ks < (p.bm == 64 && grid <= cus - 8 ? 6 : 16)) return false;
     if (blocks_sum_their_rows(M, N, K, p)) return true;
     // the producers' share must be done before a block's main loop is: 0.7 ns a row tile and value of K against
@@ -1529,7 +1553,7 @@ int prefill_rowsum_producers(int M, int N, int K, const PrefillPlan &p, int cus)
     if (p.bn != 256 || (p.bm != 64 && p.bm != 128) ||
         (M + 15) / 16 > kPrefillFoldMaxTiles || p.nb_full < 0 || p.nb_full > N / p.bn)
         return 0;
-    const int grid = prefill_grid(M, N, p), slots = cus * (prefill_halves_k(M, N, K, p, cus) ? 1 : p.bm == 128 ? 2 : 3);
+    const int grid = prefill_grid(M, N, p, cus), slots = cus * (prefill_halves_k(M, N, K, p, cus) ? 1 : p.bm == 128 ? 2 : 3);
     const int want = rowsum_producers_wanted(M), tiles8 = ((M + 15) / 16 + 7) / 8 * 8;
     const int free_slots = (slots - grid) / 8 * 8;
     if (free_slots < want) return 0;
@@ -1596,9 +1620,9 @@ hipError_t launch_prefill(const PrefillArgs &a, hipStream_t stream) {
         // (Blocks whose wavefronts share K have a unit each: the projection is inside if all of its slices' blocks find free
         // units, so that T's sums are added in one order wherever it runs.)
         if (halves) {
-            room = prefill_grid(a.M, a.N, shape) + (row_tiles * kz + 7) / 8 * 8 <= a.cus;
+            room = prefill_grid(a.M, a.N, shape, a.cus) + (row_tiles * kz + 7) / 8 * 8 <= a.cus;
         } else if (rb == 16 && a.bm == 128) {
-            const int slots = a.cus * 2, product = prefill_grid(a.M, a.N, shape);
+            const int slots = a.cus * 2, product = prefill_grid(a.M, a.N, shape, a.cus);
             if (product <= slots && product + (row_tiles * kz + 7) / 8 * 8 > slots) {
                 const int cap = (slots - product) / 8 * 8 / row_tiles;
                 room = cap >= 1;
@@ -1662,7 +1686,7 @@ hipError_t launch_prefill(const PrefillArgs &a, hipStream_t stream) {
     const int GSb = (G + KS - 1) / KS;
     if (KS > 1 && (!a.partial || !a.counters || (KS - 1) * GSb >= G)) return hipErrorInvalidValue;
     if (a.nb_full < 0 || a.nb_full > a.N / a.bn) return hipErrorInvalidValue;
-    const int grid = prefill_grid(a.M, a.N, shape);
+    const int grid = prefill_grid(a.M, a.N, shape, a.cus);
     if (fold) {
         pf.consumers = grid;
         if (inc)

@@ -28,6 +28,10 @@ SHAPES = [
     (3001, 2176, 2560, 128),    # row sums from a launch in front, added at the changes of group: 17 groups
     (1900, 4096, 4096, -1),     # the same, 32 groups
     (1024, 2048, 8192, 128),    # the same, a tile for every unit, 16 groups
+    # tiles dealt to the dies one after the other (13, 14 and 25 row blocks)
+    (777, 3584, 4608, 128),     # 64-row blocks, row sums from the blocks
+    (850, 3584, 4608, -1),      # ... from a launch in front
+    (3137, 2176, 2560, 128),    # 128-row blocks
 ]
 
 
