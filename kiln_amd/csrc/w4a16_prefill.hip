@@ -1341,6 +1341,19 @@ PrefillPlan plan_prefill(int m, int n, int k, int cus, int force_bn, int force_b
         whole.ks = 1;
         if (3 * ((m + 127) / 128) * (n / 256) >= 2 * cus && prefill_halves_k(m, n, k, whole, cus)) return whole;
     }
+    // Three slices or more of 128-row tiles, of at most 16 groups, beyond 512 rows: as many of 64-row tiles, two blocks to a
+    // unit, where these sum their rows themselves.  The taller blocks' short main loop waits for the blocks that form the row
+    // sums, one per 16 rows (us, 128 -> 64 rows: 4096 -> 2560 at 777 / 900 / 1000 rows 35.1 -> 32.2 / 35.5 -> 32.8 / 36.1 -> 34.4,
+    // 4096 -> 4096 at 640 36.5 -> 33.2, 3072 -> 2560 at 777 30.8 -> 26.9, 6144 -> 2560 at 1000 46.5 -> 44.8, the least; 51
+    // shapes and row counts, 4 to 13 %.  At 450 and 512 rows it is level to 9 %, 5120 -> 4608 2 % behind; in longer shares
+    // level, 9216 -> 2560 at 900).
+    if (best.bm == 128 && best.bn == 256 && best.nb_full == 0 && best.ks >= 3 && m > 512 &&
+        (k / kGroupK + best.ks - 1) / best.ks <= 16 && !prefill_halves_k(m, n, k, best, cus)) {
+        PrefillPlan low = best;
+        low.bm = 64;
+        const int grid = prefill_grid(m, n, low, cus);
+        if (grid > cus && grid <= 2 * cus && prefill_rowsum_producers(m, n, k, low, cus) == -2) return low;
+    }
     return best;
 }
 size_t prefill_partial_bytes(int m, int n, const PrefillPlan &p) {

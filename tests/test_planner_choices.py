@@ -124,3 +124,13 @@ def test_tall_tiles_are_whole_where_two_sets_of_wavefronts_share_them(m, k, n, k
     assert _lib.load().kiln_w4a16_debug_gemm_plan(m, n, k, CUS, out) == 0
     whole = out[4] == n // 256
     assert (out[0], out[2], out[3]) == (1, 128, 256) and (1 if whole else out[5]) == ks and out[7] == (ks == 1)
+
+
+@pytest.mark.parametrize("m,k,n,rows", [
+    (513, 4096, 4096, 64), (777, 4096, 2560, 64), (1000, 6144, 2560, 64), (1000, 3072, 2560, 64),  # short slices: 64-row blocks sum their rows
+    (512, 4096, 4608, 128), (900, 9216, 2560, 128), (777, 9216, 2560, 128),                       # up to 512 rows; longer ones
+])
+def test_short_slices_of_more_than_512_rows_are_of_64_row_tiles(m, k, n, rows):
+    out = (ctypes.c_int * 8)()
+    assert _lib.load().kiln_w4a16_debug_gemm_plan(m, n, k, CUS, out) == 0
+    assert (out[0], out[2], out[3], out[5]) == (1, rows, 256, 3) and out[4] == 0
