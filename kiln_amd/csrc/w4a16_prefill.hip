@@ -26,8 +26,10 @@
 // split exactly into three bf16 terms by the pre-pass kernel below, times the
 // group scale split exactly into two bf16 terms; six exact products per group
 // accumulate c * scale into the result (about 5 % extra matrix work).
-// Launches of several rounds of 128-row blocks, with adapters or without, take c as f32 and add it
-// where a group begins, in the rescale's multiplication (INC below): no extra matrix work.
+// Launches of several rounds of 128-row blocks, with adapters or without, and of tiles that leave no
+// compute units for the row sums, take c as f32 and add it where a group begins, in the rescale's
+// multiplication (INC below): no extra matrix work.  Where a compute unit gets one block at most, the
+// block has a second set of wavefronts for the other half of its K (WK below).
 #include <type_traits>
 
 #include "device_common.h"
@@ -323,7 +325,7 @@ __device__ __forceinline__ void prefill_fold_done(const PrefillFold &pf, int con
 // by scale(g) / scale(g+1) becomes a multiply-add, and there is no extension contraction (6 % of the products at any
 // K, and 2 us a tile).  What it costs is LDS reads: a lane's accumulators lie in 16 rows of every row tile, whose
 // values of c it reads (broadcast) in 16-byte pieces, 16 of them a group beside 32 fragments.  For launches of several
-// rounds, whose row sums come from in front anyway; where the launch's own blocks form them (RS, and FOLD's producers
+// rounds, or of a block for nearly every unit, whose row sums come from in front anyway; where the launch's own blocks form them (RS, and FOLD's producers
 // without INC) they are not there when a block begins.  FOLD and INC together: the producers run the projection onto the
 // adapters alone.
 //
@@ -1248,7 +1250,10 @@ static PrefillPlan plan_for_shape(int m, int n, int k, int cus, int bn, int bm, 
 // the cheaper plan by this cost was the faster one or within 0.8 % (the former) and 0.6 % (the latter) of it
 // on average, 18 % and 5 % at worst.  That was before the main loop was ordered by hand; on the kernel as it is, 88
 // cases -- eight shapes at 200 ... 2048 rows, both heights forced -- are 2.4 % off on average and 32 % at worst
-// (4096 -> 12288 at 420 rows: 62 us in 128-row blocks and two slices, 47 in 64-row ones).
+// (4096 -> 12288 at 420 rows: 62 us in 128-row blocks and two slices, 47 in 64-row ones).  With two sets of wavefronts to
+// lone blocks and the rules behind the choice (plan_prefill), 233 cases -- 22 shapes at 192 ... 2048 rows, both heights in
+// every number of slices -- are about 1 % off on average, 23 % at worst (6144 -> 6144 at 1300 rows, 64-row blocks in whole
+// rounds and a rest: 124 us, whole 101).
 static float plan_cost(int m, int n, int k, int cus, const PrefillPlan &p) {
     const int G = k / kGroupK, m_blocks = (m + p.bm - 1) / p.bm, n_blocks = n / p.bn;
     const float rows = p.bm == 128 ? 1.5f : 1.0f;
@@ -1528,13 +1533,18 @@ static int rowsum_producers_wanted(int M) { return ((M + 63) / 64 + 7) / 8 * 8; 
 // Blocks whose wavefronts share K (the kernel's WK): where the plan gives a compute unit one block at most, of enough groups
 // that half of them pay for the halves' meeting.  The row sums: from the blocks, from the units without a block where they
 // can be done in time, else, for whole tiles, from a launch in front, which 128-row blocks then add at the changes of group.  By the plan alone, with adapters or without, and alike for both block widths (counted in blocks
-// of 256 columns), so that calls which must agree in every bit add in one order.  (84 shapes and row counts: 12 % faster
+// of 256 columns), so that calls which must agree in every bit add in one order.  Calls with adapters pay for it: the
+// projection finds no units beside such blocks and runs in front, which costs 4 to 8 us.  In 128-row blocks of fewer than 24
+// groups that is more than the halves give (plain 0 to 11 % ahead, 3.5 on average, with adapters 5 to 11 % behind: 2560 -> 8192
+// at 777 rows 44 -> 50 us), so they keep one set; in 64-row blocks, and from 24 groups on, plain calls gain 10 to 30 %
+// and calls with adapters are between 18 % behind (2688 -> 2048 at 582 rows 20.4 -> 24.9) and 8 % ahead (4096 -> 4096 at 700
+// rows 48.2 -> 44.6).    (84 shapes and row counts: 12 % faster
 // on average, 1 % slower at worst.  Shorter shares are level or slower: 11 groups in 128-row blocks, 4096 -> 2560 at 777 rows in
 // three slices, 33.7 us either way; 64-row blocks on every unit, 2816 -> 1024 at 2000 rows, 256 blocks of 11 groups, and
 // 2048 -> 2048 at 900, 2 to 7 % slower: the units' store and start then have nothing left to hide behind.  With the sums
 // from a launch in front, tiles for nine tenths of the units or all: 4096 -> 4096 at 1900 / 2048 rows 74 -> 67 us, 4096 -> 2560
 // at 3072 82 -> 75, 8192 -> 8192 at 1024 133 -> 123, 14336 -> 4096 at 2048 228 -> 213, 28672 -> 8192 at 1000 470 -> 415,
-// 2560 -> 8192 at 1024 47.0 -> 46.1, the least.  Launches of several rounds are slower so: 2560 -> 18432 at 777 / 4096 rows 72 ->
+// 3072 -> 8192 at 1000 54.3 -> 53.0, the least.  Launches of several rounds are slower so: 2560 -> 18432 at 777 / 4096 rows 72 ->
 // 80 / 307 -> 343, one block of eight wavefronts a unit in place of two of four.)
 bool prefill_halves_k(int M, int N, int K, const PrefillPlan &p, int cus) {
     if ((p.bm != 64 && p.bm != 128) || p.nb_full < 0 || p.nb_full > N / p.bn) return false;
@@ -1543,7 +1553,7 @@ bool prefill_halves_k(int M, int N, int K, const PrefillPlan &p, int cus) {
     wide.bn = 256;
     wide.nb_full = p.nb_full * p.bn / 256;
     const int grid = prefill_grid(M, N, wide, cus), row_tiles = (M + 15) / 16;
-    if (grid > cus || (G + ks - 1) / ks < (p.bm == 64 && grid <= cus - 8 ? 6 : 16)) return false;
+    if (grid > cus || (G + ks - 1) / ks < (p.bm == 128 ? 24 : grid <= cus - 8 ? 6 : 16)) return false;
     if (blocks_sum_their_rows(M, N, K, p)) return true;
     // the producers' share must be done before a block's main loop is: 0.7 ns a row tile and value of K against
     // 1.4 us a group
@@ -1633,7 +1643,7 @@ hipError_t launch_prefill(const PrefillArgs &a, hipStream_t stream) {
         // (Blocks whose wavefronts share K have a unit each: the projection is inside if all of its slices' blocks find free
         // units, so that T's sums are added in one order wherever it runs.)
         if (halves) {
-            room = prefill_grid(a.M, a.N, shape, a.cus) + (row_tiles * kz + 7) / 8 * 8 <= a.cus;
+            room = !inc && prefill_grid(a.M, a.N, shape, a.cus) + (row_tiles * kz + 7) / 8 * 8 <= a.cus;
         } else if (rb == 16 && a.bm == 128) {
             const int slots = a.cus * 2, product = prefill_grid(a.M, a.N, shape, a.cus);
             if (product <= slots && product + (row_tiles * kz + 7) / 8 * 8 > slots) {
@@ -1703,8 +1713,7 @@ hipError_t launch_prefill(const PrefillArgs &a, hipStream_t stream) {
     if (fold) {
         pf.consumers = grid;
         if (inc)
-            return halves ? launch_sums_in_loop<true, 2>(a, grid, m_blocks, RP, KS, GSb, max_groups, pf, stream)
-                          : launch_sums_in_loop<true, 1>(a, grid, m_blocks, RP, KS, GSb, max_groups, pf, stream);
+            return launch_sums_in_loop<true, 1>(a, grid, m_blocks, RP, KS, GSb, max_groups, pf, stream);
         if (halves)
             return a.bm == 128 ? launch_fold<4, 2>(a, grid, m_blocks, RP, KS, GSb, max_groups, rs, pf, stream)
                                : launch_fold<2, 2>(a, grid, m_blocks, RP, KS, GSb, max_groups, rs, pf, stream);

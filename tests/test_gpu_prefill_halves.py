@@ -23,15 +23,15 @@ SHAPES = [
     (1300, 1664, 1536, -1),     # the same, 13 groups
     (777, 2688, 2560, 128),
     (777, 9216, 2560, 128),     # 128-row blocks, row sums from the units without a block
-    (330, 11008, 4096, -1),     # the same, slices of 18 groups, the last of 14
+    (640, 11008, 4096, -1),     # the same, slices of 29 groups, the last of 28
     (1300, 4096, 4096, 128),    # 128-row blocks, whole tiles for two thirds of the units
-    (3001, 2176, 2560, 128),    # row sums from a launch in front, added at the changes of group: 17 groups
+    (3001, 3200, 2560, 128),    # row sums from a launch in front, added at the changes of group: 25 groups
     (1900, 4096, 4096, -1),     # the same, 32 groups
-    (1024, 2048, 8192, 128),    # the same, a tile for every unit, 16 groups
+    (1024, 3072, 8192, 128),    # the same, a tile for every unit, 24 groups
     # tiles dealt to the dies one after the other (13, 14 and 25 row blocks)
     (777, 3584, 4608, 128),     # 64-row blocks, row sums from the blocks
     (850, 3584, 4608, -1),      # ... from a launch in front
-    (3137, 2176, 2560, 128),    # 128-row blocks
+    (3137, 3200, 2560, 128),    # 128-row blocks
 ]
 
 
