@@ -907,7 +907,9 @@ __global__ __launch_bounds__(64 * WM * NWN * WK, (WM == 2 && NWN == 4) ? 1 : 2) 
         }
     }
     wait_vector_loads<0>();  // stages asked for past the end still write to LDS, which the store reuses behind its barrier
-    if constexpr (FOLD) {
+    // (Every wavefront has looked at the words: the barriers of the last group's stages are behind that.  Halves of K have
+    // none in common there: their block is counted behind the barrier in front of their meeting.)
+    if constexpr (FOLD && WK == 1) {
         if (wave_all == 0) prefill_fold_done(pf, consumer, lane);
     }
 
@@ -950,7 +952,10 @@ __global__ __launch_bounds__(64 * WM * NWN * WK, (WM == 2 && NWN == 4) ? 1 : 2) 
     constexpr int MIS = MI / WK;  // row tiles a wavefront goes on with
     const int row_first = wm * MI * 32 + half * (MIS * 32);
     if constexpr (WK == 2) {
-        __syncthreads();  // every wavefront is done with the rings
+        __syncthreads();  // every wavefront is done with the rings, and has looked at a folded launch's words
+        if constexpr (FOLD) {
+            if (wave_all == 0) prefill_fold_done(pf, consumer, lane);
+        }
         f32x4 *box = reinterpret_cast<f32x4 *>(lds) + lane;  // [half][wavefront][row tile, sub-tile, four registers][lane]
         auto four = [](const f32x16 &a, int i) { return f32x4{a[4 * i], a[4 * i + 1], a[4 * i + 2], a[4 * i + 3]}; };
         auto hand_over = [&](auto firstc) {

@@ -102,3 +102,32 @@ def test_adapters_and_the_swiglu_writer(m, k, n, g):
         want_h = torch.nn.functional.silu(gate) * up
         err = (h.double() - want_h).norm(dim=1) / want_h.norm(dim=1)
         assert float(err.max()) <= 2.0 ** -7, float(err.max())
+
+
+@pytest.mark.parametrize("m,k,n,g", [(1005, 1024, 14336, 128), (883, 896, 18176, -1), (1371, 1024, 10496, 128)])
+def test_words_of_a_folded_launch_outlast_both_halves(m, k, n, g):
+    """Halves of at most four groups with row sums from the launch's first blocks: no barrier of the block lies between the
+    last half's look at the words and the end of the main loop, so the block counts itself as done (and the last one zeroes
+    the words) only where the halves meet.  Such short halves come from a caller's count of compute units."""
+    sms = 1024
+    L, plan = _lib.load(), (ctypes.c_int * 8)()
+    assert L.kiln_w4a16_debug_gemm_plan(m, n, k, sms, plan) == 0 and (plan[0], plan[2], plan[5], plan[6], plan[7]) == (1, 64, 1, 0, 1)
+    assert L.kiln_w4a16_debug_prefill_rowsum_producers(m, n, k, sms) > 0 and k // 128 <= 8
+    gen = torch.Generator(device="cuda").manual_seed(m)
+    words = torch.randint(-2**31, 2**31, (k // 16, 2 * n), dtype=torch.int64, device="cuda", generator=gen).to(torch.int32)
+    scales = (torch.rand(1 if g == -1 else k // g, n, device="cuda", generator=gen) * 0.018 + 0.002).half()
+    x = torch.randn(m, k, device="cuda", generator=gen).to(torch.bfloat16)
+    ws = torch.zeros(L.kiln_w4a16_workspace_bytes_tuned(m, n, k, -1, -1, sms), dtype=torch.uint8, device="cuda")
+    zeroed = L.kiln_w4a16_workspace_zeroed_bytes()
+    want = x.double() @ marlin_gemm.dequant_f32(words, scales, g).double()
+    first = None
+    for _ in range(20):
+        y = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+        assert L.kiln_marlin_w4a16_gemm(x.data_ptr(), words.data_ptr(), y.data_ptr(), scales.data_ptr(), m, n, k, ws.data_ptr(), g, 0,
+                                        torch.cuda.current_stream().cuda_stream, -1, -1, sms, 16) == _lib.OK
+        torch.cuda.synchronize()
+        assert int(ws[:zeroed].max()) == 0      # words and counts as they were, and nobody gave up waiting
+        err = (y.double() - want).norm(dim=1) / want.norm(dim=1)
+        assert float(err.max()) <= 2.0 ** -8, float(err.max())     # the bound of the calls above
+        first = y if first is None else first
+        assert torch.equal(y.view(torch.int16), first.view(torch.int16))
