@@ -362,10 +362,14 @@ int kiln_w4a16_layout_version(void);
  * kiln_w4a16_debug_prefill_rowsum_producers: where the matrix-core kernel's row sums come from:
  *   > 0 that many blocks of the product's own launch, 0 a launch in front, -2 every block sums its own
  *   rows, -3 another kernel takes the call, -1 bad sizes.
+ * kiln_w4a16_debug_prefill_projection_blocks: where the matrix-core kernel's calls with adapters compute x * A^T:
+ *   > 0 in that many blocks of the product's own launch, 0 in a launch in front, -3 another kernel takes the
+ *   call, -1 bad sizes.
  */
 int kiln_w4a16_debug_gemm_plan(int prob_m, int prob_n, int prob_k, int cus, int *out);
 int kiln_w4a16_debug_decode_plan(int prob_m, int prob_n, int prob_k, int cus, int *out);
 int kiln_w4a16_debug_prefill_rowsum_producers(int prob_m, int prob_n, int prob_k, int cus);
+int kiln_w4a16_debug_prefill_projection_blocks(int prob_m, int prob_n, int prob_k, int cus);
 
 #ifdef __cplusplus
 }

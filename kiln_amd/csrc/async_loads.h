@@ -47,6 +47,16 @@ __device__ __forceinline__ void load_to_lds_b32(const void *base, uint32_t lane_
                  : "memory", "m0");
 }
 
+// A pointer that is the same in all lanes, in scalar registers whatever the compiler can prove.  A vector memory
+// instruction may read a scalar register only five wait states after a vector instruction (v_readfirstlane) wrote
+// it; the compiler keeps that distance for its own loads and cannot for those inside inline asm, so it is kept here.
+__device__ __forceinline__ const char *uniform(const char *p) {
+    const uint64_t v = reinterpret_cast<uint64_t>(p);
+    uint32_t lo = __builtin_amdgcn_readfirstlane((int)(uint32_t)v), hi = __builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
+    asm volatile("s_nop 4" : "+s"(lo), "+s"(hi));
+    return reinterpret_cast<const char *>(((uint64_t)hi << 32) | lo);
+}
+
 // A zero the compiler cannot see through, defined where it is called: arithmetic that depends on
 // it stays behind the preceding asm statements instead of being hoisted to the top of a long
 // straight-line kernel (where it would hold registers for its whole length).

@@ -203,6 +203,7 @@ int prefill_grid(int m, int n, const PrefillPlan &p, int cus);
 size_t prefill_partial_bytes(int m, int n, const PrefillPlan &p);
 bool prefill_halves_k(int m, int n, int k, const PrefillPlan &p, int cus);         // do a block's wavefronts share K?
 int prefill_rowsum_producers(int m, int n, int k, const PrefillPlan &p, int cus);  // blocks of a plain launch that form the row sums inside it (0: a launch in front does, -2: every block its own)
+int prefill_projection_blocks(int m, int n, int k, const PrefillPlan &p, int cus);  // of a launch with adapters (0: the projection is in front)
 bool prefill_adds_sums_in_loop(int m, int n, int k, const PrefillPlan &p, int cus);  // row sums as f32 [K/128][M], added at the changes of group
 bool prefill_forms_next_sums(const PrefillPlan &p);                             // can its swiglu launch write next_aext?
 bool prefill_reads_row_sums(int m, int n, int k, const PrefillPlan &p);         // ... a plain launch take it as aext?

@@ -1,6 +1,7 @@
 // The LoRA projection T = scale * x * A_cat^T as the work of one 256-thread block, shared by the kernel
 // that runs it as a launch of its own and by the kernels that run it in their own launch's first blocks.
 #pragma once
+#include "async_loads.h"
 #include "device_common.h"
 
 namespace kiln {
@@ -70,8 +71,95 @@ __device__ __forceinline__ void store_b128_through(void *ptr, u32x4 v) {
     asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" : : "v"(ptr), "v"(v) : "memory");
 }
 
+// What a block does with its share of T: the tiles `wave + W it` of its RB rows, W wavefronts, IT of them to each at most.
+// Columns from r_live on are stored as zero whatever the sums hold.  A word of `done` per 16 rows.
+template <int RB, int W, int IT, int ZMAX>  // ZMAX: K slices that may meet in one T
+__device__ __forceinline__ void project_store(f32x4 (&acc)[IT], const float *sc_lds, uint16_t *__restrict__ T, int M, int RP, int r_live,
+                                              int m0, int items, int JT, float *partial, int *counters, int row_tile, int slice,
+                                              int KZ, unsigned *done, int done_copies, int done_stride) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    uint16_t *Tz = T + (size_t)slice * M * RP;
+    if (partial && KZ > 1) {
+        // One T for all of K: the slices of a row tile meet in `partial` as f32 tiles (device-scope
+        // accesses); the last block to arrive adds them in slice order, so the result does not
+        // depend on arrival order, and leaves the counter at zero.
+        __shared__ int s_last;
+        float *tile0 = partial + (size_t)row_tile * KZ * (IT * W) * 256 + lane;  // [slice][item][4][64]
+#pragma unroll
+        for (int it = 0; it < IT; ++it) {
+            const int item = wave + W * it;
+            if (item < items)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    __hip_atomic_store(tile0 + ((size_t)(slice * (IT * W) + item) * 4 + i) * 64, acc[it][i],
+                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        // each wavefront waits until its own stores have been acknowledged (a barrier alone
+        // orders nothing outside the workgroup); after the barrier the arrival is counted
+        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+        __syncthreads();
+        if (tid == 0)
+            s_last = __hip_atomic_fetch_add(counters + row_tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == KZ - 1;
+        __syncthreads();
+        if (!s_last) return;
+        // every read is requested before the first is used: device-scope reads are slow, and this
+        // round trip is hidden by nothing else
+        f32x4 part[IT][ZMAX];
+#pragma unroll
+        for (int it = 0; it < IT; ++it)
+#pragma unroll
+            for (int z = 0; z < ZMAX; ++z)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    part[it][z][i] = (wave + W * it < items && z < KZ)
+                                         ? __hip_atomic_load(tile0 + ((size_t)(z * (IT * W) + wave + W * it) * 4 + i) * 64,
+                                                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                                         : 0.f;
+#pragma unroll
+        for (int it = 0; it < IT; ++it) {
+            acc[it] = part[it][0];
+#pragma unroll
+            for (int z = 1; z < ZMAX; ++z) acc[it] += part[it][z];
+        }
+        if (tid == 0) __hip_atomic_store(counters + row_tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        Tz = T;
+    }
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+        const int item = wave + W * it;
+        if (item >= items) continue;
+        const int rt = item / JT, jt = item - rt * JT;
+        const int j = jt * 16 + (lane & 15);
+        const float sc = sc_lds[j];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int r = m0 + rt * 16 + 4 * (lane >> 4) + i;
+            const uint32_t mine = j < r_live ? f32_to_bf16_bits(acc[it][i] * sc) : 0u;
+            if (done) {  // two neighbouring columns per 32-bit device-scope store (even lanes)
+                const uint32_t next = (uint32_t)__shfl_xor((int)mine, 1, 64);
+                if ((lane & 1) == 0 && r < M)
+                    __hip_atomic_store(reinterpret_cast<uint32_t *>(Tz + (size_t)r * RP + j), mine | (next << 16),
+                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            } else if (r < M) {
+                Tz[(size_t)r * RP + j] = (uint16_t)mine;
+            }
+        }
+    }
+    if (done) {
+        // whoever gets here wrote the tile's rows of T, after every slice's stores (its own included)
+        // had been acknowledged: the extension operand of all slices is in memory too
+        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+        __syncthreads();
+        // (done_copies copies of the word, done_stride words apart, for readers too many for one address)
+        constexpr int WORDS = RB / 16;
+        if (tid < done_copies * WORDS && m0 + tid % WORDS * 16 < M)
+            __hip_atomic_store(done + (size_t)(tid / WORDS) * done_stride + row_tile * WORDS + tid % WORDS, 1u, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+    }
+}
+
 // The work of one block (256 threads): row tile `row_tile` (RB rows), K slice `slice` of `KZ`.
-// `done` (optional): a word per row tile, raised when the tile's rows of T (and, with `aext`, of the
+// `done` (optional): a word per 16 rows, raised when these rows of T (and, with `aext`, of the
 // extension operand) are in memory -- for a caller that computes the projection inside another
 // kernel's launch instead of in front of it.  Both are then written through to memory: an ordinary
 // store is complete when this die's cache has it, which a reader on another die does not see
@@ -197,82 +285,135 @@ __device__ __forceinline__ void lora_project_block(unsigned char *lds, const uin
     }
     __syncthreads();  // sc_lds (a slice may be empty: then no barrier above)
 
-    uint16_t *Tz = T + (size_t)slice * M * RP;
-    if (partial && KZ > 1) {
-        // One T for all of K: the slices of a row tile meet in `partial` as f32 tiles (device-scope
-        // accesses); the last block to arrive adds them in slice order, so the result does not
-        // depend on arrival order, and leaves the counter at zero.
-        __shared__ int s_last;
-        float *tile0 = partial + (size_t)row_tile * KZ * (IT * 4) * 256 + lane;  // [slice][item][4][64]
+    project_store<RB, 4, IT, ZMAX>(acc, sc_lds, T, M, RP, RP, m0, items, JT, partial, counters, row_tile, slice, KZ, done, done_copies,
+                                   done_stride);
+}
+
+__device__ __forceinline__ float sum_of_16_lanes(float v) {  // the additions of four __shfl_xor: 8, 4, 2, 1 lanes apart
+    auto plus = [&](auto dpp) { v += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), decltype(dpp)::value, 0xF, 0xF, true)); };
+    plus(std::integral_constant<int, 0x128>{});  // row_ror: after the first, what lies n lanes on is what lies across n lanes
+    plus(std::integral_constant<int, 0x124>{});
+    plus(std::integral_constant<int, 0x122>{});
+    plus(std::integral_constant<int, 0x121>{});
+    return v;
+}
+// The same work for blocks that run beside a product of one block per compute unit, in the few units that are left: blocks of
+// eight wavefronts, 64 rows and long shares of K.  One group of K (128 values) of the rows of x and of a_cat is a stage; the
+// stages form a ring in LDS as long as fits, filled by direct loads.  Alone a stage takes 0.36 us (24 KB; eight blocks of 512 x
+// 4224, rank 20: 18.6 us; with row sums 0.6), beside a product 0.5 to 1 us.  (lora_project_block, whose registers hold two pieces
+// of two groups, takes 1.4 us and more a piece there: its loads, its way through LDS and its products one after the other.  Words
+// of all the rows asked for ahead, to have them in this die's L2: slower, 46.8 -> 62 us at 761 x 7808 -> 2560.)
+// Unit u of a row sits at u ^ (row % 16): the 16 lanes that read one unit of 16 rows hit 16 positions.  Every wavefront asks for
+// the same number of loads a stage, rows of a_cat past the last included, so that it can count them; the row sums therefore stay
+// in LDS until the last stage is done (as stores in the loop they were waited for: 96 -> 88 us at 444 x 7040 -> 7936).  The
+// products and their order are lora_project_block's: T is the same in every bit.
+constexpr int kStreamRows = 64;
+__host__ __device__ constexpr int stream_a_rows(int RP) { return RP <= 32 ? 32 : kProjectMaxRank; }
+__host__ __device__ constexpr int stream_stages(int RP) { return RP <= 32 ? 6 : 4; }
+__host__ __device__ constexpr int stream_ring_bytes(int RP) { return stream_stages(RP) * (kStreamRows + stream_a_rows(RP)) * kGroupK * 2; }
+constexpr int kStreamMaxSums = 60;                             // groups of K to a share whose row sums fit behind the ring
+constexpr int kStreamSumBytes = kStreamRows * (int)sizeof(float);  // ... a group's
+__host__ __device__ constexpr int stream_lds_bytes(int RP, int sums) {
+    return stream_ring_bytes(RP) + kProjectMaxRank * (int)sizeof(float) + sums * kStreamSumBytes;
+}
+static_assert(stream_lds_bytes(32, kStreamMaxSums) < 160 * 1024 - 256 && stream_lds_bytes(64, 0) <= stream_lds_bytes(32, 0), "LDS");
+__device__ __forceinline__ void lora_project_stream(unsigned char *lds, const uint16_t *__restrict__ X,
+                                                    const uint16_t *__restrict__ a_cat, uint16_t *__restrict__ T, int M, int K,
+                                                    int r_total, int RP, int steps_per_slice, const LoraScales &ls, float *partial,
+                                                    int *counters, u32x4 *aext, int row_tile, int slice, int KZ, unsigned *done) {
+    constexpr int W = 8, IT = kStreamRows / 16 * (kProjectMaxRank / 16) / W, kRowBytes = kGroupK * 2;
+    const int stages = stream_stages(RP), stage_bytes = (kStreamRows + stream_a_rows(RP)) * kRowBytes;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int m0 = row_tile * kStreamRows, rows = min(kStreamRows, M - m0), JT = RP >> 4;
+    const int per_slice = steps_per_slice / (kGroupK / 32), g0 = slice * per_slice, g1 = min(K / kGroupK, g0 + per_slice);
+    const int items = (rows + 15) / 16 * JT;
+    float *sc_lds = reinterpret_cast<float *>(lds + stream_ring_bytes(RP)), *sums = sc_lds + kProjectMaxRank;
+
+    // a load fills four rows: two loads for x, one for a_cat's first 32 rows, one for what lies behind them
+    const bool more = RP > 32;
+    auto offset = [&](int first, int last) {  // of this lane's 16 bytes, `first` the first of the four rows
+        const int row = first + (lane >> 4);
+        return (uint32_t)min(row, last) * (uint32_t)K * 2u + ((lane & 15) ^ (row & 15)) * 16;
+    };
+    const uint32_t x_off0 = offset(wave * 4, rows - 1), x_off1 = offset(32 + wave * 4, rows - 1);
+    const uint32_t a_off0 = offset(wave * 4, r_total - 1), a_off1 = offset(32 + wave * 4, r_total - 1);
+    const char *const x_rows = uniform(reinterpret_cast<const char *>(X) + (size_t)m0 * K * 2);
+    const unsigned ring = (unsigned)(size_t)(lds_ptr_t)lds;
+    int into = 0;                // the stage of the ring the next request fills
+    auto request = [&](int g) {  // groups past the last: the last one, for a place nobody reads any more
+        const size_t at = (size_t)min(g, g1 - 1) * kRowBytes;
+        const char *const xb = uniform(x_rows + at), *const ab = uniform(reinterpret_cast<const char *>(a_cat) + at);
+        const unsigned to = __builtin_amdgcn_readfirstlane(ring + (unsigned)into + wave * 1024);
+        load_to_lds_b128(xb, x_off0, to);
+        load_to_lds_b128(ab, a_off0, to + kStreamRows * kRowBytes);
+        load_to_lds_b128(xb, x_off1, to + W * 1024);
+        if (more) load_to_lds_b128(ab, a_off1, to + kStreamRows * kRowBytes + W * 1024);
+        into += stage_bytes;
+        if (into == stages * stage_bytes) into = 0;
+    };
+    f32x4 acc[IT];
 #pragma unroll
-        for (int it = 0; it < IT; ++it) {
-            const int item = wave + 4 * it;
-            if (item < items)
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    __hip_atomic_store(tile0 + ((size_t)(slice * (IT * 4) + item) * 4 + i) * 64, acc[it][i],
-                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        // each wavefront waits until its own stores have been acknowledged (a barrier alone
-        // orders nothing outside the workgroup); after the barrier the arrival is counted
-        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-        __syncthreads();
-        if (tid == 0)
-            s_last = __hip_atomic_fetch_add(counters + row_tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == KZ - 1;
-        __syncthreads();
-        if (!s_last) return;
-        // every read is requested before the first is used: device-scope reads are slow, and this
-        // round trip is hidden by nothing else
-        f32x4 part[IT][ZMAX];
-#pragma unroll
-        for (int it = 0; it < IT; ++it)
-#pragma unroll
-            for (int z = 0; z < ZMAX; ++z)
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    part[it][z][i] = (wave + 4 * it < items && z < KZ)
-                                         ? __hip_atomic_load(tile0 + ((size_t)(z * (IT * 4) + wave + 4 * it) * 4 + i) * 64,
-                                                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                                         : 0.f;
-#pragma unroll
-        for (int it = 0; it < IT; ++it) {
-            acc[it] = part[it][0];
-#pragma unroll
-            for (int z = 1; z < ZMAX; ++z) acc[it] += part[it][z];
-        }
-        if (tid == 0) __hip_atomic_store(counters + row_tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        Tz = T;
+    for (int it = 0; it < IT; ++it) acc[it] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (g0 < g1) {
+        for (int g = g0; g < g0 + stages - 1; ++g) request(g);
     }
+    if (tid < kProjectMaxRank) {
+        float sc = 0.f;
+        if (tid < r_total) {
+            sc = ls.scales[ls.count - 1];
+            for (int i = ls.count - 1; i >= 0; --i)
+                if (tid < ls.ends[i]) sc = ls.scales[i];
+        }
+        sc_lds[tid] = sc;
+    }
+    const int r16 = lane & 15, q = lane >> 4;
+    int from = 0;
+    for (int g = g0; g < g1; ++g) {
+        // this wavefront's part of the stage has landed: behind it there are the other stages but one, of four loads or three
+        if (more) wait_vector_loads<(stream_stages(64) - 2) * 4>();
+        else wait_vector_loads<(stream_stages(32) - 2) * 3>();
+        wait_lds_reads();
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" : : : "memory");
+        request(g + stages - 1);  // where the stage before was
+        const unsigned char *stage = lds + from;
+        from += stage_bytes;
+        if (from == stages * stage_bytes) from = 0;
 #pragma unroll
-    for (int it = 0; it < IT; ++it) {
-        const int item = wave + 4 * it;
-        if (item >= items) continue;
-        const int rt = item / JT, jt = item - rt * JT;
-        const int j = jt * 16 + (lane & 15);
-        const float sc = sc_lds[j];
+        for (int it = 0; it < IT; ++it) {
+            const int item = wave + W * it;
+            if (item < items) {
+                const int rt = item / JT, jt = item - rt * JT;
+                const unsigned char *xp = stage + (rt * 16 + r16) * kRowBytes, *ap = stage + (kStreamRows + jt * 16 + r16) * kRowBytes;
+                bf16x8 xf[kGroupK / 32], af[kGroupK / 32];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int r = m0 + rt * 16 + 4 * (lane >> 4) + i;
-            const uint32_t mine = f32_to_bf16_bits(acc[it][i] * sc);
-            if (done) {  // two neighbouring columns per 32-bit device-scope store (even lanes)
-                const uint32_t next = (uint32_t)__shfl_xor((int)mine, 1, 64);
-                if ((lane & 1) == 0 && r < M)
-                    __hip_atomic_store(reinterpret_cast<uint32_t *>(Tz + (size_t)r * RP + j), mine | (next << 16),
-                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            } else if (r < M) {
-                Tz[(size_t)r * RP + j] = (uint16_t)mine;
+                for (int st = 0; st < kGroupK / 32; ++st) {
+                    const int unit = ((4 * st + q) ^ r16) * 16;
+                    xf[st] = *reinterpret_cast<const bf16x8 *>(xp + unit);
+                    af[st] = *reinterpret_cast<const bf16x8 *>(ap + unit);
+                }
+#pragma unroll
+                for (int st = 0; st < kGroupK / 32; ++st) acc[it] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf[st], af[st], acc[it], 0, 0, 0);
+            }
+        }
+        if (aext) {
+            // the row sums, in the order of lora_project_block's
+            const int sub = tid & 15;
+#pragma unroll
+            for (int p = 0; p < 2; ++p) {
+                const int row = p * 32 + (tid >> 4);
+                const float sum = sum_of_16_lanes(sum_bf16x8(*reinterpret_cast<const u32x4 *>(stage + row * kRowBytes + ((sub ^ (row & 15)) * 16))));
+                if (sub == 0) sums[(g - g0) * kStreamRows + row] = sum;
             }
         }
     }
-    if (done) {
-        // whoever gets here wrote the tile's rows of T, after every slice's stores (its own included)
-        // had been acknowledged: the extension operand of all slices is in memory too
-        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-        __syncthreads();
-        // (done_copies copies of the word, done_stride words apart, for readers too many for one address)
-        if (tid < done_copies)
-            __hip_atomic_store(done + (size_t)tid * done_stride + row_tile, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+    wait_vector_loads<0>();
+    __syncthreads();  // sc_lds (a slice may be empty: then no barrier above), the row sums
+    if (aext)
+        for (int i = tid; i < (g1 - g0) * kStreamRows; i += W * 64)
+            if (i % kStreamRows < rows)
+                store_b128_through(aext + (size_t)(g0 + i / kStreamRows) * M + m0 + i % kStreamRows, extension_operand(sums[i]));
+    project_store<kStreamRows, W, IT, 8>(acc, sc_lds, T, M, RP, r_total, m0, items, JT, partial, counters, row_tile, slice, KZ, done, 1, 0);
 }
 
 }  // namespace kiln

@@ -1292,6 +1292,16 @@ int kiln_w4a16_debug_prefill_rowsum_producers(int m, int n, int k, int cus) {
     return inside > 0 && g_tune.rowsum_fold == 0 ? 0 : inside;
 }
 
+// Where a GEMM of these sizes with adapters runs its projection: > 0 = in that many blocks of the matrix-core kernel's own
+// launch, 0 = in a launch in front of it, -3 = another kernel runs; -1 = bad sizes
+int kiln_w4a16_debug_prefill_projection_blocks(int m, int n, int k, int cus) {
+    if (m < 1 || cus < 1 || !shape_ok(n, k, 128)) return -1;
+    GemmPlan gp;
+    plan_gemm(m, n, k, cus, -1, -1, 1, &gp);
+    if (!gp.prefill) return -3;
+    return g_tune.lora_fold == 0 ? 0 : prefill_projection_blocks(m, n, k, gp.pf, cus);
+}
+
 #ifdef KILN_W4A16_TUNING_HOOKS
 // Only in the tuning build of the library (never in the shipped one): process-wide overrides of
 // the automatic plan for the test suite and profiling scripts (0 / -1 = automatic).  Plain

@@ -30,6 +30,7 @@
 // compute units for the row sums, take c as f32 and add it where a group begins, in the rescale's
 // multiplication (INC below): no extra matrix work.  Where a compute unit gets one block at most, the
 // block has a second set of wavefronts for the other half of its K (WK below).
+#include <climits>
 #include <type_traits>
 
 #include "device_common.h"
@@ -106,16 +107,6 @@ __device__ __forceinline__ void direct_load_b128(const void *gptr, unsigned lds_
                  :
                  : "v"(gptr), "s"(lds_addr)
                  : "memory", "m0");
-}
-
-// A pointer that is the same in all lanes, in scalar registers whatever the compiler can prove.  A vector memory
-// instruction may read a scalar register only five wait states after a vector instruction (v_readfirstlane) wrote
-// it; the compiler keeps that distance for its own loads and cannot for those inside inline asm, so it is kept here.
-__device__ __forceinline__ const char *uniform(const char *p) {
-    const uint64_t v = reinterpret_cast<uint64_t>(p);
-    uint32_t lo = __builtin_amdgcn_readfirstlane((int)(uint32_t)v), hi = __builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
-    asm volatile("s_nop 4" : "+s"(lo), "+s"(hi));
-    return reinterpret_cast<const char *>(((uint64_t)hi << 32) | lo);
 }
 
 // Where some of a block's wavefronts meet without the others: a count in LDS that each raises by one.  LDS serves a
@@ -196,7 +187,7 @@ __device__ __forceinline__ uint32_t neighbours_of_a_row(float first, float secon
 // instead of by the pre-pass kernel: for the small blocks, whose launches are bound by latency,
 // this saves a launch and the global reads of the extension operands.
 // The LoRA projection (and the extension operand) computed inside the launch that uses them: the
-// first `producers` blocks of the grid run lora_project_block (row tiles of 16 rows, K slices one
+// first `producers` blocks of the grid run lora_project_block (row tiles, K slices one
 // after the other) while the others multiply; a block of the product looks at its row tiles' words
 // behind its main loop -- long after they were raised -- and reads both operands with ordinary
 // loads (no cache on its die has seen those lines since the launch began).  The words live in
@@ -214,14 +205,19 @@ struct PrefillFold {
     float *partial;
     int *counters;           // per row tile, zero on entry and exit (not the product's own counters)
     unsigned *words;         // the zeroed region
-    int producers;           // row_tiles * kz rounded up to a multiple of 8 (the product's blocks keep their dies)
-    int row_tiles, kz, steps_per_slice;
+    int producers;           // a multiple of 8 (the product's blocks keep their dies): project_tiles * kz rounded up, or fewer (WK = 2)
+    int row_tiles;           // of 16 rows, a word each
+    int project_tiles, kz, steps_per_slice;  // the projection's row tiles (kFoldProjectRows) and K slices
     int consumers;           // blocks of the product (grid padding included)
     int sum_tiles;           // a_cat == nullptr (no adapters): the producers form the row sums only, this many
                              // 16-row tiles each
     LoraScales ls;
 };
 constexpr int kPrefillFoldTileWord = 32;
+// rows per block of a projection inside the product's launch: lora_project_block, or lora_project_stream in launches of one
+// block to a compute unit
+template <int WK>
+constexpr int kFoldProjectRows = WK == 2 ? kStreamRows : 16;
 constexpr int kPrefillFoldMaxTiles = kLoraFoldReplicaWords - kPrefillFoldTileWord;
 constexpr int kPrefillFoldSpinLimit = 1 << 20;
 // where a wavefront's early look at its words lands: the last KiB of the LDS every instance that takes part has
@@ -360,10 +356,17 @@ __global__ __launch_bounds__(64 * WM * NWN * WK, (WM == 2 && NWN == 4) ? 1 : 2) 
                                           pf.words + kPrefillFoldTileWord);
                 return;
             }
-            if (unit < pf.row_tiles * pf.kz)
-                lora_project_block<16>(lds, A, pf.a_cat, pf.t, M, K, r_total, RP, pf.steps_per_slice, pf.ls, pf.partial,
-                                       pf.counters, pf.aext, unit % pf.row_tiles, unit / pf.row_tiles, pf.kz,
-                                       pf.words + kPrefillFoldTileWord);
+            unsigned *const words = pf.words + kPrefillFoldTileWord;
+            if constexpr (WK == 2) {  // in turns, where there are more shares than blocks
+                for (int share = unit; share < pf.project_tiles * pf.kz; share += pf.producers) {
+                    if (share != unit) __syncthreads();
+                    lora_project_stream(lds, A, pf.a_cat, pf.t, M, K, r_total, RP, pf.steps_per_slice, pf.ls, pf.partial, pf.counters,
+                                        pf.aext, share % pf.project_tiles, share / pf.project_tiles, pf.kz, words);
+                }
+            } else if (unit < pf.project_tiles * pf.kz) {
+                lora_project_block<16>(lds, A, pf.a_cat, pf.t, M, K, r_total, RP, pf.steps_per_slice, pf.ls, pf.partial, pf.counters,
+                                       pf.aext, unit % pf.project_tiles, unit / pf.project_tiles, pf.kz, words);
+            }
             return;
         }
     }
@@ -1396,11 +1399,15 @@ hipError_t launch_shape_as(const PrefillArgs &a, int grid, int m_blocks, int RP,
     // asks for more LDS than two blocks could share, so the dispatcher cannot stack two blocks
     // on one unit while others idle.
     constexpr int kLdsSolo0 = (WM == 2 && NWN == 2) ? 96 * 1024 : kLdsMax;
-    constexpr int kLdsSolo = FOLD && kLdsSolo0 < kProjectLdsBytes16 ? kProjectLdsBytes16 : kLdsSolo0;
+    constexpr int kProjectLds = WK == 2 ? stream_lds_bytes(32, RS ? 0 : kStreamMaxSums) : kProjectLdsBytes16;
+    constexpr int kLdsSolo = FOLD && kLdsSolo0 < kProjectLds ? kProjectLds : kLdsSolo0;
     const hipError_t attr = allow_dynamic_lds<&w4a16_prefill_kernel<NWN, WM, MI, SWIGLU, RS, FOLD, INC, WK>>(kLdsSolo);
     if (attr != hipSuccess) return attr;
     if (WM == 2 && NWN == 2 && grid <= a.cus) lds_bytes = kLdsSolo;
-    if (FOLD && lds_bytes < kProjectLdsBytes16) lds_bytes = kProjectLdsBytes16;  // the projection's blocks stage more
+    // the projection's blocks stage more
+    const int project_lds = WK == 1 ? kProjectLdsBytes16
+                            : pf.a_cat ? stream_lds_bytes(RP, RS ? 0 : pf.steps_per_slice / 4) : 0;
+    if (FOLD && lds_bytes < project_lds) lds_bytes = project_lds;
     w4a16_prefill_kernel<NWN, WM, MI, SWIGLU, RS, FOLD, INC, WK><<<grid + (FOLD ? pf.producers : 0), 64 * NW * WK, lds_bytes, stream>>>(
         (const uint16_t *)a.A, (const u32x4 *)a.B, (const uint16_t *)a.S, (uint16_t *)a.C, (const u32x4 *)a.aext,
         a.M, a.N, a.K, a.Gs, m_blocks, (const uint16_t *)a.lora_t, (const uint16_t *)a.lora_b, a.r_total, RP,
@@ -1454,27 +1461,28 @@ int lora_project_slices(int m, int k) {
     return kz < 1 ? 1 : kz;
 }
 
-// Many rows: rows per block, row tiles, K slices (as many as keep about 256 blocks busy) and steps of
+// Many rows, `rb` a block: row tiles, K slices (as many as keep about 256 blocks busy, at most `most`) and steps of
 // 32 values per slice (whole groups).
-static void project_slicing(int m, int k, bool have_counters, int *rb_out, int *row_tiles_out, int *kz_out, int *per_slice_out) {
-    const int steps = k / 32;
-    const int rb = lora_project_rows_per_block(m, k), row_tiles = (m + rb - 1) / rb;
+struct ProjectSlicing {
+    int row_tiles, kz, per_slice;
+};
+static ProjectSlicing project_slicing(int m, int k, int rb, bool have_counters, int most) {
+    const int steps = k / 32, row_tiles = (m + rb - 1) / rb;
     const int pieces = (k + kProjectPieceK - 1) / kProjectPieceK;
     int kz = (256 + row_tiles - 1) / row_tiles;
     const int zmax = rb == 16 ? 16 : 8;  // what the kernel's meeting reads in one go
     if (kz > zmax) kz = zmax;
     if (kz > pieces) kz = pieces;
     if (row_tiles > kProjectMaxCounters || !have_counters) kz = 1;
+    if (kz > most) kz = most;
     const int per_slice = ((steps + kz - 1) / kz + 3) / 4 * 4;
-    kz = (steps + per_slice - 1) / per_slice;
-    *rb_out = rb;
-    *row_tiles_out = row_tiles;
-    *kz_out = kz;
-    *per_slice_out = per_slice;
+    return {row_tiles, (steps + per_slice - 1) / per_slice, per_slice};
 }
 
-hipError_t launch_lora_project(const PrefillArgs &a, bool few_rows, hipStream_t stream, int *slices, bool with_row_sums,
-                               bool plain_sums) {
+// `kz`, `per_slice` (many rows): the K slices of a projection that could run inside the product's launch, whose sums it
+// then adds in the same order; 0: as many as suit a launch of its own.
+static hipError_t project_in_front(const PrefillArgs &a, bool few_rows, hipStream_t stream, int *slices, bool with_row_sums,
+                                   bool plain_sums, int kz, int per_slice) {
     if (a.r_total < 1 || a.r_total > kProjectMaxRank || a.n_adapters < 1 || a.n_adapters > 8 || !a.lora_a ||
         !a.lora_t || !a.ranks || !a.scales || a.M < 1 || a.K < kGroupK)
         return hipErrorInvalidValue;
@@ -1493,8 +1501,13 @@ hipError_t launch_lora_project(const PrefillArgs &a, bool few_rows, hipStream_t 
     if (with_row_sums && !aext) return hipErrorInvalidValue;
     if (!few_rows) {
         // many rows: T whole.  K slices that meet in f32 behind T, as many as keep about 256 blocks busy.
-        int rb, row_tiles, kz, per_slice;
-        project_slicing(a.M, a.K, a.counters != nullptr, &rb, &row_tiles, &kz, &per_slice);
+        const int rb = lora_project_rows_per_block(a.M, a.K);
+        const ProjectSlicing own = project_slicing(a.M, a.K, rb, a.counters != nullptr, INT_MAX);
+        const int row_tiles = own.row_tiles;
+        if (kz == 0 || row_tiles > kProjectMaxCounters || !a.counters) {
+            kz = own.kz;
+            per_slice = own.per_slice;
+        }
         float *partial = reinterpret_cast<float *>(reinterpret_cast<char *>(a.lora_t) + (size_t)a.M * 64 * sizeof(uint16_t));
         const int lds_bytes = (rb + kProjectMaxRank) * kProjectRowBytes + kProjectMaxRank * (int)sizeof(float);
         const auto kernel = rb == 16 ? (plain_sums ? &w4a16_lora_project_kernel<16, true> : &w4a16_lora_project_kernel<16, false>)
@@ -1509,8 +1522,8 @@ hipError_t launch_lora_project(const PrefillArgs &a, bool few_rows, hipStream_t 
             a.counters, aext);
         return hipGetLastError();
     }
-    int kz = lora_project_slices(a.M, a.K);
-    const int per_slice = ((steps + kz - 1) / kz + 3) / 4 * 4;  // whole 128-value groups
+    kz = lora_project_slices(a.M, a.K);
+    per_slice = ((steps + kz - 1) / kz + 3) / 4 * 4;  // whole 128-value groups
     kz = (steps + per_slice - 1) / per_slice;
     *slices = kz;
     const int lds_bytes = (16 + kProjectMaxRank) * kProjectRowBytes + kProjectMaxRank * (int)sizeof(float);
@@ -1518,6 +1531,11 @@ hipError_t launch_lora_project(const PrefillArgs &a, bool few_rows, hipStream_t 
         (const uint16_t *)a.A, (const uint16_t *)a.lora_a, (uint16_t *)a.lora_t, a.M, a.K, a.r_total, RP, per_slice, ls,
         nullptr, nullptr, nullptr);
     return hipGetLastError();
+}
+
+hipError_t launch_lora_project(const PrefillArgs &a, bool few_rows, hipStream_t stream, int *slices, bool with_row_sums,
+                               bool plain_sums) {
+    return project_in_front(a, few_rows, stream, slices, with_row_sums, plain_sums, 0, 0);
 }
 
 // 64-row blocks form the row sums themselves when they fit next to the A ring and the launch is
@@ -1537,20 +1555,19 @@ static int rowsum_producers_wanted(int M) { return ((M + 63) / 64 + 7) / 8 * 8; 
 
 // Blocks whose wavefronts share K (the kernel's WK): where the plan gives a compute unit one block at most, of enough groups
 // that half of them pay for the halves' meeting.  The row sums: from the blocks, from the units without a block where they
-// can be done in time, else, for whole tiles, from a launch in front, which 128-row blocks then add at the changes of group.  By the plan alone, with adapters or without, and alike for both block widths (counted in blocks
-// of 256 columns), so that calls which must agree in every bit add in one order.  Calls with adapters pay for it: the
-// projection finds no units beside such blocks and runs in front, which costs 4 to 8 us.  In 128-row blocks of fewer than 24
-// groups that is more than the halves give (plain 0 to 11 % ahead, 3.5 on average, with adapters 5 to 11 % behind: 2560 -> 8192
-// at 777 rows 44 -> 50 us), so they keep one set; in 64-row blocks, and from 24 groups on, plain calls gain 10 to 30 %
-// and calls with adapters are between 18 % behind (2688 -> 2048 at 582 rows 20.4 -> 24.9) and 8 % ahead (4096 -> 4096 at 700
-// rows 48.2 -> 44.6).    (84 shapes and row counts: 12 % faster
-// on average, 1 % slower at worst.  Shorter shares are level or slower: 11 groups in 128-row blocks, 4096 -> 2560 at 777 rows in
-// three slices, 33.7 us either way; 64-row blocks on every unit, 2816 -> 1024 at 2000 rows, 256 blocks of 11 groups, and
-// 2048 -> 2048 at 900, 2 to 7 % slower: the units' store and start then have nothing left to hide behind.  With the sums
-// from a launch in front, tiles for nine tenths of the units or all: 4096 -> 4096 at 1900 / 2048 rows 74 -> 67 us, 4096 -> 2560
-// at 3072 82 -> 75, 8192 -> 8192 at 1024 133 -> 123, 14336 -> 4096 at 2048 228 -> 213, 28672 -> 8192 at 1000 470 -> 415,
-// 3072 -> 8192 at 1000 54.3 -> 53.0, the least.  Launches of several rounds are slower so: 2560 -> 18432 at 777 / 4096 rows 72 ->
-// 80 / 307 -> 343, one block of eight wavefronts a unit in place of two of four.)
+// can be done in time, else, for whole tiles, from a launch in front, which 128-row blocks then add at the changes of group.
+// By the plan alone, with adapters or without, and alike for both block widths (counted in blocks of 256 columns), so that calls
+// which must agree in every bit add in one order.  (Plain calls, 70 shapes of 200 ... 1300 rows, 1024 ... 9216 wide: 1.11 times
+// as fast on average, those that take it 1 % slower at worst.  Calls with adapters, whose projection runs beside the blocks or
+// in front, project_place: 1.06 times as fast on average, 0.86 at worst, 5 of 70 below 0.97.  Where it is not taken: shorter
+// shares are level or slower, 11 groups in 128-row blocks, 4096 -> 2560 at 777 rows in three slices, 33.7 us either way; 64-row
+// blocks on every unit, 2816 -> 1024 at 2000 rows, 256 blocks of 11 groups, and 2048 -> 2048 at 900, 2 to 7 % slower: the units'
+// store and start then have nothing left to hide behind.  128-row blocks of fewer than 24 groups gain 3.5 % plain and lost 5 to
+// 11 % with adapters, 2560 -> 8192 at 777 rows 44 -> 50 us.  With the sums from a launch in front, tiles for nine tenths of the
+// units or all: 4096 -> 4096 at 1900 / 2048 rows 74 -> 67 us, 4096 -> 2560 at 3072 82 -> 75, 8192 -> 8192 at 1024 133 -> 123,
+// 14336 -> 4096 at 2048 228 -> 213, 28672 -> 8192 at 1000 470 -> 415, 3072 -> 8192 at 1000 54.3 -> 53.0, the least.  Launches of
+// several rounds are slower so: 2560 -> 18432 at 777 / 4096 rows 72 -> 80 / 307 -> 343, one block of eight wavefronts a unit in place
+// of two of four.)
 bool prefill_halves_k(int M, int N, int K, const PrefillPlan &p, int cus) {
     if ((p.bm != 64 && p.bm != 128) || p.nb_full < 0 || p.nb_full > N / p.bn) return false;
     const int G = K / kGroupK, ks = p.ks < 1 || p.nb_full == N / p.bn ? 1 : p.ks;  // (of whole tiles alone: nothing is sliced)
@@ -1606,6 +1623,62 @@ bool prefill_adds_sums_in_loop(int M, int N, int K, const PrefillPlan &p, int cu
 bool prefill_forms_next_sums(const PrefillPlan &p) { return p.bn == 256 && (p.bm == 64 || p.bm == 128); }
 bool prefill_reads_row_sums(int M, int N, int K, const PrefillPlan &p) { return !blocks_sum_their_rows(M, N, K, p); }
 
+// Where the projection of a call with adapters runs: in so many blocks in front of the product's in its launch, or (0) in a
+// launch in front.
+//
+// A product that fits the chip's block slots in one go must still fit them with the projection's blocks
+// in front: the blocks that find no slot start when the producers leave, on whichever units the
+// dispatcher picks, and two of them on one unit beside idle units take 1.6 times as long as one (4096 ->
+// 4096 at 1700 rows, 224 blocks of 128 x 256 and 328 producers for 512 slots: 121 us against 86 at 1600
+// rows, 300 + 208 blocks; 97 with the projection in front).  So the projection is cut into fewer K slices
+// there -- its blocks stay far shorter than the product's -- and runs in front if its row tiles alone do
+// not fit.  Launches of several rounds keep all slices (gate+up at 2048 rows 189 us inside, 194 in front), and
+// so do 64-row blocks, three to a unit, which were never seen to suffer (gate+up at 512 rows, 768 blocks and
+// 256 producers for 768 slots: 62 us inside, 68 in front).
+//
+// Blocks whose wavefronts share K have a unit each, and the projection the units that are left (lora_project_stream), several
+// shares one after the other where these are few.  In front where it would not be done in time: 0.4 us a group of K (0.8 with
+// row sums) and 1.6 us a share against 1 us (128 rows: 1.2) a group of the product and 5 us around them.  Both places timed for
+// 300 shapes and ranks of 180 ... 2048 rows: inside is 1.22 times as fast on average (2048 -> 6656 at 422 rows 29.9 -> 24.0 us), in
+// front up to 1.8 times where a share is long (9216 -> 1280 at 1446 rows, two shares of 72 groups a block, 102 us inside, 66 in
+// front); the rule is 0.04 % off the better of the two on average.  (us with one set of wavefronts in brackets: 1920 -> 3840
+// at 648 rows 23.6 (26.8), 2944 -> 6400 at 291 29.5 (36.7), 7808 -> 2560 at 761 46.8 (55.3).  What stays in front, product
+// launches of two or three K slices that leave 16 units or none, costs 6 us: 2048 -> 1280 at 1296 rows 27.5 (23.6).  Blocks of the
+// projection placed where a die has most units left, instead of alike on all dies: 5 us slower.)
+struct ProjectPlace {
+    ProjectSlicing ps;
+    int producers;
+};
+static ProjectPlace project_place(int M, int N, int K, const PrefillPlan &p, int cus, bool inc, bool have_counters) {
+    const bool halves = prefill_halves_k(M, N, K, p, cus);
+    const int rb = halves ? kFoldProjectRows<2> : lora_project_rows_per_block(M, K), G = K / kGroupK;
+    ProjectPlace place{project_slicing(M, K, rb, have_counters, INT_MAX), 0};
+    ProjectSlicing &ps = place.ps;
+    if (p.bn != 256 || (p.bm != 64 && p.bm != 128) || (!halves && rb != 16) || (halves && inc)) return place;
+    int producers = (ps.row_tiles * ps.kz + 7) / 8 * 8;
+    if (halves || p.bm == 128) {
+        const int slots = halves ? cus : cus * 2, product = prefill_grid(M, N, p, cus), left = (slots - product) / 8 * 8;
+        if (product <= slots && producers > left) {
+            if (left < (halves ? 1 : ps.row_tiles)) return place;
+            ps = project_slicing(M, K, rb, have_counters, left >= ps.row_tiles ? left / ps.row_tiles : 1);
+            producers = (ps.row_tiles * ps.kz + 7) / 8 * 8;
+            if (producers > left) producers = left;
+        }
+    }
+    if (halves) {
+        const bool sums = prefill_reads_row_sums(M, N, K, p);
+        const int share = ps.per_slice / (kGroupK / 32), turns = (ps.row_tiles * ps.kz + producers - 1) / producers;
+        const int groups = p.nb_full > 0 || p.ks < 1 ? G : (G + p.ks - 1) / p.ks;
+        const int needs = (sums ? 4 : 2) * share * turns + 8 * turns, has = (p.bm == 64 ? 5 : 6) * groups + 24;
+        if ((sums && share > kStreamMaxSums) || needs > has) return place;
+    }
+    place.producers = producers;
+    return place;
+}
+int prefill_projection_blocks(int M, int N, int K, const PrefillPlan &p, int cus) {
+    return project_place(M, N, K, p, cus, prefill_adds_sums_in_loop(M, N, K, p, cus), true).producers;
+}
+
 hipError_t launch_prefill(const PrefillArgs &a, hipStream_t stream) {
     const int G = a.K / kGroupK;
     if (a.bm != 64 && a.bm != 128 && a.bm != 256) return hipErrorInvalidValue;
@@ -1632,37 +1705,10 @@ hipError_t launch_prefill(const PrefillArgs &a, hipStream_t stream) {
     bool fold = false;
     if (a.r_total > 0) {
         RP = (a.r_total + 15) / 16 * 16;
-        int rb = 0, row_tiles = 0, kz = 0, per_slice = 0;
-        project_slicing(a.M, a.K, a.counters != nullptr, &rb, &row_tiles, &kz, &per_slice);
+        const ProjectPlace place = project_place(a.M, a.N, a.K, shape, a.cus, inc, a.counters != nullptr);
+        const int row_tiles = (a.M + 15) / 16;
         const int sliced_tiles = (a.N / a.bn - a.nb_full) * ((a.M + a.bm - 1) / a.bm);
-        // A product that fits the chip's block slots in one go must still fit them with the projection's blocks
-        // in front: the blocks that find no slot start when the producers leave, on whichever units the
-        // dispatcher picks, and two of them on one unit beside idle units take 1.6 times as long as one (4096 ->
-        // 4096 at 1700 rows, 224 blocks of 128 x 256 and 328 producers for 512 slots: 121 us against 86 at 1600
-        // rows, 300 + 208 blocks; 97 with the projection in front).  So the projection is cut into fewer K slices
-        // there -- its blocks stay far shorter than the product's -- and runs in front if its row tiles alone do
-        // not fit.  Launches of several rounds keep all slices (gate+up at 2048 rows 189 us inside, 194 in front), and
-        // so do 64-row blocks, three to a unit, which were never seen to suffer (gate+up at 512 rows, 768 blocks and
-        // 256 producers for 768 slots: 62 us inside, 68 in front).
-        bool room = true;
-        // (Blocks whose wavefronts share K have a unit each: the projection is inside if all of its slices' blocks find free
-        // units, so that T's sums are added in one order wherever it runs.)
-        if (halves) {
-            room = !inc && prefill_grid(a.M, a.N, shape, a.cus) + (row_tiles * kz + 7) / 8 * 8 <= a.cus;
-        } else if (rb == 16 && a.bm == 128) {
-            const int slots = a.cus * 2, product = prefill_grid(a.M, a.N, shape, a.cus);
-            if (product <= slots && product + (row_tiles * kz + 7) / 8 * 8 > slots) {
-                const int cap = (slots - product) / 8 * 8 / row_tiles;
-                room = cap >= 1;
-                if (room) {
-                    const int steps = a.K / 32;
-                    per_slice = ((steps + cap - 1) / cap + 3) / 4 * 4;
-                    kz = (steps + per_slice - 1) / per_slice;
-                }
-            }
-        }
-        fold = room && a.lora_words && a.bn == 256 && (a.bm == 64 || a.bm == 128) && rb == 16 &&
-               a.counters && row_tiles <= kPrefillFoldMaxTiles && row_tiles <= kProjectMaxCounters - kProjectFoldCounters &&
+        fold = place.producers > 0 && a.lora_words && a.counters && row_tiles <= kPrefillFoldMaxTiles && row_tiles <= kProjectMaxCounters - kProjectFoldCounters &&
                sliced_tiles <= kProjectFoldCounters && a.n_adapters >= 1 && a.n_adapters <= 8 && a.lora_a && a.lora_t &&
                a.ranks && a.scales && a.r_total <= kProjectMaxRank;
         if (fold) {
@@ -1675,9 +1721,10 @@ hipError_t launch_prefill(const PrefillArgs &a, hipStream_t stream) {
             pf.counters = a.counters + kProjectFoldCounters;
             pf.words = a.lora_words;
             pf.row_tiles = row_tiles;
-            pf.kz = kz;
-            pf.steps_per_slice = per_slice;
-            pf.producers = (row_tiles * kz + 7) / 8 * 8;
+            pf.project_tiles = place.ps.row_tiles;
+            pf.kz = place.ps.kz;
+            pf.steps_per_slice = place.ps.per_slice;
+            pf.producers = place.producers;
             pf.ls.count = a.n_adapters;
             int end = 0;
             for (int i = 0; i < 8; ++i) {
@@ -1687,7 +1734,7 @@ hipError_t launch_prefill(const PrefillArgs &a, hipStream_t stream) {
             }
         } else {
             int slices = 1;  // many rows: T is whole
-            err = launch_lora_project(a, false, stream, &slices, !rs, inc);
+            err = project_in_front(a, false, stream, &slices, !rs, inc, place.producers > 0 ? place.ps.kz : 0, place.ps.per_slice);
             if (err != hipSuccess) return err;
             if (slices != 1) return hipErrorInvalidValue;
         }

@@ -134,3 +134,16 @@ def test_short_slices_of_more_than_512_rows_are_of_64_row_tiles(m, k, n, rows):
     out = (ctypes.c_int * 8)()
     assert _lib.load().kiln_w4a16_debug_gemm_plan(m, n, k, CUS, out) == 0
     assert (out[0], out[2], out[3], out[5]) == (1, rows, 256, 3) and out[4] == 0
+
+
+@pytest.mark.parametrize("m,k,n,inside", [
+    # calls with adapters whose product has one block to a compute unit: in the units that are left ...
+    (582, 2688, 2048, 16), (514, 1024, 6144, 40), (648, 1920, 3840, 56), (291, 2944, 6400, 40), (761, 7808, 2560, 16),
+    (800, 8192, 8192, 32), (1203, 7296, 2304, 40), (777, 2560, 2560, 96),
+    # ... unless their shares of K are too long for them: 70 groups, 33 with row sums in two turns, 21 tiles for 16 units
+    (989, 8960, 1280, 0), (664, 4224, 5632, 0), (1296, 2048, 1280, 0),
+])
+def test_where_the_projection_runs(m, k, n, inside):
+    out = (ctypes.c_int * 8)()
+    assert _lib.load().kiln_w4a16_debug_gemm_plan(m, n, k, CUS, out) == 0 and (out[0], out[7]) == (1, 1)
+    assert _lib.load().kiln_w4a16_debug_prefill_projection_blocks(m, n, k, CUS) == inside
