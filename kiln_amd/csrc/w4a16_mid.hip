@@ -303,7 +303,6 @@ __device__ __forceinline__ void mid_block(
         float s_cur[TP];
         float s_of[NG][TP];   // the scale of every group (this lane's column of each pair)
         float c_of[NG][RBN];  // -136 * (sum of the group's activations) of row 32 rb + l32
-        const s16x4 ones = {0x3F80, 0x3F80, 0x3F80, 0x3F80};  // bf16 1.0
         unrolled<0, NG>([&](auto gc) {
             constexpr int gi = decltype(gc)::value, set = gi % kSets;
             // this group's rows of A are in LDS; their fragments go to registers: lane (l32, h) holds
@@ -328,21 +327,41 @@ __device__ __forceinline__ void mid_block(
             // takes 12 cycles from the matrix unit for two values, such a product 8 for four: 64 of the former a group
             // were as long as half of its products.  Two layers of 50 rows 89.4 -> 86.4 us; 9216 -> 2560 at 48 rows 10.7 ->
             // 10.3, 2560 -> 8192 at 24 rows 6.5 -> 6.2; the same error.)
-            f32x4 sums[RBN];
+            // With adapters and three pairs the second row block's chain begins when the first's has ended, and the ones are
+            // formed for it: those instances have 256 registers and not one to spare (both at once: 20 spilled, and with
+            // loads in flight to registers the compiler takes as written, a spill could save a stale one; 2560 -> 18432 with
+            // adapters at 64 / 128 rows 18.9 -> 18.1 / 33.3 -> 32.0 us).  A chain's order of additions is the same either way.
+            constexpr bool kOneByOne = LORA && TP == 3 && RBN == 2;
+            constexpr int kChains = kOneByOne ? 1 : RBN;
 #pragma unroll
-            for (int rb = 0; rb < RBN; ++rb) sums[rb] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int rb0 = 0; rb0 < RBN; rb0 += kChains) {
+                uint32_t ones_bits = 0x3F803F80;  // bf16 (1, 1)
+                if constexpr (kOneByOne) {
+                    asm volatile("" : "+v"(ones_bits));
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                const s16x4 ones = __builtin_bit_cast(s16x4, u32x2{ones_bits, ones_bits});
+                f32x4 sums[kChains];
 #pragma unroll
-            for (int s = 0; s < 8; ++s)
+                for (int i = 0; i < kChains; ++i) sums[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int half = 0; half < 2; ++half)
+                for (int s = 0; s < 8; ++s)
 #pragma unroll
-                    for (int rb = 0; rb < RBN; ++rb) {
-                        const u32x2 four = half ? u32x2{af[rb][s].z, af[rb][s].w} : u32x2{af[rb][s].x, af[rb][s].y};
-                        sums[rb] = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(ones, __builtin_bit_cast(s16x4, four), sums[rb], 0, 0, 0);
-                    }
+                    for (int half = 0; half < 2; ++half)
 #pragma unroll
-            for (int rb = 0; rb < RBN; ++rb)
-                c_of[gi][rb] = -kCodeBias * (sums[rb][0] + __shfl_xor(sums[rb][0], 32, 64));
+                        for (int i = 0; i < kChains; ++i) {
+                            const u32x4 &v = af[rb0 + i][s];
+                            const u32x2 four = half ? u32x2{v.z, v.w} : u32x2{v.x, v.y};
+                            sums[i] = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(ones, __builtin_bit_cast(s16x4, four), sums[i], 0, 0, 0);
+                        }
+#pragma unroll
+                for (int i = 0; i < kChains; ++i)
+                    c_of[gi][rb0 + i] = -kCodeBias * (sums[i][0] + __shfl_xor(sums[i][0], 32, 64));
+                if constexpr (kOneByOne) {
+                    asm volatile("" : "+v"(c_of[gi][rb0]));
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
             wait_vector_loads<Sch::value.wait_b[gi]>();
             if constexpr (gi == 0) KILN_MID_TL(2);  // B(0) has arrived
 #pragma unroll
@@ -754,7 +773,9 @@ hipError_t launch_mid_t(const MidArgs &a, int gpw, hipStream_t stream) {
         case 1: return launch_mid_tg<TP, 1>(a, stream);
         case 2: return launch_mid_tg<TP, 2>(a, stream);
         case 3: return launch_mid_tg<TP, 3>(a, stream);
-        case 4: return launch_mid_tg<TP, 4>(a, stream);
+        case 4:
+            if constexpr (TP < 3) return launch_mid_tg<TP, 4>(a, stream);  // (three pairs: mid_plan_ok)
+            else return hipErrorInvalidValue;
         default: return hipErrorInvalidValue;
     }
 }
