@@ -355,12 +355,14 @@ __device__ __forceinline__ void mid_block(
                             sums[i] = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(ones, __builtin_bit_cast(s16x4, four), sums[i], 0, 0, 0);
                         }
 #pragma unroll
-                for (int i = 0; i < kChains; ++i)
-                    c_of[gi][rb0 + i] = -kCodeBias * (sums[i][0] + __shfl_xor(sums[i][0], 32, 64));
-                if constexpr (kOneByOne) {
-                    asm volatile("" : "+v"(c_of[gi][rb0]));
-                    __builtin_amdgcn_sched_barrier(0);
+                for (int i = 0; i < kChains; ++i) {
+                    float sum = sums[i][0] + __shfl_xor(sums[i][0], 32, 64);
+                    // (the sum and not c is held here: c's product meets its split in one multiply-add in every instance, so
+                    // that they agree in every bit)
+                    if constexpr (kOneByOne) asm volatile("" : "+v"(sum));
+                    c_of[gi][rb0 + i] = -kCodeBias * sum;
                 }
+                if constexpr (kOneByOne) __builtin_amdgcn_sched_barrier(0);
             }
             wait_vector_loads<Sch::value.wait_b[gi]>();
             if constexpr (gi == 0) KILN_MID_TL(2);  // B(0) has arrived
