@@ -75,7 +75,7 @@ STATIC_SCRATCH_BYTES = 8 << 20   # KILN_W4A16_STATIC_SCRATCH_BYTES
 
 OK, ERR_PROB_SHAPE, ERR_KERN_SHAPE, ERR_LAUNCH, ERR_ARGUMENT, ERR_ZERO_POINT, ERR_SCRATCH = range(7)
 # bits of the workspace's sticky word (KILN_W4A16_WAIT_*): which bounded wait gave up
-WAIT_DECODE_EXCHANGE, WAIT_MID_EXCHANGE, WAIT_DECODE_FOLD, WAIT_MID_FOLD, WAIT_PREFILL_FOLD = 1, 2, 4, 8, 16
+WAIT_DECODE_EXCHANGE, WAIT_MID_EXCHANGE, WAIT_DECODE_FOLD, WAIT_MID_FOLD, WAIT_PREFILL_FOLD, WAIT_PREFILL_MEETING = 1, 2, 4, 8, 16, 32
 
 # The tuning build: the same sources with -DKILN_W4A16_TUNING_HOOKS, which adds process-wide
 # overrides of the automatic plan (kiln_w4a16_debug_*).  Tests and profiling scripts that pin a
@@ -87,7 +87,7 @@ TUNING_EXPORTS = (
     "kiln_w4a16_debug_prefill_bm", "kiln_w4a16_debug_prefill_nb_full", "kiln_w4a16_debug_decode_direct_max_m",
     "kiln_w4a16_debug_decode_group_major", "kiln_w4a16_debug_decode_runs_per_launch", "kiln_w4a16_debug_tune",
     "kiln_w4a16_debug_mid", "kiln_w4a16_debug_gmp", "kiln_w4a16_debug_flagged", "kiln_w4a16_debug_lora_fold",
-    "kiln_w4a16_debug_rowsum_fold", "kiln_w4a16_debug_mid_waves",
+    "kiln_w4a16_debug_rowsum_fold", "kiln_w4a16_debug_mid_waves", "kiln_w4a16_debug_meeting",
 )
 
 _libs: dict[bool, ctypes.CDLL] = {}

@@ -100,4 +100,46 @@ __device__ __forceinline__ void wait_vector_loads() {
 }
 __device__ __forceinline__ void wait_lds_reads() { asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory"); }
 
+// Where some of a block's wavefronts meet without the others: a count in LDS that each raises by one.  LDS serves a
+// wavefront's requests in order, so who raises it has read what it asked for before.  The look is asked for some products
+// later and answered a product after that; who then finds others missing polls.  They are resident, and each raises the
+// count before it waits, so the bound -- 2^22 polls, a quarter of a second or more -- is not reached; if it is, the wavefront
+// raises kGaveUpPrefillMeeting in the workspace's sticky word, as the other bounded waits do, and goes on.  (gave_up_at: the
+// word's address less the bit, so that one register is the distance and the value.)  The loop is inside the asm statement:
+// registers that loads in flight will fill must not meet the end of a basic block.  The atomic's count comes on top of the
+// loads that later waits count, so they wait for no less.  Every lane is active.
+constexpr int kMeetingPolls = 0x400000;
+__device__ __forceinline__ void meeting_signal(unsigned lds_addr) {
+    uint32_t at, one;
+    asm volatile("s_mov_b64 exec, 1\n\tv_mov_b32 %0, %2\n\tv_mov_b32 %1, 1\n\tds_add_u32 %0, %1\n\ts_mov_b64 exec, -1"
+                 : "=&v"(at), "=&v"(one)
+                 : "s"(lds_addr)
+                 : "memory");
+}
+__device__ __forceinline__ void meeting_look(unsigned lds_addr, uint32_t &seen) {
+    asm volatile("v_mov_b32 %0, %1\n\tds_read_b32 %0, %0" : "=&v"(seen) : "s"(lds_addr) : "memory");
+}
+template <int POLLS = kMeetingPolls>
+__device__ __forceinline__ void meeting_wait(unsigned lds_addr, uint32_t &seen, int expected, const void *gave_up_at) {
+    int value, polls;
+    asm volatile("s_mov_b32 %2, %7\n"
+                 "Lmeeting_%=:\n\t"
+                 "s_waitcnt lgkmcnt(0)\n\t"
+                 "v_readfirstlane_b32 %1, %0\n\t"
+                 "s_cmp_ge_i32 %1, %4\n\t"
+                 "s_cbranch_scc1 Lmet_%=\n\t"
+                 "s_sub_u32 %2, %2, 1\n\t"
+                 "s_cbranch_scc1 Lgave_up_%=\n\t"
+                 "v_mov_b32 %0, %3\n\t"
+                 "ds_read_b32 %0, %0\n\t"
+                 "s_branch Lmeeting_%=\n"
+                 "Lgave_up_%=:\n\t"
+                 "v_mov_b32 %0, %6\n\t"
+                 "global_atomic_or %0, %0, %5\n"
+                 "Lmet_%=:"
+                 : "+v"(seen), "=&s"(value), "=&s"(polls)
+                 : "s"(lds_addr), "s"(expected), "s"(gave_up_at), "n"((int)kGaveUpPrefillMeeting), "n"(POLLS)
+                 : "memory", "scc");
+}
+
 }  // namespace kiln

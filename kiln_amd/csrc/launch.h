@@ -28,6 +28,7 @@ enum WaitGaveUp : unsigned {
     kGaveUpDecodeFold = 4u,      // a block of up to 16 rows waiting for the folded LoRA projection
     kGaveUpMidFold = 8u,         // the same in a launch of the mid-M kernel with adapters (17...320 rows)
     kGaveUpPrefillFold = 16u,    // the same on the matrix-core path
+    kGaveUpPrefillMeeting = 32u, // there: wavefronts that share a half of their block's K
 };
 
 // One launch of the decode kernel: M <= 16 rows of A against the whole weight.

@@ -6,6 +6,7 @@
 #include <unordered_map>
 
 #include "kiln_w4a16.h"
+#include "async_loads.h"
 #include "device_common.h"
 #include "launch.h"
 
@@ -82,6 +83,20 @@ struct Tuning {
 };
 #ifdef KILN_W4A16_TUNING_HOOKS
 Tuning g_tune;
+// the wait for a block's wavefronts (meeting_wait), with a bound that can be reached
+__global__ __launch_bounds__(256) void meeting_probe_kernel(int *workspace, int *raised, int arrivals, int expected) {
+    __shared__ uint32_t count;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const unsigned at = (unsigned)(size_t)(lds_ptr_t)&count;
+    if (threadIdx.x == 0) count = 0;
+    __syncthreads();
+    if (wave < arrivals) meeting_signal(at);
+    __syncthreads();
+    uint32_t seen = 0;
+    meeting_look(at, seen);
+    meeting_wait<16>(at, seen, expected, reinterpret_cast<const char *>(workspace) + kWsErrorOffset - kGaveUpPrefillMeeting);
+    if ((threadIdx.x & 63) == 0) raised[wave] = 1;
+}
 #else
 constexpr Tuning g_tune{};
 #endif
@@ -1338,6 +1353,13 @@ void kiln_w4a16_debug_tune(int waves, int run, int kslices) {
     g_tune.force_u = run;
     g_tune.force_ks = kslices;
     tuning_changed();
+}
+// One block of four wavefronts, the first `arrivals` of which raise a count that all wait to see at `expected`, sixteen
+// polls long: raised[] (four words) is what each goes on with, 1.
+int kiln_w4a16_debug_meeting(void *workspace, int *raised, int arrivals, int expected, void *stream) {
+    if (!workspace || !raised || arrivals < 0 || arrivals > 4 || expected < 0) return -1;
+    meeting_probe_kernel<<<1, 256, 0, reinterpret_cast<hipStream_t>(stream)>>>((int *)workspace, raised, arrivals, expected);
+    return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 #endif
 

@@ -109,40 +109,6 @@ __device__ __forceinline__ void direct_load_b128(const void *gptr, unsigned lds_
                  : "memory", "m0");
 }
 
-// Where some of a block's wavefronts meet without the others: a count in LDS that each raises by one.  LDS serves a
-// wavefront's requests in order, so who raises it has read what it asked for before.  The look is asked for some products
-// later and answered a product after that; who then finds others missing polls (they are resident, so the bound, one
-// second and more, is never reached).  The loop is inside the asm statement: registers that loads in flight will fill must
-// not meet the end of a basic block.  Every lane is active.
-__device__ __forceinline__ void meeting_signal(unsigned lds_addr) {
-    uint32_t at, one;
-    asm volatile("s_mov_b64 exec, 1\n\tv_mov_b32 %0, %2\n\tv_mov_b32 %1, 1\n\tds_add_u32 %0, %1\n\ts_mov_b64 exec, -1"
-                 : "=&v"(at), "=&v"(one)
-                 : "s"(lds_addr)
-                 : "memory");
-}
-__device__ __forceinline__ void meeting_look(unsigned lds_addr, uint32_t &seen) {
-    asm volatile("v_mov_b32 %0, %1\n\tds_read_b32 %0, %0" : "=&v"(seen) : "s"(lds_addr) : "memory");
-}
-__device__ __forceinline__ void meeting_wait(unsigned lds_addr, uint32_t &seen, int expected) {
-    int value, polls;
-    asm volatile("s_mov_b32 %2, 0x400000\n"
-                 "Lmeeting_%=:\n\t"
-                 "s_waitcnt lgkmcnt(0)\n\t"
-                 "v_readfirstlane_b32 %1, %0\n\t"
-                 "s_sub_u32 %2, %2, 1\n\t"
-                 "s_cbranch_scc1 Lmet_%=\n\t"
-                 "s_cmp_ge_i32 %1, %4\n\t"
-                 "s_cbranch_scc1 Lmet_%=\n\t"
-                 "v_mov_b32 %0, %3\n\t"
-                 "ds_read_b32 %0, %0\n\t"
-                 "s_branch Lmeeting_%=\n"
-                 "Lmet_%=:"
-                 : "+v"(seen), "=&s"(value), "=&s"(polls)
-                 : "s"(lds_addr), "s"(expected)
-                 : "memory", "scc");
-}
-
 // Probe builds only (-DKILN_PREFILL_TIMELINE): wall-clock stamps per block.
 #ifdef KILN_PREFILL_TIMELINE
 __device__ long long *g_timeline;
@@ -476,6 +442,7 @@ __global__ __launch_bounds__(64 * WM * NWN * WK, (WM == 2 && NWN == 4) ? 1 : 2) 
     // WK = 2: where a half's wavefronts meet once a stage (meeting_signal), and how many arrivals there will have been
     [[maybe_unused]] const unsigned meeting = (unsigned)(size_t)(lds_ptr_t)&s_meeting[half];
     [[maybe_unused]] int met = 0;
+    [[maybe_unused]] const char *const gave_up_at = uniform(reinterpret_cast<const char *>(counters) + kWsErrorOffset - kGaveUpPrefillMeeting);
     const char *a_ptr = uniform(reinterpret_cast<const char *>(A) + ((size_t)m0 * K + (size_t)g_begin * kGroupK) * 2);  // this group's stages
     const unsigned lds_base = (unsigned)(size_t)(lds_ptr_t)lds, ring_base = lds_base + ring;
     auto load_a = [&](const char *base, int slot) {
@@ -738,7 +705,7 @@ __global__ __launch_bounds__(64 * WM * NWN * WK, (WM == 2 && NWN == 4) ? 1 : 2) 
                 });
                 if constexpr (mi == 0) {
                     if constexpr (WK == 2) {
-                        meeting_wait(meeting, seen_met, met);
+                        meeting_wait(meeting, seen_met, met, gave_up_at);
                     } else {
                         wait_vector_loads<kStageLanded>();
                         wait_lds_reads();
@@ -1695,6 +1662,7 @@ hipError_t launch_prefill(const PrefillArgs &a, hipStream_t stream) {
     const bool inc = a.sums_in_loop;
     if (inc && a.bm != 128) return hipErrorInvalidValue;
     const bool halves = prefill_halves_k(a.M, a.N, a.K, shape, a.cus);
+    if (halves && !a.counters) return hipErrorInvalidValue;  // (the error word is at a fixed distance)
     const int inside = a.r_total == 0 && a.lora_words && !a.aext_ready && !inc ? prefill_rowsum_producers(a.M, a.N, a.K, shape, a.cus) : 0;
     const int sum_producers = inside > 0 ? inside : 0;
     int RP = 0;

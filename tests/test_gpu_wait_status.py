@@ -80,3 +80,27 @@ def test_module_level_health_check_reads_zero_after_ordinary_calls():
     marlin_gemm.workspace_reset()
     y = marlin_gemm.marlin_w4a16_gemm((torch.randn(16, k, device="cuda") * 0.5).to(torch.bfloat16), b, s, g)
     assert torch.isfinite(y.float()).all() and marlin_gemm.workspace_wait_status() == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("arrivals,expected", [(4, 4), (3, 4), (0, 1), (4, 2)])
+def test_a_meeting_of_wavefronts_that_gives_up_says_so(arrivals, expected):
+    """The wait of a block's wavefronts for one another, sixteen polls long: where some never come it ends, and says so in the
+    sticky word; where all have come the word stays zero."""
+    L = _lib.load_tuning()
+    try:
+        L.kiln_w4a16_debug_meeting.restype = ctypes.c_int
+        L.kiln_w4a16_debug_meeting.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_void_p]
+        zeroed, off = L.kiln_w4a16_workspace_zeroed_bytes(), L.kiln_w4a16_workspace_error_offset()
+        ws = torch.zeros(zeroed, dtype=torch.uint8, device="cuda")
+        ended = torch.zeros(4, dtype=torch.int32, device="cuda")
+        assert L.kiln_w4a16_debug_meeting(ws.data_ptr(), ended.data_ptr(), arrivals, expected,
+                                          torch.cuda.current_stream().cuda_stream) == 0
+        torch.cuda.synchronize()
+        assert ended.tolist() == [1, 1, 1, 1]
+        word = ws[off:off + 4].cpu().numpy().view(np.uint32)[0]
+        assert word == (0 if arrivals >= expected else _lib.WAIT_PREFILL_MEETING)
+        ws[off:off + 4] = 0
+        assert int(ws.max()) == 0       # and nothing else
+    finally:
+        _lib.use_shipped()
