@@ -131,3 +131,46 @@ def test_words_of_a_folded_launch_outlast_both_halves(m, k, n, g):
         assert float(err.max()) <= 2.0 ** -8, float(err.max())     # the bound of the calls above
         first = y if first is None else first
         assert torch.equal(y.view(torch.int16), first.view(torch.int16))
+
+
+@pytest.mark.parametrize("sms,m,k,n,rows,halves", [(64, 515, 1280, 2304, 128, 0), (64, 543, 2176, 1280, 64, 1), (128, 516, 1536, 1792, 64, 1),
+                                                   (128, 769, 3072, 4352, 128, 1), (200, 771, 768, 3328, 64, 1),
+                                                   (200, 1547, 1280, 3328, 128, 0)])
+def test_tiles_dealt_to_the_dies_for_other_counts_of_units(sms, m, k, n, rows, halves):
+    """Tiles that fit a caller's count of compute units, and that no rectangle of dies holds."""
+    L, plan = _lib.load(), (ctypes.c_int * 8)()
+    assert L.kiln_w4a16_debug_gemm_plan(m, n, k, sms, plan) == 0
+    assert (plan[0], plan[2], plan[6], plan[7]) == (1, rows, 0, halves)
+    gen = torch.Generator(device="cuda").manual_seed(m)
+    words = torch.randint(-2**31, 2**31, (k // 16, 2 * n), dtype=torch.int64, device="cuda", generator=gen).to(torch.int32)
+    scales = (torch.rand(k // 128, n, device="cuda", generator=gen) * 0.018 + 0.002).half()
+    x = torch.randn(m, k, device="cuda", generator=gen).to(torch.bfloat16)
+    ws = torch.zeros(L.kiln_w4a16_workspace_bytes_tuned(m, n, k, -1, -1, sms), dtype=torch.uint8, device="cuda")
+    want = x.double() @ marlin_gemm.dequant_f32(words, scales, 128).double()
+    y = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+    assert L.kiln_marlin_w4a16_gemm(x.data_ptr(), words.data_ptr(), y.data_ptr(), scales.data_ptr(), m, n, k, ws.data_ptr(), 128, 0,
+                                    torch.cuda.current_stream().cuda_stream, -1, -1, sms, 16) == _lib.OK
+    err = (y.double() - want).norm(dim=1) / want.norm(dim=1)
+    assert float(err.max()) <= 2.0 ** -8, float(err.max())      # the bound of the calls above
+    assert int(ws[:L.kiln_w4a16_workspace_zeroed_bytes()].max()) == 0
+
+
+@pytest.mark.parametrize("m,k,n,g", [(777, 2688, 2560, 128), (1300, 1664, 1536, -1)])
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan")])
+def test_what_is_not_finite_in_the_group_that_both_halves_read(m, k, n, g, value):
+    """With an odd number of groups the second half reads the first's last group and multiplies what it got by 0: rows with an
+    infinity or NaN there are not finite, as with one set of wavefronts (the surplus of the codes is inf - inf), and no other
+    row is touched."""
+    words, scales, xs = _operands(m, k, n, g)
+    plan = (ctypes.c_int * 8)()
+    _lib.load().kiln_w4a16_debug_gemm_plan(m, n, k, torch.cuda.get_device_properties(0).multi_processor_count, plan)
+    groups = -(-(k // 128) // plan[5])     # of a block: the first slice's
+    assert groups % 2 == 1
+    clean = marlin_gemm.marlin_w4a16_gemm(xs[0], words, scales, g)
+    x, hit = xs[0].clone(), torch.tensor([0, 63, 64, m - 1], device="cuda")
+    x[hit, (groups // 2) * 128 + 77] = value
+    y = marlin_gemm.marlin_w4a16_gemm(x, words, scales, g)
+    assert not bool(torch.isfinite(y[hit]).any())
+    others = torch.ones(m, dtype=torch.bool, device="cuda")
+    others[hit] = False
+    assert torch.equal(y[others].view(torch.int16), clean[others].view(torch.int16))
