@@ -252,6 +252,28 @@ kiln_marlin_status_t kiln_w4a16_stack_adapters(
     void *a_cat, void *b_cat, void *stream);
 
 /*
+ * kiln_w4a16_gemm_lora, or with `swiglu` kiln_w4a16_gemm_swiglu_lora (prob_n: the packed columns, 2 * n_out), for adapters
+ * that are not stacked: side i is a projection's adapters as they lie -- lora_a bf16 [rank, k], lora_b bf16 [rows, rank],
+ * rank a multiple of 8, both on 16 bytes -- whose columns are the GEMM's from first_row on (with `swiglu`: rows = n_out,
+ * first_row 0 for gate and 8 for up).  Up to three sides in the order of their columns; columns of no side have no
+ * low-rank term.  ranks, scales: every adapter of every side in that order, at most eight, sum(ranks) = the sides' ranks
+ * together <= 64.  What kiln_w4a16_stack_adapters in front of the stacked entry point gives, without its launch (with up to four
+ * adapters in every bit; more are projected in the launch's own order of sums here, by a launch in front there).
+ * Taken where the launch reads them itself, up to 16 rows: kiln_w4a16_takes_adapter_sides (a pure query; 1: yes) -- elsewhere
+ * KILN_W4A16_ERR_KERN_SHAPE, and the caller stacks them.
+ */
+typedef struct {
+    const void *lora_a, *lora_b;
+    int rank, first_row, rows;
+} kiln_w4a16_adapter_side;
+int kiln_w4a16_takes_adapter_sides(int prob_m, int prob_n, int prob_k, const kiln_w4a16_adapter_side *sides, int n_sides,
+                                   int swiglu, int n_adapters, int dev);
+kiln_marlin_status_t kiln_w4a16_gemm_adapter_sides(
+    const void *A, const void *B, void *C, const void *s, int prob_m, int prob_n, int prob_k,
+    void *workspace, int groupsize, int dev, void *stream, const kiln_w4a16_adapter_side *sides, int n_sides,
+    int swiglu, int n_adapters, const int *ranks, const float *scales);
+
+/*
  * out[k, n] (f32, row-major) = (code - 8) * f32(scale), read from the tile
  * layout on the device.  The device-side statement of lib.rs:425; used to
  * prove the repack bit-exact.  No counterpart entry point in the reference.

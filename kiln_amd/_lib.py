@@ -27,6 +27,8 @@ EXPORTS = (
     "kiln_w4a16_mlp",
     "kiln_w4a16_mlp_workspace_bytes",
     "kiln_w4a16_stack_adapters",
+    "kiln_w4a16_takes_adapter_sides",
+    "kiln_w4a16_gemm_adapter_sides",
     "kiln_w4a16_quantize_and_pack_device",
     "kiln_w4a16_quantize_and_pack_many_device",
     "kiln_w4a16_interleave_gate_up_device",
@@ -202,6 +204,10 @@ def _load(tuning: bool) -> ctypes.CDLL:
     L.kiln_w4a16_mlp.argtypes = [vp, vp, vp, vp, vp, vp, i, i, i, i, vp, i, i, vp]
     L.kiln_w4a16_mlp_workspace_bytes.restype = c.c_size_t
     L.kiln_w4a16_mlp_workspace_bytes.argtypes = [i, i, i, i]
+    L.kiln_w4a16_takes_adapter_sides.restype = i
+    L.kiln_w4a16_takes_adapter_sides.argtypes = [i, i, i, vp, i, i, i, i]
+    L.kiln_w4a16_gemm_adapter_sides.restype = i
+    L.kiln_w4a16_gemm_adapter_sides.argtypes = [vp, vp, vp, vp, i, i, i, vp, i, i, vp, vp, i, i, i, c.POINTER(c.c_int), c.POINTER(c.c_float)]
     L.kiln_w4a16_stack_adapters.restype = i
     L.kiln_w4a16_stack_adapters.argtypes = [c.POINTER(vp), c.POINTER(vp), c.POINTER(i), c.POINTER(i), c.POINTER(i), i, i, i, i, i,
                                             vp, vp, vp]

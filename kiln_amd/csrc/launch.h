@@ -40,6 +40,14 @@ constexpr int kDecodeFlaggedMaxSlices = 4;
 // block indices apart, which must be odd to differ modulo 8 for up to eight slices.
 inline int exchange_column_shift(int column_blocks) { return column_blocks % 2 == 0 ? 1 : 0; }
 
+// Adapters of projections that run as one GEMM, unstacked (lora_tail.h, LoraSides): q | k | v, or gate and up interleaved
+constexpr int kMaxAdapterSides = 3;
+struct AdapterSides {
+    const void *a[kMaxAdapterSides], *b[kMaxAdapterSides];
+    int ranks[kMaxAdapterSides], first[kMaxAdapterSides], rows[kMaxAdapterSides];
+    int count, interleaved;
+};
+
 struct DecodeArgs {
     const void *A;      // bf16 [M, K]
     const void *B;      // packed weights, tile layout
@@ -75,9 +83,10 @@ struct DecodeArgs {
     int lora_steps_per_slice = 0;  // 32-value steps of K per producer
     const void *lora_a = nullptr;  // bf16 [r_total, K]
     unsigned *lora_flags = nullptr;  // 64 KiB (16 replicas of flags and counts, 4 KiB apart), zero between launches
-    int lora_adapters = 0;         // 1...4
-    int lora_ends[4] = {};         // exclusive end column of adapter i (r_total past the last adapter)
-    float lora_scales[4] = {};     // its scale (0 past the last)
+    int lora_adapters = 0;         // 1...8
+    int lora_ends[8] = {};         // exclusive end column of adapter i (r_total past the last adapter)
+    float lora_scales[8] = {};     // its scale (0 past the last)
+    const AdapterSides *lora_sides = nullptr;  // with lora_producers: the adapters where they lie, lora_a and lora_b are not read
     bool swiglu = false;  // columns are gate/up interleaved by 8 inside every tile; C is [M, N/2] = silu(gate) * up
     int group_major = -1; // tuning: 0 never a group-major instance, 1 only the LDS-staged one, 2 the
                           // register-fragment one wherever a plan fits it; -1: automatic
@@ -111,6 +120,7 @@ hipError_t launch_decode(const DecodeArgs &args, hipStream_t stream);
 bool decode_gmp_ok(const DecodeArgs &a);                        // does the plan fit the private-staging instance?
 bool decode_gmp_fold_ok(const DecodeArgs &a);                   // ... with the LoRA projection folded into the launch?
 hipError_t launch_decode_gmp(const DecodeArgs &a, hipStream_t stream);
+hipError_t launch_decode_gmp_sides(const DecodeArgs &a, hipStream_t stream);  // ... with that of unstacked adapters (checked plan)
 hipError_t launch_decode_gmp_lora(const DecodeArgs &a, hipStream_t stream);  // its instances with the low-rank term (checked plan)
 
 // One launch of the mid-M kernel: runs of up to 64 rows (grid z) against the whole weight.

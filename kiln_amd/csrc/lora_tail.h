@@ -1,5 +1,7 @@
 // The low-rank term the small-M kernels add where they store a tile (gfx950 only).
 #pragma once
+#include <type_traits>
+
 #include "device_common.h"
 #include "launch.h"
 
@@ -85,6 +87,61 @@ __device__ __forceinline__ void lora_add_from_lds(f32x4 &v, const LoraTail &lo, 
     }
 }
 
+// The adapters of projections that run as one GEMM, where they lie: side i has A = bf16 [ranks, K] and B = bf16
+// [rows, ranks] of its own, ranks a multiple of 8, and the columns from col[i] on of the stacked rank axis.  Its rows of B
+// are the GEMM's columns from first[i] on; interleaved, those of every 16-column tile from first[i] (0: gate, 8: up) on,
+// eight of them.  Columns of no side have no term.  What it saves is launches, which bound these calls: stacking took one
+// of 3.4 us in front of every fused call, and q | k | v with two adapters each, six together, another of 5 us for the
+// projection, which the stacked form takes inside for four at most.  (A layer at 11 rows, two adapters of rank 8 on each
+// projection, 2560 / 9216 wide: 41.2 -> 33.1 us, four launches instead of seven.)
+struct LoraSides {
+    const uint16_t *a[kMaxAdapterSides];
+    const uint16_t *b[kMaxAdapterSides];
+    int col[kMaxAdapterSides + 1];   // past the last side: r_total
+    int first[kMaxAdapterSides];
+    int rows[kMaxAdapterSides];
+    int count;
+    int interleaved;
+};
+// the row of A of a rank column
+__device__ __forceinline__ const uint16_t *side_a_row(const LoraSides &s, int rank, int K) {
+    const uint16_t *base = s.a[0];
+    int from = 0;
+#pragma unroll
+    for (int i = 1; i < kMaxAdapterSides; ++i)
+        if (i < s.count && rank >= s.col[i]) {
+            base = s.a[i];
+            from = s.col[i];
+        }
+    return base + (size_t)(rank - from) * K;
+}
+// eight rank columns from j8 on (a multiple of 8) of a column's row of B: zeros but where they are its own side's
+__device__ __forceinline__ u32x4 side_b_unit(const LoraSides &s, int column, int j8) {
+    u32x4 v = {0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int i = 0; i < kMaxAdapterSides; ++i) {
+        const int row = s.interleaved ? (column >> 4) * 8 + (column & 7) : column - s.first[i];
+        const bool mine = s.interleaved ? (column & 8) == s.first[i] : row >= 0 && row < s.rows[i];
+        if (i < s.count && mine && j8 >= s.col[i] && j8 < s.col[i + 1])
+            v = *reinterpret_cast<const u32x4 *>(s.b[i] + (size_t)row * (s.col[i + 1] - s.col[i]) + (j8 - s.col[i]));
+    }
+    return v;
+}
+inline LoraSides lora_sides(const AdapterSides *h) {
+    LoraSides s{};
+    s.count = h->count;
+    s.interleaved = h->interleaved;
+    for (int i = 0; i < h->count; ++i) {
+        s.a[i] = (const uint16_t *)h->a[i];
+        s.b[i] = (const uint16_t *)h->b[i];
+        s.first[i] = h->first[i];
+        s.rows[i] = h->rows[i];
+        s.col[i + 1] = s.col[i] + h->ranks[i];
+    }
+    for (int i = h->count; i < kMaxAdapterSides; ++i) s.col[i + 1] = s.col[i];
+    return s;
+}
+
 // The projection T computed inside the launch that adds it, by `producers` extra blocks at the
 // front of the grid (one K slice each) while the other blocks stream their weights.  A producer
 // writes its slice of T with device-scope stores, waits until they are acknowledged and raises
@@ -111,8 +168,16 @@ struct LoraFold {
     int e0, e1, e2, e3;      // (four adapters at most: every member is a scalar register for the whole kernel)
     float s0, s1, s2, s3;
 };
+// ... of unstacked adapters, which a_cat, the tail's b and the four above do not describe.  Instances of their own: with
+// both forms in one kernel the stacked one lost 0.1 to 0.5 us a launch to the other's registers.
+struct LoraSidesFold : LoraFold {
+    LoraSides sides;
+    int ends[8];             // read with constant indices only
+    float scales[8];
+};
 constexpr int kLoraFoldMaxProducers = 16;
 constexpr int kLoraFoldMaxAdapters = 4;
+constexpr int kLoraSidesMaxAdapters = 8;
 constexpr int kLoraFoldStepsPerWave = 12;  // 32-value steps of K one producer wavefront takes, at most
 constexpr int kLoraFoldReplicas = 16;
 constexpr int kLoraFoldReplicaWords = 1024;                  // 4 KiB from one replica to the next
@@ -127,7 +192,8 @@ constexpr int kLoraFoldSpinLimit = 1 << 20;
 // Q-th step of the slice from w / JT on (JT = rp / 16 rank tiles, Q = nw / JT; nw >= JT); the Q
 // parts of a tile meet in LDS (nw KiB) and are added in ascending order.  Every wavefront of the
 // block must call this (two barriers inside).
-__device__ __forceinline__ void lora_project_slice(const uint16_t *__restrict__ X, const LoraFold &fold,
+template <class Fold>
+__device__ __forceinline__ void lora_project_slice(const uint16_t *__restrict__ X, const Fold &fold,
                                                    const LoraTail &lo, int M, int K, int slice,
                                                    unsigned char *lds, int wave, int lane, int nw) {
     const int JT = lo.rp >> 4, Q = nw / JT;
@@ -138,7 +204,9 @@ __device__ __forceinline__ void lora_project_slice(const uint16_t *__restrict__ 
     if (q < Q) {
         const int rank = jt * 16 + r;
         const uint16_t *xp = X + (size_t)min(r, M - 1) * K + kq * 8;
-        const uint16_t *ap = fold.a_cat + (size_t)min(rank, lo.r_total - 1) * K + kq * 8;
+        const uint16_t *ap;
+        if constexpr (std::is_same_v<Fold, LoraSidesFold>) ap = side_a_row(fold.sides, min(rank, lo.r_total - 1), K) + kq * 8;
+        else ap = fold.a_cat + (size_t)min(rank, lo.r_total - 1) * K + kq * 8;
         const bool live = rank < lo.r_total;  // padding columns of T are zero
         // four steps requested at a time (more in flight would raise the whole kernel's register count,
         // and with it the launch cost of calls without adapters: measured +0.45 us at 97 instead of 82)
@@ -169,10 +237,15 @@ __device__ __forceinline__ void lora_project_slice(const uint16_t *__restrict__ 
         const int j = wave * 16 + r;
         // the scale of the first adapter whose columns end behind j
         float sc = 0.f;
-        sc = j < fold.e3 ? fold.s3 : sc;
-        sc = j < fold.e2 ? fold.s2 : sc;
-        sc = j < fold.e1 ? fold.s1 : sc;
-        sc = j < fold.e0 ? fold.s0 : sc;
+        if constexpr (std::is_same_v<Fold, LoraSidesFold>) {
+#pragma unroll
+            for (int i = kLoraSidesMaxAdapters - 1; i >= 0; --i) sc = j < fold.ends[i] ? fold.scales[i] : sc;
+        } else {
+            sc = j < fold.e3 ? fold.s3 : sc;
+            sc = j < fold.e2 ? fold.s2 : sc;
+            sc = j < fold.e1 ? fold.s1 : sc;
+            sc = j < fold.e0 ? fold.s0 : sc;
+        }
         uint16_t *tz = fold.t + (size_t)slice * lo.t_rows * lo.rp;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {

@@ -36,6 +36,8 @@ struct Library {
     decltype(&kiln_w4a16_mlp_workspace_bytes) mlp_workspace_bytes = nullptr;
     decltype(&kiln_w4a16_stack_adapters) stack_adapters = nullptr;
     decltype(&kiln_w4a16_quantize_and_pack_many_device) quantize = nullptr;
+    decltype(&kiln_w4a16_takes_adapter_sides) takes_sides = nullptr;
+    decltype(&kiln_w4a16_gemm_adapter_sides) gemm_sides = nullptr;
 };
 Library g_lib;  // written by bind() under the interpreter lock, like everything below
 
@@ -294,7 +296,8 @@ bool add_side(PyObject *o, double scale, const Problem &p, int first, int rows, 
 // linear_sides(x, b_packed, scales, groupsize, swiglu, sides, widths, lora_scale, split): a GEMM whose columns belong
 // to several projections -- side by side, `widths` columns each, or with `swiglu` gate and up interleaved
 // (widths = n_out twice) -- each with its adapters or None.  Several sides, and stacked ranks that are not
-// multiples of 8, become one stacked set in a launch of their own in front.  `split`: the result comes as
+// multiples of 8, are read where they lie if the launch can, else they become one stacked set in a launch of their own in
+// front.  `split`: the result comes as
 // one view per projection.
 PyObject *py_linear_sides(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     HANDLE_TH_ERRORS
@@ -319,7 +322,13 @@ PyObject *py_linear_sides(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     if (first != p.n || (swiglu && (widths.size() != 2 || widths[0] != widths[1]))) Py_RETURN_NONE;
     Launch at_(p.device);
     if (!at_.find_workspace(p.device, g_lib.workspace_bytes(p.m, p.n, p.k))) Py_RETURN_NONE;
-    if (!sides.empty()) {
+    kiln_w4a16_adapter_side own[8];
+    for (size_t i = 0; i < sides.size(); ++i)
+        own[i] = {sides[i].a.data_ptr(), sides[i].b.data_ptr(), sides[i].rank, sides[i].first, sides[i].rows};
+    const int n_sides = (int)sides.size(), n_adapters = (int)l.ranks.size();
+    const bool in_place = !(n_sides == 1 && sides[0].rows == p.n) && n_sides > 0 &&
+                          g_lib.takes_sides(p.m, p.n, p.k, own, n_sides, swiglu ? 1 : 0, n_adapters, p.device.index());
+    if (!sides.empty() && !in_place) {
         const int padded = (l.r_total + 7) / 8 * 8;
         if (sides.size() == 1 && padded == l.r_total && sides[0].rows == p.n) {
             l.a = sides[0].a;
@@ -332,11 +341,11 @@ PyObject *py_linear_sides(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
             const void *pa[8], *pb[8];
             int ranks[8], firsts[8], rows[8];
             for (size_t i = 0; i < sides.size(); ++i) {
-                pa[i] = sides[i].a.data_ptr();
-                pb[i] = sides[i].b.data_ptr();
-                ranks[i] = sides[i].rank;
-                firsts[i] = sides[i].first;
-                rows[i] = sides[i].rows;
+                pa[i] = own[i].lora_a;
+                pb[i] = own[i].lora_b;
+                ranks[i] = own[i].rank;
+                firsts[i] = own[i].first_row;
+                rows[i] = own[i].rows;
             }
             l.ranks.back() += padded - l.r_total;  // the last adapter gets the zero columns
             l.r_total = padded;
@@ -348,7 +357,19 @@ PyObject *py_linear_sides(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     }
     at::Tensor out;
     if (!output_of(nullptr, *p.x, swiglu ? p.n / 2 : p.n, p.device, &out)) Py_RETURN_NONE;
-    if (call(p, out, swiglu, sides.empty() ? nullptr : &l, at_) != KILN_W4A16_OK) Py_RETURN_NONE;
+    int st = KILN_W4A16_OK;
+    if (in_place) {
+        const void *x = p.x->data_ptr(), *b = p.b->data_ptr();
+        void *s = p.s->data_ptr(), *c = out.data_ptr(), *ws = at_.workspace.data_ptr();
+        const int dev = p.device.index();
+        Py_BEGIN_ALLOW_THREADS
+        st = g_lib.gemm_sides(x, b, c, s, p.m, p.n, p.k, ws, p.groupsize, dev, at_.stream, own, n_sides, swiglu ? 1 : 0, n_adapters,
+                              l.ranks.data(), l.scales.data());
+        Py_END_ALLOW_THREADS
+    } else {
+        st = call(p, out, swiglu, sides.empty() ? nullptr : &l, at_);
+    }
+    if (st != KILN_W4A16_OK) Py_RETURN_NONE;
     if (!split) return THPVariable_Wrap(std::move(out));
     std::vector<int64_t> w(widths.begin(), widths.end());
     std::vector<at::Tensor> parts = out.split_with_sizes(w, -1);
@@ -527,12 +548,12 @@ PyObject *py_set_workspaces(PyObject *, PyObject *const *args, Py_ssize_t nargs)
 
 // bind(addresses of the library's functions, in the order of Library)
 PyObject *py_bind(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
-    if (nargs != 9) {
-        PyErr_SetString(PyExc_TypeError, "bind takes nine function addresses");
+    if (nargs != 11) {
+        PyErr_SetString(PyExc_TypeError, "bind takes eleven function addresses");
         return nullptr;
     }
-    void *p[9];
-    for (int i = 0; i < 9; ++i) p[i] = PyLong_AsVoidPtr(args[i]);
+    void *p[11];
+    for (int i = 0; i < 11; ++i) p[i] = PyLong_AsVoidPtr(args[i]);
     if (PyErr_Occurred()) return nullptr;
     g_lib.gemm = reinterpret_cast<decltype(g_lib.gemm)>(p[0]);
     g_lib.gemm_lora = reinterpret_cast<decltype(g_lib.gemm_lora)>(p[1]);
@@ -543,6 +564,8 @@ PyObject *py_bind(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     g_lib.mlp_workspace_bytes = reinterpret_cast<decltype(g_lib.mlp_workspace_bytes)>(p[6]);
     g_lib.stack_adapters = reinterpret_cast<decltype(g_lib.stack_adapters)>(p[7]);
     g_lib.quantize = reinterpret_cast<decltype(g_lib.quantize)>(p[8]);
+    g_lib.takes_sides = reinterpret_cast<decltype(g_lib.takes_sides)>(p[9]);
+    g_lib.gemm_sides = reinterpret_cast<decltype(g_lib.gemm_sides)>(p[10]);
     Py_RETURN_NONE;
 }
 

@@ -859,6 +859,7 @@ struct LoraSpec {
     int r_total, n_adapters;
     const int *ranks;    // host arrays of length n_adapters
     const float *scales;
+    const AdapterSides *sides = nullptr;  // in place of a and b, which are null: calls that lora_in_launch() takes
 };
 
 // Bytes a call of m rows needs, made monotone in m: the largest need of any m' <= m.  The plan
@@ -930,6 +931,35 @@ bool mlp_passes_row_sums(int m, int hidden, int n_out, int n_down, int cus, bool
            prefill_reads_row_sums(m, n_down, n_out, down->gp.pf);
 }
 
+// Does a call with adapters project x onto them in the first blocks of its own launch on the private-staging kernel?  The
+// fields of its launch that say how.  The producers take compute units of their own: where the launch still fits the
+// chip in one round (the in-projection's 256 blocks do not: 12.6 us folded against 10.6 with the launch of its own), or
+// runs in several rounds anyway (5120 -> 13824, 432 blocks: 14.8 us folded against 18.8).
+bool lora_in_launch(const GemmPlan &gp, int m, int k, int cus, const LoraSpec &lora, void *t, void *flags, DecodeArgs *f) {
+    if (g_tune.lora_fold == 0 || gp.prefill || gp.mid || gp.launches != 1 || !gp.dl[0].plan.gmp || gp.dl[0].M != m) return false;
+    const DecodePlan &plan = gp.dl[0].plan;
+    const int steps = k / 32;
+    int kz = lora_project_slices(m, k);
+    f->lora_steps_per_slice = ((steps + kz - 1) / kz + 3) / 4 * 4;  // whole 128-value groups, as the projection launch cuts them
+    kz = (steps + f->lora_steps_per_slice - 1) / f->lora_steps_per_slice;
+    f->M = m;
+    f->K = k;
+    f->KS = plan.KS;
+    f->GS = plan.GS;
+    f->waves = plan.waves;
+    f->gm_tiles = plan.gm_tiles;
+    f->r_total = lora.r_total;
+    f->lora_a = lora.a;
+    f->lora_sides = lora.sides;
+    f->lora_t = t;
+    f->lora_flags = reinterpret_cast<unsigned *>(flags);
+    f->lora_producers = f->lora_slices = kz;
+    f->lora_rows = m;
+    f->lora_adapters = lora.n_adapters;
+    const int blocks = plan.BPS * plan.KS;
+    return decode_gmp_fold_ok(*f) && (blocks + kz <= cus || blocks > cus || g_tune.lora_fold == 2);
+}
+
 // The GEMM behind every entry point: small-M or matrix-core path by row count, with the
 // optional low-rank term.
 kiln_marlin_status_t gemm_any(const void *A, const void *B, void *C, const void *s, int prob_m, int prob_n,
@@ -955,6 +985,10 @@ kiln_marlin_status_t gemm_any(const void *A, const void *B, void *C, const void 
     const WorkspaceLayout &wl = planned->wl;
     char *ws = reinterpret_cast<char *>(workspace);
     char *lora_t = ws + wl.lora_t;
+    if (lora && lora->sides) {  // (the entry point has asked: nothing else takes them)
+        DecodeArgs ask{};
+        if (!lora_in_launch(gp, prob_m, prob_k, cus, *lora, lora_t, ws, &ask)) return KILN_W4A16_ERR_KERN_SHAPE;
+    }
     if (gp.prefill) {
         PrefillArgs pa{};
         pa.A = A;
@@ -1055,37 +1089,11 @@ kiln_marlin_status_t gemm_any(const void *A, const void *B, void *C, const void 
     int rp = 0, lora_slices = 1;
     // Up to 16 rows on the private-staging kernel: the projection rides in the GEMM launch (extra
     // blocks at the front of its grid) instead of running as a launch of its own.
-    DecodeArgs fold_probe{};
-    bool fold = false;
-    int fold_steps = 0;
-    if (lora && g_tune.lora_fold != 0 && gp.launches == 1 && gp.dl[0].plan.gmp && gp.dl[0].M == prob_m) {
-        const int steps = prob_k / 32;
-        int kz = lora_project_slices(prob_m, prob_k);
-        fold_steps = ((steps + kz - 1) / kz + 3) / 4 * 4;  // whole 128-value groups, as the projection launch cuts them
-        kz = (steps + fold_steps - 1) / fold_steps;
-        fold_probe.M = prob_m;
-        fold_probe.K = prob_k;
-        fold_probe.KS = gp.dl[0].plan.KS;
-        fold_probe.GS = gp.dl[0].plan.GS;
-        fold_probe.waves = gp.dl[0].plan.waves;
-        fold_probe.gm_tiles = gp.dl[0].plan.gm_tiles;
-        fold_probe.r_total = lora->r_total;
-        fold_probe.lora_a = lora->a;
-        fold_probe.lora_t = lora_t;
-        fold_probe.lora_flags = reinterpret_cast<unsigned *>(ws + kFoldFlagOffset);
-        fold_probe.lora_producers = fold_probe.lora_slices = kz;
-        fold_probe.lora_steps_per_slice = fold_steps;
-        fold_probe.lora_rows = prob_m;
-        fold_probe.lora_adapters = lora->n_adapters;
-        // the producers take compute units of their own: where the launch still fits the chip in one round
-        // (the in-projection's 256 blocks do not: 12.6 us folded against 10.6 with the launch of its own), or
-        // runs in several rounds anyway (5120 -> 13824, 432 blocks: 14.8 us folded against 18.8)
-        const int blocks = gp.dl[0].plan.BPS * gp.dl[0].plan.KS;
-        fold = decode_gmp_fold_ok(fold_probe) && (blocks + kz <= cus || blocks > cus || g_tune.lora_fold == 2);
-        if (fold) {
-            lora_slices = kz;
-            rp = (lora->r_total + 15) / 16 * 16;
-        }
+    DecodeArgs in_launch{};
+    const bool fold = lora && lora_in_launch(gp, prob_m, prob_k, cus, *lora, lora_t, ws + kFoldFlagOffset, &in_launch);
+    if (fold) {
+        lora_slices = in_launch.lora_slices;
+        rp = (lora->r_total + 15) / 16 * 16;
     }
     if (lora && !fold) {  // the scaled projection of all rows onto the adapters, once, ahead of the runs
         PrefillArgs pj{};
@@ -1123,12 +1131,13 @@ kiln_marlin_status_t gemm_any(const void *A, const void *B, void *C, const void 
             a.lora_rows = prob_m;
             if (fold) {
                 a.lora_producers = lora_slices;
-                a.lora_steps_per_slice = fold_steps;
+                a.lora_steps_per_slice = in_launch.lora_steps_per_slice;
                 a.lora_a = lora->a;
-                a.lora_flags = fold_probe.lora_flags;
+                a.lora_sides = lora->sides;
+                a.lora_flags = in_launch.lora_flags;
                 a.lora_adapters = lora->n_adapters;
                 int end = 0;
-                for (int j = 0; j < 4; ++j) {
+                for (int j = 0; j < 8; ++j) {
                     if (j < lora->n_adapters) end += lora->ranks[j];
                     a.lora_ends[j] = end;
                     a.lora_scales[j] = j < lora->n_adapters ? lora->scales[j] : 0.f;
@@ -1430,6 +1439,74 @@ kiln_marlin_status_t kiln_w4a16_gemm_swiglu_lora(const void *A, const void *B, v
     // follow the packed columns, so an adapter of gate and one of up are two column blocks of one stacked B
     const LoraSpec lora{lora_a, lora_b, r_total, n_adapters, ranks, scales};
     return gemm_any(A, B, C, s, prob_m, 2 * n_out, prob_k, workspace, groupsize, dev, stream, -1, -1, -1, &lora, true);
+}
+
+// ---- fused calls whose projections keep adapters of their own -----------------------------------------
+static kiln_marlin_status_t sides_of(const kiln_w4a16_adapter_side *sides, int n_sides, int prob_n, int swiglu, AdapterSides *out, int *r_total) {
+    if (!sides || n_sides < 1) return KILN_W4A16_ERR_ARGUMENT;
+    if (n_sides > kMaxAdapterSides) return KILN_W4A16_ERR_KERN_SHAPE;
+    *out = AdapterSides{};
+    out->count = n_sides;
+    out->interleaved = swiglu ? 1 : 0;
+    *r_total = 0;
+    int end = 0;  // sides in the order of their columns, none twice
+    for (int i = 0; i < n_sides; ++i) {
+        const kiln_w4a16_adapter_side &s = sides[i];
+        if (s.rank < 1 || s.rank > 64 || s.rows < 1 || s.first_row < 0) return KILN_W4A16_ERR_ARGUMENT;
+        // every address the kernel forms lies inside a side's own [rank, K] and [rows, rank]
+        if (swiglu ? (s.rows != prob_n / 2 || (s.first_row != 0 && s.first_row != 8) || s.first_row < end)
+                   : (s.first_row < end || s.rows > prob_n - s.first_row))
+            return KILN_W4A16_ERR_ARGUMENT;
+        end = swiglu ? s.first_row + 8 : s.first_row + s.rows;
+        *r_total += s.rank;
+        if (s.rank % 8 != 0 || *r_total > 64) return KILN_W4A16_ERR_KERN_SHAPE;
+        out->a[i] = s.lora_a;
+        out->b[i] = s.lora_b;
+        out->ranks[i] = s.rank;
+        out->first[i] = s.first_row;
+        out->rows[i] = s.rows;
+    }
+    return KILN_W4A16_OK;
+}
+
+int kiln_w4a16_takes_adapter_sides(int prob_m, int prob_n, int prob_k, const kiln_w4a16_adapter_side *sides, int n_sides, int swiglu,
+                                   int n_adapters, int dev) {
+    AdapterSides own;
+    int r_total = 0;
+    if (prob_m < 1 || prob_m > 16 || prob_n < 1 || prob_k < 1 || !shape_ok(prob_n, prob_k, 128) || n_adapters < 1 ||
+        sides_of(sides, n_sides, prob_n, swiglu, &own, &r_total) != KILN_W4A16_OK)
+        return 0;
+    static const unsigned probe = 0;  // never dereferenced
+    DecodeArgs ask{};
+    const int cus = compute_units(dev);
+    const LoraSpec lora{nullptr, nullptr, r_total, n_adapters, nullptr, nullptr, &own};
+    return lora_in_launch(plan_call(prob_m, prob_n, prob_k, cus, -1, -1, 1)->gp, prob_m, prob_k, cus, lora, const_cast<unsigned *>(&probe),
+                          const_cast<unsigned *>(&probe), &ask) ? 1 : 0;
+}
+
+kiln_marlin_status_t kiln_w4a16_gemm_adapter_sides(const void *A, const void *B, void *C, const void *s, int prob_m, int prob_n, int prob_k,
+                                                   void *workspace, int groupsize, int dev, void *stream, const kiln_w4a16_adapter_side *sides,
+                                                   int n_sides, int swiglu, int n_adapters, const int *ranks, const float *scales) {
+    if (prob_m < 0 || prob_n < 0 || prob_k < 0) return KILN_W4A16_ERR_PROB_SHAPE;
+    if (!shape_ok(prob_n, prob_k, groupsize)) return KILN_W4A16_ERR_PROB_SHAPE;
+    AdapterSides own;
+    int r_total = 0;
+    const kiln_marlin_status_t st = sides_of(sides, n_sides, prob_n, swiglu, &own, &r_total);
+    if (st != KILN_W4A16_OK) return st;
+    if (n_adapters < 1 || !ranks || !scales) return KILN_W4A16_ERR_ARGUMENT;
+    if (n_adapters > 8) return KILN_W4A16_ERR_KERN_SHAPE;
+    int sum = 0;
+    for (int i = 0; i < n_adapters; ++i) {
+        if (ranks[i] < 1 || ranks[i] > 64) return KILN_W4A16_ERR_ARGUMENT;
+        sum += ranks[i];
+    }
+    if (sum != r_total) return KILN_W4A16_ERR_ARGUMENT;
+    if (prob_m == 0 || prob_n == 0 || prob_k == 0) return KILN_W4A16_OK;
+    for (int i = 0; i < n_sides; ++i)
+        for (const void *p : {sides[i].lora_a, sides[i].lora_b})
+            if (!p || reinterpret_cast<uintptr_t>(p) % 16 != 0) return KILN_W4A16_ERR_ARGUMENT;
+    const LoraSpec lora{nullptr, nullptr, r_total, n_adapters, ranks, scales, &own};
+    return gemm_any(A, B, C, s, prob_m, prob_n, prob_k, workspace, groupsize, dev, stream, -1, -1, -1, &lora, swiglu != 0);
 }
 
 // ---- the MLP of a layer as one call -------------------------------------------------------------------

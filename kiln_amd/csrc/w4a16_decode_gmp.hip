@@ -34,19 +34,23 @@ constexpr int kGmpSlotBytes = 16 * 256;  // one group of A: 16 rows x 128 bf16
 #ifndef KILN_GMP_HEAD
 #define KILN_GMP_HEAD 3
 #endif
-// This file is compiled twice: as it is for calls without adapters, and with -DKILN_GMP_LORA=1 for
-// calls with them (launch_decode_gmp_lora only).  What the low-rank term adds -- one wavefront more,
+// This file is compiled three times: as it is for calls without adapters, with -DKILN_GMP_LORA=1 for
+// calls with them (launch_decode_gmp_lora only), and with =2 for calls whose adapters are not stacked
+// (launch_decode_gmp_sides only).  What the low-rank term adds -- one wavefront more,
 // its arguments, the signalling between the wavefronts -- then costs calls without adapters
 // nothing: as one kernel with run-time branches it cost them 0.1...0.2 us per launch.
 #ifndef KILN_GMP_LORA
 #define KILN_GMP_LORA 0
 #endif
-constexpr bool kGmpLora = KILN_GMP_LORA != 0;
+constexpr bool kGmpLora = KILN_GMP_LORA != 0, kGmpSides = KILN_GMP_LORA == 2;
+using GmpFold = std::conditional_t<kGmpSides, LoraSidesFold, LoraFold>;
 
 // Probe builds only (-DKILN_GMP_TIMELINE): wall-clock stamps (100 MHz) per wavefront.
 #ifdef KILN_GMP_TIMELINE
-#if KILN_GMP_LORA
+#if KILN_GMP_LORA == 1
 #define g_gmp_tl g_gmp_tl_lora
+#elif KILN_GMP_LORA == 2
+#define g_gmp_tl g_gmp_tl_sides
 #endif
 __device__ long long *g_gmp_tl;
 #define KILN_GMP_TL(i, v) tl_[i] = (v)
@@ -124,6 +128,30 @@ __device__ __forceinline__ void copy_to_lds(unsigned lds_addr, const uint16_t *s
         load_to_lds_b128(src, (uint32_t)min(base + lane, units - 1) * 16u, lds_addr + (unsigned)base * 16u);
 }
 
+// The rows of B_cat of a block's tiles to LDS, [column][rank]; unstacked adapters' through registers, six 16-byte units per
+// lane in flight (five tiles and 32 rank columns: 320 units).
+template <class Sides>
+__device__ __forceinline__ void fetch_b_rows(const Sides &sides, const LoraTail &lo, unsigned char *dst, int first_tile, int tiles, int lane) {
+    const int per_row = lo.r_total >> 3, units = tiles * kTileN * per_row;
+    if constexpr (std::is_same_v<Sides, LoraSides>) {
+        for (int base = 0; base < units; base += 6 * 64) {
+            u32x4 v[6];
+#pragma unroll
+            for (int i = 0; i < 6; ++i) {
+                const int u = min(base + 64 * i + lane, units - 1), row = u / per_row;
+                v[i] = side_b_unit(sides, first_tile * kTileN + row, (u - row * per_row) * 8);
+            }
+#pragma unroll
+            for (int i = 0; i < 6; ++i) {
+                const int u = base + 64 * i + lane;
+                if (u < units) *reinterpret_cast<u32x4 *>(dst + u * 16) = v[i];
+            }
+        }
+    } else {
+        copy_to_lds((unsigned)(size_t)(lds_ptr_t)dst, lo.b + (size_t)first_tile * kTileN * lo.r_total, units, lane);
+    }
+}
+
 // One word of LDS as a signal from the adapter wavefront to the wavefronts that add the low-rank
 // term: LDS serves its requests in order, so whoever reads the word set reads the operands that
 // were written before it.  The wait is bounded like every other wait here.
@@ -152,8 +180,18 @@ constexpr unsigned kGmpSyncBytes = 16;
 // kernel's parameter list.
 struct GmpLoraArgs {
     LoraTail lo;
+    GmpFold fold;
+};
+#if KILN_GMP_LORA == 2
+constexpr int kGmpSidesOffset = (int)(offsetof(GmpLoraArgs, fold) + offsetof(LoraSidesFold, sides));
+#else
+constexpr int kGmpSidesOffset = 0;
+#endif
+struct GmpLateArgs {  // what every wavefront needs of them
+    LoraTail lo;
     LoraFold fold;
 };
+static_assert(offsetof(GmpLateArgs, fold) == offsetof(GmpLoraArgs, fold), "a GmpFold begins with a LoraFold");
 struct GmpKernelArgs {
     const uint16_t *A;
     const u32x4 *B;
@@ -180,6 +218,21 @@ constexpr uint32_t gmp_layout_word(int slot_bytes, int producers, uint32_t bits)
     return (uint32_t)slot_bytes | (uint32_t)producers << 16 | bits;
 }
 constexpr int kGmpLoraArgsOffset = (int)offsetof(GmpKernelArgs, la);
+// An argument behind the preloaded ones, read where it is needed.
+template <class V>
+__device__ __forceinline__ V read_argument(int offset) {
+    typedef const char __attribute__((address_space(4))) *kernarg_ptr_t;
+    typedef const uint32_t __attribute__((address_space(4))) *kernarg_words_t;
+    kernarg_ptr_t kernarg = (kernarg_ptr_t)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(kernarg));  // opaque: nothing read through it moves above this point
+    kernarg_words_t src = (kernarg_words_t)(kernarg + offset);
+    struct Words {
+        uint32_t w[sizeof(V) / 4];
+    } words;
+#pragma unroll
+    for (int i = 0; i < (int)(sizeof(V) / 4); ++i) words.w[i] = src[i];
+    return __builtin_bit_cast(V, words);
+}
 static_assert(sizeof(GmpLoraArgs) % 4 == 0, "read word by word");
 
 // What only the end of the kernel needs -- where the result and the partial tiles go, how a tile is
@@ -381,20 +434,8 @@ __global__ __launch_bounds__(kGmpMaxWaves * 64) void w4a16_decode_gmp_kernel(
     // What the low-rank term needs is read from the kernel arguments only now: as ordinary
     // parameters these values would sit in scalar registers through the whole main loop, which
     // already uses nearly all of them.
-    GmpLoraArgs late_args{};
-    if (__builtin_expect(adapter != 0, 0)) {  // a call without adapters does not wait for these loads
-        typedef const char __attribute__((address_space(4))) *kernarg_ptr_t;
-        typedef const uint32_t __attribute__((address_space(4))) *kernarg_words_t;
-        kernarg_ptr_t kernarg = (kernarg_ptr_t)__builtin_amdgcn_kernarg_segment_ptr();
-        asm volatile("" : "+s"(kernarg));  // opaque: nothing read through it moves above this point
-        kernarg_words_t src = (kernarg_words_t)(kernarg + kGmpLoraArgsOffset);
-        struct Words {
-            uint32_t w[sizeof(GmpLoraArgs) / 4];
-        } words;
-#pragma unroll
-        for (int i = 0; i < (int)(sizeof(GmpLoraArgs) / 4); ++i) words.w[i] = src[i];
-        late_args = __builtin_bit_cast(GmpLoraArgs, words);
-    }
+    GmpLateArgs late_args{};
+    if (__builtin_expect(adapter != 0, 0)) late_args = read_argument<GmpLateArgs>(kGmpLoraArgsOffset);  // a call without adapters does not wait
     const LoraTail &lo = late_args.lo;
     const LoraFold &fold = late_args.fold;
     // The low-rank term y += T * B_cat^T is added where a finished tile is stored, by the slice that
@@ -433,8 +474,8 @@ __global__ __launch_bounds__(kGmpMaxWaves * 64) void w4a16_decode_gmp_kernel(
         // signals.
         if (adds_term) {
             const int live_tiles = min(T, NT - tf);
-            copy_to_lds((unsigned)(size_t)(lds_ptr_t)lora_b_lds, lo.b + (size_t)tf * kTileN * lo.r_total,
-                        live_tiles * kTileN * lo.r_total / 8, lane);
+            if constexpr (kGmpSides) fetch_b_rows(read_argument<LoraSides>(kGmpLoraArgsOffset + kGmpSidesOffset), lo, lora_b_lds, tf, live_tiles, lane);
+            else fetch_b_rows(fold, lo, lora_b_lds, tf, live_tiles, lane);
             if (fold.producers > 0) {
                 KILN_GMP_TL(3, KILN_GMP_NOW());
                 const int polls = lora_fold_wait(fold, tf / T, lane);
@@ -612,7 +653,7 @@ hipError_t launch_gmp_tga(const DecodeArgs &a, hipStream_t stream) {
     const int full_waves = a.GS - a.waves * (GPW - 1);
     const int slot = gmp_slot_bytes(GPW, T);
     const int col_blocks = (NT + T - 1) / T;
-    LoraFold fold{};
+    GmpFold fold{};
     if (a.lora_producers > 0) {
         fold.a_cat = (const uint16_t *)a.lora_a;
         fold.t = (uint16_t *)const_cast<void *>(a.lora_t);
@@ -622,8 +663,16 @@ hipError_t launch_gmp_tga(const DecodeArgs &a, hipStream_t stream) {
         fold.consumers = col_blocks;
         const int *e = a.lora_ends;
         const float *sc = a.lora_scales;
+#if KILN_GMP_LORA == 2
+        fold.sides = lora_sides(a.lora_sides);
+        for (int i = 0; i < kLoraSidesMaxAdapters; ++i) {
+            fold.ends[i] = e[i];
+            fold.scales[i] = sc[i];
+        }
+#else
         fold.e0 = e[0], fold.e1 = e[1], fold.e2 = e[2], fold.e3 = e[3];
         fold.s0 = sc[0], fold.s1 = sc[1], fold.s2 = sc[2], fold.s3 = sc[3];
+#endif
     }
     const dim3 grid = fold.producers > 0 ? dim3(fold.producers + col_blocks * a.KS, 1) : dim3(col_blocks, a.KS);
     const int adapter = a.r_total > 0 ? 1 : 0;  // one wavefront more: it fetches the low-rank term's operands
@@ -668,7 +717,12 @@ hipError_t launch_gmp_t(const DecodeArgs &a, int gpw, hipStream_t stream) {
 
 #if KILN_GMP_LORA
 // The instances with the low-rank term; the caller (launch_decode_gmp) has checked the plan.
+#if KILN_GMP_LORA == 2
+hipError_t launch_decode_gmp_sides(const DecodeArgs &a, hipStream_t stream) {
+    if (!a.lora_sides) return hipErrorInvalidValue;
+#else
 hipError_t launch_decode_gmp_lora(const DecodeArgs &a, hipStream_t stream) {
+#endif
     if (a.r_total <= 0) return hipErrorInvalidValue;  // these instances count on the adapter wavefront
     const int gpw = (a.GS + a.waves - 1) / a.waves;
     switch (a.gm_tiles) {
@@ -692,7 +746,8 @@ bool decode_gmp_ok(const DecodeArgs &a) {
         // main loop uses; T is whole and belongs to exactly this launch's rows (with the fused gate/up
         // store the rows of lora_b are in the packed column order, so nothing changes here)
         if (a.r_total > 64 || a.r_total % 8 != 0 || a.waves + 1 > kGmpMaxWaves) return false;
-        if (a.lora_slices < 1 || a.lora_slices > 16 || a.lora_rows != a.M || !a.lora_t || !a.lora_b) return false;
+        if (a.lora_slices < 1 || a.lora_slices > 16 || a.lora_rows != a.M || !a.lora_t || (!a.lora_b && !a.lora_sides)) return false;
+        if (a.lora_sides && a.lora_producers < 1) return false;
     }
     if (a.KS < 1 || a.KS > 255 || a.GS < 1 || a.KS * a.GS != G || a.waves < 1 || a.waves > kGmpMaxWaves || a.waves > a.GS) return false;
     const int gpw = (a.GS + a.waves - 1) / a.waves, T = a.gm_tiles;
@@ -705,12 +760,12 @@ bool decode_gmp_ok(const DecodeArgs &a) {
 // The projection folded into the launch: one producer block per K slice of it, each with at least
 // as many wavefronts as T has rank tiles and a KiB of LDS per wavefront for their meeting.
 bool decode_gmp_fold_ok(const DecodeArgs &a) {
-    if (a.r_total < 1 || a.r_total > 64 || !a.lora_a || !a.lora_t || !a.lora_flags) return false;
+    if (a.r_total < 1 || a.r_total > 64 || (!a.lora_a && !a.lora_sides) || !a.lora_t || !a.lora_flags) return false;
     const int jt = (a.r_total + 15) / 16;
     if (a.lora_producers < 1 || a.lora_producers > kLoraFoldMaxProducers || a.lora_producers != a.lora_slices) return false;
     if (a.lora_steps_per_slice < 1 || (long)a.lora_producers * a.lora_steps_per_slice * 32 < a.K) return false;
     if (a.waves < jt || (a.lora_steps_per_slice + a.waves / jt - 1) / (a.waves / jt) > kLoraFoldStepsPerWave ||
-        a.lora_rows != a.M || a.lora_adapters < 1 || a.lora_adapters > kLoraFoldMaxAdapters) return false;
+        a.lora_rows != a.M || a.lora_adapters < 1 || a.lora_adapters > (a.lora_sides ? kLoraSidesMaxAdapters : kLoraFoldMaxAdapters)) return false;
     if (a.KS > 4) return false;  // the kernel finds a block's slice in a one-row grid by three comparisons
     const int gpw = (a.GS + a.waves - 1) / a.waves;
     return gmp_slot_bytes(gpw, a.gm_tiles) >= 1024;
@@ -721,6 +776,7 @@ hipError_t launch_decode_gmp(const DecodeArgs &a, hipStream_t stream) {
     if (a.KS > 1 && (!a.partial || !a.counters)) return hipErrorInvalidValue;
     if (a.flagged && a.KS > kGmpFlaggedSlices) return hipErrorInvalidValue;
     if (a.lora_producers > 0 && !decode_gmp_fold_ok(a)) return hipErrorInvalidValue;
+    if (a.lora_sides) return launch_decode_gmp_sides(a, stream);
     if (a.r_total > 0) return launch_decode_gmp_lora(a, stream);
     const int gpw = (a.GS + a.waves - 1) / a.waves;
     switch (a.gm_tiles) {
@@ -738,8 +794,10 @@ hipError_t launch_decode_gmp(const DecodeArgs &a, hipStream_t stream) {
 }  // namespace kiln
 
 #ifdef KILN_GMP_TIMELINE
-#if KILN_GMP_LORA
+#if KILN_GMP_LORA == 1
 extern "C" int kiln_gmp_timeline_lora(long long *buf) {
+#elif KILN_GMP_LORA == 2
+extern "C" int kiln_gmp_timeline_sides(long long *buf) {
 #else
 extern "C" int kiln_gmp_timeline(long long *buf) {
 #endif
