@@ -257,10 +257,10 @@ kiln_marlin_status_t kiln_w4a16_stack_adapters(
  * rank a multiple of 8, both on 16 bytes -- whose columns are the GEMM's from first_row on (with `swiglu`: rows = n_out,
  * first_row 0 for gate and 8 for up).  Up to three sides in the order of their columns; columns of no side have no
  * low-rank term.  ranks, scales: every adapter of every side in that order, at most eight, sum(ranks) = the sides' ranks
- * together <= 64.  What kiln_w4a16_stack_adapters in front of the stacked entry point gives, without its launch (with up to four
- * adapters in every bit; more are projected in the launch's own order of sums here, by a launch in front there).
- * Taken where the launch reads them itself, up to 16 rows: kiln_w4a16_takes_adapter_sides (a pure query; 1: yes) -- elsewhere
- * KILN_W4A16_ERR_KERN_SHAPE, and the caller stacks them.
+ * together <= 64.  What kiln_w4a16_stack_adapters in front of the stacked entry point gives, without its launch (in every bit,
+ * but for more than four adapters at up to 16 rows: projected in the launch's own order of sums here, by a launch in front there).
+ * Taken where the launch reads them itself, on the kernels of up to 16 rows and of 17 to 128 or a few hundred:
+ * kiln_w4a16_takes_adapter_sides (a pure query; 1: yes) -- elsewhere KILN_W4A16_ERR_KERN_SHAPE, and the caller stacks them.
  */
 typedef struct {
     const void *lora_a, *lora_b;

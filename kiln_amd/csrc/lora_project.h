@@ -164,12 +164,14 @@ __device__ __forceinline__ void project_store(f32x4 (&acc)[IT], const float *sc_
 // kernel's launch instead of in front of it.  Both are then written through to memory: an ordinary
 // store is complete when this die's cache has it, which a reader on another die does not see
 // before the launch ends.  PLAIN: the row sums' form (store_row_sum); never with `done`.
-template <int RB, bool PLAIN = false>  // rows per block: 16 or 64
+// SIDES: adapters that are not stacked (LoraSides; a_cat is not read), or nothing.
+template <int RB, bool PLAIN = false, class SIDES = void>  // rows per block: 16 or 64
 __device__ __forceinline__ void lora_project_block(unsigned char *lds, const uint16_t *__restrict__ X,
                                                    const uint16_t *__restrict__ a_cat, uint16_t *__restrict__ T, int M,
                                                    int K, int r_total, int RP, int steps_per_slice, const LoraScales &ls,
                                                    float *partial, int *counters, u32x4 *aext, int row_tile, int slice,
-                                                   int KZ, unsigned *done, int done_copies = 1, int done_stride = 0) {
+                                                   int KZ, unsigned *done, int done_copies = 1, int done_stride = 0,
+                                                   const SIDES *sides = nullptr) {
     constexpr int XL = RB * 32 / 256;                // 128-bit loads per thread and piece: x ...
     constexpr int AL = kProjectMaxRank * 32 / 256;   // ... and a_cat (rows from r_total on are not read)
     constexpr int IT = RB / 16;                      // tiles of T per wavefront, at most
@@ -215,7 +217,10 @@ __device__ __forceinline__ void lora_project_block(unsigned char *lds, const uin
         for (int i = 0; i < AL; ++i) {
             const int row = pr + 8 * i;
             ar[b][i] = u32x4{0u, 0u, 0u, 0u};
-            if (active && k_ok && row < r_total) ar[b][i] = *reinterpret_cast<const u32x4 *>(a_cat + (size_t)row * K + col);
+            if (active && k_ok && row < r_total) {
+                if constexpr (std::is_void_v<SIDES>) ar[b][i] = *reinterpret_cast<const u32x4 *>(a_cat + (size_t)row * K + col);
+                else ar[b][i] = *reinterpret_cast<const u32x4 *>(side_a_row(*sides, row, K) + col);
+            }
         }
     };
 

@@ -93,7 +93,8 @@ __device__ __forceinline__ void lora_add_from_lds(f32x4 &v, const LoraTail &lo, 
 // eight of them.  Columns of no side have no term.  What it saves is launches, which bound these calls: stacking took one
 // of 3.4 us in front of every fused call, and q | k | v with two adapters each, six together, another of 5 us for the
 // projection, which the stacked form takes inside for four at most.  (A layer at 11 rows, two adapters of rank 8 on each
-// projection, 2560 / 9216 wide: 41.2 -> 33.1 us, four launches instead of seven.)
+// projection, 2560 / 9216 wide: 41.2 -> 33.1 us, four launches instead of seven.  On the mid-M kernel, six launches -> four:
+// at 20 / 50 / 100 rows 52.4 -> 46.7 / 63.0 -> 57.0 / 87.7 -> 82.0 us; 1536 / 5120 wide 47.3 -> 42.0 / 48.6 -> 44.0 / 58.7 -> 53.0.)
 struct LoraSides {
     const uint16_t *a[kMaxAdapterSides];
     const uint16_t *b[kMaxAdapterSides];

@@ -960,6 +960,38 @@ bool lora_in_launch(const GemmPlan &gp, int m, int k, int cus, const LoraSpec &l
     return decode_gmp_fold_ok(*f) && (blocks + kz <= cus || blocks > cus || g_tune.lora_fold == 2);
 }
 
+// The same of the mid-M kernel, on a launch's sizes and plan: the projection's blocks are the grid's first, so they run before
+// anything that waits for them, in one round or several (gate+up with two adapters at 96 rows 34.9 -> 32.0 us, down 23.7 ->
+// 20.5).
+bool mid_lora_in_launch(const GemmPlan &gp, const LoraSpec &lora, void *flags, MidArgs *a) {
+    const int steps = a->K / 32, row_tiles = ceil_div(a->M, 16);
+    int kz = lora_project_slices(a->M, a->K);
+    const int per_slice = ((steps + kz - 1) / kz + 3) / 4 * 4;  // whole 128-value groups
+    kz = (steps + per_slice - 1) / per_slice;
+    a->lora_slices = kz;
+    a->lora_producers = row_tiles * kz;
+    a->lora_steps_per_slice = per_slice;
+    a->lora_a = lora.a;
+    a->lora_sides = lora.sides;
+    a->lora_words = reinterpret_cast<unsigned *>(flags);
+    a->lora_adapters = lora.n_adapters;
+    // (what the launch itself checks: beyond four runs of rows, or more (slice, tile) words than a copy
+    // holds, the projection runs in front -- a call of 320 rows with adapters was refused here once)
+    return g_tune.lora_fold != 0 && gp.mp.fold && lora.n_adapters <= 8 && mid_lora_fold_ok(*a);
+}
+
+// Does a call read adapters that are not stacked where they lie (LoraSides)?  Where its launch projects x onto them, on the
+// private-staging and the mid-M kernel.
+bool sides_in_launch(const GemmPlan &gp, int m, int n, int k, int cus, const LoraSpec &lora, void *t, void *flags) {
+    if (gp.prefill) return false;
+    if (gp.mid) {
+        MidArgs ask = mid_args(gp.mp, m, n, k);
+        return mid_lora_in_launch(gp, lora, flags, &ask);
+    }
+    DecodeArgs ask{};
+    return lora_in_launch(gp, m, k, cus, lora, t, flags, &ask);
+}
+
 // The GEMM behind every entry point: small-M or matrix-core path by row count, with the
 // optional low-rank term.
 kiln_marlin_status_t gemm_any(const void *A, const void *B, void *C, const void *s, int prob_m, int prob_n,
@@ -985,10 +1017,7 @@ kiln_marlin_status_t gemm_any(const void *A, const void *B, void *C, const void 
     const WorkspaceLayout &wl = planned->wl;
     char *ws = reinterpret_cast<char *>(workspace);
     char *lora_t = ws + wl.lora_t;
-    if (lora && lora->sides) {  // (the entry point has asked: nothing else takes them)
-        DecodeArgs ask{};
-        if (!lora_in_launch(gp, prob_m, prob_k, cus, *lora, lora_t, ws, &ask)) return KILN_W4A16_ERR_KERN_SHAPE;
-    }
+    if (lora && lora->sides && !sides_in_launch(gp, prob_m, prob_n, prob_k, cus, *lora, lora_t, ws)) return KILN_W4A16_ERR_KERN_SHAPE;
     if (gp.prefill) {
         PrefillArgs pa{};
         pa.A = A;
@@ -1044,23 +1073,9 @@ kiln_marlin_status_t gemm_any(const void *A, const void *B, void *C, const void 
             ma.lora_t = lora_t;
             ma.lora_b = lora->b;
             ma.r_total = lora->r_total;
-            // ... inside the product's launch where its blocks have the threads for it: the projection's blocks
-            // are the grid's first, so they run before anything that waits for them, in one round or several
-            // (gate+up with two adapters at 96 rows 34.9 -> 32.0 us, down 23.7 -> 20.5)
-            const int steps = prob_k / 32, row_tiles = ceil_div(prob_m, 16);
-            int kz = lora_project_slices(prob_m, prob_k);
-            const int per_slice = ((steps + kz - 1) / kz + 3) / 4 * 4;  // whole 128-value groups
-            kz = (steps + per_slice - 1) / per_slice;
+            // ... inside the product's launch where its blocks have the threads for it
             MidArgs folded = ma;
-            folded.lora_slices = kz;
-            folded.lora_producers = row_tiles * kz;
-            folded.lora_steps_per_slice = per_slice;
-            folded.lora_a = lora->a;
-            folded.lora_words = reinterpret_cast<unsigned *>(ws + kFoldFlagOffset);
-            folded.lora_adapters = lora->n_adapters;
-            // (what the launch itself checks: beyond four runs of rows, or more (slice, tile) words than a copy
-            // holds, the projection runs in front -- a call of 320 rows with adapters was refused here once)
-            if (g_tune.lora_fold != 0 && gp.mp.fold && lora->n_adapters <= 8 && mid_lora_fold_ok(folded)) {
+            if (mid_lora_in_launch(gp, *lora, ws + kFoldFlagOffset, &folded)) {
                 int end = 0;
                 for (int i = 0; i < 8; ++i) {
                     if (i < lora->n_adapters) end += lora->ranks[i];
@@ -1473,15 +1488,14 @@ int kiln_w4a16_takes_adapter_sides(int prob_m, int prob_n, int prob_k, const kil
                                    int n_adapters, int dev) {
     AdapterSides own;
     int r_total = 0;
-    if (prob_m < 1 || prob_m > 16 || prob_n < 1 || prob_k < 1 || !shape_ok(prob_n, prob_k, 128) || n_adapters < 1 ||
+    if (prob_m < 1 || prob_n < 1 || prob_k < 1 || !shape_ok(prob_n, prob_k, 128) || n_adapters < 1 ||
         sides_of(sides, n_sides, prob_n, swiglu, &own, &r_total) != KILN_W4A16_OK)
         return 0;
     static const unsigned probe = 0;  // never dereferenced
-    DecodeArgs ask{};
     const int cus = compute_units(dev);
     const LoraSpec lora{nullptr, nullptr, r_total, n_adapters, nullptr, nullptr, &own};
-    return lora_in_launch(plan_call(prob_m, prob_n, prob_k, cus, -1, -1, 1)->gp, prob_m, prob_k, cus, lora, const_cast<unsigned *>(&probe),
-                          const_cast<unsigned *>(&probe), &ask) ? 1 : 0;
+    return sides_in_launch(plan_call(prob_m, prob_n, prob_k, cus, -1, -1, 1)->gp, prob_m, prob_n, prob_k, cus, lora,
+                           const_cast<unsigned *>(&probe), const_cast<unsigned *>(&probe)) ? 1 : 0;
 }
 
 kiln_marlin_status_t kiln_w4a16_gemm_adapter_sides(const void *A, const void *B, void *C, const void *s, int prob_m, int prob_n, int prob_k,

@@ -28,24 +28,27 @@
 // order; K slices of a tile meet in the workspace, last arriver adds in slice order.
 #include "async_loads.h"
 #include "launch.h"
-#include "lora_project.h"
 #include "lora_tail.h"
+#include "lora_project.h"
 
 namespace kiln {
 
 namespace {
 
-// This file is compiled twice: as it is for calls without adapters, and with -DKILN_MID_LORA=1 for calls
-// with them (launch_mid_lora only), so that what the low-rank term adds costs plain calls nothing.
+// This file is compiled three times: as it is for calls without adapters, with -DKILN_MID_LORA=1 for calls
+// with them (launch_mid_lora only), so that what the low-rank term adds costs plain calls nothing, and with
+// -DKILN_MID_LORA=2 for calls whose adapters are not stacked (launch_mid_sides only).
 #ifndef KILN_MID_LORA
 #define KILN_MID_LORA 0
 #endif
-constexpr bool kMidLora = KILN_MID_LORA != 0;
+constexpr bool kMidLora = KILN_MID_LORA != 0, kMidSides = KILN_MID_LORA == 2;
 
 // Probe builds only (-DKILN_MID_TIMELINE): wall-clock stamps (100 MHz) per wavefront.
 #ifdef KILN_MID_TIMELINE
-#if KILN_MID_LORA
+#if KILN_MID_LORA == 1
 #define g_mid_tl g_mid_tl_lora
+#elif KILN_MID_LORA == 2
+#define g_mid_tl g_mid_tl_sides
 #endif
 __device__ long long *g_mid_tl;
 #define KILN_MID_TL(i) tl_[i] = (long long)__builtin_amdgcn_s_memrealtime()
@@ -132,6 +135,11 @@ struct MidLora {
     int producers, row_tiles, steps_per_slice, consumers;
     LoraScales ls;
 };
+// ... of unstacked adapters, which a_cat and b do not describe; always with producers
+struct MidLoraSides : MidLora {
+    LoraSides sides;
+};
+using MidLow = std::conditional_t<kMidSides, MidLoraSides, MidLora>;
 constexpr int kMidFoldTileWord = 32;  // a copy's words start here (the first words are the small-M kernel's)
 constexpr int kMidFoldSpinLimit = 1 << 20;
 
@@ -160,7 +168,7 @@ constexpr uint32_t kMidColumnScales = 1u << 24, kMidColShift = 1u << 25, kMidSwi
 template <int TP, int GPW, bool LORA, int RBN>
 __device__ __forceinline__ void mid_block(
     const uint16_t *__restrict__ A_all, const u32x4 *__restrict__ B, const uint16_t *__restrict__ S,
-    uint16_t *__restrict__ C_all, float *partial_all, int *counters_all, const MidShape shape, const MidLora &lo) {
+    uint16_t *__restrict__ C_all, float *partial_all, int *counters_all, const MidShape shape, const MidLow &lo) {
     const int rows = shape.rows, G = shape.G, NT = shape.NT, N = NT * kTileN, K = G * kGroupK, KS = shape.KS(), nw = shape.waves();
     const bool swiglu = shape.is(kMidSwiglu), flagged = shape.is(kMidFlagged);
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
@@ -193,10 +201,16 @@ __device__ __forceinline__ void mid_block(
             int id = blockIdx.x;
             if (id < lo.producers) {
                 const int tile = id % lo.row_tiles, slice = id / lo.row_tiles;
+                unsigned *const words = lo.words + kMidFoldTileWord + slice * lo.row_tiles;
+#if KILN_MID_LORA == 2
+                lora_project_block<16, false, LoraSides>(lds, A_all, nullptr, const_cast<uint16_t *>(lo.t), rows, K, lo.r_total, lo.rp,
+                                                         lo.steps_per_slice, lo.ls, nullptr, nullptr, nullptr, tile, slice, lo.slices,
+                                                         words, kLoraFoldReplicas, kLoraFoldReplicaWords, &lo.sides);
+#else
                 lora_project_block<16>(lds, A_all, lo.a_cat, const_cast<uint16_t *>(lo.t), rows, K, lo.r_total, lo.rp,
                                        lo.steps_per_slice, lo.ls, nullptr, nullptr, nullptr, tile, slice, lo.slices,
-                                       lo.words + kMidFoldTileWord + slice * lo.row_tiles, kLoraFoldReplicas,
-                                       kLoraFoldReplicaWords);
+                                       words, kLoraFoldReplicas, kLoraFoldReplicaWords);
+#endif
                 return;
             }
             id -= lo.producers;
@@ -491,7 +505,7 @@ __device__ __forceinline__ void mid_block(
             const int JS = lo.rp >> 4;
             for (int c = wave; c < lo.slices * JS; c += nw) {
                 const int z = c / JS, j8 = (c - z * JS) * 16 + 8 * h;  // this lane's 8 rank columns
-                const bool live_rank = j8 + 8 <= lo.r_total;           // r_total % 8 == 0: all or none
+                [[maybe_unused]] const bool live_rank = j8 + 8 <= lo.r_total;           // r_total % 8 == 0: all or none
                 u32x4 ta[RBN], tb[TP];
 #pragma unroll
                 for (int rb = 0; rb < RBN; ++rb) {
@@ -501,8 +515,12 @@ __device__ __forceinline__ void mid_block(
 #pragma unroll
                 for (int p = 0; p < TP; ++p) {
                     const int col = min(tf + 2 * p, N / kTileN - 2) * kTileN + l32;
+#if KILN_MID_LORA == 2
+                    tb[p] = side_b_unit(lo.sides, col, j8);  // (zeros past the last side's rank)
+#else
                     tb[p] = u32x4{0u, 0u, 0u, 0u};
                     if (live_rank) tb[p] = *reinterpret_cast<const u32x4 *>(lo.b + (size_t)col * lo.r_total + j8);
+#endif
                 }
 #pragma unroll
                 for (int p = 0; p < TP; ++p)
@@ -701,7 +719,7 @@ template <int TP, int GPW, bool LORA, int ROW_BLOCKS>
 __global__ __launch_bounds__((kMidWavesOf<TP, ROW_BLOCKS, LORA> * 64)) void w4a16_mid_kernel(
     const uint16_t *__restrict__ A_all, const u32x4 *__restrict__ B, const uint16_t *__restrict__ S,
     int rows, int G, int NT, uint32_t slices, uint32_t layout, int col_blocks, uint16_t *__restrict__ C_all,
-    float *partial_all, int *counters_all, MidLora lo) {
+    float *partial_all, int *counters_all, MidLow lo) {
     const MidShape shape{rows, G, NT, slices, layout, col_blocks};
     if constexpr (ROW_BLOCKS != kMidRowBlocksByRun) {
         mid_block<TP, GPW, LORA, ROW_BLOCKS>(A_all, B, S, C_all, partial_all, counters_all, shape, lo);
@@ -730,7 +748,7 @@ hipError_t launch_mid_tgs(const MidArgs &a, hipStream_t stream) {
     const int runs = (a.M + kMidRows - 1) / kMidRows;
     const int last_groups = a.K / kGroupK - (a.KS - 1) * a.GS;  // of the last slice: GS, or fewer
     const int full_waves = a.GS - a.waves * (GPW - 1), last_full_waves = last_groups - a.waves * (GPW - 1);
-    MidLora lo{};
+    MidLow lo{};
     lo.t = (const uint16_t *)a.lora_t;
     lo.b = (const uint16_t *)a.lora_b;
     lo.r_total = a.r_total;
@@ -738,6 +756,9 @@ hipError_t launch_mid_tgs(const MidArgs &a, hipStream_t stream) {
     lo.slices = a.lora_slices;
     const int col_blocks = (NT + 2 * TP - 1) / (2 * TP);
     dim3 grid(col_blocks, a.KS, runs);
+#if KILN_MID_LORA == 2
+    lo.sides = lora_sides(a.lora_sides);
+#endif
     if (a.lora_producers > 0) {
         lo.a_cat = (const uint16_t *)a.lora_a;
         lo.words = a.lora_words;
@@ -786,8 +807,14 @@ hipError_t launch_mid_t(const MidArgs &a, int gpw, hipStream_t stream) {
 
 #if KILN_MID_LORA
 // The instances with the low-rank term; the caller (launch_mid) has checked the plan.
+#if KILN_MID_LORA == 2
+hipError_t launch_mid_sides(const MidArgs &a, hipStream_t stream) {
+    if (!a.lora_sides || a.lora_sides->count < 1 || a.lora_sides->count > kMaxAdapterSides || a.lora_producers < 1) return hipErrorInvalidValue;
+#else
 hipError_t launch_mid_lora(const MidArgs &a, hipStream_t stream) {
-    if (a.r_total < 8 || a.r_total > 64 || a.r_total % 8 != 0 || !a.lora_t || !a.lora_b || a.lora_slices < 1)
+    if (!a.lora_b) return hipErrorInvalidValue;
+#endif
+    if (a.r_total < 8 || a.r_total > 64 || a.r_total % 8 != 0 || !a.lora_t || a.lora_slices < 1)
         return hipErrorInvalidValue;
     if (a.lora_producers > 0 && !mid_lora_fold_ok(a)) return hipErrorInvalidValue;
     const int gpw = (a.GS + a.waves - 1) / a.waves;
@@ -806,7 +833,7 @@ bool mid_lora_fold_ok(const MidArgs &a) {
     const int row_tiles = (a.M + 15) / 16;
     return a.waves >= 4 && a.lora_slices >= 1 && a.lora_slices <= 16 &&
            row_tiles * a.lora_slices <= kLoraFoldReplicaWords - kMidFoldTileWord &&
-           a.lora_producers == row_tiles * a.lora_slices && a.lora_a && a.lora_words && a.lora_adapters >= 1 &&
+           a.lora_producers == row_tiles * a.lora_slices && (a.lora_a || a.lora_sides) && a.lora_words && a.lora_adapters >= 1 &&
            a.lora_adapters <= 8 && a.lora_steps_per_slice >= 4 && a.lora_steps_per_slice % 4 == 0 &&
            (long)a.lora_slices * a.lora_steps_per_slice * 32 >= a.K && a.M <= 4 * kMidRows;
 }
@@ -853,7 +880,7 @@ hipError_t launch_mid(const MidArgs &a, hipStream_t stream) {
     if (!mid_plan_ok(a)) return hipErrorInvalidValue;
     if (a.KS > 1 && (!a.partial || !a.counters)) return hipErrorInvalidValue;
     if (a.flagged && !mid_flagged_ok(a)) return hipErrorInvalidValue;
-    if (a.r_total > 0) return launch_mid_lora(a, stream);
+    if (a.r_total > 0) return a.lora_sides ? launch_mid_sides(a, stream) : launch_mid_lora(a, stream);
     const int gpw = (a.GS + a.waves - 1) / a.waves;
     switch (a.pairs) {
         case 1: return launch_mid_t<1>(a, gpw, stream);
@@ -866,7 +893,9 @@ hipError_t launch_mid(const MidArgs &a, hipStream_t stream) {
 }  // namespace kiln
 
 #ifdef KILN_MID_TIMELINE
-#if KILN_MID_LORA
+#if KILN_MID_LORA == 2
+extern "C" int kiln_mid_timeline_sides(long long *buf) {
+#elif KILN_MID_LORA
 extern "C" int kiln_mid_timeline_lora(long long *buf) {
 #else
 extern "C" int kiln_mid_timeline(long long *buf) {

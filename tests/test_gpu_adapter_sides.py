@@ -1,5 +1,5 @@
 """Calls whose projections keep adapters of their own, read where they lie by the launch: against the same call on the
-stacked set -- in every bit with up to four adapters, whose projection runs in the launch either way -- and against the
+stacked set -- in every bit where its projection runs in the launch too (up to four adapters, or more than 16 rows) -- and against the
 product in 64 bits.  Tiles that cross from one projection to the next, columns without adapters, one side alone, the
 widest stacked rank, K slices, replays of a captured call."""
 import ctypes
@@ -28,7 +28,7 @@ def _takes(m, n, k, sides, swiglu=0, n_adapters=2):
 
 def test_what_is_taken():
     qkv = _sides((16, 0, 8192), (16, 8192, 1024), (16, 9216, 1024))
-    assert [_takes(m, 10240, 2560, qkv, 0, 6) for m in (0, 1, 16, 17)] == [0, 1, 1, 0]
+    assert [_takes(m, 10240, 2560, qkv, 0, 6) for m in (0, 1, 16, 17, 128, 2048)] == [0, 1, 1, 1, 1, 0]
     assert _takes(4, 10240, 2560, qkv, 0, 8) == 1 and _takes(4, 10240, 2560, qkv, 0, 9) == 0
     assert _takes(4, 10240, 2560, _sides((16, 0, 8192), (12, 8192, 1024))) == 0           # not whole units of eight
     assert _takes(4, 10240, 2560, _sides((40, 0, 8192), (32, 8192, 1024))) == 0           # more than 64 together
@@ -54,7 +54,7 @@ def test_what_is_refused():
     assert call(m=-1) == call(n=1000) == call(k=500) == 1          # the problem's shape
     argument, shape = call(sides=None), call(count=4, sides=_sides(*[(8, 256 * i, 256) for i in range(4)]))
     assert argument == call(adapters=0) == call(ranks=(ctypes.c_int * 2)(16, 8)) == call(ranks=None) == call(count=0) != _lib.OK
-    assert shape == call(m=17) == call(sides=_sides((16, 0, 512), (12, 512, 512)), ranks=(ctypes.c_int * 2)(16, 12)) != _lib.OK
+    assert shape == call(m=2048) == call(sides=_sides((16, 0, 512), (12, 512, 512)), ranks=(ctypes.c_int * 2)(16, 12)) != _lib.OK
     assert argument != shape
     assert call(sides=(Side * 2)(Side(8, 16, 16, 0, 512), Side(16, 16, 16, 512, 512))) == argument  # off 16 bytes
 
@@ -73,7 +73,7 @@ def _packed(gen, k, n, g):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("m", [1, 4, 9, 16])
+@pytest.mark.parametrize("m", [1, 4, 9, 16, 17, 33, 64, 100])  # (from 17 on the mid-M kernel: one and two row blocks, two runs)
 @pytest.mark.parametrize("k,widths,ranks,g", [
     (2560, (8192, 1024, 1024), ((8, 8), (8, 8), (8, 8)), 128),      # six adapters; blocks of three tiles cross at 8192
     (2560, (8192, 1024, 1024), ((8, 8), None, (16,)), -1),
@@ -95,7 +95,7 @@ def test_side_by_side(m, k, widths, ranks, g):
     got = torch.cat(layer.forward_same_input(kinds, x, loras), dim=1)
     stacked = lora.fuse_column_blocks([loras[kind] for kind in kinds], widths)
     want = lora.proj_forward(x, fused, stacked)
-    if len(stacked.ranks) <= 4:
+    if len(stacked.ranks) <= 4 or m > 16:  # (there the stacked set is projected inside too)
         assert torch.equal(got.view(torch.int16), want.view(torch.int16))
     exact = x.double() @ marlin_gemm.dequant_f32(fused.b_packed, fused.scales, g).double()
     low, col = torch.zeros_like(exact), 0
@@ -109,7 +109,7 @@ def test_side_by_side(m, k, widths, ranks, g):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("m", [1, 5, 16])
+@pytest.mark.parametrize("m", [1, 5, 16, 24, 50, 128])
 @pytest.mark.parametrize("k,inter,ranks,g", [
     (2560, 9216, ((8, 8), (8, 8)), 128),
     (2560, 9216, (None, (16,)), 128),
