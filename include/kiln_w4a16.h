@@ -295,7 +295,7 @@ kiln_marlin_status_t kiln_w4a16_quantize_and_pack_device(
 
 /*
  * kiln_w4a16_quantize_and_pack_device for `count` weights of one device at once: one launch for the weights of a
- * groupsize, up to sixteen (two and one per weight with groupsize -1).  pair_b, pair_s: null, or the pack of gate and up interleaved
+ * groupsize, up to sixteen (three with groupsize -1).  pair_b, pair_s: null, or the pack of gate and up interleaved
  * (kiln_w4a16_interleave_gate_up, of n columns each), into which the weight goes as well -- pair_side 0: as gate, 1: as
  * up.  Nothing is launched if any item is refused.
  */
