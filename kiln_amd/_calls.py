@@ -1,5 +1,5 @@
 """The extension that calls the library without ctypes (`kiln_amd/lib/_torch_calls.so`, built from
-csrc/torch/torch_calls.cpp): `linear`, `linear_lora`, `linear_sides`, `mlp`, `quantize`.  Each takes the plain case -- contiguous CUDA
+csrc/torch/torch_calls.cpp): `linear`, `linear_lora`, `linear_sides`, `mlp`, `quantize`, `repack`.  Each takes the plain case -- contiguous CUDA
 tensors of the right types, a workspace that is already there -- and returns None for anything else, upon
 which the wrappers here take their checked route (same kernels, the reference's error texts).
 
@@ -19,7 +19,8 @@ EXTENSION_PATH = _lib.LIB_PATH.with_name("_torch_calls.so")
 # in the order bind() takes them
 _FUNCTIONS = ("kiln_marlin_w4a16_gemm", "kiln_w4a16_gemm_lora", "kiln_w4a16_gemm_swiglu", "kiln_w4a16_gemm_swiglu_lora",
               "kiln_w4a16_mlp", "kiln_w4a16_workspace_bytes", "kiln_w4a16_mlp_workspace_bytes", "kiln_w4a16_stack_adapters",
-              "kiln_w4a16_quantize_and_pack_many_device", "kiln_w4a16_takes_adapter_sides", "kiln_w4a16_gemm_adapter_sides")
+              "kiln_w4a16_quantize_and_pack_many_device", "kiln_w4a16_takes_adapter_sides", "kiln_w4a16_gemm_adapter_sides",
+              "kiln_w4a16_repack_gptq_device")
 
 
 _ext = None
@@ -75,5 +76,5 @@ def _stand_in(name: str):
     return first_call
 
 
-_NAMES = ("linear", "linear_lora", "linear_sides", "mlp", "quantize")
-linear, linear_lora, linear_sides, mlp, quantize = map(_stand_in, _NAMES)
+_NAMES = ("linear", "linear_lora", "linear_sides", "mlp", "quantize", "repack")
+linear, linear_lora, linear_sides, mlp, quantize, repack = map(_stand_in, _NAMES)

@@ -11,11 +11,13 @@
 // callers' choice between the shipped library and the tuning build holds here too.
 #include <Python.h>
 
+#include <algorithm>
 #include <array>
 #include <cstdint>
 #include <vector>
 
 #include <ATen/ATen.h>
+#include <ATen/core/LegacyTypeDispatch.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
@@ -38,6 +40,7 @@ struct Library {
     decltype(&kiln_w4a16_quantize_and_pack_many_device) quantize = nullptr;
     decltype(&kiln_w4a16_takes_adapter_sides) takes_sides = nullptr;
     decltype(&kiln_w4a16_gemm_adapter_sides) gemm_sides = nullptr;
+    decltype(&kiln_w4a16_repack_gptq_device) repack = nullptr;
 };
 Library g_lib;  // written by bind() under the interpreter lock, like everything below
 
@@ -534,6 +537,103 @@ PyObject *py_quantize(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     END_HANDLE_TH_ERRORS
 }
 
+// Contiguous host tensors one after the other, each from a multiple of 256 bytes on, into the byte tensor `dst` on the current
+// stream: through pinned memory, `stage_bytes` at a time, the first copy one of `first_piece` bytes.  The host tensors
+// may change once this returns, the copies may still be running (the pinned block is torch's to keep until they are done).
+void upload(std::initializer_list<at::Tensor> sources, const at::Tensor &dst, int64_t stage_bytes, int64_t first_piece,
+            const c10::hip::HIPStreamMasqueradingAsCUDA &stream) {
+    const at::Tensor stage = at::empty({std::min(stage_bytes, dst.numel())}, at::TensorOptions().dtype(at::kByte).pinned_memory(true));
+    int64_t base = 0, sent = 0, at_ = 0;  // stage holds dst[base:]; dst[:sent] is on its way; dst[:at_] is staged
+    auto send = [&]() {
+        dst.narrow(0, sent, at_ - sent).copy_(stage.narrow(0, sent - base, at_ - sent), true);
+        sent = at_;
+    };
+    for (const at::Tensor &src : sources) {
+        const at::Tensor flat = src.view({-1}).view(at::kByte);
+        int64_t done = 0;
+        at_ = (at_ + 255) / 256 * 256;
+        while (done < flat.numel()) {
+            if (at_ - base >= stage.numel()) {
+                send();
+                stream.synchronize();  // the copies still read the stage
+                base = at_;
+            }
+            const int64_t piece = std::min({sent == 0 ? first_piece : stage.numel(), flat.numel() - done, base + stage.numel() - at_});
+            stage.narrow(0, at_ - base, piece).copy_(flat.narrow(0, done, piece));
+            done += piece;
+            at_ += piece;
+            if (sent == 0 && dst.numel() > first_piece) send();  // (what is no longer than that goes in one)
+        }
+    }
+    send();
+}
+
+// repack(qweight, scales, qzeros or None, k, n, groupsize, device index, stage_bytes, first_piece): a GPTQ projection's contiguous
+// host tensors uploaded and rearranged on the device's current stream -> (words, scales) when that is done.  Driven from Python
+// the same steps left more of the host's time around the link's (0.5 / 3.1 / 11.3 MiB: 59 -> 49 / 120 -> 109 / 285 -> 270 us).
+PyObject *py_repack(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
+    HANDLE_TH_ERRORS
+    if (nargs != 9 || !g_lib.repack) Py_RETURN_NONE;
+    long long number[6];  // k, n, groupsize, device, stage_bytes, first_piece
+    for (int i = 0; i < 6; ++i) {
+        number[i] = PyLong_AsLongLong(args[3 + i]);
+        if (number[i] == -1 && PyErr_Occurred()) {
+            PyErr_Clear();
+            Py_RETURN_NONE;
+        }
+    }
+    const int64_t k = number[0], n = number[1], g = number[2];
+    if ((g != -1 && g != 128) || k <= 0 || n <= 0 || k % 128 != 0 || n % 256 != 0 || k > INT32_MAX || n > INT32_MAX ||
+        number[3] < 0 || number[3] > INT8_MAX || number[4] < 256 || number[4] % 256 != 0 || number[5] < 256 || number[5] % 256 != 0)
+        Py_RETURN_NONE;
+    const int64_t groups = g == -1 ? 1 : k / 128, q_bytes = k / 2 * n, s_bytes = groups * n * 2;  // (q_bytes is a multiple of 16 KiB)
+    const at::Tensor *host[3] = {};
+    const at::ScalarType types[3] = {at::kInt, at::kHalf, at::kInt};
+    const int64_t sizes[3] = {k / 8 * n, groups * n, groups * n / 8};
+    for (int i = 0; i < 3; ++i) {
+        if (i == 2 && args[i] == Py_None) break;
+        const at::Tensor *t = tensor_of(args[i]);
+        if (!t || !t->device().is_cpu() || t->scalar_type() != types[i] || t->layout() != at::kStrided || t->numel() != sizes[i] ||
+            !t->is_contiguous())
+            Py_RETURN_NONE;
+        host[i] = t;
+    }
+    const at::Tensor q = *host[0], s = *host[1], z = host[2] ? *host[2] : at::Tensor();
+    at::Tensor b, tiled;
+    bool done = false;
+    {
+        pybind11::gil_scoped_release no_gil;
+        at::AutoDispatchBelowADInplaceOrView no_autograd;
+        const c10::Device device(c10::DeviceType::CUDA, (c10::DeviceIndex)number[3]);
+        c10::hip::HIPGuardMasqueradingAsCUDA guard(device);
+        const auto stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(device.index());
+        const at::Tensor raw = at::detail::empty_cuda({q_bytes + s_bytes}, at::kByte, device, std::nullopt);
+        b = at::detail::empty_cuda({k / 16, 2 * n}, at::kInt, device, std::nullopt);
+        tiled = at::detail::empty_cuda({groups, n}, at::kHalf, device, std::nullopt);
+        upload({q, s}, raw, number[4], number[5], stream);
+        bool eights = true;
+        if (z.defined()) {  // looked at while the copies run
+            const uint32_t *word = reinterpret_cast<const uint32_t *>(z.data_ptr());
+            uint32_t other = 0;
+            for (int64_t i = 0; i < sizes[2]; ++i) other |= word[i] ^ 0x88888888u;
+            eights = other == 0;
+        }
+        if (eights) {
+            char *const at_ = static_cast<char *>(raw.data_ptr());
+            done = g_lib.repack(at_, at_ + q_bytes, nullptr, (int)k, (int)n, (int)g, b.data_ptr(), tiled.data_ptr(), (int)number[3],
+                                (void *)stream.stream()) == KILN_W4A16_OK;
+            stream.synchronize();
+        }
+    }
+    if (!done) Py_RETURN_NONE;
+    PyObject *pb = THPVariable_Wrap(std::move(b)), *ps = THPVariable_Wrap(std::move(tiled));
+    PyObject *pair = pb && ps ? PyTuple_Pack(2, pb, ps) : nullptr;
+    Py_XDECREF(pb);
+    Py_XDECREF(ps);
+    return pair;
+    END_HANDLE_TH_ERRORS
+}
+
 // set_workspaces(marlin_gemm's dictionary of them)
 PyObject *py_set_workspaces(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     if (nargs != 1 || !PyDict_CheckExact(args[0])) {
@@ -548,12 +648,12 @@ PyObject *py_set_workspaces(PyObject *, PyObject *const *args, Py_ssize_t nargs)
 
 // bind(addresses of the library's functions, in the order of Library)
 PyObject *py_bind(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
-    if (nargs != 11) {
-        PyErr_SetString(PyExc_TypeError, "bind takes eleven function addresses");
+    if (nargs != 12) {
+        PyErr_SetString(PyExc_TypeError, "bind takes twelve function addresses");
         return nullptr;
     }
-    void *p[11];
-    for (int i = 0; i < 11; ++i) p[i] = PyLong_AsVoidPtr(args[i]);
+    void *p[12];
+    for (int i = 0; i < 12; ++i) p[i] = PyLong_AsVoidPtr(args[i]);
     if (PyErr_Occurred()) return nullptr;
     g_lib.gemm = reinterpret_cast<decltype(g_lib.gemm)>(p[0]);
     g_lib.gemm_lora = reinterpret_cast<decltype(g_lib.gemm_lora)>(p[1]);
@@ -566,6 +666,7 @@ PyObject *py_bind(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     g_lib.quantize = reinterpret_cast<decltype(g_lib.quantize)>(p[8]);
     g_lib.takes_sides = reinterpret_cast<decltype(g_lib.takes_sides)>(p[9]);
     g_lib.gemm_sides = reinterpret_cast<decltype(g_lib.gemm_sides)>(p[10]);
+    g_lib.repack = reinterpret_cast<decltype(g_lib.repack)>(p[11]);
     Py_RETURN_NONE;
 }
 
@@ -584,7 +685,7 @@ PyObject *py_set_adapter_types(PyObject *, PyObject *const *args, Py_ssize_t nar
 
 #define FAST(name, fn) {name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(fn)), METH_FASTCALL, nullptr}
 PyMethodDef g_methods[] = {FAST("linear", py_linear), FAST("linear_lora", py_linear_lora), FAST("linear_sides", py_linear_sides),
-                           FAST("mlp", py_mlp), FAST("quantize", py_quantize), FAST("set_workspaces", py_set_workspaces), FAST("bind", py_bind),
+                           FAST("mlp", py_mlp), FAST("quantize", py_quantize), FAST("repack", py_repack), FAST("set_workspaces", py_set_workspaces), FAST("bind", py_bind),
                            FAST("set_adapter_types", py_set_adapter_types), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_torch_calls", nullptr, -1, g_methods, nullptr, nullptr, nullptr, nullptr};
 

@@ -166,11 +166,6 @@ def _host_pack() -> bool:
     return os.environ.get("KILN_W4A16_HOST_PACK", "").strip().lower() in ("1", "true", "yes")
 
 
-def _empty_packed(k: int, n: int, groupsize: int, device: torch.device) -> tuple[torch.Tensor, torch.Tensor]:
-    return (torch.empty((k // 16, 2 * n), dtype=torch.int32, device=device),
-            torch.empty((1 if groupsize == -1 else k // groupsize, n), dtype=torch.float16, device=device))
-
-
 def _wrap(b: torch.Tensor, s: torch.Tensor, k: int, n: int, groupsize: int) -> MarlinPackedProj:
     """A projection over packed tensors of this process's allocator."""
     return MarlinPackedProj(b, s, groupsize, k, n, _WrappingOwner(b, s, k, n, groupsize))
@@ -291,54 +286,15 @@ _STAGE_BYTES = 32 << 20
 _FIRST_PIECE_BYTES = 2 << 20
 
 
-def _upload(sources: Sequence[torch.Tensor], dst: torch.Tensor, device: torch.device) -> None:
-    """Copy contiguous host tensors one after the other, each from a multiple of 256 bytes on, into the uint8 tensor
-    `dst` on the current stream; the host tensors may change once this returns, the copies may still be running."""
-    stage = torch.empty(min(_STAGE_BYTES, dst.numel()), dtype=torch.uint8, pin_memory=True)
-    base = sent = at = 0       # stage holds dst[base:]; dst[:sent] is on its way; dst[:at] is staged
-
-    def send():
-        nonlocal sent
-        dst[sent:at].copy_(stage[sent - base:at - base], non_blocking=True)
-        sent = at
-
-    for src in sources:
-        flat, done, at = src.view(-1).view(torch.uint8), 0, -(-at // 256) * 256
-        while done < flat.numel():
-            if at - base >= stage.numel():
-                send()
-                torch.cuda.current_stream(device).synchronize()   # the copies still read the stage
-                base = at
-            piece = min(_FIRST_PIECE_BYTES if sent == 0 else stage.numel(), flat.numel() - done, base + stage.numel() - at)
-            stage[at - base:at - base + piece].copy_(flat[done:done + piece])
-            done, at = done + piece, at + piece
-            if sent == 0:
-                send()
-    send()
-
-
 def _repack_on_device(qweight: torch.Tensor, scales: torch.Tensor, qzeros: Optional[torch.Tensor], k: int, n: int,
                       groupsize: int, device: torch.device) -> Optional[MarlinPackedProj]:
     """`pack_from_gptq` for contiguous host tensors of the checkpoint's types: uploaded through pinned memory and
     rearranged on the device.  None where the library's route has the checks (or the error) to make."""
     if _host_pack() or device.type != "cuda" or groupsize not in (-1, 128) or k == 0 or n == 0 or k % 128 != 0 or n % 256 != 0:
         return None
-    groups = 1 if groupsize == -1 else k // groupsize
-    for t, dtype, size in ((qweight, torch.int32, k // 8 * n), (scales, torch.float16, groups * n), (qzeros, torch.int32, groups * n // 8)):
-        if t is not None and (t.is_cuda or t.dtype != dtype or t.numel() != size or not t.is_contiguous()):
-            return None
-    with torch.cuda.device(device):
-        device = torch.device("cuda", torch.cuda.current_device())
-        q_bytes, s_bytes = k // 2 * n, groups * n * 2     # (q_bytes is a multiple of 16 KiB)
-        raw = torch.empty(q_bytes + s_bytes, dtype=torch.uint8, device=device)
-        b_packed, s_tiled = _empty_packed(k, n, groupsize, device)
-        _upload((qweight, scales), raw, device)
-        if qzeros is not None and not (qzeros.numpy() == -0x77777778).all():   # 0x88888888, looked at while the copies run
-            return None
-        st = _lib.load().kiln_w4a16_repack_gptq_device(raw.data_ptr(), raw.data_ptr() + q_bytes, None, k, n, groupsize, b_packed.data_ptr(),
-                                                       s_tiled.data_ptr(), device.index, torch.cuda.current_stream(device).cuda_stream)
-        torch.cuda.current_stream(device).synchronize()
-    return _wrap(b_packed, s_tiled, k, n, groupsize) if st == 0 else None
+    made = _calls.repack(qweight, scales, qzeros, k, n, groupsize, torch.cuda.current_device() if device.index is None else device.index,
+                         _STAGE_BYTES, _FIRST_PIECE_BYTES)
+    return None if made is None else _wrap(*made, k, n, groupsize)
 
 
 def matmul_bf16(x: torch.Tensor, w: MarlinPackedProj) -> torch.Tensor:
