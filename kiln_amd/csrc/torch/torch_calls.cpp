@@ -570,7 +570,10 @@ void upload(std::initializer_list<at::Tensor> sources, const at::Tensor &dst, in
 
 // repack(qweight, scales, qzeros or None, k, n, groupsize, device index, stage_bytes, first_piece): a GPTQ projection's contiguous
 // host tensors uploaded and rearranged on the device's current stream -> (words, scales) when that is done.  Driven from Python
-// the same steps left more of the host's time around the link's (0.5 / 3.1 / 11.3 MiB: 59 -> 49 / 120 -> 109 / 285 -> 270 us).
+// the same steps left more of the host's time around the link's (0.5 / 3.1 / 11.3 MiB: 60 -> 47 / 122 -> 108 / 281 -> 271 us).
+// Subclasses are taken too, since loaders keep these tensors as a Parameter of their own: qweight and scales are read
+// through views and copies only, which a subclass that runs its own operations answers as well; zero-points are read where
+// they lie, and one of those has nothing there.
 PyObject *py_repack(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     HANDLE_TH_ERRORS
     if (nargs != 9 || !g_lib.repack) Py_RETURN_NONE;
@@ -592,8 +595,8 @@ PyObject *py_repack(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     const int64_t sizes[3] = {k / 8 * n, groups * n, groups * n / 8};
     for (int i = 0; i < 3; ++i) {
         if (i == 2 && args[i] == Py_None) break;
-        const at::Tensor *t = tensor_of(args[i]);
-        if (!t || !t->device().is_cpu() || t->scalar_type() != types[i] || t->layout() != at::kStrided || t->numel() != sizes[i] ||
+        const at::Tensor *t = THPVariable_Check(args[i]) ? &THPVariable_Unpack(args[i]) : nullptr;
+        if (!t || (i == 2 && t->unsafeGetTensorImpl()->is_python_dispatch()) || !t->device().is_cpu() || t->scalar_type() != types[i] || t->layout() != at::kStrided || t->numel() != sizes[i] ||
             !t->is_contiguous())
             Py_RETURN_NONE;
         host[i] = t;
