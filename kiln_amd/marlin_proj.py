@@ -292,6 +292,7 @@ def _repack_on_device(qweight: torch.Tensor, scales: torch.Tensor, qzeros: Optio
     rearranged on the device.  None where the library's route has the checks (or the error) to make."""
     if _host_pack() or device.type != "cuda" or groupsize not in (-1, 128) or k == 0 or n == 0 or k % 128 != 0 or n % 256 != 0:
         return None
+    torch.cuda.init()    # torch's own first use of the device: it refuses a forked child, which the extension's calls do not
     made = _calls.repack(qweight, scales, qzeros, k, n, groupsize, torch.cuda.current_device() if device.index is None else device.index,
                          _STAGE_BYTES, _FIRST_PIECE_BYTES)
     return None if made is None else _wrap(*made, k, n, groupsize)

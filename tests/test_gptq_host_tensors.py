@@ -86,3 +86,11 @@ def test_same_packs_from_every_form(form, stage, monkeypatch):
     b, tiled = pack.repack_gptq(q.numpy(), s.numpy(), None, G)
     assert np.array_equal(p.b_packed.cpu().numpy(), b) and np.array_equal(p.scales.cpu().numpy().view(np.uint16), tiled.view(np.uint16))
     assert type(p.b_packed) is type(p.scales) is torch.Tensor and not p.scales.requires_grad
+
+
+def test_a_forked_childs_call_is_refused(monkeypatch):
+    """torch refuses a child that was forked after the parent used the GPU; the device given with its index or without."""
+    monkeypatch.setattr(torch.cuda, "_is_in_bad_fork", lambda: True)
+    for device in ("cuda", "cuda:0"):
+        with pytest.raises(RuntimeError, match="forked subprocess"):
+            marlin_proj.pack_from_gptq(*_tensors(), G, device)
