@@ -263,7 +263,7 @@ def pack_from_gptq(qweight: torch.Tensor, scales: torch.Tensor, qzeros: Optional
     if here is not None:
         return here
     q = np.ascontiguousarray(qweight.cpu().numpy().view(np.int32))
-    s = np.ascontiguousarray(scales.cpu().numpy().view(np.uint16))
+    s = np.ascontiguousarray(scales.detach().cpu().numpy().view(np.uint16))
     z = None if qzeros is None else np.ascontiguousarray(qzeros.cpu().numpy().view(np.int32))
     out = ctypes.c_void_p()
     dev = -1 if device.type != "cuda" else (device.index if device.index is not None else torch.cuda.current_device())

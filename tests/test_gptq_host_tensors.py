@@ -94,3 +94,12 @@ def test_a_forked_childs_call_is_refused(monkeypatch):
     for device in ("cuda", "cuda:0"):
         with pytest.raises(RuntimeError, match="forked subprocess"):
             marlin_proj.pack_from_gptq(*_tensors(), G, device)
+
+
+def test_scales_with_a_gradient_on_the_host_route():
+    """A shape the library has no pack for yields None, whatever form its tensors come in."""
+    q = torch.zeros(4, 100, dtype=torch.int32)
+    for as_form in FORMS.values():
+        s = as_form(torch.ones(1, 100).half())
+        assert marlin_proj.pack_from_gptq(as_form(q), s, None, -1, "cpu") is None
+        assert marlin_proj.pack_from_gptq(as_form(q), s, None, -1, "cuda:0") is None
