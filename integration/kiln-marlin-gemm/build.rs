@@ -6,7 +6,7 @@
 // skipping the kernel.
 //
 // What is compiled is not spelled out here: csrc/objects.list names every object of the library as
-// `object:source[:extra flag]` (some kernel files are compiled twice, the second time with a define
+// `object:source[:extra flag]` (some kernel files are compiled again with a define
 // that adds the low-rank term), and the Makefile that builds the shared library for the C and
 // Python harnesses reads the same file, so the two builds cannot drift apart.
 use std::{env, fs, path::PathBuf, process::Command};

@@ -95,6 +95,9 @@ __device__ __forceinline__ void lora_add_from_lds(f32x4 &v, const LoraTail &lo, 
 // projection, which the stacked form takes inside for four at most.  (A layer at 11 rows, two adapters of rank 8 on each
 // projection, 2560 / 9216 wide: 41.2 -> 33.1 us, four launches instead of seven.  On the mid-M kernel, six launches -> four:
 // at 20 / 50 / 100 rows 52.4 -> 46.7 / 63.0 -> 57.0 / 87.7 -> 82.0 us; 1536 / 5120 wide 47.3 -> 42.0 / 48.6 -> 44.0 / 58.7 -> 53.0.)
+// Not all of what goes is won: the gate | up launch alone takes 10.6 us at 11 rows where it took 9.2 behind the launch that
+// stacked (3.4).  Why is not known: that launch had just read A and B, which left them in the caches, and the row of A is
+// found here through a choice per lane.
 struct LoraSides {
     const uint16_t *a[kMaxAdapterSides];
     const uint16_t *b[kMaxAdapterSides];

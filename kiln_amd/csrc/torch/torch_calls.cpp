@@ -298,10 +298,11 @@ bool add_side(PyObject *o, double scale, const Problem &p, int first, int rows, 
 
 // linear_sides(x, b_packed, scales, groupsize, swiglu, sides, widths, lora_scale, split): a GEMM whose columns belong
 // to several projections -- side by side, `widths` columns each, or with `swiglu` gate and up interleaved
-// (widths = n_out twice) -- each with its adapters or None.  Several sides, and stacked ranks that are not
-// multiples of 8, are read where they lie if the launch can, else they become one stacked set in a launch of their own in
-// front.  `split`: the result comes as
-// one view per projection.
+// (widths = n_out twice) -- each with its adapters or None.  One projection over all columns with a stacked rank that is a
+// multiple of 8 is what the entry points with adapters take as it is.  Else the launch reads every projection's own where
+// they lie -- one to three of them, each one's rank a multiple of 8, on the kernels that
+// kiln_w4a16_takes_adapter_sides names -- and all others become one stacked set in a launch of their own in front.
+// `split`: the result comes as one view per projection.
 PyObject *py_linear_sides(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     HANDLE_TH_ERRORS
     Problem p;

@@ -859,7 +859,7 @@ struct LoraSpec {
     int r_total, n_adapters;
     const int *ranks;    // host arrays of length n_adapters
     const float *scales;
-    const AdapterSides *sides = nullptr;  // in place of a and b, which are null: calls that lora_in_launch() takes
+    const AdapterSides *sides = nullptr;  // in place of a and b, which are null: calls that sides_in_launch() takes
 };
 
 // Bytes a call of m rows needs, made monotone in m: the largest need of any m' <= m.  The plan

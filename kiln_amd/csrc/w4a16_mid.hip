@@ -37,7 +37,8 @@ namespace {
 
 // This file is compiled three times: as it is for calls without adapters, with -DKILN_MID_LORA=1 for calls
 // with them (launch_mid_lora only), so that what the low-rank term adds costs plain calls nothing, and with
-// -DKILN_MID_LORA=2 for calls whose adapters are not stacked (launch_mid_sides only).
+// -DKILN_MID_LORA=2 for calls whose adapters are not stacked (launch_mid_sides only; apart as on the small-M kernel, where
+// one form for both was measured slower: here that was not measured, and the two take the same registers to within three).
 #ifndef KILN_MID_LORA
 #define KILN_MID_LORA 0
 #endif
@@ -344,7 +345,8 @@ __device__ __forceinline__ void mid_block(
             // With adapters and three pairs the second row block's chain begins when the first's has ended, and the ones are
             // formed for it: those instances have 256 registers and not one to spare (both at once: 20 spilled, and with
             // loads in flight to registers the compiler takes as written, a spill could save a stale one; 2560 -> 18432 with
-            // adapters at 64 / 128 rows 18.9 -> 18.1 / 33.3 -> 32.0 us).  A chain's order of additions is the same either way.
+            // adapters at 64 / 128 rows 18.9 -> 18.1 / 33.3 -> 32.0 us).  A chain's order of additions is the same either way
+            // among the passes of two row blocks.
             constexpr bool kOneByOne = LORA && TP == 3 && RBN == 2;
             constexpr int kChains = kOneByOne ? 1 : RBN;
 #pragma unroll
@@ -358,7 +360,9 @@ __device__ __forceinline__ void mid_block(
                 // One row block: two chains, of a fragment's halves -- such a product needs the one before it two wait states
                 // earlier, and with the other row block's chain gone nothing stood in them (2560 -> 8192 at 20 rows 6.60 -> 6.37
                 // us, 2560 -> 18432 at 32 10.11 -> 9.87, 9216 -> 2560 at 20 7.85 -> 7.73; 30 shapes at 17 ... 32 rows 0.9 % faster on
-                // average, 4 % at best, 0.6 % slower at worst).
+                // average, 4 % at best, 0.6 % slower at worst).  The halves are added behind the last product, so a group's
+                // sum can round otherwise than in a pass of two row blocks: a row's result depends on whether its run has
+                // more than 32 rows (error against 64 bits over five shapes level or 0.2 % less than with one chain).
                 constexpr bool kHalves = RBN == 1;
                 f32x4 sums[kChains];
                 [[maybe_unused]] f32x4 second = {0.f, 0.f, 0.f, 0.f};
@@ -380,7 +384,7 @@ __device__ __forceinline__ void mid_block(
                     const float own = kHalves ? sums[i][0] + second[0] : sums[i][0];
                     float sum = own + __shfl_xor(own, 32, 64);
                     // (the sum and not c is held here: c's product meets its split in one multiply-add in every instance, so
-                    // that they agree in every bit)
+                    // that those of one number of row blocks agree in every bit)
                     if constexpr (kOneByOne) asm volatile("" : "+v"(sum));
                     c_of[gi][rb0 + i] = -kCodeBias * sum;
                 }

@@ -106,9 +106,9 @@ class LayerProjections:
                            lora_scale: float = 1.0) -> Tuple[torch.Tensor, ...]:
         """The projections `kinds` of one input: one launch on their side-by-side pack where `pack_layers`
         built it (the results are column ranges of one output tensor), else one `forward` each.  `loras`
-        maps a kind to its adapter(s); on the fused pack they become one stacked set whose projection of x
-        is computed once for all members (stacked rank <= 64 and <= 8 adapters, else the members run
-        one by one)."""
+        maps a kind to its adapter(s); on the fused pack x is projected onto those of all members at once, read
+        where they lie or stacked in front of the launch (stacked rank <= 64 and <= 8 adapters, else the members
+        run one by one)."""
         kinds = tuple(kinds)
         loras = loras or {}
         fused = self.same_input_fused.get(kinds)
