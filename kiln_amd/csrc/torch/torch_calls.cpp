@@ -574,7 +574,7 @@ void upload(std::initializer_list<at::Tensor> sources, const at::Tensor &dst, in
 // the same steps left more of the host's time around the link's (0.5 / 3.1 / 11.3 MiB: 60 -> 47 / 122 -> 108 / 281 -> 271 us).
 // Subclasses are taken too, since loaders keep these tensors as a Parameter of their own: qweight and scales are read
 // through views and copies only, which a subclass that runs its own operations answers as well; zero-points are read where
-// they lie, and one of those has nothing there.
+// they lie, and one of those, or a tensor without memory, has nothing there.
 PyObject *py_repack(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     HANDLE_TH_ERRORS
     if (nargs != 9 || !g_lib.repack) Py_RETURN_NONE;
@@ -597,7 +597,10 @@ PyObject *py_repack(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     for (int i = 0; i < 3; ++i) {
         if (i == 2 && args[i] == Py_None) break;
         const at::Tensor *t = THPVariable_Check(args[i]) ? &THPVariable_Unpack(args[i]) : nullptr;
-        if (!t || (i == 2 && t->unsafeGetTensorImpl()->is_python_dispatch()) || !t->device().is_cpu() || t->scalar_type() != types[i] || t->layout() != at::kStrided || t->numel() != sizes[i] ||
+        const bool read_in_place = i == 2;
+        if (!t || (read_in_place && (t->unsafeGetTensorImpl()->is_python_dispatch() || !t->has_storage() || !t->storage().data() ||
+                                     t->is_neg())) ||
+            !t->device().is_cpu() || t->scalar_type() != types[i] || t->layout() != at::kStrided || t->numel() != sizes[i] ||
             !t->is_contiguous())
             Py_RETURN_NONE;
         host[i] = t;

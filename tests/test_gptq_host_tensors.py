@@ -72,6 +72,10 @@ def test_what_takes_the_devices_route(form):
 def test_zero_points_that_cannot_be_read_in_place_are_the_host_routes():
     q, s, z = _tensors()
     assert _takes(Wrapped(q), Wrapped(s), z) and not _takes(q, s, Wrapped(z))
+    # zeros that have no memory, words that stand for their negatives, memory that was given back
+    assert not _takes(q, s, torch._efficientzerotensor(z.shape, dtype=torch.int32)) and not _takes(q, s, torch._neg_view(z))
+    z.untyped_storage().resize_(0)
+    assert not _takes(q, s, z)
 
 
 @pytest.mark.gpu
