@@ -252,6 +252,13 @@ kiln_marlin_status_t kiln_w4a16_stack_adapters(
     void *a_cat, void *b_cat, void *stream);
 
 /*
+ * Do the entry points with adapters take a stacked rank as it is at its best (1), or is it worth rounding up to a multiple
+ * of 8 with zeros in front (0: kiln_w4a16_stack_adapters)?  Multiples of 8 always; on some shapes of up to 16 rows multiples
+ * of 4.  A pure query; every rank up to 64 is taken either way.
+ */
+int kiln_w4a16_takes_rank(int prob_m, int prob_n, int prob_k, int r_total, int dev);
+
+/*
  * kiln_w4a16_gemm_lora, or with `swiglu` kiln_w4a16_gemm_swiglu_lora (prob_n: the packed columns, 2 * n_out), for adapters
  * that are not stacked: side i is a projection's adapters as they lie -- lora_a bf16 [rank, k], lora_b bf16 [rows, rank],
  * rank a multiple of 8, both on 16 bytes -- whose columns are the GEMM's from first_row on (with `swiglu`: rows = n_out,

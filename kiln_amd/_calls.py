@@ -20,7 +20,7 @@ EXTENSION_PATH = _lib.LIB_PATH.with_name("_torch_calls.so")
 _FUNCTIONS = ("kiln_marlin_w4a16_gemm", "kiln_w4a16_gemm_lora", "kiln_w4a16_gemm_swiglu", "kiln_w4a16_gemm_swiglu_lora",
               "kiln_w4a16_mlp", "kiln_w4a16_workspace_bytes", "kiln_w4a16_mlp_workspace_bytes", "kiln_w4a16_stack_adapters",
               "kiln_w4a16_quantize_and_pack_many_device", "kiln_w4a16_takes_adapter_sides", "kiln_w4a16_gemm_adapter_sides",
-              "kiln_w4a16_repack_gptq_device")
+              "kiln_w4a16_repack_gptq_device", "kiln_w4a16_takes_rank")
 
 
 _ext = None

@@ -27,6 +27,7 @@ EXPORTS = (
     "kiln_w4a16_mlp",
     "kiln_w4a16_mlp_workspace_bytes",
     "kiln_w4a16_stack_adapters",
+    "kiln_w4a16_takes_rank",
     "kiln_w4a16_takes_adapter_sides",
     "kiln_w4a16_gemm_adapter_sides",
     "kiln_w4a16_quantize_and_pack_device",
@@ -204,6 +205,8 @@ def _load(tuning: bool) -> ctypes.CDLL:
     L.kiln_w4a16_mlp.argtypes = [vp, vp, vp, vp, vp, vp, i, i, i, i, vp, i, i, vp]
     L.kiln_w4a16_mlp_workspace_bytes.restype = c.c_size_t
     L.kiln_w4a16_mlp_workspace_bytes.argtypes = [i, i, i, i]
+    L.kiln_w4a16_takes_rank.restype = i
+    L.kiln_w4a16_takes_rank.argtypes = [i, i, i, i, i]
     L.kiln_w4a16_takes_adapter_sides.restype = i
     L.kiln_w4a16_takes_adapter_sides.argtypes = [i, i, i, vp, i, i, i, i]
     L.kiln_w4a16_gemm_adapter_sides.restype = i

@@ -39,6 +39,15 @@ __device__ __forceinline__ void load_to_lds_b128(const void *base, uint32_t lane
                  : "memory", "m0");
 }
 
+// ... by no lane unless `at` < `end`: nothing is read then, and the wait counter moves as if it had been.
+__device__ __forceinline__ void load_to_lds_b128_if(int at, int end, const void *gptr, unsigned lds_addr) {
+    asm volatile("s_cmp_lt_i32 %2, %3\n\ts_cselect_b64 exec, -1, 0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\t"
+                 "global_load_lds_dwordx4 %0, off\n\ts_mov_b64 exec, -1"
+                 :
+                 : "v"(gptr), "s"(lds_addr), "n"(at), "s"(end)
+                 : "memory", "m0", "scc");
+}
+
 // ... and 4 bytes per lane, at lds_addr + 4 * lane.
 __device__ __forceinline__ void load_to_lds_b32(const void *base, uint32_t lane_off, unsigned lds_addr) {
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
@@ -73,6 +82,9 @@ __device__ __forceinline__ void load_b128_streaming(u32x4 &dst, const void *base
 __device__ __forceinline__ void load_u16(uint32_t &dst, const void *base, uint32_t lane_off) {
     asm volatile("global_load_ushort %0, %1, %2" : "=&v"(dst) : "v"(lane_off), "s"(base) : "memory");
 }
+__device__ __forceinline__ void load_b64(u32x2 &dst, const void *ptr) {
+    asm volatile("global_load_dwordx2 %0, %1, off" : "=&v"(dst) : "v"(ptr) : "memory");
+}
 
 // Device-scope (coherent across the dies) 128-bit accesses: one instruction where four 32-bit
 // atomic accesses would be four.  The load is a request like the ones above: wait, then pin.
@@ -88,6 +100,7 @@ __device__ __forceinline__ void load_b128_device_scope(u32x4 &dst, const void *p
 
 // Orders every later use of v after this point (and hence after the preceding wait).
 __device__ __forceinline__ void pin_loaded(u32x4 &v) { asm volatile("" : "+v"(v)); }
+__device__ __forceinline__ void pin_loaded(u32x2 &v) { asm volatile("" : "+v"(v)); }
 __device__ __forceinline__ void pin_loaded(uint32_t &v) { asm volatile("" : "+v"(v)); }
 
 // Waits as inline asm with a memory clobber: unlike the s_waitcnt builtin, the compiler keeps

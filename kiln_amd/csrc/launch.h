@@ -86,7 +86,9 @@ struct DecodeArgs {
     int lora_adapters = 0;         // 1...8
     int lora_ends[8] = {};         // exclusive end column of adapter i (r_total past the last adapter)
     float lora_scales[8] = {};     // its scale (0 past the last)
-    const AdapterSides *lora_sides = nullptr;  // with lora_producers: the adapters where they lie, lora_a and lora_b are not read
+    const AdapterSides *lora_sides = nullptr;  // with lora_producers or own_tiles: the adapters where they lie, lora_a and lora_b are not read
+    int own_tiles = 0;             // 1, 2: every block projects x onto the (up to 16, 32) rank columns of its own columns by
+                                   // itself; lora_t and the fields behind it but ends, scales and sides are not used
     bool swiglu = false;  // columns are gate/up interleaved by 8 inside every tile; C is [M, N/2] = silu(gate) * up
     int group_major = -1; // tuning: 0 never a group-major instance, 1 only the LDS-staged one, 2 the
                           // register-fragment one wherever a plan fits it; -1: automatic
@@ -121,6 +123,8 @@ bool decode_gmp_ok(const DecodeArgs &a);                        // does the plan
 bool decode_gmp_fold_ok(const DecodeArgs &a);                   // ... with the LoRA projection folded into the launch?
 hipError_t launch_decode_gmp(const DecodeArgs &a, hipStream_t stream);
 hipError_t launch_decode_gmp_sides(const DecodeArgs &a, hipStream_t stream);  // ... with that of unstacked adapters (checked plan)
+hipError_t launch_decode_gmp_own1(const DecodeArgs &a, hipStream_t stream);   // ... with a projection of each block's own (checked plan)
+hipError_t launch_decode_gmp_own2(const DecodeArgs &a, hipStream_t stream);
 hipError_t launch_decode_gmp_lora(const DecodeArgs &a, hipStream_t stream);  // its instances with the low-rank term (checked plan)
 
 // One launch of the mid-M kernel: runs of up to 64 rows (grid z) against the whole weight.

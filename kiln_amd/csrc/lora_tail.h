@@ -179,8 +179,67 @@ struct LoraSidesFold : LoraFold {
     int ends[8];             // read with constant indices only
     float scales[8];
 };
-constexpr int kLoraFoldMaxProducers = 16;
 constexpr int kLoraFoldMaxAdapters = 4;
+// The adapters of a call whose blocks project x onto them by themselves (own_tiles): the sides of LoraSides, one for a
+// stacked set, prepared so that a row or a unit is found without a branch.  A side that is absent has no columns.
+// (Plain members, not arrays: what is picked from an array by a condition goes through scratch memory.)
+static_assert(kMaxAdapterSides == 3, "three members of each kind below");
+struct OwnSidesA {
+    uint64_t a0, a1, a2;           // less col[i] rows of A: the row of a stacked rank column is that many rows on
+    int col1, col2, col3;          // the first stacked rank column of side 1, 2, past the last one
+    int first0, first1, first2;    // the columns of the GEMM that have a term of the side lie in [first, end)
+    int end0, end1, end2;
+    int unused;
+};
+struct OwnSidesB {
+    uint64_t b0, b1, b2;
+    int col1, col2, col3;
+    int first0, first1, first2;    // columns whose masked index lies in [first, first + span) are the side's
+    int span0, span1, span2;
+    int key_mask, row_shift, low_mask;  // interleaved 8, 1, 7: row = 8 (column / 16) + column % 8; else -1, 0, 15 ...
+    int row_counts_from_first;     // ... and 1: less the side's first column
+    int unused;
+};
+struct OwnScales {
+    int ends[8];                   // read with constant indices only
+    float scales[8];
+};
+struct OwnArgs {
+    OwnSidesA a;
+    OwnSidesB b;
+    OwnScales scales;
+};
+struct LoraOwnFold : LoraFold {
+    OwnArgs own;
+};
+inline OwnArgs own_args(const DecodeArgs &d) {
+    const AdapterSides &h = *d.lora_sides;
+    // Up to four adapters give the bits of the stacked set (kLoraFoldMaxAdapters): every block has all ranks, in their places.
+    const bool all = h.interleaved || d.lora_adapters <= kLoraFoldMaxAdapters;
+    uint64_t a[3] = {}, b[3] = {};
+    int col[4] = {}, first[3] = {}, end[3] = {}, key[3] = {}, span[3] = {};
+    for (int i = 0; i < kMaxAdapterSides; ++i) {
+        col[i + 1] = col[i];
+        if (i >= h.count) continue;
+        a[i] = reinterpret_cast<uint64_t>(h.a[i]) - (uint64_t)col[i] * d.K * 2;
+        b[i] = reinterpret_cast<uint64_t>(h.b[i]);
+        first[i] = all ? 0 : h.first[i];
+        end[i] = all ? d.N : h.first[i] + h.rows[i];
+        key[i] = h.first[i];
+        span[i] = h.interleaved ? 8 : h.rows[i];
+        col[i + 1] += h.ranks[i];
+    }
+    OwnArgs o{};
+    o.a = OwnSidesA{a[0], a[1], a[2], col[1], col[2], col[3], first[0], first[1], first[2], end[0], end[1], end[2], 0};
+    o.b = OwnSidesB{b[0], b[1], b[2], col[1], col[2], col[3], key[0], key[1], key[2], span[0], span[1], span[2],
+                    h.interleaved ? 8 : -1, h.interleaved ? 1 : 0, h.interleaved ? 7 : 15, h.interleaved ? 0 : 1, 0};
+    for (int i = 0; i < 8; ++i) {
+        o.scales.ends[i] = d.lora_ends[i];
+        o.scales.scales[i] = d.lora_scales[i];
+    }
+    return o;
+}
+constexpr int kLoraFoldMaxProducers = 16;
 constexpr int kLoraSidesMaxAdapters = 8;
 constexpr int kLoraFoldStepsPerWave = 12;  // 32-value steps of K one producer wavefront takes, at most
 constexpr int kLoraFoldReplicas = 16;

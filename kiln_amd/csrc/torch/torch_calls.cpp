@@ -39,6 +39,7 @@ struct Library {
     decltype(&kiln_w4a16_stack_adapters) stack_adapters = nullptr;
     decltype(&kiln_w4a16_quantize_and_pack_many_device) quantize = nullptr;
     decltype(&kiln_w4a16_takes_adapter_sides) takes_sides = nullptr;
+    decltype(&kiln_w4a16_takes_rank) takes_rank = nullptr;
     decltype(&kiln_w4a16_gemm_adapter_sides) gemm_sides = nullptr;
     decltype(&kiln_w4a16_repack_gptq_device) repack = nullptr;
 };
@@ -298,10 +299,9 @@ bool add_side(PyObject *o, double scale, const Problem &p, int first, int rows, 
 
 // linear_sides(x, b_packed, scales, groupsize, swiglu, sides, widths, lora_scale, split): a GEMM whose columns belong
 // to several projections -- side by side, `widths` columns each, or with `swiglu` gate and up interleaved
-// (widths = n_out twice) -- each with its adapters or None.  One projection over all columns with a stacked rank that is a
-// multiple of 8 is what the entry points with adapters take as it is.  Else the launch reads every projection's own where
-// they lie -- one to three of them, each one's rank a multiple of 8, on the kernels that
-// kiln_w4a16_takes_adapter_sides names -- and all others become one stacked set in a launch of their own in front.
+// (widths = n_out twice) -- each with its adapters or None.  One projection over all columns with a stacked rank that
+// kiln_w4a16_takes_rank names is what the entry points with adapters take as it is.  Else the launch reads every projection's own where
+// they lie -- one to three of them, where kiln_w4a16_takes_adapter_sides says so -- and all others become one stacked set in a launch of their own in front.
 // `split`: the result comes as one view per projection.
 PyObject *py_linear_sides(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     HANDLE_TH_ERRORS
@@ -330,11 +330,12 @@ PyObject *py_linear_sides(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     for (size_t i = 0; i < sides.size(); ++i)
         own[i] = {sides[i].a.data_ptr(), sides[i].b.data_ptr(), sides[i].rank, sides[i].first, sides[i].rows};
     const int n_sides = (int)sides.size(), n_adapters = (int)l.ranks.size();
-    const bool in_place = !(n_sides == 1 && sides[0].rows == p.n) && n_sides > 0 &&
+    const bool as_it_is = n_sides == 1 && sides[0].rows == p.n && g_lib.takes_rank(p.m, p.n, p.k, sides[0].rank, p.device.index());
+    const bool in_place = !as_it_is && n_sides > 0 &&
                           g_lib.takes_sides(p.m, p.n, p.k, own, n_sides, swiglu ? 1 : 0, n_adapters, p.device.index());
     if (!sides.empty() && !in_place) {
         const int padded = (l.r_total + 7) / 8 * 8;
-        if (sides.size() == 1 && padded == l.r_total && sides[0].rows == p.n) {
+        if (as_it_is) {
             l.a = sides[0].a;
             l.b = sides[0].b;
         } else {
@@ -655,12 +656,12 @@ PyObject *py_set_workspaces(PyObject *, PyObject *const *args, Py_ssize_t nargs)
 
 // bind(addresses of the library's functions, in the order of Library)
 PyObject *py_bind(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
-    if (nargs != 12) {
-        PyErr_SetString(PyExc_TypeError, "bind takes twelve function addresses");
+    if (nargs != 13) {
+        PyErr_SetString(PyExc_TypeError, "bind takes thirteen function addresses");
         return nullptr;
     }
-    void *p[12];
-    for (int i = 0; i < 12; ++i) p[i] = PyLong_AsVoidPtr(args[i]);
+    void *p[13];
+    for (int i = 0; i < 13; ++i) p[i] = PyLong_AsVoidPtr(args[i]);
     if (PyErr_Occurred()) return nullptr;
     g_lib.gemm = reinterpret_cast<decltype(g_lib.gemm)>(p[0]);
     g_lib.gemm_lora = reinterpret_cast<decltype(g_lib.gemm_lora)>(p[1]);
@@ -674,6 +675,7 @@ PyObject *py_bind(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     g_lib.takes_sides = reinterpret_cast<decltype(g_lib.takes_sides)>(p[9]);
     g_lib.gemm_sides = reinterpret_cast<decltype(g_lib.gemm_sides)>(p[10]);
     g_lib.repack = reinterpret_cast<decltype(g_lib.repack)>(p[11]);
+    g_lib.takes_rank = reinterpret_cast<decltype(g_lib.takes_rank)>(p[12]);
     Py_RETURN_NONE;
 }
 

@@ -1,5 +1,6 @@
 // extern "C" entry points of libkiln_marlin_gemm (device side) and the
 // dispatcher that replaces `marlin_cuda` (crates/kiln-marlin-gemm/csrc/marlin_kernel.cu:731-819).
+#include <algorithm>
 #include <initializer_list>
 #include <memory>
 #include <mutex>
@@ -54,6 +55,7 @@ struct DecodePlan {
     long cost = -1;
     int gm_tiles = 0;   // > 0: for the LDS-staged group-major instance, tiles per block
     bool gmp = false;   // with gm_tiles > 0: for the private-staging group-major instance
+    int own = 0;        // gmp, with adapters: rank tiles a block projects x onto by itself
 };
 
 enum class DecodeMode { kStaged, kDirect, kRegs };
@@ -78,7 +80,8 @@ struct Tuning {
     int mid_waves = 0;                // > 0: its wavefronts per block, at most
     int flagged = -1;                 // 0 = K slices always meet through counters, -1 = automatic
     int lora_fold = -1;               // 0 = the LoRA projection always runs as a launch of its own, -1 = automatic,
-                                      // 2 = in the launch wherever the kernel can (whatever the grid's size)
+                                      // 2 = in the launch wherever the kernel can (whatever the grid's size), 3 = every
+                                      // block's own wherever the kernel can
     int rowsum_fold = -1;             // 0 = the matrix-core kernel's row sums always come from a launch in front, -1 = automatic
 };
 #ifdef KILN_W4A16_TUNING_HOOKS
@@ -238,7 +241,8 @@ constexpr long kRegsHandicap = 8;
 // the private-staging group-major instance with a given plan, if the shape takes it
 // lora: the plan must also hold for a call with adapters, whatever their ranks (one wavefront more per
 // block and the low-rank term's operands in LDS: checked for the largest rank and slice count)
-bool gmp_plan(int m, int n, int k, int tiles, int waves, int ks, bool lora, DecodePlan *plan) {
+// own: it takes adapters whose projection is each block's own, of this many times eight ranks
+bool gmp_plan(int m, int n, int k, int tiles, int waves, int ks, bool lora, DecodePlan *plan, int own = 0) {
     const int G = k / kGroupK, NT = n / kTileN;
     if (ks < 1 || G % ks != 0 || tiles < 1) return false;
     DecodeArgs a;
@@ -249,7 +253,13 @@ bool gmp_plan(int m, int n, int k, int tiles, int waves, int ks, bool lora, Deco
     a.GS = G / ks;
     a.waves = waves < a.GS ? waves : a.GS;
     a.gm_tiles = tiles;
-    if (lora) {
+    static const AdapterSides some_sides{};  // (the check asks for non-null operands only)
+    if (own > 0) {
+        a.own_tiles = (own + 1) / 2;
+        a.r_total = 64;
+        a.lora_sides = &some_sides;
+        a.lora_adapters = 1;
+    } else if (lora) {
         static const uint16_t probe = 0;  // never dereferenced: the check only asks for non-null operands
         a.r_total = 64;
         a.lora_slices = 16;
@@ -265,6 +275,7 @@ bool gmp_plan(int m, int n, int k, int tiles, int waves, int ks, bool lora, Deco
     plan->U = tiles * ceil_div(a.GS, a.waves);
     plan->BPS = ceil_div(NT, tiles);
     plan->gmp = true;
+    plan->own = a.own_tiles;
     return true;
 }
 
@@ -288,7 +299,9 @@ bool flagged_exchange_fits(int ks, int n) {
 // slices: 7.1 us with the parts as their own arrival flags, 8.4 through counters; four, six, eight
 // slices through counters 9.2, 9.9, 11.2).  A call with adapters plans for the chip less the blocks
 // that project x onto the adapters, so that the projection can ride in the same launch.
-bool plan_decode_gmp(int m, int n, int k, int cus, bool lora, DecodePlan *best) {
+// (own > 0: one whose blocks project x onto their own adapters, this many times eight ranks; its blocks are a plain call's,
+// lora is false.)
+bool plan_decode_gmp(int m, int n, int k, int cus, bool lora, DecodePlan *best, int own = 0, float *cost_of_best = nullptr) {
     const int G = k / kGroupK, NT = n / kTileN;
     // (a caller may name a part of the chip, `sms`: never plan for less than one unit)
     if (lora && g_tune.lora_fold != 0 && cus > lora_project_slices(m, k)) cus -= lora_project_slices(m, k);
@@ -301,6 +314,7 @@ bool plan_decode_gmp(int m, int n, int k, int cus, bool lora, DecodePlan *best) 
     float best_cost = -1.f;
     for (int ks = 1; ks <= kMaxKSlices && ks <= G; ++ks) {
         if (G % ks != 0) continue;
+        if (own > 0 && ks > 1 && !flagged_exchange_fits(ks, n)) continue;  // (no workspace beyond what the call has anyway)
         const int GS = G / ks;
         for (int waves : kWaves) {
             for (int T = 1; T <= 6; ++T) {
@@ -310,9 +324,9 @@ bool plan_decode_gmp(int m, int n, int k, int cus, bool lora, DecodePlan *best) 
                 // 8.4 us at one row against 10.4 in two rounds of two-tile blocks); elsewhere they
                 // measured 5 to 15 % slower than 12 on the same tiles and slices
                 DecodePlan p;
-                if (waves == most && (lora || T != 1 || GS % 16 != 0) && gmp_plan(m, n, k, T, 12, ks, lora, &p)) continue;
-                if (!gmp_plan(m, n, k, T, waves, ks, lora, &p)) continue;
-                const int rounds = ceil_div(ceil_div(NT, T) * ks, cus);
+                if (waves == most && (lora || T != 1 || GS % 16 != 0) && gmp_plan(m, n, k, T, 12, ks, lora, &p, own)) continue;
+                if (!gmp_plan(m, n, k, T, waves, ks, lora, &p, own)) continue;
+                const int rounds = ceil_div((ceil_div(NT, T) + (own > 0 && T > 1 ? 2 : 0)) * ks, cus);  // (blocks end at a side's end)
                 // The exchange: through counters 0.4 us per slice + 1.2; with the parts as their own
                 // arrival flags it grows with the tiles polled, 0.0037 us per (slice - 1) and tile
                 // (down projection, 160 tiles: 0.4 / 1.1 / 1.9 us at two / three / four slices;
@@ -328,7 +342,8 @@ bool plan_decode_gmp(int m, int n, int k, int cus, bool lora, DecodePlan *best) 
                 // wavefronts with three or more tiles each measure 3 to 7 % below twelve on the same
                 // tiles (fewer partial tiles to add at the end: gate+up at 16 rows 7.9 -> 7.6 us,
                 // q|k|v side by side 6.5 -> 6.15); with adapters the twelve stay (not measured).
-                float cost = 2.8f + rounds * (0.036f * T * GS + 0.0125f * a_kib_per_group * GS) +
+                // A block's own projection stages its rows of A_cat as it does A, 2 KiB a group and eight ranks.
+                float cost = 2.8f + rounds * (0.036f * T * GS + 0.0125f * (a_kib_per_group + 2 * own) * GS) +
                              0.08f * T * ceil_div(GS, p.waves) + exchange + 1.0f * (rounds - 1);
                 if (waves == 8 && T >= 3 && !lora) cost *= 0.95f;
                 if (best_cost < 0.f || cost < best_cost - 1e-4f) {
@@ -338,6 +353,7 @@ bool plan_decode_gmp(int m, int n, int k, int cus, bool lora, DecodePlan *best) 
             }
         }
     }
+    if (cost_of_best) *cost_of_best = best_cost;
     return best_cost >= 0.f;
 }
 
@@ -665,8 +681,61 @@ MidArgs mid_args(const MidPlan &mp, int m, int n, int k) {
     return a;
 }
 
+// Kinds of calls with adapters beside choose_decode's 1 and 2: those whose blocks of up to 16 rows may project x onto their
+// columns' adapters by themselves.
+struct OwnKind {
+    int eights;    // the ranks a block has, in eights, 1...4
+    bool sides;    // more than four adapters, not stacked
+    bool general;  // a rank that is a multiple of 4 only: else the call is of kind 2 (1 if not), or padded to 8 in front
+};
+constexpr int kFirstOwnKind = 3;
+constexpr int own_kind(const OwnKind &o) { return kFirstOwnKind + (o.eights - 1) + (o.sides ? 4 : 0) + (o.general ? 8 : 0); }
+constexpr OwnKind own_kind_of(int lora) {
+    const int v = lora - kFirstOwnKind;
+    return OwnKind{v % 4 + 1, (v & 4) != 0, (v & 8) != 0};
+}
+
+// Does every block project x onto its adapters by itself, and by which plan?  Against the projection in the launch's first
+// blocks, whose chain of round trips ends 5.5 to 6 us after the launch begins (6.2 where the adapters are not stacked) but
+// runs beside the streaming blocks: a launch that takes longer than that hides it, where a block's own projection adds its
+// share of A_cat to what the block stages.  The two plans' costs and constants were fitted to both, forced, on 15 shapes with
+// stacked adapters of 8 to 32 ranks and on the four calls of a layer at hidden 1024, 1536, 2560 and 4096 with adapters of 16
+// and 8 ranks a projection, at 1 to 16 rows: 8.9 % less time over these 310 cases than the first blocks alone, where the
+// better of the two each time is 10 %; the worst loss is 7 % (4096 -> 4096 with 8 ranks at one row, 5.7 -> 6.1 us).  What a
+// rank that is no multiple of 8 would cost otherwise is a launch that pads it (3 us).
+bool plan_own_projection(int m, int n, int k, int cus, const OwnKind &kind, DecodePlan *own) {
+    if (g_tune.gmp_tiles > 0)
+        return (g_tune.gmp_ks == 1 || flagged_exchange_fits(g_tune.gmp_ks, n)) &&
+               gmp_plan(m, n, k, g_tune.gmp_tiles, g_tune.gmp_waves, g_tune.gmp_ks, false, own, kind.eights);
+    float cost = 0.f, first_blocks = 0.f;
+    if (!plan_decode_gmp(m, n, k, cus, false, own, kind.eights, &cost)) return false;
+    DecodePlan other;
+    if (g_tune.lora_fold == 3 || !plan_decode_gmp(m, n, k, cus, true, &other, 0, &first_blocks)) return true;
+    if (kind.general) return cost <= std::max(first_blocks + 2.f, 8.f);
+    return cost <= (kind.sides ? std::max(first_blocks + 1.0f, 6.2f) : std::max(first_blocks - 0.5f, 5.6f));
+}
+
+// lora: as choose_decode takes it, or an OwnKind
 void plan_gemm(int m, int n, int k, int cus, int thread_k, int thread_n, int lora, GemmPlan *gp) {
     *gp = GemmPlan{};
+    if (lora >= kFirstOwnKind) {
+        const OwnKind kind = own_kind_of(lora);
+        DecodePlan own;
+        const bool forced = g_tune.mid == 1 || g_tune.prefill_min_m != 0 || g_tune.decode_group_major != -1 || g_tune.decode_direct_max_m >= 0 ||
+                            g_tune.force_ks || g_tune.force_u || g_tune.force_waves;
+        if (m <= 16 && thread_k <= 0 && thread_n <= 0 && !forced && (size_t)(n / kTileN) * sizeof(int) <= kCounterCapacity &&
+            plan_own_projection(m, n, k, cus, kind, &own)) {
+            DecodeLaunch &l = gp->dl[gp->launches++];
+            l.r0 = 0;
+            l.M = m;
+            l.rows = 0;
+            l.plan = own;
+            l.direct = false;
+            gp->decode_partial = decode_launch_partial_bytes(l, n, k);
+            return;
+        }
+        lora = kind.general ? 2 : 1;
+    }
     // mid_min_rows() ... mid_max_rows() rows: the mid-M kernel, one pass over the weights per 64 rows (with
     // adapters whose stacked rank is a multiple of 8: the low-rank term is added from a projection that runs
     // in the launch's first blocks where it fits, else from one launched in front)
@@ -862,6 +931,25 @@ struct LoraSpec {
     const AdapterSides *sides = nullptr;  // in place of a and b, which are null: calls that sides_in_launch() takes
 };
 
+// The `lora` of plan_gemm for a call: which kernels can take its adapters.  A block of up to 16 rows that projects x onto
+// the adapters by itself does so for all of them, or, where more than four lie side by side, for those that its columns have
+// a term of (up to four, the call is one with the stacked set in every bit: the same choice, plan and places).  Blocks end
+// where a side does, whole tiles.
+int lora_kind(const LoraSpec *lora, int m) {
+    if (!lora) return 0;
+    const int otherwise = lora->r_total % 8 == 0 ? 1 : 2;
+    if (m > 16 || (g_tune.lora_fold != -1 && g_tune.lora_fold != 3) || lora->r_total % 4 != 0) return otherwise;
+    int ranks = lora->r_total;
+    const bool many = lora->sides && lora->n_adapters > 4;
+    if (lora->sides && !lora->sides->interleaved) {
+        const AdapterSides &s = *lora->sides;
+        if (many) ranks = *std::max_element(s.ranks, s.ranks + s.count);
+        for (int i = 0; i < s.count; ++i)
+            if (s.first[i] % kTileN != 0) return otherwise;
+    }
+    return ranks <= 32 ? own_kind({(ranks + 7) / 8, many, lora->r_total % 8 != 0}) : otherwise;
+}
+
 // Bytes a call of m rows needs, made monotone in m: the largest need of any m' <= m.  The plan
 // (and with it the need) changes with m' only through the small-M and mid-M runs (m' <= 1024 here; beyond
 // that only overrides keep a call on that path) and through the matrix-core kernel's row blocks
@@ -984,6 +1072,7 @@ bool mid_lora_in_launch(const GemmPlan &gp, const LoraSpec &lora, void *flags, M
 // private-staging and the mid-M kernel.
 bool sides_in_launch(const GemmPlan &gp, int m, int n, int k, int cus, const LoraSpec &lora, void *t, void *flags) {
     if (gp.prefill) return false;
+    if (!gp.mid && gp.dl[0].plan.own > 0) return true;
     if (gp.mid) {
         MidArgs ask = mid_args(gp.mp, m, n, k);
         return mid_lora_in_launch(gp, lora, flags, &ask);
@@ -1010,9 +1099,8 @@ kiln_marlin_status_t gemm_any(const void *A, const void *B, void *C, const void 
 
     const int cus = sms > 0 ? sms : compute_units(dev);
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    const int lora_kind = !lora ? 0 : (lora->r_total % 8 == 0 ? 1 : 2);
     const std::shared_ptr<const PlannedCall> planned =
-        plan_call(prob_m, prob_n, prob_k, cus, thread_k > 0 ? thread_k : -1, thread_n > 0 ? thread_n : -1, lora_kind);
+        plan_call(prob_m, prob_n, prob_k, cus, thread_k > 0 ? thread_k : -1, thread_n > 0 ? thread_n : -1, lora_kind(lora, prob_m));
     const GemmPlan &gp = planned->gp;
     const WorkspaceLayout &wl = planned->wl;
     char *ws = reinterpret_cast<char *>(workspace);
@@ -1105,12 +1193,14 @@ kiln_marlin_status_t gemm_any(const void *A, const void *B, void *C, const void 
     // Up to 16 rows on the private-staging kernel: the projection rides in the GEMM launch (extra
     // blocks at the front of its grid) instead of running as a launch of its own.
     DecodeArgs in_launch{};
-    const bool fold = lora && lora_in_launch(gp, prob_m, prob_k, cus, *lora, lora_t, ws + kFoldFlagOffset, &in_launch);
+    const int own = lora && gp.launches == 1 ? gp.dl[0].plan.own : 0;  // ... or every block of it has one of its own
+    const AdapterSides stacked = lora ? AdapterSides{{lora->a}, {lora->b}, {lora->r_total}, {0}, {prob_n}, 1, 0} : AdapterSides{};
+    const bool fold = lora && own == 0 && lora_in_launch(gp, prob_m, prob_k, cus, *lora, lora_t, ws + kFoldFlagOffset, &in_launch);
     if (fold) {
         lora_slices = in_launch.lora_slices;
         rp = (lora->r_total + 15) / 16 * 16;
     }
-    if (lora && !fold) {  // the scaled projection of all rows onto the adapters, once, ahead of the runs
+    if (lora && !fold && own == 0) {  // the scaled projection of all rows onto the adapters, once, ahead of the runs
         PrefillArgs pj{};
         pj.A = A;
         pj.M = prob_m;
@@ -1144,12 +1234,17 @@ kiln_marlin_status_t gemm_any(const void *A, const void *B, void *C, const void 
             a.r_total = lora->r_total;
             a.lora_slices = lora_slices;
             a.lora_rows = prob_m;
-            if (fold) {
+            if (own > 0) {
+                a.own_tiles = own;
+                a.lora_sides = lora->sides ? lora->sides : &stacked;
+            } else if (fold) {
                 a.lora_producers = lora_slices;
                 a.lora_steps_per_slice = in_launch.lora_steps_per_slice;
                 a.lora_a = lora->a;
                 a.lora_sides = lora->sides;
                 a.lora_flags = in_launch.lora_flags;
+            }
+            if (own > 0 || fold) {
                 a.lora_adapters = lora->n_adapters;
                 int end = 0;
                 for (int j = 0; j < 8; ++j) {
@@ -1484,6 +1579,14 @@ static kiln_marlin_status_t sides_of(const kiln_w4a16_adapter_side *sides, int n
     return KILN_W4A16_OK;
 }
 
+int kiln_w4a16_takes_rank(int prob_m, int prob_n, int prob_k, int r_total, int dev) {
+    if (prob_m < 1 || prob_n < 1 || prob_k < 1 || !shape_ok(prob_n, prob_k, 128) || r_total < 1 || r_total > 64) return 0;
+    if (r_total % 8 == 0) return 1;
+    const LoraSpec lora{nullptr, nullptr, r_total, 1, nullptr, nullptr};
+    const auto planned = plan_call(prob_m, prob_n, prob_k, compute_units(dev), -1, -1, lora_kind(&lora, prob_m));
+    return planned->gp.launches == 1 && planned->gp.dl[0].plan.own > 0 ? 1 : 0;
+}
+
 int kiln_w4a16_takes_adapter_sides(int prob_m, int prob_n, int prob_k, const kiln_w4a16_adapter_side *sides, int n_sides, int swiglu,
                                    int n_adapters, int dev) {
     AdapterSides own;
@@ -1494,7 +1597,7 @@ int kiln_w4a16_takes_adapter_sides(int prob_m, int prob_n, int prob_k, const kil
     static const unsigned probe = 0;  // never dereferenced
     const int cus = compute_units(dev);
     const LoraSpec lora{nullptr, nullptr, r_total, n_adapters, nullptr, nullptr, &own};
-    return sides_in_launch(plan_call(prob_m, prob_n, prob_k, cus, -1, -1, 1)->gp, prob_m, prob_n, prob_k, cus, lora,
+    return sides_in_launch(plan_call(prob_m, prob_n, prob_k, cus, -1, -1, lora_kind(&lora, prob_m))->gp, prob_m, prob_n, prob_k, cus, lora,
                            const_cast<unsigned *>(&probe), const_cast<unsigned *>(&probe)) ? 1 : 0;
 }
 

@@ -34,16 +34,22 @@ constexpr int kGmpSlotBytes = 16 * 256;  // one group of A: 16 rows x 128 bf16
 #ifndef KILN_GMP_HEAD
 #define KILN_GMP_HEAD 3
 #endif
-// This file is compiled three times: as it is for calls without adapters, with -DKILN_GMP_LORA=1 for
-// calls with them (launch_decode_gmp_lora only), and with =2 for calls whose adapters are not stacked
-// (launch_decode_gmp_sides only).  What the low-rank term adds -- one wavefront more,
+// This file is compiled five times: as it is for calls without adapters, with -DKILN_GMP_LORA=1 for
+// calls with them (launch_decode_gmp_lora only), with =2 for calls whose adapters are not stacked
+// (launch_decode_gmp_sides only), and with =3 and =4 for calls with either whose blocks need one or two
+// tiles of 16 rank columns, which each block projects x onto by itself (launch_decode_gmp_own1 and _own2).
+// What the low-rank term adds -- one wavefront more,
 // its arguments, the signalling between the wavefronts -- then costs calls without adapters
 // nothing: as one kernel with run-time branches it cost them 0.1...0.2 us per launch.
 #ifndef KILN_GMP_LORA
 #define KILN_GMP_LORA 0
 #endif
-constexpr bool kGmpLora = KILN_GMP_LORA != 0, kGmpSides = KILN_GMP_LORA == 2;
-using GmpFold = std::conditional_t<kGmpSides, LoraSidesFold, LoraFold>;
+constexpr bool kGmpLora = KILN_GMP_LORA == 1 || KILN_GMP_LORA == 2, kGmpSides = KILN_GMP_LORA == 2;
+constexpr int kOwnTiles = KILN_GMP_LORA >= 3 ? KILN_GMP_LORA - 2 : 0;  // rank tiles a block projects x onto by itself
+#if KILN_GMP_LORA >= 3
+#define w4a16_decode_gmp_kernel w4a16_decode_gmp_own_kernel  // (the name profiles show)
+#endif
+using GmpFold = std::conditional_t<kGmpSides, LoraSidesFold, std::conditional_t<(kOwnTiles > 0), LoraOwnFold, LoraFold>>;
 
 // Probe builds only (-DKILN_GMP_TIMELINE): wall-clock stamps (100 MHz) per wavefront.
 #ifdef KILN_GMP_TIMELINE
@@ -51,6 +57,10 @@ using GmpFold = std::conditional_t<kGmpSides, LoraSidesFold, LoraFold>;
 #define g_gmp_tl g_gmp_tl_lora
 #elif KILN_GMP_LORA == 2
 #define g_gmp_tl g_gmp_tl_sides
+#elif KILN_GMP_LORA == 3
+#define g_gmp_tl g_gmp_tl_own1
+#elif KILN_GMP_LORA == 4
+#define g_gmp_tl g_gmp_tl_own2
 #endif
 __device__ long long *g_gmp_tl;
 #define KILN_GMP_TL(i, v) tl_[i] = (v)
@@ -73,13 +83,15 @@ constexpr int kGmpMaxChunks = 16;        // chunks per wavefront, at most (strai
 // The activations of a group are requested one group ahead, not all at once: every block stages
 // its own copy of the slice, as many bytes through L2 as the weights at 16 rows, and a burst of
 // them at the start keeps the wavefronts in the issue stage while the weight stream runs dry.
+// OWN rank tiles: A_cat(g), 4 LDS-direct loads a tile, behind A(0) and, as its one slot is read before, behind the
+// fragments of group g - 1; behind A_cat(0) the tile's rows of B_cat, two loads at most.
 struct GmpSchedule {
-    int wait_a[kGmpMaxChunks];      // by group
+    int wait_a[kGmpMaxChunks];      // by group: A(g) and A_cat(g)
     int wait_chunk[kGmpMaxChunks];  // by chunk
 };
-constexpr GmpSchedule gmp_schedule(int T, int groups, int AQ) {
+constexpr GmpSchedule gmp_schedule(int T, int groups, int AQ, int OWN) {
     const int U = T * groups;
-    int kind[3 * kGmpMaxChunks] = {}, idx[3 * kGmpMaxChunks] = {}, size[3 * kGmpMaxChunks] = {};
+    int kind[4 * kGmpMaxChunks] = {}, idx[4 * kGmpMaxChunks] = {}, size[4 * kGmpMaxChunks] = {};
     int n = 0;
     auto push = [&](int k, int i, int sz) {
         kind[n] = k;
@@ -98,24 +110,35 @@ constexpr GmpSchedule gmp_schedule(int T, int groups, int AQ) {
     };
     for (int j = 0; j < kGmpHead && j < U; ++j) push(1, j, 2);
     push(0, 0, AQ);
+    if (OWN > 0) {
+        push(2, 0, 4 * OWN);
+        push(3, 0, OWN);
+    }
     GmpSchedule s{};
     for (int j = 0; j < U; ++j) {
         if (j + kGmpHead < U) push(1, j + kGmpHead, 2);
         if (j % T == 0) {
             const int g = j / T;
             if (g + 1 < groups) push(0, g + 1, AQ);
-            s.wait_a[g] = issued_after(0, g);
+            s.wait_a[g] = issued_after(OWN > 0 ? 2 : 0, g);
+            if (OWN > 0 && g + 1 < groups) push(2, g + 1, 4 * OWN);
         }
         s.wait_chunk[j] = issued_after(1, j);
     }
     return s;
 }
-template <int T, int GROUPS, int AQ>
+template <int T, int GROUPS, int AQ, int OWN>
 struct GmpScheduleOf {
-    static constexpr GmpSchedule value = gmp_schedule(T, GROUPS, AQ);
+    static constexpr GmpSchedule value = gmp_schedule(T, GROUPS, AQ, OWN);
 };
 
 constexpr int gmp_slots(int gpw) { return gpw < 2 ? gpw : 2; }
+// wavefronts of a block, at most; own: as many as have their slots in 160 KiB of LDS (10 or 13 of the instances of two
+// rank tiles, which need more registers than 16 can have)
+constexpr int gmp_max_waves(int gpw, int own) {
+    const int fit = (160 * 1024 - 128) / ((gmp_slots(gpw) + own) * kGmpSlotBytes);
+    return own == 0 || fit > kGmpMaxWaves ? kGmpMaxWaves : fit;
+}
 constexpr int kGmpFlaggedSlices = kDecodeFlaggedMaxSlices;  // most K slices the counter-free exchange takes
 constexpr int kGmpSpinLimit = 1 << 20;  // polls of the other slices' parts before the adding wavefront gives up
 
@@ -175,6 +198,68 @@ constexpr uint32_t kGmpLooked = 1, kGmpOperandsReady = 2;  // values of the sign
 // Two words at the start of the adapter wavefront's part of LDS: the signal and the arrival count.
 constexpr unsigned kGmpSyncBytes = 16;
 
+// The low-rank term from a projection that every block forms by itself (OWN tiles of 16 rank columns).  A wavefront has
+// its groups of x in LDS already; it stages the same groups of the rows of A that the block's columns have a term of
+// beside them and adds one product a tile and 32 values of K -- (A_cat x^T), so that a lane ends with four rank columns of
+// a row of x, which is the layout the term's own product takes.  The wavefronts' parts meet with the partial tiles, T is
+// rounded once per K slice of the GEMM, and every slice adds its own T times B_cat^T to its own part (the term is linear
+// in T).  No block waits for another: the projection in the launch's first blocks is a chain of round trips across the chip
+// -- start, operands, T to memory, flags, T copied -- that ends 5.4...6.3 us after the launch begins whatever the GEMM is.
+// What it costs instead is A_cat through L2 once per block, 4 KiB a group and rank tile (A itself is as much at 16 rows).
+// Measured (us, projection in the launch's first blocks -> each block's own): 1024 -> 4096 with two adapters of rank 8 at 16
+// rows 6.0 -> 4.1, 2048 -> 2048 with two of rank 16 6.9 -> 5.6, q | k | v of 2560 -> 8192 / 1024 / 1024 with two of rank 8 each at
+// 11 rows 8.2 -> 7.4, of 1024 -> 3072 / 1024 / 1024 at 16 rows 7.5 -> 4.3; rank 12, which those blocks read only padded by a
+// launch in front, 2560 -> 10240 at 16 rows 10.5 -> 7.3.  Beyond the launches the dispatcher's rule takes it loses: 2560 ->
+// 18432 with 32 ranks at one row 7.5 -> 9.8, 160 KiB of A_cat a block at 0.0125 us a KiB on top of the weights.
+// Everything below is free of branches: it runs while the first weights are in flight to registers.
+struct OwnWindow {  // the stacked rank columns that the block's columns have a term of
+    int lo, ranks;
+};
+[[maybe_unused]] __device__ __forceinline__ OwnWindow own_window(const OwnSidesA &s, int first_column, int end_column) {
+    const bool here0 = (s.first0 < end_column) & (s.end0 > first_column), here1 = (s.first1 < end_column) & (s.end1 > first_column),
+               here2 = (s.first2 < end_column) & (s.end2 > first_column);
+    int lo = here2 ? s.col2 : s.col3, hi = here0 ? s.col1 : 0;
+    lo = here1 ? s.col1 : lo;
+    lo = here0 ? 0 : lo;
+    hi = here1 ? s.col2 : hi;
+    hi = here2 ? s.col3 : hi;
+    lo = min(lo, hi);
+    return OwnWindow{lo, hi - lo};
+}
+// A member in a scalar register of its own (a choice between members would otherwise become one between their addresses, in
+// scratch memory).
+template <class V>
+__device__ __forceinline__ V scalar(V v) {
+    asm("" : "+s"(v));
+    return v;
+}
+// the row of A of a stacked rank column
+[[maybe_unused]] __device__ __forceinline__ const char *own_a_row(const OwnSidesA &s, int rank, uint32_t row_bytes) {
+    const uint64_t a1 = scalar(s.a1), a2 = scalar(s.a2);
+    uint64_t base = scalar(s.a0);
+    base = rank >= s.col1 ? a1 : base;
+    base = rank >= s.col2 ? a2 : base;
+    return reinterpret_cast<const char *>(base + (uint64_t)(uint32_t)rank * row_bytes);
+}
+// Where four rank columns from `rank` on of a column's row of B_cat lie; false (and an address that can be read): no term.
+[[maybe_unused]] __device__ __forceinline__ bool own_b_unit(const OwnSidesB &s, int column, int rank, const void **at) {
+    const int key = column & s.key_mask, row = ((column & ~15) >> s.row_shift) + (column & s.low_mask);
+    uint64_t p = scalar(s.b0), from = 0;
+    bool live = false;
+    auto side = [&](uint64_t b, int first, int span, int col, int end) {
+        const int width = end - col;
+        const bool mine = ((uint32_t)(key - first) < (uint32_t)span) & ((uint32_t)(rank - col) < (uint32_t)width);
+        p = mine ? b : p;
+        from = mine ? (uint64_t)(int64_t)((row - first * s.row_counts_from_first) * width + rank - col) * 2 : from;
+        live |= mine;
+    };
+    side(scalar(s.b0), s.first0, s.span0, 0, s.col1);
+    side(scalar(s.b1), s.first1, s.span1, s.col1, s.col2);
+    side(scalar(s.b2), s.first2, s.span2, s.col2, s.col3);
+    *at = reinterpret_cast<const void *>(p + from);
+    return live;
+}
+
 // The kernel's last argument and where it sits among the arguments: the kernel reads it late, through
 // the argument segment's address (see there), so its place is spelled out as a struct with the
 // kernel's parameter list.
@@ -187,6 +272,14 @@ constexpr int kGmpSidesOffset = (int)(offsetof(GmpLoraArgs, fold) + offsetof(Lor
 #else
 constexpr int kGmpSidesOffset = 0;
 #endif
+#if KILN_GMP_LORA >= 3
+constexpr int kOwnOffset = (int)(offsetof(GmpLoraArgs, fold) + offsetof(LoraOwnFold, own));
+#else
+constexpr int kOwnOffset = 0;
+#endif
+constexpr int kOwnAOffset = kOwnOffset + (int)offsetof(OwnArgs, a), kOwnBOffset = kOwnOffset + (int)offsetof(OwnArgs, b),
+              kOwnScalesOffset = kOwnOffset + (int)offsetof(OwnArgs, scales);
+constexpr int kOwnScaleBytes = 2 * 16 * (int)sizeof(float);  // a scale per rank column of the block, behind the slots
 struct GmpLateArgs {  // what every wavefront needs of them
     LoraTail lo;
     LoraFold fold;
@@ -270,10 +363,13 @@ static_assert(sizeof(GmpTailArgs) == 32, "eight words");
 // fewer), AQ = LDS-direct loads per group of A: 4 (16 rows), 2 (M <= 8) or 1 (M <= 4: rows 0...3
 // only; the other rows of the product are computed from whatever LDS holds and never stored).
 template <int T, int GPW, int AQ, bool LORA>
-__global__ __launch_bounds__(kGmpMaxWaves * 64) void w4a16_decode_gmp_kernel(
+__global__ __launch_bounds__(gmp_max_waves(GPW, kOwnTiles) * 64) void w4a16_decode_gmp_kernel(
     const uint16_t *__restrict__ A, const u32x4 *__restrict__ B, const uint16_t *__restrict__ S, uint32_t shape,
-    uint32_t layout, int G, int NT, int GS, int col_blocks, uint16_t *__restrict__ C_arg, float *partial_arg,
+    uint32_t layout, int G_arg, int NT_arg, int GS_arg, int col_blocks_arg, uint16_t *__restrict__ C_arg, float *partial_arg,
     int *counters_arg, GmpLoraArgs la) {
+    // (own projections: 16 bits each, the upper ones say where the sides of the adapters meet, own_borders)
+    constexpr uint32_t kLow = kOwnTiles > 0 ? 0xFFFFu : 0xFFFFFFFFu;
+    const int G = (uint32_t)G_arg & kLow, NT = (uint32_t)NT_arg & kLow, GS = (uint32_t)GS_arg & kLow, col_blocks = (uint32_t)col_blocks_arg & kLow;
     const int M = shape & 255, full_waves = (shape >> 8) & 255, nw_all = (shape >> 16) & 255, KS = shape >> 24;
     const int slot_bytes = layout & 0xFFFF;
     const int producers = LORA ? (layout >> 16) & 255 : 0, adapter = LORA && (layout & kGmpAdapter) ? 1 : 0;
@@ -320,7 +416,15 @@ __global__ __launch_bounds__(kGmpMaxWaves * 64) void w4a16_decode_gmp_kernel(
     // in one die's L2 (measured: 2...3 us per poll instead of 0.5).
     int col_block = bx + ((layout & kGmpColShift) ? ks : 0);
     if (col_block >= col_blocks) col_block -= col_blocks;  // at most three past the end, of sixteen tiles or more
-    const int tf = col_block * T;  // first tile of the block; tiles from NT on do not exist
+    int tf = col_block * T, tile_end = NT;  // first tile of the block; tiles from tile_end on are not its own
+    if constexpr (kOwnTiles > 0) {  // the blocks of a side end where it does: no block has columns of two
+        const int blocks0 = (uint32_t)G_arg >> 16, blocks1 = (uint32_t)col_blocks_arg >> 16;  // ... of the first, of the first two
+        const int end0 = (uint32_t)NT_arg >> 16, end1 = (uint32_t)GS_arg >> 16;
+        const int before = col_block < blocks0 ? 0 : (col_block < blocks1 ? blocks0 : blocks1);
+        const int from = col_block < blocks0 ? 0 : (col_block < blocks1 ? end0 : end1);
+        tile_end = col_block < blocks0 ? end0 : (col_block < blocks1 ? end1 : NT);
+        tf = from + (col_block - before) * T;
+    }
     const bool full = wave < full_waves;
     const int g_first = full ? wave * GPW : full_waves * GPW + (wave - full_waves) * (GPW - 1);
     const int g0 = ks * GS + g_first;  // all slices have GS groups
@@ -334,7 +438,7 @@ __global__ __launch_bounds__(kGmpMaxWaves * 64) void w4a16_decode_gmp_kernel(
     // one 64-bit address per operand, 32-bit distances from it
     const bool column_scales = (layout & kGmpColumnScales) != 0;
     const uint32_t scale_groups = column_scales ? 1u : (uint32_t)G;
-    const int last_tile = NT - 1 - tf;
+    const int last_tile = tile_end - 1 - tf;
     const char *const b_first = reinterpret_cast<const char *>(B) + (size_t)((uint32_t)tf * (uint32_t)G + (uint32_t)g0) * 1024;
     const char *const s_first = reinterpret_cast<const char *>(S) +
                                 (size_t)((uint32_t)tf * scale_groups + (column_scales ? 0u : (uint32_t)g0)) * (kTileN * 2);
@@ -369,13 +473,55 @@ __global__ __launch_bounds__(kGmpMaxWaves * 64) void w4a16_decode_gmp_kernel(
 #pragma unroll
     for (int ti = 0; ti < T; ++ti) y[ti] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    // Straight-line code from the first request to the last use, one instance per group count.
-    auto run = [&](auto nc) {
-        constexpr int NGR = decltype(nc)::value, U = T * NGR;
-        using Sch = GmpScheduleOf<T, NGR, AQ>;
+    // The block's own projection: parts of T, the operand of the tile that this wavefront stores first, the block's ranks
+    [[maybe_unused]] f32x4 t_part[kOwnTiles + 1];
+    [[maybe_unused]] u32x2 b_own[kOwnTiles + 1];
+    [[maybe_unused]] bool b_live[kOwnTiles + 1];
+    [[maybe_unused]] OwnWindow own{0, 0};
+#pragma unroll
+    for (int j = 0; j < kOwnTiles; ++j) t_part[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    // Straight-line code from the first request to the last use, one instance per group count (and number of rank tiles).
+    auto run = [&](auto nc, auto oc) {
+        constexpr int NGR = decltype(nc)::value, U = T * NGR, OWN = decltype(oc)::value;
+        using Sch = GmpScheduleOf<T, NGR, AQ, OWN>;
         unrolled<0, (kGmpHead < U ? kGmpHead : U)>(request_chunk);
         request_a(0, 0);
         if constexpr (LORA) __syncthreads();  // the adapter wavefront has zeroed the words the block meets on
+        [[maybe_unused]] const char *a_own[4 * OWN + 1];
+        [[maybe_unused]] const unsigned own_addr = mine_addr + NS * kGmpSlotBytes;
+        [[maybe_unused]] auto request_own = [&] {  // the next group of A_cat, as request_a lays out A
+#pragma unroll
+            for (int i = 0; i < 4 * OWN; ++i) {  // ranks come in fours, a load; past the block's nothing is asked for
+                load_to_lds_b128_if(4 * i, own.ranks, a_own[i], own_addr + i * 1024);
+                a_own[i] += 256;
+            }
+        };
+        if constexpr (OWN > 0) {
+            const OwnSidesA sides_a = read_argument<OwnSidesA>(kGmpLoraArgsOffset + kOwnAOffset);
+            own = own_window(sides_a, tf * kTileN, (tf + min(T, tile_end - tf)) * kTileN);
+#pragma unroll
+            for (int i = 0; i < 4 * OWN; ++i)  // (past the block's ranks: an address nothing is asked of)
+                a_own[i] = own_a_row(sides_a, own.lo + 4 * i + (lane >> 4), row_pitch) +
+                           ((uint32_t)g0 * 256u + (((lane & 15) ^ ((4 * i + (lane >> 4)) & 15)) << 4));
+            request_own();
+            const OwnSidesB sides_b = read_argument<OwnSidesB>(kGmpLoraArgsOffset + kOwnBOffset);
+#pragma unroll
+            for (int j = 0; j < OWN; ++j) {
+                const void *at;
+                b_live[j] = own_b_unit(sides_b, (tf + min(wave, last_tile)) * kTileN + (lane & 15), own.lo + 16 * j + 4 * (lane >> 4), &at);
+                load_b64(b_own[j], at);
+            }
+            // the scale of every rank column, by every wavefront alike
+            const OwnScales by_adapter = read_argument<OwnScales>(kGmpLoraArgsOffset + kOwnScalesOffset);
+            float scale = 0.f;
+#pragma unroll
+            for (int i = kLoraSidesMaxAdapters - 1; i >= 0; --i) {
+                const float of_adapter = scalar(by_adapter.scales[i]);
+                scale = own.lo + (lane & 31) < by_adapter.ends[i] ? of_adapter : scale;
+            }
+            reinterpret_cast<float *>(lds + nw_all * slot_bytes)[lane & 31] = scale;
+        }
         u32x4 af[4];
         f32x4 offset_term;
         unrolled<0, U>([&](auto jc) {
@@ -395,6 +541,21 @@ __global__ __launch_bounds__(kGmpMaxWaves * 64) void w4a16_decode_gmp_kernel(
 #pragma unroll
                 for (int t = 0; t < 4; ++t)
                     af[t] = *reinterpret_cast<const u32x4 *>(ap + (((4 * t + (lane >> 4)) ^ (lane & 15)) << 4));
+                if constexpr (OWN > 0) {
+                    u32x4 of[4 * OWN];
+                    const unsigned char *op = mine + NS * kGmpSlotBytes + (lane & 15) * 256;
+#pragma unroll
+                    for (int i = 0; i < 4 * OWN; ++i)
+                        of[i] = *reinterpret_cast<const u32x4 *>(op + (i >> 2) * 4096 + (((4 * (i & 3) + (lane >> 4)) ^ (lane & 15)) << 4));
+                    if constexpr (gi + 1 < NGR) {
+                        wait_lds_reads();  // the slot's fragments are in registers
+                        request_own();
+                    }
+#pragma unroll
+                    for (int i = 0; i < 4 * OWN; ++i)
+                        t_part[i >> 2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, of[i]),
+                                                                                 __builtin_bit_cast(bf16x8, af[i & 3]), t_part[i >> 2], 0, 0, 0);
+                }
                 offset_term = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int t = 0; t < 4; ++t)
@@ -414,16 +575,23 @@ __global__ __launch_bounds__(kGmpMaxWaves * 64) void w4a16_decode_gmp_kernel(
                                                           acc, 0, 0, 0);
             y[ti] += acc * f16_bits_to_f32((uint16_t)sc[set]);
         });
+#pragma unroll
+        for (int j = 0; j < OWN; ++j) pin_loaded(b_own[j]);  // issued ahead of the last chunk
     };
     if (__builtin_expect(!adapter_wave, 1)) {
-        if (full) run(std::integral_constant<int, GPW>{});
-        else if constexpr (GPW > 1) run(std::integral_constant<int, GPW - 1>{});
+        auto run_groups = [&](auto oc) {
+            if (full) run(std::integral_constant<int, GPW>{}, oc);
+            else if constexpr (GPW > 1) run(std::integral_constant<int, GPW - 1>{}, oc);
+        };
+        run_groups(std::integral_constant<int, kOwnTiles>{});
         // every wavefront's partial tiles into its own piece of LDS, then tile ti = their sum in
         // wavefront (= ascending K) order, one tile per wavefront at a time
         KILN_GMP_TL(1, KILN_GMP_NOW());
         f32x4 *slots = reinterpret_cast<f32x4 *>(mine);
 #pragma unroll
         for (int ti = 0; ti < T; ++ti) slots[ti * 64 + lane] = y[ti];
+#pragma unroll
+        for (int j = 0; j < kOwnTiles; ++j) slots[(T + j) * 64 + lane] = t_part[j];
     } else if constexpr (LORA) {
         const unsigned sync_addr = (unsigned)(size_t)(lds_ptr_t)(lds + nw * slot_bytes);
         lds_signal_store(sync_addr, 0u);
@@ -514,9 +682,28 @@ __global__ __launch_bounds__(kGmpMaxWaves * 64) void w4a16_decode_gmp_kernel(
     int *const counters = tail.counters;
     const bool swiglu = (tail.layout & kGmpSwiglu) != 0, flagged = (tail.layout & kGmpFlagged) != 0;
     const int q4 = lane >> 4, c = lane & 15;
-    const int tiles = min(T, NT - tf);
+    const int tiles = min(T, tile_end - tf);
     if constexpr (LORA) {
         if (wave < tiles) lds_signal_wait(arrivals_addr(), nw);  // every main wavefront's partial tiles are in LDS
+    }
+    // T of the block's own ranks, as the term's operand: a lane has row lane % 16 of x and the rank columns 4 q4 ... + 3 of
+    // either tile; B's operand is read in the same order.
+    [[maybe_unused]] u32x4 t_own = {0u, 0u, 0u, 0u};
+    if constexpr (kOwnTiles > 0) {
+        if (wave < tiles) {
+            const float *scales = reinterpret_cast<const float *>(lds + nw_all * slot_bytes);
+#pragma unroll
+            for (int j = 0; j < kOwnTiles; ++j) {
+                f32x4 part = {0.f, 0.f, 0.f, 0.f};
+                for (int wv = 0; wv < nw; ++wv) part += reinterpret_cast<const f32x4 *>(lds + wv * slot_bytes)[(T + j) * 64 + lane];
+                part *= *reinterpret_cast<const f32x4 *>(scales + 16 * j + 4 * q4);
+                uint32_t bits[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) bits[i] = 16 * j + 4 * q4 + i < own.ranks ? (uint32_t)f32_to_bf16_bits(part[i]) : 0u;
+                t_own[2 * j] = bits[0] | bits[1] << 16;
+                t_own[2 * j + 1] = bits[2] | bits[3] << 16;
+            }
+        }
     }
     for (int ti = wave; ti < tiles; ti += nw) {
         const int tt = tf + ti;
@@ -524,6 +711,24 @@ __global__ __launch_bounds__(kGmpMaxWaves * 64) void w4a16_decode_gmp_kernel(
         // 0.1...0.3 us slower per launch than this loop)
         f32x4 sum = {0.f, 0.f, 0.f, 0.f};
         for (int wv = 0; wv < nw; ++wv) sum += reinterpret_cast<const f32x4 *>(lds + wv * slot_bytes)[ti * 64 + lane];
+        if constexpr (kOwnTiles > 0) {
+            if (ti != wave) {  // a block of fewer wavefronts than tiles
+                const OwnSidesB sides_b = read_argument<OwnSidesB>(kGmpLoraArgsOffset + kOwnBOffset);
+#pragma unroll
+                for (int j = 0; j < kOwnTiles; ++j) {
+                    const void *at;
+                    b_live[j] = own_b_unit(sides_b, tt * kTileN + c, own.lo + 16 * j + 4 * q4, &at);
+                    b_own[j] = *reinterpret_cast<const u32x2 *>(at);
+                }
+            }
+            u32x4 b_op = {0u, 0u, 0u, 0u};
+#pragma unroll
+            for (int j = 0; j < kOwnTiles; ++j) {
+                b_op[2 * j] = b_live[j] ? b_own[j].x : 0u;
+                b_op[2 * j + 1] = b_live[j] ? b_own[j].y : 0u;
+            }
+            sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, t_own), __builtin_bit_cast(bf16x8, b_op), sum, 0, 0, 0);
+        }
         if (KS > 1 && flagged) {
             // The slices of the tile meet in a part of the workspace that is all zero between
             // launches.  A word there is either zero (not written yet) or the complement of a
@@ -640,9 +845,25 @@ size_t gmp_adapter_lds_bytes(const DecodeArgs &a) {
     return kGmpSyncBytes + b_bytes + (size_t)a.lora_slices * a.lora_rows * rp * 2 + 1024;
 }
 
-int gmp_slot_bytes(int gpw, int tiles) {
-    const int a = gmp_slots(gpw) * kGmpSlotBytes, r = tiles * 1024;
+// own: rank tiles the block projects x onto by itself
+int gmp_slot_bytes(int gpw, int tiles, int own) {
+    const int a = (gmp_slots(gpw) + own) * kGmpSlotBytes, r = (tiles + own) * 1024;
     return a > r ? a : r;
+}
+
+// Where the second and the third of the adapters' sides begin, in tiles and in blocks: a block has columns of one of them.
+struct GmpBorders {
+    int end0, blocks0, end1, blocks1;
+};
+[[maybe_unused]] GmpBorders own_borders(const DecodeArgs &a) {
+    const AdapterSides &s = *a.lora_sides;
+    const int NT = a.N / kTileN, T = a.gm_tiles;
+    GmpBorders b{NT, 0, NT, 0};
+    if (!s.interleaved && s.count > 1) b.end0 = s.first[1] / kTileN;
+    if (!s.interleaved && s.count > 2) b.end1 = s.first[2] / kTileN;
+    b.blocks0 = (b.end0 + T - 1) / T;
+    b.blocks1 = b.blocks0 + (b.end1 - b.end0 + T - 1) / T;
+    return b;
 }
 
 template <int T, int GPW, int AQ>
@@ -651,10 +872,23 @@ hipError_t launch_gmp_tga(const DecodeArgs &a, hipStream_t stream) {
     if (attr != hipSuccess) return attr;
     const int NT = a.N / kTileN;
     const int full_waves = a.GS - a.waves * (GPW - 1);
-    const int slot = gmp_slot_bytes(GPW, T);
-    const int col_blocks = (NT + T - 1) / T;
+    const int slot = gmp_slot_bytes(GPW, T, kOwnTiles);
+    int col_blocks = (NT + T - 1) / T;
+    uint32_t in_upper[4] = {0u, 0u, 0u, 0u};  // of G, NT, GS and the column blocks
+    if constexpr (kOwnTiles > 0) {
+        const GmpBorders b = own_borders(a);
+        col_blocks = b.blocks1 + (NT - b.end1 + T - 1) / T;
+        in_upper[0] = (uint32_t)b.blocks0 << 16;
+        in_upper[1] = (uint32_t)b.end0 << 16;
+        in_upper[2] = (uint32_t)b.end1 << 16;
+        in_upper[3] = (uint32_t)b.blocks1 << 16;
+    }
     GmpFold fold{};
-    if (a.lora_producers > 0) {
+    if constexpr (kOwnTiles > 0) {
+#if KILN_GMP_LORA >= 3
+        fold.own = own_args(a);
+#endif
+    } else if (a.lora_producers > 0) {
         fold.a_cat = (const uint16_t *)a.lora_a;
         fold.t = (uint16_t *)const_cast<void *>(a.lora_t);
         fold.flags = a.lora_flags;
@@ -675,14 +909,14 @@ hipError_t launch_gmp_tga(const DecodeArgs &a, hipStream_t stream) {
 #endif
     }
     const dim3 grid = fold.producers > 0 ? dim3(fold.producers + col_blocks * a.KS, 1) : dim3(col_blocks, a.KS);
-    const int adapter = a.r_total > 0 ? 1 : 0;  // one wavefront more: it fetches the low-rank term's operands
-    const size_t lds_bytes = (size_t)a.waves * slot + gmp_adapter_lds_bytes(a);
+    const int adapter = kGmpLora && a.r_total > 0 ? 1 : 0;  // one wavefront more: it fetches the low-rank term's operands
+    const size_t lds_bytes = (size_t)a.waves * slot + (kOwnTiles > 0 ? kOwnScaleBytes : gmp_adapter_lds_bytes(a));
     const uint32_t bits = (a.Gs == 1 ? kGmpColumnScales : 0u) | (adapter ? kGmpAdapter : 0u) | (a.swiglu ? kGmpSwiglu : 0u) |
                           (a.flagged ? kGmpFlagged | (exchange_column_shift(col_blocks) ? kGmpColShift : 0u) : 0u);
     w4a16_decode_gmp_kernel<T, GPW, AQ, kGmpLora><<<grid, (a.waves + adapter) * 64, lds_bytes, stream>>>(
         (const uint16_t *)a.A, (const u32x4 *)a.B, (const uint16_t *)a.S,
-        gmp_shape_word(a.M, full_waves, a.waves + adapter, a.KS), gmp_layout_word(slot, fold.producers, bits), a.K / kGroupK,
-        NT, a.GS, col_blocks, (uint16_t *)a.C, a.partial, a.counters, GmpLoraArgs{lora_tail(a), fold});
+        gmp_shape_word(a.M, full_waves, a.waves + adapter, a.KS), gmp_layout_word(slot, fold.producers, bits), a.K / kGroupK | in_upper[0],
+        NT | in_upper[1], a.GS | in_upper[2], col_blocks | in_upper[3], (uint16_t *)a.C, a.partial, a.counters, GmpLoraArgs{lora_tail(a), fold});
     return hipGetLastError();
 }
 
@@ -717,13 +951,17 @@ hipError_t launch_gmp_t(const DecodeArgs &a, int gpw, hipStream_t stream) {
 
 #if KILN_GMP_LORA
 // The instances with the low-rank term; the caller (launch_decode_gmp) has checked the plan.
-#if KILN_GMP_LORA == 2
+#if KILN_GMP_LORA == 3
+hipError_t launch_decode_gmp_own1(const DecodeArgs &a, hipStream_t stream) {
+#elif KILN_GMP_LORA == 4
+hipError_t launch_decode_gmp_own2(const DecodeArgs &a, hipStream_t stream) {
+#elif KILN_GMP_LORA == 2
 hipError_t launch_decode_gmp_sides(const DecodeArgs &a, hipStream_t stream) {
     if (!a.lora_sides) return hipErrorInvalidValue;
 #else
 hipError_t launch_decode_gmp_lora(const DecodeArgs &a, hipStream_t stream) {
 #endif
-    if (a.r_total <= 0) return hipErrorInvalidValue;  // these instances count on the adapter wavefront
+    if (a.r_total <= 0 || a.own_tiles != kOwnTiles) return hipErrorInvalidValue;  // these instances count on the adapter wavefront
     const int gpw = (a.GS + a.waves - 1) / a.waves;
     switch (a.gm_tiles) {
         case 1: return launch_gmp_t<1>(a, gpw, stream);
@@ -741,7 +979,9 @@ hipError_t launch_decode_gmp_lora(const DecodeArgs &a, hipStream_t stream) {
 bool decode_gmp_ok(const DecodeArgs &a) {
     const int G = a.K / kGroupK;
     if (a.M < 1 || a.M > 16 || a.gm_tiles < 1 || a.gm_tiles > 6) return false;
-    if (a.r_total > 0) {
+    if (a.own_tiles > 0) {  // (a wavefront of its own for the adapters, T and its words: none of these)
+        if (a.N / kTileN > 0xFFFF || G > 0xFFFF || a.own_tiles > 2 || a.r_total < 1 || a.r_total > 64 || !a.lora_sides || a.lora_adapters < 1 || a.lora_adapters > kLoraSidesMaxAdapters) return false;
+    } else if (a.r_total > 0) {
         // the low-rank term's operands are read from LDS in 16-byte pieces by one wavefront more than the
         // main loop uses; T is whole and belongs to exactly this launch's rows (with the fused gate/up
         // store the rows of lora_b are in the packed column order, so nothing changes here)
@@ -751,10 +991,12 @@ bool decode_gmp_ok(const DecodeArgs &a) {
     }
     if (a.KS < 1 || a.KS > 255 || a.GS < 1 || a.KS * a.GS != G || a.waves < 1 || a.waves > kGmpMaxWaves || a.waves > a.GS) return false;
     const int gpw = (a.GS + a.waves - 1) / a.waves, T = a.gm_tiles;
+    if (a.waves > gmp_max_waves(gpw, a.own_tiles)) return false;
     if (gpw > (T <= 2 ? 6 : 3) || T * gpw > kGmpMaxChunks) return false;
     const int full_waves = a.GS - a.waves * (gpw - 1);
     if (full_waves < 1 || full_waves > a.waves) return false;
-    return (size_t)a.waves * gmp_slot_bytes(gpw, T) + gmp_adapter_lds_bytes(a) <= (size_t)decode_max_lds_bytes();
+    return (size_t)a.waves * gmp_slot_bytes(gpw, T, a.own_tiles) + (a.own_tiles > 0 ? kOwnScaleBytes : gmp_adapter_lds_bytes(a)) <=
+           (size_t)decode_max_lds_bytes();
 }
 
 // The projection folded into the launch: one producer block per K slice of it, each with at least
@@ -768,7 +1010,7 @@ bool decode_gmp_fold_ok(const DecodeArgs &a) {
         a.lora_rows != a.M || a.lora_adapters < 1 || a.lora_adapters > (a.lora_sides ? kLoraSidesMaxAdapters : kLoraFoldMaxAdapters)) return false;
     if (a.KS > 4) return false;  // the kernel finds a block's slice in a one-row grid by three comparisons
     const int gpw = (a.GS + a.waves - 1) / a.waves;
-    return gmp_slot_bytes(gpw, a.gm_tiles) >= 1024;
+    return gmp_slot_bytes(gpw, a.gm_tiles, 0) >= 1024;
 }
 
 hipError_t launch_decode_gmp(const DecodeArgs &a, hipStream_t stream) {
@@ -776,6 +1018,7 @@ hipError_t launch_decode_gmp(const DecodeArgs &a, hipStream_t stream) {
     if (a.KS > 1 && (!a.partial || !a.counters)) return hipErrorInvalidValue;
     if (a.flagged && a.KS > kGmpFlaggedSlices) return hipErrorInvalidValue;
     if (a.lora_producers > 0 && !decode_gmp_fold_ok(a)) return hipErrorInvalidValue;
+    if (a.own_tiles > 0) return a.own_tiles == 1 ? launch_decode_gmp_own1(a, stream) : launch_decode_gmp_own2(a, stream);
     if (a.lora_sides) return launch_decode_gmp_sides(a, stream);
     if (a.r_total > 0) return launch_decode_gmp_lora(a, stream);
     const int gpw = (a.GS + a.waves - 1) / a.waves;
@@ -798,6 +1041,10 @@ hipError_t launch_decode_gmp(const DecodeArgs &a, hipStream_t stream) {
 extern "C" int kiln_gmp_timeline_lora(long long *buf) {
 #elif KILN_GMP_LORA == 2
 extern "C" int kiln_gmp_timeline_sides(long long *buf) {
+#elif KILN_GMP_LORA == 3
+extern "C" int kiln_gmp_timeline_own1(long long *buf) {
+#elif KILN_GMP_LORA == 4
+extern "C" int kiln_gmp_timeline_own2(long long *buf) {
 #else
 extern "C" int kiln_gmp_timeline(long long *buf) {
 #endif

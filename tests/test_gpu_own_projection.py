@@ -1,0 +1,106 @@
+"""Calls of up to 16 rows whose blocks project x onto their adapters by themselves, every instance, against the product in
+64 bits and the projection in a launch of its own; and where adapters are taken that way."""
+import ctypes
+
+import pytest
+import torch
+
+from kiln_amd import _lib, lora, marlin_gemm
+from tests.test_gpu_adapter_sides import Side, _all_adapters, _packed
+
+
+def _instances():
+    """(tiles per block, wavefronts, groups of a slice, K slices, ranks): groups per wavefront even and uneven, one wavefront
+    for several tiles, one and two rank tiles, ranks that fill a load of four rows or a tile and those that do not."""
+    cases = []
+    for tiles in range(1, 7):
+        for waves, gs, ks in ((1, 1, 1), (3, 3, 2), (8, 20, 1), (12, 12, 1), (12, 24, 3), (10, 20, 1), (7, 20, 1), (8, 32, 1), (10, 50, 1)):
+            gpw = -(-gs // waves)
+            if gpw > (6 if tiles <= 2 else 3) or tiles * gpw > 16:
+                continue
+            for r in (4, 12) if (tiles + gs) % 2 else (20, 28):
+                own, slots = (r + 15) // 16, min(gpw, 2)
+                if waves <= min(16, (160 * 1024 - 128) // ((slots + own) * 4096)):
+                    cases.append((tiles, waves, gs, ks, r))
+    return cases
+
+
+def _reference(x, w, sets):
+    """(result, low-rank term) in 64 bits; sets: (StackedLora or None, first column) of each projection"""
+    base = x.double() @ marlin_gemm.dequant_f32(w.b_packed, w.scales, w.groupsize).double()
+    low = torch.zeros_like(base)
+    for s, first in sets:
+        col = 0
+        for r, scale in zip(s.ranks, s.scales) if s is not None else ():
+            low[:, first:first + s.b_cat.shape[0]] += scale * (x.double() @ s.a_cat[col:col + r].double().t()) @ s.b_cat[:, col:col + r].double().t()
+            col += r
+    return base + low, low
+
+
+def _assert_close(y, want, low):
+    # the result rounded once to bf16 and T once per slice of K, half an ulp each: 2^-8 of a row of either at most
+    assert bool(((y.double() - want).norm(dim=1) <= 2.0 ** -8 * (want.norm(dim=1) + low.norm(dim=1))).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tiles,waves,gs,ks,r", _instances())
+def test_every_instance(tiles, waves, gs, ks, r):
+    L, k, n = _lib.load_tuning(), gs * ks * 128, 512
+    gen = torch.Generator(device="cuda").manual_seed(tiles * k + r)
+    w = _packed(gen, k, n, 128 if gs % 2 == 0 else -1)
+    # several adapters with scales of their own, zero among them
+    ad, = _all_adapters(gen, k, (n,), ((r,) if r == 4 else (r - 9, 1, 8),))
+    ad = lora.StackedLora(ad.a_cat, ad.b_cat, ad.ranks, ad.scales[:-1] + (0.0,) if r > 4 else ad.scales)
+    for m in (1, 4, 5, 8, 11, 16):
+        x = torch.randn(m, k, device="cuda", generator=gen).bfloat16()
+        L.kiln_w4a16_debug_gmp(tiles, waves, ks)
+        L.kiln_w4a16_debug_lora_fold(3)
+        assert L.kiln_w4a16_takes_rank(m, n, k, r, -1) == 1
+        got = marlin_gemm.marlin_w4a16_gemm_lora(x, w.b_packed, w.scales, w.groupsize, ad.a_cat, ad.b_cat, ad.ranks, ad.scales)
+        L.kiln_w4a16_debug_gmp(0, 0, 0)
+        L.kiln_w4a16_debug_lora_fold(0)
+        other = marlin_gemm.marlin_w4a16_gemm_lora(x, w.b_packed, w.scales, w.groupsize, ad.a_cat, ad.b_cat, ad.ranks, ad.scales)
+        want, low = _reference(x, w, [(ad, 0)])
+        _assert_close(got, want, low)
+        _assert_close(other, want, low)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [1, 7, 16])
+@pytest.mark.parametrize("k,widths,ranks", [
+    (512, (256, 512, 256), (None, (8, 8), (8, 8, 8))),         # columns of no side; blocks of one side's ranks
+    (1024, (1280, 256, 256), ((16, 16), (8,), (8, 8))),        # a side of two rank tiles
+    (4608, (256, 768, 256), ((8, 8), (8, 8), (8, 8))),         # K slices
+    (640, (256, 256, 256), ((8,), (16,), (8,))),               # up to four adapters: every block has all of them
+])
+def test_more_than_four_adapters_side_by_side(k, widths, ranks, m):
+    L, n = _lib.load_tuning(), sum(widths)
+    gen = torch.Generator(device="cuda").manual_seed(k + m)
+    w = _packed(gen, k, n, 128)
+    adapters = _all_adapters(gen, k, widths, ranks)
+    x = torch.randn(m, k, device="cuda", generator=gen).bfloat16()
+    x[-1, 3] = float("inf")  # one row's infinity stays in its row
+    firsts = [sum(widths[:i]) for i in range(len(widths))]
+    own = [(a, f) for a, f in zip(adapters, firsts) if a is not None]
+    sides = (Side * len(own))(*(Side(a.a_cat.data_ptr(), a.b_cat.data_ptr(), a.a_cat.shape[0], f, a.b_cat.shape[0]) for a, f in own))
+    each, scales = sum((a.ranks for a, _ in own), ()), sum((a.scales for a, _ in own), ())
+    stream = torch.cuda.current_stream().cuda_stream
+    want, low = _reference(x[:-1], w, list(zip(adapters, firsts)))
+    for plan in ((0, 0, 0), (5, 4, 1), (3, 4, 1)) if k < 4608 else ((0, 0, 0), (5, 9, 2), (3, 6, 2)):
+        L.kiln_w4a16_debug_gmp(*plan)
+        L.kiln_w4a16_debug_lora_fold(3)
+        ws = marlin_gemm._workspace(x.device, stream, L.kiln_w4a16_workspace_bytes(m, n, k))
+        out = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+        assert L.kiln_w4a16_gemm_adapter_sides(x.data_ptr(), w.b_packed.data_ptr(), out.data_ptr(), w.scales.data_ptr(), m, n, k, ws.data_ptr(), 128,
+                                               x.device.index, stream, sides, len(own), 0, len(each), (ctypes.c_int * len(each))(*each),
+                                               (ctypes.c_float * len(each))(*scales)) == _lib.OK
+        _assert_close(out[:-1], want, low)
+        assert not bool(out[-1].isfinite().any())
+
+
+def test_ranks_that_are_taken_as_they_are():
+    """Multiples of 8 always; of 4 where blocks project by themselves, up to 32 and 16 rows; nothing else."""
+    takes = _lib.load().kiln_w4a16_takes_rank
+    assert [r for r in range(0, 67) if takes(4, 2560, 2560, r, -1)] == sorted({4, 12, 20, 28} | set(range(8, 65, 8)))
+    assert [m for m in (0, 1, 16, 17, 64) if takes(m, 2560, 2560, 12, -1)] == [1, 16]
+    assert takes(4, 2560, 2500, 12, -1) == takes(4, 100, 2560, 12, -1) == 0  # no shape of the kernels
