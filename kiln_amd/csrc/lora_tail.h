@@ -95,9 +95,8 @@ __device__ __forceinline__ void lora_add_from_lds(f32x4 &v, const LoraTail &lo, 
 // projection, which the stacked form takes inside for four at most.  (A layer at 11 rows, two adapters of rank 8 on each
 // projection, 2560 / 9216 wide: 41.2 -> 33.1 us, four launches instead of seven.  On the mid-M kernel, six launches -> four:
 // at 20 / 50 / 100 rows 52.4 -> 46.7 / 63.0 -> 57.0 / 87.7 -> 82.0 us; 1536 / 5120 wide 47.3 -> 42.0 / 48.6 -> 44.0 / 58.7 -> 53.0.)
-// Not all of what goes is won: the gate | up launch alone takes 10.6 us at 11 rows where it took 9.2 behind the launch that
-// stacked (3.4).  Why is not known: that launch had just read A and B, which left them in the caches, and the row of A is
-// found here through a choice per lane.
+// (The gate | up launch alone then took 10.6 us at 11 rows where it took 9.2 behind the launch that stacked: its adapter
+// wavefront waited for the rows of B before it looked at the producers' flags, which it does no longer.)
 struct LoraSides {
     const uint16_t *a[kMaxAdapterSides];
     const uint16_t *b[kMaxAdapterSides];
@@ -107,6 +106,13 @@ struct LoraSides {
     int count;
     int interleaved;
 };
+// A value in a scalar register of its own (a choice between an argument's members would otherwise become one between their
+// addresses, in scratch memory).
+template <class V>
+__device__ __forceinline__ V scalar(V v) {
+    asm("" : "+s"(v));
+    return v;
+}
 // the row of A of a rank column
 __device__ __forceinline__ const uint16_t *side_a_row(const LoraSides &s, int rank, int K) {
     const uint16_t *base = s.a[0];
@@ -119,17 +125,24 @@ __device__ __forceinline__ const uint16_t *side_a_row(const LoraSides &s, int ra
         }
     return base + (size_t)(rank - from) * K;
 }
-// eight rank columns from j8 on (a multiple of 8) of a column's row of B: zeros but where they are its own side's
-__device__ __forceinline__ u32x4 side_b_unit(const LoraSides &s, int column, int j8) {
-    u32x4 v = {0u, 0u, 0u, 0u};
+// Where eight rank columns from j8 on (a multiple of 8) of a column's row of B lie; not live: no side's.  Found without a branch.
+struct SideUnit {
+    const void *at;
+    bool live;
+};
+__device__ __forceinline__ SideUnit side_b_unit(const LoraSides &s, int column, int j8) {
+    uint64_t at = reinterpret_cast<uint64_t>(s.b[0]);
+    bool live = false;
 #pragma unroll
     for (int i = 0; i < kMaxAdapterSides; ++i) {
-        const int row = s.interleaved ? (column >> 4) * 8 + (column & 7) : column - s.first[i];
-        const bool mine = s.interleaved ? (column & 8) == s.first[i] : row >= 0 && row < s.rows[i];
-        if (i < s.count && mine && j8 >= s.col[i] && j8 < s.col[i + 1])
-            v = *reinterpret_cast<const u32x4 *>(s.b[i] + (size_t)row * (s.col[i + 1] - s.col[i]) + (j8 - s.col[i]));
+        const int row = s.interleaved ? (column >> 4) * 8 + (column & 7) : column - s.first[i], ranks = s.col[i + 1] - s.col[i];
+        const bool in_side = s.interleaved ? (column & 8) == s.first[i] : (uint32_t)row < (uint32_t)s.rows[i];
+        const bool mine = in_side & ((uint32_t)(j8 - s.col[i]) < (uint32_t)ranks);  // (never of a side past the last: no ranks)
+        const uint64_t b = scalar(reinterpret_cast<uint64_t>(s.b[i]));
+        at = mine ? b + (uint64_t)(uint32_t)(row * ranks + j8 - s.col[i]) * 2 : at;
+        live |= mine;
     }
-    return v;
+    return SideUnit{reinterpret_cast<const void *>(at), live};
 }
 inline LoraSides lora_sides(const AdapterSides *h) {
     LoraSides s{};

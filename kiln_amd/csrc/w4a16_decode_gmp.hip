@@ -151,27 +151,24 @@ __device__ __forceinline__ void copy_to_lds(unsigned lds_addr, const uint16_t *s
         load_to_lds_b128(src, (uint32_t)min(base + lane, units - 1) * 16u, lds_addr + (unsigned)base * 16u);
 }
 
-// The rows of B_cat of a block's tiles to LDS, [column][rank]; unstacked adapters' through registers, six 16-byte units per
-// lane in flight (five tiles and 32 rank columns: 320 units).
+// The rows of B_cat of a block's tiles to LDS, [column][rank], in flight when this returns.  Unstacked adapters': each lane's unit
+// from where its side's row lies, zeros written where a column has no such rank.  (Through registers, the wavefront waited
+// for the units before it looked at the producers' flags, 5.2 us with a side at a time behind a condition, 4.7 without: gate
+// | up of 2560 with two adapters of rank 8 a side at 11 rows 10.3 -> 9.7 -> 9.2 us, of 4096 19.5 -> 16.9.)
 template <class Sides>
 __device__ __forceinline__ void fetch_b_rows(const Sides &sides, const LoraTail &lo, unsigned char *dst, int first_tile, int tiles, int lane) {
-    const int per_row = lo.r_total >> 3, units = tiles * kTileN * per_row;
+    const uint32_t per_row = lo.r_total >> 3, units = tiles * kTileN * per_row;
+    const unsigned dst_addr = (unsigned)(size_t)(lds_ptr_t)dst;
     if constexpr (std::is_same_v<Sides, LoraSides>) {
-        for (int base = 0; base < units; base += 6 * 64) {
-            u32x4 v[6];
-#pragma unroll
-            for (int i = 0; i < 6; ++i) {
-                const int u = min(base + 64 * i + lane, units - 1), row = u / per_row;
-                v[i] = side_b_unit(sides, first_tile * kTileN + row, (u - row * per_row) * 8);
-            }
-#pragma unroll
-            for (int i = 0; i < 6; ++i) {
-                const int u = base + 64 * i + lane;
-                if (u < units) *reinterpret_cast<u32x4 *>(dst + u * 16) = v[i];
-            }
+        const uint32_t inverse = (0x10000u + per_row - 1) / per_row;  // u / per_row for the few hundred units there are
+        for (uint32_t base = 0; base < units; base += 64) {
+            const uint32_t u = base + lane, row = u * inverse >> 16;
+            const SideUnit unit = side_b_unit(sides, first_tile * kTileN + row, (u - row * per_row) * 8);
+            if (unit.live && u < units) load_to_lds_b128(unit.at, dst_addr + base * 16u);
+            else if (u < units) *reinterpret_cast<u32x4 *>(dst + u * 16) = u32x4{0u, 0u, 0u, 0u};
         }
     } else {
-        copy_to_lds((unsigned)(size_t)(lds_ptr_t)dst, lo.b + (size_t)first_tile * kTileN * lo.r_total, units, lane);
+        copy_to_lds(dst_addr, lo.b + (size_t)first_tile * kTileN * lo.r_total, units, lane);
     }
 }
 
@@ -225,13 +222,6 @@ struct OwnWindow {  // the stacked rank columns that the block's columns have a 
     hi = here2 ? s.col3 : hi;
     lo = min(lo, hi);
     return OwnWindow{lo, hi - lo};
-}
-// A member in a scalar register of its own (a choice between members would otherwise become one between their addresses, in
-// scratch memory).
-template <class V>
-__device__ __forceinline__ V scalar(V v) {
-    asm("" : "+s"(v));
-    return v;
 }
 // the row of A of a stacked rank column
 [[maybe_unused]] __device__ __forceinline__ const char *own_a_row(const OwnSidesA &s, int rank, uint32_t row_bytes) {

@@ -528,7 +528,9 @@ __device__ __forceinline__ void mid_block(
                 for (int p = 0; p < TP; ++p) {
                     const int col = min(tf + 2 * p, N / kTileN - 2) * kTileN + l32;
 #if KILN_MID_LORA == 2
-                    tb[p] = side_b_unit(lo.sides, col, j8);  // (zeros past the last side's rank)
+                    const SideUnit unit = side_b_unit(lo.sides, col, j8);  // (not live past the last side's rank)
+                    tb[p] = u32x4{0u, 0u, 0u, 0u};
+                    if (unit.live) tb[p] = *reinterpret_cast<const u32x4 *>(unit.at);
 #else
                     tb[p] = u32x4{0u, 0u, 0u, 0u};
                     if (live_rank) tb[p] = *reinterpret_cast<const u32x4 *>(lo.b + (size_t)col * lo.r_total + j8);
