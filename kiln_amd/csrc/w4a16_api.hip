@@ -696,13 +696,15 @@ constexpr OwnKind own_kind_of(int lora) {
 }
 
 // Does every block project x onto its adapters by itself, and by which plan?  Against the projection in the launch's first
-// blocks, whose chain of round trips ends 5.5 to 6 us after the launch begins (6.2 where the adapters are not stacked) but
-// runs beside the streaming blocks: a launch that takes longer than that hides it, where a block's own projection adds its
-// share of A_cat to what the block stages.  The two plans' costs and constants were fitted to both, forced, on 15 shapes with
-// stacked adapters of 8 to 32 ranks and on the four calls of a layer at hidden 1024, 1536, 2560 and 4096 with adapters of 16
-// and 8 ranks a projection, at 1 to 16 rows: 8.9 % less time over these 310 cases than the first blocks alone, where the
-// better of the two each time is 10 %; the worst loss is 7 % (4096 -> 4096 with 8 ranks at one row, 5.7 -> 6.1 us).  What a
-// rank that is no multiple of 8 would cost otherwise is a launch that pads it (3 us).
+// blocks, whose chain of round trips ends 5.5 to 6 us after the launch begins but runs beside the streaming blocks: a launch
+// that takes longer than that hides it, where a block's own projection adds its share of A_cat to what the block stages --
+// of its own side only, where more than four adapters lie side by side (kind.sides), which therefore goes further.  The lines
+// were fitted to both ways, forced, with both plans' costs: on 15 shapes with stacked adapters of 8 to 32 ranks and on the four
+// calls of a layer at hidden 1024, 1536, 2560 and 4096 with adapters of 16, 32 and 8 ranks a projection, at 1 to 16 rows.  The
+// choice takes 8 to 9 % less time than the first blocks alone, the better of the two each time 9 to 10 %; q | k | v of 2560 with two
+// adapters of rank 8 each at 11 rows 7.2 against 7.9 us, of 4096 with two of rank 4 9.6 against 10.3 the other way (kind.sides:
+// costs of 7.3 and 9.6); the worst loss is 7 % (4096 -> 4096 with 8 ranks at one row, 5.7 -> 6.1 us).  What a rank that is no
+// multiple of 8 would cost otherwise is a launch that pads it (3 us).
 bool plan_own_projection(int m, int n, int k, int cus, const OwnKind &kind, DecodePlan *own) {
     if (g_tune.gmp_tiles > 0)
         return (g_tune.gmp_ks == 1 || flagged_exchange_fits(g_tune.gmp_ks, n)) &&
@@ -712,7 +714,7 @@ bool plan_own_projection(int m, int n, int k, int cus, const OwnKind &kind, Deco
     DecodePlan other;
     if (g_tune.lora_fold == 3 || !plan_decode_gmp(m, n, k, cus, true, &other, 0, &first_blocks)) return true;
     if (kind.general) return cost <= std::max(first_blocks + 2.f, 8.f);
-    return cost <= (kind.sides ? std::max(first_blocks + 1.0f, 6.2f) : std::max(first_blocks - 0.5f, 5.6f));
+    return cost <= std::max(first_blocks - 0.5f, kind.sides ? 7.4f : 5.6f);
 }
 
 // lora: as choose_decode takes it, or an OwnKind
