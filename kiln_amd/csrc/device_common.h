@@ -127,4 +127,20 @@ __device__ __forceinline__ bf16x8 bf16x8_zero() {
     return __builtin_bit_cast(bf16x8, r);
 }
 
+// An argument behind the preloaded ones, read where it is needed.
+template <class V>
+__device__ __forceinline__ V read_argument(int offset) {
+    typedef const char __attribute__((address_space(4))) *kernarg_ptr_t;
+    typedef const uint32_t __attribute__((address_space(4))) *kernarg_words_t;
+    kernarg_ptr_t kernarg = (kernarg_ptr_t)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(kernarg));  // opaque: nothing read through it moves above this point
+    kernarg_words_t src = (kernarg_words_t)(kernarg + offset);
+    struct Words {
+        uint32_t w[sizeof(V) / 4];
+    } words;
+#pragma unroll
+    for (int i = 0; i < (int)(sizeof(V) / 4); ++i) words.w[i] = src[i];
+    return __builtin_bit_cast(V, words);
+}
+
 }  // namespace kiln

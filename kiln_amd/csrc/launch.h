@@ -156,6 +156,8 @@ struct MidArgs {
     const void *lora_a = nullptr;    // bf16 [r_total, K]
     const AdapterSides *lora_sides = nullptr;  // with lora_producers: the adapters where they lie, lora_a and lora_b are not read
     unsigned *lora_words = nullptr;  // 64 KiB that are zero between launches (lora_tail.h)
+    int own_tiles = 0;               // 1, 2: every block projects x onto the (up to 16, 32) rank columns of its own columns by
+                                     // itself; of the fields around this one r_total, lora_sides, adapters, ends and scales
     int lora_adapters = 0;           // 1...8
     int lora_ends[8] = {};           // exclusive end column of adapter i on the stacked rank axis
     float lora_scales[8] = {};
@@ -169,6 +171,8 @@ bool mid_plan_ok(const MidArgs &a);
 size_t mid_partial_bytes(const MidArgs &a);
 hipError_t launch_mid(const MidArgs &a, hipStream_t stream);
 hipError_t launch_mid_lora(const MidArgs &a, hipStream_t stream);  // its instances with the low-rank term (checked plan)
+hipError_t launch_mid_own1(const MidArgs &a, hipStream_t stream);   // ... with a projection of each block's own
+hipError_t launch_mid_own2(const MidArgs &a, hipStream_t stream);
 hipError_t launch_mid_sides(const MidArgs &a, hipStream_t stream);  // ... of unstacked adapters
 
 // One launch of the prefill path (row-sum pre-pass + MFMA kernel), any M >= 1.

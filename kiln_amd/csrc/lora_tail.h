@@ -87,6 +87,13 @@ __device__ __forceinline__ void lora_add_from_lds(f32x4 &v, const LoraTail &lo, 
     }
 }
 
+// A value in a scalar register of its own (a choice between an argument's members would otherwise become one between their
+// addresses, in scratch memory).
+template <class V>
+__device__ __forceinline__ V scalar(V v) {
+    asm("" : "+s"(v));
+    return v;
+}
 // The adapters of projections that run as one GEMM, where they lie: side i has A = bf16 [ranks, K] and B = bf16
 // [rows, ranks] of its own, ranks a multiple of 8, and the columns from col[i] on of the stacked rank axis.  Its rows of B
 // are the GEMM's columns from first[i] on; interleaved, those of every 16-column tile from first[i] (0: gate, 8: up) on,
@@ -106,13 +113,6 @@ struct LoraSides {
     int count;
     int interleaved;
 };
-// A value in a scalar register of its own (a choice between an argument's members would otherwise become one between their
-// addresses, in scratch memory).
-template <class V>
-__device__ __forceinline__ V scalar(V v) {
-    asm("" : "+s"(v));
-    return v;
-}
 // the row of A of a rank column
 __device__ __forceinline__ const uint16_t *side_a_row(const LoraSides &s, int rank, int K) {
     const uint16_t *base = s.a[0];
@@ -225,10 +225,56 @@ struct OwnArgs {
 struct LoraOwnFold : LoraFold {
     OwnArgs own;
 };
-inline OwnArgs own_args(const DecodeArgs &d) {
+// On the device, free of branches: it runs while the first weights are in flight to registers.
+struct OwnWindow {  // the stacked rank columns that the block's columns have a term of
+    int lo, ranks;
+};
+[[maybe_unused]] __device__ __forceinline__ OwnWindow own_window(const OwnSidesA &s, int first_column, int end_column) {
+    const bool here0 = (s.first0 < end_column) & (s.end0 > first_column), here1 = (s.first1 < end_column) & (s.end1 > first_column),
+               here2 = (s.first2 < end_column) & (s.end2 > first_column);
+    int lo = here2 ? s.col2 : s.col3, hi = here0 ? s.col1 : 0;
+    lo = here1 ? s.col1 : lo;
+    lo = here0 ? 0 : lo;
+    hi = here1 ? s.col2 : hi;
+    hi = here2 ? s.col3 : hi;
+    lo = min(lo, hi);
+    return OwnWindow{lo, hi - lo};
+}
+// the row of A of a stacked rank column
+[[maybe_unused]] __device__ __forceinline__ const char *own_a_row(const OwnSidesA &s, int rank, uint32_t row_bytes) {
+    const uint64_t a1 = scalar(s.a1), a2 = scalar(s.a2);
+    uint64_t base = scalar(s.a0);
+    base = rank >= s.col1 ? a1 : base;
+    base = rank >= s.col2 ? a2 : base;
+    return reinterpret_cast<const char *>(base + (uint64_t)(uint32_t)rank * row_bytes);
+}
+// Where four rank columns from `rank` on of a column's row of B_cat lie; false (and an address that can be read): no term.
+[[maybe_unused]] __device__ __forceinline__ bool own_b_unit(const OwnSidesB &s, int column, int rank, const void **at) {
+    const int key = column & s.key_mask, row = ((column & ~15) >> s.row_shift) + (column & s.low_mask);
+    uint64_t p = scalar(s.b0);
+    int from = 0;
+    bool live = false;
+    auto side = [&](uint64_t b, int first, int span, int col, int end) {
+        const int width = end - col;
+        const bool mine = ((uint32_t)(key - first) < (uint32_t)span) & ((uint32_t)(rank - col) < (uint32_t)width);
+        p = mine ? b : p;
+        // (of 24 bits: cheap enough that the compiler forms it for every side instead of behind a branch)
+        const int at_unit = __mul24(row - __mul24(first, s.row_counts_from_first), width) + rank - col;
+        from = mine ? at_unit : from;
+        live |= mine;
+    };
+    side(scalar(s.b0), s.first0, s.span0, 0, s.col1);
+    side(scalar(s.b1), s.first1, s.span1, s.col1, s.col2);
+    side(scalar(s.b2), s.first2, s.span2, s.col2, s.col3);
+    *at = reinterpret_cast<const void *>(p + (uint64_t)(uint32_t)from * 2);
+    return live;
+}
+template <class Args>  // DecodeArgs, MidArgs
+OwnArgs own_args(const Args &d) {
     const AdapterSides &h = *d.lora_sides;
-    // Up to four adapters give the bits of the stacked set (kLoraFoldMaxAdapters): every block has all ranks, in their places.
-    const bool all = h.interleaved || d.lora_adapters <= kLoraFoldMaxAdapters;
+    // Up to four adapters, and any number beyond 16 rows, give the bits of the stacked set: every block has all ranks, in
+    // their places.
+    const bool all = h.interleaved || d.lora_adapters <= kLoraFoldMaxAdapters || d.M > 16;
     uint64_t a[3] = {}, b[3] = {};
     int col[4] = {}, first[3] = {}, end[3] = {}, key[3] = {}, span[3] = {};
     for (int i = 0; i < kMaxAdapterSides; ++i) {
@@ -251,6 +297,18 @@ inline OwnArgs own_args(const DecodeArgs &d) {
         o.scales.scales[i] = d.lora_scales[i];
     }
     return o;
+}
+// Where the second and the third side begin, in tiles and in blocks of T tiles: a block has columns of one of them.
+struct OwnBorders {
+    int end0, blocks0, end1, blocks1;
+};
+inline OwnBorders own_borders(const AdapterSides &s, int NT, int T) {
+    OwnBorders b{NT, 0, NT, 0};
+    if (!s.interleaved && s.count > 1) b.end0 = s.first[1] / kTileN;
+    if (!s.interleaved && s.count > 2) b.end1 = s.first[2] / kTileN;
+    b.blocks0 = (b.end0 + T - 1) / T;
+    b.blocks1 = b.blocks0 + (b.end1 - b.end0 + T - 1) / T;
+    return b;
 }
 constexpr int kLoraFoldMaxProducers = 16;
 constexpr int kLoraSidesMaxAdapters = 8;

@@ -468,6 +468,7 @@ struct MidPlan {
     int KS = 1, GS = 0, waves = 0, pairs = 1;
     float cost = 0.f;
     bool fold = true;  // with adapters: the projection in the launch's first blocks (where the launch can)
+    int own = 0;       // ... or rank tiles every block projects x onto by itself
 };
 struct GemmPlan {
     bool prefill = false;
@@ -475,6 +476,8 @@ struct GemmPlan {
     bool sums_in_loop = false;  // PrefillArgs::sums_in_loop
     bool mid = false;
     MidPlan mp{};
+    bool own_sides = false;     // blocks that project x by themselves: unstacked adapters too (those calls that the kernels
+                                // with the projection in their first blocks take)
     int launches = 0;
     DecodeLaunch dl[kMaxDecodeLaunches];
     size_t decode_partial = 0;  // bytes of partial tiles the largest launch exchanges
@@ -605,7 +608,8 @@ bool mid_flagged(const MidArgs &a) {
 // 40 rows, 4096 -> 11008 at 17: three pairs in two slices where two pairs unsliced would lead).  Eight
 // narrow outputs of a long K swept afterwards (4096 -> 512 ... 8192 -> 3072 at 24, 64 and 128 rows): within
 // 4 % of the best plan but on 6144 -> 1536 (6...12 %: 12 groups dealt to 8 wavefronts count as 16).
-MidPlan plan_mid_waves(int m, int n, int k, int cus, bool lora, bool ten_beyond_32_rows) {
+// eights > 0: a plan whose blocks project x onto this many times eight ranks by themselves (lora is false).
+MidPlan plan_mid_waves(int m, int n, int k, int cus, bool lora, bool ten_beyond_32_rows, int eights = 0) {
     MidPlan best;
     const int G = k / kGroupK, runs = ceil_div(m, mid_max_rows_per_run());
     for (int pairs = 1; pairs <= 3; ++pairs) {
@@ -633,10 +637,13 @@ MidPlan plan_mid_waves(int m, int n, int k, int cus, bool lora, bool ten_beyond_
             // unsliced, 9216 -> 2560 13.1 -> 12.0 and 8192 -> 8192 21.0 -> 19.8 in two slices, but 13824 -> 5120 in three
             // slices of 6 x 4 + 4 x 3 groups 22.2 against 20.0 in four slices of eight wavefronts)
             if (lora && ks > 2) max_waves = 8;
+            a.own_tiles = (eights + 1) / 2;
+            if (eights > 0) max_waves = std::min(max_waves, eights > 2 ? 6 : 8);  // (LDS)
             if (g_tune.mid_waves > 0) max_waves = std::min(g_tune.mid_waves, mid_max_waves(m, pairs, lora));
             a.waves = a.GS < max_waves ? a.GS : max_waves;
             a.pairs = pairs;
             if (!mid_plan_ok(a)) continue;
+            if (eights > 0 && ks > 1 && !mid_flagged(a)) continue;  // (no workspace beyond what the call has anyway)
             const int col_blocks = mid_column_blocks(a);
             if ((size_t)runs * col_blocks * sizeof(int) > kCounterCapacity) continue;
             const int gpw = ceil_div(a.GS, a.waves), rounds = ceil_div(col_blocks * ks * runs, cus);
@@ -645,13 +652,17 @@ MidPlan plan_mid_waves(int m, int n, int k, int cus, bool lora, bool ten_beyond_
             // 26.6 us in six even slices and 28.4...30.1 in five of 22 + 22 + 22 + 22 + 20 groups, which this model
             // would prefer by the 1.7 us of a slice's exchange)
             const float uneven = G % ks != 0 ? 2.0f : 0.f;
-            const float cost = rounds * gpw * (0.75f + 0.55f * pairs) + 4.5f + exchange + 2.0f * (rounds - 1) + uneven;
+            // (a block's own projection: the rows of A_cat and their products in every group step, the more of them the
+            // fewer wavefronts there are to overlap with)
+            const float own = eights == 0 ? 0.f : (m <= 32 ? 0.2f : 0.35f) + 0.05f * eights + 0.2f * (pairs - 1);
+            const float cost = rounds * gpw * (0.75f + 0.55f * pairs + own) + 4.5f + exchange + 2.0f * (rounds - 1) + uneven;
             if (!best.ok || cost < best.cost) {
                 best.ok = true;
                 best.KS = ks;
                 best.GS = a.GS;
                 best.waves = a.waves;
                 best.pairs = pairs;
+                best.own = a.own_tiles;
                 best.cost = cost;
             }
         }
@@ -677,6 +688,7 @@ MidArgs mid_args(const MidPlan &mp, int m, int n, int k) {
     a.GS = mp.GS;
     a.waves = mp.waves;
     a.pairs = mp.pairs;
+    a.own_tiles = mp.own;
     a.flagged = mid_flagged(a);
     return a;
 }
@@ -717,9 +729,45 @@ bool plan_own_projection(int m, int n, int k, int cus, const OwnKind &kind, Deco
     return cost <= std::max(first_blocks - 0.5f, kind.sides ? 7.4f : 5.6f);
 }
 
+// The plan of the mid-M kernel with the projection in the launch's first blocks where they fit (its fold), or in front.
+MidPlan plan_mid_lora(int m, int n, int k, int cus) {
+    // with adapters the projection runs in the launch's first blocks: plan for the chip less those
+    const int producers = g_tune.lora_fold != 0 ? ceil_div(m, 16) * lora_project_slices(m, k) : 0;
+    MidPlan mp = plan_mid(m, n, k, cus > 2 * producers ? cus - producers : cus, true);
+    // ... unless the plan for the whole chip is ahead by more than the projection's own launch costs (3 us: what
+    // calls of one plan either way differ by) -- where the product's blocks just fill the chip, the producers push
+    // the plan into another round or another shape: 2560 -> 12288 with two adapters at 128 rows, 128 blocks
+    // of three pairs per run, 26.6 us folded against 22.7 in front; 3584 -> 37888 at 96 rows 81 against 68
+    if (producers > 0 && cus > 2 * producers && g_tune.lora_fold != 2) {
+        MidPlan whole = plan_mid(m, n, k, cus, true);
+        if (whole.ok && (!mp.ok || whole.cost + 3.0f < mp.cost)) {
+            whole.fold = false;
+            mp = whole;
+        }
+    }
+    return mp;
+}
+
+// As plan_own_projection, on the mid-M kernel: there the projection in the first blocks ends 8 us and more after the launch
+// begins, and the launches that are shorter than that without adapters gain most.  Fitted to both ways, forced, on the
+// four calls of a layer at hidden 1024, 1536, 2560 and 4096 with adapters of 8 to 32 ranks at 20, 32, 50, 64 and 100 rows: 14 % less time
+// than the first blocks alone where both exist, the better of the two each time 14.5 % (2048 -> 1024 with 16 ranks at 32 rows 8.2 -> 5.9
+// us, 1024 -> 5632 with 16 9.0 -> 5.4, 9216 -> 2560 at 50 15.1 -> 14.0; 2560 -> 18432 at 20 11.7 against 12.0 the other way, and at 50,
+// where three pairs leave no registers for T and two take another round, 16.5 against 25).
+bool plan_mid_own_projection(int m, int n, int k, int cus, const OwnKind &kind, MidPlan *own) {
+    *own = plan_mid_waves(m, n, k, cus, false, false, kind.eights);
+    if (!own->ok || g_tune.lora_fold == 3) return own->ok;
+    const MidPlan other = plan_mid_lora(m, n, k, cus);
+    if (!other.ok) return true;
+    return own->cost <= (kind.general ? std::max(other.cost + 2.f, 11.5f) : std::max(other.cost + 0.2f, 9.55f));
+}
+
+bool first_blocks_take_sides(int m, int n, int k, int cus);
+
 // lora: as choose_decode takes it, or an OwnKind
 void plan_gemm(int m, int n, int k, int cus, int thread_k, int thread_n, int lora, GemmPlan *gp) {
     *gp = GemmPlan{};
+    const bool prefill_pinned = g_tune.prefill_bm != 0 || g_tune.prefill_bn != 0 || g_tune.prefill_ks != 0 || g_tune.prefill_nb_full >= 0;
     if (lora >= kFirstOwnKind) {
         const OwnKind kind = own_kind_of(lora);
         DecodePlan own;
@@ -734,6 +782,14 @@ void plan_gemm(int m, int n, int k, int cus, int thread_k, int thread_n, int lor
             l.plan = own;
             l.direct = false;
             gp->decode_partial = decode_launch_partial_bytes(l, n, k);
+            gp->own_sides = first_blocks_take_sides(m, n, k, cus);
+            return;
+        }
+        if (m > 16 && thread_k <= 0 && thread_n <= 0 && !prefill_pinned && g_tune.prefill_min_m == 0 && g_tune.mid != 0 &&
+            (g_tune.mid == 1 || (m >= mid_min_rows(n, k, true) && m <= mid_max_rows(n, k, true))) &&
+            plan_mid_own_projection(m, n, k, cus, kind, &gp->mp)) {
+            gp->mid = true;
+            gp->own_sides = first_blocks_take_sides(m, n, k, cus);
             return;
         }
         lora = kind.general ? 2 : 1;
@@ -742,7 +798,6 @@ void plan_gemm(int m, int n, int k, int cus, int thread_k, int thread_n, int lor
     // adapters whose stacked rank is a multiple of 8: the low-rank term is added from a projection that runs
     // in the launch's first blocks where it fits, else from one launched in front)
     // (a call pinned to a block shape of the matrix-core kernel goes there)
-    const bool prefill_pinned = g_tune.prefill_bm != 0 || g_tune.prefill_bn != 0 || g_tune.prefill_ks != 0 || g_tune.prefill_nb_full >= 0;
     // (with adapters also below 17 rows where the small-M launch would have to take the projection from a launch in
     // front -- its blocks fill the chip and leave the producers no units of their own -- and this kernel need not:
     // 11008 -> 4096, 256 blocks of two tiles in two slices, with two adapters 15.3...17.0 us at 1...16 rows, here 13.9...14.4)
@@ -759,20 +814,7 @@ void plan_gemm(int m, int n, int k, int cus, int thread_k, int thread_n, int lor
         (g_tune.mid == 1 ||
          (!prefill_pinned && g_tune.prefill_min_m == 0 && (m >= mid_min_rows(n, k, lora != 0) || few_rows_here) &&
           m <= mid_max_rows(n, k, lora != 0)))) {
-        // with adapters the projection runs in the launch's first blocks: plan for the chip less those
-        const int producers = lora && g_tune.lora_fold != 0 ? ceil_div(m, 16) * lora_project_slices(m, k) : 0;
-        MidPlan mp = plan_mid(m, n, k, cus > 2 * producers ? cus - producers : cus, lora != 0);
-        // ... unless the plan for the whole chip is ahead by more than the projection's own launch costs (3 us: what
-        // calls of one plan either way differ by) -- where the product's blocks just fill the chip, the producers push
-        // the plan into another round or another shape: 2560 -> 12288 with two adapters at 128 rows, 128 blocks
-        // of three pairs per run, 26.6 us folded against 22.7 in front; 3584 -> 37888 at 96 rows 81 against 68
-        if (producers > 0 && cus > 2 * producers && g_tune.lora_fold != 2) {
-            MidPlan whole = plan_mid(m, n, k, cus, true);
-            if (whole.ok && (!mp.ok || whole.cost + 3.0f < mp.cost)) {
-                whole.fold = false;
-                mp = whole;
-            }
-        }
+        const MidPlan mp = lora ? plan_mid_lora(m, n, k, cus) : plan_mid(m, n, k, cus, false);
         if (mp.ok) {
             gp->mid = true;
             gp->mp = mp;
@@ -935,14 +977,14 @@ struct LoraSpec {
 
 // The `lora` of plan_gemm for a call: which kernels can take its adapters.  A block of up to 16 rows that projects x onto
 // the adapters by itself does so for all of them, or, where more than four lie side by side, for those that its columns have
-// a term of (up to four, the call is one with the stacked set in every bit: the same choice, plan and places).  Blocks end
-// where a side does, whole tiles.
+// a term of (up to four, the call is one with the stacked set in every bit: the same choice, plan and places; beyond 16 rows
+// it is whatever their number).  Blocks end where a side does, whole tiles.
 int lora_kind(const LoraSpec *lora, int m) {
     if (!lora) return 0;
     const int otherwise = lora->r_total % 8 == 0 ? 1 : 2;
-    if (m > 16 || (g_tune.lora_fold != -1 && g_tune.lora_fold != 3) || lora->r_total % 4 != 0) return otherwise;
+    if (m > 4 * mid_max_rows_per_run() || lora->n_adapters > 8 || (g_tune.lora_fold != -1 && g_tune.lora_fold != 3) || lora->r_total % 4 != 0) return otherwise;
     int ranks = lora->r_total;
-    const bool many = lora->sides && lora->n_adapters > 4;
+    const bool many = lora->sides && lora->n_adapters > 4 && m <= 16;
     if (lora->sides && !lora->sides->interleaved) {
         const AdapterSides &s = *lora->sides;
         if (many) ranks = *std::max_element(s.ranks, s.ranks + s.count);
@@ -1074,13 +1116,21 @@ bool mid_lora_in_launch(const GemmPlan &gp, const LoraSpec &lora, void *flags, M
 // private-staging and the mid-M kernel.
 bool sides_in_launch(const GemmPlan &gp, int m, int n, int k, int cus, const LoraSpec &lora, void *t, void *flags) {
     if (gp.prefill) return false;
-    if (!gp.mid && gp.dl[0].plan.own > 0) return true;
+    if (gp.mid ? gp.mp.own > 0 : gp.dl[0].plan.own > 0) return gp.own_sides;
     if (gp.mid) {
         MidArgs ask = mid_args(gp.mp, m, n, k);
         return mid_lora_in_launch(gp, lora, flags, &ask);
     }
     DecodeArgs ask{};
     return lora_in_launch(gp, m, k, cus, lora, t, flags, &ask);
+}
+
+bool first_blocks_take_sides(int m, int n, int k, int cus) {
+    static unsigned probe = 0;  // never dereferenced
+    const AdapterSides some{{&probe}, {&probe}, {8}, {0}, {n}, 1, 0};
+    GemmPlan gp;
+    plan_gemm(m, n, k, cus, -1, -1, 1, &gp);
+    return sides_in_launch(gp, m, n, k, cus, LoraSpec{nullptr, nullptr, 8, 1, nullptr, nullptr, &some}, &probe, &probe);
 }
 
 // The GEMM behind every entry point: small-M or matrix-core path by row count, with the
@@ -1163,9 +1213,14 @@ kiln_marlin_status_t gemm_any(const void *A, const void *B, void *C, const void 
             ma.lora_t = lora_t;
             ma.lora_b = lora->b;
             ma.r_total = lora->r_total;
-            // ... inside the product's launch where its blocks have the threads for it
+            // ... inside the product's launch where its blocks have the threads for it, or by every block itself
             MidArgs folded = ma;
-            if (mid_lora_in_launch(gp, *lora, ws + kFoldFlagOffset, &folded)) {
+            const AdapterSides stacked{{lora->a}, {lora->b}, {lora->r_total}, {0}, {prob_n}, 1, 0};
+            if (gp.mp.own > 0) {
+                folded.lora_sides = lora->sides ? lora->sides : &stacked;
+                folded.lora_adapters = lora->n_adapters;
+            }
+            if (gp.mp.own > 0 || mid_lora_in_launch(gp, *lora, ws + kFoldFlagOffset, &folded)) {
                 int end = 0;
                 for (int i = 0; i < 8; ++i) {
                     if (i < lora->n_adapters) end += lora->ranks[i];
@@ -1586,7 +1641,7 @@ int kiln_w4a16_takes_rank(int prob_m, int prob_n, int prob_k, int r_total, int d
     if (r_total % 8 == 0) return 1;
     const LoraSpec lora{nullptr, nullptr, r_total, 1, nullptr, nullptr};
     const auto planned = plan_call(prob_m, prob_n, prob_k, compute_units(dev), -1, -1, lora_kind(&lora, prob_m));
-    return planned->gp.launches == 1 && planned->gp.dl[0].plan.own > 0 ? 1 : 0;
+    return planned->gp.mid ? planned->gp.mp.own > 0 : planned->gp.launches == 1 && planned->gp.dl[0].plan.own > 0;
 }
 
 int kiln_w4a16_takes_adapter_sides(int prob_m, int prob_n, int prob_k, const kiln_w4a16_adapter_side *sides, int n_sides, int swiglu,

@@ -47,7 +47,7 @@ constexpr int kGmpSlotBytes = 16 * 256;  // one group of A: 16 rows x 128 bf16
 constexpr bool kGmpLora = KILN_GMP_LORA == 1 || KILN_GMP_LORA == 2, kGmpSides = KILN_GMP_LORA == 2;
 constexpr int kOwnTiles = KILN_GMP_LORA >= 3 ? KILN_GMP_LORA - 2 : 0;  // rank tiles a block projects x onto by itself
 #if KILN_GMP_LORA >= 3
-#define w4a16_decode_gmp_kernel w4a16_decode_gmp_own_kernel  // (the name profiles show)
+#define w4a16_decode_gmp_kernel w4a16_decode_gmp_kernel_own  // (the name profiles show)
 #endif
 using GmpFold = std::conditional_t<kGmpSides, LoraSidesFold, std::conditional_t<(kOwnTiles > 0), LoraOwnFold, LoraFold>>;
 
@@ -208,47 +208,6 @@ constexpr unsigned kGmpSyncBytes = 16;
 // 11 rows 8.2 -> 7.4, of 1024 -> 3072 / 1024 / 1024 at 16 rows 7.5 -> 4.3; rank 12, which those blocks read only padded by a
 // launch in front, 2560 -> 10240 at 16 rows 10.5 -> 7.3.  Beyond the launches the dispatcher's rule takes it loses: 2560 ->
 // 18432 with 32 ranks at one row 7.5 -> 9.8, 160 KiB of A_cat a block at 0.0125 us a KiB on top of the weights.
-// Everything below is free of branches: it runs while the first weights are in flight to registers.
-struct OwnWindow {  // the stacked rank columns that the block's columns have a term of
-    int lo, ranks;
-};
-[[maybe_unused]] __device__ __forceinline__ OwnWindow own_window(const OwnSidesA &s, int first_column, int end_column) {
-    const bool here0 = (s.first0 < end_column) & (s.end0 > first_column), here1 = (s.first1 < end_column) & (s.end1 > first_column),
-               here2 = (s.first2 < end_column) & (s.end2 > first_column);
-    int lo = here2 ? s.col2 : s.col3, hi = here0 ? s.col1 : 0;
-    lo = here1 ? s.col1 : lo;
-    lo = here0 ? 0 : lo;
-    hi = here1 ? s.col2 : hi;
-    hi = here2 ? s.col3 : hi;
-    lo = min(lo, hi);
-    return OwnWindow{lo, hi - lo};
-}
-// the row of A of a stacked rank column
-[[maybe_unused]] __device__ __forceinline__ const char *own_a_row(const OwnSidesA &s, int rank, uint32_t row_bytes) {
-    const uint64_t a1 = scalar(s.a1), a2 = scalar(s.a2);
-    uint64_t base = scalar(s.a0);
-    base = rank >= s.col1 ? a1 : base;
-    base = rank >= s.col2 ? a2 : base;
-    return reinterpret_cast<const char *>(base + (uint64_t)(uint32_t)rank * row_bytes);
-}
-// Where four rank columns from `rank` on of a column's row of B_cat lie; false (and an address that can be read): no term.
-[[maybe_unused]] __device__ __forceinline__ bool own_b_unit(const OwnSidesB &s, int column, int rank, const void **at) {
-    const int key = column & s.key_mask, row = ((column & ~15) >> s.row_shift) + (column & s.low_mask);
-    uint64_t p = scalar(s.b0), from = 0;
-    bool live = false;
-    auto side = [&](uint64_t b, int first, int span, int col, int end) {
-        const int width = end - col;
-        const bool mine = ((uint32_t)(key - first) < (uint32_t)span) & ((uint32_t)(rank - col) < (uint32_t)width);
-        p = mine ? b : p;
-        from = mine ? (uint64_t)(int64_t)((row - first * s.row_counts_from_first) * width + rank - col) * 2 : from;
-        live |= mine;
-    };
-    side(scalar(s.b0), s.first0, s.span0, 0, s.col1);
-    side(scalar(s.b1), s.first1, s.span1, s.col1, s.col2);
-    side(scalar(s.b2), s.first2, s.span2, s.col2, s.col3);
-    *at = reinterpret_cast<const void *>(p + from);
-    return live;
-}
 
 // The kernel's last argument and where it sits among the arguments: the kernel reads it late, through
 // the argument segment's address (see there), so its place is spelled out as a struct with the
@@ -301,21 +260,6 @@ constexpr uint32_t gmp_layout_word(int slot_bytes, int producers, uint32_t bits)
     return (uint32_t)slot_bytes | (uint32_t)producers << 16 | bits;
 }
 constexpr int kGmpLoraArgsOffset = (int)offsetof(GmpKernelArgs, la);
-// An argument behind the preloaded ones, read where it is needed.
-template <class V>
-__device__ __forceinline__ V read_argument(int offset) {
-    typedef const char __attribute__((address_space(4))) *kernarg_ptr_t;
-    typedef const uint32_t __attribute__((address_space(4))) *kernarg_words_t;
-    kernarg_ptr_t kernarg = (kernarg_ptr_t)__builtin_amdgcn_kernarg_segment_ptr();
-    asm volatile("" : "+s"(kernarg));  // opaque: nothing read through it moves above this point
-    kernarg_words_t src = (kernarg_words_t)(kernarg + offset);
-    struct Words {
-        uint32_t w[sizeof(V) / 4];
-    } words;
-#pragma unroll
-    for (int i = 0; i < (int)(sizeof(V) / 4); ++i) words.w[i] = src[i];
-    return __builtin_bit_cast(V, words);
-}
 static_assert(sizeof(GmpLoraArgs) % 4 == 0, "read word by word");
 
 // What only the end of the kernel needs -- where the result and the partial tiles go, how a tile is
@@ -841,21 +785,6 @@ int gmp_slot_bytes(int gpw, int tiles, int own) {
     return a > r ? a : r;
 }
 
-// Where the second and the third of the adapters' sides begin, in tiles and in blocks: a block has columns of one of them.
-struct GmpBorders {
-    int end0, blocks0, end1, blocks1;
-};
-[[maybe_unused]] GmpBorders own_borders(const DecodeArgs &a) {
-    const AdapterSides &s = *a.lora_sides;
-    const int NT = a.N / kTileN, T = a.gm_tiles;
-    GmpBorders b{NT, 0, NT, 0};
-    if (!s.interleaved && s.count > 1) b.end0 = s.first[1] / kTileN;
-    if (!s.interleaved && s.count > 2) b.end1 = s.first[2] / kTileN;
-    b.blocks0 = (b.end0 + T - 1) / T;
-    b.blocks1 = b.blocks0 + (b.end1 - b.end0 + T - 1) / T;
-    return b;
-}
-
 template <int T, int GPW, int AQ>
 hipError_t launch_gmp_tga(const DecodeArgs &a, hipStream_t stream) {
     const hipError_t attr = allow_dynamic_lds<&w4a16_decode_gmp_kernel<T, GPW, AQ, kGmpLora>>(decode_max_lds_bytes());
@@ -866,7 +795,7 @@ hipError_t launch_gmp_tga(const DecodeArgs &a, hipStream_t stream) {
     int col_blocks = (NT + T - 1) / T;
     uint32_t in_upper[4] = {0u, 0u, 0u, 0u};  // of G, NT, GS and the column blocks
     if constexpr (kOwnTiles > 0) {
-        const GmpBorders b = own_borders(a);
+        const OwnBorders b = own_borders(*a.lora_sides, NT, T);
         col_blocks = b.blocks1 + (NT - b.end1 + T - 1) / T;
         in_upper[0] = (uint32_t)b.blocks0 << 16;
         in_upper[1] = (uint32_t)b.end0 << 16;

@@ -35,14 +35,20 @@ namespace kiln {
 
 namespace {
 
-// This file is compiled three times: as it is for calls without adapters, with -DKILN_MID_LORA=1 for calls
+// This file is compiled five times: as it is for calls without adapters, with -DKILN_MID_LORA=1 for calls
 // with them (launch_mid_lora only), so that what the low-rank term adds costs plain calls nothing, and with
 // -DKILN_MID_LORA=2 for calls whose adapters are not stacked (launch_mid_sides only; apart as on the small-M kernel, where
-// one form for both was measured slower: here that was not measured, and the two take the same registers to within three).
+// one form for both was measured slower: here that was not measured, and the two take the same registers to within three);
+// =3 and =4 are for calls with either whose blocks project x onto one or two tiles of 16 rank columns by themselves
+// (launch_mid_own1, launch_mid_own2).
 #ifndef KILN_MID_LORA
 #define KILN_MID_LORA 0
 #endif
-constexpr bool kMidLora = KILN_MID_LORA != 0, kMidSides = KILN_MID_LORA == 2;
+constexpr bool kMidLora = KILN_MID_LORA == 1 || KILN_MID_LORA == 2, kMidSides = KILN_MID_LORA == 2;
+constexpr int kMidOwn = KILN_MID_LORA >= 3 ? KILN_MID_LORA - 2 : 0;  // rank tiles a block projects x onto by itself
+#if KILN_MID_LORA >= 3
+#define w4a16_mid_kernel w4a16_mid_kernel_own  // (the name profiles show)
+#endif
 
 // Probe builds only (-DKILN_MID_TIMELINE): wall-clock stamps (100 MHz) per wavefront.
 #ifdef KILN_MID_TIMELINE
@@ -50,6 +56,10 @@ constexpr bool kMidLora = KILN_MID_LORA != 0, kMidSides = KILN_MID_LORA == 2;
 #define g_mid_tl g_mid_tl_lora
 #elif KILN_MID_LORA == 2
 #define g_mid_tl g_mid_tl_sides
+#elif KILN_MID_LORA == 3
+#define g_mid_tl g_mid_tl_own1
+#elif KILN_MID_LORA == 4
+#define g_mid_tl g_mid_tl_own2
 #endif
 __device__ long long *g_mid_tl;
 #define KILN_MID_TL(i) tl_[i] = (long long)__builtin_amdgcn_s_memrealtime()
@@ -66,6 +76,15 @@ constexpr int kMidSlotBytes = kMidRows * 256;   // one group of A: 64 rows x 128
 constexpr int kMidALoads = 16;                  // LDS-direct loads per group of A
 constexpr int kMidMaxGroups = 4;                // groups per wavefront, at most
 constexpr int kMidFlaggedSlices = kDecodeFlaggedMaxSlices;  // most K slices the counter-free exchange takes
+// A projection of each block's own (kMidOwn; as on the small-M kernel): a wavefront stages its groups of A_cat behind its slot and
+// adds eight 32x32x16 products a group and row block, A_cat's fragments against those of x that it holds anyway; the parts of T
+// meet behind one more barrier, a wavefront for every 16 ranks of a row block rounds its piece and adds the term's products to
+// its own partial tiles.  (The whole term costs 2 us on the shortest launches, where the projection in the first blocks, its
+// words and T's way back cost 5 to 6: 1024 -> 1024 with 8 ranks at 20 rows 7.8 -> 4.8 us, with 32 at 32 8.4 -> 5.4.)  Instances that have no registers for T
+// -- three pairs of tiles, or two and three groups to a wavefront, with both row blocks -- do not exist.
+constexpr int kMidOwnBytes = 16 * 256;          // one group of a rank tile's rows of A_cat
+// wavefronts of a block that projects x by itself, at most: 160 KiB of LDS
+constexpr int mid_own_max_waves(int own) { return 160 * 1024 / (kMidSlotBytes + own * kMidOwnBytes); }
 constexpr int kMidSpinLimit = 1 << 20;          // polls of the other slices' parts before the adding wavefront gives up
 
 // Issue order of a wavefront's loads -- A(g): NA LDS-direct loads (16, or 8 where a run has at most 32
@@ -77,14 +96,17 @@ constexpr int kMidSpinLimit = 1 << 20;          // polls of the other slices' pa
 //   step g: [wait for A(g)] fragments to registers, A(g+DA), B(g+D), [wait for B(g)], products.
 // DA = groups of A in flight: 1 where a group fills the wavefront's slot (64 rows), 2 where it fills half
 // (one row block per pass: the halves take turns).
-// wait_a[g] / wait_b[g] = loads issued after A(g) / B(g) up to that wait: what may still be
+// OWN rank tiles: A_cat(0), 4 LDS-direct loads a tile, and the block's rows of B_cat, NB loads, end the first line; step g ends
+// with [wait for A_cat(g)] its products with x, A_cat(g+1).
+// wait_a[g] / wait_b[g] / wait_own[g] = loads issued after A(g) / B(g) / A_cat(g) up to that wait: what may still be
 // outstanding when the wait returns.
 struct MidSchedule {
     int wait_a[kMidMaxGroups];
     int wait_b[kMidMaxGroups];
+    int wait_own[kMidMaxGroups];
 };
-constexpr MidSchedule mid_schedule(int ng, int nl, int d, int na, int da) {
-    int kind[4 * kMidMaxGroups] = {}, grp[4 * kMidMaxGroups] = {}, size[4 * kMidMaxGroups] = {};
+constexpr MidSchedule mid_schedule(int ng, int nl, int d, int na, int da, int own, int nb) {
+    int kind[5 * kMidMaxGroups] = {}, grp[5 * kMidMaxGroups] = {}, size[5 * kMidMaxGroups] = {};
     int n = 0;
     auto push = [&](int k, int g, int sz) {
         kind[n] = k;
@@ -104,19 +126,27 @@ constexpr MidSchedule mid_schedule(int ng, int nl, int d, int na, int da) {
     push(0, 0, na);
     for (int g = 0; g < d && g < ng; ++g) push(1, g, nl);
     for (int g = 1; g < da && g < ng; ++g) push(0, g, na);
+    if (own > 0) {
+        push(2, 0, 4 * own);
+        push(3, 0, nb);
+    }
     MidSchedule s{};
     for (int g = 0; g < ng; ++g) {
         s.wait_a[g] = issued_after(0, g);
         if (g + da < ng) push(0, g + da, na);
         if (g + d < ng) push(1, g + d, nl);
         s.wait_b[g] = issued_after(1, g);
+        if (own > 0) {
+            s.wait_own[g] = issued_after(2, g);
+            if (g + 1 < ng) push(2, g + 1, 4 * own);
+        }
     }
     return s;
 }
 
-template <int NG, int NL, int D, int NA, int DA>
+template <int NG, int NL, int D, int NA, int DA, int OWN, int NB>
 struct MidScheduleOf {
-    static constexpr MidSchedule value = mid_schedule(NG, NL, D, NA, DA);
+    static constexpr MidSchedule value = mid_schedule(NG, NL, D, NA, DA, OWN, NB);
 };
 
 // The low-rank term of a call with adapters (LORA instances): T = the scaled projection of x onto the
@@ -140,7 +170,11 @@ struct MidLora {
 struct MidLoraSides : MidLora {
     LoraSides sides;
 };
-using MidLow = std::conditional_t<kMidSides, MidLoraSides, MidLora>;
+// ... projected onto by every block itself: none of the members above
+struct MidLoraOwn : MidLora {
+    OwnArgs own;
+};
+using MidLow = std::conditional_t<kMidSides, MidLoraSides, std::conditional_t<(kMidOwn > 0), MidLoraOwn, MidLora>>;
 constexpr int kMidFoldTileWord = 32;  // a copy's words start here (the first words are the small-M kernel's)
 constexpr int kMidFoldSpinLimit = 1 << 20;
 
@@ -153,6 +187,7 @@ struct MidShape {
     int rows, G, NT;
     uint32_t slices, layout;
     int col_blocks;
+    int end0 = 0, blocks0 = 0, end1 = 0, blocks1 = 0;  // a projection of each block's own: where the adapters' sides meet, in tiles and blocks
     __device__ __forceinline__ int GS() const { return slices & 0xFFFF; }
     __device__ __forceinline__ int KS() const { return slices >> 16; }
     __device__ __forceinline__ int full_waves() const { return layout & 255; }               // wavefronts of GPW groups
@@ -161,6 +196,24 @@ struct MidShape {
     __device__ __forceinline__ bool is(uint32_t bit) const { return (layout & bit) != 0; }
 };
 constexpr uint32_t kMidColumnScales = 1u << 24, kMidColShift = 1u << 25, kMidSwiglu = 1u << 26, kMidFlagged = 1u << 27;
+
+struct MidKernelArgs {  // where the last argument's parts are
+    const uint16_t *A;
+    const u32x4 *B;
+    const uint16_t *S;
+    int rows, G, NT;
+    uint32_t slices, layout;
+    int col_blocks;
+    uint16_t *C;
+    float *partial;
+    int *counters;
+    MidLow lo;
+};
+#if KILN_MID_LORA >= 3
+constexpr int kMidOwnOffset = (int)(offsetof(MidKernelArgs, lo) + offsetof(MidLoraOwn, own));
+#else
+constexpr int kMidOwnOffset = 0;
+#endif
 
 // The work of one block.  RBN: row blocks of 32 its pass computes -- 2, or 1 where the block's run of rows
 // has at most 32 (a launch of up to 32 rows, or the last run of a longer one: half the loads of A, fragment
@@ -234,7 +287,13 @@ __device__ __forceinline__ void mid_block(
     // are slow when they meet in one die's L2).
     int cb = bx + (shape.is(kMidColShift) ? ks : 0);
     if (cb >= ncb) cb -= ncb;  // at most three past the end, of four blocks or more
-    const int tf = cb * (2 * TP);  // first 16-column tile of the block
+    int tf = cb * (2 * TP), tile_end = NT;  // first 16-column tile of the block; tiles from tile_end on are not its own
+    if constexpr (kMidOwn > 0) {  // the blocks of a side of the adapters end where it does: no block has columns of two
+        const int before = cb < shape.blocks0 ? 0 : (cb < shape.blocks1 ? shape.blocks0 : shape.blocks1);
+        const int from = cb < shape.blocks0 ? 0 : (cb < shape.blocks1 ? shape.end0 : shape.end1);
+        tile_end = cb < shape.blocks0 ? shape.end0 : (cb < shape.blocks1 ? shape.end1 : NT);
+        tf = from + (cb - before) * (2 * TP);
+    }
     // the first `fw` wavefronts own GPW groups each, the others GPW - 1; the last slice may have fewer groups
     // than the others (K in groups not a multiple of the slices) and then fewer wavefronts of GPW
     const int fw = ks == KS - 1 ? shape.last_full_waves() : shape.full_waves();
@@ -271,7 +330,7 @@ __device__ __forceinline__ void mid_block(
     // one 64-bit address per operand, 32-bit distances from it
     const bool column_scales = shape.is(kMidColumnScales);
     const uint32_t scale_groups = column_scales ? 1u : (uint32_t)G;
-    const int last_pair_tile = NT - 2 - tf;  // a pair past the last tile reads the last pair; never stored
+    const int last_pair_tile = tile_end - 2 - tf;  // a pair past the last tile reads the last pair; never stored
     const uint32_t b_lane = (uint32_t)(l32 >> 4) * (uint32_t)G * 1024u + (uint32_t)((l32 & 15) + 16 * h) * 16u;
     const uint32_t s_lane = (uint32_t)(l32 >> 4) * scale_groups * (kTileN * 2) + (uint32_t)(l32 & 15) * 2u;
     const char *const b_first = reinterpret_cast<const char *>(B) + (size_t)((uint32_t)tf * (uint32_t)G + (uint32_t)g0) * 1024;
@@ -305,16 +364,66 @@ __device__ __forceinline__ void mid_block(
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[p][rb][r] = 0.f;
 
+    // The block's own projection: parts of T (lane (l32, h): ranks 8 q + 4 h ... + 3 of row 32 rb + l32), the operand of the step
+    // of 16 ranks that this wavefront finishes, the scale of rank column lane % 32, the block's ranks
+    [[maybe_unused]] f32x16 t_part[2];
+    [[maybe_unused]] u32x2 b_own[TP][2];
+    [[maybe_unused]] bool b_live[TP][2];
+    [[maybe_unused]] float own_scale = 0.f;
+    [[maybe_unused]] OwnWindow own_ranks{0, 0};
+    constexpr int kOwnItems = kMidOwn * RBN;  // (16 ranks, row block): a wavefront's each
+    const int own_step = kOwnItems > 0 ? min(wave, kOwnItems - 1) / RBN : 0;
+    unsigned char *own_area = lds + nw * kMidSlotBytes + wave * (kMidOwn * kMidOwnBytes);
+    if constexpr (kMidOwn > 0) {
+#pragma unroll
+        for (int rb = 0; rb < RBN; ++rb)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) t_part[rb][r] = 0.f;
+    }
+
     // The wavefront's groups: straight-line code from the first request to the last use, one
     // instance per group count (a register that an asm load fills must be requested, waited for and
     // used inside one basic block).
     auto run = [&](auto nc) {
         constexpr int NG = decltype(nc)::value;
         constexpr int NL = 3 * TP;
-        using Sch = MidScheduleOf<NG, NL, D, kMidALoads * RBN / 2, kASlots>;
+        using Sch = MidScheduleOf<NG, NL, D, kMidALoads * RBN / 2, kASlots, kMidOwn, 2 * TP>;
         request_a(0);
         unrolled<0, (D < NG ? D : NG)>(request_b);
         if constexpr (kASlots == 2 && NG > 1) request_a(1);
+        [[maybe_unused]] const char *a_own[4 * kMidOwn + 1];
+        [[maybe_unused]] const unsigned own_addr = (unsigned)(size_t)(lds_ptr_t)own_area;
+        [[maybe_unused]] auto request_own = [&] {  // the next group of A_cat, as request_a lays out A; ranks come in fours, a load
+#pragma unroll
+            for (int i = 0; i < 4 * kMidOwn; ++i) {
+                load_to_lds_b128_if(4 * i, own_ranks.ranks, a_own[i], own_addr + i * 1024);
+                a_own[i] += 256;
+            }
+        };
+        if constexpr (kMidOwn > 0) {
+            const OwnSidesA sides_a = read_argument<OwnSidesA>(kMidOwnOffset + (int)offsetof(OwnArgs, a));
+            own_ranks = own_window(sides_a, tf * kTileN, min(tf + 2 * TP, tile_end) * kTileN);
+#pragma unroll
+            for (int i = 0; i < 4 * kMidOwn; ++i)  // (past the block's ranks: an address nothing is asked of)
+                a_own[i] = own_a_row(sides_a, own_ranks.lo + 4 * i + (lane >> 4), row_pitch) +
+                           ((uint32_t)g0 * 256u + (((lane & 15) ^ ((4 * i + (lane >> 4)) & 15)) << 4));
+            request_own();
+            const OwnSidesB sides_b = read_argument<OwnSidesB>(kMidOwnOffset + (int)offsetof(OwnArgs, b));
+#pragma unroll
+            for (int p = 0; p < TP; ++p)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    const void *at;
+                    b_live[p][j] = own_b_unit(sides_b, (tf + min(2 * p, last_pair_tile)) * kTileN + l32, own_ranks.lo + 16 * own_step + 8 * j + 4 * h, &at);
+                    load_b64(b_own[p][j], at);
+                }
+            const OwnScales by_adapter = read_argument<OwnScales>(kMidOwnOffset + (int)offsetof(OwnArgs, scales));
+#pragma unroll
+            for (int i = kLoraSidesMaxAdapters - 1; i >= 0; --i) {
+                const float of_adapter = scalar(by_adapter.scales[i]);
+                own_scale = own_ranks.lo + l32 < by_adapter.ends[i] ? of_adapter : own_scale;
+            }
+        }
         float s_cur[TP];
         float s_of[NG][TP];   // the scale of every group (this lane's column of each pair)
         float c_of[NG][RBN];  // -136 * (sum of the group's activations) of row 32 rb + l32
@@ -420,7 +529,28 @@ __device__ __forceinline__ void mid_block(
                         acc[p][rb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, af[rb][s]), bexp,
                                                                              acc[p][rb], 0, 0, 0);
                 }
+            if constexpr (kMidOwn > 0) {  // (A_cat x^T); one rank tile: twice, in the product's two halves
+                wait_vector_loads<Sch::value.wait_own[gi]>();
+#pragma unroll
+                for (int s = 0; s < 8; ++s) {
+                    const u32x4 of = *reinterpret_cast<const u32x4 *>(own_area + (l32 & (16 * kMidOwn - 1)) * 256 + (((2 * s + h) ^ (l32 & 15)) << 4));
+#pragma unroll
+                    for (int rb = 0; rb < RBN; ++rb)
+                        t_part[rb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, of), __builtin_bit_cast(bf16x8, af[rb][s]),
+                                                                             t_part[rb], 0, 0, 0);
+                }
+                if constexpr (gi + 1 < NG) {
+                    wait_lds_reads();
+                    request_own();
+                }
+            }
         });
+        if constexpr (kMidOwn > 0) {
+#pragma unroll
+            for (int p = 0; p < TP; ++p)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) pin_loaded(b_own[p][j]);  // issued ahead of the last A_cat
+        }
         // out of the last group's units
 #pragma unroll
         for (int p = 0; p < TP; ++p)
@@ -545,6 +675,45 @@ __device__ __forceinline__ void mid_block(
             }
         }
     }
+    if constexpr (kMidOwn > 0) {
+        // The wavefronts' parts of T meet, (16 ranks, row block) by a wavefront; it rounds its piece and adds the term's products
+        // to its own partial tiles, which the meeting below sums with everything else.  Every K slice has a T of its own.
+#pragma unroll
+        for (int rb = 0; rb < RBN; ++rb)
+#pragma unroll
+            for (int q = 0; q < 2 * kMidOwn; ++q)
+                reinterpret_cast<f32x4 *>(own_area)[(rb * 2 * kMidOwn + q) * 64 + lane] =
+                    f32x4{t_part[rb][4 * q], t_part[rb][4 * q + 1], t_part[rb][4 * q + 2], t_part[rb][4 * q + 3]};
+        __syncthreads();
+        if (wave < kOwnItems) {
+            const int item_rb = wave % RBN;
+            const unsigned char *parts = lds + nw * kMidSlotBytes;
+            uint32_t bits[8];
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+                for (int wv = 0; wv < nw; ++wv)
+                    sum += reinterpret_cast<const f32x4 *>(parts + wv * (kMidOwn * kMidOwnBytes))[(item_rb * 2 * kMidOwn + 2 * own_step + j) * 64 + lane];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int rank = 16 * own_step + 8 * j + 4 * h + i;
+                    const float t = sum[i] * __shfl(own_scale, rank, 64);
+                    bits[4 * j + i] = rank < own_ranks.ranks ? (uint32_t)f32_to_bf16_bits(t) : 0u;
+                }
+            }
+            const u32x4 t_own = {bits[0] | bits[1] << 16, bits[2] | bits[3] << 16, bits[4] | bits[5] << 16, bits[6] | bits[7] << 16};
+#pragma unroll
+            for (int p = 0; p < TP; ++p) {
+                const u32x4 b_op = {b_live[p][0] ? b_own[p][0].x : 0u, b_live[p][0] ? b_own[p][0].y : 0u, b_live[p][1] ? b_own[p][1].x : 0u,
+                                    b_live[p][1] ? b_own[p][1].y : 0u};
+#pragma unroll
+                for (int rb = 0; rb < RBN; ++rb)
+                    if (RBN == 1 || rb == item_rb)
+                        acc[p][rb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, t_own), __builtin_bit_cast(bf16x8, b_op),
+                                                                             acc[p][rb], 0, 0, 0);
+            }
+        }
+    }
     KILN_MID_TL(5);  // main loop done
 
     // --- the wavefronts' partial tiles meet in LDS, as many pairs at a time as a wavefront's 16 KiB slot
@@ -559,7 +728,7 @@ __device__ __forceinline__ void mid_block(
     auto store_item = [&](f32x4 v, int item) {
         const int q = item & 3, rb = (item >> 2) & 1, p = item >> 3;
         const int row0 = 32 * rb + 8 * q + 4 * h;
-        const bool live = tf + 2 * p < NT;  // false: a pair past the last tile (grid padding)
+        const bool live = tf + 2 * p < tile_end;  // false: a pair past the last tile (grid padding)
         if (!swiglu) {
             uint16_t *dst = C + (size_t)row0 * N + (tf + 2 * p) * kTileN + l32;
 #pragma unroll
@@ -727,14 +896,17 @@ constexpr int kMidOneRowBlock = 1, kMidTwoRowBlocks = 2, kMidRowBlocksByRun = 0;
 // (one pair per block: 114...153 registers whatever the row blocks, so ten wavefronts there too; with adapters the
 // one-row-block instances: 162...166)
 template <int TP, int ROW_BLOCKS, bool LORA>
-constexpr int kMidWavesOf = ROW_BLOCKS == kMidOneRowBlock || (!LORA && TP == 1) ? kMidWavesMost : kMidWaves;
+constexpr int kMidWavesOf = kMidOwn > 0 ? mid_own_max_waves(kMidOwn) : ROW_BLOCKS == kMidOneRowBlock || (!LORA && TP == 1) ? kMidWavesMost : kMidWaves;
 
 template <int TP, int GPW, bool LORA, int ROW_BLOCKS>
 __global__ __launch_bounds__((kMidWavesOf<TP, ROW_BLOCKS, LORA> * 64)) void w4a16_mid_kernel(
     const uint16_t *__restrict__ A_all, const u32x4 *__restrict__ B, const uint16_t *__restrict__ S,
     int rows, int G, int NT, uint32_t slices, uint32_t layout, int col_blocks, uint16_t *__restrict__ C_all,
     float *partial_all, int *counters_all, MidLow lo) {
-    const MidShape shape{rows, G, NT, slices, layout, col_blocks};
+    MidShape shape{rows, G, NT, slices, layout, col_blocks};
+    if constexpr (kMidOwn > 0)  // 16 bits each, the upper ones say where the sides of the adapters meet
+        shape = MidShape{rows & 0xFFFF, G & 0xFFFF, NT & 0xFFFF, slices, layout, col_blocks & 0xFFFF, (int)((uint32_t)NT >> 16), (int)((uint32_t)G >> 16),
+                         (int)((uint32_t)rows >> 16), (int)((uint32_t)col_blocks >> 16)};
     if constexpr (ROW_BLOCKS != kMidRowBlocksByRun) {
         mid_block<TP, GPW, LORA, ROW_BLOCKS>(A_all, B, S, C_all, partial_all, counters_all, shape, lo);
     } else {
@@ -756,7 +928,8 @@ __global__ __launch_bounds__((kMidWavesOf<TP, ROW_BLOCKS, LORA> * 64)) void w4a1
 
 template <int TP, int GPW, int ROW_BLOCKS>
 hipError_t launch_mid_tgs(const MidArgs &a, hipStream_t stream) {
-    const hipError_t attr = allow_dynamic_lds<&w4a16_mid_kernel<TP, GPW, kMidLora, ROW_BLOCKS>>(kMidWavesOf<TP, ROW_BLOCKS, kMidLora> * kMidSlotBytes);
+    const hipError_t attr = allow_dynamic_lds<&w4a16_mid_kernel<TP, GPW, kMidLora, ROW_BLOCKS>>(kMidWavesOf<TP, ROW_BLOCKS, kMidLora> *
+                                                                                              (kMidSlotBytes + kMidOwn * kMidOwnBytes));
     if (attr != hipSuccess) return attr;
     const int NT = a.N / kTileN;
     const int runs = (a.M + kMidRows - 1) / kMidRows;
@@ -768,7 +941,17 @@ hipError_t launch_mid_tgs(const MidArgs &a, hipStream_t stream) {
     lo.r_total = a.r_total;
     lo.rp = (a.r_total + 15) / 16 * 16;
     lo.slices = a.lora_slices;
-    const int col_blocks = (NT + 2 * TP - 1) / (2 * TP);
+    int col_blocks = (NT + 2 * TP - 1) / (2 * TP);
+    uint32_t in_upper[4] = {0u, 0u, 0u, 0u};  // of rows, G, NT and the column blocks
+#if KILN_MID_LORA >= 3
+    lo.own = own_args(a);
+    const OwnBorders b = own_borders(*a.lora_sides, NT, 2 * TP);
+    col_blocks = b.blocks1 + (NT - b.end1 + 2 * TP - 1) / (2 * TP);
+    in_upper[0] = (uint32_t)b.end1 << 16;
+    in_upper[1] = (uint32_t)b.blocks0 << 16;
+    in_upper[2] = (uint32_t)b.end0 << 16;
+    in_upper[3] = (uint32_t)b.blocks1 << 16;
+#endif
     dim3 grid(col_blocks, a.KS, runs);
 #if KILN_MID_LORA == 2
     lo.sides = lora_sides(a.lora_sides);
@@ -790,18 +973,23 @@ hipError_t launch_mid_tgs(const MidArgs &a, hipStream_t stream) {
     const uint32_t layout = (uint32_t)full_waves | (uint32_t)last_full_waves << 8 | (uint32_t)a.waves << 16 |
                             (a.Gs == 1 ? kMidColumnScales : 0u) | (a.swiglu ? kMidSwiglu : 0u) |
                             (a.flagged ? kMidFlagged | (exchange_column_shift(col_blocks) ? kMidColShift : 0u) : 0u);
-    w4a16_mid_kernel<TP, GPW, kMidLora, ROW_BLOCKS><<<grid, a.waves * 64, a.waves * kMidSlotBytes, stream>>>(
-        (const uint16_t *)a.A, (const u32x4 *)a.B, (const uint16_t *)a.S, a.M, a.K / kGroupK, NT,
-        (uint32_t)a.GS | (uint32_t)a.KS << 16, layout, col_blocks, (uint16_t *)a.C, a.partial, a.counters, lo);
+    w4a16_mid_kernel<TP, GPW, kMidLora, ROW_BLOCKS><<<grid, a.waves * 64, a.waves * (kMidSlotBytes + kMidOwn * kMidOwnBytes), stream>>>(
+        (const uint16_t *)a.A, (const u32x4 *)a.B, (const uint16_t *)a.S, a.M | in_upper[0], a.K / kGroupK | in_upper[1], NT | in_upper[2],
+        (uint32_t)a.GS | (uint32_t)a.KS << 16, layout, col_blocks | in_upper[3], (uint16_t *)a.C, a.partial, a.counters, lo);
     return hipGetLastError();
 }
 
 template <int TP, int GPW>
 hipError_t launch_mid_tg(const MidArgs &a, hipStream_t stream) {
     if (a.M <= 32) return launch_mid_tgs<TP, GPW, kMidOneRowBlock>(a, stream);
+    if constexpr (kMidOwn > 0) {  // (three pairs, or two and three groups a wavefront: no registers left for T)
+        if constexpr (TP == 1 || (TP == 2 && GPW <= 2)) return launch_mid_tgs<TP, GPW, kMidTwoRowBlocks>(a, stream);
+        else return hipErrorInvalidValue;
+    }
     const int last_run = a.M - (a.M - 1) / kMidRows * kMidRows;
-    return last_run <= 32 ? launch_mid_tgs<TP, GPW, kMidRowBlocksByRun>(a, stream)
-                          : launch_mid_tgs<TP, GPW, kMidTwoRowBlocks>(a, stream);
+    if constexpr (kMidOwn == 0)
+        return last_run <= 32 ? launch_mid_tgs<TP, GPW, kMidRowBlocksByRun>(a, stream)
+                              : launch_mid_tgs<TP, GPW, kMidTwoRowBlocks>(a, stream);
 }
 
 template <int TP>
@@ -821,16 +1009,25 @@ hipError_t launch_mid_t(const MidArgs &a, int gpw, hipStream_t stream) {
 
 #if KILN_MID_LORA
 // The instances with the low-rank term; the caller (launch_mid) has checked the plan.
-#if KILN_MID_LORA == 2
+#if KILN_MID_LORA >= 3
+#if KILN_MID_LORA == 3
+hipError_t launch_mid_own1(const MidArgs &a, hipStream_t stream) {
+#else
+hipError_t launch_mid_own2(const MidArgs &a, hipStream_t stream) {
+#endif
+    if (a.own_tiles != kMidOwn) return hipErrorInvalidValue;
+#elif KILN_MID_LORA == 2
 hipError_t launch_mid_sides(const MidArgs &a, hipStream_t stream) {
     if (!a.lora_sides || a.lora_sides->count < 1 || a.lora_sides->count > kMaxAdapterSides || a.lora_producers < 1) return hipErrorInvalidValue;
 #else
 hipError_t launch_mid_lora(const MidArgs &a, hipStream_t stream) {
     if (!a.lora_b) return hipErrorInvalidValue;
 #endif
+#if KILN_MID_LORA <= 2
     if (a.r_total < 8 || a.r_total > 64 || a.r_total % 8 != 0 || !a.lora_t || a.lora_slices < 1)
         return hipErrorInvalidValue;
     if (a.lora_producers > 0 && !mid_lora_fold_ok(a)) return hipErrorInvalidValue;
+#endif
     const int gpw = (a.GS + a.waves - 1) / a.waves;
     switch (a.pairs) {
         case 1: return launch_mid_t<1>(a, gpw, stream);
@@ -869,6 +1066,12 @@ bool mid_plan_ok(const MidArgs &a) {
     const int G = a.K / kGroupK;
     // slices of GS groups; the last one may be shorter (11008 = 86 groups = 29 + 29 + 28)
     if (a.KS < 1 || a.KS > 0x7FFF || a.GS < 1 || a.KS * a.GS < G || (a.KS - 1) * a.GS >= G) return false;
+    if (a.own_tiles > 0) {  // (16 bits for each of the sizes; a wavefront for every 16 ranks of a row block)
+        const int row_blocks = a.M > 32 ? 2 : 1;
+        if (a.own_tiles > 2 || a.M > 0xFFFF || a.N / kTileN > 0xFFFF || G > 0xFFFF || (row_blocks == 2 && a.pairs == 3) ||
+            (row_blocks == 2 && a.pairs == 2 && a.GS > 2 * a.waves) || a.waves < a.own_tiles * row_blocks || a.waves > mid_own_max_waves(a.own_tiles))
+            return false;
+    }
     if (a.waves < 1 || a.waves > mid_max_waves(a.M, a.pairs, a.r_total > 0) || a.waves > a.GS) return false;
     const int gpw = (a.GS + a.waves - 1) / a.waves;
     if (gpw > kMidMaxGroups || (a.pairs == 3 && gpw == 4)) return false;  // (3, 4) would spill registers
@@ -880,9 +1083,12 @@ bool mid_plan_ok(const MidArgs &a) {
 
 // The counter-free exchange deals a pair's items (eight, or four of a pass over one row block) to the block's
 // first wavefronts, one each: blocks of eight wavefronts or more.
-bool mid_flagged_ok(const MidArgs &a) { return a.KS > 1 && a.KS <= kMidFlaggedSlices && a.waves >= kMidWaves; }
+bool mid_flagged_ok(const MidArgs &a) {
+    return a.KS > 1 && a.KS <= kMidFlaggedSlices && a.waves >= (a.own_tiles > 0 && a.M <= 32 ? kMidWaves / 2 : kMidWaves);
+}
 
-int mid_column_blocks(const MidArgs &a) { return (a.N / kTileN + 2 * a.pairs - 1) / (2 * a.pairs); }
+// (a projection of each block's own: up to two more, where sides of the adapters meet inside a block)
+int mid_column_blocks(const MidArgs &a) { return (a.N / kTileN + 2 * a.pairs - 1) / (2 * a.pairs) + (a.own_tiles > 0 ? 2 : 0); }
 
 size_t mid_partial_bytes(const MidArgs &a) {
     if (a.KS <= 1) return 0;
@@ -894,6 +1100,10 @@ hipError_t launch_mid(const MidArgs &a, hipStream_t stream) {
     if (!mid_plan_ok(a)) return hipErrorInvalidValue;
     if (a.KS > 1 && (!a.partial || !a.counters)) return hipErrorInvalidValue;
     if (a.flagged && !mid_flagged_ok(a)) return hipErrorInvalidValue;
+    if (a.own_tiles > 0) {
+        if (!a.lora_sides || a.r_total < 4 || a.lora_adapters < 1 || a.lora_adapters > kLoraSidesMaxAdapters) return hipErrorInvalidValue;
+        return a.own_tiles == 1 ? launch_mid_own1(a, stream) : launch_mid_own2(a, stream);
+    }
     if (a.r_total > 0) return a.lora_sides ? launch_mid_sides(a, stream) : launch_mid_lora(a, stream);
     const int gpw = (a.GS + a.waves - 1) / a.waves;
     switch (a.pairs) {
@@ -907,7 +1117,11 @@ hipError_t launch_mid(const MidArgs &a, hipStream_t stream) {
 }  // namespace kiln
 
 #ifdef KILN_MID_TIMELINE
-#if KILN_MID_LORA == 2
+#if KILN_MID_LORA == 3
+extern "C" int kiln_mid_timeline_own1(long long *buf) {
+#elif KILN_MID_LORA == 4
+extern "C" int kiln_mid_timeline_own2(long long *buf) {
+#elif KILN_MID_LORA == 2
 extern "C" int kiln_mid_timeline_sides(long long *buf) {
 #elif KILN_MID_LORA
 extern "C" int kiln_mid_timeline_lora(long long *buf) {

@@ -1,4 +1,4 @@
-"""Calls of up to 16 rows whose blocks project x onto their adapters by themselves, every instance, against the product in
+"""Calls whose blocks project x onto their adapters by themselves, every instance, against the product in
 64 bits and the projection in a launch of its own; and where adapters are taken that way."""
 import ctypes
 
@@ -65,6 +65,42 @@ def test_every_instance(tiles, waves, gs, ks, r):
         _assert_close(other, want, low)
 
 
+def _mid_instances():
+    """(pairs of tiles per block, groups of a slice, K slices, ranks) of the kernel of 17 rows on: one to four groups to a
+    wavefront, dealt evenly and not, slices that meet, one and two rank tiles."""
+    cases = []
+    for pairs in (1, 2, 3):
+        for gs, ks in ((4, 1), (6, 3), (8, 2), (11, 1), (20, 1), (23, 1), (8, 4)):
+            for r in (4, 16, 20, 32):
+                waves = min(gs, 8 if r <= 16 else 6)
+                gpw = -(-gs // waves)
+                if gpw > 4 or (pairs == 3 and gpw > 3) or (ks > 1 and waves < 8 and r > 16 and gs > 6):
+                    continue
+                cases.append((pairs, gs, ks, r))
+    return cases
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("pairs,gs,ks,r", _mid_instances())
+def test_every_instance_from_17_rows_on(pairs, gs, ks, r):
+    L, k, n = _lib.load_tuning(), gs * ks * 128, 768
+    gen = torch.Generator(device="cuda").manual_seed(pairs * k + r)
+    w = _packed(gen, k, n, 128 if gs % 2 == 0 else -1)
+    ad, = _all_adapters(gen, k, (n,), ((r,) if r <= 16 else (r - 9, 1, 8),))
+    taken = 0
+    for m in (17, 32, 33, 64, 65, 100, 130):
+        x = torch.randn(m, k, device="cuda", generator=gen).bfloat16()
+        L.kiln_w4a16_debug_mid(1, pairs, ks)
+        L.kiln_w4a16_debug_lora_fold(3)
+        # (a rank that is a multiple of 8 is taken either way: the one below it, on the same plan, says whether blocks project it)
+        own = L.kiln_w4a16_takes_rank(m, n, k, r if r % 8 else r - 4, -1)
+        assert own == 0 or pairs < 3 or m <= 32  # three pairs and two row blocks: no registers for T
+        taken += own
+        got = marlin_gemm.marlin_w4a16_gemm_lora(x, w.b_packed, w.scales, w.groupsize, ad.a_cat, ad.b_cat, ad.ranks, ad.scales)
+        _assert_close(got, *_reference(x, w, [(ad, 0)]))
+    assert taken >= (7 if pairs == 1 and ks == 1 else 2)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("m", [1, 7, 16])
 @pytest.mark.parametrize("k,widths,ranks", [
@@ -99,8 +135,8 @@ def test_more_than_four_adapters_side_by_side(k, widths, ranks, m):
 
 
 def test_ranks_that_are_taken_as_they_are():
-    """Multiples of 8 always; of 4 where blocks project by themselves, up to 32 and 16 rows; nothing else."""
+    """Multiples of 8 always; of 4 where blocks project by themselves, up to 32 and on the kernels of few rows; nothing else."""
     takes = _lib.load().kiln_w4a16_takes_rank
     assert [r for r in range(0, 67) if takes(4, 2560, 2560, r, -1)] == sorted({4, 12, 20, 28} | set(range(8, 65, 8)))
-    assert [m for m in (0, 1, 16, 17, 64) if takes(m, 2560, 2560, 12, -1)] == [1, 16]
+    assert [m for m in (0, 1, 16, 17, 64, 256, 300) if takes(m, 2560, 2560, 12, -1)] == [1, 16, 17, 64]
     assert takes(4, 2560, 2500, 12, -1) == takes(4, 100, 2560, 12, -1) == 0  # no shape of the kernels
