@@ -415,9 +415,9 @@ __global__ __launch_bounds__(gmp_max_waves(GPW, kOwnTiles) * 64) void w4a16_deco
 #pragma unroll
     for (int j = 0; j < kOwnTiles; ++j) t_part[j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    // Straight-line code from the first request to the last use, one instance per group count (and number of rank tiles).
-    auto run = [&](auto nc, auto oc) {
-        constexpr int NGR = decltype(nc)::value, U = T * NGR, OWN = decltype(oc)::value;
+    // Straight-line code from the first request to the last use, one instance per group count.
+    auto run = [&](auto nc) {
+        constexpr int NGR = decltype(nc)::value, U = T * NGR, OWN = kOwnTiles;
         using Sch = GmpScheduleOf<T, NGR, AQ, OWN>;
         unrolled<0, (kGmpHead < U ? kGmpHead : U)>(request_chunk);
         request_a(0, 0);
@@ -476,7 +476,7 @@ __global__ __launch_bounds__(gmp_max_waves(GPW, kOwnTiles) * 64) void w4a16_deco
                 for (int t = 0; t < 4; ++t)
                     af[t] = *reinterpret_cast<const u32x4 *>(ap + (((4 * t + (lane >> 4)) ^ (lane & 15)) << 4));
                 if constexpr (OWN > 0) {
-                    u32x4 of[4 * OWN];
+                    u32x4 of[4 * OWN + 1];
                     const unsigned char *op = mine + NS * kGmpSlotBytes + (lane & 15) * 256;
 #pragma unroll
                     for (int i = 0; i < 4 * OWN; ++i)
@@ -513,11 +513,8 @@ __global__ __launch_bounds__(gmp_max_waves(GPW, kOwnTiles) * 64) void w4a16_deco
         for (int j = 0; j < OWN; ++j) pin_loaded(b_own[j]);  // issued ahead of the last chunk
     };
     if (__builtin_expect(!adapter_wave, 1)) {
-        auto run_groups = [&](auto oc) {
-            if (full) run(std::integral_constant<int, GPW>{}, oc);
-            else if constexpr (GPW > 1) run(std::integral_constant<int, GPW - 1>{}, oc);
-        };
-        run_groups(std::integral_constant<int, kOwnTiles>{});
+        if (full) run(std::integral_constant<int, GPW>{});
+        else if constexpr (GPW > 1) run(std::integral_constant<int, GPW - 1>{});
         // every wavefront's partial tiles into its own piece of LDS, then tile ti = their sum in
         // wavefront (= ascending K) order, one tile per wavefront at a time
         KILN_GMP_TL(1, KILN_GMP_NOW());
