@@ -88,6 +88,7 @@ constexpr int kGmpMaxChunks = 16;        // chunks per wavefront, at most (strai
 struct GmpSchedule {
     int wait_a[kGmpMaxChunks];      // by group: A(g) and A_cat(g)
     int wait_chunk[kGmpMaxChunks];  // by chunk
+    int wait_b_cat;                 // at the end: of up to three chunks the last is ahead of the rows of B_cat
 };
 constexpr GmpSchedule gmp_schedule(int T, int groups, int AQ, int OWN) {
     const int U = T * groups;
@@ -125,6 +126,7 @@ constexpr GmpSchedule gmp_schedule(int T, int groups, int AQ, int OWN) {
         }
         s.wait_chunk[j] = issued_after(1, j);
     }
+    s.wait_b_cat = issued_after(3, 0);
     return s;
 }
 template <int T, int GROUPS, int AQ, int OWN>
@@ -509,8 +511,11 @@ __global__ __launch_bounds__(gmp_max_waves(GPW, kOwnTiles) * 64) void w4a16_deco
                                                           acc, 0, 0, 0);
             y[ti] += acc * f16_bits_to_f32((uint16_t)sc[set]);
         });
+        if constexpr (OWN > 0) {
+            wait_vector_loads<(Sch::value.wait_b_cat < 63 ? Sch::value.wait_b_cat : 63)>();
 #pragma unroll
-        for (int j = 0; j < OWN; ++j) pin_loaded(b_own[j]);  // issued ahead of the last chunk
+            for (int j = 0; j < OWN; ++j) pin_loaded(b_own[j]);
+        }
     };
     if (__builtin_expect(!adapter_wave, 1)) {
         if (full) run(std::integral_constant<int, GPW>{});

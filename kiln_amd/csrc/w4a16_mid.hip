@@ -99,11 +99,13 @@ constexpr int kMidSpinLimit = 1 << 20;          // polls of the other slices' pa
 // OWN rank tiles: A_cat(0), 4 LDS-direct loads a tile, and the block's rows of B_cat, NB loads, end the first line; step g ends
 // with [wait for A_cat(g)] its products with x, A_cat(g+1).
 // wait_a[g] / wait_b[g] / wait_own[g] = loads issued after A(g) / B(g) / A_cat(g) up to that wait: what may still be
-// outstanding when the wait returns.
+// outstanding when the wait returns; wait_b_cat = those behind the rows of B_cat up to the end (none of a wavefront of one
+// group: its only A_cat is ahead of them, so no other wait covers them).
 struct MidSchedule {
     int wait_a[kMidMaxGroups];
     int wait_b[kMidMaxGroups];
     int wait_own[kMidMaxGroups];
+    int wait_b_cat;
 };
 constexpr MidSchedule mid_schedule(int ng, int nl, int d, int na, int da, int own, int nb) {
     int kind[5 * kMidMaxGroups] = {}, grp[5 * kMidMaxGroups] = {}, size[5 * kMidMaxGroups] = {};
@@ -141,6 +143,7 @@ constexpr MidSchedule mid_schedule(int ng, int nl, int d, int na, int da, int ow
             if (g + 1 < ng) push(2, g + 1, 4 * own);
         }
     }
+    s.wait_b_cat = issued_after(3, 0);
     return s;
 }
 
@@ -546,10 +549,11 @@ __device__ __forceinline__ void mid_block(
             }
         });
         if constexpr (kMidOwn > 0) {
+            wait_vector_loads<(Sch::value.wait_b_cat < 63 ? Sch::value.wait_b_cat : 63)>();
 #pragma unroll
             for (int p = 0; p < TP; ++p)
 #pragma unroll
-                for (int j = 0; j < 2; ++j) pin_loaded(b_own[p][j]);  // issued ahead of the last A_cat
+                for (int j = 0; j < 2; ++j) pin_loaded(b_own[p][j]);
         }
         // out of the last group's units
 #pragma unroll
@@ -1066,10 +1070,12 @@ bool mid_plan_ok(const MidArgs &a) {
     const int G = a.K / kGroupK;
     // slices of GS groups; the last one may be shorter (11008 = 86 groups = 29 + 29 + 28)
     if (a.KS < 1 || a.KS > 0x7FFF || a.GS < 1 || a.KS * a.GS < G || (a.KS - 1) * a.GS >= G) return false;
-    if (a.own_tiles > 0) {  // (16 bits for each of the sizes; a wavefront for every 16 ranks of a row block)
+    if (a.own_tiles > 0) {  // (16 bits for each of the sizes; a wavefront for every 16 ranks of a row block, with groups of its own:
+                            // one without has not fetched the rows of B_cat)
         const int row_blocks = a.M > 32 ? 2 : 1;
         if (a.own_tiles > 2 || a.M > 0xFFFF || a.N / kTileN > 0xFFFF || G > 0xFFFF || (row_blocks == 2 && a.pairs == 3) ||
-            (row_blocks == 2 && a.pairs == 2 && a.GS > 2 * a.waves) || a.waves < a.own_tiles * row_blocks || a.waves > mid_own_max_waves(a.own_tiles))
+            (row_blocks == 2 && a.pairs == 2 && a.GS > 2 * a.waves) || a.waves < a.own_tiles * row_blocks ||
+            G - (a.KS - 1) * a.GS < a.own_tiles * row_blocks || a.waves > mid_own_max_waves(a.own_tiles))
             return false;
     }
     if (a.waves < 1 || a.waves > mid_max_waves(a.M, a.pairs, a.r_total > 0) || a.waves > a.GS) return false;

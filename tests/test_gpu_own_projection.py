@@ -140,3 +140,16 @@ def test_ranks_that_are_taken_as_they_are():
     assert [r for r in range(0, 67) if takes(4, 2560, 2560, r, -1)] == sorted({4, 12, 20, 28} | set(range(8, 65, 8)))
     assert [m for m in (0, 1, 16, 17, 64, 256, 300) if takes(m, 2560, 2560, 12, -1)] == [1, 16, 17, 64]
     assert takes(4, 2560, 2500, 12, -1) == takes(4, 100, 2560, 12, -1) == 0  # no shape of the kernels
+
+
+def test_a_wavefront_without_groups_finishes_no_ranks():
+    """1664 = 4 + 4 + 4 + 1 groups: one wavefront of the last slice has any, and two rank tiles are two wavefronts' to finish."""
+    L = _lib.load_tuning()
+    taken = {}
+    for k in (1664, 1792, 2048):
+        L.kiln_w4a16_debug_mid(1, 1, 4)
+        L.kiln_w4a16_debug_lora_fold(3)
+        taken[k] = [L.kiln_w4a16_takes_rank(m, 512, k, r, -1) for m in (17, 32) for r in (12, 20, 28)]
+    L.kiln_w4a16_debug_mid(-1, 0, 0)
+    L.kiln_w4a16_debug_lora_fold(-1)
+    assert taken == {1664: [1, 0, 0] * 2, 1792: [1, 1, 1] * 2, 2048: [1, 1, 1] * 2}
