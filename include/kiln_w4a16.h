@@ -253,8 +253,8 @@ kiln_marlin_status_t kiln_w4a16_stack_adapters(
 
 /*
  * Do the entry points with adapters take a stacked rank as it is at its best (1), or is it worth rounding up to a multiple
- * of 8 with zeros in front (0: kiln_w4a16_stack_adapters)?  Multiples of 8 always; on some shapes of up to 16 rows multiples
- * of 4.  A pure query; every rank up to 64 is taken either way.
+ * of 8 with zeros in front (0: kiln_w4a16_stack_adapters)?  Multiples of 8 always; multiples of 4
+ * up to 32 on calls of up to 16 rows, and of a few hundred, whose launch is short.  A pure query; every rank up to 64 is taken either way.
  */
 int kiln_w4a16_takes_rank(int prob_m, int prob_n, int prob_k, int r_total, int dev);
 
