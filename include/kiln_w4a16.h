@@ -396,11 +396,17 @@ int kiln_w4a16_layout_version(void);
  * kiln_w4a16_debug_prefill_projection_blocks: where the matrix-core kernel's calls with adapters compute x * A^T:
  *   > 0 in that many blocks of the product's own launch, 0 in a launch in front, -3 another kernel takes the
  *   call, -1 bad sizes.
+ * kiln_w4a16_debug_adapter_blocks: the 16-column tiles that the column blocks of a call with unstacked adapters take,
+ *   out[capacity] = {0 another path takes the call, 1 small-M kernel, 2 mid-M kernel; tiles of a block; K slices; tiles of 16
+ *   rank columns that every block projects x onto by itself, 0: the launch's first blocks do}, then {first tile, end of its
+ *   own tiles} for every column block.  Returns their count, -1 for sizes or sides that no call may have.
  */
 int kiln_w4a16_debug_gemm_plan(int prob_m, int prob_n, int prob_k, int cus, int *out);
 int kiln_w4a16_debug_decode_plan(int prob_m, int prob_n, int prob_k, int cus, int *out);
 int kiln_w4a16_debug_prefill_rowsum_producers(int prob_m, int prob_n, int prob_k, int cus);
 int kiln_w4a16_debug_prefill_projection_blocks(int prob_m, int prob_n, int prob_k, int cus);
+int kiln_w4a16_debug_adapter_blocks(int prob_m, int prob_n, int prob_k, int cus, const kiln_w4a16_adapter_side *sides, int n_sides,
+                                    int swiglu, int n_adapters, int *out, int capacity);
 
 #ifdef __cplusplus
 }

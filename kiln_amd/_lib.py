@@ -45,6 +45,7 @@ EXPORTS = (
     "kiln_w4a16_debug_decode_plan",
     "kiln_w4a16_debug_prefill_rowsum_producers",
     "kiln_w4a16_debug_prefill_projection_blocks",
+    "kiln_w4a16_debug_adapter_blocks",
 )
 
 # every symbol include/kiln_marlin_proj.h declares
@@ -194,6 +195,8 @@ def _load(tuning: bool) -> ctypes.CDLL:
     L.kiln_w4a16_debug_prefill_rowsum_producers.argtypes = [i, i, i, i]
     L.kiln_w4a16_debug_prefill_projection_blocks.restype = i
     L.kiln_w4a16_debug_prefill_projection_blocks.argtypes = [i, i, i, i]
+    L.kiln_w4a16_debug_adapter_blocks.restype = i
+    L.kiln_w4a16_debug_adapter_blocks.argtypes = [i, i, i, i, vp, i, i, i, c.POINTER(c.c_int), i]
     L.kiln_w4a16_gemm_lora.restype = i
     L.kiln_w4a16_gemm_lora.argtypes = [vp, vp, vp, vp, i, i, i, vp, i, i, vp, vp, vp, i, i,
                                        c.POINTER(c.c_int), c.POINTER(c.c_float)]

@@ -5,6 +5,8 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include "layout.h"
+
 namespace kiln {
 
 // The start of every workspace, zero whenever no launch is running:
@@ -47,6 +49,34 @@ struct AdapterSides {
     int ranks[kMaxAdapterSides], first[kMaxAdapterSides], rows[kMaxAdapterSides];
     int count, interleaved;
 };
+
+// The 16-column tiles of a column block: its own are those before `end`, as many as a block takes.
+struct BlockTiles {
+    int first, end;
+};
+// ... of the mid-M kernel, which takes tiles in pairs: first and end are even whatever the adapters' sides (their blocks have
+// all ranks, and the row of B_cat is found per column; blocks that ended where a side does had half a pair left there).
+__host__ __device__ constexpr BlockTiles mid_block_tiles(int column_block, int pairs, int tiles) { return {column_block * 2 * pairs, tiles}; }
+
+// Where the second and the third side begin, in tiles and in blocks of T tiles: a block has columns of one of them.
+struct OwnBorders {
+    int end0, blocks0, end1, blocks1;
+};
+inline OwnBorders own_borders(const AdapterSides &s, int NT, int T) {
+    OwnBorders b{NT, 0, NT, 0};
+    if (!s.interleaved && s.count > 1) b.end0 = s.first[1] / kTileN;
+    if (!s.interleaved && s.count > 2) b.end1 = s.first[2] / kTileN;
+    b.blocks0 = (b.end0 + T - 1) / T;
+    b.blocks1 = b.blocks0 + (b.end1 - b.end0 + T - 1) / T;
+    return b;
+}
+inline int own_column_blocks(const OwnBorders &b, int NT, int T) { return b.blocks1 + (NT - b.end1 + T - 1) / T; }
+__host__ __device__ __forceinline__ BlockTiles own_block_tiles(const OwnBorders &b, int column_block, int NT, int T) {
+    const int before = column_block < b.blocks0 ? 0 : (column_block < b.blocks1 ? b.blocks0 : b.blocks1);
+    const int from = column_block < b.blocks0 ? 0 : (column_block < b.blocks1 ? b.end0 : b.end1);
+    const int end = column_block < b.blocks0 ? b.end0 : (column_block < b.blocks1 ? b.end1 : NT);
+    return BlockTiles{from + (column_block - before) * T, end};
+}
 
 struct DecodeArgs {
     const void *A;      // bf16 [M, K]

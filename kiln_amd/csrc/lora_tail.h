@@ -298,18 +298,6 @@ OwnArgs own_args(const Args &d) {
     }
     return o;
 }
-// Where the second and the third side begin, in tiles and in blocks of T tiles: a block has columns of one of them.
-struct OwnBorders {
-    int end0, blocks0, end1, blocks1;
-};
-inline OwnBorders own_borders(const AdapterSides &s, int NT, int T) {
-    OwnBorders b{NT, 0, NT, 0};
-    if (!s.interleaved && s.count > 1) b.end0 = s.first[1] / kTileN;
-    if (!s.interleaved && s.count > 2) b.end1 = s.first[2] / kTileN;
-    b.blocks0 = (b.end0 + T - 1) / T;
-    b.blocks1 = b.blocks0 + (b.end1 - b.end0 + T - 1) / T;
-    return b;
-}
 constexpr int kLoraFoldMaxProducers = 16;
 constexpr int kLoraSidesMaxAdapters = 8;
 constexpr int kLoraFoldStepsPerWave = 12;  // 32-value steps of K one producer wavefront takes, at most

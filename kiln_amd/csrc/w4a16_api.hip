@@ -978,7 +978,8 @@ struct LoraSpec {
 // The `lora` of plan_gemm for a call: which kernels can take its adapters.  A block of up to 16 rows that projects x onto
 // the adapters by itself does so for all of them, or, where more than four lie side by side, for those that its columns have
 // a term of (up to four, the call is one with the stacked set in every bit: the same choice, plan and places; beyond 16 rows
-// it is whatever their number).  Blocks end where a side does, whole tiles.
+// it is whatever their number).  Up to 16 rows blocks end where a side does, whole tiles; beyond, they are what they are without
+// sides, which may begin at any column.
 int lora_kind(const LoraSpec *lora, int m) {
     if (!lora) return 0;
     const int otherwise = lora->r_total % 8 == 0 ? 1 : 2;
@@ -988,7 +989,7 @@ int lora_kind(const LoraSpec *lora, int m) {
     if (lora->sides && !lora->sides->interleaved) {
         const AdapterSides &s = *lora->sides;
         if (many) ranks = *std::max_element(s.ranks, s.ranks + s.count);
-        for (int i = 0; i < s.count; ++i)
+        for (int i = 0; i < s.count && m <= 16; ++i)
             if (s.first[i] % kTileN != 0) return otherwise;
     }
     return ranks <= 32 ? own_kind({(ranks + 7) / 8, many, lora->r_total % 8 != 0}) : otherwise;
@@ -1491,6 +1492,39 @@ int kiln_w4a16_debug_prefill_projection_blocks(int m, int n, int k, int cus) {
     plan_gemm(m, n, k, cus, -1, -1, 1, &gp);
     if (!gp.prefill) return -3;
     return g_tune.lora_fold == 0 ? 0 : prefill_projection_blocks(m, n, k, gp.pf, cus);
+}
+
+// Which tiles the column blocks of a call with unstacked adapters take: out = {0 nothing that follows holds, 1 small-M kernel,
+// 2 mid-M kernel; tiles of a block; K slices; rank tiles a block projects x onto by itself}, then {first tile, end of its own
+// tiles} of every column block, as many as fit `capacity` numbers.  The count of the column blocks, -1 for bad arguments.
+static kiln_marlin_status_t sides_of(const kiln_w4a16_adapter_side *sides, int n_sides, int prob_n, int swiglu, AdapterSides *out, int *r_total);
+int kiln_w4a16_debug_adapter_blocks(int m, int n, int k, int cus, const kiln_w4a16_adapter_side *sides, int n_sides, int swiglu, int n_adapters,
+                                    int *out, int capacity) {
+    AdapterSides own;
+    int r_total = 0;
+    if (m < 1 || cus < 1 || capacity < 4 || !shape_ok(n, k, 128) || n_adapters < 1 || sides_of(sides, n_sides, n, swiglu, &own, &r_total) != KILN_W4A16_OK)
+        return -1;
+    const LoraSpec lora{nullptr, nullptr, r_total, n_adapters, nullptr, nullptr, &own};
+    GemmPlan gp;
+    plan_gemm(m, n, k, cus, -1, -1, lora_kind(&lora, m), &gp);
+    for (int i = 0; i < 4; ++i) out[i] = 0;
+    if (gp.prefill || (!gp.mid && (gp.launches != 1 || !gp.dl[0].plan.gmp))) return 0;
+    const DecodePlan &plan = gp.dl[0].plan;
+    const int NT = n / kTileN, per_block = gp.mid ? 2 * gp.mp.pairs : plan.gm_tiles, rank_tiles = gp.mid ? gp.mp.own : plan.own;
+    const OwnBorders borders = own_borders(own, NT, per_block);
+    const bool ends_with_sides = !gp.mid && rank_tiles > 0;
+    const int blocks = ends_with_sides ? own_column_blocks(borders, NT, per_block) : ceil_div(NT, per_block);
+    out[0] = gp.mid ? 2 : 1;
+    out[1] = per_block;
+    out[2] = gp.mid ? gp.mp.KS : plan.KS;
+    out[3] = rank_tiles;
+    for (int i = 0; i < blocks && 4 + 2 * i + 1 < capacity; ++i) {
+        const BlockTiles t = gp.mid ? mid_block_tiles(i, gp.mp.pairs, NT)
+                                    : ends_with_sides ? own_block_tiles(borders, i, NT, per_block) : BlockTiles{i * per_block, NT};
+        out[4 + 2 * i] = t.first;
+        out[4 + 2 * i + 1] = t.end;
+    }
+    return blocks;
 }
 
 #ifdef KILN_W4A16_TUNING_HOOKS

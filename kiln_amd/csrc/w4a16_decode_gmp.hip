@@ -354,12 +354,11 @@ __global__ __launch_bounds__(gmp_max_waves(GPW, kOwnTiles) * 64) void w4a16_deco
     if (col_block >= col_blocks) col_block -= col_blocks;  // at most three past the end, of sixteen tiles or more
     int tf = col_block * T, tile_end = NT;  // first tile of the block; tiles from tile_end on are not its own
     if constexpr (kOwnTiles > 0) {  // the blocks of a side end where it does: no block has columns of two
-        const int blocks0 = (uint32_t)G_arg >> 16, blocks1 = (uint32_t)col_blocks_arg >> 16;  // ... of the first, of the first two
-        const int end0 = (uint32_t)NT_arg >> 16, end1 = (uint32_t)GS_arg >> 16;
-        const int before = col_block < blocks0 ? 0 : (col_block < blocks1 ? blocks0 : blocks1);
-        const int from = col_block < blocks0 ? 0 : (col_block < blocks1 ? end0 : end1);
-        tile_end = col_block < blocks0 ? end0 : (col_block < blocks1 ? end1 : NT);
-        tf = from + (col_block - before) * T;
+        const OwnBorders borders{(int)((uint32_t)NT_arg >> 16), (int)((uint32_t)G_arg >> 16), (int)((uint32_t)GS_arg >> 16),
+                                 (int)((uint32_t)col_blocks_arg >> 16)};
+        const BlockTiles mine = own_block_tiles(borders, col_block, NT, T);
+        tf = mine.first;
+        tile_end = mine.end;
     }
     const bool full = wave < full_waves;
     const int g_first = full ? wave * GPW : full_waves * GPW + (wave - full_waves) * (GPW - 1);
@@ -798,7 +797,7 @@ hipError_t launch_gmp_tga(const DecodeArgs &a, hipStream_t stream) {
     uint32_t in_upper[4] = {0u, 0u, 0u, 0u};  // of G, NT, GS and the column blocks
     if constexpr (kOwnTiles > 0) {
         const OwnBorders b = own_borders(*a.lora_sides, NT, T);
-        col_blocks = b.blocks1 + (NT - b.end1 + T - 1) / T;
+        col_blocks = own_column_blocks(b, NT, T);
         in_upper[0] = (uint32_t)b.blocks0 << 16;
         in_upper[1] = (uint32_t)b.end0 << 16;
         in_upper[2] = (uint32_t)b.end1 << 16;

@@ -190,7 +190,6 @@ struct MidShape {
     int rows, G, NT;
     uint32_t slices, layout;
     int col_blocks;
-    int end0 = 0, blocks0 = 0, end1 = 0, blocks1 = 0;  // a projection of each block's own: where the adapters' sides meet, in tiles and blocks
     __device__ __forceinline__ int GS() const { return slices & 0xFFFF; }
     __device__ __forceinline__ int KS() const { return slices >> 16; }
     __device__ __forceinline__ int full_waves() const { return layout & 255; }               // wavefronts of GPW groups
@@ -290,13 +289,8 @@ __device__ __forceinline__ void mid_block(
     // are slow when they meet in one die's L2).
     int cb = bx + (shape.is(kMidColShift) ? ks : 0);
     if (cb >= ncb) cb -= ncb;  // at most three past the end, of four blocks or more
-    int tf = cb * (2 * TP), tile_end = NT;  // first 16-column tile of the block; tiles from tile_end on are not its own
-    if constexpr (kMidOwn > 0) {  // the blocks of a side of the adapters end where it does: no block has columns of two
-        const int before = cb < shape.blocks0 ? 0 : (cb < shape.blocks1 ? shape.blocks0 : shape.blocks1);
-        const int from = cb < shape.blocks0 ? 0 : (cb < shape.blocks1 ? shape.end0 : shape.end1);
-        tile_end = cb < shape.blocks0 ? shape.end0 : (cb < shape.blocks1 ? shape.end1 : NT);
-        tf = from + (cb - before) * (2 * TP);
-    }
+    const BlockTiles tiles = mid_block_tiles(cb, TP, NT);
+    const int tf = tiles.first, tile_end = tiles.end;
     // the first `fw` wavefronts own GPW groups each, the others GPW - 1; the last slice may have fewer groups
     // than the others (K in groups not a multiple of the slices) and then fewer wavefronts of GPW
     const int fw = ks == KS - 1 ? shape.last_full_waves() : shape.full_waves();
@@ -907,10 +901,7 @@ __global__ __launch_bounds__((kMidWavesOf<TP, ROW_BLOCKS, LORA> * 64)) void w4a1
     const uint16_t *__restrict__ A_all, const u32x4 *__restrict__ B, const uint16_t *__restrict__ S,
     int rows, int G, int NT, uint32_t slices, uint32_t layout, int col_blocks, uint16_t *__restrict__ C_all,
     float *partial_all, int *counters_all, MidLow lo) {
-    MidShape shape{rows, G, NT, slices, layout, col_blocks};
-    if constexpr (kMidOwn > 0)  // 16 bits each, the upper ones say where the sides of the adapters meet
-        shape = MidShape{rows & 0xFFFF, G & 0xFFFF, NT & 0xFFFF, slices, layout, col_blocks & 0xFFFF, (int)((uint32_t)NT >> 16), (int)((uint32_t)G >> 16),
-                         (int)((uint32_t)rows >> 16), (int)((uint32_t)col_blocks >> 16)};
+    const MidShape shape{rows, G, NT, slices, layout, col_blocks};
     if constexpr (ROW_BLOCKS != kMidRowBlocksByRun) {
         mid_block<TP, GPW, LORA, ROW_BLOCKS>(A_all, B, S, C_all, partial_all, counters_all, shape, lo);
     } else {
@@ -945,16 +936,9 @@ hipError_t launch_mid_tgs(const MidArgs &a, hipStream_t stream) {
     lo.r_total = a.r_total;
     lo.rp = (a.r_total + 15) / 16 * 16;
     lo.slices = a.lora_slices;
-    int col_blocks = (NT + 2 * TP - 1) / (2 * TP);
-    uint32_t in_upper[4] = {0u, 0u, 0u, 0u};  // of rows, G, NT and the column blocks
+    const int col_blocks = (NT + 2 * TP - 1) / (2 * TP);
 #if KILN_MID_LORA >= 3
     lo.own = own_args(a);
-    const OwnBorders b = own_borders(*a.lora_sides, NT, 2 * TP);
-    col_blocks = b.blocks1 + (NT - b.end1 + 2 * TP - 1) / (2 * TP);
-    in_upper[0] = (uint32_t)b.end1 << 16;
-    in_upper[1] = (uint32_t)b.blocks0 << 16;
-    in_upper[2] = (uint32_t)b.end0 << 16;
-    in_upper[3] = (uint32_t)b.blocks1 << 16;
 #endif
     dim3 grid(col_blocks, a.KS, runs);
 #if KILN_MID_LORA == 2
@@ -978,8 +962,8 @@ hipError_t launch_mid_tgs(const MidArgs &a, hipStream_t stream) {
                             (a.Gs == 1 ? kMidColumnScales : 0u) | (a.swiglu ? kMidSwiglu : 0u) |
                             (a.flagged ? kMidFlagged | (exchange_column_shift(col_blocks) ? kMidColShift : 0u) : 0u);
     w4a16_mid_kernel<TP, GPW, kMidLora, ROW_BLOCKS><<<grid, a.waves * 64, a.waves * (kMidSlotBytes + kMidOwn * kMidOwnBytes), stream>>>(
-        (const uint16_t *)a.A, (const u32x4 *)a.B, (const uint16_t *)a.S, a.M | in_upper[0], a.K / kGroupK | in_upper[1], NT | in_upper[2],
-        (uint32_t)a.GS | (uint32_t)a.KS << 16, layout, col_blocks | in_upper[3], (uint16_t *)a.C, a.partial, a.counters, lo);
+        (const uint16_t *)a.A, (const u32x4 *)a.B, (const uint16_t *)a.S, a.M, a.K / kGroupK, NT,
+        (uint32_t)a.GS | (uint32_t)a.KS << 16, layout, col_blocks, (uint16_t *)a.C, a.partial, a.counters, lo);
     return hipGetLastError();
 }
 
@@ -1070,10 +1054,10 @@ bool mid_plan_ok(const MidArgs &a) {
     const int G = a.K / kGroupK;
     // slices of GS groups; the last one may be shorter (11008 = 86 groups = 29 + 29 + 28)
     if (a.KS < 1 || a.KS > 0x7FFF || a.GS < 1 || a.KS * a.GS < G || (a.KS - 1) * a.GS >= G) return false;
-    if (a.own_tiles > 0) {  // (16 bits for each of the sizes; a wavefront for every 16 ranks of a row block, with groups of its own:
-                            // one without has not fetched the rows of B_cat)
+    if (a.own_tiles > 0) {  // (a wavefront for every 16 ranks of a row block, with groups of its own: one without has not
+                            // fetched the rows of B_cat)
         const int row_blocks = a.M > 32 ? 2 : 1;
-        if (a.own_tiles > 2 || a.M > 0xFFFF || a.N / kTileN > 0xFFFF || G > 0xFFFF || (row_blocks == 2 && a.pairs == 3) ||
+        if (a.own_tiles > 2 || (row_blocks == 2 && a.pairs == 3) ||
             (row_blocks == 2 && a.pairs == 2 && a.GS > 2 * a.waves) || a.waves < a.own_tiles * row_blocks ||
             G - (a.KS - 1) * a.GS < a.own_tiles * row_blocks || a.waves > mid_own_max_waves(a.own_tiles))
             return false;
@@ -1093,8 +1077,7 @@ bool mid_flagged_ok(const MidArgs &a) {
     return a.KS > 1 && a.KS <= kMidFlaggedSlices && a.waves >= (a.own_tiles > 0 && a.M <= 32 ? kMidWaves / 2 : kMidWaves);
 }
 
-// (a projection of each block's own: up to two more, where sides of the adapters meet inside a block)
-int mid_column_blocks(const MidArgs &a) { return (a.N / kTileN + 2 * a.pairs - 1) / (2 * a.pairs) + (a.own_tiles > 0 ? 2 : 0); }
+int mid_column_blocks(const MidArgs &a) { return (a.N / kTileN + 2 * a.pairs - 1) / (2 * a.pairs); }
 
 size_t mid_partial_bytes(const MidArgs &a) {
     if (a.KS <= 1) return 0;

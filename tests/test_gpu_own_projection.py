@@ -134,6 +134,72 @@ def test_more_than_four_adapters_side_by_side(k, widths, ranks, m):
         assert not bool(out[-1].isfinite().any())
 
 
+# (k, K slices, columns, (rank, first column, columns) of each side): sides that begin inside a block of one to three pairs of
+# tiles, on an odd tile, inside a tile, behind columns of no side
+SIDES_ANYWHERE = [
+    (1024, 1, 1024, ((8, 0, 272), (8, 272, 752))),
+    (1024, 2, 1024, ((8, 0, 48), (16, 48, 208), (8, 256, 768))),
+    (2048, 2, 1024, ((16, 0, 528), (16, 528, 496))),
+    (640, 1, 768, ((8, 16, 16), (8, 48, 400), (16, 496, 256))),
+    (1024, 1, 768, ((8, 0, 264), (8, 264, 100), (8, 381, 387))),
+    (2048, 2, 1024, ((8, 0, 528), (8, 528, 496))),
+    (2304, 3, 512, ((24, 0, 496), (8, 496, 16))),
+]
+# (rows, pairs of tiles per block, one of those): with two row blocks three pairs have no instance, and slices meet in blocks of
+# eight wavefronts, which two rank tiles leave no room for
+SIDES_ANYWHERE_CASES = [(m, pairs, i) for m in (17, 20, 33, 64, 100) for pairs in (1, 2, 3) for i, (_, ks, _, places) in enumerate(SIDES_ANYWHERE)
+                        if m <= 32 or (pairs < 3 and (ks == 1 or sum(p[0] for p in places) <= 16))]
+
+
+def _side_table(adapters, places):
+    at = [(a.a_cat.data_ptr(), a.b_cat.data_ptr()) for a in adapters] if adapters else [(16, 16)] * len(places)
+    return (Side * len(places))(*(Side(*ab, r, first, rows) for ab, (r, first, rows) in zip(at, places)))
+
+
+def _assert_own(L, m, n, k, ks, pairs, places):
+    L.kiln_w4a16_debug_mid(1, pairs, ks)
+    L.kiln_w4a16_debug_lora_fold(3)
+    plan = (ctypes.c_int * 4)()
+    blocks = L.kiln_w4a16_debug_adapter_blocks(m, n, k, 256, _side_table(None, places), len(places), 0, len(places), plan, 4)
+    assert (blocks, *plan) == (-(-n // (32 * pairs)), 2, 2 * pairs, ks, (sum(r for r, _, _ in places) + 15) // 16)
+
+
+def test_sides_that_begin_anywhere_are_projected_by_every_block():
+    L = _lib.load_tuning()
+    for m, pairs, i in SIDES_ANYWHERE_CASES:
+        k, ks, n, places = SIDES_ANYWHERE[i]
+        _assert_own(L, m, n, k, ks, pairs, places)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,pairs,i", SIDES_ANYWHERE_CASES)
+def test_sides_that_begin_anywhere_from_17_rows_on(m, pairs, i):
+    L, (k, ks, n, places) = _lib.load_tuning(), SIDES_ANYWHERE[i]
+    gen = torch.Generator(device="cuda").manual_seed(k + n + m)
+    w = _packed(gen, k, n, 128 if pairs == 2 else -1)
+    adapters = [_all_adapters(gen, k, (rows,), ((r,),))[0] for r, _, rows in places]
+    adapters = [lora.StackedLora(a.a_cat, a.b_cat, a.ranks, (0.5 + 0.25 * i,)) for i, a in enumerate(adapters)]
+    firsts = [first for _, first, _ in places]
+    x = torch.randn(m, k, device="cuda", generator=gen).bfloat16()
+    sides = _side_table(adapters, places)
+    ranks, scales = sum((a.ranks for a in adapters), ()), sum((a.scales for a in adapters), ())
+    a_cat, b_cat, col = torch.cat([a.a_cat for a in adapters]).contiguous(), torch.zeros(n, sum(ranks), dtype=torch.bfloat16, device="cuda"), 0
+    for a, (r, first, rows) in zip(adapters, places):
+        b_cat[first:first + rows, col:col + r] = a.b_cat
+        col += r
+    _assert_own(L, m, n, k, ks, pairs, places)
+    stream = torch.cuda.current_stream().cuda_stream
+    ws = marlin_gemm._workspace(x.device, stream, L.kiln_w4a16_workspace_bytes(m, n, k))
+    # rows behind the last that must stay as they are: a block that stored past its columns would reach them
+    out = torch.full((m + 1, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+    assert L.kiln_w4a16_gemm_adapter_sides(x.data_ptr(), w.b_packed.data_ptr(), out.data_ptr(), w.scales.data_ptr(), m, n, k, ws.data_ptr(), w.groupsize,
+                                           x.device.index, stream, sides, len(places), 0, len(ranks), (ctypes.c_int * len(ranks))(*ranks),
+                                           (ctypes.c_float * len(ranks))(*scales)) == _lib.OK
+    want = marlin_gemm.marlin_w4a16_gemm_lora(x, w.b_packed, w.scales, w.groupsize, a_cat, b_cat, ranks, scales)
+    assert bool(out[m].isnan().all()) and torch.equal(out[:m].view(torch.int16), want.view(torch.int16))
+    _assert_close(out[:m], *_reference(x, w, list(zip(adapters, firsts))))
+
+
 def test_ranks_that_are_taken_as_they_are():
     """Multiples of 8 always; of 4 where blocks project by themselves, up to 32 and on the kernels of few rows; nothing else."""
     takes = _lib.load().kiln_w4a16_takes_rank
