@@ -711,12 +711,15 @@ constexpr OwnKind own_kind_of(int lora) {
 // blocks, whose chain of round trips ends 5.5 to 6 us after the launch begins but runs beside the streaming blocks: a launch
 // that takes longer than that hides it, where a block's own projection adds its share of A_cat to what the block stages --
 // of its own side only, where more than four adapters lie side by side (kind.sides), which therefore goes further.  The lines
-// were fitted to both ways, forced, with both plans' costs: on 15 shapes with stacked adapters of 8 to 32 ranks and on the four
-// calls of a layer at hidden 1024, 1536, 2560 and 4096 with adapters of 16, 32 and 8 ranks a projection, at 1 to 16 rows.  The
-// choice takes 8 to 9 % less time than the first blocks alone, the better of the two each time 9 to 10 %; q | k | v of 2560 with two
-// adapters of rank 8 each at 11 rows 7.2 against 7.9 us, of 4096 with two of rank 4 9.6 against 10.3 the other way (kind.sides:
-// costs of 7.3 and 9.6); the worst loss is 7 % (4096 -> 4096 with 8 ranks at one row, 5.7 -> 6.1 us).  What a rank that is no
-// multiple of 8 would cost otherwise is a launch that pads it (3 us).
+// were drawn by both ways, forced, with both plans' costs, on some 100 shapes of K 1024 ... 9216 with stacked adapters of 8 to 32
+// ranks at 1 to 16 rows.  The fewer ranks, the sooner the chain ends (in launches that are shorter, 5.2 ... 6.3 us with 8 ranks, 5.4 ...
+// 6.6 with 16, 5.8 ... 7.3 with 32), so the lower the line: 5.25 with 8 (at 5.6 it took 1536 -> 12288 at one row from 6.0 to 6.4 us,
+// 4096 -> 3584 from 5.9 to 6.2, 2560 -> 7936 at 8 rows from 6.55 to 6.85), 5.55 with 16, 5.6 beyond.  Longer launches have to be ahead by
+// 1 us of cost: by less, blocks of one tile that fill the chip lost to the other way's two tiles (4096 -> 4096 with 8 ranks at one row
+// 6.15 -> 6.45 us, 5120 -> 4096 6.75 -> 7.15).  As it stands nothing measured is slower than by the first blocks by more than 3 %.
+// kind.sides: 210 calls of a layer at six hidden sizes 1024 ... 4096 with four to six adapters take 6.7 % less time than by the first
+// blocks, the better of the two each time 7.0 % less, the worst is 4 % more (gate | up of 2048 -> 5632 with six at 11 rows, 7.5 -> 7.8 us).
+// What a rank that is no multiple of 8 would cost otherwise is a launch that pads it (3 us).
 bool plan_own_projection(int m, int n, int k, int cus, const OwnKind &kind, DecodePlan *own) {
     if (g_tune.gmp_tiles > 0)
         return (g_tune.gmp_ks == 1 || flagged_exchange_fits(g_tune.gmp_ks, n)) &&
@@ -726,7 +729,8 @@ bool plan_own_projection(int m, int n, int k, int cus, const OwnKind &kind, Deco
     DecodePlan other;
     if (g_tune.lora_fold == 3 || !plan_decode_gmp(m, n, k, cus, true, &other, 0, &first_blocks)) return true;
     if (kind.general) return cost <= std::max(first_blocks + 2.f, 8.f);
-    return cost <= std::max(first_blocks - 0.5f, kind.sides ? 7.4f : 5.6f);
+    if (kind.sides) return cost <= std::max(first_blocks - 0.5f, 7.4f);
+    return cost <= std::max(first_blocks - 1.0f, kind.eights == 1 ? 5.25f : kind.eights == 2 ? 5.55f : 5.6f);
 }
 
 // The plan of the mid-M kernel with the projection in the launch's first blocks where they fit (its fold), or in front.

@@ -58,6 +58,25 @@ def test_automatic_plans(n, k, rank):
     assert own > 0
 
 
+def _own(m, k, n, rank):
+    plan, _ = _blocks(_lib.load(), m, n, k, [(rank, 0, n)], 1)
+    return plan[3] > 0
+
+
+@pytest.mark.parametrize("m,k,n,rank,own", [
+    # short launches, the fewer ranks the shorter
+    (1, 1024, 4096, 8, 1), (16, 1024, 4096, 8, 1), (1, 2560, 2560, 8, 1), (1, 2048, 2048, 32, 1), (1, 2560, 4096, 8, 1), (11, 1536, 8192, 8, 1),
+    # 8 and 16 ranks whose projection in the first blocks ends before the launch would anyway
+    (1, 1536, 12288, 8, 0), (8, 1536, 12288, 8, 0), (1, 1536, 12288, 16, 0), (1, 4096, 3584, 8, 0), (8, 2560, 7936, 8, 0),
+    # longer ones: blocks of one tile that fill the chip against two tiles a block
+    (1, 4096, 4096, 8, 0), (11, 4096, 4096, 8, 0), (1, 5120, 4096, 8, 0), (8, 5120, 4096, 8, 0), (1, 6144, 4096, 8, 0),
+    # ... and those that are ahead by more
+    (1, 8192, 4096, 8, 1), (4, 5504, 7936, 16, 1),
+])
+def test_where_blocks_of_up_to_16_rows_project_by_themselves(m, k, n, rank, own):
+    assert _own(m, k, n, rank) == bool(own)
+
+
 @pytest.mark.parametrize("pairs", [1, 2, 3])
 def test_plans_of_every_width_from_17_rows_on(pairs):
     L, n, k = _lib.load_tuning(), 1024, 1024
