@@ -707,6 +707,16 @@ constexpr OwnKind own_kind_of(int lora) {
     return OwnKind{v % 4 + 1, (v & 4) != 0, (v & 8) != 0};
 }
 
+// Does a call of up to 16 rows with adapters, by this plan of the private-staging kernel, go to the mid-M kernel instead?  Where
+// that launch would have to take the projection from a launch in front -- its blocks fill the chip and leave the producers
+// no units of their own -- and the mid-M kernel need not: 11008 -> 4096, 256 blocks of two tiles in two slices, with two
+// adapters 15.3...17.0 us at 1...16 rows, there 13.9...14.4.
+bool few_rows_on_mid(const DecodePlan &plan, int m, int k, int cus) {
+    const int steps = k / 32, kz0 = lora_project_slices(m, k), per = ((steps + kz0 - 1) / kz0 + 3) / 4 * 4;
+    const int kz = (steps + per - 1) / per, blocks = plan.BPS * plan.KS;
+    return blocks <= cus && blocks + kz > cus;
+}
+
 // Does every block project x onto its adapters by itself, and by which plan?  Against the projection in the launch's first
 // blocks, whose chain of round trips ends 5.5 to 6 us after the launch begins but runs beside the streaming blocks: a launch
 // that takes longer than that hides it, where a block's own projection adds its share of A_cat to what the block stages --
@@ -714,12 +724,18 @@ constexpr OwnKind own_kind_of(int lora) {
 // were drawn by both ways, forced, with both plans' costs, on some 100 shapes of K 1024 ... 9216 with stacked adapters of 8 to 32
 // ranks at 1 to 16 rows.  The fewer ranks, the sooner the chain ends (in launches that are shorter, 5.2 ... 6.3 us with 8 ranks, 5.4 ...
 // 6.6 with 16, 5.8 ... 7.3 with 32), so the lower the line: 5.25 with 8 (at 5.6 it took 1536 -> 12288 at one row from 6.0 to 6.4 us,
-// 4096 -> 3584 from 5.9 to 6.2, 2560 -> 7936 at 8 rows from 6.55 to 6.85), 5.55 with 16, 5.6 beyond.  Longer launches have to be ahead by
-// 1 us of cost: by less, blocks of one tile that fill the chip lost to the other way's two tiles (4096 -> 4096 with 8 ranks at one row
-// 6.15 -> 6.45 us, 5120 -> 4096 6.75 -> 7.15).  As it stands nothing measured is slower than by the first blocks by more than 3 %.
+// 4096 -> 3584 from 5.9 to 6.2, 2560 -> 7936 at 8 rows from 6.55 to 6.85), 5.55 with 16, 5.6 beyond and in K slices (4096 -> 1024 in
+// four, a cost of 5.28, 5.85 -> 5.3).  Longer launches have to be ahead by half a microsecond of cost, by one where blocks of all of K
+// fill the chip: those lost by less to the other way's wider blocks (4096 -> 4096 with 8 ranks at one row 6.15 -> 6.45 us, 5120 ->
+// 4096 6.75 -> 7.15; while 5504 -> 7936 with 24, 248 blocks ahead by 0.8, gains: 12.6 -> 11.1).  As it stands nothing measured is
+// slower than by the first blocks by more than 3 %.
 // kind.sides: 210 calls of a layer at six hidden sizes 1024 ... 4096 with four to six adapters take 6.7 % less time than by the first
 // blocks, the better of the two each time 7.0 % less, the worst is 4 % more (gate | up of 2048 -> 5632 with six at 11 rows, 7.5 -> 7.8 us).
 // What a rank that is no multiple of 8 would cost otherwise is a launch that pads it (3 us).
+// Plans of more than one round of blocks, which long weights have, are ahead up to a cost of 14 only (11008 -> 4096 with 8 ranks at one
+// row 14.5 -> 13.6 us, 13568 -> 4096 15.3 -> 15.1, 18176 -> 4096 17.0 -> 17.6), and never where the call would go to the mid-M kernel
+// (few_rows_on_mid: 11008 -> 4096 at 16 rows 13.3 there against 16.4, 12032 -> 4096 13.4 against 17.5, 6016 -> 8192 13.8 against
+// 16.7); a rank that is padded for it otherwise, up to a cost of 15.
 bool plan_own_projection(int m, int n, int k, int cus, const OwnKind &kind, DecodePlan *own) {
     if (g_tune.gmp_tiles > 0)
         return (g_tune.gmp_ks == 1 || flagged_exchange_fits(g_tune.gmp_ks, n)) &&
@@ -728,9 +744,15 @@ bool plan_own_projection(int m, int n, int k, int cus, const OwnKind &kind, Deco
     if (!plan_decode_gmp(m, n, k, cus, false, own, kind.eights, &cost)) return false;
     DecodePlan other;
     if (g_tune.lora_fold == 3 || !plan_decode_gmp(m, n, k, cus, true, &other, 0, &first_blocks)) return true;
+    if (own->BPS * own->KS > cus) {
+        const bool on_mid = few_rows_on_mid(other, m, k, cus);
+        if (kind.general ? on_mid && cost > 15.f : on_mid || cost > 14.f) return false;
+    }
     if (kind.general) return cost <= std::max(first_blocks + 2.f, 8.f);
     if (kind.sides) return cost <= std::max(first_blocks - 0.5f, 7.4f);
-    return cost <= std::max(first_blocks - 1.0f, kind.eights == 1 ? 5.25f : kind.eights == 2 ? 5.55f : 5.6f);
+    const bool fills = own->KS == 1 && own->BPS <= cus && own->BPS >= cus - 2;
+    const float line = own->KS > 1 || kind.eights > 2 ? 5.6f : kind.eights == 2 ? 5.55f : 5.25f;
+    return cost <= std::max(first_blocks - (fills ? 1.0f : 0.5f), line);
 }
 
 // The plan of the mid-M kernel with the projection in the launch's first blocks where they fit (its fold), or in front.
@@ -802,17 +824,11 @@ void plan_gemm(int m, int n, int k, int cus, int thread_k, int thread_n, int lor
     // adapters whose stacked rank is a multiple of 8: the low-rank term is added from a projection that runs
     // in the launch's first blocks where it fits, else from one launched in front)
     // (a call pinned to a block shape of the matrix-core kernel goes there)
-    // (with adapters also below 17 rows where the small-M launch would have to take the projection from a launch in
-    // front -- its blocks fill the chip and leave the producers no units of their own -- and this kernel need not:
-    // 11008 -> 4096, 256 blocks of two tiles in two slices, with two adapters 15.3...17.0 us at 1...16 rows, here 13.9...14.4)
+    // (with adapters also below 17 rows: few_rows_on_mid)
     bool few_rows_here = false;
     if (lora == 1 && m <= 16 && g_tune.lora_fold != 0 && g_tune.lora_fold != 2 && g_tune.gmp_tiles == 0 && thread_k <= 0 && thread_n <= 0) {
         DecodePlan dp;
-        if (plan_decode_gmp(m, n, k, cus, true, &dp)) {
-            const int steps = k / 32, kz0 = lora_project_slices(m, k), per = ((steps + kz0 - 1) / kz0 + 3) / 4 * 4;
-            const int kz = (steps + per - 1) / per, blocks = dp.BPS * dp.KS;
-            few_rows_here = blocks <= cus && blocks + kz > cus;
-        }
+        if (plan_decode_gmp(m, n, k, cus, true, &dp)) few_rows_here = few_rows_on_mid(dp, m, k, cus);
     }
     if (lora != 2 && thread_k <= 0 && thread_n <= 0 && g_tune.mid != 0 &&
         (g_tune.mid == 1 ||

@@ -71,10 +71,20 @@ def _own(m, k, n, rank):
     # longer ones: blocks of one tile that fill the chip against two tiles a block
     (1, 4096, 4096, 8, 0), (11, 4096, 4096, 8, 0), (1, 5120, 4096, 8, 0), (8, 5120, 4096, 8, 0), (1, 6144, 4096, 8, 0),
     # ... and those that are ahead by more
-    (1, 8192, 4096, 8, 1), (4, 5504, 7936, 16, 1),
+    (1, 8192, 4096, 8, 1), (4, 5504, 7936, 16, 1), (1, 5504, 7936, 24, 1), (1, 4096, 1024, 8, 1), (8, 8192, 2048, 8, 1),
+    # two rounds of blocks against one, and against the mid-M kernel, where such a call goes from 8 rows on
+    (1, 11008, 4096, 8, 1), (4, 12032, 4096, 8, 1), (1, 18176, 4096, 8, 0), (1, 9088, 8192, 8, 0),
+    (8, 11008, 4096, 8, 0), (16, 11008, 4096, 8, 0), (16, 12032, 4096, 8, 0), (11, 5504, 8192, 8, 0), (16, 7808, 8192, 8, 0),
+    (16, 5504, 7936, 8, 1), (11, 5504, 7936, 32, 1),
 ])
 def test_where_blocks_of_up_to_16_rows_project_by_themselves(m, k, n, rank, own):
     assert _own(m, k, n, rank) == bool(own)
+
+
+def test_a_rank_that_is_padded_otherwise_takes_two_rounds_of_blocks_for_longer():
+    takes = _lib.load().kiln_w4a16_takes_rank
+    assert [takes(m, 4096, 11008, 4, -1) for m in (1, 8, 16)] == [1, 1, 0]
+    assert [takes(m, 4096, 12032, 4, -1) for m in (1, 8, 16)] == [1, 1, 0]
 
 
 @pytest.mark.parametrize("pairs", [1, 2, 3])
