@@ -58,14 +58,22 @@ struct BlockTiles {
 // all ranks, and the row of B_cat is found per column; blocks that ended where a side does had half a pair left there).
 __host__ __device__ constexpr BlockTiles mid_block_tiles(int column_block, int pairs, int tiles) { return {column_block * 2 * pairs, tiles}; }
 
-// Where the second and the third side begin, in tiles and in blocks of T tiles: a block has columns of one of them.
+// Does a block that projects x onto the adapters by itself have the ranks of its own columns' side only, and end where that side
+// does?  Up to 16 rows and from five adapters side by side on.  Up to four adapters, and any number beyond 16 rows, give the
+// bits of the stacked set: every block has all ranks, in their places, and is a plain call's; so is one of gate | up, whose
+// every tile has columns of both sides.
+constexpr int kLoraFoldMaxAdapters = 4;
+inline bool own_blocks_end_with_sides(const AdapterSides &s, int adapters, int rows) {
+    return !s.interleaved && s.count > 1 && adapters > kLoraFoldMaxAdapters && rows <= 16;
+}
+// Where the second and the third side begin, in tiles and in blocks of T tiles: such a block has columns of one of them.
 struct OwnBorders {
     int end0, blocks0, end1, blocks1;
 };
-inline OwnBorders own_borders(const AdapterSides &s, int NT, int T) {
+inline OwnBorders own_borders(const AdapterSides &s, bool end_with_sides, int NT, int T) {
     OwnBorders b{NT, 0, NT, 0};
-    if (!s.interleaved && s.count > 1) b.end0 = s.first[1] / kTileN;
-    if (!s.interleaved && s.count > 2) b.end1 = s.first[2] / kTileN;
+    if (end_with_sides) b.end0 = s.first[1] / kTileN;
+    if (end_with_sides && s.count > 2) b.end1 = s.first[2] / kTileN;
     b.blocks0 = (b.end0 + T - 1) / T;
     b.blocks1 = b.blocks0 + (b.end1 - b.end0 + T - 1) / T;
     return b;

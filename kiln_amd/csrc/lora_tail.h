@@ -192,7 +192,6 @@ struct LoraSidesFold : LoraFold {
     int ends[8];             // read with constant indices only
     float scales[8];
 };
-constexpr int kLoraFoldMaxAdapters = 4;
 // The adapters of a call whose blocks project x onto them by themselves (own_tiles): the sides of LoraSides, one for a
 // stacked set, prepared so that a row or a unit is found without a branch.  A side that is absent has no columns.
 // (Plain members, not arrays: what is picked from an array by a condition goes through scratch memory.)
@@ -272,9 +271,7 @@ struct OwnWindow {  // the stacked rank columns that the block's columns have a 
 template <class Args>  // DecodeArgs, MidArgs
 OwnArgs own_args(const Args &d) {
     const AdapterSides &h = *d.lora_sides;
-    // Up to four adapters, and any number beyond 16 rows, give the bits of the stacked set: every block has all ranks, in
-    // their places.
-    const bool all = h.interleaved || d.lora_adapters <= kLoraFoldMaxAdapters || d.M > 16;
+    const bool all = !own_blocks_end_with_sides(h, d.lora_adapters, d.M);
     uint64_t a[3] = {}, b[3] = {};
     int col[4] = {}, first[3] = {}, end[3] = {}, key[3] = {}, span[3] = {};
     for (int i = 0; i < kMaxAdapterSides; ++i) {

@@ -299,9 +299,9 @@ bool flagged_exchange_fits(int ks, int n) {
 // slices: 7.1 us with the parts as their own arrival flags, 8.4 through counters; four, six, eight
 // slices through counters 9.2, 9.9, 11.2).  A call with adapters plans for the chip less the blocks
 // that project x onto the adapters, so that the projection can ride in the same launch.
-// (own > 0: one whose blocks project x onto their own adapters, this many times eight ranks; its blocks are a plain call's,
-// lora is false.)
-bool plan_decode_gmp(int m, int n, int k, int cus, bool lora, DecodePlan *best, int own = 0, float *cost_of_best = nullptr) {
+// (own > 0: one whose blocks project x onto their own adapters, this many times eight ranks; its blocks are a plain call's, or
+// end at `borders` places where a side of the adapters does; lora is false.)
+bool plan_decode_gmp(int m, int n, int k, int cus, bool lora, DecodePlan *best, int own = 0, int borders = 0, float *cost_of_best = nullptr) {
     const int G = k / kGroupK, NT = n / kTileN;
     // (a caller may name a part of the chip, `sms`: never plan for less than one unit)
     if (lora && g_tune.lora_fold != 0 && cus > lora_project_slices(m, k)) cus -= lora_project_slices(m, k);
@@ -326,7 +326,7 @@ bool plan_decode_gmp(int m, int n, int k, int cus, bool lora, DecodePlan *best, 
                 DecodePlan p;
                 if (waves == most && (lora || T != 1 || GS % 16 != 0) && gmp_plan(m, n, k, T, 12, ks, lora, &p, own)) continue;
                 if (!gmp_plan(m, n, k, T, waves, ks, lora, &p, own)) continue;
-                const int rounds = ceil_div((ceil_div(NT, T) + (own > 0 && T > 1 ? 2 : 0)) * ks, cus);  // (blocks end at a side's end)
+                const int rounds = ceil_div((ceil_div(NT, T) + (T > 1 ? borders : 0)) * ks, cus);
                 // The exchange: through counters 0.4 us per slice + 1.2; with the parts as their own
                 // arrival flags it grows with the tiles polled, 0.0037 us per (slice - 1) and tile
                 // (down projection, 160 tiles: 0.4 / 1.1 / 1.9 us at two / three / four slices;
@@ -693,65 +693,56 @@ MidArgs mid_args(const MidPlan &mp, int m, int n, int k) {
     return a;
 }
 
-// Kinds of calls with adapters beside choose_decode's 1 and 2: those whose blocks of up to 16 rows may project x onto their
-// columns' adapters by themselves.
+// Kinds of calls with adapters beside choose_decode's 1 and 2: those whose blocks may project x onto their columns' adapters by
+// themselves, on either kernel.
 struct OwnKind {
     int eights;    // the ranks a block has, in eights, 1...4
-    bool sides;    // more than four adapters, not stacked
+    bool sides;    // up to 16 rows: more than four adapters, not stacked
     bool general;  // a rank that is a multiple of 4 only: else the call is of kind 2 (1 if not), or padded to 8 in front
+    int borders;   // between sides with which blocks end (own_blocks_end_with_sides), 0...2
 };
 constexpr int kFirstOwnKind = 3;
-constexpr int own_kind(const OwnKind &o) { return kFirstOwnKind + (o.eights - 1) + (o.sides ? 4 : 0) + (o.general ? 8 : 0); }
+constexpr int own_kind(const OwnKind &o) { return kFirstOwnKind + (o.eights - 1) + (o.sides ? 4 : 0) + (o.general ? 8 : 0) + 16 * o.borders; }
 constexpr OwnKind own_kind_of(int lora) {
     const int v = lora - kFirstOwnKind;
-    return OwnKind{v % 4 + 1, (v & 4) != 0, (v & 8) != 0};
-}
-
-// Does a call of up to 16 rows with adapters, by this plan of the private-staging kernel, go to the mid-M kernel instead?  Where
-// that launch would have to take the projection from a launch in front -- its blocks fill the chip and leave the producers
-// no units of their own -- and the mid-M kernel need not: 11008 -> 4096, 256 blocks of two tiles in two slices, with two
-// adapters 15.3...17.0 us at 1...16 rows, there 13.9...14.4.
-bool few_rows_on_mid(const DecodePlan &plan, int m, int k, int cus) {
-    const int steps = k / 32, kz0 = lora_project_slices(m, k), per = ((steps + kz0 - 1) / kz0 + 3) / 4 * 4;
-    const int kz = (steps + per - 1) / per, blocks = plan.BPS * plan.KS;
-    return blocks <= cus && blocks + kz > cus;
+    return OwnKind{v % 4 + 1, (v & 4) != 0, (v & 8) != 0, v / 16};
 }
 
 // Does every block project x onto its adapters by itself, and by which plan?  Against the projection in the launch's first
 // blocks, whose chain of round trips ends 5.5 to 6 us after the launch begins but runs beside the streaming blocks: a launch
 // that takes longer than that hides it, where a block's own projection adds its share of A_cat to what the block stages --
 // of its own side only, where more than four adapters lie side by side (kind.sides), which therefore goes further.  The lines
-// were drawn by both ways, forced, with both plans' costs, on some 100 shapes of K 1024 ... 9216 with stacked adapters of 8 to 32
-// ranks at 1 to 16 rows.  The fewer ranks, the sooner the chain ends (in launches that are shorter, 5.2 ... 6.3 us with 8 ranks, 5.4 ...
-// 6.6 with 16, 5.8 ... 7.3 with 32), so the lower the line: 5.25 with 8 (at 5.6 it took 1536 -> 12288 at one row from 6.0 to 6.4 us,
-// 4096 -> 3584 from 5.9 to 6.2, 2560 -> 7936 at 8 rows from 6.55 to 6.85), 5.55 with 16, 5.6 beyond and in K slices (4096 -> 1024 in
-// four, a cost of 5.28, 5.85 -> 5.3).  Longer launches have to be ahead by half a microsecond of cost, by one where blocks of all of K
-// fill the chip: those lost by less to the other way's wider blocks (4096 -> 4096 with 8 ranks at one row 6.15 -> 6.45 us, 5120 ->
-// 4096 6.75 -> 7.15; while 5504 -> 7936 with 24, 248 blocks ahead by 0.8, gains: 12.6 -> 11.1).  As it stands nothing measured is
-// slower than by the first blocks by more than 3 %.
+// were drawn by both ways, forced, with both plans' costs, on 150 shapes with stacked adapters of 8 to 32 ranks at 1 to 16 rows:
+// - The fewer ranks, the sooner the chain ends (in launches that are shorter, 5.2 ... 6.3 us with 8 ranks, 5.4 ... 6.6 with 16, 5.8 ...
+//   7.3 with 32), so the lower the line: 5.25 with 8 (at 5.6 it took 4096 -> 3584 at one row from 5.9 to 6.2 us, 2560 -> 7936 at 8 rows
+//   from 6.55 to 6.85), 5.55 with 16, 5.6 beyond and in K slices (4096 -> 1024 in four, a cost of 5.28, 5.85 -> 5.3).
+// - Longer launches have to be ahead by half a microsecond of cost, by one where blocks of all of K fill the chip and the other
+//   way has wider ones: those lost by less (4096 -> 4096 with 8 ranks at one row 6.15 -> 6.45 us, 5120 -> 4096 6.75 -> 7.15, 4096 -> 8192
+//   7.25 -> 7.9; 2048 -> 8192 5.75 -> 5.95, hence the lower line at one row, where the chain is shortest).
+// - In several rounds, blocks of up to three tiles have a compute unit's LDS to themselves where the first way's share it by twos
+//   (6656 -> 16128 with 8 ranks at 8 rows 18.5 -> 20.7, 15104 -> 7936 19.8 -> 23.4): only wider ones (8192 -> 19712 at 16 rows 40 -> 25),
+//   or against five slices and more (9216 -> 15616 at one row 37.5 -> 24).
+// - Three and four slices cost the first way less than it says: 12288 -> 4096 at one row 9.9 against 10.65, 14336 -> 4096 11.0 against 12.0.
+// As it stands 5454 calls of 1 to 100 rows take 4.5 % less time than by the first blocks alone; four of them take more by 3 to 4.4 %
+// (8192 -> 8192 with 8 ranks at one row, 12.4 -> 12.9 us), no other by as much.
 // kind.sides: 210 calls of a layer at six hidden sizes 1024 ... 4096 with four to six adapters take 6.7 % less time than by the first
 // blocks, the better of the two each time 7.0 % less, the worst is 4 % more (gate | up of 2048 -> 5632 with six at 11 rows, 7.5 -> 7.8 us).
 // What a rank that is no multiple of 8 would cost otherwise is a launch that pads it (3 us).
-// Plans of more than one round of blocks, which long weights have, are ahead up to a cost of 14 only (11008 -> 4096 with 8 ranks at one
-// row 14.5 -> 13.6 us, 13568 -> 4096 15.3 -> 15.1, 18176 -> 4096 17.0 -> 17.6), and never where the call would go to the mid-M kernel
-// (few_rows_on_mid: 11008 -> 4096 at 16 rows 13.3 there against 16.4, 12032 -> 4096 13.4 against 17.5, 6016 -> 8192 13.8 against
-// 16.7); a rank that is padded for it otherwise, up to a cost of 15.
 bool plan_own_projection(int m, int n, int k, int cus, const OwnKind &kind, DecodePlan *own) {
     if (g_tune.gmp_tiles > 0)
         return (g_tune.gmp_ks == 1 || flagged_exchange_fits(g_tune.gmp_ks, n)) &&
                gmp_plan(m, n, k, g_tune.gmp_tiles, g_tune.gmp_waves, g_tune.gmp_ks, false, own, kind.eights);
     float cost = 0.f, first_blocks = 0.f;
-    if (!plan_decode_gmp(m, n, k, cus, false, own, kind.eights, &cost)) return false;
+    if (!plan_decode_gmp(m, n, k, cus, false, own, kind.eights, kind.borders, &cost)) return false;
     DecodePlan other;
-    if (g_tune.lora_fold == 3 || !plan_decode_gmp(m, n, k, cus, true, &other, 0, &first_blocks)) return true;
-    if (own->BPS * own->KS > cus) {
-        const bool on_mid = few_rows_on_mid(other, m, k, cus);
-        if (kind.general ? on_mid && cost > 15.f : on_mid || cost > 14.f) return false;
-    }
+    if (g_tune.lora_fold == 3 || !plan_decode_gmp(m, n, k, cus, true, &other, 0, 0, &first_blocks)) return true;
     if (kind.general) return cost <= std::max(first_blocks + 2.f, 8.f);
+    const int blocks = own->BPS * own->KS;
+    if (blocks > cus && own->gm_tiles < 4 && other.KS < 5) return false;
+    if ((other.KS == 3 || other.KS == 4) && own->KS < other.KS) first_blocks -= 1.6f;
     if (kind.sides) return cost <= std::max(first_blocks - 0.5f, 7.4f);
-    const bool fills = own->KS == 1 && own->BPS <= cus && own->BPS >= cus - 2;
-    const float line = own->KS > 1 || kind.eights > 2 ? 5.6f : kind.eights == 2 ? 5.55f : 5.25f;
+    const bool fills = own->KS == 1 && blocks <= cus && blocks >= cus - 2 && other.gm_tiles > own->gm_tiles;
+    const float line = own->KS > 1 || kind.eights > 2 ? 5.6f : kind.eights == 2 ? 5.55f : fills && m == 1 ? 4.8f : 5.25f;
     return cost <= std::max(first_blocks - (fills ? 1.0f : 0.5f), line);
 }
 
@@ -779,13 +770,17 @@ MidPlan plan_mid_lora(int m, int n, int k, int cus) {
 // four calls of a layer at hidden 1024, 1536, 2560 and 4096 with adapters of 8 to 32 ranks at 20, 32, 50, 64 and 100 rows: 14 % less time
 // than the first blocks alone where both exist, the better of the two each time 14.5 % (2048 -> 1024 with 16 ranks at 32 rows 8.2 -> 5.9
 // us, 1024 -> 5632 with 16 9.0 -> 5.4, 9216 -> 2560 at 50 15.1 -> 14.0; 2560 -> 18432 at 20 11.7 against 12.0 the other way, and at 50,
-// where three pairs leave no registers for T and two take another round, 16.5 against 25).
+// where three pairs leave no registers for T and two take another round, 16.5 against 25).  Launches whose blocks just fill the chip
+// are among those that gain: 4096 -> 4096 with 8 ranks at 24 rows 10.8 -> 8.55 us, 1024 -> 8192 8.7 -> 5.8, 2560 -> 8192 9.5 -> 8.6, at 50 rows
+// 12.8 -> 11.5 (the planner once counted two blocks more than they have, and so a second round).  From a cost of 11 on it has to be
+// ahead: 3072 -> 16384 with 16 ranks at 32 rows, level by cost, 12.8 -> 13.45.
 bool plan_mid_own_projection(int m, int n, int k, int cus, const OwnKind &kind, MidPlan *own) {
     *own = plan_mid_waves(m, n, k, cus, false, false, kind.eights);
     if (!own->ok || g_tune.lora_fold == 3) return own->ok;
     const MidPlan other = plan_mid_lora(m, n, k, cus);
     if (!other.ok) return true;
-    return own->cost <= (kind.general ? std::max(other.cost + 2.f, 11.5f) : std::max(other.cost + 0.2f, 9.55f));
+    if (kind.general) return own->cost <= std::max(other.cost + 2.f, 11.5f);
+    return own->cost <= std::max(other.cost + (own->cost > 11.f ? -0.2f : 0.2f), 9.55f);
 }
 
 bool first_blocks_take_sides(int m, int n, int k, int cus);
@@ -824,11 +819,17 @@ void plan_gemm(int m, int n, int k, int cus, int thread_k, int thread_n, int lor
     // adapters whose stacked rank is a multiple of 8: the low-rank term is added from a projection that runs
     // in the launch's first blocks where it fits, else from one launched in front)
     // (a call pinned to a block shape of the matrix-core kernel goes there)
-    // (with adapters also below 17 rows: few_rows_on_mid)
+    // (with adapters also below 17 rows where the small-M launch would have to take the projection from a launch in
+    // front -- its blocks fill the chip and leave the producers no units of their own -- and this kernel need not:
+    // 11008 -> 4096, 256 blocks of two tiles in two slices, with two adapters 15.3...17.0 us at 1...16 rows, here 13.9...14.4)
     bool few_rows_here = false;
     if (lora == 1 && m <= 16 && g_tune.lora_fold != 0 && g_tune.lora_fold != 2 && g_tune.gmp_tiles == 0 && thread_k <= 0 && thread_n <= 0) {
         DecodePlan dp;
-        if (plan_decode_gmp(m, n, k, cus, true, &dp)) few_rows_here = few_rows_on_mid(dp, m, k, cus);
+        if (plan_decode_gmp(m, n, k, cus, true, &dp)) {
+            const int steps = k / 32, kz0 = lora_project_slices(m, k), per = ((steps + kz0 - 1) / kz0 + 3) / 4 * 4;
+            const int kz = (steps + per - 1) / per, blocks = dp.BPS * dp.KS;
+            few_rows_here = blocks <= cus && blocks + kz > cus;
+        }
     }
     if (lora != 2 && thread_k <= 0 && thread_n <= 0 && g_tune.mid != 0 &&
         (g_tune.mid == 1 ||
@@ -998,21 +999,22 @@ struct LoraSpec {
 // The `lora` of plan_gemm for a call: which kernels can take its adapters.  A block of up to 16 rows that projects x onto
 // the adapters by itself does so for all of them, or, where more than four lie side by side, for those that its columns have
 // a term of (up to four, the call is one with the stacked set in every bit: the same choice, plan and places; beyond 16 rows
-// it is whatever their number).  Up to 16 rows blocks end where a side does, whole tiles; beyond, they are what they are without
-// sides, which may begin at any column.
+// it is whatever their number).  The latter's blocks end where a side does, whole tiles; all others are a plain call's, and the
+// sides may begin at any column.
 int lora_kind(const LoraSpec *lora, int m) {
     if (!lora) return 0;
     const int otherwise = lora->r_total % 8 == 0 ? 1 : 2;
     if (m > 4 * mid_max_rows_per_run() || lora->n_adapters > 8 || (g_tune.lora_fold != -1 && g_tune.lora_fold != 3) || lora->r_total % 4 != 0) return otherwise;
-    int ranks = lora->r_total;
-    const bool many = lora->sides && lora->n_adapters > 4 && m <= 16;
-    if (lora->sides && !lora->sides->interleaved) {
+    int ranks = lora->r_total, borders = 0;
+    if (lora->sides && own_blocks_end_with_sides(*lora->sides, lora->n_adapters, m)) {
         const AdapterSides &s = *lora->sides;
-        if (many) ranks = *std::max_element(s.ranks, s.ranks + s.count);
-        for (int i = 0; i < s.count && m <= 16; ++i)
+        ranks = *std::max_element(s.ranks, s.ranks + s.count);
+        borders = s.count - 1;
+        for (int i = 1; i < s.count; ++i)
             if (s.first[i] % kTileN != 0) return otherwise;
     }
-    return ranks <= 32 ? own_kind({(ranks + 7) / 8, many, lora->r_total % 8 != 0}) : otherwise;
+    const bool many = lora->sides && lora->n_adapters > kLoraFoldMaxAdapters && m <= 16;
+    return ranks <= 32 ? own_kind({(ranks + 7) / 8, many, lora->r_total % 8 != 0, borders}) : otherwise;
 }
 
 // Bytes a call of m rows needs, made monotone in m: the largest need of any m' <= m.  The plan
@@ -1531,16 +1533,16 @@ int kiln_w4a16_debug_adapter_blocks(int m, int n, int k, int cus, const kiln_w4a
     if (gp.prefill || (!gp.mid && (gp.launches != 1 || !gp.dl[0].plan.gmp))) return 0;
     const DecodePlan &plan = gp.dl[0].plan;
     const int NT = n / kTileN, per_block = gp.mid ? 2 * gp.mp.pairs : plan.gm_tiles, rank_tiles = gp.mid ? gp.mp.own : plan.own;
-    const OwnBorders borders = own_borders(own, NT, per_block);
-    const bool ends_with_sides = !gp.mid && rank_tiles > 0;
-    const int blocks = ends_with_sides ? own_column_blocks(borders, NT, per_block) : ceil_div(NT, per_block);
+    const bool end_with_sides = !gp.mid && rank_tiles > 0 && own_blocks_end_with_sides(own, n_adapters, m);
+    const OwnBorders borders = own_borders(own, end_with_sides, NT, per_block);
+    const int blocks = rank_tiles > 0 && !gp.mid ? own_column_blocks(borders, NT, per_block) : ceil_div(NT, per_block);
     out[0] = gp.mid ? 2 : 1;
     out[1] = per_block;
     out[2] = gp.mid ? gp.mp.KS : plan.KS;
     out[3] = rank_tiles;
     for (int i = 0; i < blocks && 4 + 2 * i + 1 < capacity; ++i) {
         const BlockTiles t = gp.mid ? mid_block_tiles(i, gp.mp.pairs, NT)
-                                    : ends_with_sides ? own_block_tiles(borders, i, NT, per_block) : BlockTiles{i * per_block, NT};
+                                                    : own_block_tiles(borders, i, NT, per_block);
         out[4 + 2 * i] = t.first;
         out[4 + 2 * i + 1] = t.end;
     }

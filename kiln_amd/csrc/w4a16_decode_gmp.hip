@@ -796,7 +796,7 @@ hipError_t launch_gmp_tga(const DecodeArgs &a, hipStream_t stream) {
     int col_blocks = (NT + T - 1) / T;
     uint32_t in_upper[4] = {0u, 0u, 0u, 0u};  // of G, NT, GS and the column blocks
     if constexpr (kOwnTiles > 0) {
-        const OwnBorders b = own_borders(*a.lora_sides, NT, T);
+        const OwnBorders b = own_borders(*a.lora_sides, own_blocks_end_with_sides(*a.lora_sides, a.lora_adapters, a.M), NT, T);
         col_blocks = own_column_blocks(b, NT, T);
         in_upper[0] = (uint32_t)b.blocks0 << 16;
         in_upper[1] = (uint32_t)b.end0 << 16;

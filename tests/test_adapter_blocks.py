@@ -58,6 +58,22 @@ def test_automatic_plans(n, k, rank):
     assert own > 0
 
 
+@pytest.mark.parametrize("tiles", [2, 3, 5])
+def test_blocks_of_up_to_16_rows_end_with_sides_from_five_adapters_on(tiles):
+    L, n, k = _lib.load_tuning(), 1024, 1024
+    for borders in _splits(n):
+        sides = [(8, first, end - first) for first, end in zip((0,) + borders, borders + (n,))]
+        for n_adapters in (len(sides), 4, 5, 8):
+            L.kiln_w4a16_debug_gmp(tiles, 4, 1)
+            L.kiln_w4a16_debug_lora_fold(3)
+            plan, blocks = _blocks(L, 7, n, k, sides, n_adapters)
+            assert plan == (SMALL, tiles, 1, (8 * len(sides) + 15) // 16 if n_adapters <= 4 else 1)
+            _walk(plan, blocks, n // 16)
+            ends = {0, n // 16} | ({b // 16 for b in borders} if n_adapters > 4 else set())
+            assert {end for _, end in blocks} | {0} == ends
+            assert n_adapters > 4 or len(blocks) == -(-n // (16 * tiles))
+
+
 def _own(m, k, n, rank):
     plan, _ = _blocks(_lib.load(), m, n, k, [(rank, 0, n)], 1)
     return plan[3] > 0
@@ -67,24 +83,23 @@ def _own(m, k, n, rank):
     # short launches, the fewer ranks the shorter
     (1, 1024, 4096, 8, 1), (16, 1024, 4096, 8, 1), (1, 2560, 2560, 8, 1), (1, 2048, 2048, 32, 1), (1, 2560, 4096, 8, 1), (11, 1536, 8192, 8, 1),
     # 8 and 16 ranks whose projection in the first blocks ends before the launch would anyway
-    (1, 1536, 12288, 8, 0), (8, 1536, 12288, 8, 0), (1, 1536, 12288, 16, 0), (1, 4096, 3584, 8, 0), (8, 2560, 7936, 8, 0),
-    # longer ones: blocks of one tile that fill the chip against two tiles a block
-    (1, 4096, 4096, 8, 0), (11, 4096, 4096, 8, 0), (1, 5120, 4096, 8, 0), (8, 5120, 4096, 8, 0), (1, 6144, 4096, 8, 0),
-    # ... and those that are ahead by more
-    (1, 8192, 4096, 8, 1), (4, 5504, 7936, 16, 1), (1, 5504, 7936, 24, 1), (1, 4096, 1024, 8, 1), (8, 8192, 2048, 8, 1),
-    # two rounds of blocks against one, and against the mid-M kernel, where such a call goes from 8 rows on
-    (1, 11008, 4096, 8, 1), (4, 12032, 4096, 8, 1), (1, 18176, 4096, 8, 0), (1, 9088, 8192, 8, 0),
-    (8, 11008, 4096, 8, 0), (16, 11008, 4096, 8, 0), (16, 12032, 4096, 8, 0), (11, 5504, 8192, 8, 0), (16, 7808, 8192, 8, 0),
-    (16, 5504, 7936, 8, 1), (11, 5504, 7936, 32, 1),
+    (1, 1536, 16384, 8, 0), (1, 1536, 16384, 16, 0), (1, 4096, 3584, 8, 0), (8, 2560, 7936, 8, 0),
+    # K slices, which few blocks have
+    (1, 4096, 1024, 8, 1), (8, 8192, 2048, 8, 1),
+    # blocks of all of K that fill the chip, against wider ones, and others
+    (1, 4096, 4096, 8, 0), (11, 4096, 4096, 8, 0), (1, 5120, 4096, 8, 0), (8, 5120, 4096, 8, 0), (1, 6144, 4096, 8, 0), (1, 2048, 8192, 8, 0),
+    (1, 4096, 8192, 8, 0), (1, 2560, 8192, 8, 0), (4, 2048, 8192, 8, 1), (4, 5504, 7936, 16, 1), (1, 5504, 7936, 24, 1), (1, 5504, 8192, 24, 1),
+    # launches that fill the chip in one round: no border, no second round
+    (1, 11008, 4096, 8, 1), (16, 11008, 4096, 8, 1), (16, 12032, 4096, 16, 1), (1, 1024, 8192, 16, 1), (1, 2048, 8192, 16, 1),
+    # several rounds: wide blocks, or against many slices
+    (8, 6656, 16128, 8, 0), (8, 15104, 7936, 8, 0), (16, 8192, 19712, 8, 1), (1, 9216, 15616, 8, 1),
+    # the first way in three and four slices
+    (1, 12288, 4096, 8, 0), (8, 14336, 4096, 8, 0),
+    # from 17 rows on
+    (24, 4096, 4096, 8, 1), (24, 1024, 8192, 16, 1), (50, 2560, 8192, 16, 1), (64, 1536, 16384, 8, 1), (32, 3072, 16384, 16, 0),
 ])
-def test_where_blocks_of_up_to_16_rows_project_by_themselves(m, k, n, rank, own):
+def test_where_blocks_project_by_themselves(m, k, n, rank, own):
     assert _own(m, k, n, rank) == bool(own)
-
-
-def test_a_rank_that_is_padded_otherwise_takes_two_rounds_of_blocks_for_longer():
-    takes = _lib.load().kiln_w4a16_takes_rank
-    assert [takes(m, 4096, 11008, 4, -1) for m in (1, 8, 16)] == [1, 1, 0]
-    assert [takes(m, 4096, 12032, 4, -1) for m in (1, 8, 16)] == [1, 1, 0]
 
 
 @pytest.mark.parametrize("pairs", [1, 2, 3])

@@ -200,6 +200,38 @@ def test_sides_that_begin_anywhere_from_17_rows_on(m, pairs, i):
     _assert_close(out[:m], *_reference(x, w, list(zip(adapters, firsts))))
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [1, 7, 16])
+@pytest.mark.parametrize("tiles", [1, 3, 5])
+@pytest.mark.parametrize("i", [i for i, (_, _, _, places) in enumerate(SIDES_ANYWHERE) if sum(p[0] for p in places) <= 32])
+def test_up_to_four_adapters_that_begin_anywhere_give_the_stacked_sets_bits(i, tiles, m):
+    L, (k, ks, n, places) = _lib.load_tuning(), SIDES_ANYWHERE[i]
+    gen = torch.Generator(device="cuda").manual_seed(k + n + m)
+    w = _packed(gen, k, n, 128)
+    adapters = [_all_adapters(gen, k, (rows,), ((r,),))[0] for r, _, rows in places]
+    adapters = [lora.StackedLora(a.a_cat, a.b_cat, a.ranks, (0.5 + 0.25 * i,)) for i, a in enumerate(adapters)]
+    x = torch.randn(m, k, device="cuda", generator=gen).bfloat16()
+    ranks, scales = sum((a.ranks for a in adapters), ()), sum((a.scales for a in adapters), ())
+    a_cat, b_cat, col = torch.cat([a.a_cat for a in adapters]).contiguous(), torch.zeros(n, sum(ranks), dtype=torch.bfloat16, device="cuda"), 0
+    for a, (r, first, rows) in zip(adapters, places):
+        b_cat[first:first + rows, col:col + r] = a.b_cat
+        col += r
+    sides = _side_table(adapters, places)
+    L.kiln_w4a16_debug_gmp(tiles, 6, ks)
+    L.kiln_w4a16_debug_lora_fold(3)
+    plan = (ctypes.c_int * 4)()
+    blocks = L.kiln_w4a16_debug_adapter_blocks(m, n, k, 256, sides, len(places), 0, len(places), plan, 4)
+    assert (blocks, *plan) == (-(-n // (16 * tiles)), 1, tiles, ks, (sum(ranks) + 15) // 16)
+    ws = marlin_gemm._workspace(x.device, torch.cuda.current_stream().cuda_stream, L.kiln_w4a16_workspace_bytes(m, n, k))
+    out = torch.full((m + 1, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+    assert L.kiln_w4a16_gemm_adapter_sides(x.data_ptr(), w.b_packed.data_ptr(), out.data_ptr(), w.scales.data_ptr(), m, n, k, ws.data_ptr(), 128,
+                                           x.device.index, torch.cuda.current_stream().cuda_stream, sides, len(places), 0, len(ranks),
+                                           (ctypes.c_int * len(ranks))(*ranks), (ctypes.c_float * len(ranks))(*scales)) == _lib.OK
+    want = marlin_gemm.marlin_w4a16_gemm_lora(x, w.b_packed, w.scales, 128, a_cat, b_cat, ranks, scales)
+    assert bool(out[m].isnan().all()) and torch.equal(out[:m].view(torch.int16), want.view(torch.int16))
+    _assert_close(out[:m], *_reference(x, w, [(a, first) for a, (_, first, _) in zip(adapters, places)]))
+
+
 def test_ranks_that_are_taken_as_they_are():
     """Multiples of 8 always; of 4 where blocks project by themselves, up to 32 and on the kernels of few rows; nothing else."""
     takes = _lib.load().kiln_w4a16_takes_rank
