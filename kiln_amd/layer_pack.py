@@ -29,7 +29,7 @@ from typing import Dict, List, Optional, Sequence, Tuple
 import torch
 
 from . import _calls, marlin_gemm, marlin_proj
-from .lora import fuse_column_blocks, proj_forward, swiglu_forward, swiglu_lora_fits
+from .lora import fuse_column_blocks, proj_forward, sides_again, swiglu_forward, swiglu_lora_fits
 from .marlin_proj import MarlinPackedProj, MarlinProjError
 
 
@@ -113,13 +113,14 @@ class LayerProjections:
         loras = loras or {}
         fused = self.same_input_fused.get(kinds)
         if fused is not None:
-            ys = _calls.linear_sides(x, fused.b_packed, fused.scales, fused.groupsize, False, tuple(map(loras.get, kinds)),
-                                     tuple(self.packed[k].n for k in kinds), lora_scale, True)
+            own, widths = tuple(map(loras.get, kinds)), tuple(self.packed[k].n for k in kinds)
+            ys = _calls.linear_sides(x, fused.b_packed, fused.scales, fused.groupsize, False, own, widths, lora_scale, True)
+            if ys is None:
+                ys = sides_again(x, fused, False, own, widths, lora_scale, True)
             if ys is not None:
                 return ys
         stacked = None
         if fused is not None and any(loras.get(k) is not None for k in kinds):
-            widths = [self.packed[k].n for k in kinds]
             stacked = fuse_column_blocks([loras.get(k) for k in kinds], widths, lora_scale)
             if sum(stacked.ranks) > 64 or len(stacked.ranks) > 8:
                 fused = None

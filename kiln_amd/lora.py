@@ -72,6 +72,17 @@ def merge_concat(adapters: Sequence[LoraProjectionWeights], weights: Sequence[fl
     return LoraProjectionWeights(a_cat, b_cat)
 
 
+def sides_again(x: torch.Tensor, packed: MarlinPackedProj, swiglu: bool, adapters: tuple, widths: tuple, lora_scale: float, split: bool):
+    """A call that `_calls.linear_sides`, which wants a contiguous x and a workspace that is there, has not taken: both are made
+    and the call repeated, before the checked routes, which stack the adapters, get their turn (None).  Where blocks project x
+    by themselves a stacked set may be projected elsewhere, T be rounded at other places and the result differ in bits: by those
+    routes the first call of a stream differed from the calls after it, and one on a strided x from one on its copy."""
+    if not x.is_cuda or x.dtype != torch.bfloat16 or x.dim() not in (2, 3) or x.shape[-1] != packed.k or x.numel() == 0:
+        return None
+    marlin_gemm.stream_workspace(x, packed.n)
+    return _calls.linear_sides(x.contiguous(), packed.b_packed, packed.scales, packed.groupsize, swiglu, adapters, widths, lora_scale, split)
+
+
 def proj_forward(x: torch.Tensor, packed: MarlinPackedProj, lora, lora_scale: float = 1.0) -> torch.Tensor:
     """`base = matmul_bf16(x, packed)`; with LoRA, `base + delta` in one kernel
     (forward.rs:2932-2939).  `lora` is None, a LoraProjectionWeights (scaled by `lora_scale`)
@@ -79,6 +90,8 @@ def proj_forward(x: torch.Tensor, packed: MarlinPackedProj, lora, lora_scale: fl
     if lora is None:
         return matmul_bf16(x, packed)
     y = _calls.linear_sides(x, packed.b_packed, packed.scales, packed.groupsize, False, (lora,), (packed.n,), lora_scale, False)
+    if y is None:
+        y = sides_again(x, packed, False, (lora,), (packed.n,), lora_scale, False)
     if y is not None:
         return y
     if isinstance(lora, LoraProjectionWeights):
@@ -104,8 +117,10 @@ def swiglu_forward(x: torch.Tensor, gate_up: MarlinPackedProj, gate_lora=None, u
     the two `mlp_proj_forward` calls with `lora_layer.gate_proj` / `up_proj`, `silu` and the multiply of
     forward.rs:2771-2819.  `gate_lora` / `up_lora` are None, a LoraProjectionWeights (scaled by
     `lora_scale`) or a StackedLora; together at most 64 rank columns and 8 adapters."""
-    y = _calls.linear_sides(x, gate_up.b_packed, gate_up.scales, gate_up.groupsize, True, (gate_lora, up_lora),
-                            (gate_up.n // 2, gate_up.n // 2), lora_scale, False)
+    widths = (gate_up.n // 2, gate_up.n // 2)
+    y = _calls.linear_sides(x, gate_up.b_packed, gate_up.scales, gate_up.groupsize, True, (gate_lora, up_lora), widths, lora_scale, False)
+    if y is None:
+        y = sides_again(x, gate_up, True, (gate_lora, up_lora), widths, lora_scale, False)
     if y is not None:
         return y
     if x.dim() not in (2, 3) or x.shape[-1] != gate_up.k:

@@ -43,6 +43,13 @@ def _workspace(device: torch.device, stream_ptr: int, nbytes: int) -> torch.Tens
     return ws
 
 
+def stream_workspace(a: torch.Tensor, n: int) -> torch.Tensor:
+    """The workspace of the current stream of `a`'s device, large enough for a GEMM of `a`, `[..., k]`, and n columns."""
+    with torch.cuda.device(a.device):
+        stream = torch.cuda.current_stream(a.device).cuda_stream
+        return _workspace(a.device, stream, _lib.load().kiln_w4a16_workspace_bytes(a.numel() // a.shape[-1], n, a.shape[-1]))
+
+
 def workspace_wait_status(device: torch.device | None = None) -> int:
     """OR of the sticky words of every workspace this module holds on `device` (all devices if None):
     0 unless a bounded wait inside some launch gave up (`_lib.WAIT_*` says which kind).  Synchronises
