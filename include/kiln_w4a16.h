@@ -253,8 +253,10 @@ kiln_marlin_status_t kiln_w4a16_stack_adapters(
 
 /*
  * Do the entry points with adapters take a stacked rank as it is at its best (1), or is it worth rounding up to a multiple
- * of 8 with zeros in front (0: kiln_w4a16_stack_adapters)?  Multiples of 8 always; multiples of 4
- * up to 32 on calls of up to 16 rows, and of a few hundred, whose launch is short.  A pure query; every rank up to 64 is taken either way.
+ * of 8 with zeros in front (0: kiln_w4a16_stack_adapters)?  Multiples of 8 always; multiples of 4 up to 32 where the
+ * dispatcher has every block project x by itself, at any row count and mostly on short launches: 5120 -> 27648 takes none at
+ * one row, 9216 -> 2560 takes 4 and 12 there and 20 too from 5 on.  So ask for each (m, n, k).  A pure query; every rank up to 64 is taken
+ * either way.
  */
 int kiln_w4a16_takes_rank(int prob_m, int prob_n, int prob_k, int r_total, int dev);
 

@@ -1017,10 +1017,6 @@ int lora_kind(const LoraSpec *lora, int m) {
     return ranks <= 32 ? own_kind({(ranks + 7) / 8, many, lora->r_total % 8 != 0, borders}) : otherwise;
 }
 
-// Bytes a call of m rows needs, made monotone in m: the largest need of any m' <= m.  The plan
-// (and with it the need) changes with m' only through the small-M and mid-M runs (m' <= 1024 here; beyond
-// that only overrides keep a call on that path) and through the matrix-core kernel's row blocks
-// of 64 or 128 rows, so those m' are the ones evaluated.
 #ifndef KILN_W4A16_TUNING_HOOKS
 // What workspace_bytes_upto found, by its arguments: the sizing walks over hundreds of plans (0.35...0.55 ms
 // of host time from 512 rows on), and callers that size per call -- the Python wrappers do -- ask for the
@@ -1042,6 +1038,11 @@ std::mutex g_size_mutex;
 std::unordered_map<SizeKey, size_t, SizeKeyHash> g_size_cache;
 #endif
 
+// Bytes a call of m rows needs, made monotone in m: the largest need of any m' <= m.  The plan
+// (and with it the need) changes with m' only through the small-M and mid-M runs (m' <= 1024 here; beyond
+// that only overrides keep a call on that path) and through the matrix-core kernel's row blocks
+// of 64 or 128 rows, so those m' are the ones evaluated.
+// (Calls whose blocks project x by themselves need no more: their K slices meet in the zeroed region or not at all.)
 size_t workspace_bytes_upto(int m, int n, int k, int cus, int thread_k, int thread_n) {
 #ifndef KILN_W4A16_TUNING_HOOKS
     const SizeKey key{m, n, k, cus, thread_k, thread_n};

@@ -135,8 +135,8 @@ struct GmpScheduleOf {
 };
 
 constexpr int gmp_slots(int gpw) { return gpw < 2 ? gpw : 2; }
-// wavefronts of a block, at most; own: as many as have their slots in 160 KiB of LDS (10 or 13 of the instances of two
-// rank tiles, which need more registers than 16 can have)
+// wavefronts of a block, at most; own: as many as have their slots in 160 KiB of LDS (of two rank tiles 9 with two slots of A
+// each and 13 with one, of one tile 13 with two; the former also need more registers than 16 wavefronts can have)
 constexpr int gmp_max_waves(int gpw, int own) {
     const int fit = (160 * 1024 - 128) / ((gmp_slots(gpw) + own) * kGmpSlotBytes);
     return own == 0 || fit > kGmpMaxWaves ? kGmpMaxWaves : fit;

@@ -50,8 +50,8 @@ def stack_adapters(adapters: Sequence[LoraProjectionWeights], scales: Sequence[f
 def pad_rank(stacked: StackedLora) -> StackedLora:
     """The same adapters with the stacked rank rounded up to a multiple of 8 (the last adapter gets zero rows of A
     and zero columns of B, which add exact zeros): the library's kernels with the low-rank term built in take
-    stacked ranks that are multiples of 8, any other goes the general route (a call of 16 rows on the widest
-    projection: 14 us against 9).  Worth doing once where adapters are loaded; the calls below do it where they
+    stacked ranks that are multiples of 8 (and of 4 where `kiln_w4a16_takes_rank` says so), any other goes the general
+    route (a call of 16 rows on the widest projection: 14 us against 9).  Worth doing once where adapters are loaded; the calls below do it where they
     stack per call.  Unchanged if the rank is a multiple of 8 already or would pass 64."""
     r_total = sum(stacked.ranks)
     pad = -r_total % 8

@@ -125,6 +125,11 @@ def test_more_than_four_adapters_side_by_side(k, widths, ranks, m):
     for plan in ((0, 0, 0), (5, 4, 1), (3, 4, 1)) if k < 4608 else ((0, 0, 0), (5, 9, 2), (3, 6, 2)):
         L.kiln_w4a16_debug_gmp(*plan)
         L.kiln_w4a16_debug_lora_fold(3)
+        # the blocks' own way: of one side's ranks and ending with it from five adapters on, of all ranks else
+        info, many = (ctypes.c_int * 4)(), len(each) > 4
+        blocks = L.kiln_w4a16_debug_adapter_blocks(m, n, k, 256, sides, len(own), 0, len(each), info, 4)
+        most = max(a.a_cat.shape[0] for a, _ in own) if many else sum(each)
+        assert info[0] == 1 and info[3] == (most + 15) // 16 and (many or blocks == -(-n // (16 * info[1])))
         ws = marlin_gemm._workspace(x.device, stream, L.kiln_w4a16_workspace_bytes(m, n, k))
         out = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda")
         assert L.kiln_w4a16_gemm_adapter_sides(x.data_ptr(), w.b_packed.data_ptr(), out.data_ptr(), w.scales.data_ptr(), m, n, k, ws.data_ptr(), 128,
@@ -238,6 +243,9 @@ def test_ranks_that_are_taken_as_they_are():
     assert [r for r in range(0, 67) if takes(4, 2560, 2560, r, -1)] == sorted({4, 12, 20, 28} | set(range(8, 65, 8)))
     assert [m for m in (0, 1, 16, 17, 64, 256, 300) if takes(m, 2560, 2560, 12, -1)] == [1, 16, 17, 64]
     assert takes(4, 2560, 2500, 12, -1) == takes(4, 100, 2560, 12, -1) == 0  # no shape of the kernels
+    # long launches of up to 16 rows take fewer of them as they are, or none
+    assert [[r for r in (4, 12, 20, 28, 8) if takes(m, 27648, 5120, r, -1)] for m in (1, 8, 16)] == [[8]] * 3
+    assert [[r for r in (4, 12, 20, 28) if takes(m, 2560, 9216, r, -1)] for m in (1, 16)] == [[4, 12], [4, 12, 20]]
 
 
 def test_a_wavefront_without_groups_finishes_no_ranks():
