@@ -519,9 +519,12 @@ PyObject *py_quantize(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
             first += items[(size_t)i].n;
         }
         // The first run's weights go ahead, as soon as their memory is there, so that the GPU works on them while the host
-        // makes the rest ready (a dozen tensors and a launch, 10 to 15 us): where they take it 4 us and more, one launch of
-        // weights with scales per group (per column they would be three).  A layer of 2560 / 9216, seven weights: 100.9 -> 97.6 us.
-        if (r == 0 && !paired && head.g == 128 && head.k * columns >= (int64_t)8 << 20 && runs[r].size() < items.size()) {
+        // makes the rest ready (a dozen tensors and a launch, 10 to 15 us): one launch of weights with scales per group (per
+        // column they would be three) that takes it 6 us and more.  A layer of 2560 / 9216, seven weights: 100.9 -> 97.6 us; the call
+        // on layers of other widths, full and linear attention: 4096 / 12288 171 -> 168 and 177 -> 172, 2048 / 5632 (16.8 M and 18.9 M weights in the
+        // run) 67.4 -> 65.6 and 66.4 -> 63.9, 1792 / 4864 (13.8 and 15.1) 63.1 -> 63.1 and 61.2 -> 60.5, but 1536 / 5120 (10.2 and 10.6) 62.4 ->
+        // 63.9 and 58.1 -> 59.2: the launch more costs what the GPU gains on them.
+        if (r == 0 && !paired && head.g == 128 && head.k * columns >= (int64_t)14 << 20 && runs[r].size() < items.size()) {
             for (int i : runs[r]) {
                 queue(items[(size_t)i]);
                 launched[(size_t)i] = true;

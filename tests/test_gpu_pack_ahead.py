@@ -8,7 +8,7 @@ from kiln_amd import marlin_proj
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("groupsize", [128, -1])
-@pytest.mark.parametrize("columns", [3840, 4096])  # of 2048 rows: below and from 8 Mi weights on
+@pytest.mark.parametrize("columns", [3840, 4096, 6912, 7168])  # of 2048 rows: below and from 14 Mi weights on
 @pytest.mark.parametrize("others", [0, 1, 3])
 def test_the_run_ahead_and_the_rest(columns, others, groupsize):
     gen = torch.Generator(device="cuda").manual_seed(columns + others)
