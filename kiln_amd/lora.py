@@ -79,7 +79,8 @@ def sides_again(x: torch.Tensor, packed: MarlinPackedProj, swiglu: bool, adapter
     routes the first call of a stream differed from the calls after it, and one on a strided x from one on its copy."""
     if not x.is_cuda or x.dtype != torch.bfloat16 or x.dim() not in (2, 3) or x.shape[-1] != packed.k or x.numel() == 0:
         return None
-    marlin_gemm.stream_workspace(x, packed.n)
+    if not marlin_gemm.make_workspace(x, packed.n) and x.is_contiguous():
+        return None    # refused for another reason
     return _calls.linear_sides(x.contiguous(), packed.b_packed, packed.scales, packed.groupsize, swiglu, adapters, widths, lora_scale, split)
 
 

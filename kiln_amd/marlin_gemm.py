@@ -43,11 +43,12 @@ def _workspace(device: torch.device, stream_ptr: int, nbytes: int) -> torch.Tens
     return ws
 
 
-def stream_workspace(a: torch.Tensor, n: int) -> torch.Tensor:
-    """The workspace of the current stream of `a`'s device, large enough for a GEMM of `a`, `[..., k]`, and n columns."""
+def make_workspace(a: torch.Tensor, n: int) -> bool:
+    """See to it that the current stream of `a`'s device has a workspace for a GEMM of `a`, `[..., k]`, and n columns; had it none?"""
     with torch.cuda.device(a.device):
         stream = torch.cuda.current_stream(a.device).cuda_stream
-        return _workspace(a.device, stream, _lib.load().kiln_w4a16_workspace_bytes(a.numel() // a.shape[-1], n, a.shape[-1]))
+        before = _workspaces.get((a.device.index, stream))
+        return _workspace(a.device, stream, _lib.load().kiln_w4a16_workspace_bytes(a.numel() // a.shape[-1], n, a.shape[-1])) is not before
 
 
 def workspace_wait_status(device: torch.device | None = None) -> int:
